@@ -1,5 +1,5 @@
-"""Builds binarybrain_amd/lib/libbbhip.so (hand-written HIP kernels + the C ABI) for gfx950 with hipcc, and the
-C++ programs that exercise the host-side model classes."""
+"""Builds binarybrain_amd/lib/libbbhip.so (hand-written HIP kernels + the C ABI) for gfx950 with hipcc, the extension module that the
+Python layer calls it through, and the C++ programs that exercise the host-side model classes."""
 import os
 import subprocess
 
@@ -8,6 +8,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libbbhip.so")
+NATIVE_PATH = os.path.join(LIB_DIR, "_bbops.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # packed fp32 VALU instructions are disabled on purpose: scalar fp32 code must not be auto-vectorised into v_pk_* forms
@@ -33,6 +34,19 @@ def build_library(verbose=False):
     return LIB_PATH
 
 
+def build_native(verbose=False):
+    """lib/_bbops.so: the extension module that binarybrain_amd/ops.py calls the library through (host code only)."""
+    import sysconfig
+    import torch
+    t = os.path.dirname(torch.__file__)
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I" + os.path.join(t, "include"),
+          "-I" + os.path.join(t, "include", "torch", "csrc", "api", "include"), "-I/opt/rocm/include", "-I" + sysconfig.get_paths()["include"],
+          os.path.join(CSRC, "ops_native.cpp"), "-o", NATIVE_PATH, "-L" + LIB_DIR, "-lbbhip", "-L" + os.path.join(t, "lib"),
+          "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10_hip", "-lc10", "-Wl,-rpath,$ORIGIN"], verbose)
+    return NATIVE_PATH
+
+
 def build_bench_probe(verbose=False):
     """bench_gather_probe.so beside bench.py: the instrumentation kernel of `bench.py --workload gather_ceiling` (not part of the library)."""
     out = os.path.join(ROOT, "bench_gather_probe.so")
@@ -56,3 +70,4 @@ def build_cpp_tests(verbose=False):
 
 if __name__ == "__main__":
     print(build_library(verbose=True))
+    print(build_native(verbose=True))

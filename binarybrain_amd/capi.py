@@ -1,8 +1,10 @@
 """ctypes binding of the C ABI in include/bbhip.h.  Device memory and streams come from torch; nothing here computes."""
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
-from .build import LIB_PATH
+from .build import LIB_PATH, NATIVE_PATH
 
 _lib = None
 
@@ -160,3 +162,21 @@ def ptr(t):
 def stream_ptr():
     import torch
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+class _Native:
+    """The extension module of csrc/ops_native.cpp, loaded by its first use; its functions become attributes of this object."""
+
+    def __getattr__(self, name):
+        lib()
+        if not os.path.exists(NATIVE_PATH):
+            raise BbhipError("%s is missing: build it with `python -m binarybrain_amd.build` (or __graft_entry__.build())" % NATIVE_PATH)
+        import torch        # noqa: F401  the extension links against torch's libraries
+        loader = importlib.machinery.ExtensionFileLoader("_bbops", NATIVE_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_bbops", NATIVE_PATH, loader=loader))
+        module.set_error_type(BbhipError)
+        self.__dict__.update((k, v) for k, v in vars(module).items() if not k.startswith("__"))
+        return self.__dict__[name]
+
+
+native = _Native()

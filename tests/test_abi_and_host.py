@@ -74,3 +74,14 @@ def test_binding_header_signatures():
         build_cpp_tests()
     res = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
     assert res.returncode == 0 and "signatures equal the reference's declarations" in res.stdout, res.stdout
+
+
+def test_native_calls_check_their_arguments():
+    import torch
+    from binarybrain_amd import capi, ops
+    with pytest.raises(capi.BbhipError, match="device tensors"):
+        ops.stochastic_lut_forward(6, torch.zeros(8, 64), torch.zeros((2, 6), dtype=torch.int32), torch.zeros(2, 64), 64)
+    with pytest.raises(TypeError, match="expected a torch tensor"):
+        capi.native.fp32_Vector_set(3, 1.0, 4)
+    with pytest.raises(TypeError, match="arguments"):
+        capi.native.fp32_Vector_set(3)
