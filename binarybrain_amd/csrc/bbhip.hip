@@ -14,6 +14,7 @@
 
 #include "../../include/bbhip.h"
 #include "lut_kernels.hpp"
+#include "corner_backward_kernels.hpp"
 #include "vector_kernels.hpp"
 #include "conv_kernels.hpp"
 #include "tail_kernels.hpp"
@@ -143,12 +144,6 @@ bool use_corner_values(int xmode)
 bool pack_binarized_input(void) { static bool const on = env_switch("BBHIP_PACK", true); return on; }
 // the corner-value forward kernel derives a node's tables in the wavefront where no packing launch carries the preparation (0 = a table launch)
 bool inline_tables(void) { static bool const on = env_switch("BBHIP_INLINE_TABLES", true); return on; }
-// packed rows in the dx kernel read with one scalar load per row and pass where pitch and alignment allow (0 = vector loads + read-lanes)
-bool term_from_corner_values(void) { static bool const on = env_switch("BBHIP_TERM_NODES", true); return on; }
-bool dx_indexed(void) { static bool const on = env_switch("BBHIP_DX_INDEXED", true); return on; }
-bool dx_wide_rows(void) { static bool const on = env_switch("BBHIP_DX_WIDE", true); return on; }
-int dx_wide_max_rows(void) { static int const v = env_int("BBHIP_DX_WIDE_ROWS", 1024); return v; }
-
 // frames per unit; both are rounded to wavefront multiples where used
 int fwd_nodes_per_wave(void) { static int v = env_int("BBHIP_FWD_NODES", 2); return v >= 2 ? 2 : 1; }
 // Frames per forward unit.  fp32 rows are gathered through L2, and a 256-frame piece of every input row is what one XCD's L2
@@ -312,10 +307,6 @@ template <int N>
 int dispatch_backward(int xmode, int kind, int dxmode, BwdArgs const &a, hipStream_t st)
 {
     dim3 const grid(a.tt.blocks + a.slab_count * a.tiles.count), block(kBlock);
-    if (xmode == kXBit && kind == 1 && dxmode == kDxNone && a.V != nullptr) {       // batch-norm window from the corner values
-        hipLaunchKernelGGL((lut_backward_kernel<N, kXBit, 1, kDxNone, true>), grid, block, 0, st, a);
-        return 0;
-    }
 #define BBHIP_BWD_CASE(X, K, M) if (xmode == X && kind == K && dxmode == M) { hipLaunchKernelGGL((lut_backward_kernel<N, X, K, M>), grid, block, 0, st, a); return 0; }
     BBHIP_BWD_CASE(kXClamp,  0, kDxAtomic) BBHIP_BWD_CASE(kXClamp,  0, kDxTmp)
     BBHIP_BWD_CASE(kXBinary, 0, kDxAtomic) BBHIP_BWD_CASE(kXBinary, 0, kDxTmp)
@@ -334,11 +325,6 @@ template <int N, int U>
 int dispatch_dx_u(int xmode, DxArgs const &a, hipStream_t st)
 {
     dim3 const grid(a.fin_blocks + a.chunk_count * a.tiles.count), block(kBlock);
-    if (use_corner_values(xmode)) {         // the term table then holds corner values
-        if (xmode == kXBit) { hipLaunchKernelGGL((lut_dx_corner_kernel<N, kXBit, U>),    grid, block, 0, st, a); }
-        else                { hipLaunchKernelGGL((lut_dx_corner_kernel<N, kXBinary, U>), grid, block, 0, st, a); }
-        return 0;
-    }
     switch (xmode) {
     case kXClamp:  hipLaunchKernelGGL((lut_dx_kernel<N, kXClamp, U>),  grid, block, 0, st, a); return 0;
     case kXBinary: hipLaunchKernelGGL((lut_dx_kernel<N, kXBinary, U>), grid, block, 0, st, a); return 0;
@@ -640,11 +626,137 @@ int check_backward(BackwardCall const &c, int dxmode)
     return 0;
 }
 
+// Frames per unit of the per-corner sums.  A launch runs in ceil(workgroups / 512) rounds of resident workgroups (two per compute unit: 64 KB of
+// bins each), a unit costs its frames plus about 1024 frames' worth of set-up and closing sums, and more than one slab per node needs the fold
+// launch (about 3072 frames' worth on top): the slab length with the least of it.
+int corner_slab_frames(int frame_size, int tile_count)
+{
+    if (bwd_slab_frames() > 0) { return ceil_div(bwd_slab_frames(), 256) * 256; }
+    auto cost = [&](long long frames) {
+        long long const slabs = (frame_size + frames - 1) / frames, rounds = (slabs * tile_count + 511) / 512;
+        return rounds * ((frames < frame_size ? frames : frame_size) + 1024) + (slabs > 1 ? 3072 : 0);
+    };
+    int best = ceil_div(frame_size, 256) * 256;
+    for (int cand = 1024; cand < frame_size && cand <= 65536; cand *= 2) { if (cost(cand) < cost(best)) { best = cand; } }
+    return best;
+}
+
+template <int N, bool BN>
+int launch_corner_backward(CornerSumsArgs const &s, int slab_count, hipStream_t st)
+{
+    {
+        ScopedTimer tm(kTimeBackward, st);
+        hipLaunchKernelGGL((lut_corner_sums_kernel<N, BN>), dim3(s.slab_count * s.tiles.count), dim3(kBlock), 0, st, s);
+    }
+    BBHIP_LAUNCH_CHECK();
+    if (slab_count > 1) {
+        hipLaunchKernelGGL((lut_corner_fold_kernel<N, BN>), dim3(s.node_size), dim3(kBlock), 0, st, s.fold, s.partial, s.V ? s.V : s.V_out, s.node_size, slab_count);
+        BBHIP_LAUNCH_CHECK();
+    }
+    return 0;
+}
+
+template <int N, bool BN>
+int dispatch_dx_table(int quads, DxTableArgs const &t, hipStream_t st)
+{
+    dim3 const grid(t.dx.chunk_count * t.dx.tiles.count), block(kBlock);
+    ScopedTimer tm(kTimeDx, st);
+    switch (quads) {
+    case 1:  hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, 1>), grid, block, 0, st, t); break;
+    case 2:  hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, 2>), grid, block, 0, st, t); break;
+    default: hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, 4>), grid, block, 0, st, t); break;
+    }
+    BBHIP_LAUNCH_CHECK();
+    return 0;
+}
+
+// Two-valued inputs with the deterministic dx (corner_backward_kernels.hpp): per-corner sums, fold, dx from kept corner indices.
+template <int N>
+int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHint packed, PreparedTablesHint tables, int dw_overwrite)
+{
+    constexpr int NN = 1 << N;
+    if (check_backward(call, kDxNone)) { return 1; }
+    BackwardCall c = call;
+    // fp32 frames are packed to bits first, unless the caller kept the packed copy from the forward call
+    bool const from_fp32 = (c.xmode == kXBinary);
+    bool const have_bits = from_fp32 && packed.bits != nullptr && packed.holds_input && packed.rows == c.input_node_size &&
+                           packed.row_words >= (c.frame_size + 31) / 32 && packed.row_words % 8 == 0 &&
+                           (reinterpret_cast<uintptr_t>(packed.bits) & 31u) == 0;
+    if (from_fp32) { c.x_stride = have_bits ? packed.row_words : packed_row_words(c.frame_size); }
+
+    int const O = c.output_node_size, tile_count = ceil_div(O, kWavesPerBlk);
+    int slab = corner_slab_frames(c.frame_size, tile_count);
+    size_t const slab_bytes = (size_t)O * NN * sizeof(float) * (c.bn ? 2 : 1);
+    while ((size_t)ceil_div(c.frame_size, slab) * slab_bytes > ((size_t)256 << 20) && slab < c.frame_size) { slab *= 2; }
+    int const slab_count = ceil_div(c.frame_size, slab);
+    if ((long long)slab_count * tile_count > 0x7fffffffLL) { return fail("backward: grid too large"); }
+    int const own_words = ceil_div(c.frame_size, 32) * 8;
+
+    // the nodes' corner values: from the buffer that the caller kept from this step's forward call, else derived by the sums kernel
+    size_t const v_bytes     = align256((size_t)O * NN * sizeof(float));
+    bool const   have_tables = tables.holds_tables && tables_fit(tables, 2 * v_bytes);
+    size_t const own_bytes   = align256((size_t)O * own_words * sizeof(uint32_t));
+    size_t const const_bytes = c.bn ? align256((size_t)O * sizeof(float4)) : 0;
+    size_t const part_bytes  = slab_count > 1 ? align256((size_t)slab_count * slab_bytes) : 0;
+    size_t const bits_bytes  = (from_fp32 && !have_bits) ? align256((size_t)c.input_node_size * c.x_stride * sizeof(uint32_t)) : 0;
+    char *base = nullptr;
+    if (arena_get(v_bytes + own_bytes + const_bytes + part_bytes + bits_bytes, &base, st)) { return 1; }
+    float    *V      = reinterpret_cast<float *>(base);
+    uint32_t *own    = reinterpret_cast<uint32_t *>(base + v_bytes);
+    float4   *consts = reinterpret_cast<float4 *>(base + v_bytes + own_bytes);
+    float    *part   = reinterpret_cast<float *>(base + v_bytes + own_bytes + const_bytes);
+    uint32_t *bits   = reinterpret_cast<uint32_t *>(base + v_bytes + own_bytes + const_bytes + part_bytes);
+    if (have_tables) { V = reinterpret_cast<float *>(reinterpret_cast<char *>(tables.buf) + v_bytes); }
+    if (have_bits) { c.x = packed.bits; }
+    else if (from_fp32) {
+        if (launch_binarize_pack(reinterpret_cast<float const *>(call.x), call.x_stride, bits, c.x_stride, c.input_node_size, c.frame_size, st)) { return 1; }
+        c.x = bits;
+    }
+
+    CornerSumsArgs s{};
+    s.x = reinterpret_cast<uint32_t const *>(c.x); s.dy = c.dy; s.idx = c.idx;
+    if (have_tables) { s.V = V; }
+    else             { s.W_inline = c.W; s.V_out = V; }
+    s.lut_binarize = c.lut_binarize; s.bias = c.bias;
+    s.node_size = O; s.frame_size = c.frame_size; s.x_stride = c.x_stride; s.dy_stride = c.frame_stride;
+    s.slab = slab; s.slab_count = slab_count; s.tiles = make_tile_divisor(tile_count);
+    s.own = own; s.own_stride = own_words; s.partial = part;
+    s.fold.mean = c.mean; s.fold.rstd = c.rstd; s.fold.gamma = c.gamma; s.fold.beta = c.beta; s.fold.inv_frames = 1.0f / (float)c.frame_size;
+    s.fold.frame_size = c.frame_size; s.fold.lo = 0.5f - c.bias; s.fold.hi = 0.5f + c.bias;
+    s.fold.dW = c.dW; s.fold.overwrite = dw_overwrite; s.fold.node_consts = consts;
+    s.dy_quads = (c.frame_stride >= ((c.frame_size + 3) & ~3)) ? 1 : 0;
+    if (c.bn ? launch_corner_backward<N, true>(s, slab_count, st) : launch_corner_backward<N, false>(s, slab_count, st)) { return 1; }
+
+    DxTableArgs t{};
+    // Frames per pass: a term's table and its loads are shared by the steps of a pass, so long passes where all the rows of dy and of indices
+    // that a pass gathers from (5 bytes per node and frame) stay in an XCD's L2; halved while the launch would fall short of workgroups.
+    static int const quads_env = env_int("BBHIP_DX_QUADS", 0);
+    int quads = (O <= 512) ? 4 : (O <= 1024) ? 2 : 1;
+    while (quads > 1 && (long long)ceil_div(c.frame_size, quads * 256) * ceil_div(c.input_node_size, kWavesPerBlk) < 2048) { quads /= 2; }
+    if (quads_env == 1 || quads_env == 2 || quads_env == 4) { quads = quads_env; }
+    DxArgs &d = t.dx;
+    d.dy = c.dy; d.dx = c.dx; d.rev = c.rev; d.rev_stride = c.rev_stride; d.input_node_size = c.input_node_size; d.frame_size = c.frame_size;
+    d.dy_stride = c.frame_stride; d.dx_stride = c.frame_stride;
+    d.chunk = quads * 256; d.chunk_count = ceil_div(c.frame_size, d.chunk);
+    bool const split   = dx_split_lists(c.rev_stride - 1, (long long)d.chunk_count * ceil_div(c.input_node_size, kWavesPerBlk));
+    int const in_tiles = split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
+    if ((long long)d.chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
+    d.tiles = make_tile_divisor(in_tiles); d.split = split ? 1 : 0;
+    t.dy_quads = s.dy_quads;
+    t.dx_quads = (c.frame_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(c.dx) & 15u) == 0) ? 1 : 0;
+    t.own = own; t.own_stride = own_words; t.V = V; t.node_consts = consts;
+    t.gamma = c.gamma; t.beta = c.beta; t.inv_step = 1.0f / (s.fold.hi - s.fold.lo);
+    return c.bn ? dispatch_dx_table<N, true>(quads, t, st) : dispatch_dx_table<N, false>(quads, t, st);
+}
+
 template <int N>
 int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packed = PackedInputHint{nullptr, 0, 0, 0},
                  PreparedTablesHint tables = PreparedTablesHint{nullptr, 0, 0}, int dw_overwrite = 0)
 {
     constexpr int NN = 1 << N;
+    // two-valued inputs, deterministic dx: the pass over per-corner sums (needs neither term table nor LUT evaluation).  It takes slopes
+    // from differences of corner values, which lose digits as the two values of an input move together: from 1/8 apart.
+    if (g_dx_mode == 0 && use_corner_values(call.xmode) && fabsf(call.bias) >= 0.0625f) { return run_backward_corner<N>(call, st, packed, tables, dw_overwrite); }
     int dxmode = (g_dx_mode == 1) ? kDxAtomic : (g_dx_mode == 2) ? kDxTmp : kDxNone;
     // The term table of the deterministic dx kernel has one slot per (input node, position in the longest fan-out list).  With
     // evenly used inputs that is about the number of connections; wiring in which a few inputs feed very many nodes would make
@@ -658,16 +770,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
     }
     if (check_backward(call, dxmode)) { return 1; }
 
-    // fp32 frames that the layer binarizes at 0.5 are packed to bits once (reading them once costs less than the three
-    // kernels of this pass gain from packed rows); from here on the call is a packed-bit call
-    BackwardCall c = call;
-    bool const pack = (c.xmode == kXBinary) && dxmode == kDxNone && use_corner_values(kXBinary) && pack_binarized_input();
-    // a caller that kept the packed copy of this input from the forward call hands it back: nothing to pack
-    bool const have_bits = pack && packed.bits != nullptr && packed.holds_input && packed.rows == c.input_node_size &&
-                           packed.row_words >= (c.frame_size + 31) / 32 && packed.row_words % 8 == 0 &&
-                           (reinterpret_cast<uintptr_t>(packed.bits) & 31u) == 0;
-    if (pack) { c.xmode = kXBit; c.x_stride = have_bits ? packed.row_words : packed_row_words(c.frame_size); c.x = nullptr; }   // else: a place in the arena below
-
+    BackwardCall const &c = call;
     int const tile_count = ceil_div(c.output_node_size, kWavesPerBlk);
     int const range      = (dxmode == kDxTmp) ? (c.tmp_frame_size < c.frame_size ? c.tmp_frame_size : c.frame_size) : c.frame_size;
     int const range_count = ceil_div(c.frame_size, range);
@@ -710,26 +813,12 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
     int const stat_chunk       = fwd_chunk_frames(c.xmode, c.frame_size, ceil_div(c.output_node_size, kWavesPerBlk * stat_npw));
     int const stat_chunk_count = ceil_div(c.frame_size, stat_chunk);
     size_t const stat_bytes = c.bn ? align256((size_t)stat_chunk_count * c.output_node_size * 2 * sizeof(float)) : 0;
-    // Batch-norm backward of a small batch over packed rows: the statistics pass (passes of four steps over 32-byte groups of the rows)
-    // keeps the corner index it forms of every (node, frame), a byte each, and the dx kernel looks a term's value up at that index
-    // instead of reading the consumer's other five rows and forming the index again (lut_dx_indexed_kernel): a third of the vector
-    // instructions per term.  That pays where dy and the indices stay close to the compute units (classifier step: dx of the three
-    // layers 43.9 -> 38 us); at 4096 x 4096 x 8192 and at the conv block's 230 400 frames the dx kernel is bound by the gather of its
-    // dy rows and the kept bytes only add traffic (128.5 vs 128.1 us, 121 vs 114 us, statistics pass + 6 us): up to 32 MiB of both.
-    int const own_words = ceil_div(c.frame_size, 256) * kWave;
-    bool const indexed = c.bn && dxmode == kDxNone && corner && term_from_corner_values() && c.xmode == kXBit && dx_indexed() &&
-                         dx_pass_steps_env() == 0 && (dx_chunk_frames_env() == 0 || dx_chunk_frames_env() % 256 == 0) &&
-                         c.x_stride % 8 == 0 && stat_chunk % 256 == 0 &&
-                         (size_t)c.output_node_size * c.frame_size * 5 <= ((size_t)32 << 20);
-    size_t const own_bytes = indexed ? align256((size_t)c.output_node_size * own_words * sizeof(uint32_t)) : 0;
-    size_t const term_count = (dxmode == kDxNone) ? (size_t)c.input_node_size * (size_t)(c.rev_stride - 1) * (kTermHead + (indexed ? NN : NN / 2)) : 0;
+    size_t const term_count = (dxmode == kDxNone) ? (size_t)c.input_node_size * (size_t)(c.rev_stride - 1) * (kTermHead + NN / 2) : 0;
     size_t const dtab_bytes = align256(term_count * sizeof(int));
     size_t const dyh_bytes  = (dxmode == kDxNone && c.bn) ? align256((size_t)c.output_node_size * c.frame_stride * sizeof(float)) : 0;
     size_t const v_bytes = corner ? c_bytes : 0;
-    size_t const bits_bytes = (pack && !have_bits) ? align256((size_t)c.input_node_size * c.x_stride * sizeof(uint32_t)) : 0;
     char *base = nullptr;
-    if (arena_get(c_bytes + part_bytes + stat_bytes + dtab_bytes + dyh_bytes + v_bytes + bits_bytes + own_bytes, &base, st)) { return 1; }
-    uint32_t *own = indexed ? reinterpret_cast<uint32_t *>(base + c_bytes + part_bytes + stat_bytes + dtab_bytes + dyh_bytes + v_bytes + bits_bytes) : nullptr;
+    if (arena_get(c_bytes + part_bytes + stat_bytes + dtab_bytes + dyh_bytes + v_bytes, &base, st)) { return 1; }
     float *V    = corner ? reinterpret_cast<float *>(base + c_bytes + part_bytes + stat_bytes + dtab_bytes + dyh_bytes) : nullptr;
     float *C    = reinterpret_cast<float *>(base);
     float *part = reinterpret_cast<float *>(base + c_bytes);
@@ -745,56 +834,25 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         V = corner ? reinterpret_cast<float *>(reinterpret_cast<char *>(tables.buf) + c_bytes) : nullptr;
     }
     bool const prep = (c.bn || dxmode != kDxNone) && !have_tables;
-    if (have_bits) {
-        c.x = packed.bits;
-        if (prep) {
-            launch_table_prep<N>(c.W, C, c.output_node_size, c.lut_binarize, st, V, c.bias);
-            BBHIP_LAUNCH_CHECK();
-        }
-    }
-    else if (pack) {
-        uint32_t *bits = reinterpret_cast<uint32_t *>(base + c_bytes + part_bytes + stat_bytes + dtab_bytes + dyh_bytes + v_bytes);
-        float const *src = reinterpret_cast<float const *>(call.x);
-        if (prep) {
-            if (launch_pack_and_prep<N>(src, call.x_stride, bits, c.x_stride, c.input_node_size, c.frame_size,
-                                        c.W, C, V, c.output_node_size, c.lut_binarize, c.bias, st)) { return 1; }
-        }
-        else if (launch_binarize_pack(src, call.x_stride, bits, c.x_stride, c.input_node_size, c.frame_size, st)) { return 1; }
-        c.x = bits;
-    }
-    else if (prep) {
+    if (prep) {
         launch_table_prep<N>(c.W, C, c.output_node_size, c.lut_binarize, st, V, c.bias);
         BBHIP_LAUNCH_CHECK();
     }
     // the term table of the dx kernel is built by extra workgroups at the end of the table-gradient launch
     TermArgs tt{};
     if (dxmode == kDxNone && term_count > 0) {
-        size_t const records = (size_t)c.input_node_size * (size_t)(c.rev_stride - 1);
-        size_t const per_block = (size_t)kWavesPerBlk * kTermRecordsPerWave;
-        size_t const blocks = (((records + per_block - 1) / per_block) + 7) & ~(size_t)7;            // whole rounds over the XCDs
-        if (records > 0x7fffffffULL || blocks + (size_t)slab_total * tile_count > 0x7fffffffULL) { return fail("backward: grid too large"); }
-        tt.fan = make_tile_divisor(c.rev_stride - 1);
+        int const blocks = (ceil_div(c.output_node_size, kWavesPerBlk) + 7) & ~7;                    // whole rounds over the XCDs
+        if ((long long)blocks + (long long)slab_total * tile_count > 0x7fffffffLL) { return fail("backward: grid too large"); }
+        tt.fan_slots = c.rev_stride - 1;
         tt.W = c.W; tt.idx = c.idx; tt.rev = c.rev; tt.term = term;
         tt.x_base = (unsigned long long)(uintptr_t)c.x; tt.x_row_pitch_bytes = (unsigned long long)c.x_stride * 4ULL;
         tt.dy_base = (unsigned long long)(uintptr_t)(c.bn ? (void const *)dyh : (void const *)c.dy);
         tt.dy_row_pitch_bytes = (unsigned long long)c.frame_stride * 4ULL;
-        tt.lut_binarize = c.lut_binarize; tt.rev_stride = c.rev_stride; tt.input_node_size = c.input_node_size;
-        tt.blocks = (int)blocks;
-        tt.corner = use_corner_values(c.xmode) ? 1 : 0;
-        tt.lo = 0.5f - c.bias; tt.hi = 0.5f + c.bias;
-        // node by node: coefficient records always, value records where the nodes' corner values are at hand (batch-norm backward)
-        if (term_from_corner_values() && (corner || tt.corner == 0)) {
-            tt.V = corner ? V : nullptr; tt.node_size = c.output_node_size;
-            tt.blocks = (ceil_div(c.output_node_size, kWavesPerBlk) + 7) & ~7;
-            if (indexed) {      // ... and point at the rows of kept corner indices instead of the input rows
-                tt.indexed = 1;
-                tt.x_base = (unsigned long long)(uintptr_t)own; tt.x_row_pitch_bytes = (unsigned long long)own_words * 4ULL;
-            }
-        }
+        tt.lut_binarize = c.lut_binarize; tt.rev_stride = c.rev_stride; tt.node_size = c.output_node_size; tt.blocks = blocks;
     }
 
     BwdArgs a{};
-    a.x = c.x; a.dy = c.dy; a.idx = c.idx; a.C = C; a.V = V;
+    a.x = c.x; a.dy = c.dy; a.idx = c.idx; a.C = C;
     a.dw_partial = part;
     a.mean = c.mean; a.rstd = c.rstd; a.dmean = c.dmean_tmp; a.dvar = c.dvar_tmp;
     a.node_size = c.output_node_size; a.frame_size = c.frame_size;
@@ -814,7 +872,6 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         f.node_size = c.output_node_size; f.frame_size = c.frame_size; f.x_stride = c.x_stride;
         f.chunk = stat_chunk; f.chunk_count = stat_chunk_count; f.tiles = make_tile_divisor(stat_tiles);
         f.bias = c.bias; f.gamma = c.gamma; f.beta = c.beta;
-        if (indexed) { f.own_index_out = own; f.own_stride = own_words; }
         if (dispatch_forward<N>(c.xmode, kYClamp, 3, f, npw, st)) { return 1; }
         BBHIP_LAUNCH_CHECK();
         if (stat_chunk_count <= kInlineStatUnits) {
@@ -859,22 +916,8 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
     }
 
     if (dxmode == kDxNone) {
-        bool const bit_corner = (c.xmode == kXBit) && use_corner_values(c.xmode);
-        int const steps  = dx_pass_steps_env() ? dx_pass_steps_env() : (bit_corner ? 4 : 2);        // wavefront-steps per pass: {1, 2, 4}
-        // Packed rows with up to about a thousand input nodes (the layers of a convolution: tens to hundreds of channels x taps, very
-        // many frames): the words of a pass are read with one scalar load per row — the rows then stay in the scalar cache.  With
-        // more rows they do not, and the vector loads are faster (dx kernel at 324 / 512 / 1024 / 2048 rows: 94 / 107 / 138 / 141 us
-        // against 104 / 127 / 147 / 135 us; 4096 rows: 385 against 319 us per step).
-        bool const wide = bit_corner && dx_wide_rows() && steps == 4 && c.input_node_size <= dx_wide_max_rows() && c.x_stride % 8 == 0 &&
-                          (reinterpret_cast<uintptr_t>(c.x) % 32u) == 0;
-        int frames = dx_chunk_frames_env() ? dx_chunk_frames_env() : (bit_corner ? 256 : 128);
-        if (wide && dx_chunk_frames_env() == 0) {
-            // ... and such layers have few wavefronts' worth of input nodes and many frames: units of 1024 frames, so that a
-            // wavefront's set-up (its list, its share of it) serves four passes, halved while the launch would fall short of workgroups
-            // (conv block 0.602 -> 0.590 ms; the same units for a 4096-row layer: 0.338 -> 0.358 ms, hence only here)
-            frames = 1024;
-            while (frames > 256 && (long long)ceil_div(c.frame_size, frames) * ceil_div(c.input_node_size, kWavesPerBlk) < 2048) { frames /= 2; }
-        }
+        int const steps  = dx_pass_steps_env() ? dx_pass_steps_env() : 2;                             // wavefront-steps per pass: {1, 2, 4}
+        int const frames = dx_chunk_frames_env() ? dx_chunk_frames_env() : 128;
         int const chunk  = ((frames + kWave * steps - 1) / (kWave * steps)) * (kWave * steps);
         int const chunk_count = ceil_div(c.frame_size, chunk);
         // few input nodes with long work lists: the four wavefronts of a workgroup share one input node (DxArgs::split)
@@ -892,18 +935,9 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         d.fin_overwrite = dw_overwrite;
         d.fin_blocks = (ceil_div(c.output_node_size * NN, kBlock) + 7) & ~7;
         if ((long long)d.fin_blocks + (long long)chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
-        d.own_stride = own_words;
         {
             ScopedTimer tm(kTimeDx, st);
-            if (indexed) {
-                dim3 const grid(d.fin_blocks + d.chunk_count * d.tiles.count), block(kBlock);
-                hipLaunchKernelGGL((lut_dx_indexed_kernel<N>), grid, block, 0, st, d);
-            }
-            else if (wide) {
-                dim3 const grid(d.fin_blocks + d.chunk_count * d.tiles.count), block(kBlock);
-                hipLaunchKernelGGL((lut_dx_corner_kernel<N, kXBit, 4, true>), grid, block, 0, st, d);
-            }
-            else if (dispatch_dx<N>(c.xmode, steps, d, st)) { return 1; }
+            if (dispatch_dx<N>(c.xmode, steps, d, st)) { return 1; }
         }
         BBHIP_LAUNCH_CHECK();
         return 0;
@@ -1174,7 +1208,6 @@ int bbhip_GetSwitch(char const *name)
     if (!name) { return -1; }
     if (!strcmp(name, "corner")) { return use_corner_values(kXBit) ? 1 : 0; }
     if (!strcmp(name, "pack"))   { return pack_binarized_input() ? 1 : 0; }
-    if (!strcmp(name, "dx_wide")) { return dx_wide_rows() ? 1 : 0; }
     if (!strcmp(name, "inline_tables")) { return inline_tables() ? 1 : 0; }
     return -1;
 }

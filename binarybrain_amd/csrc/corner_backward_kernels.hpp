@@ -1,0 +1,458 @@
+// Backward pass of the LUT layers on two-valued inputs (packed bits; fp32 frames binarized at 0.5 are packed first).
+//
+// Over two-valued inputs a node's frames fall into 2^N corners, and everything that the backward pass needs of them is, per corner,
+//     D[p] = the sum of dy over the frames at corner p,     n[p] = the number of those frames.
+// With batch-norm, dL/d(LUT output) of a frame at corner p is  open[p] gamma rstd dy + dmean + V[p] dvar / F  (reference:
+// DifferentiableLutN.h:1206-1250), where open[p] says whether the batch-norm output of the corner lies inside the hard-tanh window, so
+//     sum of g              = sum_p open[p] D[p],           sum of g (v - mean) = sum_p open[p] D[p] (V[p] - mean),
+//     gradient at corner p  G[p] = open[p] gamma rstd D[p] + n[p] (dmean + V[p] dvar / F),
+//     dW[i]                 = sum_p G[p] prod_j (bit_j(i) ? x_j(p) : 1 - x_j(p)).
+// One pass over the inputs and dy gives D and n (lut_corner_sums_kernel), the rest is arithmetic on 2^N values per node (corner_fold): no
+// statistics pass of its own, no polynomial, no 2^N multiply-adds per frame, and no row of dL/d(LUT output) is written.  The dx kernel
+// (lut_dx_table_kernel) applies the same two terms per corner:  dx = sum over consumers of  A[p] dy + B[p].
+#pragma once
+
+#include "lut_kernels.hpp"
+
+namespace bbhip {
+
+struct CornerFoldArgs {
+    float const *mean, *rstd;           // batch-norm
+    float gamma, beta, inv_frames;
+    int   frame_size;
+    float lo, hi;                       // the two input values, 1/2 -+ bias
+    float *dW;
+    int   overwrite;                    // dW = instead of dW +=
+    float4 *node_consts;                // batch-norm: mean, rstd, dmean, dvar / F of each node, for the dx kernel
+};
+
+// Lane p (of every group of 2^N lanes) holds the node's V[p], D[p], n[p]: the node's table gradient and, with batch-norm, its constants
+template <int N, bool BN>
+__device__ __forceinline__ void corner_fold(CornerFoldArgs const &a, int node, int lane, float v, float D, float n)
+{
+    constexpr int NN = 1 << N;
+    float G = D;
+    if (BN) {
+        float const mean = a.mean[node], rstd = a.rstd[node];
+        float const t = batch_norm_output(v, mean, rstd, a.gamma, a.beta);
+        float const g = (t <= 0.0f || t >= 1.0f) ? 0.0f : D;
+        float const counted = (lane < NN) ? g : 0.0f;                   // narrow tables repeat over the wavefront
+        float const s0 = wave_sum(counted), s1 = wave_sum(counted * (v - mean));
+        float dmean, dvar;
+        batch_gradient_statistics(s0, s1, mean, rstd, a.gamma, a.frame_size, dmean, dvar);
+        dvar *= a.inv_frames;
+        G = __builtin_fmaf(g, a.gamma * rstd, n * __builtin_fmaf(v, dvar, dmean));
+        if (lane == 0) { a.node_consts[node] = make_float4(mean, rstd, dmean, dvar); }
+    }
+    // per input: (G0, G1) -> ((1 - lo) G0 + (1 - hi) G1, lo G0 + hi G1), and 1 - lo = hi: either lane keeps hi of its own and takes lo of the other's
+#pragma unroll
+    for (int j = 0; j < N; ++j) { G = __builtin_fmaf(a.hi, G, a.lo * __shfl_xor(G, 1 << j, 64)); }
+    if (lane < NN) {
+        float *out = a.dW + (size_t)node * NN + lane;
+        *out = a.overwrite ? G : *out + G;
+    }
+}
+
+struct CornerSumsArgs {
+    uint32_t const *x;
+    float const *dy;
+    int const   *idx;
+    float const *V;             // [O][2^N] corner values, or null:
+    float const *W_inline;      // the wavefront derives them from the table; the wavefront of a node's first slab stores them to V_out
+    float       *V_out;
+    int   lut_binarize;
+    float bias;
+    int   node_size, frame_size, x_stride, dy_stride;
+    int   slab, slab_count;     // frames per unit, a multiple of 256
+    TileDivisor tiles;
+    int   dy_quads;             // rows of dy hold whole groups of four frames: one 16-byte load per lane and pass
+    uint32_t *own;              // the corner index of every (node, frame), a byte each in frame order, for the dx kernel: rows of own_stride words
+    int   own_stride;
+    float *partial;             // several slabs: [slab][O][BN ? 2 : 1][2^N], D and then n
+    CornerFoldArgs fold;        // one slab: the wavefront folds its sums itself
+};
+
+// Words of N inputs (32 frames) -> the 32 corner indices, a byte each in frame order: quad[i] holds the frames 4 i .. 4 i + 3.
+// Eight rows of four bytes are transposed bit by bit (rows a power of two apart exchange bit fields: three rounds), which leaves frame
+// 8 c + j in byte c of row j, then byte by byte: about two instructions per frame and lane where building an index bit by bit takes N.
+template <int N>
+__device__ __forceinline__ void corner_bytes(uint32_t const (&w)[N], uint32_t (&quad)[8])
+{
+    uint32_t r[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) { r[k] = (k < N) ? w[k < N ? k : 0] : 0u; }
+    auto exchange = [&](int i, int j, int s, uint32_t low) {
+        uint32_t const a = r[i], b = r[j];
+        r[i] = (a & low) | ((b << s) & ~low);
+        r[j] = ((a >> s) & low) | (b & ~low);
+    };
+#pragma unroll
+    for (int k = 0; k < 4; ++k) { exchange(k, k + 4, 4, 0x0f0f0f0fu); }
+#pragma unroll
+    for (int k = 0; k < 8; k += 4) { exchange(k, k + 2, 2, 0x33333333u); exchange(k + 1, k + 3, 2, 0x33333333u); }
+#pragma unroll
+    for (int k = 0; k < 8; k += 2) { exchange(k, k + 1, 1, 0x55555555u); }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {           // rows 4 h .. 4 h + 3: byte c of row j -> byte j of quad 2 c + h
+        uint32_t const *q = r + 4 * h;
+        uint32_t const p0 = __builtin_amdgcn_perm(q[1], q[0], 0x05010400u), p1 = __builtin_amdgcn_perm(q[3], q[2], 0x05010400u);      // bytes 0, 1 of row pairs
+        uint32_t const p2 = __builtin_amdgcn_perm(q[1], q[0], 0x07030602u), p3 = __builtin_amdgcn_perm(q[3], q[2], 0x07030602u);      // bytes 2, 3
+        quad[0 + h] = __builtin_amdgcn_perm(p1, p0, 0x05040100u);
+        quad[2 + h] = __builtin_amdgcn_perm(p1, p0, 0x07060302u);
+        quad[4 + h] = __builtin_amdgcn_perm(p3, p2, 0x05040100u);
+        quad[6 + h] = __builtin_amdgcn_perm(p3, p2, 0x07060302u);
+    }
+}
+
+__device__ __forceinline__ void wave_fence(void)
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// four consecutive frames of a row from byte offset off; quads: the row holds whole groups of four
+__device__ __forceinline__ float4 load_quad(__amdgpu_buffer_rsrc_t r, uint32_t off, bool quads)
+{
+    if (quads) {
+        auto const q = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+        return make_float4(__uint_as_float(q[0]), __uint_as_float(q[1]), __uint_as_float(q[2]), __uint_as_float(q[3]));
+    }
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { v[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off + 4 * j, 0, 0)); }
+    return make_float4(v[0], v[1], v[2], v[3]);
+}
+
+// valid bytes of a row for load_quad: whole groups of four where the row holds them (frames past the last read 0 or the row's padding)
+__device__ __forceinline__ uint32_t quad_row_bytes(int frame_size, bool quads)
+{
+    return (uint32_t)(quads ? (frame_size + 3) & ~3 : frame_size) * 4u;
+}
+
+// sums over the 64 columns of row (lane mod ROWS) of a wavefront's [ROWS][64] block in LDS.  A lane takes four columns at a time, in an order
+// of its own, so that the lanes that are served together read different banks; with fewer than 64 rows several lanes share one.
+template <int ROWS, typename V4>
+__device__ __forceinline__ auto row_sum(V4 const *block, int lane)
+{
+    int const p = lane & (ROWS - 1), part = lane / ROWS;
+    decltype(block[0].x + block[0].x) s = 0;
+#pragma unroll
+    for (int g = 0; g < ROWS / 4; ++g) {
+        V4 const q = block[p * (kWave / 4) + part * (ROWS / 4) + (g ^ (p & (ROWS / 4 - 1)))];
+        s += (q.x + q.y) + (q.z + q.w);
+    }
+#pragma unroll
+    for (int o = ROWS; o < kWave; o <<= 1) { s += __shfl_xor(s, o, 64); }
+    return s;
+}
+
+// One wavefront = one node x one slab of frames, in blocks of 2048 frames.  A lane loads the words of 32 frames of each input and turns them
+// into corner indices (corner_bytes), which go to memory for the dx kernel and through LDS to the lanes that hold the frames' dy: a pass is 256
+// frames, four consecutive ones per lane.  Each lane keeps bins of its own in LDS ([corner][lane]: no two lanes share an address, and the 64 lanes
+// of a step always touch 64 different banks) and adds its dy by a plain read-add-write: 12 clocks per step of 64 frames and CU, where the 64
+// multiply-adds of a polynomial form take 64 vector instructions per step and an LDS float atomic (ds_add_f32) 193 clocks.  n: a lane counts,
+// for each set of inputs, the frames of its words where all of them are set (2 instructions per set and 32 frames); the lanes' counts
+// are added at the end and differences over the sets give the corners' counts.
+// The bins leave two workgroups per compute unit: dy is requested four passes ahead and the words a block ahead, as vector loads
+// (scalar loads would be waited for with the LDS accesses: 101 us for the first shape below).
+// Measured against the statistics and table-gradient launches that it replaces: 216 nodes x 230400 frames 65 us (3.8 TB/s of dy and indices)
+// instead of 53 + 141; 4096 x 8192 42 us instead of 31 + 106; 6144 x 1024 20 us instead of 11 + 30.
+template <int N, bool BN>
+__global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs a)
+{
+    constexpr int NN = 1 << N, kPasses = 8, kAhead = 4;
+    __shared__ __align__(16) float bins[kWavesPerBlk][NN * kWave];
+    __shared__ __align__(16) uint32_t quads[kWavesPerBlk][kPasses * kWave];
+    int const B   = a.slab_count * a.tiles.count;
+    int const lid = xcd_remap(blockIdx.x, B);
+    int sl, tile;
+    split_tile(lid, a.tiles, sl, tile);
+    int const wv   = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    int const node = tile * kWavesPerBlk + wv;
+    if (node >= a.node_size) { return; }
+    int const lane = threadIdx.x & (kWave - 1);
+
+    int const f_begin = sl * a.slab;
+    int const f_end   = min(f_begin + a.slab, a.frame_size);
+    bool const quad_rows = a.dy_quads != 0;
+    __amdgpu_buffer_rsrc_t const dyr = row_descriptor(a.dy, node, a.dy_stride, quad_row_bytes(a.frame_size, quad_rows));
+    uint32_t const x_row_bytes = (uint32_t)((a.frame_size + 31) >> 5) * 4u;
+    __amdgpu_buffer_rsrc_t xr[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) { xr[k] = row_descriptor(a.x, a.idx[node * N + k], a.x_stride, x_row_bytes); }
+
+    uint32_t w_next[N];
+    auto request_words = [&](int base) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) { w_next[k] = __builtin_amdgcn_raw_buffer_load_b32(xr[k], (uint32_t)((base >> 5) + lane) * 4u, 0, 0); }
+    };
+    float4 dy[kAhead];
+    request_words(f_begin);
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) { dy[i] = load_quad(dyr, (uint32_t)(f_begin + i * 4 * kWave + 4 * lane) * 4u, quad_rows); }
+
+    float v;                                                            // lane p: V[p]
+    if (a.V != nullptr) { v = a.V[(size_t)node * NN + (lane & (NN - 1))]; }
+    else {
+        int const i = lane & (NN - 1);
+        float w = a.W_inline[(size_t)node * NN + i];
+        if (a.lut_binarize) { w = (w > 0.5f) ? 1.0f : 0.0f; }
+        v = corner_butterfly<N>(centred_butterfly<N>(w, i), i, a.bias);
+    }
+
+    float *const mine = bins[wv];
+#pragma unroll
+    for (int i = 0; i < NN / 4; ++i) { *reinterpret_cast<float4 *>(mine + (i * kWave + lane) * 4) = make_float4(0.0f, 0.0f, 0.0f, 0.0f); }
+    wave_fence();
+
+    uint32_t count[BN ? NN : 1];                                        // [S]: frames of the lane's words where every input of S is set
+#pragma unroll
+    for (int i = 0; i < (BN ? NN : 1); ++i) { count[i] = 0; }
+
+    for (int base = f_begin; base < f_end; base += kPasses * 4 * kWave) {
+        uint32_t quad[8];
+        {
+            uint32_t w[N];
+#pragma unroll
+            for (int k = 0; k < N; ++k) { w[k] = w_next[k]; }
+            request_words(base + kPasses * 4 * kWave);                  // (past the row: zeros)
+            corner_bytes<N>(w, quad);
+            int const live = f_end - (base + 32 * lane);                // frames of the lane's words that belong to the slab
+            if (live > 0) {
+                uint4 *out = reinterpret_cast<uint4 *>(a.own + (size_t)node * a.own_stride + ((base >> 2) + 8 * lane));
+                out[0] = make_uint4(quad[0], quad[1], quad[2], quad[3]);
+                out[1] = make_uint4(quad[4], quad[5], quad[6], quad[7]);
+            }
+            uint4 *ex = reinterpret_cast<uint4 *>(quads[wv] + 8 * lane);
+            ex[0] = make_uint4(quad[0], quad[1], quad[2], quad[3]);
+            ex[1] = make_uint4(quad[4], quad[5], quad[6], quad[7]);
+            if constexpr (BN) {
+                uint32_t all[NN];
+                all[0] = (live >= 32) ? 0xffffffffu : (live <= 0) ? 0u : ((1u << live) - 1u);
+                count[0] += __popc(all[0]);
+#pragma unroll
+                for (int s = 1; s < NN; ++s) {
+                    all[s] = all[s & (s - 1)] & w[__builtin_ctz(s)];
+                    count[s] += __popc(all[s]);
+                }
+            }
+        }
+        wave_fence();
+        uint32_t at[kPasses];
+#pragma unroll
+        for (int i = 0; i < kPasses; ++i) { at[i] = quads[wv][i * kWave + lane]; }
+#pragma unroll
+        for (int i = 0; i < kPasses; ++i) {
+            int const fb = base + i * 4 * kWave;
+            if (fb >= f_end) { break; }                                 // wave-uniform
+            float4 d = dy[i % kAhead];
+            dy[i % kAhead] = load_quad(dyr, (uint32_t)(fb + kAhead * 4 * kWave + 4 * lane) * 4u, quad_rows);
+            if (fb + 4 * kWave > a.frame_size) {                        // the row's padding may hold anything
+                int const f = fb + 4 * lane;
+                if (f     >= a.frame_size) { d.x = 0.0f; }
+                if (f + 1 >= a.frame_size) { d.y = 0.0f; }
+                if (f + 2 >= a.frame_size) { d.z = 0.0f; }
+                if (f + 3 >= a.frame_size) { d.w = 0.0f; }
+            }
+            mine[(at[i] & 0xffu) * kWave + lane] += d.x;
+            mine[((at[i] >> 8) & 0xffu) * kWave + lane] += d.y;
+            mine[((at[i] >> 16) & 0xffu) * kWave + lane] += d.z;
+            mine[(at[i] >> 24) * kWave + lane] += d.w;
+        }
+        wave_fence();
+    }
+
+    float const D = row_sum<NN>(reinterpret_cast<float4 const *>(mine), lane);
+    uint32_t n = 0;
+    if constexpr (BN) {
+        wave_fence();
+        uint32_t *const cells = reinterpret_cast<uint32_t *>(mine);
+#pragma unroll
+        for (int s = 0; s < NN; ++s) { cells[s * kWave + lane] = count[s]; }
+        wave_fence();
+        n = row_sum<NN>(reinterpret_cast<uint4 const *>(cells), lane);  // lane S: frames where every input of S is set (the others either way)
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            uint32_t const o = __shfl_xor(n, 1 << k, 64);
+            if (!((lane >> k) & 1)) { n -= o; }                         // ... minus those where input k is set too
+        }
+    }
+
+    if (a.slab_count == 1) { corner_fold<N, BN>(a.fold, node, lane, v, D, (float)n); }
+    else if (lane < NN) {
+        float *out = a.partial + ((size_t)sl * a.node_size + node) * (BN ? 2 * NN : NN) + lane;
+        out[0] = D;
+        if (BN) { out[NN] = (float)n; }
+    }
+    if (a.V_out != nullptr && sl == 0 && lane < NN) { a.V_out[(size_t)node * NN + lane] = v; }
+}
+
+// Several slabs per node: a workgroup per node adds them up, each wavefront every fourth slab, and folds.
+template <int N, bool BN>
+__global__ __launch_bounds__(kBlock) void lut_corner_fold_kernel(CornerFoldArgs a, float const *__restrict__ partial, float const *__restrict__ V,
+                                                                 int node_size, int slab_count)
+{
+    constexpr int NN = 1 << N, REC = BN ? 2 * NN : NN;
+    __shared__ float red[2][kWavesPerBlk][kWave];
+    int const node = blockIdx.x;
+    int const wv = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+    float const *in = partial + (size_t)node * REC + (lane & (NN - 1));
+    float D = 0.0f, n = 0.0f;
+#pragma unroll 4
+    for (int s = wv; s < slab_count; s += kWavesPerBlk) {
+        float const *q = in + (size_t)s * node_size * REC;
+        D += q[0];
+        if (BN) { n += q[NN]; }
+    }
+    red[0][wv][lane] = D;
+    red[1][wv][lane] = n;
+    __syncthreads();
+    if (wv != 0) { return; }
+#pragma unroll
+    for (int w = 1; w < kWavesPerBlk; ++w) { D += red[0][w][lane]; n += red[1][w][lane]; }
+    corner_fold<N, BN>(a, node, lane, V[(size_t)node * NN + (lane & (NN - 1))], D, n);
+}
+
+struct DxTableArgs {
+    DxArgs dx;                          // units, work lists, split mode and rows as in lut_dx_kernel (no term table, no rider)
+    uint32_t const *own;                // kept corner indices, a byte per frame, rows of own_stride words
+    int   own_stride;
+    int   dy_quads, dx_quads;           // rows hold whole groups of four frames (dx: 16-byte aligned as well)
+    float const *V;                     // [O][2^N]
+    float4 const *node_consts;          // batch-norm: mean, rstd, dmean, dvar / F
+    float gamma, beta, inv_step;        // inv_step = 1 / (hi - lo)
+};
+
+// Input-centric dx over kept corner indices.  One wavefront owns dx[input][256 Q frames], four consecutive frames per lane and quad, and walks the
+// input's consumers in the reverse table's order (split mode: a quarter of them).  A consumer's term of a frame at corner p is  A[p] dy + B[p]  with
+//     A[p] = dV/dx_k[p] open[p] gamma rstd,   B[p] = dV/dx_k[p] (dmean + V[p] dvar / F)           (plain layers: A = dV/dx_k, B = 0),
+// and y is linear in input k, so dV/dx_k[p] = (V[k at hi] - V[k at lo]) / (hi - lo): lane p computes entry p from the node's 2^N corner values
+// and four constants (272 bytes per node that all its consumers share), the wavefront puts the table into LDS, and the frames fetch their
+// entry from there: a random 8-byte LDS read takes 4.5 clocks per CU and step where two ds_bpermute take 14.  Per term and pass one vector load
+// of V, Q of indices and Q of dy; the next term's are in flight while a term is evaluated.
+// Measured against the kernel that formed the indices from the packed rows: 27 inputs x 216 nodes x 230400 frames (Q = 2) 90 us instead of 117,
+// 4096 x 4096 x 8192 (Q = 1; 2: 142, 4: 162) 117 us instead of 138, where an XCD's L2 just holds what the chunk's passes gather from.
+template <int N, bool BN, int Q>
+__global__ __launch_bounds__(kBlock) void lut_dx_table_kernel(DxTableArgs t)
+{
+    constexpr int NN = 1 << N, kPass = 4 * kWave * Q;
+    using Entry = std::conditional_t<BN, float2, float>;
+    DxArgs const &a = t.dx;
+    int const lid = xcd_remap(blockIdx.x, a.chunk_count * a.tiles.count);
+    int ck, tile;
+    split_tile(lid, a.tiles, ck, tile);
+    __shared__ __align__(16) float4 part[kWavesPerBlk][Q][kWave];
+    __shared__ Entry table[kWavesPerBlk][2][NN];
+    int const wave = threadIdx.x / kWave;
+    int in, share;
+    dx_list_share(a, tile, wave, in, share);
+    if (in >= a.input_node_size) { return; }                            // (workgroup-uniform in split mode)
+    int const lane = threadIdx.x & (kWave - 1);
+
+    typedef __attribute__((address_space(4))) int const const_int;
+    typedef __attribute__((address_space(4))) float const const_float;
+    const_int *list = (const_int *)(a.rev + (size_t)in * a.rev_stride);
+    int t_begin, t_end;
+    dx_list_range(list[0], share, t_begin, t_end);
+    list += 1;
+    bool const dy_quads = t.dy_quads != 0;
+    uint32_t const y_row_bytes = quad_row_bytes(a.frame_size, dy_quads), i_row_bytes = (uint32_t)t.own_stride * 4u;
+    int const f_begin = ck * kPass, f_lane = f_begin + 4 * lane;
+
+    float4 acc[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) { acc[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f); }
+
+    uint32_t iw_next[Q];
+    float4 dy_next[Q];
+    float v_next = 0.0f, c_next[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    int k_next = 0, e_ahead = 0;
+    auto request = [&](int e) {
+        int const node = (int)((uint32_t)e / (uint32_t)N);
+        k_next = e - node * N;
+        __amdgpu_buffer_rsrc_t const ir  = row_descriptor(t.own, node, t.own_stride, i_row_bytes);
+        __amdgpu_buffer_rsrc_t const dyr = row_descriptor(a.dy, node, a.dy_stride, y_row_bytes);
+        v_next = t.V[(size_t)node * NN + (lane & (NN - 1))];
+        if (BN) {
+            const_float *c = (const_float *)(t.node_consts + node);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { c_next[i] = c[i]; }
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) { iw_next[q] = __builtin_amdgcn_raw_buffer_load_b32(ir, (uint32_t)(f_lane + q * 4 * kWave), 0, 0); }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) { dy_next[q] = load_quad(dyr, (uint32_t)(f_lane + q * 4 * kWave) * 4u, dy_quads); }
+    };
+    if (t_begin < t_end) {
+        request(list[t_begin]);
+        if (t_begin + 1 < t_end) { e_ahead = list[t_begin + 1]; }
+    }
+    for (int i = t_begin; i < t_end; ++i) {
+        uint32_t iw[Q];
+        float4 dy[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) { iw[q] = iw_next[q]; dy[q] = dy_next[q]; }
+        float const v = v_next, mean = c_next[0], rstd = c_next[1], dmean = c_next[2], dvar = c_next[3];
+        int const k = k_next;
+        if (i + 1 < t_end) {
+            request(e_ahead);
+            if (i + 2 < t_end) { e_ahead = list[i + 2]; }
+        }
+        float const other = __shfl_xor(v, 1 << k, 64);
+        float const slope = (((lane >> k) & 1) ? (v - other) : (other - v)) * t.inv_step;
+        Entry *const tab = table[wave][i & 1];
+        if constexpr (BN) {
+            float const y = batch_norm_output(v, mean, rstd, t.gamma, t.beta);
+            float const A = (y <= 0.0f || y >= 1.0f) ? 0.0f : slope * (t.gamma * rstd);
+            if (lane < NN) { tab[lane] = make_float2(A, slope * __builtin_fmaf(v, dvar, dmean)); }
+        }
+        else { if (lane < NN) { tab[lane] = slope; } }
+        wave_fence();
+        auto add = [&](float &sum, float d, uint32_t corner) {
+            Entry const e = tab[corner];
+            if constexpr (BN) { sum = __builtin_fmaf(d, e.x, sum + e.y); }
+            else              { sum = __builtin_fmaf(d, e, sum); }
+        };
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            add(acc[q].x, dy[q].x, iw[q] & 0xffu);
+            add(acc[q].y, dy[q].y, (iw[q] >> 8) & 0xffu);
+            add(acc[q].z, dy[q].z, (iw[q] >> 16) & 0xffu);
+            add(acc[q].w, dy[q].w, iw[q] >> 24);
+        }
+    }
+
+    if (a.split) {                              // the shares of the list, added in wavefront order (dx_store_pass)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) { part[wave][q][lane] = acc[q]; }
+        __syncthreads();
+        if (wave != 0) { return; }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+#pragma unroll
+            for (int w = 1; w < kWavesPerBlk; ++w) {
+                float4 const o = part[w][q][lane];
+                acc[q].x += o.x; acc[q].y += o.y; acc[q].z += o.z; acc[q].w += o.w;
+            }
+        }
+    }
+    float *const row = a.dx + (size_t)in * a.dx_stride;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        int const f = f_lane + q * 4 * kWave;
+        if (t.dx_quads && f + 3 < a.frame_size) {
+            typedef float f32x4 __attribute__((ext_vector_type(4)));
+            f32x4 const o = {acc[q].x, acc[q].y, acc[q].z, acc[q].w};
+            __builtin_nontemporal_store(o, reinterpret_cast<f32x4 *>(row + f));
+        }
+        else {
+            if (f     < a.frame_size) { row[f]     = acc[q].x; }
+            if (f + 1 < a.frame_size) { row[f + 1] = acc[q].y; }
+            if (f + 2 < a.frame_size) { row[f + 2] = acc[q].z; }
+            if (f + 3 < a.frame_size) { row[f + 3] = acc[q].w; }
+        }
+    }
+}
+
+}  // namespace bbhip

@@ -236,7 +236,6 @@ struct FwdArgs {
     // row of own_stride words holds frames f + l, f + 64 + l, f + 128 + l, f + 192 + l.  The output launch of the same call
     // (own_index: the same buffer) then reads a word per lane and four steps instead of gathering the fp32 frames a second time.
     // Units of both launches begin at multiples of 256 frames.  Needs no count of the input's rows.
-    // The statistics pass of a backward call (kind 3, passes of four steps) keeps them the same way for lut_dx_indexed_kernel.
     uint32_t       *own_index_out;
     uint32_t const *own_index;
     int   own_stride;
@@ -691,9 +690,9 @@ __device__ __forceinline__ void corner_unit_pass(FwdArgs const &a, void const *(
                                                  int f_begin, int f_end, int f_last, float &s1, float &s2)
 {
     constexpr int U = (XMODE == kXBit && !WIDE && OWN == kOwnNone) ? 2 : 4;
-    // passes of four steps leave their corner indices in `own`: the statistics kinds keep them where the call asks for it
-    // (kind 2 over fp32 frames: for the output launch; kind 3: for the dx kernel of the same backward call, lut_dx_indexed_kernel)
-    constexpr bool kKeepIndex = (U == 4) && (OWN == kOwnNone) && ((XMODE == kXBinary && KIND == 2) || KIND == 3);
+    // passes of four steps leave their corner indices in `own`: the statistics kind over fp32 frames keeps them for the output launch
+    // where the call asks for it
+    constexpr bool kKeepIndex = (U == 4) && (OWN == kOwnNone) && XMODE == kXBinary && KIND == 2;
     for (int fb = f_begin; fb < f_end; fb += kWave * U) {
         uint32_t own;
         corner_pass_any<N, XMODE, YMODE, KIND, WIDE, OWN>(a, rows, tabs, node, lane, fb, f_end, f_last, s1, s2, own);
@@ -888,19 +887,10 @@ struct TermArgs {
     int const   *rev;           // reverse table [I][rev_stride]
     int         *term;          // the records
     unsigned long long x_base, x_row_pitch_bytes, dy_base, dy_row_pitch_bytes;
-    int lut_binarize, rev_stride, input_node_size;
-    TileDivisor fan;            // division by the slots per input, rev_stride - 1
-    int blocks;                 // workgroups that build records (kWavesPerBlk * kTermRecordsPerWave records each); 0 = nothing to build
-    int corner;                 // 1: records hold the derivative's corner values for two-valued inputs (lut_dx_corner_kernel)
-    float lo, hi;               //    the two input values, 1/2 -+ bias
-    // node_size > 0: the records are built node by node (term_table_node_block: `blocks` then counts workgroups of kWavesPerBlk nodes) —
-    // coefficient records (corner = 0) from W, value records from the nodes' corner values V, which the call then has at hand
-    float const *V;             // [O][2^N], or null
+    int lut_binarize, rev_stride;
+    int fan_slots;              // slots per input, rev_stride - 1
     int node_size;
-    // ... and indexed != 0: the records are those of lut_dx_indexed_kernel: kTermHead + 2^N dwords, head = the address of the consumer's
-    // row of kept corner indices (x_base / x_row_pitch_bytes describe that buffer) and of its dy row, then the value at every corner of
-    // the node (all N inputs: the two corners that differ in input k hold the same)
-    int indexed;
+    int blocks;                 // workgroups that build records (kWavesPerBlk nodes each); 0 = nothing to build
 };
 
 // input j of a node's connections with connection k left out (j < N - 1, may differ per lane; k and the array index are compile-time)
@@ -913,117 +903,30 @@ __device__ __forceinline__ int ins_other(int const (&ins)[N], int k, int j)
     return r;
 }
 
-// A wavefront builds kTermRecordsPerWave consecutive records: lane i holds entry i of a consumer's table while it is
-// brought into the plain basis.  The records' loads go out together — reverse-table entries, then wiring and tables — so a
-// wavefront pays the two memory round trips of a record once for all of them (one record per wavefront made the builder
-// the longest part of the table-gradient launch of a layer with few nodes and many connections per input).
-// Slots beyond an input's fan-out are never read by the dx kernel and are left alone.
-constexpr int kTermRecordsPerWave = 4;
-
-template <int N>
-__device__ __forceinline__ void term_table_block(TermArgs const &a, int block)
-{
-    static_assert(2 * N <= kTermHead && kTermHead <= kWave, "head size");
-    constexpr int NN = 1 << N, HN = NN / 2, REC = kTermHead + HN, R = kTermRecordsPerWave;
-    int const total = a.fan.count * a.input_node_size;          // records, below 2^31 (checked on the host)
-    int const rec0  = __builtin_amdgcn_readfirstlane((block * kWavesPerBlk + (int)(threadIdx.x / kWave)) * R);
-    if (rec0 >= total) { return; }
-    int const lane = threadIdx.x & (kWave - 1);
-    // wave-uniform loads of tables that no kernel of the call writes: scalar loads through the constant address space
-    typedef __attribute__((address_space(4))) int const const_int;
-    const_int *rev = (const_int *)a.rev;
-
-    int in[R], slot[R], cnt[R], e[R];
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-        int const rec = min(rec0 + q, total - 1);               // (a wavefront past the last record repeats it and stores nothing)
-        split_tile(rec, a.fan, in[q], slot[q]);                 // rec = in * max_fan + slot
-        const_int *r = rev + (size_t)in[q] * a.rev_stride;
-        cnt[q] = r[0];
-        e[q]   = r[1 + slot[q]];                                // inside the row for every slot
-    }
-    bool  live[R];
-    int   k[R], node[R], head[R];
-    float v[R];
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-        live[q] = (rec0 + q < total) && (slot[q] < cnt[q]);
-        int const eq = live[q] ? e[q] : 0;                      // (whatever an unused slot holds is not followed)
-        k[q]    = eq % N;
-        node[q] = eq / N;
-        head[q] = 0;
-        if (lane < 2 * N) {
-            int const j = lane >> 1;
-            unsigned long long const addr = (j < N - 1) ? a.x_base + (unsigned long long)(unsigned)a.idx[node[q] * N + ((j < k[q]) ? j : j + 1)] * a.x_row_pitch_bytes
-                                                        : a.dy_base + (unsigned long long)(unsigned)node[q] * a.dy_row_pitch_bytes;
-            head[q] = (lane & 1) ? (int)(addr >> 32) : (int)(addr & 0xffffffffULL);
-        }
-        v[q] = 0.0f;
-        if (lane < NN) { v[q] = a.W[(size_t)node[q] * NN + lane]; }
-    }
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-        if (!live[q]) { continue; }                             // wave-uniform
-        int *out = a.term + (size_t)(rec0 + q) * REC;
-        if (lane < kTermHead) { out[lane] = head[q]; }
-        // P = plain-basis coefficients of W' (W' = lut_binarize ? W > 0.5 : W): the butterfly (a, b) -> (a, b - a) per index bit.
-        // For two-valued inputs the record holds values instead of coefficients: dy/dx_k at the corner where every other
-        // input j takes lo or hi.  W' is the table of y at x in {0, 1}^N and y is linear in each input, so input j != k
-        // interpolates, (a, b) -> (a + lo (b - a), a + hi (b - a)), and input k differentiates, (a, b) -> (., b - a).
-        float w = v[q];
-        if (a.lut_binarize) { w = (w > 0.5f) ? 1.0f : 0.0f; }
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            float const o   = __shfl_xor(w, 1 << j, 64);
-            bool const  up  = (lane >> j) & 1;
-            if (a.corner && j != k[q]) {
-                float const lower = up ? o : w, step = up ? (w - o) : (o - w);
-                w = __builtin_fmaf(up ? a.hi : a.lo, step, lower);
-            }
-            else {
-                w = up ? (w - o) : w;
-            }
-        }
-        if (lane < NN && ((lane >> k[q]) & 1)) {
-            int const sidx = (lane & ((1 << k[q]) - 1)) | ((lane >> (k[q] + 1)) << k[q]);      // the entry's index with bit k taken out
-            out[kTermHead + sidx] = __float_as_int(w);
-        }
-    }
-}
-
-// The same records built node by node: a wavefront takes a node, and for each of its N connections finds the connection's place in the
-// reverse-table row of its input (the lanes compare a row's entries with the connection id), and writes the record there.  Coefficient
-// records share one butterfly per node (the plain-basis table does not depend on the connection).  Value records (two-valued inputs) are
-// built where the call has already derived the node's corner values V: y is linear in input k between its two values, so dy/dx_k at a
-// corner of the other inputs is (V[k at hi] - V[k at lo]) / (hi - lo), one cross-lane exchange instead of a butterfly per record.  The
-// work is O x N records, not I x (largest fan-out) slots, and a fraction of the instructions per record: for a layer of 784 inputs and
-// 6144 nodes 2.5 us instead of 10.5 us.
+// The records are built node by node: a wavefront takes a node, and for each of its N connections finds the connection's place in the
+// reverse-table row of its input (the lanes compare a row's entries with the connection id), and writes the record there.  They share one
+// butterfly per node (the plain-basis table does not depend on the connection).  Slots beyond an input's fan-out are never read by the dx
+// kernel and are left alone.
 template <int N>
 __device__ __forceinline__ void term_table_node_block(TermArgs const &a, int block)
 {
-    constexpr int NN = 1 << N, HN = NN / 2;
-    int const REC = kTermHead + (a.indexed ? NN : HN);
+    static_assert(2 * N <= kTermHead && kTermHead <= kWave, "head size");
+    constexpr int NN = 1 << N, HN = NN / 2, REC = kTermHead + HN;
     int const node = __builtin_amdgcn_readfirstlane(block * kWavesPerBlk + (int)(threadIdx.x / kWave));
     if (node >= a.node_size) { return; }
     int const lane = threadIdx.x & (kWave - 1);
     typedef __attribute__((address_space(4))) int const const_int;
     const_int *rev = (const_int *)a.rev;
     const_int *idx = (const_int *)a.idx;
-    float v;
-    if (a.V != nullptr) { v = a.V[(size_t)node * NN + (lane & (NN - 1))]; }
-    else {
-        // coefficient records: P = plain-basis coefficients of W' (W' = lut_binarize ? W > 0.5 : W), the butterfly (a, b) -> (a, b - a)
-        // per index bit, as term_table_block forms them per record (same operations: same bits); a record takes the entries whose
-        // index has the connection's bit set
-        v = a.W[(size_t)node * NN + (lane & (NN - 1))];
-        if (a.lut_binarize) { v = (v > 0.5f) ? 1.0f : 0.0f; }
+    // P = plain-basis coefficients of W' (W' = lut_binarize ? W > 0.5 : W), the butterfly (a, b) -> (a, b - a) per index bit; a record
+    // takes the entries whose index has the connection's bit set
+    float v = a.W[(size_t)node * NN + (lane & (NN - 1))];
+    if (a.lut_binarize) { v = (v > 0.5f) ? 1.0f : 0.0f; }
 #pragma unroll
-        for (int j = 0; j < N; ++j) {
-            float const o = __shfl_xor(v, 1 << j, 64);
-            v = ((lane >> j) & 1) ? (v - o) : v;
-        }
+    for (int j = 0; j < N; ++j) {
+        float const o = __shfl_xor(v, 1 << j, 64);
+        v = ((lane >> j) & 1) ? (v - o) : v;
     }
-    float const inv_step = 1.0f / (a.hi - a.lo);
     int ins[N], cnt[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) { ins[k] = idx[node * N + k]; }
@@ -1040,19 +943,7 @@ __device__ __forceinline__ void term_table_node_block(TermArgs const &a, int blo
             if (m != 0) { slot = base + (int)__builtin_ctzll(m); }
         }
         if (slot < 0) { continue; }                                             // (a reverse table that does not list the connection: nothing to write)
-        int *out = a.term + ((size_t)ins[k] * a.fan.count + slot) * REC;
-        float const other = __shfl_xor(v, 1 << k, 64);
-        if (a.indexed) {
-            // the node's row of kept corner indices and its dy row; the value at every corner of the node (both corners of input k)
-            if (lane < 4) {
-                unsigned long long const addr = (lane < 2) ? a.x_base + (unsigned long long)(unsigned)node * a.x_row_pitch_bytes
-                                                           : a.dy_base + (unsigned long long)(unsigned)node * a.dy_row_pitch_bytes;
-                out[lane] = (lane & 1) ? (int)(addr >> 32) : (int)(addr & 0xffffffffULL);
-            }
-            float const step = ((lane >> k) & 1) ? (v - other) : (other - v);
-            if (lane < NN) { out[kTermHead + lane] = __float_as_int(step * inv_step); }
-            continue;
-        }
+        int *out = a.term + ((size_t)ins[k] * a.fan_slots + slot) * REC;
         if (lane < 2 * N) {
             int const j = lane >> 1;
             unsigned long long const addr = (j < N - 1) ? a.x_base + (unsigned long long)(unsigned)ins_other<N>(ins, k, j) * a.x_row_pitch_bytes
@@ -1061,7 +952,7 @@ __device__ __forceinline__ void term_table_node_block(TermArgs const &a, int blo
         }
         if (lane < NN && ((lane >> k) & 1)) {
             int const sidx = (lane & ((1 << k) - 1)) | ((lane >> (k + 1)) << k);          // the corner's index with bit k taken out
-            out[kTermHead + sidx] = __float_as_int((a.V != nullptr) ? (v - other) * inv_step : v);
+            out[kTermHead + sidx] = __float_as_int(v);
         }
     }
 }
@@ -1090,7 +981,6 @@ struct BwdArgs {
     TileDivisor tiles;
     float bias, gamma, beta, inv_frames;
     TermArgs tt;                // kDxNone: the last tt.blocks workgroups of the launch build the dx kernel's term table
-    float const *V;             // [O][2^N] corner values (CORNER variant)
     float const *stat_partial;  // BN, not null: dmean / dvar come from the stat_count (<= kInlineStatUnits) partial sums
     int   stat_count;           //     [unit][O][2] that the kind 3 launch left, added up by every wavefront for its node
 };
@@ -1109,10 +999,7 @@ enum DxMode : int { kDxAtomic = 0, kDxTmp = 1, kDxNone = 2 };
 
 // BWD_KIND: 0 = plain LUT backward, 1 = backward through batch-norm (its statistics pass is kind 3 of the forward kernel)
 // DXMODE  : how (whether) the per-connection input gradients leave the kernel
-// CORNER (packed bits, batch-norm, dx left to the dx kernel): the LUT output that the batch-norm window needs comes from
-// the node's corner values (index by add-with-carry from the lane masks, ds_bpermute) instead of the 64-term polynomial,
-// and the table leaves the scalar registers.
-template <int N, int XMODE, int BWD_KIND, int DXMODE, bool CORNER = false>
+template <int N, int XMODE, int BWD_KIND, int DXMODE>
 __global__ __launch_bounds__(kBlock) void lut_backward_kernel(BwdArgs a)
 {
     using D = LutDims<N>;
@@ -1124,8 +1011,7 @@ __global__ __launch_bounds__(kBlock) void lut_backward_kernel(BwdArgs a)
     int const B   = a.slab_count * a.tiles.count;
     if (DXMODE == kDxNone) {
         if (bid >= B) {
-            if (a.tt.node_size > 0) { term_table_node_block<N>(a.tt, bid - B); }
-            else                   { term_table_block<N>(a.tt, bid - B); }
+            term_table_node_block<N>(a.tt, bid - B);
             return;
         }
     }
@@ -1138,8 +1024,7 @@ __global__ __launch_bounds__(kBlock) void lut_backward_kernel(BwdArgs a)
     int const lane = threadIdx.x & (kWave - 1);
 
     // the table itself enters only the batch-norm kinds (the LUT output is recomputed) and the per-connection gradients
-    static_assert(!CORNER || (XMODE == kXBit && BWD_KIND != 0 && DXMODE == kDxNone), "corner values: packed bits, batch-norm, no dx here");
-    constexpr bool kNeedTable = ((BWD_KIND != 0) || (DXMODE != kDxNone)) && !CORNER;
+    constexpr bool kNeedTable = (BWD_KIND != 0) || (DXMODE != kDxNone);
     // (the partial sums stay on the vector ALU here: the matrix unit's operand registers would cost this kernel a wavefront of
     // occupancy, which measured slower; the batch-norm statistics pass, which only recomputes the LUT output, runs in the
     // forward kernel instead)
@@ -1148,8 +1033,6 @@ __global__ __launch_bounds__(kBlock) void lut_backward_kernel(BwdArgs a)
         LutEval<N>::load_table(a.C + (size_t)node * D::NN, C);
         LutEval<N>::pin_constants(C, cv);
     }
-    int corner = 0;
-    if (CORNER) { corner = __float_as_int(a.V[(size_t)node * D::NN + (lane & (D::NN - 1))]); }      // lane p holds V[p]
     void const *rows[N];
     int ins[N];
 #pragma unroll
@@ -1174,11 +1057,6 @@ __global__ __launch_bounds__(kBlock) void lut_backward_kernel(BwdArgs a)
         dvarf = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(dvarf)));
     }
     float const grs = a.gamma * rstd;
-    int corner_open = 0;        // lane p: 1 where the batch-norm output of corner p lies inside the hard-tanh window, else 0
-    if (CORNER) {
-        float const t = batch_norm_output(__int_as_float(corner), mean, rstd, a.gamma, a.beta);
-        corner_open = (t <= 0.0f || t >= 1.0f) ? 0 : 1;
-    }
 
     int const f_begin = a.f_base + sl * a.slab;
     int const f_end   = min(f_begin + a.slab, a.f_limit);
@@ -1223,18 +1101,9 @@ __global__ __launch_bounds__(kBlock) void lut_backward_kernel(BwdArgs a)
 
             if (BWD_KIND != 0) {
                 // hard-tanh window on the batch-norm output (reference: DifferentiableLutN.h:1206-1211, 1241-1246)
-                float v;
-                if constexpr (CORNER) {
-                    // the window depends on the corner alone: lane p decided it for corner p before the loop (same operations)
-                    int const index4 = (int)(corner_index<N, XMODE>(raw[u]) << 2);
-                    v = __int_as_float(__builtin_amdgcn_ds_bpermute(index4, corner));
-                    if (__builtin_amdgcn_ds_bpermute(index4, corner_open) == 0) { d = 0.0f; }
-                }
-                else {
-                    v = LutEval<N>::combine(h, q);
-                    float const t = batch_norm_output(v, mean, rstd, a.gamma, a.beta);
-                    if (t <= 0.0f || t >= 1.0f) { d = 0.0f; }
-                }
+                float const v = LutEval<N>::combine(h, q);
+                float const t = batch_norm_output(v, mean, rstd, a.gamma, a.beta);
+                if (t <= 0.0f || t >= 1.0f) { d = 0.0f; }
                 // dL/d(LUT output) (reference: DifferentiableLutN.h:1248-1250)
                 d = ok ? (__builtin_fmaf(d, grs, dmean) + v * dvarf) : 0.0f;
                 if (DXMODE == kDxNone && ok) { a.dx[(size_t)node * a.dx_stride + f] = d; }
@@ -1334,7 +1203,6 @@ struct DxArgs {
     float       *fin_dW;
     int   fin_node_size, fin_slab_count, fin_blocks;
     int   fin_overwrite;        // dW = instead of dW += (the caller's dW holds nothing: bbhip_HintTableGradientOverwrite)
-    int   own_stride;           // lut_dx_indexed_kernel: words per node row of the kept corner indices
 };
 
 // ------------------------------------------------------------------------------------------------
@@ -1556,267 +1424,6 @@ __global__ __launch_bounds__(kBlock) void lut_dx_kernel(DxArgs a)
             T::issue(head, xoff, yoff, x_row_bytes, y_row_bytes, st);
             T::load_coefficients(rec + (size_t)t * T::REC, Dk);
             T::accumulate(st, Dk, bit, lo, hi, acc);
-        }
-        dx_store_pass<U>(a, part, in, wave, lane, f_begin, acc);
-    }
-}
-
-// ------------------------------------------------------------------------------------------------
-//  Input-centric dx for two-valued inputs (packed bits, fp32 binarized at 0.5).  A term's dy/dx_k is one of 2^(N-1)
-//  values, chosen by the other inputs' bits: the term record holds that table (term_table_block with corner = 1), lane p
-//  keeps entry p, and a lane fetches the entry of its frame with ds_bpermute: about a dozen vector instructions per term
-//  and step instead of the polynomial's 43.  Units, work list and the dW rider are those of lut_dx_kernel; fp32 rows are
-//  loaded as there and compared with 0.5, packed rows take one load per row and pass (see below).
-// ------------------------------------------------------------------------------------------------
-template <int N, int XMODE, int U, bool WIDE = false>
-__global__ __launch_bounds__(kBlock) void lut_dx_corner_kernel(DxArgs a)
-{
-    static_assert(XMODE == kXBit || XMODE == kXBinary, "corner values need two-valued inputs");
-    static_assert(!WIDE || XMODE == kXBit, "scalar loads of whole passes are for packed rows");
-    using T = DxTerm<N, XMODE, U>;
-    int const bid = blockIdx.x;
-    int const B   = a.chunk_count * a.tiles.count;
-    if (bid >= B) { dw_finalize_block<N>(a.fin_partial, a.fin_dW, a.fin_node_size, a.fin_slab_count, bid - B, a.fin_overwrite); return; }
-    int const lid  = xcd_remap(bid, B);
-    int ck, tile;
-    split_tile(lid, a.tiles, ck, tile);
-    __shared__ float part[kWavesPerBlk][U][kWave];
-    int const wave = threadIdx.x / kWave;
-    int in, share;
-    dx_list_share(a, tile, wave, in, share);
-    if (in >= a.input_node_size) { return; }            // (workgroup-uniform in split mode)
-    int const lane = threadIdx.x & (kWave - 1);
-
-    int const cnt = a.rev[(size_t)in * a.rev_stride];
-    int t_begin, t_end;
-    dx_list_range(cnt, share, t_begin, t_end);
-    typedef __attribute__((address_space(4))) int const const_int;
-    const_int *rec = (const_int *)(a.term + (size_t)in * (a.rev_stride - 1) * T::REC);
-    int const *rec_v = a.term + (size_t)in * (a.rev_stride - 1) * T::REC + kTermHead + (lane & (T::HN - 1));
-    uint32_t const y_row_bytes = (uint32_t)a.frame_size * 4u;
-    uint32_t const x_row_bytes = (XMODE == kXBit) ? (uint32_t)((a.frame_size + 31) >> 5) * 4u : y_row_bytes;
-
-    for (int f_begin = ck * a.chunk; f_begin < min((ck + 1) * a.chunk, a.frame_size); f_begin += kWave * U) {
-        uint32_t const f0   = (uint32_t)(f_begin + lane);
-        uint32_t const yoff = f0 * 4u;
-        uint32_t const xoff = (XMODE == kXBit) ? (f0 >> 5) * 4u : yoff;
-        uint32_t const wordoff = ((uint32_t)(f_begin >> 5) + (uint32_t)(lane & (2 * U - 1))) * 4u;      // packed rows: word (lane mod 2 U) of the pass
-        float acc[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) { acc[u] = 0.0f; }
-
-        // Packed rows: a term is a round trip — its head (row addresses, scalar loads), then the rows' words and dy — and a few
-        // dozen instructions, so the walk is bound by latency.  Two terms are in flight: while term t is evaluated, the rows of
-        // term t + 1 have been requested and the head of term t + 2 is on its way.
-        if constexpr (XMODE == kXBit) {
-            // The 64 U frames of a pass are 2 U words of a packed row, the same for every lane: one load per row brings them
-            // in (lane i holds word i of the pass), each step's two words are read back as a lane mask, and the index costs
-            // one add-with-carry per input.  Per term and pass: M + U + 1 vector memory instructions instead of (M + 1) U + 1.
-            constexpr int HEAD = 2 * T::M + 2;
-            int head[HEAD];
-            uint32_t w_next[T::M];
-            float dy_next[U];
-            int values_next = 0;
-            auto load_head = [&](int t) {
-#pragma unroll
-                for (int i = 0; i < HEAD; ++i) { head[i] = rec[(size_t)t * T::REC + i]; }
-            };
-            auto request_rows = [&](int t) {                      // of the term whose head is in `head`
-#pragma unroll
-                for (int j = 0; j < T::M; ++j) {
-                    __amdgpu_buffer_rsrc_t const d = address_descriptor((uint32_t)head[2 * j], (uint32_t)head[2 * j + 1], x_row_bytes);
-                    w_next[j] = __builtin_amdgcn_raw_buffer_load_b32(d, wordoff, 0, 0);
-                }
-                __amdgpu_buffer_rsrc_t const dyr = address_descriptor((uint32_t)head[2 * T::M], (uint32_t)head[2 * T::M + 1], y_row_bytes);
-#pragma unroll
-                for (int u = 0; u < U; ++u) { dy_next[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(dyr, yoff + u * (kWave * 4u), 0, 0)); }
-                values_next = rec_v[(size_t)t * T::REC];        // lane p: the term's value at corner p
-            };
-            if constexpr (WIDE) {
-                // Row pitch a multiple of 2 U words: the 2 U words of a pass are ONE scalar load per row (32 bytes with U = 4), each
-                // step's lane mask is a register pair of it, and the 2 M U read-lanes of the form below go away (a third of this
-                // kernel's instructions).  A term's corner indices are formed one term ahead, as soon as its words are there,
-                // so only the head of term t + 2 and the words of term t + 1 sit in scalar registers.
-                typedef uint32_t u32x8 __attribute__((ext_vector_type(2 * U)));
-                typedef __attribute__((address_space(4))) u32x8 const const_u32x8;
-                uint32_t index_next[U];
-                auto request_wide = [&](int t) {                  // of the term whose head is in `head`: its indices, dy, values
-                    u32x8 wq[T::M];
-#pragma unroll
-                    for (int j = 0; j < T::M; ++j) {
-                        uint64_t const row = ((uint64_t)(uint32_t)head[2 * j + 1] << 32) | (uint32_t)head[2 * j];
-                        wq[j] = *(const_u32x8 *)(row + (uint64_t)(uint32_t)(f_begin >> 5) * 4u);
-                    }
-                    __amdgpu_buffer_rsrc_t const dyr = address_descriptor((uint32_t)head[2 * T::M], (uint32_t)head[2 * T::M + 1], y_row_bytes);
-#pragma unroll
-                    for (int u = 0; u < U; ++u) { dy_next[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(dyr, yoff + u * (kWave * 4u), 0, 0)); }
-                    values_next = rec_v[(size_t)t * T::REC];
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        uint32_t index = 0;                        // most significant input first: index = 2 index + bit
-#pragma unroll
-                        for (int j = T::M - 1; j >= 0; --j) {
-                            uint64_t const mask = (uint64_t)wq[j][2 * u] | ((uint64_t)wq[j][2 * u + 1] << 32);
-                            uint64_t carry;
-                            asm("v_addc_co_u32_e64 %0, %1, %2, %2, %3" : "=v"(index), "=s"(carry) : "v"(index), "s"(mask));
-                        }
-                        index_next[u] = index << 2;
-                    }
-                };
-                if (t_begin < t_end) {
-                    load_head(t_begin);
-                    request_wide(t_begin);
-                    if (t_begin + 1 < t_end) { load_head(t_begin + 1); }
-                }
-                for (int t = t_begin; t < t_end; ++t) {
-                    uint32_t idx4[U];
-                    float dyv[U];
-#pragma unroll
-                    for (int u = 0; u < U; ++u) { idx4[u] = index_next[u]; dyv[u] = dy_next[u]; }
-                    int const values = values_next;
-                    if (t + 1 < t_end) {
-                        request_wide(t + 1);
-                        if (t + 2 < t_end) { load_head(t + 2); }
-                    }
-#pragma unroll
-                    for (int u = 0; u < U; ++u) {
-                        float const d = __int_as_float(__builtin_amdgcn_ds_bpermute((int)idx4[u], values));
-                        acc[u] = __builtin_fmaf(dyv[u], d, acc[u]);
-                    }
-                }
-                dx_store_pass<U>(a, part, in, wave, lane, f_begin, acc);
-                continue;
-            }
-            if (t_begin < t_end) {
-                load_head(t_begin);
-                request_rows(t_begin);
-                if (t_begin + 1 < t_end) { load_head(t_begin + 1); }
-            }
-            for (int t = t_begin; t < t_end; ++t) {
-                uint32_t w[T::M];
-                float dyv[U];
-#pragma unroll
-                for (int j = 0; j < T::M; ++j) { w[j] = w_next[j]; }
-#pragma unroll
-                for (int u = 0; u < U; ++u) { dyv[u] = dy_next[u]; }
-                int const values = values_next;
-                if (t + 1 < t_end) {
-                    request_rows(t + 1);
-                    if (t + 2 < t_end) { load_head(t + 2); }
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    uint32_t index = 0;                            // most significant input first: index = 2 index + bit
-#pragma unroll
-                    for (int j = T::M - 1; j >= 0; --j) {
-                        uint64_t const mask = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)w[j], 2 * u) |
-                                              ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)w[j], 2 * u + 1) << 32);
-                        uint64_t carry;
-                        asm("v_addc_co_u32_e64 %0, %1, %2, %2, %3" : "=v"(index), "=s"(carry) : "v"(index), "s"(mask));
-                    }
-                    float const d = __int_as_float(__builtin_amdgcn_ds_bpermute((int)(index << 2), values));
-                    acc[u] = __builtin_fmaf(dyv[u], d, acc[u]);
-                }
-            }
-            dx_store_pass<U>(a, part, in, wave, lane, f_begin, acc);
-            continue;
-        }
-        for (int t = t_begin; t < t_end; ++t) {
-            int const values = rec_v[(size_t)t * T::REC];          // lane p: the term's value at corner p
-            typename T::Stage st;
-            T::issue(rec + (size_t)t * T::REC, xoff, yoff, x_row_bytes, y_row_bytes, st);
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                uint32_t index = 0;
-#pragma unroll
-                for (int j = 0; j < T::M; ++j) { index |= (__uint_as_float(st.raw[u][j]) > 0.5f) ? (4u << j) : 0u; }
-                float const d = __int_as_float(__builtin_amdgcn_ds_bpermute((int)index, values));
-                acc[u] = __builtin_fmaf(st.dyv[u], d, acc[u]);
-            }
-        }
-        dx_store_pass<U>(a, part, in, wave, lane, f_begin, acc);
-    }
-}
-
-// ------------------------------------------------------------------------------------------------
-//  Input-centric dx from kept corner indices (batch-norm backward over two-valued inputs).  The statistics pass of the same
-//  call has formed the corner index of every (node, frame) and kept it, a byte each (FwdArgs::own_index_out); a term's
-//  dy/dx_k is its record's value at that corner (term_table_node_block with indexed = 1), so a term costs per pass one word of
-//  indices and four of dy per lane, and per step a byte extract, ds_bpermute and the multiply-add: no row of the other inputs
-//  is read and no index is formed.  Units (multiples of 256 frames), work list, split mode and the dW rider are those of
-//  lut_dx_corner_kernel, and so is the order of the sums: the same bits.
-// ------------------------------------------------------------------------------------------------
-template <int N>
-__global__ __launch_bounds__(kBlock) void lut_dx_indexed_kernel(DxArgs a)
-{
-    constexpr int U = 4, NN = 1 << N, REC = kTermHead + NN, HEAD = 4;
-    int const bid = blockIdx.x;
-    int const B   = a.chunk_count * a.tiles.count;
-    if (bid >= B) { dw_finalize_block<N>(a.fin_partial, a.fin_dW, a.fin_node_size, a.fin_slab_count, bid - B, a.fin_overwrite); return; }
-    int const lid  = xcd_remap(bid, B);
-    int ck, tile;
-    split_tile(lid, a.tiles, ck, tile);
-    __shared__ float part[kWavesPerBlk][U][kWave];
-    int const wave = threadIdx.x / kWave;
-    int in, share;
-    dx_list_share(a, tile, wave, in, share);
-    if (in >= a.input_node_size) { return; }            // (workgroup-uniform in split mode)
-    int const lane = threadIdx.x & (kWave - 1);
-
-    int const cnt = a.rev[(size_t)in * a.rev_stride];
-    int t_begin, t_end;
-    dx_list_range(cnt, share, t_begin, t_end);
-    typedef __attribute__((address_space(4))) int const const_int;
-    const_int *rec = (const_int *)(a.term + (size_t)in * (a.rev_stride - 1) * REC);
-    int const *rec_v = a.term + (size_t)in * (a.rev_stride - 1) * REC + kTermHead + (lane & (NN - 1));
-    uint32_t const y_row_bytes = (uint32_t)a.frame_size * 4u;
-    uint32_t const i_row_bytes = (uint32_t)a.own_stride * 4u;
-
-    for (int f_begin = ck * a.chunk; f_begin < min((ck + 1) * a.chunk, a.frame_size); f_begin += kWave * U) {
-        uint32_t const yoff = (uint32_t)(f_begin + lane) * 4u;
-        uint32_t const ioff = ((uint32_t)(f_begin >> 8) * kWave + (uint32_t)lane) * 4u;     // byte u of the word: frame f_begin + 64 u + lane
-        float acc[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) { acc[u] = 0.0f; }
-
-        // two terms in flight, as in lut_dx_corner_kernel: while term t is evaluated, the words of term t + 1 have been
-        // requested and the head of term t + 2 is on its way (four in flight measured slower: 136 vs 128 us at 4096 x 4096 x 8192)
-        int head[HEAD];
-        uint32_t iw_next = 0;
-        float dy_next[U];
-        int values_next = 0;
-        auto load_head = [&](int t) {
-#pragma unroll
-            for (int i = 0; i < HEAD; ++i) { head[i] = rec[(size_t)t * REC + i]; }
-        };
-        auto request = [&](int t) {                           // of the term whose head is in `head`
-            __amdgpu_buffer_rsrc_t const ir = address_descriptor((uint32_t)head[0], (uint32_t)head[1], i_row_bytes);
-            iw_next = __builtin_amdgcn_raw_buffer_load_b32(ir, ioff, 0, 0);
-            __amdgpu_buffer_rsrc_t const dyr = address_descriptor((uint32_t)head[2], (uint32_t)head[3], y_row_bytes);
-#pragma unroll
-            for (int u = 0; u < U; ++u) { dy_next[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(dyr, yoff + u * (kWave * 4u), 0, 0)); }
-            values_next = rec_v[(size_t)t * REC];              // lane p: the term's value at corner p
-        };
-        if (t_begin < t_end) {
-            load_head(t_begin);
-            request(t_begin);
-            if (t_begin + 1 < t_end) { load_head(t_begin + 1); }
-        }
-        for (int t = t_begin; t < t_end; ++t) {
-            uint32_t const iw = iw_next;
-            float dyv[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) { dyv[u] = dy_next[u]; }
-            int const values = values_next;
-            if (t + 1 < t_end) {
-                request(t + 1);
-                if (t + 2 < t_end) { load_head(t + 2); }
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                float const d = __int_as_float(__builtin_amdgcn_ds_bpermute((int)((iw >> (8 * u)) & 0xffu), values));
-                acc[u] = __builtin_fmaf(dyv[u], d, acc[u]);
-            }
         }
         dx_store_pass<U>(a, part, in, wave, lane, f_begin, acc);
     }

@@ -1,0 +1,67 @@
+"""GPU parity of the backward pass over two-valued inputs (per-corner sums, fold, dx from kept corner indices) at the sizes where its kernels
+have edges: last words and last groups of four frames, passes of 256 and blocks of 2048 frames, several slabs per node, shared work lists."""
+import numpy as np
+import pytest
+
+import oracle
+from binarybrain_amd import synth
+from util import assert_bwd, dev, host
+
+pytestmark = pytest.mark.gpu
+
+
+# inputs, nodes, frames, row pitch of the fp32 buffers (0: the frame buffer's)
+SHAPES = [(7, 3, 1, 0), (7, 3, 5, 0), (9, 5, 31, 31), (16, 9, 33, 35), (40, 70, 255, 255), (6, 130, 257, 0), (24, 4, 2047, 2047), (12, 6, 2049, 2052),
+          (27, 36, 6001, 6001), (8, 40, 20001, 0), (600, 520, 300, 0), (1030, 1100, 65, 0)]
+
+
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 6])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_corner_backward(n, shape):
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    I, O, F, stride = shape
+    stride = stride or synth.frame_stride_fp32(F)
+    rng = np.random.default_rng(100 * n + F)
+    idx = synth.wiring(rng, I, O, n); W = synth.lut_tables(rng, O, n)
+    x = synth.uniform_frames(rng, I, F, stride); dy = synth.normal_frames(rng, O, F, stride)
+    xb = synth.pack_bits((x[:, :F] > 0.5).astype(np.uint8), (F + 31) // 32)
+    _, mean, rstd, _, _ = oracle.differentiable_lut_forward_training(n, x, idx, W, F, np.zeros(O, np.float32), np.ones(O, np.float32))
+    want = {True: oracle.differentiable_lut_backward(n, x, dy, idx, W, F, mean, rstd),
+            False: oracle.stochastic_lut_backward(n, x, dy, idx, W, F, input_binary=True, simd=False)}
+    dy[:, F:] = np.nan                              # what lies behind the frames enters nothing
+    d_x, d_xb, d_dy, d_idx, d_W = dev(x), dev(xb), dev(dy), dev(idx), dev(W)
+    rev = ops.reverse_table(d_idx, I)
+    start = dev(np.full_like(W, 0.25))
+    for bn in ((True, False) if F > 4 else (False,)):            # (the gradient through the statistics of a frame or two is rounding alone)
+        dx_ref, dW_ref = want[bn]
+        got = []
+        for packed in (False, True):
+            dW = start.clone()
+            if bn:
+                args = (n, d_xb if packed else d_x, d_dy, d_idx, d_W, dW, F, dev(mean), dev(rstd), rev)
+                dx = (ops.bit_differentiable_lut_backward if packed else ops.differentiable_lut_backward)(*args)
+            else:
+                args = (n, d_xb if packed else d_x, d_dy, d_idx, d_W, dW, F, rev)
+                dx = ops.bit_stochastic_lut_backward(*args) if packed else ops.stochastic_lut_backward(*args, input_binary=True)
+            assert_bwd(host(dx)[:, :F], dx_ref[:, :F], "dx bn=%d packed=%d" % (bn, packed))
+            assert_bwd(host(dW) - 0.25, dW_ref, "dW bn=%d packed=%d" % (bn, packed))
+            got.append((host(dx)[:, :F], host(dW)))
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("bias", [0.0, 0.01, 0.0625])
+def test_input_values_that_nearly_meet(bias):
+    """slopes are not taken from differences of corner values where those lose digits"""
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    rng = np.random.default_rng(3)
+    I, O, F = 20, 30, 200
+    stride = synth.frame_stride_fp32(F)
+    idx = synth.wiring(rng, I, O, 6); W = synth.lut_tables(rng, O, 6)
+    x = synth.uniform_frames(rng, I, F, stride); dy = synth.normal_frames(rng, O, F, stride)
+    dx_ref, dW_ref = oracle.stochastic_lut_backward(6, x, dy, idx, W, F, input_binary=True, bias=bias, simd=False)
+    dW = dev(np.zeros_like(W))
+    d_idx = dev(idx)
+    dx = ops.stochastic_lut_backward(6, dev(x), dev(dy), d_idx, dev(W), dW, F, ops.reverse_table(d_idx, I), input_binary=True, bias=bias)
+    assert_bwd(host(dx)[:, :F], dx_ref[:, :F], "dx"); assert_bwd(host(dW), dW_ref, "dW")
