@@ -1872,15 +1872,15 @@ int bbhip_fp32_ClassifierTail_ForwardBackward(float const *dev_x_buf, float *dev
     if (frame_stride < frame_size) { return fail("%s: frame stride shorter than the frames", __func__); }
     if (ch_size > 16) { return fail("%s: at most 16 classes (ch_size=%d): call the four entries one by one", __func__, ch_size); }
     if ((long long)ch_size * n > 0x7fffffffLL) { return fail("%s: connection table too large", __func__); }
-    // per-input sums, logits and gradients of 64 frames, then the table: within 64 KiB of LDS
-    size_t const lds = ((size_t)input_node_size + 2 * 16) * 64 * sizeof(float) + (((size_t)ch_size * n + 3) & ~(size_t)3) * sizeof(int);
-    if (lds > 64u * 1024u) {
-        return fail("%s: input_node_size=%d nodes and ch_size*n=%d table entries need %zu bytes of LDS, 65536 are there (192 nodes with 2048 entries, "
-                    "216 with 512): call the four entries one by one", __func__, input_node_size, ch_size * n, lds);
+    constexpr int CH = 16;
+    // (the limit that the entry documents)
+    if (((size_t)input_node_size + 2 * CH) * 64 * sizeof(float) + (((size_t)ch_size * n + 3) & ~(size_t)3) * sizeof(int) > 64u * 1024u) {
+        return fail("%s: input_node_size=%d nodes and ch_size*n=%d table entries are more than the one launch takes (192 nodes with 2048 entries, "
+                    "216 with 512): call the four entries one by one", __func__, input_node_size, ch_size * n);
     }
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
-    hipLaunchKernelGGL(classifier_tail_kernel<16>, dim3((unsigned)ceil_div(frame_stride, 64)), dim3(64 * kClassifierTailWaves), lds, st, dev_x_buf, dev_y_buf, dev_dx_buf,
+    hipLaunchKernelGGL(classifier_tail_kernel<CH>, dim3((unsigned)ceil_div(frame_stride, 64)), dim3(64 * CH), lds, st, dev_x_buf, dev_y_buf, dev_dx_buf,
                        dev_input_index, dev_t_buf, dev_dy_buf, dev_loss_buf, dev_accuracy_buf, dev_category_buf, t_sum,
                        output_sum ? 1.0f : 1.0f / (float)n, n, input_node_size, ch_size, frame_size, frame_stride, binarize_input);
     BBHIP_LAUNCH_CHECK();
