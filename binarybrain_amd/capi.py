@@ -42,6 +42,7 @@ _SIGNATURES = {
     "bbhip_HintPackedInput": (None, [_vp, _i, _i, _i]),
     "bbhip_HintPackedOutput": (None, [_vp, _i, _i]),
     "bbhip_HintTableGradientOverwrite": (None, [_i]),
+    "bbhip_HintZeroOutputPadding": (None, [_i]),
     "bbhip_HintPreparedTables": (None, [_vp, C.c_size_t, _i]),
     "bbhip_PreparedTablesBytes": (C.c_size_t, [_i, _i]),
     "bbhip_GetDxMode": (C.c_int, []),

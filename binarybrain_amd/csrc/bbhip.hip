@@ -78,9 +78,11 @@ struct PackedOutputHint { uint32_t *bits; int rows, row_words; };
 thread_local PackedOutputHint g_packed_out_hint = {nullptr, 0, 0};
 // bbhip_HintTableGradientOverwrite: the next backward call writes dW instead of adding to it
 thread_local int g_dw_overwrite_hint = 0;
+// bbhip_HintZeroOutputPadding: the next call with packed output writes its rows up to the row pitch
+thread_local int g_zero_padding_hint = 0;
 static inline void clear_hints(void)
 {
-    g_dw_overwrite_hint = 0;
+    g_dw_overwrite_hint = 0; g_zero_padding_hint = 0;
     g_input_node_hint = 0; g_packed_hint = PackedInputHint{nullptr, 0, 0, 0}; g_tables_hint = PreparedTablesHint{nullptr, 0, 0};
     g_packed_out_hint = PackedOutputHint{nullptr, 0, 0};
 }
@@ -359,6 +361,7 @@ struct ForwardCall {
     float gamma, beta, momentum;
     // non-null: W (the same buffer) is clamped in place to [clamp_lo, clamp_hi] by the table-preparation launch
     float *clamp_W; float clamp_lo, clamp_hi;
+    int zero_padding;            // packed output: zeros behind the last frame's word, up to the row pitch
 };
 
 // the kernels address a frame inside its node row with a 32-bit byte offset
@@ -517,6 +520,7 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
     a.x_stride = c.x_stride; a.y_stride = c.y_stride;
     a.chunk = chunk; a.chunk_count = chunk_count; a.tiles = make_tile_divisor(tile_count);
     a.bias = c.bias; a.gamma = c.gamma; a.beta = c.beta;
+    a.zero_padding = c.zero_padding;
 
     int kind = 0;
     if (c.bn == 1 && corner && chunk_count == 1) {
@@ -576,6 +580,8 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
 
 int forward_entry(ForwardCall const &c, void *stream, Scratch const *fixed = nullptr)
 {
+    ForwardCall c = call;
+    c.zero_padding = g_zero_padding_hint;
     // the hints are spent by this call, whatever becomes of it; a buffer for the packed copy also says how many rows the input has
     PackedInputHint const packed = fixed ? PackedInputHint{nullptr, 0, 0, 0} : g_packed_hint;
     int const input_rows = fixed ? 0 : (packed.bits ? packed.rows : g_input_node_hint);
@@ -1226,6 +1232,7 @@ size_t bbhip_PreparedTablesBytes(int n, int node_size)
     return 2 * align256((size_t)node_size * ((size_t)1 << n) * sizeof(float));
 }
 
+void bbhip_HintZeroOutputPadding(int zero) { g_zero_padding_hint = zero != 0; }
 void bbhip_HintTableGradientOverwrite(int overwrite) { g_dw_overwrite_hint = overwrite != 0; }
 
 void bbhip_HintPackedOutput(int *dev_bits, int rows, int row_words)
@@ -2104,7 +2111,7 @@ int bbhip_fp32_HardTanh_Backward(float const *dev_x_buf, float const *dev_dy_buf
                           stream, __func__);
 }
 
-static int launch_real_to_binary(float const *x, void *y, bool bit, unsigned depth_modulation_size, unsigned frame_modulation_size,
+static int launch_real_to_binary(float const *x, void *y, bool bit, bool zero_padding, unsigned depth_modulation_size, unsigned frame_modulation_size,
                                  float input_range_lo, float input_range_hi, unsigned point_size, unsigned x_depth_size, unsigned x_frame_size,
                                  unsigned x_frame_stride, unsigned y_frame_stride, int binarize, void *stream, char const *name)
 {
@@ -2131,7 +2138,9 @@ static int launch_real_to_binary(float const *x, void *y, bool bit, unsigned dep
     // packed rows are assembled from whole threads either way; fp32 rows need 16-byte rows for the wide stores
     bool const wide = bit || ((reinterpret_cast<uintptr_t>(y) & 15u) == 0 && (y_frame_stride & 3u) == 0);
     unsigned blocks;
-    if (modulation_grid((int)y_nodes, (int)y_frames, wide, a.f_blocks, blocks, name)) { return 1; }
+    // (packed rows are written as far as the launch reaches: to the row pitch where the caller wants its padding zeroed)
+    long long const reach = (zero_padding && (long long)y_frame_stride * 32 <= 0x7fffffffLL) ? (long long)y_frame_stride * 32 : y_frames;
+    if (modulation_grid((int)y_nodes, (int)reach, wide, a.f_blocks, blocks, name)) { return 1; }
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
     dim3 const grid(blocks), block(kModBlock);
@@ -2156,7 +2165,8 @@ int bbhip_fp32_bit_RealToBinary_Forward(float const *dev_x_buf, int *dev_y_buf, 
                                         unsigned x_frame_size, unsigned x_frame_stride, unsigned y_frame_stride, int binarize, void *stream)
 {
     clear_hints();                                 // a hint is for the next LUT forward call only
-    return launch_real_to_binary(dev_x_buf, dev_y_buf, true, depth_modulation_size, frame_modulation_size, input_range_lo, input_range_hi,
+    bool const zero_padding = g_zero_padding_hint != 0;
+    return launch_real_to_binary(dev_x_buf, dev_y_buf, true, zero_padding, depth_modulation_size, frame_modulation_size, input_range_lo, input_range_hi,
                                  point_size, x_depth_size, x_frame_size, x_frame_stride, y_frame_stride, binarize, stream, __func__);
 }
 
@@ -2769,6 +2779,7 @@ int bbhip_bit_BinaryLut6_Forward(int const *dev_x_buf, int *dev_y_buf, int const
                                  int node_size, int frame_size, int frame_stride, void *stream)
 {
     clear_hints();                                 // a hint is for the next LUT forward call only
+    int const zero_padding = g_zero_padding_hint;
     BBHIP_REQUIRE(dev_x_buf != nullptr && dev_y_buf != nullptr && dev_input_index != nullptr && dev_table != nullptr);
     BBHIP_REQUIRE(node_size > 0 && node_size <= (0x7fffffff >> 6) && frame_size > 0);
     BBHIP_REQUIRE(frame_stride >= (frame_size + 31) / 32);
@@ -2795,11 +2806,16 @@ int bbhip_bit_BinaryLut6_Forward(int const *dev_x_buf, int *dev_y_buf, int const
         dim3 const grid(a.chunk_count * a.tiles.count), block(kBlock);
         bool const exact = (node_size % npw) == 0;
         switch (npw) {
-        case 1: hipLaunchKernelGGL((binary_lut6_kernel<1, true>), grid, block, 0, st, a); break;
-        case 2: if (exact) { hipLaunchKernelGGL((binary_lut6_kernel<2, true>), grid, block, 0, st, a); }
+        bool const pad = zero_padding && frame_stride > a.word_count;
+        case 1: if (pad) { hipLaunchKernelGGL((binary_lut6_kernel<1, true, true>), grid, block, 0, st, a); }
+                else     { hipLaunchKernelGGL((binary_lut6_kernel<1, true>), grid, block, 0, st, a); }
+                break;
+        case 2: if (pad)        { hipLaunchKernelGGL((binary_lut6_kernel<2, false, true>), grid, block, 0, st, a); }
+                else if (exact) { hipLaunchKernelGGL((binary_lut6_kernel<2, true>), grid, block, 0, st, a); }
                 else       { hipLaunchKernelGGL((binary_lut6_kernel<2, false>), grid, block, 0, st, a); }
                 break;
-        default: if (exact) { hipLaunchKernelGGL((binary_lut6_kernel<4, true>), grid, block, 0, st, a); }
+        default: if (pad)       { hipLaunchKernelGGL((binary_lut6_kernel<4, false, true>), grid, block, 0, st, a); }
+                 else if (exact) { hipLaunchKernelGGL((binary_lut6_kernel<4, true>), grid, block, 0, st, a); }
                  else       { hipLaunchKernelGGL((binary_lut6_kernel<4, false>), grid, block, 0, st, a); }
                  break;
         }
@@ -2813,6 +2829,7 @@ int bbhip_bit_BinaryLutN_Forward(int n, int const *dev_x_buf, int *dev_y_buf, in
 {
     if (n == 6) { return bbhip_bit_BinaryLut6_Forward(dev_x_buf, dev_y_buf, dev_input_index, dev_table, node_size, frame_size, frame_stride, stream); }
     clear_hints();
+    int const zero_padding = g_zero_padding_hint;
     if (n < 2 || n > 6) { return fail("%s: LUT width n=%d not in 2..6", __func__, n); }
     BBHIP_REQUIRE(dev_x_buf != nullptr && dev_y_buf != nullptr && dev_input_index != nullptr && dev_table != nullptr);
     BBHIP_REQUIRE(node_size > 0 && node_size <= (0x7fffffff >> 6) && frame_size > 0);
@@ -2820,7 +2837,7 @@ int bbhip_bit_BinaryLutN_Forward(int n, int const *dev_x_buf, int *dev_y_buf, in
     hipStream_t st = static_cast<hipStream_t>(stream);
     uint32_t const *x = reinterpret_cast<uint32_t const *>(dev_x_buf);
     uint32_t *y = reinterpret_cast<uint32_t *>(dev_y_buf);
-    int const words = (frame_size + 31) / 32;
+    int const words = zero_padding ? frame_stride : (frame_size + 31) / 32;
     ScopedTimer tm(kTimeBinary, st);
     for (int n0 = 0; n0 < node_size; n0 += 65535) {            // grid.y is limited to 65535 nodes per launch
         dim3 const grid(ceil_div(words, kBlock), (node_size - n0 < 65535) ? node_size - n0 : 65535), block(kBlock);

@@ -241,6 +241,7 @@ struct FwdArgs {
     int   own_stride;
     // kStatPartial: units per node of the launch that left the partial sums, where the output launch has other units (0: the same)
     int   stat_units;
+    int   zero_padding;         // packed output: the wavefront of a node's last unit writes 0 behind the last frame's word, up to the row pitch
 };
 
 // kStatInline: the call has one unit per node, so the wavefront that writes a node's output first sums the node's statistics
@@ -309,6 +310,12 @@ __device__ __forceinline__ void zero_packed_tail(FwdArgs const &a, int ck, int n
 {
     if (a.y_bits == nullptr || ck != a.chunk_count - 1 || !live) { return; }
     for (int w = ((a.frame_size + 31) >> 5) + lane; w < a.y_bits_stride; w += kWave) { a.y_bits[(size_t)node * a.y_bits_stride + w] = 0u; }
+}
+
+__device__ __forceinline__ void zero_output_padding(FwdArgs const &a, int ck, int node, bool live, int lane)
+{
+    if (a.zero_padding == 0 || ck != a.chunk_count - 1 || !live) { return; }
+    for (int w = ((a.frame_size + 31) >> 5) + lane; w < a.y_stride; w += kWave) { reinterpret_cast<uint32_t *>(a.y)[(size_t)node * a.y_stride + w] = 0u; }
 }
 
 // per (unit, node) partial sums of the statistics kinds
@@ -527,6 +534,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     if (YMODE == kYBinarize && (FWD_KIND == 0 || FWD_KIND == 1)) {
 #pragma unroll
         for (int p = 0; p < NPW; ++p) { zero_packed_tail(a, ck, node[p], live[p], lane); }
+    }
+    if (YMODE == kYBit) {
+#pragma unroll
+        for (int p = 0; p < NPW; ++p) { zero_output_padding(a, ck, node[p], live[p], lane); }
     }
     if (FWD_KIND == 0 && kMatrix) {           // (at the end: a store ahead of the unit's loads would be waited for with them)
 #pragma unroll
@@ -818,6 +829,7 @@ __global__ __launch_bounds__(kBlock) void lut_forward_corner_kernel(FwdArgs a)
     if (FWD_KIND == 2 || FWD_KIND == 3) { forward_store_stats(a, ck, node, true, lane, s1, s2); }
     if (FWD_KIND == 1) { forward_store_statistics(a, node, true, ck, lane, mean, var, rstd); }
     if (YMODE == kYBinarize && (FWD_KIND == 0 || FWD_KIND == 1)) { zero_packed_tail(a, ck, node, true, lane); }
+    if (YMODE == kYBit) { zero_output_padding(a, ck, node, true, lane); }
     if (a.W_inline != nullptr && ck == 0 && lane < NN) {
         if (clamp_store)         { a.clamp_W[(size_t)node * NN + lane] = table_w; }
         if (a.C_out != nullptr)  { a.C_out[(size_t)node * NN + lane] = table_c; }
@@ -1663,7 +1675,9 @@ __device__ __forceinline__ void bin_index_words(uint32_t table_lo, uint32_t tabl
     for (int j = 0; j < 8; ++j) { iw[j] = (uint32_t)__builtin_amdgcn_readlane((int)v, j); }
 }
 
-template <int NPW, bool EXACT>   // nodes per wavefront; EXACT: the node count is a multiple of NPW, no wavefront has nodes to skip
+// nodes per wavefront; EXACT: the node count is a multiple of NPW, no wavefront has nodes to skip; PAD: the wavefronts of a row's last unit write 0
+// behind the last frame's word, up to the row pitch (a branch at the kernel's end costs the large shape 1 %, hence a variant of its own)
+template <int NPW, bool EXACT, bool PAD = false>
 __global__ __launch_bounds__(kBlock) void binary_lut6_kernel(BinArgs a)
 {
     int const B    = a.chunk_count * a.tiles.count;
@@ -1749,6 +1763,12 @@ __global__ __launch_bounds__(kBlock) void binary_lut6_kernel(BinArgs a)
             }
         }
     }
+    if (PAD && w_end == a.word_count) {                          // wave-uniform
+#pragma unroll
+        for (int p = 0; p < NPW; ++p) {
+            for (int w = a.word_count + lane; live[p] && w < a.stride; w += kWave) { a.y[(size_t)(node0 + p) * a.stride + w] = 0u; }
+        }
+    }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1766,7 +1786,10 @@ __global__ __launch_bounds__(kBlock) void binary_lutn_kernel(uint32_t const *__r
     int const node = node0 + (int)blockIdx.y;
     int const w = blockIdx.x * kBlock + threadIdx.x;
     int const words = (frame_size + 31) >> 5;
-    if (w >= words) { return; }
+    if (w >= words) {                               // (launched where the caller wants the row's padding zeroed)
+        if (w < stride) { y[(size_t)node * stride + w] = 0u; }
+        return;
+    }
     uint32_t const t = (uint32_t)table[node];
     uint32_t sel[N];
 #pragma unroll

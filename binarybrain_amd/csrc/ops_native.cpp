@@ -113,7 +113,7 @@ void *current_stream(void) { return at::hip::getCurrentHIPStreamMasqueradingAsCU
 void clear_hints(void)
 {
     bbhip_HintInputNodeSize(0); bbhip_HintPackedInput(nullptr, 0, 0, 0); bbhip_HintPackedOutput(nullptr, 0, 0);
-    bbhip_HintTableGradientOverwrite(0); bbhip_HintPreparedTables(nullptr, 0, 0);
+    bbhip_HintTableGradientOverwrite(0); bbhip_HintPreparedTables(nullptr, 0, 0); bbhip_HintZeroOutputPadding(0);
 }
 
 // One entry point with the interpreter lock released; a failure becomes a BbhipError with the library's message.
@@ -176,6 +176,14 @@ template <class E> E *data(OptTensor t) { return t ? static_cast<E *>((*t).data_
 
 int rows_of(T t)   { return (int)t.size(0); }
 int stride_of(T t) { return (int)t.size(1); }
+
+// packed output rows: the caller's, or new ones whose padding the next call zeroes (the library is told, no fill launch)
+at::Tensor packed_output(OptTensor out, T like, int64_t rows, int64_t words)
+{
+    if (out) { return *out; }
+    bbhip_HintZeroOutputPadding(1);
+    return rows_i32(like, rows, words);
+}
 
 void require(bool ok, char const *what) { if (!ok) { throw Failed(what); } }
 
@@ -304,7 +312,7 @@ bit_differentiable_lut_forward_training(int n, T x, T idx, T W, int frames, T ru
                                         float bias, bool lut_binarize, Clamp clamp, OptTensor tables, OptTensor out, bool hints)
 {
     int const O = rows_of(idx), S = stride_of(x);
-    at::Tensor y = out ? *out : zeros_i32(x, O, S), mean = line_f32(x, O), rstd = line_f32(x, O);
+    at::Tensor y = packed_output(out, x, O, S), mean = line_f32(x, O), rstd = line_f32(x, O);
     if (hints) { hint_tables(tables, false); }
     if (clamp.on) {
         call(bbhip_bit_fp32_DifferentiableLutN_ForwardTrainingClampW, n, data<int const>(x), data<int>(y), data<int const>(idx), data<float>(W),
@@ -338,7 +346,7 @@ at::Tensor bit_differentiable_lut_forward_inference(int n, T x, T idx, T W, int 
                                                     bool lut_binarize)
 {
     int const O = rows_of(idx), S = stride_of(x);
-    at::Tensor y = zeros_i32(x, O, S);
+    at::Tensor y = packed_output(OptTensor{nullptr}, x, O, S);
     call(bbhip_bit_fp32_DifferentiableLutN_ForwardInference, n, data<int const>(x), data<int>(y), data<int const>(idx), data<float const>(W),
          data<float const>(running_mean), data<float const>(running_var), gamma, beta, bias, O, frames, S, (int)lut_binarize, current_stream());
     return y;
@@ -397,7 +405,7 @@ at::Tensor bit_differentiable_lut_backward(int n, T x, T dy, T idx, T W, T dW, i
 at::Tensor binary_lut_forward(int n, T x, T idx, T table, int frames, OptTensor out)
 {
     int const O = rows_of(idx), S = stride_of(x);
-    at::Tensor y = out ? *out : zeros_i32(x, O, S);
+    at::Tensor y = packed_output(out, x, O, S);
     call(bbhip_bit_BinaryLutN_Forward, n, data<int const>(x), data<int>(y), data<int const>(idx), data<int const>(table), O, frames, S, current_stream());
     return y;
 }
@@ -422,6 +430,7 @@ classifier_tail(T x, T idx, T t, int frames, float t_sum, bool input_binary, boo
 // ---- buffers for the wrappers that stay in Python ------------------------------------------------------------------------------------
 at::Tensor new_rows(T like, int rows, int stride)  { return rows_f32(like, rows, stride); }
 at::Tensor new_bits(T like, int rows, int words)   { return rows_i32(like, rows, words); }
+at::Tensor new_padded_bits(T like, int rows, int words) { return packed_output(OptTensor{nullptr}, like, rows, words); }     // for the next call's output
 at::Tensor new_zero_bits(T like, int rows, int words) { return zeros_i32(like, rows, words); }
 at::Tensor new_line(T like, int n)                 { return line_f32(like, n); }
 
@@ -437,7 +446,7 @@ PyMethodDef methods[] = {
     BBHIP_FUNCTION(differentiable_lut_forward_inference), BBHIP_FUNCTION(bit_differentiable_lut_forward_inference),
     BBHIP_FUNCTION(differentiable_lut_forward_nobn), BBHIP_FUNCTION(differentiable_lut_backward), BBHIP_FUNCTION(bit_differentiable_lut_backward),
     BBHIP_FUNCTION(binary_lut_forward), BBHIP_FUNCTION(classifier_tail),
-    BBHIP_FUNCTION(new_rows), BBHIP_FUNCTION(new_bits), BBHIP_FUNCTION(new_zero_bits), BBHIP_FUNCTION(new_line),
+    BBHIP_FUNCTION(new_rows), BBHIP_FUNCTION(new_bits), BBHIP_FUNCTION(new_padded_bits), BBHIP_FUNCTION(new_zero_bits), BBHIP_FUNCTION(new_line),
     BBHIP_ENTRY(fp32_Vector_set), BBHIP_ENTRY(fp32_Vector_clamp), BBHIP_ENTRY(fp32_Vector_add_ex), BBHIP_ENTRY(fp32_Vector_mul_ex),
     BBHIP_ENTRY(fp32_Vector_div_ex), BBHIP_ENTRY(fp32_Vector_sqrt), BBHIP_ENTRY(fp32_Vector_exp), BBHIP_ENTRY(fp32_Vector_min),
     BBHIP_ENTRY(fp32_Vector_min_v), BBHIP_ENTRY(fp32_Vector_max), BBHIP_ENTRY(fp32_Vector_max_v),

@@ -289,7 +289,7 @@ def real_to_binary_forward(x, depth, points, frame_size, frame_mod=1, depth_mod=
         y_stride = (out_frames + 31) // 32 if bit else out_frames
     nodes = depth * depth_mod * points
     if bit:
-        y = native.new_zero_bits(x, nodes, y_stride)
+        y = native.new_padded_bits(x, nodes, y_stride)
         f = native.fp32_bit_RealToBinary_Forward
     else:
         y = native.new_rows(x, nodes, y_stride)
@@ -487,7 +487,7 @@ def bit_stochastic_lut_forward(n, xbits, idx, W, frame_size, y_stride, lut_binar
 
 def bit_bit_stochastic_lut_forward(n, xbits, idx, W, frame_size, lut_binarize=False, bias=0.25):
     O = idx.shape[0]
-    y = native.new_zero_bits(xbits, O, xbits.shape[1])
+    y = native.new_padded_bits(xbits, O, xbits.shape[1])
     native.bit_bit_fp32_StochasticLut_Forward(n, xbits, y, idx, W, O, frame_size, xbits.shape[1], int(lut_binarize), bias)
     return y
 

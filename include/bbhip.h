@@ -132,6 +132,13 @@ void bbhip_HintPackedOutput(int *dev_bits, int rows, int row_words);
  * Same bits as zero-fill followed by the plain call.  Thread-local, spent by the next entry called on the thread. */
 void bbhip_HintTableGradientOverwrite(int overwrite);
 
+/* ---- packed output rows written whole (no counterpart in the reference) ----
+ * The entries that write rows of packed bits write the words that hold frames and leave the rest of the row pitch alone, as the reference's
+ * do; a caller that allocates a row buffer for one call zero-fills it first.  Given right before a forward call of a LUT layer with packed
+ * output (StochasticLut, DifferentiableLut, BinaryLut) or of bbhip_fp32_bit_RealToBinary_Forward, the call also writes 0 to the words of every output
+ * row behind the last frame's, up to the row pitch: the fill launch falls away.  Thread-local, spent by the next entry called on the thread. */
+void bbhip_HintZeroOutputPadding(int zero);
+
 /* No counterpart in the reference.  A caller-owned device buffer (256-byte aligned, bbhip_PreparedTablesBytes(n, node_size) bytes) for the
  * tables that a LUT call derives from W before its kernels run (centred coefficients, corner values).  Given right before a forward call
  * (holds_tables = 0), the call writes them there instead of into the library's scratch memory; given right before the backward call of

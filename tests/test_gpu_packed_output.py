@@ -126,3 +126,26 @@ def test_table_gradient_written_instead_of_accumulated(ops, batch_norm, dx_mode)
         assert float((dW1 - 2 * dW0).abs().max()) <= 1e-5 * float(dW0.abs().max())
     finally:
         ops.set_dx_mode(0)
+
+
+@pytest.mark.parametrize("n", [2, 4, 6])
+@pytest.mark.parametrize("F", [1, 33, 64, 65, 2048, 2049, 5000])
+def test_packed_rows_written_whole(n, F):
+    """outputs that the wrappers allocate are zero behind the last frame, whatever the memory held"""
+    import torch
+    from binarybrain_amd import ops
+    rng = np.random.default_rng(n + F)
+    I, O, words = 9, 11, synth.frame_stride_bit(F)
+    xb = dev(synth.bernoulli_bits(rng, I, F, words)); idx = dev(synth.wiring(rng, I, O, n)); W = dev(synth.lut_tables(rng, O, n))
+    table = dev(rng.integers(0, 1 << min(31, 1 << n), (O, 2 if n == 6 else 1)).astype(np.int32))
+    rm, rv = torch.full((O,), 0.5, device="cuda"), torch.ones(O, device="cuda")
+    x = dev(synth.uniform_frames(rng, I, F))
+    calls = [lambda: ops.binary_lutn_forward(n, xb, idx, table, F), lambda: ops.bit_bit_stochastic_lut_forward(n, xb, idx, W, F),
+             lambda: ops.bit_differentiable_lut_forward_inference(n, xb, idx, W, F, rm, rv),
+             lambda: ops.bit_differentiable_lut_forward_training(n, xb, idx, W, F, rm.clone(), rv.clone())[0],
+             lambda: ops.real_to_binary_forward(x, 1, I, F, 1, bit=True, y_stride=words)]
+    for call in calls:
+        y = call()
+        dirty = torch.full_like(y, -1); del y, dirty        # the allocator hands this memory to the next output
+        bits = synth.unpack_bits(host(call()), words * 32)
+        assert not bits[:, F:].any()
