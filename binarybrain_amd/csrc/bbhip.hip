@@ -578,7 +578,7 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
     return 0;
 }
 
-int forward_entry(ForwardCall const &c, void *stream, Scratch const *fixed = nullptr)
+int forward_entry(ForwardCall const &call, void *stream, Scratch const *fixed = nullptr)
 {
     ForwardCall c = call;
     c.zero_padding = g_zero_padding_hint;
@@ -1885,6 +1885,7 @@ int bbhip_fp32_ClassifierTail_ForwardBackward(float const *dev_x_buf, float *dev
         return fail("%s: input_node_size=%d nodes and ch_size*n=%d table entries are more than the one launch takes (192 nodes with 2048 entries, "
                     "216 with 512): call the four entries one by one", __func__, input_node_size, ch_size * n);
     }
+    size_t const lds = 5 * CH * 64 * sizeof(float) + (size_t)ch_size * n * sizeof(int);
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
     hipLaunchKernelGGL(classifier_tail_kernel<CH>, dim3((unsigned)ceil_div(frame_stride, 64)), dim3(64 * CH), lds, st, dev_x_buf, dev_y_buf, dev_dx_buf,
@@ -2156,7 +2157,7 @@ int bbhip_fp32_RealToBinary_Forward(float const *dev_x_buf, float *dev_y_buf, un
                                     unsigned x_frame_size, unsigned x_frame_stride, unsigned y_frame_stride, int binarize, void *stream)
 {
     clear_hints();                                 // a hint is for the next LUT forward call only
-    return launch_real_to_binary(dev_x_buf, dev_y_buf, false, depth_modulation_size, frame_modulation_size, input_range_lo, input_range_hi,
+    return launch_real_to_binary(dev_x_buf, dev_y_buf, false, false, depth_modulation_size, frame_modulation_size, input_range_lo, input_range_hi,
                                  point_size, x_depth_size, x_frame_size, x_frame_stride, y_frame_stride, binarize, stream, __func__);
 }
 
@@ -2164,8 +2165,8 @@ int bbhip_fp32_bit_RealToBinary_Forward(float const *dev_x_buf, int *dev_y_buf, 
                                         float input_range_lo, float input_range_hi, unsigned point_size, unsigned x_depth_size,
                                         unsigned x_frame_size, unsigned x_frame_stride, unsigned y_frame_stride, int binarize, void *stream)
 {
-    clear_hints();                                 // a hint is for the next LUT forward call only
     bool const zero_padding = g_zero_padding_hint != 0;
+    clear_hints();                                 // a hint is for the next LUT forward call only
     return launch_real_to_binary(dev_x_buf, dev_y_buf, true, zero_padding, depth_modulation_size, frame_modulation_size, input_range_lo, input_range_hi,
                                  point_size, x_depth_size, x_frame_size, x_frame_stride, y_frame_stride, binarize, stream, __func__);
 }
@@ -2778,8 +2779,8 @@ int bbhip_bit_fp32_DifferentiableLutN_Backward(int n, int const *dev_x_buf, floa
 int bbhip_bit_BinaryLut6_Forward(int const *dev_x_buf, int *dev_y_buf, int const *dev_input_index, int const *dev_table,
                                  int node_size, int frame_size, int frame_stride, void *stream)
 {
-    clear_hints();                                 // a hint is for the next LUT forward call only
     int const zero_padding = g_zero_padding_hint;
+    clear_hints();                                 // a hint is for the next LUT forward call only
     BBHIP_REQUIRE(dev_x_buf != nullptr && dev_y_buf != nullptr && dev_input_index != nullptr && dev_table != nullptr);
     BBHIP_REQUIRE(node_size > 0 && node_size <= (0x7fffffff >> 6) && frame_size > 0);
     BBHIP_REQUIRE(frame_stride >= (frame_size + 31) / 32);
@@ -2805,8 +2806,8 @@ int bbhip_bit_BinaryLut6_Forward(int const *dev_x_buf, int *dev_y_buf, int const
         ScopedTimer tm(kTimeBinary, st);
         dim3 const grid(a.chunk_count * a.tiles.count), block(kBlock);
         bool const exact = (node_size % npw) == 0;
-        switch (npw) {
         bool const pad = zero_padding && frame_stride > a.word_count;
+        switch (npw) {
         case 1: if (pad) { hipLaunchKernelGGL((binary_lut6_kernel<1, true, true>), grid, block, 0, st, a); }
                 else     { hipLaunchKernelGGL((binary_lut6_kernel<1, true>), grid, block, 0, st, a); }
                 break;
@@ -2828,8 +2829,8 @@ int bbhip_bit_BinaryLutN_Forward(int n, int const *dev_x_buf, int *dev_y_buf, in
                                  int node_size, int frame_size, int frame_stride, void *stream)
 {
     if (n == 6) { return bbhip_bit_BinaryLut6_Forward(dev_x_buf, dev_y_buf, dev_input_index, dev_table, node_size, frame_size, frame_stride, stream); }
-    clear_hints();
     int const zero_padding = g_zero_padding_hint;
+    clear_hints();
     if (n < 2 || n > 6) { return fail("%s: LUT width n=%d not in 2..6", __func__, n); }
     BBHIP_REQUIRE(dev_x_buf != nullptr && dev_y_buf != nullptr && dev_input_index != nullptr && dev_table != nullptr);
     BBHIP_REQUIRE(node_size > 0 && node_size <= (0x7fffffff >> 6) && frame_size > 0);

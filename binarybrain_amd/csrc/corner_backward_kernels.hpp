@@ -2,10 +2,13 @@
 //
 // Over two-valued inputs a node's frames fall into 2^N corners, and everything that the backward pass needs of them is, per corner,
 //     D[p] = the sum of dy over the frames at corner p,     n[p] = the number of those frames.
-// With batch-norm, dL/d(LUT output) of a frame at corner p is  open[p] gamma rstd dy + dmean + V[p] dvar / F  (reference:
-// DifferentiableLutN.h:1206-1250), where open[p] says whether the batch-norm output of the corner lies inside the hard-tanh window, so
-//     sum of g              = sum_p open[p] D[p],           sum of g (v - mean) = sum_p open[p] D[p] (V[p] - mean),
-//     gradient at corner p  G[p] = open[p] gamma rstd D[p] + n[p] (dmean + V[p] dvar / F),
+// With batch-norm, dL/d(LUT output) of a frame at corner p is  open[p] gamma rstd dy + E[p]  (reference: DifferentiableLutN.h:1206-1250), where
+// open[p] says whether the batch-norm output of the corner lies inside the hard-tanh window and E[p] is the gradient through the statistics, so
+//     sum of g              s0 = sum_p open[p] D[p],        sum of g (v - mean)   s1 = sum_p open[p] D[p] (V[p] - mean),
+//     E[p] = shift + (V[p] - mean) scale,   shift = -gamma rstd s0 / F,   scale = -gamma rstd^3 s1 / F
+//            (the reference's dmean + V dvar / F with mean dvar / F left out of both: where V is hundreds of times its own spread that
+//            difference costs two digits),
+//     gradient at corner p  G[p] = open[p] gamma rstd D[p] + n[p] E[p],
 //     dW[i]                 = sum_p G[p] prod_j (bit_j(i) ? x_j(p) : 1 - x_j(p)).
 // One pass over the inputs and dy gives D and n (lut_corner_sums_kernel), the rest is arithmetic on 2^N values per node (corner_fold): no
 // statistics pass of its own, no polynomial, no 2^N multiply-adds per frame, and no row of dL/d(LUT output) is written.  The dx kernel
@@ -23,34 +26,40 @@ struct CornerFoldArgs {
     float lo, hi;                       // the two input values, 1/2 -+ bias
     float *dW;
     int   overwrite;                    // dW = instead of dW +=
-    float4 *node_consts;                // batch-norm: mean, rstd, dmean, dvar / F of each node, for the dx kernel
+    float4 *node_consts;                // batch-norm: mean, rstd, shift, scale of each node, for the dx kernel
 };
 
 // Lane p (of every group of 2^N lanes) holds the node's V[p], D[p], n[p]: the node's table gradient and, with batch-norm, its constants
+// (mean, rstd and the entry of dW that the gradient adds to: loaded by the caller, long before)
+struct CornerFoldInputs { float mean, rstd, dW; };
 template <int N, bool BN>
-__device__ __forceinline__ void corner_fold(CornerFoldArgs const &a, int node, int lane, float v, float D, float n)
+__device__ __forceinline__ CornerFoldInputs corner_fold_inputs(CornerFoldArgs const &a, int node, int lane)
+{
+    CornerFoldInputs q{0.0f, 1.0f, 0.0f};
+    if (BN) { q.mean = a.mean[node]; q.rstd = a.rstd[node]; }
+    if (!a.overwrite) { q.dW = a.dW[((size_t)node << N) + (lane & ((1 << N) - 1))]; }
+    return q;
+}
+template <int N, bool BN>
+__device__ __forceinline__ void corner_fold(CornerFoldArgs const &a, CornerFoldInputs const &q, int node, int lane, float v, float D, float n)
 {
     constexpr int NN = 1 << N;
     float G = D;
     if (BN) {
-        float const mean = a.mean[node], rstd = a.rstd[node];
+        float const mean = q.mean, rstd = q.rstd;
         float const t = batch_norm_output(v, mean, rstd, a.gamma, a.beta);
         float const g = (t <= 0.0f || t >= 1.0f) ? 0.0f : D;
         float const counted = (lane < NN) ? g : 0.0f;                   // narrow tables repeat over the wavefront
         float const s0 = wave_sum(counted), s1 = wave_sum(counted * (v - mean));
-        float dmean, dvar;
-        batch_gradient_statistics(s0, s1, mean, rstd, a.gamma, a.frame_size, dmean, dvar);
-        dvar *= a.inv_frames;
-        G = __builtin_fmaf(g, a.gamma * rstd, n * __builtin_fmaf(v, dvar, dmean));
-        if (lane == 0) { a.node_consts[node] = make_float4(mean, rstd, dmean, dvar); }
+        float const shift = -(a.gamma * s0) * rstd * a.inv_frames;
+        float const scale = -(a.gamma * s1) * (rstd * rstd) * rstd * a.inv_frames;
+        G = __builtin_fmaf(g, a.gamma * rstd, n * __builtin_fmaf(v - mean, scale, shift));
+        if (lane == 0) { a.node_consts[node] = make_float4(mean, rstd, shift, scale); }
     }
     // per input: (G0, G1) -> ((1 - lo) G0 + (1 - hi) G1, lo G0 + hi G1), and 1 - lo = hi: either lane keeps hi of its own and takes lo of the other's
 #pragma unroll
-    for (int j = 0; j < N; ++j) { G = __builtin_fmaf(a.hi, G, a.lo * __shfl_xor(G, 1 << j, 64)); }
-    if (lane < NN) {
-        float *out = a.dW + (size_t)node * NN + lane;
-        *out = a.overwrite ? G : *out + G;
-    }
+    for (int j = 0; j < N; ++j) { G = __builtin_fmaf(a.hi, G, a.lo * lane_xor(G, 1 << j)); }
+    if (lane < NN) { a.dW[(size_t)node * NN + lane] = a.overwrite ? G : q.dW + G; }
 }
 
 struct CornerSumsArgs {
@@ -143,7 +152,7 @@ __device__ __forceinline__ auto row_sum(V4 const *block, int lane)
         s += (q.x + q.y) + (q.z + q.w);
     }
 #pragma unroll
-    for (int o = ROWS; o < kWave; o <<= 1) { s += __shfl_xor(s, o, 64); }
+    for (int o = ROWS; o < kWave; o <<= 1) { s += lane_xor(s, o); }
     return s;
 }
 
@@ -192,6 +201,8 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) { dy[i] = load_quad(dyr, (uint32_t)(f_begin + i * 4 * kWave + 4 * lane) * 4u, quad_rows); }
 
+    CornerFoldInputs fold_in{};
+    if (a.slab_count == 1) { fold_in = corner_fold_inputs<N, BN>(a.fold, node, lane); }
     float v;                                                            // lane p: V[p]
     if (a.V != nullptr) { v = a.V[(size_t)node * NN + (lane & (NN - 1))]; }
     else {
@@ -274,12 +285,12 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
         n = row_sum<NN>(reinterpret_cast<uint4 const *>(cells), lane);  // lane S: frames where every input of S is set (the others either way)
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-            uint32_t const o = __shfl_xor(n, 1 << k, 64);
+            uint32_t const o = lane_xor(n, 1 << k);
             if (!((lane >> k) & 1)) { n -= o; }                         // ... minus those where input k is set too
         }
     }
 
-    if (a.slab_count == 1) { corner_fold<N, BN>(a.fold, node, lane, v, D, (float)n); }
+    if (a.slab_count == 1) { corner_fold<N, BN>(a.fold, fold_in, node, lane, v, D, (float)n); }
     else if (lane < NN) {
         float *out = a.partial + ((size_t)sl * a.node_size + node) * (BN ? 2 * NN : NN) + lane;
         out[0] = D;
@@ -298,6 +309,8 @@ __global__ __launch_bounds__(kBlock) void lut_corner_fold_kernel(CornerFoldArgs 
     int const node = blockIdx.x;
     int const wv = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
     float const *in = partial + (size_t)node * REC + (lane & (NN - 1));
+    CornerFoldInputs const fold_in = corner_fold_inputs<N, BN>(a, node, lane);
+    float const v = V[(size_t)node * NN + (lane & (NN - 1))];
     float D = 0.0f, n = 0.0f;
 #pragma unroll 4
     for (int s = wv; s < slab_count; s += kWavesPerBlk) {
@@ -311,7 +324,7 @@ __global__ __launch_bounds__(kBlock) void lut_corner_fold_kernel(CornerFoldArgs 
     if (wv != 0) { return; }
 #pragma unroll
     for (int w = 1; w < kWavesPerBlk; ++w) { D += red[0][w][lane]; n += red[1][w][lane]; }
-    corner_fold<N, BN>(a, node, lane, V[(size_t)node * NN + (lane & (NN - 1))], D, n);
+    corner_fold<N, BN>(a, fold_in, node, lane, v, D, n);
 }
 
 struct DxTableArgs {
@@ -320,13 +333,13 @@ struct DxTableArgs {
     int   own_stride;
     int   dy_quads, dx_quads;           // rows hold whole groups of four frames (dx: 16-byte aligned as well)
     float const *V;                     // [O][2^N]
-    float4 const *node_consts;          // batch-norm: mean, rstd, dmean, dvar / F
+    float4 const *node_consts;          // batch-norm: mean, rstd, shift, scale
     float gamma, beta, inv_step;        // inv_step = 1 / (hi - lo)
 };
 
 // Input-centric dx over kept corner indices.  One wavefront owns dx[input][256 Q frames], four consecutive frames per lane and quad, and walks the
 // input's consumers in the reverse table's order (split mode: a quarter of them).  A consumer's term of a frame at corner p is  A[p] dy + B[p]  with
-//     A[p] = dV/dx_k[p] open[p] gamma rstd,   B[p] = dV/dx_k[p] (dmean + V[p] dvar / F)           (plain layers: A = dV/dx_k, B = 0),
+//     A[p] = dV/dx_k[p] open[p] gamma rstd,   B[p] = dV/dx_k[p] E[p]           (plain layers: A = dV/dx_k, B = 0),
 // and y is linear in input k, so dV/dx_k[p] = (V[k at hi] - V[k at lo]) / (hi - lo): lane p computes entry p from the node's 2^N corner values
 // and four constants (272 bytes per node that all its consumers share), the wavefront puts the table into LDS, and the frames fetch their
 // entry from there: a random 8-byte LDS read takes 4.5 clocks per CU and step where two ds_bpermute take 14.  Per term and pass one vector load
@@ -393,7 +406,7 @@ __global__ __launch_bounds__(kBlock) void lut_dx_table_kernel(DxTableArgs t)
         float4 dy[Q];
 #pragma unroll
         for (int q = 0; q < Q; ++q) { iw[q] = iw_next[q]; dy[q] = dy_next[q]; }
-        float const v = v_next, mean = c_next[0], rstd = c_next[1], dmean = c_next[2], dvar = c_next[3];
+        float const v = v_next, mean = c_next[0], rstd = c_next[1], shift = c_next[2], scale = c_next[3];
         int const k = k_next;
         if (i + 1 < t_end) {
             request(e_ahead);
@@ -405,7 +418,7 @@ __global__ __launch_bounds__(kBlock) void lut_dx_table_kernel(DxTableArgs t)
         if constexpr (BN) {
             float const y = batch_norm_output(v, mean, rstd, t.gamma, t.beta);
             float const A = (y <= 0.0f || y >= 1.0f) ? 0.0f : slope * (t.gamma * rstd);
-            if (lane < NN) { tab[lane] = make_float2(A, slope * __builtin_fmaf(v, dvar, dmean)); }
+            if (lane < NN) { tab[lane] = make_float2(A, slope * __builtin_fmaf(v - mean, scale, shift)); }
         }
         else { if (lane < NN) { tab[lane] = slope; } }
         wave_fence();

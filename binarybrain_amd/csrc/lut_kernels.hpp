@@ -33,7 +33,7 @@ __device__ __forceinline__ int xcd_remap(int b, int B)
 __device__ __forceinline__ float wave_sum(float v)
 {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) { v += __shfl_xor(v, o, 64); }
+    for (int o = 32; o > 0; o >>= 1) { v += lane_xor(v, o); }
     return v;
 }
 
@@ -53,7 +53,7 @@ __device__ __forceinline__ float centred_butterfly(float v, int i)
 {
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-        float const o = __shfl_xor(v, 1 << j, 64);
+        float const o = lane_xor(v, 1 << j);
         v = ((i >> j) & 1) ? (v - o) : (v + o) * 0.5f;
     }
     return v;
@@ -65,7 +65,7 @@ __device__ __forceinline__ float corner_butterfly(float v, int i, float bias)
 {
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-        float const o = __shfl_xor(v, 1 << j, 64);
+        float const o = lane_xor(v, 1 << j);
         v = ((i >> j) & 1) ? __builtin_fmaf(bias, v, o) : __builtin_fmaf(-bias, o, v);
     }
     return v;
@@ -122,7 +122,7 @@ __device__ __forceinline__ void dw_finalize_block(float const *__restrict__ part
     int const i = t & (NN - 1);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-        float const o = __shfl_xor(v, 1 << j, 64);
+        float const o = lane_xor(v, 1 << j);
         v = ((i >> j) & 1) ? (o * 0.5f + v) : (v * 0.5f - o);
     }
     if (t < total) { dW[t] = overwrite ? v : dW[t] + v; }
@@ -457,7 +457,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
                 if (a.lut_binarize) { v = (v > 0.5f) ? 1.0f : 0.0f; }
 #pragma unroll
                 for (int j = 0; j < N; ++j) {                 // as table_prep_block: (a, b) -> ((a + b) / 2, b - a) per index bit
-                    float const o = __shfl_xor(v, 1 << j, 64);
+                    float const o = lane_xor(v, 1 << j);
                     v = ((lane >> j) & 1) ? (v - o) : (v + o) * 0.5f;
                 }
                 mq[p].take(v, lane);
@@ -936,7 +936,7 @@ __device__ __forceinline__ void term_table_node_block(TermArgs const &a, int blo
     if (a.lut_binarize) { v = (v > 0.5f) ? 1.0f : 0.0f; }
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-        float const o = __shfl_xor(v, 1 << j, 64);
+        float const o = lane_xor(v, 1 << j);
         v = ((lane >> j) & 1) ? (v - o) : v;
     }
     int ins[N], cnt[N];
@@ -1185,8 +1185,8 @@ __global__ __launch_bounds__(kBlock) void lut_backward_kernel(BwdArgs a)
 #pragma unroll
             for (int t = 0; t < 16; ++t) { s += red[wv][r][qd * 16 + t]; }
         }
-        s += __shfl_xor(s, 1, 64);
-        s += __shfl_xor(s, 2, 64);
+        s += lane_xor(s, 1);
+        s += lane_xor(s, 2);
         if (qd == 0 && r < CNT) { out[ps * 16 + r] = s; }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -1523,9 +1523,9 @@ __device__ __forceinline__ void binarize_pack4_block(float const *__restrict__ x
             ((f + 2 < frame_size && t.z > 0.5f) ? 4u : 0u) | ((f + 3 < frame_size && t.w > 0.5f) ? 8u : 0u);
     }
     v <<= 4 * (threadIdx.x & 7);
-    v |= __shfl_xor(v, 1, 64);
-    v |= __shfl_xor(v, 2, 64);
-    v |= __shfl_xor(v, 4, 64);
+    v |= lane_xor(v, 1);
+    v |= lane_xor(v, 2);
+    v |= lane_xor(v, 4);
     int const w = q >> 3;
     if ((threadIdx.x & 7) == 0 && w < y_stride) { bits[(size_t)node * y_stride + w] = v; }
 }

@@ -38,6 +38,32 @@ struct LutDims {
     static constexpr int NN = 1 << N;
 };
 
+// The value of lane (lane ^ M), M a power of two known at compile time (after unrolling).  Within a row of 16 lanes by a data-parallel move, across
+// rows by the row swaps of gfx950: 11 ns for an exchange and an addition where __shfl_xor, which goes through the LDS crossbar, takes 31; a
+// small launch is a chain of a dozen or two of them.  Every lane of the wavefront calls this.
+__device__ __forceinline__ int lane_xor(int v, int M)
+{
+    switch (M) {
+    case 1:  return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);                // quad_perm [1, 0, 3, 2]
+    case 2:  return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true);                // quad_perm [2, 3, 0, 1]
+    case 4: {
+        int const up = __builtin_amdgcn_update_dpp(v, v, 0x104, 0xf, 0x5, false);           // row_shl:4 into lanes 0-3, 8-11 of each row
+        return __builtin_amdgcn_update_dpp(up, v, 0x114, 0xf, 0xa, false);                  // row_shr:4 into lanes 4-7, 12-15
+    }
+    case 8:  return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, true);               // row_ror:8
+    case 16: {
+        auto const s = __builtin_amdgcn_permlane16_swap(v, v, false, false);                // [0]: even rows twice, [1]: odd rows twice
+        return (threadIdx.x & 16) ? s[0] : s[1];
+    }
+    default: {
+        auto const s = __builtin_amdgcn_permlane32_swap(v, v, false, false);                // [0]: lower half twice, [1]: upper half twice
+        return (threadIdx.x & 32) ? s[0] : s[1];
+    }
+    }
+}
+__device__ __forceinline__ float    lane_xor(float v, int M)    { return __int_as_float(lane_xor(__float_as_int(v), M)); }
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v, int M) { return (uint32_t)lane_xor((int)v, M); }
+
 // how a kernel reads its inputs
 enum XMode : int {
     kXClamp  = 0,   // fp32 frames, clamp to [0,1]                 (StochasticLutN.h:542)

@@ -17,6 +17,7 @@
 #include <stdint.h>
 
 #include "bn_kernels.hpp"
+#include "lut_math.hpp"
 #include "tile_divisor.hpp"
 #include "vector_kernels.hpp"
 
@@ -67,9 +68,9 @@ __device__ __forceinline__ void store_packed_bits(uint32_t bits, uint32_t *__res
 {
     if constexpr (W == 4) {
         uint32_t v = bits << (4 * (threadIdx.x & 7));
-        v |= __shfl_xor(v, 1, 64);
-        v |= __shfl_xor(v, 2, 64);
-        v |= __shfl_xor(v, 4, 64);
+        v |= lane_xor(v, 1);
+        v |= lane_xor(v, 2);
+        v |= lane_xor(v, 4);
         int const w = f >> 5;
         if ((threadIdx.x & 7) == 0 && w < y_stride) { row[w] = v; }
     }
