@@ -667,7 +667,8 @@ int dispatch_dx_table(int quads, DxTableArgs const &t, hipStream_t st)
 {
     dim3 const grid(t.dx.chunk_count * t.dx.tiles.count), block(kBlock);
     ScopedTimer tm(kTimeDx, st);
-    switch (quads) {
+    if (t.far) { hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, 1, true>), grid, block, 0, st, t); }
+    else switch (quads) {
     case 1:  hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, 1>), grid, block, 0, st, t); break;
     case 2:  hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, 2>), grid, block, 0, st, t); break;
     default: hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, 4>), grid, block, 0, st, t); break;
@@ -702,14 +703,14 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     size_t const v_bytes     = align256((size_t)O * NN * sizeof(float));
     bool const   have_tables = tables.holds_tables && tables_fit(tables, 2 * v_bytes);
     size_t const own_bytes   = align256((size_t)O * own_words * sizeof(uint32_t));
-    size_t const const_bytes = c.bn ? align256((size_t)O * sizeof(float4)) : 0;
+    size_t const const_bytes = c.bn ? align256((size_t)O * sizeof(NodeConsts)) : 0;
     size_t const part_bytes  = slab_count > 1 ? align256((size_t)slab_count * slab_bytes) : 0;
     size_t const bits_bytes  = (from_fp32 && !have_bits) ? align256((size_t)c.input_node_size * c.x_stride * sizeof(uint32_t)) : 0;
     char *base = nullptr;
     if (arena_get(v_bytes + own_bytes + const_bytes + part_bytes + bits_bytes, &base, st)) { return 1; }
     float    *V      = reinterpret_cast<float *>(base);
     uint32_t *own    = reinterpret_cast<uint32_t *>(base + v_bytes);
-    float4   *consts = reinterpret_cast<float4 *>(base + v_bytes + own_bytes);
+    NodeConsts *consts = reinterpret_cast<NodeConsts *>(base + v_bytes + own_bytes);
     float    *part   = reinterpret_cast<float *>(base + v_bytes + own_bytes + const_bytes);
     uint32_t *bits   = reinterpret_cast<uint32_t *>(base + v_bytes + own_bytes + const_bytes + part_bytes);
     if (have_tables) { V = reinterpret_cast<float *>(reinterpret_cast<char *>(tables.buf) + v_bytes); }
@@ -740,6 +741,8 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     int quads = (O <= 512) ? 4 : (O <= 1024) ? 2 : 1;
     while (quads > 1 && (long long)ceil_div(c.frame_size, quads * 256) * ceil_div(c.input_node_size, kWavesPerBlk) < 2048) { quads /= 2; }
     if (quads_env == 1 || quads_env == 2 || quads_env == 4) { quads = quads_env; }
+    t.far = !s.dy_quads || (long long)O * c.frame_stride * 4 > 0xffffffffLL || (long long)O * own_words * 4 > 0xffffffffLL;
+    if (t.far) { quads = 1; }
     DxArgs &d = t.dx;
     d.dy = c.dy; d.dx = c.dx; d.rev = c.rev; d.rev_stride = c.rev_stride; d.input_node_size = c.input_node_size; d.frame_size = c.frame_size;
     d.dy_stride = c.frame_stride; d.dx_stride = c.frame_stride;
@@ -748,10 +751,8 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     int const in_tiles = split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
     if ((long long)d.chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
     d.tiles = make_tile_divisor(in_tiles); d.split = split ? 1 : 0;
-    t.dy_quads = s.dy_quads;
     t.dx_quads = (c.frame_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(c.dx) & 15u) == 0) ? 1 : 0;
-    t.own = own; t.own_stride = own_words; t.V = V; t.node_consts = consts;
-    t.gamma = c.gamma; t.beta = c.beta; t.inv_step = 1.0f / (s.fold.hi - s.fold.lo);
+    t.own = own; t.own_stride = own_words; t.node_size = O; t.V = V; t.node_consts = consts; t.inv_step = 1.0f / (s.fold.hi - s.fold.lo);
     return c.bn ? dispatch_dx_table<N, true>(quads, t, st) : dispatch_dx_table<N, false>(quads, t, st);
 }
 

@@ -26,8 +26,12 @@ struct CornerFoldArgs {
     float lo, hi;                       // the two input values, 1/2 -+ bias
     float *dW;
     int   overwrite;                    // dW = instead of dW +=
-    float4 *node_consts;                // batch-norm: mean, rstd, shift, scale of each node, for the dx kernel
+    struct NodeConsts *node_consts;     // batch-norm: what the dx kernel needs of each node beside its corner values
 };
+
+// A[p] and B[p] of the dx kernel are, for a connection with difference d[p] = V[input at hi] - V[input at lo],
+//     A[p] = open[p] ? d[p] gain : 0,     B[p] = d[p] (shift + (V[p] - mean) scale)            (gain, shift, scale divided by hi - lo)
+struct __align__(32) NodeConsts { float mean, gain, shift, scale; uint64_t open; uint64_t unused; };
 
 // Lane p (of every group of 2^N lanes) holds the node's V[p], D[p], n[p]: the node's table gradient and, with batch-norm, its constants
 // (mean, rstd and the entry of dW that the gradient adds to: loaded by the caller, long before)
@@ -54,7 +58,9 @@ __device__ __forceinline__ void corner_fold(CornerFoldArgs const &a, CornerFoldI
         float const shift = -(a.gamma * s0) * rstd * a.inv_frames;
         float const scale = -(a.gamma * s1) * (rstd * rstd) * rstd * a.inv_frames;
         G = __builtin_fmaf(g, a.gamma * rstd, n * __builtin_fmaf(v - mean, scale, shift));
-        if (lane == 0) { a.node_consts[node] = make_float4(mean, rstd, shift, scale); }
+        uint64_t const open = __ballot(!(t <= 0.0f || t >= 1.0f));
+        float const inv_step = 1.0f / (a.hi - a.lo);
+        if (lane == 0) { a.node_consts[node] = NodeConsts{mean, a.gamma * rstd * inv_step, shift * inv_step, scale * inv_step, open, 0}; }
     }
     // per input: (G0, G1) -> ((1 - lo) G0 + (1 - hi) G1, lo G0 + hi G1), and 1 - lo = hi: either lane keeps hi of its own and takes lo of the other's
 #pragma unroll
@@ -331,22 +337,28 @@ struct DxTableArgs {
     DxArgs dx;                          // units, work lists, split mode and rows as in lut_dx_kernel (no term table, no rider)
     uint32_t const *own;                // kept corner indices, a byte per frame, rows of own_stride words
     int   own_stride;
-    int   dy_quads, dx_quads;           // rows hold whole groups of four frames (dx: 16-byte aligned as well)
+    int   node_size;
+    int   far;                          // see lut_dx_table_kernel
+    int   dx_quads;                     // rows of dx start on 16 bytes
     float const *V;                     // [O][2^N]
-    float4 const *node_consts;          // batch-norm: mean, rstd, shift, scale
-    float gamma, beta, inv_step;        // inv_step = 1 / (hi - lo)
+    NodeConsts const *node_consts;      // batch-norm
+    float inv_step;                     // 1 / (hi - lo)
 };
 
 // Input-centric dx over kept corner indices.  One wavefront owns dx[input][256 Q frames], four consecutive frames per lane and quad, and walks the
 // input's consumers in the reverse table's order (split mode: a quarter of them).  A consumer's term of a frame at corner p is  A[p] dy + B[p]  with
 //     A[p] = dV/dx_k[p] open[p] gamma rstd,   B[p] = dV/dx_k[p] E[p]           (plain layers: A = dV/dx_k, B = 0),
 // and y is linear in input k, so dV/dx_k[p] = (V[k at hi] - V[k at lo]) / (hi - lo): lane p computes entry p from the node's 2^N corner values
-// and four constants (272 bytes per node that all its consumers share), the wavefront puts the table into LDS, and the frames fetch their
+// and its constants (288 bytes per node that all its consumers share), the wavefront puts the table into LDS, and the frames fetch their
 // entry from there: a random 8-byte LDS read takes 4.5 clocks per CU and step where two ds_bpermute take 14.  Per term and pass one vector load
 // of V, Q of indices and Q of dy; the next term's are in flight while a term is evaluated.
-// Measured against the kernel that formed the indices from the packed rows: 27 inputs x 216 nodes x 230400 frames (Q = 2) 90 us instead of 117,
-// 4096 x 4096 x 8192 (Q = 1; 2: 142, 4: 162) 117 us instead of 138, where an XCD's L2 just holds what the chunk's passes gather from.
-template <int N, bool BN, int Q>
+// The kernel is bound by vector instructions (4 per element and about 20 per term) and by what its L2 delivers: rows are addressed by a 32-bit
+// offset into the whole buffer, dy by one 16-byte load per lane and quad, and a lane past the last frame reads whatever lies there.
+// FAR: buffers of 4 GiB and more, and rows of dy that do not hold whole groups of four: a descriptor per row, single words.
+// Measured against the kernel that formed the indices from the packed rows: 27 inputs x 216 nodes x 230400 frames (Q = 2) 85 us instead of 117;
+// 4096 x 4096 x 8192 (Q = 1) 108 us instead of 138: 745 MB of L2 misses at 6.9 TB/s.  Half as many frames per wavefront miss 479 MB, but the walk's
+// scalar instructions and loads per term then take 144 us; four terms in flight and constants by vector loads were slower at every Q.
+template <int N, bool BN, int Q, bool FAR = false>
 __global__ __launch_bounds__(kBlock) void lut_dx_table_kernel(DxTableArgs t)
 {
     constexpr int NN = 1 << N, kPass = 4 * kWave * Q;
@@ -364,75 +376,85 @@ __global__ __launch_bounds__(kBlock) void lut_dx_table_kernel(DxTableArgs t)
     int const lane = threadIdx.x & (kWave - 1);
 
     typedef __attribute__((address_space(4))) int const const_int;
-    typedef __attribute__((address_space(4))) float const const_float;
+    typedef __attribute__((address_space(4))) NodeConsts const const_consts;
     const_int *list = (const_int *)(a.rev + (size_t)in * a.rev_stride);
+    const_consts *consts = (const_consts *)t.node_consts;
     int t_begin, t_end;
     dx_list_range(list[0], share, t_begin, t_end);
     list += 1;
-    bool const dy_quads = t.dy_quads != 0;
-    uint32_t const y_row_bytes = quad_row_bytes(a.frame_size, dy_quads), i_row_bytes = (uint32_t)t.own_stride * 4u;
-    int const f_begin = ck * kPass, f_lane = f_begin + 4 * lane;
+    int const f_lane = ck * kPass + 4 * lane;
+    uint32_t const dy_bytes = (uint32_t)(t.node_size - 1) * (uint32_t)a.dy_stride * 4u + quad_row_bytes(a.frame_size, true);
+    __amdgpu_buffer_rsrc_t const dyr = row_descriptor(a.dy, 0, 0, FAR ? 0u : dy_bytes);
+    __amdgpu_buffer_rsrc_t const ir  = row_descriptor(t.own, 0, 0, FAR ? 0u : (uint32_t)t.node_size * (uint32_t)t.own_stride * 4u);
+    __amdgpu_buffer_rsrc_t const vr  = row_descriptor(t.V, 0, 0, (uint32_t)t.node_size * (NN * 4u));
 
     float4 acc[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) { acc[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f); }
 
-    uint32_t iw_next[Q];
-    float4 dy_next[Q];
-    float v_next = 0.0f, c_next[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    int k_next = 0, e_ahead = 0;
-    auto request = [&](int e) {
-        int const node = (int)((uint32_t)e / (uint32_t)N);
-        k_next = e - node * N;
-        __amdgpu_buffer_rsrc_t const ir  = row_descriptor(t.own, node, t.own_stride, i_row_bytes);
-        __amdgpu_buffer_rsrc_t const dyr = row_descriptor(a.dy, node, a.dy_stride, y_row_bytes);
-        v_next = t.V[(size_t)node * NN + (lane & (NN - 1))];
+    struct Stage { uint32_t iw[Q]; float4 dy[Q]; float v; float mean, gain, shift, scale; uint64_t open; int k; };
+    auto request = [&](int e, Stage &s) {
+        uint32_t const node = (uint32_t)e / (uint32_t)N;
+        s.k = e - (int)node * N;
+        s.v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(vr, (lane & (NN - 1)) * 4, node * (NN * 4u), 0));
         if (BN) {
-            const_float *c = (const_float *)(t.node_consts + node);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) { c_next[i] = c[i]; }
+            const_consts &c = consts[node];
+            s.mean = c.mean; s.gain = c.gain; s.shift = c.shift; s.scale = c.scale; s.open = c.open;
         }
+        __amdgpu_buffer_rsrc_t const i_row = FAR ? row_descriptor(t.own, (int)node, t.own_stride, (uint32_t)t.own_stride * 4u) : ir;
+        __amdgpu_buffer_rsrc_t const d_row = FAR ? row_descriptor(a.dy, (int)node, a.dy_stride, (uint32_t)a.frame_size * 4u) : dyr;
+        uint32_t const i_off = FAR ? 0u : node * (uint32_t)t.own_stride * 4u, d_off = FAR ? 0u : node * (uint32_t)a.dy_stride * 4u;
 #pragma unroll
-        for (int q = 0; q < Q; ++q) { iw_next[q] = __builtin_amdgcn_raw_buffer_load_b32(ir, (uint32_t)(f_lane + q * 4 * kWave), 0, 0); }
+        for (int q = 0; q < Q; ++q) { s.iw[q] = __builtin_amdgcn_raw_buffer_load_b32(i_row, (uint32_t)(f_lane + q * 4 * kWave), i_off, 0); }
 #pragma unroll
-        for (int q = 0; q < Q; ++q) { dy_next[q] = load_quad(dyr, (uint32_t)(f_lane + q * 4 * kWave) * 4u, dy_quads); }
+        for (int q = 0; q < Q; ++q) {
+            if constexpr (FAR) { s.dy[q] = load_quad(d_row, (uint32_t)(f_lane + q * 4 * kWave) * 4u, false); continue; }
+            auto const d = __builtin_amdgcn_raw_buffer_load_b128(d_row, (uint32_t)(f_lane + q * 4 * kWave) * 4u, d_off, 0);
+            s.dy[q] = make_float4(__uint_as_float(d[0]), __uint_as_float(d[1]), __uint_as_float(d[2]), __uint_as_float(d[3]));
+        }
     };
-    if (t_begin < t_end) {
-        request(list[t_begin]);
-        if (t_begin + 1 < t_end) { e_ahead = list[t_begin + 1]; }
-    }
-    for (int i = t_begin; i < t_end; ++i) {
-        uint32_t iw[Q];
-        float4 dy[Q];
-#pragma unroll
-        for (int q = 0; q < Q; ++q) { iw[q] = iw_next[q]; dy[q] = dy_next[q]; }
-        float const v = v_next, mean = c_next[0], rstd = c_next[1], shift = c_next[2], scale = c_next[3];
-        int const k = k_next;
-        if (i + 1 < t_end) {
-            request(e_ahead);
-            if (i + 2 < t_end) { e_ahead = list[i + 2]; }
-        }
-        float const other = __shfl_xor(v, 1 << k, 64);
-        float const slope = (((lane >> k) & 1) ? (v - other) : (other - v)) * t.inv_step;
-        Entry *const tab = table[wave][i & 1];
+    auto add = [&](Stage const &s, Entry *tab) {
+        float const other = __int_as_float(__builtin_amdgcn_ds_bpermute((lane * 4) ^ (4 << s.k), __float_as_int(s.v)));
+        // V[k at hi] - V[k at lo]: the lane's own value minus the other's, negated where the lane holds the lower corner
+        float const d = __uint_as_float(__float_as_uint(s.v - other) ^ (((uint32_t)~lane << (31 - s.k)) & 0x80000000u));
         if constexpr (BN) {
-            float const y = batch_norm_output(v, mean, rstd, t.gamma, t.beta);
-            float const A = (y <= 0.0f || y >= 1.0f) ? 0.0f : slope * (t.gamma * rstd);
-            if (lane < NN) { tab[lane] = make_float2(A, slope * __builtin_fmaf(v - mean, scale, shift)); }
+            float const A = __builtin_amdgcn_inverse_ballot_w64(s.open) ? d * s.gain : 0.0f;
+            if (NN == kWave || lane < NN) { tab[lane] = make_float2(A, d * __builtin_fmaf(s.v - s.mean, s.scale, s.shift)); }
         }
-        else { if (lane < NN) { tab[lane] = slope; } }
+        else { if (NN == kWave || lane < NN) { tab[lane] = d * t.inv_step; } }
         wave_fence();
-        auto add = [&](float &sum, float d, uint32_t corner) {
+        auto one = [&](float &sum, float y, uint32_t corner) {
             Entry const e = tab[corner];
-            if constexpr (BN) { sum = __builtin_fmaf(d, e.x, sum + e.y); }
-            else              { sum = __builtin_fmaf(d, e, sum); }
+            if constexpr (BN) { sum = __builtin_fmaf(y, e.x, sum + e.y); }
+            else              { sum = __builtin_fmaf(y, e, sum); }
         };
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            add(acc[q].x, dy[q].x, iw[q] & 0xffu);
-            add(acc[q].y, dy[q].y, (iw[q] >> 8) & 0xffu);
-            add(acc[q].z, dy[q].z, (iw[q] >> 16) & 0xffu);
-            add(acc[q].w, dy[q].w, iw[q] >> 24);
+            one(acc[q].x, s.dy[q].x, s.iw[q] & 0xffu);
+            one(acc[q].y, s.dy[q].y, (s.iw[q] >> 8) & 0xffu);
+            one(acc[q].z, s.dy[q].z, (s.iw[q] >> 16) & 0xffu);
+            one(acc[q].w, s.dy[q].w, s.iw[q] >> 24);
+        }
+    };
+    // two stages in turn; the list is read a term ahead of the requests
+    Stage s0, s1;
+    int e_ahead = 0;
+    if (t_begin < t_end) {
+        request(list[t_begin], s0);
+        e_ahead = list[min(t_begin + 1, t_end - 1)];
+    }
+    for (int i = t_begin; i < t_end; i += 2) {
+        if (i + 1 < t_end) {
+            request(e_ahead, s1);
+            e_ahead = list[min(i + 2, t_end - 1)];
+        }
+        add(s0, table[wave][0]);
+        if (i + 1 < t_end) {
+            if (i + 2 < t_end) {
+                request(e_ahead, s0);
+                e_ahead = list[min(i + 3, t_end - 1)];
+            }
+            add(s1, table[wave][1]);
         }
     }
 
