@@ -14,6 +14,7 @@
 
 #include "../../include/bbhip.h"
 #include "lut_kernels.hpp"
+#include "corner_forward_kernels.hpp"
 #include "corner_backward_kernels.hpp"
 #include "vector_kernels.hpp"
 #include "conv_kernels.hpp"
@@ -259,6 +260,15 @@ void launch_forward(FwdArgs const &a, int npw, hipStream_t st)
     if constexpr (XMODE == kXBit || XMODE == kXBinary) {
         // two-valued inputs: the corner-value kernel wherever the caller prepared the values (one node per wavefront)
         if (a.V != nullptr) {
+            if constexpr (KIND != 3 && (XMODE == kXBit || (YMODE == kYBinarize && KIND == 1))) {
+                if (a.node_waves > 0) {
+                    bool const fused = (KIND == 1) && a.stat_mode == kStatInline;
+                    int const waves = a.node_waves > kWavesPerBlk ? a.node_waves : kWavesPerBlk;
+                    int const index_blocks = fused ? waves / a.node_waves * ceil_div(a.frame_size, kByteBlock) : waves;
+                    hipLaunchKernelGGL((lut_forward_bytes_kernel<N, XMODE, YMODE, KIND>), grid, dim3(waves * kWave), forward_bytes_lds(waves, index_blocks), st, a);
+                    return;
+                }
+            }
             if constexpr (XMODE == kXBit && YMODE == kYBinarize && KIND == 1) {
                 if (a.own_index != nullptr) {      // corner indices kept by the statistics launch of the same call
                     hipLaunchKernelGGL((lut_forward_corner_kernel<N, XMODE, YMODE, KIND, false, kOwnMemory>), grid, block, 0, st, a);
@@ -460,12 +470,22 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
     if (bits_wanted) { c.xmode = kXBit; c.x_stride = to_caller ? packed.row_words : packed_row_words(c.frame_size); c.x = have_bits ? packed.bits : nullptr; }
     bool const corner     = use_corner_values(c.xmode);
     int const npw         = corner ? 1 : fwd_nodes_per_wave();
-    int const tile_count  = ceil_div(c.node_size, kWavesPerBlk * npw);
-    // Batch-norm training pass of a small batch on the corner-value kernel: one unit per node, so that the wavefront that writes a
-    // node's output can sum the node's statistics itself (kStatInline) and the statistics launch falls away — at up to 1024 frames
-    // a launch costs more than the second evaluation of the unit does.  BBHIP_FWD_CHUNK set in the environment keeps its say.
-    bool const one_unit   = (c.bn == 1) && corner && c.frame_size <= 1024 && fwd_chunk_frames_env() == 0;
-    int const chunk       = one_unit ? 1024 : fwd_chunk_frames(c.xmode, c.frame_size, tile_count);
+    // Two-valued inputs from 1025 frames: the kernel that forms the corner indices of 32 frames per lane at a time (below that most of its lanes
+    // have no frames: 11.2 us instead of 9.6 for 6144 nodes x 1024 frames, 5.3 instead of 4.0 for 1024 x 64).  A batch-norm training pass is one
+    // launch of it while the indices of a node's frames fit in LDS.  fp32 frames whose row count nobody told come along, gathered, while
+    // there is little to gather: a launch over all frames at a time loses the order in which the L2s hold pieces of large inputs.
+    bool const byte_bits  = corner && c.xmode == kXBit && c.frame_size > 1024;
+    bool const byte_fused = (c.bn == 1) && corner && c.frame_size > 1024 && c.frame_size <= kByteFusedFrames && fwd_chunk_frames_env() == 0 &&
+                            (byte_bits || (fixed == nullptr && (long long)c.node_size * c.frame_size <= (1 << 21)));
+    // wavefronts per node: a block of 2048 frames for each, up to a workgroup
+    int node_waves = (byte_bits || byte_fused) ? 1 : 0;
+    while (byte_fused && node_waves < kByteWaves && node_waves * kByteBlock < c.frame_size) { node_waves *= 2; }
+    int const tile_count  = ceil_div(c.node_size, node_waves > 1 ? (node_waves < kWavesPerBlk ? kWavesPerBlk / node_waves : 1) : kWavesPerBlk * npw);
+    // Batch-norm training pass of a small batch on the corner-value kernels: one unit per node, so that the wavefronts that write a
+    // node's output can sum the node's statistics themselves (kStatInline) and the statistics launch falls away.  BBHIP_FWD_CHUNK set in the environment keeps its say.
+    bool const one_unit   = byte_fused || ((c.bn == 1) && corner && c.frame_size <= 1024 && fwd_chunk_frames_env() == 0);
+    int const chunk       = byte_fused ? ceil_div(c.frame_size, kByteBlock) * kByteBlock : one_unit ? 1024 :
+                            (byte_bits && fwd_chunk_frames_env() == 0) ? kByteBlock : fwd_chunk_frames(c.xmode, c.frame_size, tile_count);
     int const chunk_count = ceil_div(c.frame_size, chunk);
     if ((long long)chunk_count * tile_count > 0x7fffffffLL) { return fail("forward: grid too large"); }
 
@@ -521,11 +541,12 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
     a.chunk = chunk; a.chunk_count = chunk_count; a.tiles = make_tile_divisor(tile_count);
     a.bias = c.bias; a.gamma = c.gamma; a.beta = c.beta;
     a.zero_padding = c.zero_padding;
+    a.node_waves = node_waves;
+    a.y_quads = (c.y_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(c.y) & 15u) == 0) ? 1 : 0;
 
     int kind = 0;
     if (c.bn == 1 && corner && chunk_count == 1) {
-        // one unit per node and the cheap corner-value kernel: its wavefronts sum the statistics of their node themselves
-        // before they write its output, which saves the statistics launch (the evaluation it repeats costs less than that)
+        // one unit per node on a corner-value kernel: its wavefronts sum the statistics of their node themselves before they write its output
         a.stat_mode = kStatInline; a.momentum = c.momentum;
         a.mean_out = c.mean; a.rstd_out = c.rstd; a.running_mean = c.running_mean; a.running_var = c.running_var;
         kind = 1;

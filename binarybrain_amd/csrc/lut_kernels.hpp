@@ -241,6 +241,9 @@ struct FwdArgs {
     int   own_stride;
     // kStatPartial: units per node of the launch that left the partial sums, where the output launch has other units (0: the same)
     int   stat_units;
+    // lut_forward_bytes_kernel (node_waves > 0 where a call takes it): wavefronts that share a node in a one-launch training pass, and whether
+    // rows of fp32 output start on 16 bytes
+    int   node_waves, y_quads;
     int   zero_padding;         // packed output: the wavefront of a node's last unit writes 0 behind the last frame's word, up to the row pitch
 };
 
