@@ -16,6 +16,7 @@
 #include "lut_kernels.hpp"
 #include "corner_forward_kernels.hpp"
 #include "corner_backward_kernels.hpp"
+#include "table_gradient_kernels.hpp"
 #include "vector_kernels.hpp"
 #include "conv_kernels.hpp"
 #include "tail_kernels.hpp"
@@ -449,6 +450,36 @@ int launch_pack_and_prep(float const *x, int x_stride, uint32_t *bits, int bit_s
     return 0;
 }
 
+// Layers on real-valued inputs that are bound by latency and launches and not by how they gather rows: all frames of a node at a time
+// (lut_forward_node_kernel, lut_node_gradient_kernel) cost less than the launches that this saves.  Beyond, the kernels that take the frames in pieces
+// keep the gathered rows in L2: training step of 2048 nodes x 2048 frames 93 us node by node, 98 in pieces; 1000 x 3000 81 and 73; 100 x 4000 25 and 31.
+bool small_real_layer(int node_size, int frame_size)
+{
+    return frame_size <= kNodeWaves * kNodeSteps * kWave && (long long)node_size * frame_size <= (frame_size <= 2048 ? 1 << 22 : 1 << 19);
+}
+int real_node_waves(int frame_size) { return ceil_div(frame_size, kNodeSteps * kWave); }
+int real_nodes_per_block(int node_waves) { return ceil_div(kWavesPerBlk, node_waves); }       // (at least four wavefronts: the term table rides along)
+
+template <int N>
+int run_forward_real_node(ForwardCall const &c, hipStream_t st, PreparedTablesHint tables)
+{
+    FwdArgs a{};
+    a.x = c.x; a.y = c.y; a.idx = c.idx; a.node_size = c.node_size; a.frame_size = c.frame_size; a.x_stride = c.x_stride; a.y_stride = c.y_stride;
+    a.gamma = c.gamma; a.beta = c.beta; a.momentum = c.momentum;
+    a.mean_out = c.mean; a.rstd_out = c.rstd; a.running_mean = c.running_mean; a.running_var = c.running_var;
+    a.W_inline = c.W; a.lut_binarize = c.lut_binarize; a.clamp_W = c.clamp_W; a.clamp_lo = c.clamp_lo; a.clamp_hi = c.clamp_hi;
+    if (tables_fit(tables, align256((size_t)c.node_size * (1 << N) * sizeof(float)))) { a.C_out = tables.buf; }
+    a.node_waves = real_node_waves(c.frame_size);
+    int const per_block = real_nodes_per_block(a.node_waves);
+    a.tiles = make_tile_divisor(ceil_div(c.node_size, per_block));
+    {
+        ScopedTimer tm(kTimeForward, st);
+        hipLaunchKernelGGL(lut_forward_node_kernel<N>, dim3(a.tiles.count), dim3(per_block * a.node_waves * kWave), 0, st, a);
+    }
+    BBHIP_LAUNCH_CHECK();
+    return 0;
+}
+
 template <int N>
 int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch const *fixed = nullptr,
                 PackedInputHint packed = PackedInputHint{nullptr, 0, 0, 0}, PreparedTablesHint tables = PreparedTablesHint{nullptr, 0, 0},
@@ -469,6 +500,9 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
     bool const pack = bits_wanted && !have_bits;
     if (bits_wanted) { c.xmode = kXBit; c.x_stride = to_caller ? packed.row_words : packed_row_words(c.frame_size); c.x = have_bits ? packed.bits : nullptr; }
     bool const corner     = use_corner_values(c.xmode);
+    if (c.bn == 1 && c.xmode == kXClamp && c.ymode == kYClamp && small_real_layer(c.node_size, c.frame_size) && fwd_chunk_frames_env() == 0) {
+        return run_forward_real_node<N>(c, st, tables);
+    }
     int const npw         = corner ? 1 : fwd_nodes_per_wave();
     // Two-valued inputs from 1025 frames: the kernel that forms the corner indices of 32 frames per lane at a time (below that most of its lanes
     // have no frames: 11.2 us instead of 9.6 for 6144 nodes x 1024 frames, 5.3 instead of 4.0 for 1024 x 64).  A batch-norm training pass is one
@@ -778,6 +812,20 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
 }
 
 template <int N>
+void launch_node_gradient(BackwardCall const &c, BwdArgs const &a, float const *C, float *dyh, int overwrite, hipStream_t st)
+{
+    NodeGradientArgs g{};
+    g.x = c.x; g.dy = c.dy; g.idx = c.idx; g.node_size = c.output_node_size; g.frame_size = c.frame_size;
+    g.x_stride = c.x_stride; g.dy_stride = c.frame_stride; g.dW = c.dW; g.overwrite = overwrite; g.tt = a.tt;
+    g.W = c.W; g.C = C; g.lut_binarize = c.lut_binarize;
+    g.mean = c.mean; g.rstd = c.rstd; g.gamma = c.gamma; g.beta = c.beta; g.inv_frames = a.inv_frames;
+    g.dyh = dyh; g.dyh_stride = c.frame_stride; g.node_waves = real_node_waves(c.frame_size);
+    int const per_block = real_nodes_per_block(g.node_waves);
+    g.node_tiles = ceil_div(c.output_node_size, per_block);
+    hipLaunchKernelGGL(lut_node_gradient_kernel<N>, dim3(g.tt.blocks + g.node_tiles), dim3(per_block * g.node_waves * kWave), 0, st, g);
+}
+
+template <int N>
 int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packed = PackedInputHint{nullptr, 0, 0, 0},
                  PreparedTablesHint tables = PreparedTablesHint{nullptr, 0, 0}, int dw_overwrite = 0)
 {
@@ -820,6 +868,9 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         slab = 4096;
         for (int cand = 2048; cand >= 256; cand /= 2) { if (cost(cand) < cost(slab)) { slab = cand; } }
     }
+    // small layers on real-valued inputs: statistics, table gradient and all in one launch ahead of the dx kernel
+    bool const node_launch = dxmode == kDxNone && c.bn && c.xmode == kXClamp && bwd_slab_frames() == 0 && small_real_layer(c.output_node_size, c.frame_size);
+    if (node_launch) { slab = ceil_div(c.frame_size, kWave) * kWave; }
     for (;;) {
         long long slabs = (long long)range_count * ceil_div(range, slab);
         if (slabs * c.output_node_size * NN * (long long)sizeof(float) <= (256LL << 20) || slab >= range) { break; }
@@ -861,7 +912,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         C = tables.buf;
         V = corner ? reinterpret_cast<float *>(reinterpret_cast<char *>(tables.buf) + c_bytes) : nullptr;
     }
-    bool const prep = (c.bn || dxmode != kDxNone) && !have_tables;
+    bool const prep = (c.bn || dxmode != kDxNone) && !have_tables && !node_launch;
     if (prep) {
         launch_table_prep<N>(c.W, C, c.output_node_size, c.lut_binarize, st, V, c.bias);
         BBHIP_LAUNCH_CHECK();
@@ -888,7 +939,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
     a.slab = slab; a.tiles = make_tile_divisor(tile_count);
     a.bias = c.bias; a.gamma = c.gamma; a.beta = c.beta; a.inv_frames = 1.0f / (float)c.frame_size;
 
-    if (c.bn) {
+    if (c.bn && !node_launch) {
         // phase 0: per-node sums over ALL frames, then dmean / dvar.  It only recomputes the LUT output, so it runs in the
         // forward kernel (kind 3): frame chunks that keep the gathered rows in L2, partial sums from the matrix unit
         int const npw = stat_npw;
@@ -931,7 +982,8 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         a.tt = (r == 0) ? tt : TermArgs{};
         {
             ScopedTimer tm(kTimeBackward, st);
-            if (dispatch_backward<N>(c.xmode, c.bn ? 1 : 0, dxmode, a, st)) { return 1; }
+            if (node_launch) { launch_node_gradient<N>(c, a, have_tables ? C : nullptr, dyh, dw_overwrite, st); }
+            else if (dispatch_backward<N>(c.xmode, c.bn ? 1 : 0, dxmode, a, st)) { return 1; }
         }
         BBHIP_LAUNCH_CHECK();
         if (dxmode == kDxTmp) {
@@ -961,7 +1013,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         // folding the slab sums into dW rides at the end of this launch
         d.fin_partial = part; d.fin_dW = c.dW; d.fin_node_size = c.output_node_size; d.fin_slab_count = slab_total;
         d.fin_overwrite = dw_overwrite;
-        d.fin_blocks = (ceil_div(c.output_node_size * NN, kBlock) + 7) & ~7;
+        d.fin_blocks = !node_launch ? (ceil_div(c.output_node_size * NN, kBlock) + 7) & ~7 : 0;      // (lut_node_gradient_kernel adds to dW itself)
         if ((long long)d.fin_blocks + (long long)chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
         {
             ScopedTimer tm(kTimeDx, st);

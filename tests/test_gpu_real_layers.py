@@ -1,0 +1,44 @@
+"""GPU parity of batch-norm training over real-valued inputs where one launch takes all frames of a node, at its edges: wavefront steps, wavefronts
+per node, the largest calls that it serves and the first that go to the kernels beyond."""
+import numpy as np
+import pytest
+
+import oracle
+from binarybrain_amd import synth
+from util import assert_bwd, assert_fwd, dev, host
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(9, 5, 3), (16, 9, 64), (7, 33, 65), (40, 6, 256), (12, 13, 257), (30, 3, 511), (8, 70, 513), (10, 7, 1025), (50, 21, 2048), (6, 5, 2049), (9, 4, 4096),
+          (11, 3, 4097)]
+
+
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 6])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_real_valued_training(n, shape):
+    import torch
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    I, O, F = shape
+    rng = np.random.default_rng(100 * n + F)
+    stride = synth.frame_stride_fp32(F)
+    idx = synth.wiring(rng, I, O, n); W = synth.lut_tables(rng, O, n)
+    x = synth.uniform_frames(rng, I, F, stride, -0.1, 1.1); dy = synth.normal_frames(rng, O, F, stride)
+    y_ref, mean, rstd, rm_ref, rv_ref = oracle.differentiable_lut_forward_training(n, x, idx, W, F, np.zeros(O, np.float32), np.ones(O, np.float32), binary_mode=False)
+    x[:, F:] = np.nan; dy[:, F:] = np.nan           # what lies behind the frames enters nothing
+    d_x, d_dy, d_idx, d_W = dev(x), dev(dy), dev(idx), dev(W)
+    rev = ops.reverse_table(d_idx, I)
+    got = []
+    for tables in (None, ops.prepared_tables_buffer(n, O)):
+        rm, rv = torch.zeros(O, device="cuda"), torch.ones(O, device="cuda")
+        y, m, r = ops.differentiable_lut_forward_training(n, d_x, d_idx, d_W, F, rm, rv, binary_mode=False, clamp_w=(-9.0, 9.0), tables=tables)
+        assert np.allclose(host(m), mean, rtol=1e-4, atol=1e-6) and np.allclose(host(r), rstd, rtol=1e-3)
+        assert np.allclose(host(rm), rm_ref, rtol=1e-4, atol=1e-6) and np.allclose(host(rv), rv_ref, rtol=1e-3)
+        assert np.abs(host(y)[:, :F] - y_ref[:, :F]).max() <= 2e-4
+        dx_ref, dW_ref = oracle.differentiable_lut_backward(n, x, dy, idx, W, F, mean, rstd, binary_mode=False)
+        dW = torch.full((O, 1 << n), 0.25, device="cuda")
+        dx = ops.differentiable_lut_backward(n, d_x, d_dy, d_idx, d_W, dW, F, dev(mean), dev(rstd), rev, binary_mode=False, tables=tables)
+        if F > 4:                                   # (the gradient through the statistics of a frame or two is rounding alone)
+            assert_bwd(host(dx)[:, :F], dx_ref[:, :F], "dx"); assert_bwd(host(dW) - 0.25, dW_ref, "dW")
+        got.append((host(y)[:, :F], host(m), host(dx)[:, :F], host(dW)))
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
