@@ -173,13 +173,17 @@ int bwd_slab_frames(void)  { static int v = env_int("BBHIP_BWD_SLAB", 0);  retur
 // per-term set-up per frame.  0: not set in the environment.
 int dx_chunk_frames_env(void) { static int v = env_int("BBHIP_DX_CHUNK", 0); return ((v + 63) / 64) * 64; }
 int dx_pass_steps_env(void)   { static int v = env_int("BBHIP_DX_STEPS", 0); return (v <= 0) ? 0 : (v <= 1) ? 1 : (v <= 2) ? 2 : 4; }
-// dx work lists split over the four wavefronts of a workgroup (DxArgs::split): where one wavefront per (input node, unit) would
-// leave the launch with fewer than 4096 workgroups and the lists are long enough to share.  BBHIP_DX_SPLIT = 0 / 1 forces it.
-bool dx_split_lists(int max_fan, long long workgroups)
+// Wavefronts that share an input's work list in the dx kernels (DxArgs::split), 0 = none: four where one wavefront per (input node, unit) would
+// leave the launch with fewer than 4096 workgroups and the lists are long enough to share, sixteen where with four the launch
+// would still have less than two wavefronts per SIMD (not where the rows of dy outgrow the L2s: the wavefronts of a launch then walk the nodes together,
+// and sixteen places in the lists at a time cost 6 % at 40 inputs, 8000 nodes, 4000 frames).  BBHIP_DX_SPLIT = 0 / 1 forces none / four.
+// Measured: training step of 59 inputs x 1594 nodes x 27 frames 30.0 -> 18.9 us, 50 x 3000 x 200 (StochasticLut4) 39.3 -> 22.3 us.
+int dx_split_lists(int max_fan, int input_node_size, int node_size, int frame_size, int chunk_count)
 {
     static int const env = env_int("BBHIP_DX_SPLIT", 2);
-    if (env == 0 || env == 1) { return env == 1; }
-    return max_fan >= 16 && workgroups < 4096;
+    if (env == 0 || env == 1) { return env * kWavesPerBlk; }
+    if (max_fan < 16 || (long long)chunk_count * ((input_node_size + kWavesPerBlk - 1) / kWavesPerBlk) >= 4096) { return 0; }
+    return (max_fan >= 32 && (long long)chunk_count * input_node_size < 1024 && (long long)node_size * frame_size <= (1 << 22)) ? kDxWaves : kWavesPerBlk;
 }
 // BinaryLut6 units of 128 words: 8192 input rows x 512 bytes is what an XCD's 4 MiB L2 holds (1.2 GB fetched per launch at
 // the benchmark shape; 192-word units fetch 1.9 GB, 256-word units 2.3 GB).  With the per-wavefront set-up at its
@@ -337,12 +341,15 @@ int dispatch_backward(int xmode, int kind, int dxmode, BwdArgs const &a, hipStre
 template <int N, int U>
 int dispatch_dx_u(int xmode, DxArgs const &a, hipStream_t st)
 {
-    dim3 const grid(a.fin_blocks + a.chunk_count * a.tiles.count), block(kBlock);
-    switch (xmode) {
-    case kXClamp:  hipLaunchKernelGGL((lut_dx_kernel<N, kXClamp, U>),  grid, block, 0, st, a); return 0;
-    case kXBinary: hipLaunchKernelGGL((lut_dx_kernel<N, kXBinary, U>), grid, block, 0, st, a); return 0;
-    case kXBit:    hipLaunchKernelGGL((lut_dx_kernel<N, kXBit, U>),    grid, block, 0, st, a); return 0;
+    dim3 const grid(a.fin_blocks + a.chunk_count * a.tiles.count), block((a.split ? a.split : kWavesPerBlk) * kWave);
+#define BBHIP_DX_CASE(X)                                                                                                       \
+    if (xmode == X) {                                                                                                          \
+        if (a.split > kWavesPerBlk) { hipLaunchKernelGGL((lut_dx_kernel<N, X, U, kDxWaves>), grid, block, 0, st, a); }       \
+        else                        { hipLaunchKernelGGL((lut_dx_kernel<N, X, U, kWavesPerBlk>), grid, block, 0, st, a); }   \
+        return 0;                                                                                                              \
     }
+    BBHIP_DX_CASE(kXClamp) BBHIP_DX_CASE(kXBinary) BBHIP_DX_CASE(kXBit)
+#undef BBHIP_DX_CASE
     return fail("dx variant (x=%d) not built", xmode);
 }
 
@@ -720,14 +727,19 @@ int launch_corner_backward(CornerSumsArgs const &s, int slab_count, hipStream_t 
 template <int N, bool BN>
 int dispatch_dx_table(int quads, DxTableArgs const &t, hipStream_t st)
 {
-    dim3 const grid(t.dx.chunk_count * t.dx.tiles.count), block(kBlock);
+    int const waves = t.dx.split ? t.dx.split : kWavesPerBlk;
+    dim3 const grid(t.dx.chunk_count * t.dx.tiles.count), block(waves * kWave);
     ScopedTimer tm(kTimeDx, st);
-    if (t.far) { hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, 1, true>), grid, block, 0, st, t); }
-    else switch (quads) {
-    case 1:  hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, 1>), grid, block, 0, st, t); break;
-    case 2:  hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, 2>), grid, block, 0, st, t); break;
-    default: hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, 4>), grid, block, 0, st, t); break;
+#define BBHIP_DX_CASE(Q, FAR)                                                                                                                  \
+    {                                                                                                                                          \
+        if (waves > kWavesPerBlk) { hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, Q, kDxWaves, FAR>), grid, block, 0, st, t); }             \
+        else                      { hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, Q, kWavesPerBlk, FAR>), grid, block, 0, st, t); }         \
     }
+    if (t.far)           BBHIP_DX_CASE(1, true)
+    else if (quads == 1) BBHIP_DX_CASE(1, false)
+    else if (quads == 2) BBHIP_DX_CASE(2, false)
+    else                 BBHIP_DX_CASE(4, false)
+#undef BBHIP_DX_CASE
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -802,10 +814,10 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     d.dy = c.dy; d.dx = c.dx; d.rev = c.rev; d.rev_stride = c.rev_stride; d.input_node_size = c.input_node_size; d.frame_size = c.frame_size;
     d.dy_stride = c.frame_stride; d.dx_stride = c.frame_stride;
     d.chunk = quads * 256; d.chunk_count = ceil_div(c.frame_size, d.chunk);
-    bool const split   = dx_split_lists(c.rev_stride - 1, (long long)d.chunk_count * ceil_div(c.input_node_size, kWavesPerBlk));
+    int const split    = dx_split_lists(c.rev_stride - 1, c.input_node_size, O, c.frame_size, d.chunk_count);
     int const in_tiles = split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
     if ((long long)d.chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
-    d.tiles = make_tile_divisor(in_tiles); d.split = split ? 1 : 0;
+    d.tiles = make_tile_divisor(in_tiles); d.split = split;
     t.dx_quads = (c.frame_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(c.dx) & 15u) == 0) ? 1 : 0;
     t.own = own; t.own_stride = own_words; t.node_size = O; t.V = V; t.node_consts = consts; t.inv_step = 1.0f / (s.fold.hi - s.fold.lo);
     return c.bn ? dispatch_dx_table<N, true>(quads, t, st) : dispatch_dx_table<N, false>(quads, t, st);
@@ -1000,8 +1012,8 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         int const frames = dx_chunk_frames_env() ? dx_chunk_frames_env() : 128;
         int const chunk  = ((frames + kWave * steps - 1) / (kWave * steps)) * (kWave * steps);
         int const chunk_count = ceil_div(c.frame_size, chunk);
-        // few input nodes with long work lists: the four wavefronts of a workgroup share one input node (DxArgs::split)
-        bool const split   = dx_split_lists(c.rev_stride - 1, (long long)chunk_count * ceil_div(c.input_node_size, kWavesPerBlk));
+        // few input nodes with long work lists: the wavefronts of a workgroup share one input node (DxArgs::split)
+        int const split    = dx_split_lists(c.rev_stride - 1, c.input_node_size, c.output_node_size, c.frame_size, chunk_count);
         int const in_tiles = split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
         if ((long long)chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
         DxArgs d{};
@@ -1009,7 +1021,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         d.rev_stride = c.rev_stride; d.input_node_size = c.input_node_size; d.frame_size = c.frame_size;
         d.x_stride = c.x_stride; d.dy_stride = c.frame_stride; d.dx_stride = c.frame_stride;
         d.chunk = chunk; d.chunk_count = chunk_count; d.tiles = make_tile_divisor(in_tiles);
-        d.bias = c.bias; d.split = split ? 1 : 0;
+        d.bias = c.bias; d.split = split;
         // folding the slab sums into dW rides at the end of this launch
         d.fin_partial = part; d.fin_dW = c.dW; d.fin_node_size = c.output_node_size; d.fin_slab_count = slab_total;
         d.fin_overwrite = dw_overwrite;

@@ -308,7 +308,7 @@ struct DxTableArgs {
 };
 
 // Input-centric dx over kept corner indices.  One wavefront owns dx[input][256 Q frames], four consecutive frames per lane and quad, and walks the
-// input's consumers in the reverse table's order (split mode: a quarter of them).  A consumer's term of a frame at corner p is  A[p] dy + B[p]  with
+// input's consumers in the reverse table's order (split mode: a part of them).  A consumer's term of a frame at corner p is  A[p] dy + B[p]  with
 //     A[p] = dV/dx_k[p] open[p] gamma rstd,   B[p] = dV/dx_k[p] E[p]           (plain layers: A = dV/dx_k, B = 0),
 // and y is linear in input k, so dV/dx_k[p] = (V[k at hi] - V[k at lo]) / (hi - lo): lane p computes entry p from the node's 2^N corner values
 // and its constants (288 bytes per node that all its consumers share), the wavefront puts the table into LDS, and the frames fetch their
@@ -320,8 +320,8 @@ struct DxTableArgs {
 // Measured against the kernel that formed the indices from the packed rows: 27 inputs x 216 nodes x 230400 frames (Q = 2) 85 us instead of 117;
 // 4096 x 4096 x 8192 (Q = 1) 108 us instead of 138: 745 MB of L2 misses at 6.9 TB/s.  Half as many frames per wavefront miss 479 MB, but the walk's
 // scalar instructions and loads per term then take 144 us; four terms in flight and constants by vector loads were slower at every Q.
-template <int N, bool BN, int Q, bool FAR = false>
-__global__ __launch_bounds__(kBlock) void lut_dx_table_kernel(DxTableArgs t)
+template <int N, bool BN, int Q, int WAVES, bool FAR = false>
+__global__ __launch_bounds__(WAVES * kWave) void lut_dx_table_kernel(DxTableArgs t)
 {
     constexpr int NN = 1 << N, kPass = 4 * kWave * Q;
     using Entry = std::conditional_t<BN, float2, float>;
@@ -329,8 +329,8 @@ __global__ __launch_bounds__(kBlock) void lut_dx_table_kernel(DxTableArgs t)
     int const lid = xcd_remap(blockIdx.x, a.chunk_count * a.tiles.count);
     int ck, tile;
     split_tile(lid, a.tiles, ck, tile);
-    __shared__ __align__(16) float4 part[kWavesPerBlk][Q][kWave];
-    __shared__ Entry table[kWavesPerBlk][2][NN];
+    __shared__ __align__(16) float4 part[WAVES][Q][kWave];
+    __shared__ Entry table[WAVES][2][NN];
     int const wave = threadIdx.x / kWave;
     int in, share;
     dx_list_share(a, tile, wave, in, share);
@@ -342,7 +342,7 @@ __global__ __launch_bounds__(kBlock) void lut_dx_table_kernel(DxTableArgs t)
     const_int *list = (const_int *)(a.rev + (size_t)in * a.rev_stride);
     const_consts *consts = (const_consts *)t.node_consts;
     int t_begin, t_end;
-    dx_list_range(list[0], share, t_begin, t_end);
+    dx_list_range<WAVES>(list[0], share, t_begin, t_end);
     list += 1;
     int const f_lane = ck * kPass + 4 * lane;
     uint32_t const dy_bytes = (uint32_t)(t.node_size - 1) * (uint32_t)a.dy_stride * 4u + quad_row_bytes(a.frame_size, true);
@@ -428,7 +428,7 @@ __global__ __launch_bounds__(kBlock) void lut_dx_table_kernel(DxTableArgs t)
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
 #pragma unroll
-            for (int w = 1; w < kWavesPerBlk; ++w) {
+            for (int w = 1; w < WAVES; ++w) {
                 float4 const o = part[w][q][lane];
                 acc[q].x += o.x; acc[q].y += o.y; acc[q].z += o.z; acc[q].w += o.w;
             }

@@ -1208,7 +1208,7 @@ struct DxArgs {
     int   chunk, chunk_count;
     TileDivisor tiles;
     float bias;
-    // split != 0: the four wavefronts of a workgroup share ONE input node and a quarter of its work list each; their sums are
+    // split != 0: the wavefronts of a workgroup share ONE input node and an equal part of its work list each; their sums are
     // added in wavefront order through LDS.  For layers with few input nodes and long lists (784 inputs feeding 6144 nodes:
     // 47 consumers each), where one wavefront per (input, unit) leaves most of the device idle behind a long serial walk.
     // tiles then counts input nodes, not groups of four.
@@ -1330,7 +1330,9 @@ struct DxTerm {
     }
 };
 
-// The wavefront's share of an input node's work list (the whole list, or a quarter of it in split mode) ...
+constexpr int kDxWaves = 16;                // wavefronts that share a work list where four are not enough
+
+// The wavefront's share of an input node's work list (the whole list, or its part in split mode) ...
 __device__ __forceinline__ void dx_list_share(DxArgs const &a, int tile, int wave, int &in, int &t_scale)
 {
     // (the wavefront's number within the workgroup is the same in all its lanes; saying so keeps everything derived from it —
@@ -1339,17 +1341,18 @@ __device__ __forceinline__ void dx_list_share(DxArgs const &a, int tile, int wav
     in      = __builtin_amdgcn_readfirstlane(a.split ? tile : tile * kWavesPerBlk + w);
     t_scale = a.split ? w : -1;
 }
+template <int WAVES>
 __device__ __forceinline__ void dx_list_range(int cnt, int share, int &t_begin, int &t_end)
 {
-    t_begin = (share < 0) ? 0   : (cnt * share) / kWavesPerBlk;
-    t_end   = (share < 0) ? cnt : (cnt * (share + 1)) / kWavesPerBlk;
+    t_begin = (share < 0) ? 0   : (cnt * share) / WAVES;
+    t_end   = (share < 0) ? cnt : (cnt * (share + 1)) / WAVES;
 }
 
 // ... and the end of a pass: the lane's U sums go to dx — directly, or in split mode added over the workgroup's wavefronts
 // in wavefront order (a fixed order: results do not depend on timing) by the first of them.  Every wavefront of the
 // workgroup must come here (the barrier).
-template <int U>
-__device__ __forceinline__ void dx_store_pass(DxArgs const &a, float (&part)[kWavesPerBlk][U][kWave], int in, int wave, int lane,
+template <int U, int WAVES>
+__device__ __forceinline__ void dx_store_pass(DxArgs const &a, float (&part)[WAVES][U][kWave], int in, int wave, int lane,
                                               int f_begin, float (&acc)[U])
 {
     if (a.split) {
@@ -1361,7 +1364,7 @@ __device__ __forceinline__ void dx_store_pass(DxArgs const &a, float (&part)[kWa
             for (int u = 0; u < U; ++u) {
                 float sum = part[0][u][lane];
 #pragma unroll
-                for (int w = 1; w < kWavesPerBlk; ++w) { sum += part[w][u][lane]; }
+                for (int w = 1; w < WAVES; ++w) { sum += part[w][u][lane]; }
                 acc[u] = sum;
             }
         }
@@ -1375,19 +1378,23 @@ __device__ __forceinline__ void dx_store_pass(DxArgs const &a, float (&part)[kWa
     }
 }
 
-template <int N, int XMODE, int U>
-__global__ __launch_bounds__(kBlock) void lut_dx_kernel(DxArgs a)
+// WAVES: wavefronts of a workgroup; kDxWaves: split mode
+template <int N, int XMODE, int U, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void lut_dx_kernel(DxArgs a)
 {
     using T = DxTerm<N, XMODE, U>;
     // the table-gradient partial sums are complete before this launch and independent of it: folding them into dW rides at
     // the end of this launch instead of taking a launch of its own
     int const bid = blockIdx.x;
     int const B   = a.chunk_count * a.tiles.count;
-    if (bid >= B) { dw_finalize_block<N>(a.fin_partial, a.fin_dW, a.fin_node_size, a.fin_slab_count, bid - B, a.fin_overwrite); return; }
+    if (bid >= B) {
+        if (WAVES == kWavesPerBlk || threadIdx.x < kBlock) { dw_finalize_block<N>(a.fin_partial, a.fin_dW, a.fin_node_size, a.fin_slab_count, bid - B, a.fin_overwrite); }
+        return;
+    }
     int const lid  = xcd_remap(bid, B);
     int ck, tile;
     split_tile(lid, a.tiles, ck, tile);
-    __shared__ float part[kWavesPerBlk][U][kWave];
+    __shared__ float part[WAVES][U][kWave];
     int const wave = threadIdx.x / kWave;
     int in, share;
     dx_list_share(a, tile, wave, in, share);
@@ -1396,7 +1403,7 @@ __global__ __launch_bounds__(kBlock) void lut_dx_kernel(DxArgs a)
 
     int const cnt = a.rev[(size_t)in * a.rev_stride];
     int t_begin, t_end;
-    dx_list_range(cnt, share, t_begin, t_end);
+    dx_list_range<WAVES>(cnt, share, t_begin, t_end);
     // The term table is read through the constant address space: its wave-uniform loads stay scalar loads wherever
     // they are placed relative to the stores of this kernel (the table is written by an earlier kernel).
     typedef __attribute__((address_space(4))) int const const_int;
@@ -1440,7 +1447,7 @@ __global__ __launch_bounds__(kBlock) void lut_dx_kernel(DxArgs a)
             T::load_coefficients(rec + (size_t)t * T::REC, Dk);
             T::accumulate(st, Dk, bit, lo, hi, acc);
         }
-        dx_store_pass<U>(a, part, in, wave, lane, f_begin, acc);
+        dx_store_pass<U, WAVES>(a, part, in, wave, lane, f_begin, acc);
     }
 }
 
