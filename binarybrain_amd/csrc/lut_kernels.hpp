@@ -194,6 +194,34 @@ struct Gather<N, kXBit> {
     }
 };
 
+// the same with four frames per lane (16-byte loads; rows 16-byte aligned, x_stride a multiple of 4): a lane's four bits
+// are shifted to their place in the word that eight neighbouring lanes share and the eight are combined by three exchanges
+__device__ __forceinline__ void binarize_pack4_block(float const *__restrict__ x, uint32_t *__restrict__ bits,
+                                                     int frame_size, int x_stride, int y_stride, int node, int block)
+{
+    int const q    = block * kBlock + threadIdx.x;          // group of four frames
+    int const f    = q * 4;
+    uint32_t v = 0;
+    if (f < frame_size) {
+        float4 const t = *reinterpret_cast<float4 const *>(x + (size_t)node * x_stride + f);
+        v = (t.x > 0.5f ? 1u : 0u) | ((f + 1 < frame_size && t.y > 0.5f) ? 2u : 0u) |
+            ((f + 2 < frame_size && t.z > 0.5f) ? 4u : 0u) | ((f + 3 < frame_size && t.w > 0.5f) ? 8u : 0u);
+    }
+    v <<= 4 * (threadIdx.x & 7);
+    v |= lane_xor(v, 1);
+    v |= lane_xor(v, 2);
+    v |= lane_xor(v, 4);
+    int const w = q >> 3;
+    if ((threadIdx.x & 7) == 0 && w < y_stride) { bits[(size_t)node * y_stride + w] = v; }
+}
+
+// the packed copy of fp32 rows, made by extra workgroups of a launch
+struct PackRider {
+    float const *x;  uint32_t *bits;  int x_stride, y_stride;
+    TileDivisor row_blocks;     // workgroups per packed row
+    int blocks;                 // rows * row_blocks.count; 0 = nothing to pack
+};
+
 struct FwdArgs {
     void const  *x;
     void        *y;
@@ -244,6 +272,9 @@ struct FwdArgs {
     // lut_forward_bytes_kernel (node_waves > 0 where a call takes it): wavefronts that share a node in a one-launch training pass, and whether
     // rows of fp32 output start on 16 bytes
     int   node_waves, y_quads;
+    // lut_forward_corner_kernel over the fp32 frames of a small batch-norm training pass: the last pack.blocks workgroups make the packed copy of the
+    // input that the backward call takes
+    PackRider pack;
     int   zero_padding;         // packed output: the wavefront of a node's last unit writes 0 behind the last frame's word, up to the row pitch
 };
 
@@ -735,6 +766,14 @@ __global__ __launch_bounds__(kBlock) void lut_forward_corner_kernel(FwdArgs a)
     static_assert(OWN == kOwnNone || (OWN == kOwnMemory && XMODE == kXBit && !WIDE && FWD_KIND == 1), "kept corner indices: output launch only");
     constexpr int NN = 1 << N;
     int const B    = a.chunk_count * a.tiles.count;
+    if constexpr (XMODE == kXBinary && YMODE == kYBinarize && FWD_KIND == 1) {
+        if ((int)blockIdx.x >= B) {
+            int row, block;
+            split_tile(blockIdx.x - B, a.pack.row_blocks, row, block);
+            binarize_pack4_block(a.pack.x, a.pack.bits, a.frame_size, a.pack.x_stride, a.pack.y_stride, row, block);
+            return;
+        }
+    }
     int const lid  = xcd_remap(blockIdx.x, B);
     int ck, tile;
     split_tile(lid, a.tiles, ck, tile);
@@ -1517,27 +1556,6 @@ __global__ __launch_bounds__(kBlock) void binarize_pack_kernel(float const *__re
     int const w = (f & ~(kWave - 1)) >> 5;                 // first word of the wavefront's 64 frames
     if (lane == 0  && w     < y_stride) { bits[(size_t)node * y_stride + w]     = (uint32_t)m; }
     if (lane == 32 && w + 1 < y_stride) { bits[(size_t)node * y_stride + w + 1] = (uint32_t)(m >> 32); }
-}
-
-// the same with four frames per lane (16-byte loads; rows 16-byte aligned, x_stride a multiple of 4): a lane's four bits
-// are shifted to their place in the word that eight neighbouring lanes share and the eight are combined by three exchanges
-__device__ __forceinline__ void binarize_pack4_block(float const *__restrict__ x, uint32_t *__restrict__ bits,
-                                                     int frame_size, int x_stride, int y_stride, int node, int block)
-{
-    int const q    = block * kBlock + threadIdx.x;          // group of four frames
-    int const f    = q * 4;
-    uint32_t v = 0;
-    if (f < frame_size) {
-        float4 const t = *reinterpret_cast<float4 const *>(x + (size_t)node * x_stride + f);
-        v = (t.x > 0.5f ? 1u : 0u) | ((f + 1 < frame_size && t.y > 0.5f) ? 2u : 0u) |
-            ((f + 2 < frame_size && t.z > 0.5f) ? 4u : 0u) | ((f + 3 < frame_size && t.w > 0.5f) ? 8u : 0u);
-    }
-    v <<= 4 * (threadIdx.x & 7);
-    v |= lane_xor(v, 1);
-    v |= lane_xor(v, 2);
-    v |= lane_xor(v, 4);
-    int const w = q >> 3;
-    if ((threadIdx.x & 7) == 0 && w < y_stride) { bits[(size_t)node * y_stride + w] = v; }
 }
 
 __global__ __launch_bounds__(kBlock) void binarize_pack4_kernel(float const *__restrict__ x, uint32_t *__restrict__ bits,
