@@ -725,7 +725,12 @@ int launch_corner_backward(CornerSumsArgs const &s, int slab_count, hipStream_t 
 {
     {
         ScopedTimer tm(kTimeBackward, st);
-        hipLaunchKernelGGL((lut_corner_sums_kernel<N, BN>), dim3(s.slab_count * s.tiles.count), dim3(kBlock), 0, st, s);
+        dim3 const grid(s.slab_count * s.tiles.count);
+        bool launched = false;
+        if constexpr (N >= 5) {             // (with few corners the atomics that count them collide, and the plain form has little to keep anyway)
+            if (slab_count == 1 && s.frame_size <= kShortSlab) { hipLaunchKernelGGL((lut_corner_sums_kernel<N, BN, true>), grid, dim3(kBlock), 0, st, s); launched = true; }
+        }
+        if (!launched) { hipLaunchKernelGGL((lut_corner_sums_kernel<N, BN, false>), grid, dim3(kBlock), 0, st, s); }
     }
     BBHIP_LAUNCH_CHECK();
     if (slab_count > 1) {

@@ -69,6 +69,8 @@ __device__ __forceinline__ void corner_fold(CornerFoldArgs const &a, CornerFoldI
     if (lane < NN) { a.dW[(size_t)node * NN + lane] = a.overwrite ? G : q.dW + G; }
 }
 
+constexpr int kShortSlab = 1024, kShortColumns = 32;            // see lut_corner_sums_kernel
+
 struct CornerSumsArgs {
     uint32_t const *x;
     float const *dy;
@@ -107,16 +109,18 @@ __device__ __forceinline__ uint32_t quad_row_bytes(int frame_size, bool quads)
     return (uint32_t)(quads ? (frame_size + 3) & ~3 : frame_size) * 4u;
 }
 
-// sums over the 64 columns of row (lane mod ROWS) of a wavefront's [ROWS][64] block in LDS.  A lane takes four columns at a time, in an order
+// sums over the COLS columns of row (lane mod ROWS) of a wavefront's [ROWS][COLS] block in LDS.  A lane takes four columns at a time, in an order
 // of its own, so that the lanes that are served together read different banks; with fewer than 64 rows several lanes share one.
-template <int ROWS, typename V4>
+template <int ROWS, int COLS, typename V4>
 __device__ __forceinline__ auto row_sum(V4 const *block, int lane)
 {
+    constexpr int LANES = kWave / ROWS, EACH = COLS / 4 / LANES;        // lanes per row, groups of four columns for each
+    static_assert(EACH >= 1, "a group of columns for every lane");
     int const p = lane & (ROWS - 1), part = lane / ROWS;
     decltype(block[0].x + block[0].x) s = 0;
 #pragma unroll
-    for (int g = 0; g < ROWS / 4; ++g) {
-        V4 const q = block[p * (kWave / 4) + part * (ROWS / 4) + (g ^ (p & (ROWS / 4 - 1)))];
+    for (int g = 0; g < EACH; ++g) {
+        V4 const q = block[p * (COLS / 4) + part * EACH + (g ^ (p & (EACH - 1)))];
         s += (q.x + q.y) + (q.z + q.w);
     }
 #pragma unroll
@@ -135,12 +139,17 @@ __device__ __forceinline__ auto row_sum(V4 const *block, int lane)
 // (scalar loads would be waited for with the LDS accesses: 101 us for the first shape below).
 // Measured against the statistics and table-gradient launches that it replaces: 216 nodes x 230400 frames 65 us (3.8 TB/s of dy and indices)
 // instead of 53 + 141; 4096 x 8192 42 us instead of 31 + 106; 6144 x 1024 20 us instead of 11 + 30.
-template <int N, bool BN>
+// SHORT: up to kShortSlab frames in one slab.  Such a launch is a chain of latencies, so what counts is how many wavefronts share a compute unit: two
+// lanes share a column of bins (they add in turn), and the corners are counted by integer atomics (one instruction per step, and nothing to add up).
+// 6144 nodes x 1024 frames 20.5 -> 14.9 us, 6000 x 100 17.4 -> 9.6 us; four lanes per column measured the same or slower.
+template <int N, bool BN, bool SHORT>
 __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs a)
 {
-    constexpr int NN = 1 << N, kPasses = 8, kAhead = 4;
-    __shared__ __align__(16) float bins[kWavesPerBlk][NN * kWave];
+    constexpr int NN = 1 << N, kAhead = 4, kPasses = SHORT ? kShortSlab / (4 * kWave) : 8, COLS = SHORT ? kShortColumns : kWave;
+    static_assert(!SHORT || kPasses <= kAhead, "all of dy requested ahead");
+    __shared__ __align__(16) float bins[kWavesPerBlk][NN * COLS];
     __shared__ __align__(16) uint32_t quads[kWavesPerBlk][kPasses * kWave];
+    __shared__ uint32_t counts[kWavesPerBlk][(BN && SHORT) ? NN : 1];
     int const B   = a.slab_count * a.tiles.count;
     int const lid = xcd_remap(blockIdx.x, B);
     int sl, tile;
@@ -182,12 +191,14 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
 
     float *const mine = bins[wv];
 #pragma unroll
-    for (int i = 0; i < NN / 4; ++i) { *reinterpret_cast<float4 *>(mine + (i * kWave + lane) * 4) = make_float4(0.0f, 0.0f, 0.0f, 0.0f); }
+    for (int i = 0; i < NN * COLS / (4 * kWave); ++i) { *reinterpret_cast<float4 *>(mine + (i * kWave + lane) * 4) = make_float4(0.0f, 0.0f, 0.0f, 0.0f); }
+    if (BN && SHORT && lane < NN) { counts[wv][lane] = 0; }
     wave_fence();
 
-    uint32_t count[BN ? NN : 1];                                        // [S]: frames of the lane's words where every input of S is set
+    constexpr bool kCountSets = BN && !SHORT;
+    uint32_t count[kCountSets ? NN : 1];                                // [S]: frames of the lane's words where every input of S is set
 #pragma unroll
-    for (int i = 0; i < (BN ? NN : 1); ++i) { count[i] = 0; }
+    for (int i = 0; i < (kCountSets ? NN : 1); ++i) { count[i] = 0; }
 
     for (int base = f_begin; base < f_end; base += kPasses * 4 * kWave) {
         uint32_t quad[8];
@@ -195,7 +206,7 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
             uint32_t w[N];
 #pragma unroll
             for (int k = 0; k < N; ++k) { w[k] = w_next[k]; }
-            request_words(base + kPasses * 4 * kWave);                  // (past the row: zeros)
+            if (!SHORT) { request_words(base + kPasses * 4 * kWave); }  // (past the row: zeros)
             corner_bytes<N>(w, quad);
             int const live = f_end - (base + 32 * lane);                // frames of the lane's words that belong to the slab
             if (live > 0) {
@@ -203,10 +214,12 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
                 out[0] = make_uint4(quad[0], quad[1], quad[2], quad[3]);
                 out[1] = make_uint4(quad[4], quad[5], quad[6], quad[7]);
             }
-            uint4 *ex = reinterpret_cast<uint4 *>(quads[wv] + 8 * lane);
-            ex[0] = make_uint4(quad[0], quad[1], quad[2], quad[3]);
-            ex[1] = make_uint4(quad[4], quad[5], quad[6], quad[7]);
-            if constexpr (BN) {
+            if (!SHORT || lane < kPasses * 8) {                         // (the lanes whose words hold frames of the slab)
+                uint4 *ex = reinterpret_cast<uint4 *>(quads[wv] + 8 * lane);
+                ex[0] = make_uint4(quad[0], quad[1], quad[2], quad[3]);
+                ex[1] = make_uint4(quad[4], quad[5], quad[6], quad[7]);
+            }
+            if constexpr (kCountSets) {
                 uint32_t all[NN];
                 all[0] = (live >= 32) ? 0xffffffffu : (live <= 0) ? 0u : ((1u << live) - 1u);
                 count[0] += __popc(all[0]);
@@ -226,7 +239,7 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
             int const fb = base + i * 4 * kWave;
             if (fb >= f_end) { break; }                                 // wave-uniform
             float4 d = dy[i % kAhead];
-            dy[i % kAhead] = load_quad(dyr, (uint32_t)(fb + kAhead * 4 * kWave + 4 * lane) * 4u, quad_rows);
+            if (!SHORT) { dy[i % kAhead] = load_quad(dyr, (uint32_t)(fb + kAhead * 4 * kWave + 4 * lane) * 4u, quad_rows); }
             if (fb + 4 * kWave > a.frame_size) {                        // the row's padding may hold anything
                 int const f = fb + 4 * lane;
                 if (f     >= a.frame_size) { d.x = 0.0f; }
@@ -234,23 +247,42 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
                 if (f + 2 >= a.frame_size) { d.z = 0.0f; }
                 if (f + 3 >= a.frame_size) { d.w = 0.0f; }
             }
-            mine[(at[i] & 0xffu) * kWave + lane] += d.x;
-            mine[((at[i] >> 8) & 0xffu) * kWave + lane] += d.y;
-            mine[((at[i] >> 16) & 0xffu) * kWave + lane] += d.z;
-            mine[(at[i] >> 24) * kWave + lane] += d.w;
+            if constexpr (BN && SHORT) {
+                int const f = fb + 4 * lane;
+                if (f     < f_end) { atomicAdd(&counts[wv][at[i] & 0xffu], 1u); }
+                if (f + 1 < f_end) { atomicAdd(&counts[wv][(at[i] >> 8) & 0xffu], 1u); }
+                if (f + 2 < f_end) { atomicAdd(&counts[wv][(at[i] >> 16) & 0xffu], 1u); }
+                if (f + 3 < f_end) { atomicAdd(&counts[wv][at[i] >> 24], 1u); }
+            }
+            auto add_all = [&]() {
+                int const col = lane & (COLS - 1);
+                mine[(at[i] & 0xffu) * COLS + col] += d.x;
+                mine[((at[i] >> 8) & 0xffu) * COLS + col] += d.y;
+                mine[((at[i] >> 16) & 0xffu) * COLS + col] += d.z;
+                mine[(at[i] >> 24) * COLS + col] += d.w;
+            };
+            if constexpr (COLS == kWave) { add_all(); }
+            else {
+#pragma unroll
+                for (int turn = 0; turn < kWave / COLS; ++turn) {
+                    if (lane / COLS == turn) { add_all(); }
+                    wave_fence();
+                }
+            }
         }
         wave_fence();
     }
 
-    float const D = row_sum<NN>(reinterpret_cast<float4 const *>(mine), lane);
+    float const D = row_sum<NN, COLS>(reinterpret_cast<float4 const *>(mine), lane);
     uint32_t n = 0;
-    if constexpr (BN) {
+    if constexpr (BN && SHORT) { n = counts[wv][lane & (NN - 1)]; }
+    if constexpr (kCountSets) {
         wave_fence();
         uint32_t *const cells = reinterpret_cast<uint32_t *>(mine);
 #pragma unroll
         for (int s = 0; s < NN; ++s) { cells[s * kWave + lane] = count[s]; }
         wave_fence();
-        n = row_sum<NN>(reinterpret_cast<uint4 const *>(cells), lane);  // lane S: frames where every input of S is set (the others either way)
+        n = row_sum<NN, kWave>(reinterpret_cast<uint4 const *>(cells), lane);  // lane S: frames where every input of S is set (the others either way)
 #pragma unroll
         for (int k = 0; k < N; ++k) {
             uint32_t const o = lane_xor(n, 1 << k);
