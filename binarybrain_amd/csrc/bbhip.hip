@@ -10,6 +10,8 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/bbhip.h"
@@ -237,6 +239,19 @@ inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
+// A launch without the call-configuration stack and the copies that the <<<>>> form's host stub goes through: 2.7 us of host time for a kernel
+// with 400 bytes of arguments instead of 3.2, and the host is what a program of small layers waits for.  Errors are read by BBHIP_LAUNCH_CHECK.
+template <class... P, class... A>
+void launch(void (*kernel)(P...), dim3 grid, dim3 block, unsigned lds_bytes, hipStream_t st, A const &... args)
+{
+    // an argument of the parameter's own type is passed where it lies
+    std::tuple<std::conditional_t<std::is_same_v<P, A>, A const &, P>...> const held{args...};
+    std::apply([&](auto const &... v) {
+        void *where[] = {const_cast<void *>(static_cast<void const *>(&v))...};
+        (void)hipLaunchKernel(reinterpret_cast<void const *>(kernel), grid, block, where, lds_bytes, st);
+    }, held);
+}
+
 // ------------------------------------------------------------------------------------------------
 //  dispatch helpers
 // ------------------------------------------------------------------------------------------------
@@ -255,7 +270,7 @@ void launch_table_prep(float const *W, float *C, int node_size, int lut_binarize
                        float *clamp_W = nullptr, float clamp_lo = 0.0f, float clamp_hi = 0.0f)
 {
     int const total = node_size * (1 << N);
-    hipLaunchKernelGGL(table_prep_kernel<N>, dim3(ceil_div(total, kBlock)), dim3(kBlock), 0, st, W, C, node_size, lut_binarize, V, bias, clamp_W, clamp_lo, clamp_hi);
+    launch(table_prep_kernel<N>, dim3(ceil_div(total, kBlock)), dim3(kBlock), 0, st, W, C, node_size, lut_binarize, V, bias, clamp_W, clamp_lo, clamp_hi);
 }
 
 template <int N, int XMODE, int YMODE, int KIND>
@@ -270,29 +285,29 @@ void launch_forward(FwdArgs const &a, int npw, hipStream_t st)
                     bool const fused = (KIND == 1) && a.stat_mode == kStatInline;
                     int const waves = a.node_waves > kWavesPerBlk ? a.node_waves : kWavesPerBlk;
                     int const index_blocks = fused ? waves / a.node_waves * ceil_div(a.frame_size, kByteBlock) : waves;
-                    hipLaunchKernelGGL((lut_forward_bytes_kernel<N, XMODE, YMODE, KIND>), grid, dim3(waves * kWave), forward_bytes_lds(waves, index_blocks), st, a);
+                    launch((lut_forward_bytes_kernel<N, XMODE, YMODE, KIND>), grid, dim3(waves * kWave), forward_bytes_lds(waves, index_blocks), st, a);
                     return;
                 }
             }
             if constexpr (XMODE == kXBit && YMODE == kYBinarize && KIND == 1) {
                 if (a.own_index != nullptr) {      // corner indices kept by the statistics launch of the same call
-                    hipLaunchKernelGGL((lut_forward_corner_kernel<N, XMODE, YMODE, KIND, false, kOwnMemory>), grid, block, 0, st, a);
+                    launch((lut_forward_corner_kernel<N, XMODE, YMODE, KIND, false, kOwnMemory>), grid, block, 0, st, a);
                     return;
                 }
             }
             if constexpr (XMODE == kXBit) {
                 // 32-byte scalar loads where they stay inside the row pitch and never straddle a unit
                 if (a.x_stride % 8 == 0 && a.chunk % 256 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 3u) == 0) {
-                    hipLaunchKernelGGL((lut_forward_corner_kernel<N, XMODE, YMODE, KIND, true>), grid, block, 0, st, a);
+                    launch((lut_forward_corner_kernel<N, XMODE, YMODE, KIND, true>), grid, block, 0, st, a);
                     return;
                 }
             }
-            hipLaunchKernelGGL((lut_forward_corner_kernel<N, XMODE, YMODE, KIND>), grid, block, 0, st, a);
+            launch((lut_forward_corner_kernel<N, XMODE, YMODE, KIND>), grid, block, 0, st, a);
             return;
         }
     }
-    if (npw == 2) { hipLaunchKernelGGL((lut_forward_kernel<N, XMODE, YMODE, KIND, 2>), grid, block, 0, st, a); }
-    else          { hipLaunchKernelGGL((lut_forward_kernel<N, XMODE, YMODE, KIND, 1>), grid, block, 0, st, a); }
+    if (npw == 2) { launch((lut_forward_kernel<N, XMODE, YMODE, KIND, 2>), grid, block, 0, st, a); }
+    else          { launch((lut_forward_kernel<N, XMODE, YMODE, KIND, 1>), grid, block, 0, st, a); }
 }
 
 // xmode / ymode / kind are runtime values here; the combinations that exist are enumerated explicitly
@@ -324,7 +339,7 @@ template <int N>
 int dispatch_backward(int xmode, int kind, int dxmode, BwdArgs const &a, hipStream_t st)
 {
     dim3 const grid(a.tt.blocks + a.slab_count * a.tiles.count), block(kBlock);
-#define BBHIP_BWD_CASE(X, K, M) if (xmode == X && kind == K && dxmode == M) { hipLaunchKernelGGL((lut_backward_kernel<N, X, K, M>), grid, block, 0, st, a); return 0; }
+#define BBHIP_BWD_CASE(X, K, M) if (xmode == X && kind == K && dxmode == M) { launch((lut_backward_kernel<N, X, K, M>), grid, block, 0, st, a); return 0; }
     BBHIP_BWD_CASE(kXClamp,  0, kDxAtomic) BBHIP_BWD_CASE(kXClamp,  0, kDxTmp)
     BBHIP_BWD_CASE(kXBinary, 0, kDxAtomic) BBHIP_BWD_CASE(kXBinary, 0, kDxTmp)
     BBHIP_BWD_CASE(kXBit,    0, kDxAtomic) BBHIP_BWD_CASE(kXBit,    0, kDxTmp)
@@ -344,8 +359,8 @@ int dispatch_dx_u(int xmode, DxArgs const &a, hipStream_t st)
     dim3 const grid(a.fin_blocks + a.chunk_count * a.tiles.count), block((a.split ? a.split : kWavesPerBlk) * kWave);
 #define BBHIP_DX_CASE(X)                                                                                                       \
     if (xmode == X) {                                                                                                          \
-        if (a.split > kWavesPerBlk) { hipLaunchKernelGGL((lut_dx_kernel<N, X, U, kDxWaves>), grid, block, 0, st, a); }       \
-        else                        { hipLaunchKernelGGL((lut_dx_kernel<N, X, U, kWavesPerBlk>), grid, block, 0, st, a); }   \
+        if (a.split > kWavesPerBlk) { launch((lut_dx_kernel<N, X, U, kDxWaves>), grid, block, 0, st, a); }       \
+        else                        { launch((lut_dx_kernel<N, X, U, kWavesPerBlk>), grid, block, 0, st, a); }   \
         return 0;                                                                                                              \
     }
     BBHIP_DX_CASE(kXClamp) BBHIP_DX_CASE(kXBinary) BBHIP_DX_CASE(kXBit)
@@ -421,11 +436,11 @@ int launch_binarize_pack(float const *x, int x_stride, uint32_t *bits, int bit_s
         float const *src = x + (size_t)n0 * x_stride;
         uint32_t *dst = bits + (size_t)n0 * bit_stride;
         if (x_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15u) == 0) {
-            hipLaunchKernelGGL(binarize_pack4_kernel, dim3(ceil_div(bit_stride * 8, kBlock), rows), dim3(kBlock), 0, st,
+            launch(binarize_pack4_kernel, dim3(ceil_div(bit_stride * 8, kBlock), rows), dim3(kBlock), 0, st,
                                src, dst, frame_size, x_stride, bit_stride);
         }
         else {
-            hipLaunchKernelGGL(binarize_pack_kernel, dim3(ceil_div(bit_stride * 32, kBlock), rows), dim3(kBlock), 0, st,
+            launch(binarize_pack_kernel, dim3(ceil_div(bit_stride * 32, kBlock), rows), dim3(kBlock), 0, st,
                                src, dst, frame_size, x_stride, bit_stride);
         }
     }
@@ -447,7 +462,7 @@ int launch_pack_and_prep(float const *x, int x_stride, uint32_t *bits, int bit_s
         a.row_blocks = make_tile_divisor(row_blocks); a.pack_blocks = (int)pack_blocks;
         a.W = W; a.C = C; a.V = V; a.node_size = node_size; a.lut_binarize = lut_binarize; a.bias = bias;
         a.clamp_W = clamp_W; a.clamp_lo = clamp_lo; a.clamp_hi = clamp_hi;
-        hipLaunchKernelGGL(binarize_pack4_prep_kernel<N>, dim3((unsigned)(pack_blocks + prep_blocks)), dim3(kBlock), 0, st, a);
+        launch(binarize_pack4_prep_kernel<N>, dim3((unsigned)(pack_blocks + prep_blocks)), dim3(kBlock), 0, st, a);
         BBHIP_LAUNCH_CHECK();
         return 0;
     }
@@ -481,7 +496,7 @@ int run_forward_real_node(ForwardCall const &c, hipStream_t st, PreparedTablesHi
     a.tiles = make_tile_divisor(ceil_div(c.node_size, per_block));
     {
         ScopedTimer tm(kTimeForward, st);
-        hipLaunchKernelGGL(lut_forward_node_kernel<N>, dim3(a.tiles.count), dim3(per_block * a.node_waves * kWave), 0, st, a);
+        launch(lut_forward_node_kernel<N>, dim3(a.tiles.count), dim3(per_block * a.node_waves * kWave), 0, st, a);
     }
     BBHIP_LAUNCH_CHECK();
     return 0;
@@ -626,7 +641,7 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
         }
         else {
             int const npb = stat_nodes_per_block(chunk_count);
-            hipLaunchKernelGGL(bn_forward_finalize_kernel, dim3(ceil_div(c.node_size, npb)), dim3(kBlock), 0, st,
+            launch(bn_forward_finalize_kernel, dim3(ceil_div(c.node_size, npb)), dim3(kBlock), 0, st,
                                stat, C, NN, c.mean, c.rstd, c.running_mean, c.running_var, c.momentum,
                                c.node_size, chunk_count, c.frame_size, npb);
             BBHIP_LAUNCH_CHECK();
@@ -728,13 +743,13 @@ int launch_corner_backward(CornerSumsArgs const &s, int slab_count, hipStream_t 
         dim3 const grid(s.slab_count * s.tiles.count);
         bool launched = false;
         if constexpr (N >= 5) {             // (with few corners the atomics that count them collide, and the plain form has little to keep anyway)
-            if (slab_count == 1 && s.frame_size <= kShortSlab) { hipLaunchKernelGGL((lut_corner_sums_kernel<N, BN, true>), grid, dim3(kBlock), 0, st, s); launched = true; }
+            if (slab_count == 1 && s.frame_size <= kShortSlab) { launch((lut_corner_sums_kernel<N, BN, true>), grid, dim3(kBlock), 0, st, s); launched = true; }
         }
-        if (!launched) { hipLaunchKernelGGL((lut_corner_sums_kernel<N, BN, false>), grid, dim3(kBlock), 0, st, s); }
+        if (!launched) { launch((lut_corner_sums_kernel<N, BN, false>), grid, dim3(kBlock), 0, st, s); }
     }
     BBHIP_LAUNCH_CHECK();
     if (slab_count > 1) {
-        hipLaunchKernelGGL((lut_corner_fold_kernel<N, BN>), dim3(s.node_size), dim3(kBlock), 0, st, s.fold, s.partial, s.V ? s.V : s.V_out, s.node_size, slab_count);
+        launch((lut_corner_fold_kernel<N, BN>), dim3(s.node_size), dim3(kBlock), 0, st, s.fold, s.partial, s.V ? s.V : s.V_out, s.node_size, slab_count);
         BBHIP_LAUNCH_CHECK();
     }
     return 0;
@@ -748,8 +763,8 @@ int dispatch_dx_table(int quads, DxTableArgs const &t, hipStream_t st)
     ScopedTimer tm(kTimeDx, st);
 #define BBHIP_DX_CASE(Q, FAR)                                                                                                                  \
     {                                                                                                                                          \
-        if (waves > kWavesPerBlk) { hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, Q, kDxWaves, FAR>), grid, block, 0, st, t); }             \
-        else                      { hipLaunchKernelGGL((lut_dx_table_kernel<N, BN, Q, kWavesPerBlk, FAR>), grid, block, 0, st, t); }         \
+        if (waves > kWavesPerBlk) { launch((lut_dx_table_kernel<N, BN, Q, kDxWaves, FAR>), grid, block, 0, st, t); }             \
+        else                      { launch((lut_dx_table_kernel<N, BN, Q, kWavesPerBlk, FAR>), grid, block, 0, st, t); }         \
     }
     if (t.far)           BBHIP_DX_CASE(1, true)
     else if (quads == 1) BBHIP_DX_CASE(1, false)
@@ -850,7 +865,7 @@ void launch_node_gradient(BackwardCall const &c, BwdArgs const &a, float const *
     g.dyh = dyh; g.dyh_stride = c.frame_stride; g.node_waves = real_node_waves(c.frame_size);
     int const per_block = real_nodes_per_block(g.node_waves);
     g.node_tiles = ceil_div(c.output_node_size, per_block);
-    hipLaunchKernelGGL(lut_node_gradient_kernel<N>, dim3(g.tt.blocks + g.node_tiles), dim3(per_block * g.node_waves * kWave), 0, st, g);
+    launch(lut_node_gradient_kernel<N>, dim3(g.tt.blocks + g.node_tiles), dim3(per_block * g.node_waves * kWave), 0, st, g);
 }
 
 template <int N>
@@ -986,7 +1001,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         }
         else {
             int const npb = stat_nodes_per_block(stat_chunk_count);
-            hipLaunchKernelGGL(bn_backward_finalize_kernel, dim3(ceil_div(c.output_node_size, npb)), dim3(kBlock), 0, st,
+            launch(bn_backward_finalize_kernel, dim3(ceil_div(c.output_node_size, npb)), dim3(kBlock), 0, st,
                                stat, c.mean, c.rstd, c.dmean_tmp, c.dvar_tmp, c.gamma, c.output_node_size, stat_chunk_count, c.frame_size, npb);
             BBHIP_LAUNCH_CHECK();
         }
@@ -994,7 +1009,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
 
     if (dxmode == kDxAtomic) {
         size_t const count = (size_t)c.input_node_size * c.frame_stride;
-        hipLaunchKernelGGL(fill_kernel, dim3((unsigned)((count + kBlock * 4 - 1) / (kBlock * 4))), dim3(kBlock), 0, st, c.dx, 0.0f, count);
+        launch(fill_kernel, dim3((unsigned)((count + kBlock * 4 - 1) / (kBlock * 4))), dim3(kBlock), 0, st, c.dx, 0.0f, count);
         BBHIP_LAUNCH_CHECK();
     }
 
@@ -1016,7 +1031,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         BBHIP_LAUNCH_CHECK();
         if (dxmode == kDxTmp) {
             dim3 const grid(ceil_div(a.f_limit - a.f_base, kBlock), c.input_node_size < 65535 ? c.input_node_size : 65535);
-            hipLaunchKernelGGL(dx_gather_kernel, grid, dim3(kBlock), 0, st, c.dx_tmp, c.dx, c.rev, c.rev_stride,
+            launch(dx_gather_kernel, grid, dim3(kBlock), 0, st, c.dx_tmp, c.dx, c.rev, c.rev_stride,
                                c.input_node_size, a.f_base, a.f_limit, c.frame_stride, c.tmp_frame_stride);
             BBHIP_LAUNCH_CHECK();
         }
@@ -1052,7 +1067,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
     }
 
     int const total = c.output_node_size * NN;
-    hipLaunchKernelGGL(dw_finalize_kernel<N>, dim3(ceil_div(total, kBlock)), dim3(kBlock), 0, st, part, c.dW, c.output_node_size, slab_total, dw_overwrite);
+    launch(dw_finalize_kernel<N>, dim3(ceil_div(total, kBlock)), dim3(kBlock), 0, st, part, c.dW, c.output_node_size, slab_total, dw_overwrite);
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -1163,7 +1178,7 @@ int vector_op(float *dst, float const *src0, float const *src1, float a, float b
                           (vec_binary<OP>() ? reinterpret_cast<uintptr_t>(src1) : 0)) & 15) == 0;
     size_t const blocks = ((size_t)size + kVecBlock * 4 - 1) / (kVecBlock * 4);
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    hipLaunchKernelGGL(vector_op_kernel<OP>, dim3((unsigned)blocks), dim3(kVecBlock), 0, static_cast<hipStream_t>(stream),
+    launch(vector_op_kernel<OP>, dim3((unsigned)blocks), dim3(kVecBlock), 0, static_cast<hipStream_t>(stream),
                        dst, src0, src1, a, b, c, d, (size_t)size, aligned);
     BBHIP_LAUNCH_CHECK();
     return 0;
@@ -1356,7 +1371,7 @@ int bbhip_fp32_Vector_set(float *dev_dst, float a, int size, void *stream)
     clear_hints();                                 // a hint is for the next LUT forward call only
     BBHIP_REQUIRE(dev_dst != nullptr && size >= 0);
     if (size == 0) { return 0; }
-    hipLaunchKernelGGL(fill_kernel, dim3(ceil_div(size, kBlock * 4)), dim3(kBlock), 0, static_cast<hipStream_t>(stream), dev_dst, a, (size_t)size);
+    launch(fill_kernel, dim3(ceil_div(size, kBlock * 4)), dim3(kBlock), 0, static_cast<hipStream_t>(stream), dev_dst, a, (size_t)size);
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -1366,7 +1381,7 @@ int bbhip_fp32_Vector_clamp(float *dev_dst, float const *dev_src, float lo, floa
     clear_hints();                                 // a hint is for the next LUT forward call only
     BBHIP_REQUIRE(dev_dst != nullptr && dev_src != nullptr && size >= 0);
     if (size == 0) { return 0; }
-    hipLaunchKernelGGL(clamp_kernel, dim3(ceil_div(size, kBlock)), dim3(kBlock), 0, static_cast<hipStream_t>(stream), dev_dst, dev_src, lo, hi, size);
+    launch(clamp_kernel, dim3(ceil_div(size, kBlock)), dim3(kBlock), 0, static_cast<hipStream_t>(stream), dev_dst, dev_src, lo, hi, size);
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -1438,12 +1453,12 @@ int adam_entry(bool zero_grads, int size, int const *dev_size_table, float *cons
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
     dim3 const grid(kAdamBlocksPerTensor, (unsigned)size), block(kVecBlock);
     if (zero_grads) {
-        hipLaunchKernelGGL(adam_kernel<true>, grid, block, 0, static_cast<hipStream_t>(stream),
+        launch(adam_kernel<true>, grid, block, 0, static_cast<hipStream_t>(stream),
                            dev_size_table, dev_params_buf_table, dev_grads_buf_table, dev_m_buf_table, dev_v_buf_table,
                            lr_t, 1.0f - beta1, 1.0f - beta2);
     }
     else {
-        hipLaunchKernelGGL(adam_kernel<false>, grid, block, 0, static_cast<hipStream_t>(stream),
+        launch(adam_kernel<false>, grid, block, 0, static_cast<hipStream_t>(stream),
                            dev_size_table, dev_params_buf_table, dev_grads_buf_table, dev_m_buf_table, dev_v_buf_table,
                            lr_t, 1.0f - beta1, 1.0f - beta2);
     }
@@ -1480,7 +1495,7 @@ int bbhip_fp32_Im2Col_Forward(float const *dev_x_buf, float *dev_y_buf, int x_st
     long long const blocks = (long long)a.c * a.fh * a.fw * a.q_tiles * a.f_tiles;
     if (blocks > 0x7fffffffLL) { return fail("%s: grid too large", __func__); }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    hipLaunchKernelGGL(im2col_forward_kernel, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream), a);
+    launch(im2col_forward_kernel, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream), a);
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -1501,7 +1516,7 @@ int bbhip_bit_Im2Col_Forward(int const *dev_x_buf, int *dev_y_buf, int x_stride,
     long long const blocks = (total + kConvBlock - 1) / kConvBlock;
     if (blocks > 0x7fffffffLL) { return fail("%s: grid too large", __func__); }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    hipLaunchKernelGGL(im2col_forward_bit_kernel, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream), a, words, total);
+    launch(im2col_forward_bit_kernel, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream), a, words, total);
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -1524,8 +1539,8 @@ int bbhip_fp32_Im2Col_Backward(float const *dev_dy_buf, float *dev_dx_buf, int x
     long long const blocks = (long long)a.c * p_tiles * a.f_tiles;
     if (blocks > 0x7fffffffLL) { return fail("%s: grid too large", __func__); }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    if (tf == 64) { hipLaunchKernelGGL(im2col_backward_kernel<64>, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream), a, p_tiles); }
-    else          { hipLaunchKernelGGL(im2col_backward_kernel<16>, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream), a, p_tiles); }
+    if (tf == 64) { launch(im2col_backward_kernel<64>, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream), a, p_tiles); }
+    else          { launch(im2col_backward_kernel<16>, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream), a, p_tiles); }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -1552,7 +1567,7 @@ int bbhip_fp32_Col2Im_Forward(float const *dev_x_buf, float *dev_y_buf, int w_si
     long long const blocks = (long long)c_size * xy_tiles * f_tiles;
     if (blocks > 0x7fffffffLL) { return fail("%s: grid too large", __func__); }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    hipLaunchKernelGGL(col2im_kernel<true>, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream),
+    launch(col2im_kernel<true>, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream),
                        dev_x_buf, dev_y_buf, hw, c_size, input_frame_stride, output_frame_size, output_frame_stride, xy_tiles, f_tiles);
     BBHIP_LAUNCH_CHECK();
     return 0;
@@ -1567,7 +1582,7 @@ int bbhip_fp32_Col2Im_Backward(float const *dev_dy_buf, float *dev_dx_buf, int w
     long long const blocks = (long long)c_size * xy_tiles * f_tiles;
     if (blocks > 0x7fffffffLL) { return fail("%s: grid too large", __func__); }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    hipLaunchKernelGGL(col2im_kernel<false>, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream),
+    launch(col2im_kernel<false>, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream),
                        dev_dy_buf, dev_dx_buf, hw, c_size, input_frame_stride, output_frame_size, output_frame_stride, xy_tiles, f_tiles);
     BBHIP_LAUNCH_CHECK();
     return 0;
@@ -1583,7 +1598,7 @@ int bbhip_bit_Col2Im_Forward(int const *dev_x_buf, int *dev_y_buf, int w_size, i
     long long const blocks = (total + kConvBlock - 1) / kConvBlock;
     if (blocks > 0x7fffffffLL) { return fail("%s: grid too large", __func__); }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    hipLaunchKernelGGL(col2im_forward_bit_kernel, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream),
+    launch(col2im_forward_bit_kernel, dim3((unsigned)blocks), dim3(kConvBlock), 0, static_cast<hipStream_t>(stream),
                        reinterpret_cast<uint32_t const *>(dev_x_buf), reinterpret_cast<uint32_t *>(dev_y_buf), hw, input_frame_stride,
                        output_frame_size, output_frame_stride, words, total);
     BBHIP_LAUNCH_CHECK();
@@ -1605,10 +1620,10 @@ static int launch_pool(PoolArgs const &a, bool backward, void *stream, char cons
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
     dim3 const grid((unsigned)blocks), block(kConvBlock);
-    if (backward) { if (wide) { hipLaunchKernelGGL((stochastic_maxpool2x2_backward_kernel<4>), grid, block, 0, st, a, f_blocks); }
-                    else      { hipLaunchKernelGGL((stochastic_maxpool2x2_backward_kernel<1>), grid, block, 0, st, a, f_blocks); } }
-    else          { if (wide) { hipLaunchKernelGGL((stochastic_maxpool2x2_forward_kernel<4>), grid, block, 0, st, a, f_blocks); }
-                    else      { hipLaunchKernelGGL((stochastic_maxpool2x2_forward_kernel<1>), grid, block, 0, st, a, f_blocks); } }
+    if (backward) { if (wide) { launch((stochastic_maxpool2x2_backward_kernel<4>), grid, block, 0, st, a, f_blocks); }
+                    else      { launch((stochastic_maxpool2x2_backward_kernel<1>), grid, block, 0, st, a, f_blocks); } }
+    else          { if (wide) { launch((stochastic_maxpool2x2_forward_kernel<4>), grid, block, 0, st, a, f_blocks); }
+                    else      { launch((stochastic_maxpool2x2_forward_kernel<1>), grid, block, 0, st, a, f_blocks); } }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -1659,7 +1674,7 @@ static int average_lut_forward(float const *dev_x_buf, float *dev_y_buf, int con
     long long const blocks = (long long)node_size * f_blocks;
     if (blocks > 0x7fffffffLL) { return fail("%s: grid too large", name); }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    hipLaunchKernelGGL(average_lut_forward_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, static_cast<hipStream_t>(stream), dev_x_buf,
+    launch(average_lut_forward_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, static_cast<hipStream_t>(stream), dev_x_buf,
                        dev_y_buf, dev_input_index, n, frame_size, frame_stride, binarize_input, binarize_output, f_blocks,
                        mean ? 1.0f / (float)n : 1.0f);
     BBHIP_LAUNCH_CHECK();
@@ -1694,7 +1709,7 @@ int bbhip_bit_AverageLut_Forward(int const *dev_x_buf, int *dev_y_buf, int const
     dim3 const grid((unsigned)blocks), block(kTailBlock);
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
-#define BBHIP_AVERAGE_BIT(P) hipLaunchKernelGGL(average_lut_forward_bit_kernel<P>, grid, block, 0, st, dev_x_buf, dev_y_buf, dev_input_index, n, words, frame_stride, w_blocks)
+#define BBHIP_AVERAGE_BIT(P) launch(average_lut_forward_bit_kernel<P>, grid, block, 0, st, dev_x_buf, dev_y_buf, dev_input_index, n, words, frame_stride, w_blocks)
     switch (planes) {
     case 1: BBHIP_AVERAGE_BIT(1); break;
     case 2: BBHIP_AVERAGE_BIT(2); break;
@@ -1705,7 +1720,7 @@ int bbhip_bit_AverageLut_Forward(int const *dev_x_buf, int *dev_y_buf, int const
     case 7: BBHIP_AVERAGE_BIT(7); break;
     case 8: BBHIP_AVERAGE_BIT(8); break;
     default:
-        hipLaunchKernelGGL(average_lut_forward_bit_wide_kernel, grid, block, 0, st, dev_x_buf, dev_y_buf, dev_input_index, n, words, frame_stride, w_blocks);
+        launch(average_lut_forward_bit_wide_kernel, grid, block, 0, st, dev_x_buf, dev_y_buf, dev_input_index, n, words, frame_stride, w_blocks);
     }
 #undef BBHIP_AVERAGE_BIT
     BBHIP_LAUNCH_CHECK();
@@ -1725,7 +1740,7 @@ int bbhip_fp32_AverageLut_Backward(float const *dev_dy_buf, float *dev_dx_buf, i
     hipStream_t const st = static_cast<hipStream_t>(stream);
     if (walk_whole_table(total, input_node_size, frame_size)) {
         ScopedTimer tm(kTimeOther, st);
-        hipLaunchKernelGGL(average_lut_backward_small_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, dev_dy_buf, dev_dx_buf, dev_input_index,
+        launch(average_lut_backward_small_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, dev_dy_buf, dev_dx_buf, dev_input_index,
                            total, n, frame_size, frame_stride, f_blocks);
         BBHIP_LAUNCH_CHECK();
         return 0;
@@ -1735,10 +1750,10 @@ int bbhip_fp32_AverageLut_Backward(float const *dev_dy_buf, float *dev_dx_buf, i
     if (arena_get(offsets_bytes + sizeof(int) * (size_t)total, &scratch, static_cast<hipStream_t>(stream))) { return 1; }
     int *offsets = reinterpret_cast<int *>(scratch), *list = reinterpret_cast<int *>(scratch + offsets_bytes);
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    hipLaunchKernelGGL(average_lut_reverse_kernel, dim3((unsigned)ceil_div(input_node_size + 1, kTailBlock)), dim3(kTailBlock), 0, st,
+    launch(average_lut_reverse_kernel, dim3((unsigned)ceil_div(input_node_size + 1, kTailBlock)), dim3(kTailBlock), 0, st,
                        dev_input_index, total, n, input_node_size, offsets, list, 0);
     BBHIP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(average_lut_backward_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, dev_dy_buf, dev_dx_buf, offsets, list, n,
+    launch(average_lut_backward_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, dev_dy_buf, dev_dx_buf, offsets, list, n,
                        frame_size, frame_stride, f_blocks);
     BBHIP_LAUNCH_CHECK();
     return 0;
@@ -1753,7 +1768,7 @@ int bbhip_fp32_MaxLut_Forward(float const *dev_x_buf, float *dev_y_buf, int cons
     long long const blocks = (long long)node_size * f_blocks;
     if (blocks > 0x7fffffffLL) { return fail("%s: grid too large", __func__); }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    hipLaunchKernelGGL(max_lut_forward_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, static_cast<hipStream_t>(stream), dev_x_buf,
+    launch(max_lut_forward_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, static_cast<hipStream_t>(stream), dev_x_buf,
                        dev_y_buf, dev_input_index, n, frame_size, frame_stride, binarize_input, binarize_output, f_blocks);
     BBHIP_LAUNCH_CHECK();
     return 0;
@@ -1769,7 +1784,7 @@ int bbhip_bit_MaxLut_Forward(int const *dev_x_buf, int *dev_y_buf, int const *de
     long long const blocks = (long long)node_size * w_blocks;
     if (blocks > 0x7fffffffLL) { return fail("%s: grid too large", __func__); }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    hipLaunchKernelGGL(max_lut_forward_bit_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, static_cast<hipStream_t>(stream), dev_x_buf,
+    launch(max_lut_forward_bit_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, static_cast<hipStream_t>(stream), dev_x_buf,
                        dev_y_buf, dev_input_index, n, words, frame_stride, w_blocks);
     BBHIP_LAUNCH_CHECK();
     return 0;
@@ -1792,11 +1807,11 @@ static int launch_max_lut_backward(void const *x, bool bits, float const *dy, fl
     if (walk_whole_table(total, input_node_size, frame_size)) {
         ScopedTimer tm(kTimeOther, st);
         if (bits) {
-            hipLaunchKernelGGL(max_lut_backward_small_kernel<true>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, x, dy, dx, idx, total, n,
+            launch(max_lut_backward_small_kernel<true>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, x, dy, dx, idx, total, n,
                                frame_size, x_stride, dy_stride, 0, f_blocks);
         }
         else {
-            hipLaunchKernelGGL(max_lut_backward_small_kernel<false>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, x, dy, dx, idx, total, n,
+            launch(max_lut_backward_small_kernel<false>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, x, dy, dx, idx, total, n,
                                frame_size, x_stride, dy_stride, binarize_input, f_blocks);
         }
         BBHIP_LAUNCH_CHECK();
@@ -1807,15 +1822,15 @@ static int launch_max_lut_backward(void const *x, bool bits, float const *dy, fl
     if (arena_get(offsets_bytes + sizeof(int) * (size_t)total, &scratch, st)) { return 1; }
     int *offsets = reinterpret_cast<int *>(scratch), *list = reinterpret_cast<int *>(scratch + offsets_bytes);
     ScopedTimer tm(kTimeOther, st);
-    hipLaunchKernelGGL(average_lut_reverse_kernel, dim3((unsigned)ceil_div(input_node_size + 1, kTailBlock)), dim3(kTailBlock), 0, st,
+    launch(average_lut_reverse_kernel, dim3((unsigned)ceil_div(input_node_size + 1, kTailBlock)), dim3(kTailBlock), 0, st,
                        idx, total, n, input_node_size, offsets, list, 1);
     BBHIP_LAUNCH_CHECK();
     if (bits) {
-        hipLaunchKernelGGL(max_lut_backward_kernel<true>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, x, dy, dx, idx, offsets, list, n,
+        launch(max_lut_backward_kernel<true>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, x, dy, dx, idx, offsets, list, n,
                            frame_size, x_stride, dy_stride, 0, f_blocks);
     }
     else {
-        hipLaunchKernelGGL(max_lut_backward_kernel<false>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, x, dy, dx, idx, offsets, list, n,
+        launch(max_lut_backward_kernel<false>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, x, dy, dx, idx, offsets, list, n,
                            frame_size, x_stride, dy_stride, binarize_input, f_blocks);
     }
     BBHIP_LAUNCH_CHECK();
@@ -1852,8 +1867,8 @@ static int launch_reduce_forward(void const *x, bool bits, float *y, int input_n
     hipStream_t const st = static_cast<hipStream_t>(stream);
     int const mux = input_node_size / output_node_size;
     ScopedTimer tm(kTimeOther, st);
-    if (bits) { hipLaunchKernelGGL(reduce_forward_kernel<true>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, x, y, mux, output_node_size, frame_size, x_stride, y_stride, f_blocks); }
-    else      { hipLaunchKernelGGL(reduce_forward_kernel<false>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, x, y, mux, output_node_size, frame_size, x_stride, y_stride, f_blocks); }
+    if (bits) { launch(reduce_forward_kernel<true>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, x, y, mux, output_node_size, frame_size, x_stride, y_stride, f_blocks); }
+    else      { launch(reduce_forward_kernel<false>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, x, y, mux, output_node_size, frame_size, x_stride, y_stride, f_blocks); }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -1884,7 +1899,7 @@ int bbhip_fp32_Reduce_Backward(float const *dev_dy_buf, float *dev_dx_buf, int i
     long long const blocks = (long long)input_node_size * f_blocks;
     if (blocks > 0x7fffffffLL) { return fail("%s: grid too large", __func__); }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    hipLaunchKernelGGL(reduce_backward_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, static_cast<hipStream_t>(stream), dev_dy_buf, dev_dx_buf,
+    launch(reduce_backward_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, static_cast<hipStream_t>(stream), dev_dy_buf, dev_dx_buf,
                        input_node_size / output_node_size, output_node_size, frame_size, frame_stride, f_blocks);
     BBHIP_LAUNCH_CHECK();
     return 0;
@@ -1905,15 +1920,15 @@ static int launch_mean_squared_error(float const *y, float const *t, float *dy, 
     double *partial = reinterpret_cast<double *>(scratch);
     ScopedTimer tm(kTimeOther, st);
     if (loss) {
-        hipLaunchKernelGGL(mean_squared_error_kernel<true>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, y, t, dy, partial, grad_scale, loss_scale,
+        launch(mean_squared_error_kernel<true>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, y, t, dy, partial, grad_scale, loss_scale,
                            node_size, frame_size, frame_stride, f_blocks);
     }
     else {
-        hipLaunchKernelGGL(mean_squared_error_kernel<false>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, y, t, dy, partial, grad_scale, loss_scale,
+        launch(mean_squared_error_kernel<false>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, y, t, dy, partial, grad_scale, loss_scale,
                            node_size, frame_size, frame_stride, f_blocks);
     }
     BBHIP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(mean_squared_error_sum_kernel, dim3((unsigned)ceil_div(buf_size < frame_size ? buf_size : frame_size, kTailBlock)), dim3(kTailBlock),
+    launch(mean_squared_error_sum_kernel, dim3((unsigned)ceil_div(buf_size < frame_size ? buf_size : frame_size, kTailBlock)), dim3(kTailBlock),
                        0, st, partial, buf, buf_size, groups, frame_size);
     BBHIP_LAUNCH_CHECK();
     return 0;
@@ -1955,16 +1970,16 @@ int bbhip_fp32_LossSoftmaxCrossEntropy(float const *dev_y_buf, float const *dev_
     }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
     if (ch_size <= 16) {
-        hipLaunchKernelGGL(softmax_cross_entropy_few_kernel<16>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, dev_y_buf, dev_t_buf, dev_dy_buf,
+        launch(softmax_cross_entropy_few_kernel<16>, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, dev_y_buf, dev_t_buf, dev_dy_buf,
                            partial, t_sum, pix_size, ch_size, frame_size, frame_stride, f_blocks);
     }
     else {
-        hipLaunchKernelGGL(softmax_cross_entropy_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, dev_y_buf, dev_t_buf, dev_dy_buf, partial,
+        launch(softmax_cross_entropy_kernel, dim3((unsigned)blocks), dim3(kTailBlock), 0, st, dev_y_buf, dev_t_buf, dev_dy_buf, partial,
                            t_sum, pix_size, ch_size, frame_size, frame_stride, f_blocks);
     }
     BBHIP_LAUNCH_CHECK();
     if (pix_size > 1) {
-        hipLaunchKernelGGL(loss_pixel_sum_kernel, dim3((unsigned)f_blocks), dim3(kTailBlock), 0, st, partial, dev_loss_buf, pix_size, frame_size);
+        launch(loss_pixel_sum_kernel, dim3((unsigned)f_blocks), dim3(kTailBlock), 0, st, partial, dev_loss_buf, pix_size, frame_size);
         BBHIP_LAUNCH_CHECK();
     }
     return 0;
@@ -1990,7 +2005,7 @@ int bbhip_fp32_ClassifierTail_ForwardBackward(float const *dev_x_buf, float *dev
     size_t const lds = 5 * CH * 64 * sizeof(float) + (size_t)ch_size * n * sizeof(int);
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
-    hipLaunchKernelGGL(classifier_tail_kernel<CH>, dim3((unsigned)ceil_div(frame_stride, 64)), dim3(64 * CH), lds, st, dev_x_buf, dev_y_buf, dev_dx_buf,
+    launch(classifier_tail_kernel<CH>, dim3((unsigned)ceil_div(frame_stride, 64)), dim3(64 * CH), lds, st, dev_x_buf, dev_y_buf, dev_dx_buf,
                        dev_input_index, dev_t_buf, dev_dy_buf, dev_loss_buf, dev_accuracy_buf, dev_category_buf, t_sum,
                        output_sum ? 1.0f : 1.0f / (float)n, n, input_node_size, ch_size, frame_size, frame_stride, binarize_input);
     BBHIP_LAUNCH_CHECK();
@@ -2006,7 +2021,7 @@ int bbhip_fp32_MetricsCategoricalAccuracy(float const *dev_y_buf, float const *d
     if (frame_stride < frame_size) { return fail("%s: frame stride shorter than the frames", __func__); }
     if ((long long)pix_size * ch_size > 0x7fffffffLL) { return fail("%s: node count too large", __func__); }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));
-    hipLaunchKernelGGL(categorical_accuracy_kernel, dim3((unsigned)ceil_div(frame_size, kTailBlock)), dim3(kTailBlock), 0,
+    launch(categorical_accuracy_kernel, dim3((unsigned)ceil_div(frame_size, kTailBlock)), dim3(kTailBlock), 0,
                        static_cast<hipStream_t>(stream), dev_y_buf, dev_t_buf, dev_accuracy_buf, dev_category_buf, pix_size, ch_size, frame_size,
                        frame_stride);
     BBHIP_LAUNCH_CHECK();
@@ -2038,8 +2053,8 @@ static int launch_bn_rows(BnArgs const &a, int node_size, bool backward, void *s
     ScopedTimer tm(kTimeOther, st);
 #define BBHIP_BN_ROWS(W, HELD)                                                                                  \
     do {                                                                                                        \
-        if (backward) { hipLaunchKernelGGL((bn_backward_kernel<W, HELD>), grid, block, 0, st, a); }             \
-        else          { hipLaunchKernelGGL((bn_forward_training_kernel<W, HELD>), grid, block, 0, st, a); }     \
+        if (backward) { launch((bn_backward_kernel<W, HELD>), grid, block, 0, st, a); }             \
+        else          { launch((bn_forward_training_kernel<W, HELD>), grid, block, 0, st, a); }     \
     } while (0)
     if (wide) { if (held) { BBHIP_BN_ROWS(4, true); } else { BBHIP_BN_ROWS(4, false); } }
     else      { if (held) { BBHIP_BN_ROWS(1, true); } else { BBHIP_BN_ROWS(1, false); } }
@@ -2058,12 +2073,12 @@ static int launch_bn_apply(BnArgs const &a, int node_size, bool from_running, vo
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
     if (wide) {
-        if (from_running) { hipLaunchKernelGGL((bn_apply_kernel<4, true>), grid, block, 0, st, a, f_blocks); }
-        else              { hipLaunchKernelGGL((bn_apply_kernel<4, false>), grid, block, 0, st, a, f_blocks); }
+        if (from_running) { launch((bn_apply_kernel<4, true>), grid, block, 0, st, a, f_blocks); }
+        else              { launch((bn_apply_kernel<4, false>), grid, block, 0, st, a, f_blocks); }
     }
     else {
-        if (from_running) { hipLaunchKernelGGL((bn_apply_kernel<1, true>), grid, block, 0, st, a, f_blocks); }
-        else              { hipLaunchKernelGGL((bn_apply_kernel<1, false>), grid, block, 0, st, a, f_blocks); }
+        if (from_running) { launch((bn_apply_kernel<1, true>), grid, block, 0, st, a, f_blocks); }
+        else              { launch((bn_apply_kernel<1, false>), grid, block, 0, st, a, f_blocks); }
     }
     BBHIP_LAUNCH_CHECK();
     return 0;
@@ -2158,8 +2173,8 @@ static int launch_row_map(int op, float const *x, float const *dy, float *out, f
     dim3 const grid(blocks), block(kModBlock);
 #define BBHIP_ROW_MAP(OP)                                                                               \
     do {                                                                                                \
-        if (wide) { hipLaunchKernelGGL((row_map_kernel<OP, 4>), grid, block, 0, st, a); }               \
-        else      { hipLaunchKernelGGL((row_map_kernel<OP, 1>), grid, block, 0, st, a); }               \
+        if (wide) { launch((row_map_kernel<OP, 4>), grid, block, 0, st, a); }               \
+        else      { launch((row_map_kernel<OP, 1>), grid, block, 0, st, a); }               \
     } while (0)
     switch (op) {
     case kMapBinarize:  BBHIP_ROW_MAP(kMapBinarize); break;
@@ -2193,8 +2208,8 @@ int bbhip_fp32_bit_Binarize_Forward(float const *dev_x_buf, int *dev_y_buf, floa
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
     uint32_t *const y = reinterpret_cast<uint32_t *>(dev_y_buf);
-    if (wide) { hipLaunchKernelGGL((binarize_bits_kernel<4>), dim3(blocks), dim3(kModBlock), 0, st, dev_x_buf, y, binary_th, frame_size, x_frame_stride, y_frame_stride, f_blocks); }
-    else      { hipLaunchKernelGGL((binarize_bits_kernel<1>), dim3(blocks), dim3(kModBlock), 0, st, dev_x_buf, y, binary_th, frame_size, x_frame_stride, y_frame_stride, f_blocks); }
+    if (wide) { launch((binarize_bits_kernel<4>), dim3(blocks), dim3(kModBlock), 0, st, dev_x_buf, y, binary_th, frame_size, x_frame_stride, y_frame_stride, f_blocks); }
+    else      { launch((binarize_bits_kernel<1>), dim3(blocks), dim3(kModBlock), 0, st, dev_x_buf, y, binary_th, frame_size, x_frame_stride, y_frame_stride, f_blocks); }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -2247,9 +2262,9 @@ static int launch_real_to_binary(float const *x, void *y, bool bit, bool zero_pa
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
     dim3 const grid(blocks), block(kModBlock);
-    if (bit)       { hipLaunchKernelGGL((real_to_binary_kernel<true, 4>), grid, block, 0, st, a); }
-    else if (wide) { hipLaunchKernelGGL((real_to_binary_kernel<false, 4>), grid, block, 0, st, a); }
-    else           { hipLaunchKernelGGL((real_to_binary_kernel<false, 1>), grid, block, 0, st, a); }
+    if (bit)       { launch((real_to_binary_kernel<true, 4>), grid, block, 0, st, a); }
+    else if (wide) { launch((real_to_binary_kernel<false, 4>), grid, block, 0, st, a); }
+    else           { launch((real_to_binary_kernel<false, 1>), grid, block, 0, st, a); }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -2301,8 +2316,8 @@ static int launch_binary_to_real_forward(void const *x, bool bit, float *y, int 
     if (modulation_grid(y_node_size, y_frame_size, false, a.f_blocks, blocks, name)) { return 1; }
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
-    if (bit) { hipLaunchKernelGGL((binary_to_real_forward_kernel<true>), dim3(blocks), dim3(kModBlock), 0, st, a); }
-    else     { hipLaunchKernelGGL((binary_to_real_forward_kernel<false>), dim3(blocks), dim3(kModBlock), 0, st, a); }
+    if (bit) { launch((binary_to_real_forward_kernel<true>), dim3(blocks), dim3(kModBlock), 0, st, a); }
+    else     { launch((binary_to_real_forward_kernel<false>), dim3(blocks), dim3(kModBlock), 0, st, a); }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -2341,8 +2356,8 @@ int bbhip_fp32_BinaryToReal_Backward(float const *dev_dy_buf, float *dev_dx_buf,
     if (modulation_grid(node_mux_size * y_node_size, x_frame_size, wide, a.f_blocks, blocks, __func__)) { return 1; }
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
-    if (wide) { hipLaunchKernelGGL((binary_to_real_backward_kernel<4>), dim3(blocks), dim3(kModBlock), 0, st, a, x_frame_size); }
-    else      { hipLaunchKernelGGL((binary_to_real_backward_kernel<1>), dim3(blocks), dim3(kModBlock), 0, st, a, x_frame_size); }
+    if (wide) { launch((binary_to_real_backward_kernel<4>), dim3(blocks), dim3(kModBlock), 0, st, a, x_frame_size); }
+    else      { launch((binary_to_real_backward_kernel<1>), dim3(blocks), dim3(kModBlock), 0, st, a, x_frame_size); }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -2403,10 +2418,10 @@ int bbhip_fp32_MaxPooling_Forward(float const *dev_x_buf, float *dev_y_buf, int 
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
     dim3 const grid(blocks), block(kPoolBlock);
-    if (wide) { if (two) { hipLaunchKernelGGL((max_pooling_forward_kernel<4, true>), grid, block, 0, st, a); }
-                else     { hipLaunchKernelGGL((max_pooling_forward_kernel<4, false>), grid, block, 0, st, a); } }
-    else      { if (two) { hipLaunchKernelGGL((max_pooling_forward_kernel<1, true>), grid, block, 0, st, a); }
-                else     { hipLaunchKernelGGL((max_pooling_forward_kernel<1, false>), grid, block, 0, st, a); } }
+    if (wide) { if (two) { launch((max_pooling_forward_kernel<4, true>), grid, block, 0, st, a); }
+                else     { launch((max_pooling_forward_kernel<4, false>), grid, block, 0, st, a); } }
+    else      { if (two) { launch((max_pooling_forward_kernel<1, true>), grid, block, 0, st, a); }
+                else     { launch((max_pooling_forward_kernel<1, false>), grid, block, 0, st, a); } }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -2429,7 +2444,7 @@ int bbhip_bit_MaxPooling_Forward(int const *dev_x_buf, int *dev_y_buf, int filte
     if (window_grid_flat(a, c_size, output_h_size, output_w_size, words, blocks, total, __func__)) { return 1; }
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
-    hipLaunchKernelGGL(max_pooling_bit_forward_kernel, dim3(blocks), dim3(kPoolBlock), 0, st, a, words, total);
+    launch(max_pooling_bit_forward_kernel, dim3(blocks), dim3(kPoolBlock), 0, st, a, words, total);
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -2451,8 +2466,8 @@ int bbhip_fp32_MaxPooling_Backward(int const *dev_argmax_buf, float const *dev_d
     if (window_grid(a, c_size, output_h_size, output_w_size, frame_size, wide ? 4 : 1, blocks, __func__)) { return 1; }
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
-    if (wide) { hipLaunchKernelGGL((max_pooling_backward_kernel<4>), dim3(blocks), dim3(kPoolBlock), 0, st, a); }
-    else      { hipLaunchKernelGGL((max_pooling_backward_kernel<1>), dim3(blocks), dim3(kPoolBlock), 0, st, a); }
+    if (wide) { launch((max_pooling_backward_kernel<4>), dim3(blocks), dim3(kPoolBlock), 0, st, a); }
+    else      { launch((max_pooling_backward_kernel<1>), dim3(blocks), dim3(kPoolBlock), 0, st, a); }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -2473,7 +2488,7 @@ int bbhip_bit_fp32_MaxPooling_Backward(int const *dev_x_buf, float const *dev_dy
     if (window_grid(a, c_size, output_h_size, output_w_size, frame_size, 1, blocks, __func__)) { return 1; }
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
-    hipLaunchKernelGGL(max_pooling_bit_backward_kernel, dim3(blocks), dim3(kPoolBlock), 0, st, a);
+    launch(max_pooling_bit_backward_kernel, dim3(blocks), dim3(kPoolBlock), 0, st, a);
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -2501,17 +2516,17 @@ static int launch_up_sampling(void const *x, float const *dy, void *out, bool bi
     if (backward) {
         if (window_grid(a, c_size, input_h_size, input_w_size, items, wide ? 4 : 1, blocks, name)) { return 1; }
         ScopedTimer tm(kTimeOther, st);
-        if (wide) { hipLaunchKernelGGL((up_sampling_backward_kernel<4>), dim3(blocks), dim3(kPoolBlock), 0, st, a); }
-        else      { hipLaunchKernelGGL((up_sampling_backward_kernel<1>), dim3(blocks), dim3(kPoolBlock), 0, st, a); }
+        if (wide) { launch((up_sampling_backward_kernel<4>), dim3(blocks), dim3(kPoolBlock), 0, st, a); }
+        else      { launch((up_sampling_backward_kernel<1>), dim3(blocks), dim3(kPoolBlock), 0, st, a); }
     }
     else {
         long long total = 0;
         if (bit) { if (window_grid_flat(a, c_size, input_h_size * filter_h_size, input_w_size * filter_w_size, items, blocks, total, name)) { return 1; } }
         else if (window_grid(a, c_size, input_h_size * filter_h_size, input_w_size * filter_w_size, items, wide ? 4 : 1, blocks, name)) { return 1; }
         ScopedTimer tm(kTimeOther, st);
-        if (bit)       { hipLaunchKernelGGL((up_sampling_forward_kernel<true, 1>), dim3(blocks), dim3(kPoolBlock), 0, st, a, items, total); }
-        else if (wide) { hipLaunchKernelGGL((up_sampling_forward_kernel<false, 4>), dim3(blocks), dim3(kPoolBlock), 0, st, a, items, total); }
-        else           { hipLaunchKernelGGL((up_sampling_forward_kernel<false, 1>), dim3(blocks), dim3(kPoolBlock), 0, st, a, items, total); }
+        if (bit)       { launch((up_sampling_forward_kernel<true, 1>), dim3(blocks), dim3(kPoolBlock), 0, st, a, items, total); }
+        else if (wide) { launch((up_sampling_forward_kernel<false, 4>), dim3(blocks), dim3(kPoolBlock), 0, st, a, items, total); }
+        else           { launch((up_sampling_forward_kernel<false, 1>), dim3(blocks), dim3(kPoolBlock), 0, st, a, items, total); }
     }
     BBHIP_LAUNCH_CHECK();
     return 0;
@@ -2560,8 +2575,8 @@ static int launch_shuffle(int const *src, int *dst, unsigned unit_size, unsigned
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
     dim3 const grid((unsigned)((total + kPoolBlock - 1) / kPoolBlock)), block(kPoolBlock);
-    if (wide) { hipLaunchKernelGGL(row_shuffle_kernel<4>, grid, block, 0, st, a, total); }
-    else      { hipLaunchKernelGGL(row_shuffle_kernel<1>, grid, block, 0, st, a, total); }
+    if (wide) { launch(row_shuffle_kernel<4>, grid, block, 0, st, a, total); }
+    else      { launch(row_shuffle_kernel<1>, grid, block, 0, st, a, total); }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -2592,7 +2607,7 @@ int bbhip_fp32_ConvBitToReal(int const *dev_x_buf, float *dev_y_buf, float value
     // grid.y is limited to 65535 rows per launch
     for (int n0 = 0; n0 < node_size; n0 += 65535) {
         int const rows = (node_size - n0 < 65535) ? node_size - n0 : 65535;
-        hipLaunchKernelGGL(conv_bit_to_real_kernel, dim3(ceil_div(frame_size, kBlock), rows), dim3(kBlock), 0, static_cast<hipStream_t>(stream),
+        launch(conv_bit_to_real_kernel, dim3(ceil_div(frame_size, kBlock), rows), dim3(kBlock), 0, static_cast<hipStream_t>(stream),
                            reinterpret_cast<uint32_t const *>(dev_x_buf) + (size_t)n0 * x_frame_stride,
                            dev_y_buf + (size_t)n0 * y_frame_stride, value0, value1, frame_size, x_frame_stride, y_frame_stride);
         BBHIP_LAUNCH_CHECK();
@@ -2910,16 +2925,16 @@ int bbhip_bit_BinaryLut6_Forward(int const *dev_x_buf, int *dev_y_buf, int const
         bool const exact = (node_size % npw) == 0;
         bool const pad = zero_padding && frame_stride > a.word_count;
         switch (npw) {
-        case 1: if (pad) { hipLaunchKernelGGL((binary_lut6_kernel<1, true, true>), grid, block, 0, st, a); }
-                else     { hipLaunchKernelGGL((binary_lut6_kernel<1, true>), grid, block, 0, st, a); }
+        case 1: if (pad) { launch((binary_lut6_kernel<1, true, true>), grid, block, 0, st, a); }
+                else     { launch((binary_lut6_kernel<1, true>), grid, block, 0, st, a); }
                 break;
-        case 2: if (pad)        { hipLaunchKernelGGL((binary_lut6_kernel<2, false, true>), grid, block, 0, st, a); }
-                else if (exact) { hipLaunchKernelGGL((binary_lut6_kernel<2, true>), grid, block, 0, st, a); }
-                else       { hipLaunchKernelGGL((binary_lut6_kernel<2, false>), grid, block, 0, st, a); }
+        case 2: if (pad)        { launch((binary_lut6_kernel<2, false, true>), grid, block, 0, st, a); }
+                else if (exact) { launch((binary_lut6_kernel<2, true>), grid, block, 0, st, a); }
+                else       { launch((binary_lut6_kernel<2, false>), grid, block, 0, st, a); }
                 break;
-        default: if (pad)       { hipLaunchKernelGGL((binary_lut6_kernel<4, false, true>), grid, block, 0, st, a); }
-                 else if (exact) { hipLaunchKernelGGL((binary_lut6_kernel<4, true>), grid, block, 0, st, a); }
-                 else       { hipLaunchKernelGGL((binary_lut6_kernel<4, false>), grid, block, 0, st, a); }
+        default: if (pad)       { launch((binary_lut6_kernel<4, false, true>), grid, block, 0, st, a); }
+                 else if (exact) { launch((binary_lut6_kernel<4, true>), grid, block, 0, st, a); }
+                 else       { launch((binary_lut6_kernel<4, false>), grid, block, 0, st, a); }
                  break;
         }
     }
@@ -2945,10 +2960,10 @@ int bbhip_bit_BinaryLutN_Forward(int n, int const *dev_x_buf, int *dev_y_buf, in
     for (int n0 = 0; n0 < node_size; n0 += 65535) {            // grid.y is limited to 65535 nodes per launch
         dim3 const grid(ceil_div(words, kBlock), (node_size - n0 < 65535) ? node_size - n0 : 65535), block(kBlock);
         switch (n) {
-        case 2: hipLaunchKernelGGL(binary_lutn_kernel<2>, grid, block, 0, st, x, y, dev_input_index, dev_table, n0, frame_size, frame_stride); break;
-        case 3: hipLaunchKernelGGL(binary_lutn_kernel<3>, grid, block, 0, st, x, y, dev_input_index, dev_table, n0, frame_size, frame_stride); break;
-        case 4: hipLaunchKernelGGL(binary_lutn_kernel<4>, grid, block, 0, st, x, y, dev_input_index, dev_table, n0, frame_size, frame_stride); break;
-        default: hipLaunchKernelGGL(binary_lutn_kernel<5>, grid, block, 0, st, x, y, dev_input_index, dev_table, n0, frame_size, frame_stride); break;
+        case 2: launch(binary_lutn_kernel<2>, grid, block, 0, st, x, y, dev_input_index, dev_table, n0, frame_size, frame_stride); break;
+        case 3: launch(binary_lutn_kernel<3>, grid, block, 0, st, x, y, dev_input_index, dev_table, n0, frame_size, frame_stride); break;
+        case 4: launch(binary_lutn_kernel<4>, grid, block, 0, st, x, y, dev_input_index, dev_table, n0, frame_size, frame_stride); break;
+        default: launch(binary_lutn_kernel<5>, grid, block, 0, st, x, y, dev_input_index, dev_table, n0, frame_size, frame_stride); break;
         }
         BBHIP_LAUNCH_CHECK();
     }

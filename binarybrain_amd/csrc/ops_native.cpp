@@ -13,6 +13,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -166,10 +167,12 @@ PyObject *wrapped(PyObject *, PyObject *const *args, Py_ssize_t n)
 }
 
 // ---- buffers -------------------------------------------------------------------------------------------------------------------
-at::Tensor rows_f32(T like, int64_t rows, int64_t stride) { return at::empty({rows, stride}, like.options().dtype(at::kFloat)); }
-at::Tensor rows_i32(T like, int64_t rows, int64_t words)  { return at::empty({rows, words}, like.options().dtype(at::kInt)); }
+// (what at::empty comes to for device tensors, without the dispatcher's passes)
+at::Tensor new_tensor(T like, at::IntArrayRef sizes, at::ScalarType type) { return at::Tensor(at::detail::empty_cuda(sizes, type, like.device(), std::nullopt)); }
+at::Tensor rows_f32(T like, int64_t rows, int64_t stride) { return new_tensor(like, {rows, stride}, at::kFloat); }
+at::Tensor rows_i32(T like, int64_t rows, int64_t words)  { return new_tensor(like, {rows, words}, at::kInt); }
 at::Tensor zeros_i32(T like, int64_t rows, int64_t words) { return at::zeros({rows, words}, like.options().dtype(at::kInt)); }
-at::Tensor line_f32(T like, int64_t n) { return at::empty({n}, like.options().dtype(at::kFloat)); }
+at::Tensor line_f32(T like, int64_t n) { return new_tensor(like, {n}, at::kFloat); }
 
 template <class E> E *data(T t) { return static_cast<E *>(t.data_ptr()); }
 template <class E> E *data(OptTensor t) { return t ? static_cast<E *>((*t).data_ptr()) : nullptr; }
@@ -366,14 +369,24 @@ at::Tensor differentiable_lut_forward_nobn(int n, T x, T idx, T W, int frames, f
     return y;
 }
 
-// dmean and dvar are scratch of the call: the two halves of one buffer
+// dmean and dvar are scratch of the call, the two halves of one buffer; the library writes them only where a node has more than 256 units of at
+// least 64 frames.  Below, the call gets an address that it does not touch.
+struct SumsScratch { at::Tensor t; float *p; };
+SumsScratch sums_scratch(T like, int nodes, int frames, float *untouched)
+{
+    if (frames <= 256 * 64) { return SumsScratch{at::Tensor(), untouched}; }
+    SumsScratch s{line_f32(like, 2 * (int64_t)nodes), nullptr};
+    s.p = data<float>(s.t);
+    return s;
+}
+
 at::Tensor differentiable_lut_backward(int n, T x, T dy, T idx, T W, T dW, int frames, T mean, T rstd, OptTensor rev, float gamma, float beta, float bias,
                                        bool lut_binarize, bool binary_mode, double max_tmp_bytes, OptTensor packed, OptTensor tables, bool overwrite,
                                        bool hints)
 {
     int const I = rows_of(x), O = rows_of(idx), S = stride_of(dy);
     at::Tensor dx = rows_f32(x, I, S);
-    at::Tensor const sums = line_f32(x, 2 * (int64_t)O);
+    SumsScratch const sums = sums_scratch(x, O, frames, data<float>(dx));
     DxTmp const tmp = dx_tmp_of(x, O, n, frames, (int64_t)max_tmp_bytes);
     if (hints) {
         hint_input(x, packed, true, false);
@@ -381,8 +394,8 @@ at::Tensor differentiable_lut_backward(int n, T x, T dy, T idx, T W, T dW, int f
     }
     if (overwrite) { bbhip_HintTableGradientOverwrite(1); }
     call(bbhip_fp32_DifferentiableLutN_Backward, n, data<float const>(x), data<float const>(dy), data<float>(dx), tmp.p, data<int const>(idx),
-         data<int const>(rev), data<float const>(W), data<float>(dW), data<float const>(mean), data<float const>(rstd), data<float>(sums),
-         data<float>(sums) + O, gamma, beta, bias, rev ? stride_of(*rev) : 0, I, O, frames, S, tmp.frames, tmp.stride, (int)lut_binarize, (int)binary_mode,
+         data<int const>(rev), data<float const>(W), data<float>(dW), data<float const>(mean), data<float const>(rstd), sums.p, sums.p + O,
+         gamma, beta, bias, rev ? stride_of(*rev) : 0, I, O, frames, S, tmp.frames, tmp.stride, (int)lut_binarize, (int)binary_mode,
          current_stream());
     return dx;
 }
@@ -392,12 +405,12 @@ at::Tensor bit_differentiable_lut_backward(int n, T x, T dy, T idx, T W, T dW, i
 {
     int const I = rows_of(x), O = rows_of(idx), S = stride_of(dy);
     at::Tensor dx = rows_f32(dy, I, S);
-    at::Tensor const sums = line_f32(dy, 2 * (int64_t)O);
+    SumsScratch const sums = sums_scratch(dy, O, frames, data<float>(dx));
     DxTmp const tmp = dx_tmp_of(dy, O, n, frames, (int64_t)max_tmp_bytes);
     if (hints) { hint_tables(tables, true); }
     call(bbhip_bit_fp32_DifferentiableLutN_Backward, n, data<int const>(x), data<float const>(dy), data<float>(dx), tmp.p, data<int const>(idx),
-         data<int const>(rev), data<float const>(W), data<float>(dW), data<float const>(mean), data<float const>(rstd), data<float>(sums),
-         data<float>(sums) + O, gamma, beta, bias, rev ? stride_of(*rev) : 0, I, O, frames, S, stride_of(x), tmp.frames, tmp.stride, (int)lut_binarize,
+         data<int const>(rev), data<float const>(W), data<float>(dW), data<float const>(mean), data<float const>(rstd), sums.p, sums.p + O,
+         gamma, beta, bias, rev ? stride_of(*rev) : 0, I, O, frames, S, stride_of(x), tmp.frames, tmp.stride, (int)lut_binarize,
          current_stream());
     return dx;
 }
@@ -416,10 +429,10 @@ classifier_tail(T x, T idx, T t, int frames, float t_sum, bool input_binary, boo
 {
     int const ch = rows_of(idx), n = stride_of(idx), S = stride_of(x), I = rows_of(x);
     require(t.size(1) == S, "classifier_tail: t must have the row pitch of x");
-    at::Tensor y, dy, accuracy, category, dx = rows_f32(x, I, S), loss = at::empty({frames}, x.options().dtype(at::kDouble));
+    at::Tensor y, dy, accuracy, category, dx = rows_f32(x, I, S), loss = new_tensor(x, {frames}, at::kDouble);
     if (want_y)  { y = rows_f32(x, ch, S); }
     if (want_dy) { dy = rows_f32(x, ch, S); }
-    if (want_accuracy) { accuracy = at::empty({frames}, x.options().dtype(at::kInt)); category = at::empty({frames}, x.options().dtype(at::kInt)); }
+    if (want_accuracy) { accuracy = new_tensor(x, {frames}, at::kInt); category = new_tensor(x, {frames}, at::kInt); }
     auto const f = [](at::Tensor const &a) { return a.defined() ? data<float>(a) : nullptr; };
     auto const i = [](at::Tensor const &a) { return a.defined() ? data<int>(a) : nullptr; };
     call(bbhip_fp32_ClassifierTail_ForwardBackward, data<float const>(x), f(y), data<float>(dx), data<int const>(idx), data<float const>(t), f(dy),
