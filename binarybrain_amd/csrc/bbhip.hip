@@ -19,6 +19,7 @@
 #include "corner_forward_kernels.hpp"
 #include "corner_backward_kernels.hpp"
 #include "table_gradient_kernels.hpp"
+#include "small_backward_kernels.hpp"
 #include "vector_kernels.hpp"
 #include "conv_kernels.hpp"
 #include "tail_kernels.hpp"
@@ -580,9 +581,10 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
                                     c.W, C, V, c.node_size, c.lut_binarize, c.bias, st, c.clamp_W, c.clamp_lo, c.clamp_hi)) { return 1; }
         c.x = bits;
     }
-    // plain output of a call with one unit per node on the polynomial kernel: the wavefronts prepare their node's table
-    // themselves (FwdArgs::W_inline), clamp it in place where the entry asks for that, and the table launch falls away
-    bool const inline_table = (c.bn == 0) && !corner && chunk_count == 1 && LutMatrixQ<N>::kUsable && !tables_to_caller;
+    // plain output on the polynomial kernel: the wavefronts prepare their node's table themselves (FwdArgs::W_inline), clamp it in place where the
+    // entry asks for that, and the table launch falls away.  In calls of many units the butterfly in each of them costs more than the launch
+    // (4096 nodes x 8192 frames, 131072 units: + 11 us against 5); at 48000 units the two are equal, at 12000 it saves 1.5 us of 34.
+    bool const inline_table = (c.bn == 0) && !corner && (long long)chunk_count * c.node_size <= (1 << 15) && !tables_to_caller;
     // the corner-value kernel derives a node's tables in the wavefront in any case where no packing launch is there to carry the
     // preparation: the first launch of the call does it and stores them for the launches (and the backward call) that follow
     bool const inline_corner = corner && !pack && inline_tables();
@@ -868,6 +870,59 @@ void launch_node_gradient(BackwardCall const &c, BwdArgs const &a, float const *
     launch(lut_node_gradient_kernel<N>, dim3(g.tt.blocks + g.node_tiles), dim3(per_block * g.node_waves * kWave), 0, st, g);
 }
 
+// Plain layers on real-valued inputs whose backward pass is one launch (lut_small_backward_kernel).  Per frame that kernel does more than the two
+// launches of larger layers, the more so the wider the table: 1024 nodes x 1000 frames 25.0 us a training step instead of 29.2, 1000 x 2000 39.2 and 38.5,
+// 2000 x 2000 67 and 63; four inputs per node 1531 x 1999 31.0 instead of 33.1, 4000 x 4000 144 and 134; three inputs 2000 x 4000 53.7 instead of 55.1.
+// Long work lists (40 inputs, 2000 nodes of five, 1300 frames) 44 and 38.
+bool small_plain_layer(BackwardCall const &c)
+{
+    if (c.bn || c.xmode != kXClamp || bwd_slab_frames() > 0 || dx_chunk_frames_env() > 0 || dx_pass_steps_env() > 0) { return false; }
+    if ((long long)c.input_node_size * c.x_stride >= (1LL << 30) || (long long)c.output_node_size * c.frame_stride >= (1LL << 30)) { return false; }
+    long long const node_frames = (long long)c.output_node_size * c.frame_size;
+    if (c.rev_stride > 32 && node_frames > (5LL << 18)) { return false; }
+    return node_frames << c.n <= (c.n >= 5 ? 5LL << 24 : 1LL << 26);
+}
+
+template <int N>
+int run_backward_small(BackwardCall const &c, hipStream_t st, int dw_overwrite)
+{
+    SmallBackwardArgs s{};
+    DxArgs &d = s.dx;
+    d.x = c.x; d.dy = c.dy; d.dx = c.dx; d.rev = c.rev; d.rev_stride = c.rev_stride; d.input_node_size = c.input_node_size; d.frame_size = c.frame_size;
+    d.x_stride = c.x_stride; d.dy_stride = c.frame_stride; d.dx_stride = c.frame_stride;
+    // Wavefront-steps per unit: a term's coefficients serve that many, as long as a workgroup for each compute unit remains (where workgroups share
+    // work lists, four at four steps): 300 inputs x 500 frames 17.8 / 16.8 / 18.7 us in steps of 1 / 2 / 4 (2400 / 1200 / 600 workgroups), 1024 x 1000
+    // 30.1 / 26.2 / 25.0 (4096 / 2048 / 1024), 100 x 300 11.5 / 12.7 / 15.4 (125 / 75 / 50).
+    int steps = 4, in_tiles = 0;
+    for (;; steps /= 2) {
+        d.chunk = steps * kWave; d.chunk_count = ceil_div(c.frame_size, d.chunk);
+        d.split = dx_split_lists(c.rev_stride - 1, c.input_node_size, c.output_node_size, c.frame_size, d.chunk_count);
+        in_tiles = d.split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
+        bool const enough = (long long)d.chunk_count * in_tiles >= ((d.split && steps == 4) ? 1024 : 256) && c.frame_size > d.chunk / 2;
+        if (steps == 1 || enough) { break; }
+    }
+    d.tiles = make_tile_divisor(in_tiles);
+    s.idx = c.idx; s.W = c.W; s.lut_binarize = c.lut_binarize; s.node_size = c.output_node_size; s.dW = c.dW; s.overwrite = dw_overwrite;
+    int const waves = d.split > kWavesPerBlk ? kDxWaves : kWavesPerBlk;
+    s.node_waves = 1;
+    while (s.node_waves < waves && s.node_waves * 4 * kWave < c.frame_size) { s.node_waves *= 2; }
+    s.node_tiles = ceil_div(c.output_node_size, waves / s.node_waves);
+    if ((long long)s.node_tiles + (long long)d.chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
+    dim3 const grid(s.node_tiles + d.chunk_count * in_tiles), block(waves * kWave);
+    {
+        ScopedTimer tm(kTimeBackward, st);
+#define BBHIP_SMALL_CASE(U)                                                                                                  \
+        if (waves > kWavesPerBlk) { launch((lut_small_backward_kernel<N, U, kDxWaves>), grid, block, 0, st, s); }            \
+        else                      { launch((lut_small_backward_kernel<N, U, kWavesPerBlk>), grid, block, 0, st, s); }
+        if (steps == 1)      { BBHIP_SMALL_CASE(1) }
+        else if (steps == 2) { BBHIP_SMALL_CASE(2) }
+        else                 { BBHIP_SMALL_CASE(4) }
+#undef BBHIP_SMALL_CASE
+    }
+    BBHIP_LAUNCH_CHECK();
+    return 0;
+}
+
 template <int N>
 int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packed = PackedInputHint{nullptr, 0, 0, 0},
                  PreparedTablesHint tables = PreparedTablesHint{nullptr, 0, 0}, int dw_overwrite = 0)
@@ -888,6 +943,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         if (slots > 8 * links + 65536) { dxmode = (call.dx_tmp != nullptr && call.tmp_frame_size > 0) ? kDxTmp : kDxAtomic; }
     }
     if (check_backward(call, dxmode)) { return 1; }
+    if (dxmode == kDxNone && small_plain_layer(call)) { return run_backward_small<N>(call, st, dw_overwrite); }
 
     BackwardCall const &c = call;
     int const tile_count = ceil_div(c.output_node_size, kWavesPerBlk);

@@ -244,10 +244,10 @@ struct FwdArgs {
                                 // kStatPartial: from the partial sums that a kind 2 launch of the same shape left in stat_partial
     float momentum;             // kStatPartial: the wavefront of a node's first unit also stores the statistics:
     float *mean_out, *rstd_out, *running_mean, *running_var;
-    // Not null (plain output, one unit per node, widths whose table fits one vector register): no table-preparation launch has
-    // run; the wavefront brings its node's table W' into the centred basis itself — 2^N loads, one per lane, and the
-    // butterfly of table_prep_block over the lanes.  A call of a few hundred frames is two launches' worth of latency, not work.
-    // With clamp_W (below) the table is first clamped and written back, as in the corner-value kernel.
+    // Not null (plain output of calls of few units): no table-preparation launch has run; the wavefront brings its node's table W' into
+    // the centred basis itself — 2^N loads, one per lane, and the butterfly of table_prep_block over the lanes.  A call of a few hundred
+    // frames is two launches' worth of latency, not work.  With clamp_W (below) the table is first clamped, and written back by the wavefront
+    // of the node's first unit (the others read either value and clamp it too), as in the corner-value kernel.
     float const *W_inline;
     int   lut_binarize;
     // lut_forward_corner_kernel with W_inline: the node's tables go to C_out / V_out as well (the wavefront of the node's first unit
@@ -479,21 +479,21 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
     }
 #pragma unroll
     for (int p = 0; p < NPW; ++p) {
+        bool const derive = FWD_KIND == 0 && a.W_inline != nullptr;
+        float v = 0.0f;
+        if (derive) {
+            v = a.W_inline[(size_t)node[p] * D::NN + (lane & (D::NN - 1))];
+            if (a.clamp_W != nullptr) {                       // the table clamped in place as well, by the wavefront of the node's first unit
+                float const wc = fminf(a.clamp_hi, fmaxf(a.clamp_lo, v));
+                clamp_store[p] = (ck == 0) && live[p] && (lane < D::NN) && (wc != v);
+                v = wc;
+                clamp_w[p] = wc;
+            }
+            if (a.lut_binarize) { v = (v > 0.5f) ? 1.0f : 0.0f; }
+            v = centred_butterfly<N>(v, lane);
+        }
         if constexpr (kMatrix) {
-            if (FWD_KIND == 0 && a.W_inline != nullptr) {
-                float v = a.W_inline[(size_t)node[p] * D::NN + (lane & (D::NN - 1))];
-                if (a.clamp_W != nullptr) {                   // the table clamped in place as well, by the wavefront of the node's first unit
-                    float const wc = fminf(a.clamp_hi, fmaxf(a.clamp_lo, v));
-                    clamp_store[p] = (ck == 0) && live[p] && (lane < D::NN) && (wc != v);
-                    v = wc;
-                    clamp_w[p] = wc;
-                }
-                if (a.lut_binarize) { v = (v > 0.5f) ? 1.0f : 0.0f; }
-#pragma unroll
-                for (int j = 0; j < N; ++j) {                 // as table_prep_block: (a, b) -> ((a + b) / 2, b - a) per index bit
-                    float const o = lane_xor(v, 1 << j);
-                    v = ((lane >> j) & 1) ? (v - o) : (v + o) * 0.5f;
-                }
+            if (derive) {
                 mq[p].take(v, lane);
                 C[p][0] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
             }
@@ -503,7 +503,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
             }
         }
         else {
-            LutEval<N>::load_table(a.C + (size_t)node[p] * D::NN, C[p]);
+            if (derive) {
+#pragma unroll
+                for (int i = 0; i < D::NN; ++i) { C[p][i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i)); }
+            }
+            else { LutEval<N>::load_table(a.C + (size_t)node[p] * D::NN, C[p]); }
             LutEval<N>::pin_constants(C[p], cv[p]);
         }
 #pragma unroll
@@ -573,7 +577,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) voi
 #pragma unroll
         for (int p = 0; p < NPW; ++p) { zero_output_padding(a, ck, node[p], live[p], lane); }
     }
-    if (FWD_KIND == 0 && kMatrix) {           // (at the end: a store ahead of the unit's loads would be waited for with them)
+    if (FWD_KIND == 0) {                      // (at the end: a store ahead of the unit's loads would be waited for with them)
 #pragma unroll
         for (int p = 0; p < NPW; ++p) {
             if (clamp_store[p]) { a.clamp_W[(size_t)node[p] * D::NN + lane] = clamp_w[p]; }

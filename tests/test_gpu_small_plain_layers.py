@@ -1,0 +1,42 @@
+"""GPU parity of StochasticLut training steps whose backward pass is one launch, at its edges: wavefront steps and units, work lists shared by four and
+by sixteen wavefronts, the largest call that it serves and the first that goes to the kernels beyond."""
+import numpy as np
+import pytest
+
+import oracle
+from binarybrain_amd import synth
+from util import assert_bwd, assert_fwd, dev, host
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(9, 5, 1), (16, 9, 64), (7, 33, 65), (40, 6, 256), (12, 13, 257), (1100, 30, 300), (260, 11, 2047), (70, 1200, 130), (40, 3000, 20),
+          (300, 640, 2048), (300, 641, 2048)]
+
+
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 6])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_small_plain_training(n, shape):
+    import torch
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    I, O, F = shape
+    rng = np.random.default_rng(10 * n + F)
+    stride = synth.frame_stride_fp32(F)
+    idx = synth.wiring(rng, I, O, n); W = synth.lut_tables(rng, O, n)
+    x = synth.uniform_frames(rng, I, F, stride, -0.1, 1.1); dy = synth.normal_frames(rng, O, F, stride)
+    binarize = bool(n & 1)
+    y_ref = oracle.stochastic_lut_forward(n, x, idx, W, F, input_binary=False, lut_binarize=binarize)
+    dx_ref, dW_ref = oracle.stochastic_lut_backward(n, x, dy, idx, W, F, input_binary=False, lut_binarize=binarize)
+    x[:, F:] = np.nan; dy[:, F:] = np.nan           # what lies behind the frames enters nothing
+    d_x, d_dy, d_idx, d_W = dev(x), dev(dy), dev(idx), dev(W)
+    rev = ops.reverse_table(d_idx, I)
+    y = ops.stochastic_lut_forward(n, d_x, d_idx, d_W, F, input_binary=False, lut_binarize=binarize)
+    assert_fwd(host(y)[:, :F], y_ref[:, :F])
+    got = []
+    for overwrite in (False, True, True):
+        dW = torch.full((O, 1 << n), 0.0 if not overwrite else np.nan, device="cuda")
+        dx = ops.stochastic_lut_backward(n, d_x, d_dy, d_idx, d_W, dW, F, rev, input_binary=False, lut_binarize=binarize, overwrite_dw=overwrite)
+        assert_bwd(host(dx)[:, :F], dx_ref[:, :F])
+        assert_bwd(host(dW), dW_ref)
+        got.append((host(dx)[:, :F], host(dW)))
+    assert all(np.array_equal(a, b) for g in got[1:] for a, b in zip(got[0], g))        # the same bits each time
