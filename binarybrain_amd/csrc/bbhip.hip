@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -803,7 +804,7 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     size_t const v_bytes     = align256((size_t)O * NN * sizeof(float));
     bool const   have_tables = tables.holds_tables && tables_fit(tables, 2 * v_bytes);
     size_t const own_bytes   = align256((size_t)O * own_words * sizeof(uint32_t));
-    size_t const const_bytes = c.bn ? align256((size_t)O * sizeof(NodeConsts)) : 0;
+    size_t const const_bytes = c.bn ? align256((size_t)O * sizeof(NodeConsts) + sizeof(uint32_t)) : 0;     // (and the word `discard` behind them)
     size_t const part_bytes  = slab_count > 1 ? align256((size_t)slab_count * slab_bytes) : 0;
     size_t const bits_bytes  = (from_fp32 && !have_bits) ? align256((size_t)c.input_node_size * c.x_stride * sizeof(uint32_t)) : 0;
     char *base = nullptr;
@@ -831,6 +832,8 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     s.fold.mean = c.mean; s.fold.rstd = c.rstd; s.fold.gamma = c.gamma; s.fold.beta = c.beta; s.fold.inv_frames = 1.0f / (float)c.frame_size;
     s.fold.frame_size = c.frame_size; s.fold.lo = 0.5f - c.bias; s.fold.hi = 0.5f + c.bias;
     s.fold.dW = c.dW; s.fold.overwrite = dw_overwrite; s.fold.node_consts = consts;
+    static std::atomic<uint32_t> calls{0};
+    s.fold.discard = reinterpret_cast<uint32_t *>(consts + O); s.fold.call = calls.fetch_add(1, std::memory_order_relaxed);
     s.dy_quads = (c.frame_stride >= ((c.frame_size + 3) & ~3)) ? 1 : 0;
     if (c.bn ? launch_corner_backward<N, true>(s, slab_count, st) : launch_corner_backward<N, false>(s, slab_count, st)) { return 1; }
 
@@ -853,6 +856,7 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     d.tiles = make_tile_divisor(in_tiles); d.split = split;
     t.dx_quads = (c.frame_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(c.dx) & 15u) == 0) ? 1 : 0;
     t.own = own; t.own_stride = own_words; t.node_size = O; t.V = V; t.node_consts = consts; t.inv_step = 1.0f / (s.fold.hi - s.fold.lo);
+    t.discard = s.fold.discard; t.call = s.fold.call;
     return c.bn ? dispatch_dx_table<N, true>(quads, t, st) : dispatch_dx_table<N, false>(quads, t, st);
 }
 

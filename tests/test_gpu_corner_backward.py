@@ -65,3 +65,33 @@ def test_input_values_that_nearly_meet(bias):
     d_idx = dev(idx)
     dx = ops.stochastic_lut_backward(6, dev(x), dev(dy), d_idx, dev(W), dW, F, ops.reverse_table(d_idx, I), input_binary=True, bias=bias)
     assert_bwd(host(dx)[:, :F], dx_ref[:, :F], "dx"); assert_bwd(host(dW), dW_ref, "dW")
+
+
+@pytest.mark.parametrize("n", [2, 4, 6])
+@pytest.mark.parametrize("shape", [(7, 3, 33, 0), (40, 70, 255, 255), (24, 40, 1300, 0), (12, 600, 3000, 0), (1030, 1100, 65, 0), (27, 36, 20001, 0)])
+def test_a_discarded_gradient_may_hold_anything(n, shape):
+    """dy counts as 0 where the batch-norm output lies outside the hard-tanh window, also where it is infinite or no number: the same bits as with
+    zeros there.  One frame of values per lane and of every kind of dx launch: single words, shared lists, one to four groups of 256 frames."""
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    I, O, F, stride = shape
+    stride = stride or synth.frame_stride_fp32(F)
+    rng = np.random.default_rng(n + F)
+    idx = synth.wiring(rng, I, O, n); W = synth.lut_tables(rng, O, n)
+    x = synth.uniform_frames(rng, I, F, stride); dy = synth.normal_frames(rng, O, F, stride)
+    v = oracle.stochastic_lut_forward(n, x, idx, W, F, input_binary=True, simd=False)[:, :F].astype(np.float64)
+    mean, rstd = v.mean(axis=1), 1.0 / np.sqrt(v.var(axis=1) + 1e-5)
+    t = (v - mean[:, None]) * rstd[:, None] + 0.5                  # gamma 1: about two frames in three lie outside
+    closed = (t < -1e-3) | (t > 1.001)
+    assert 0.2 < closed.mean() < 0.95
+    poisoned = dy.copy()
+    poisoned[:, :F][closed] = rng.choice(np.array([np.inf, -np.inf, np.nan, 3.0e38], np.float32), int(closed.sum()))
+    dy[:, :F][closed] = 0.0
+    d_x, d_idx, d_W = dev(x), dev(idx), dev(W)
+    rev = ops.reverse_table(d_idx, I)
+    got = []
+    for g in (dy, poisoned):
+        dW = dev(np.zeros_like(W))
+        dx = ops.differentiable_lut_backward(n, d_x, dev(g), d_idx, d_W, dW, F, dev(mean.astype(np.float32)), dev(rstd.astype(np.float32)), rev, gamma=1.0)
+        got.append((host(dx)[:, :F], host(dW)))
+    assert np.isfinite(got[1][0]).all() and all(np.array_equal(a, b) for a, b in zip(*got))
