@@ -844,7 +844,8 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     int quads = (O <= 512) ? 4 : (O <= 1024) ? 2 : 1;
     while (quads > 1 && (long long)ceil_div(c.frame_size, quads * 256) * ceil_div(c.input_node_size, kWavesPerBlk) < 2048) { quads /= 2; }
     if (quads_env == 1 || quads_env == 2 || quads_env == 4) { quads = quads_env; }
-    t.far = !s.dy_quads || (long long)O * c.frame_stride * 4 > 0xffffffffLL || (long long)O * own_words * 4 > 0xffffffffLL;
+    t.far = !s.dy_quads || (long long)O * c.frame_stride * 4 > 0xffffffffLL || (long long)O * own_words * 4 > 0xffffffffLL ||
+            (long long)O * NN * 4 > 0xffffffffLL;
     if (t.far) { quads = 1; }
     DxArgs &d = t.dx;
     d.dy = c.dy; d.dx = c.dx; d.rev = c.rev; d.rev_stride = c.rev_stride; d.input_node_size = c.input_node_size; d.frame_size = c.frame_size;

@@ -357,7 +357,7 @@ struct DxTableArgs {
 // of V, Q of indices and Q of dy; the next term's are in flight while a term is evaluated.
 // The kernel is bound by vector instructions (4 per element and about 20 per term) and by what its L2 delivers: rows are addressed by a 32-bit
 // offset into the whole buffer, dy by one 16-byte load per lane and quad, and a lane past the last frame reads whatever lies there.
-// FAR: buffers of 4 GiB and more, and rows of dy that do not hold whole groups of four: a descriptor per row, single words.
+// FAR: buffers (dy, indices, V) of 4 GiB and more, and rows of dy that do not hold whole groups of four: a descriptor per row, single words.
 // Behind a closed hard-tanh window dy counts as 0, whatever it is.  A = 0 gives that for finite values; where the per-corner sums say that there are
 // others (*discard), a walk of its own sets the values of closed corners to 0 first (three instructions per element more).  A
 // training step of 3003 nodes x 5005 frames takes 0.6 us longer for that than without, of 76; with a test per term in one walk 1.4.
@@ -395,7 +395,7 @@ __global__ __launch_bounds__(WAVES * kWave) void lut_dx_table_kernel(DxTableArgs
     uint32_t const dy_bytes = (uint32_t)(t.node_size - 1) * (uint32_t)a.dy_stride * 4u + quad_row_bytes(a.frame_size, true);
     __amdgpu_buffer_rsrc_t const dyr = row_descriptor(a.dy, 0, 0, FAR ? 0u : dy_bytes);
     __amdgpu_buffer_rsrc_t const ir  = row_descriptor(t.own, 0, 0, FAR ? 0u : (uint32_t)t.node_size * (uint32_t)t.own_stride * 4u);
-    __amdgpu_buffer_rsrc_t const vr  = row_descriptor(t.V, 0, 0, (uint32_t)t.node_size * (NN * 4u));
+    __amdgpu_buffer_rsrc_t const vr  = row_descriptor(t.V, 0, 0, FAR ? 0u : (uint32_t)t.node_size * (NN * 4u));
 
     float4 acc[Q];
 #pragma unroll
@@ -405,7 +405,8 @@ __global__ __launch_bounds__(WAVES * kWave) void lut_dx_table_kernel(DxTableArgs
     auto request = [&](int e, Stage &s) {
         uint32_t const node = (uint32_t)e / (uint32_t)N;
         s.k = e - (int)node * N;
-        s.v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(vr, (lane & (NN - 1)) * 4, node * (NN * 4u), 0));
+        __amdgpu_buffer_rsrc_t const v_row = FAR ? row_descriptor(t.V, (int)node, NN, NN * 4u) : vr;
+        s.v = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(v_row, (lane & (NN - 1)) * 4, FAR ? 0u : node * (NN * 4u), 0));
         if (BN) {
             const_consts &c = consts[node];
             s.mean = c.mean; s.gain = c.gain; s.shift = c.shift; s.scale = c.scale; s.open = c.open;

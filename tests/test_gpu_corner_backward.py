@@ -95,3 +95,35 @@ def test_a_discarded_gradient_may_hold_anything(n, shape):
         dx = ops.differentiable_lut_backward(n, d_x, dev(g), d_idx, d_W, dW, F, dev(mean.astype(np.float32)), dev(rstd.astype(np.float32)), rev, gamma=1.0)
         got.append((host(dx)[:, :F], host(dW)))
     assert np.isfinite(got[1][0]).all() and all(np.array_equal(a, b) for a, b in zip(*got))
+
+
+def test_corner_values_beyond_4_gib():
+    """2^24 + 64 nodes of six inputs: their corner values do not fit one buffer of 32-bit offsets, while dy and the indices do"""
+    import torch
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    n, I, O, F = 6, 1 << 16, (1 << 24) + 64, 32
+    gen = torch.Generator(device="cuda"); gen.manual_seed(4)
+    idx = (torch.arange(n * O, dtype=torch.int32, device="cuda") % I).reshape(O, n)
+    link = torch.arange(I, dtype=torch.int32, device="cuda")[:, None] + I * torch.arange((n * O + I - 1) // I, dtype=torch.int32, device="cuda")[None, :]
+    rev = torch.cat([(link < n * O).sum(dim=1, dtype=torch.int32)[:, None], torch.where(link < n * O, link, 0)], dim=1).contiguous()
+    x = torch.randint(-(1 << 31), 1 << 31, (I, 1), device="cuda", generator=gen).to(torch.int32)
+    W = torch.rand((O, 1 << n), device="cuda", generator=gen)
+    dy = torch.randn((O, F), device="cuda", generator=gen)
+    dW = torch.zeros_like(W)
+    # input values 0 and 1: a corner value is a table entry, and entry p of the table gradient the sum at corner p alone
+    dx = ops.bit_stochastic_lut_backward(n, x, dy, idx, W, dW, F, rev, bias=0.5)
+    base = torch.arange(O, device="cuda") << n
+    for f in (0, 17, 31):
+        bit = ((x[:, 0] >> f) & 1).long()
+        corner = sum(bit[idx[:, k].long()] << k for k in range(n))
+        want = torch.zeros(I, dtype=torch.float64, device="cuda")
+        for k in range(n):
+            slope = W.view(-1)[base + (corner | (1 << k))] - W.view(-1)[base + (corner & ~(1 << k))]
+            want.index_add_(0, idx[:, k].long(), slope.double() * dy[:, f].double())
+        assert_bwd(host(dx[:, f]), host(want), "dx of frame %d" % f)
+    for first in (0, O - 1000):
+        bits = (x[idx[first:first + 1000].long(), 0][:, :, None] >> torch.arange(F, device="cuda")) & 1
+        corner = sum(bits[:, k].long() << k for k in range(n))
+        want = torch.zeros((1000, 1 << n), dtype=torch.float64, device="cuda").scatter_add_(1, corner, dy[first:first + 1000].double())
+        assert_bwd(host(dW[first:first + 1000]), host(want), "dW")
