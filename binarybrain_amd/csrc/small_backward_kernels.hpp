@@ -107,7 +107,8 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
                 o.dy[u] = *reinterpret_cast<float const *>(reinterpret_cast<char const *>(dyr) + (uint32_t)min(fb + u * kWave + lane, f_last) * 4u);
             }
         };
-        TableGradient<N> grad;
+        using Gradient = TableGradient<N, 2>;
+        Gradient grad;
         grad.clear(lane);
         auto add = [&](int fb, Operands const &o) {
 #pragma unroll
@@ -132,8 +133,8 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
             if (sub != 0) { return; }
             for (int k = 1; k < nw; ++k) { sum += part[wave + k][0][lane]; }
         }
-        if (live && TableGradient<N>::owns_entry(lane)) {
-            float *out = s.dW + (size_t)node * NN + TableGradient<N>::table_entry(lane);
+        if (live && Gradient::owns_entry(lane)) {
+            float *out = s.dW + (size_t)node * NN + Gradient::table_entry(lane);
             *out = s.overwrite ? sum : *out + sum;
         }
         return;

@@ -7,24 +7,30 @@ namespace bbhip {
 
 // dW[e] = sum over frames of  d prod_j (bit_j(e) ? x_j : 1 - x_j)  is for each node a sum of outer products: with the corner products of inputs
 // 0, 1 as a column and those of inputs 2, 3 as a row, one v_mfma_f32_4x4x1_16b_f32 adds the 4 x 4 products of sixteen frames, a quad of lanes
-// each, in the time of two vector instructions where 16 fused multiply-adds per lane and four frames would take four.  Inputs 4 and 5 scale the
-// column and the row: four products per frame, sixteen accumulator registers per lane instead of 64, and the sum over the quads at the end takes
-// 30 instructions instead of a transposition of 64 registers through LDS.  That end is what pays in a small layer; over long slabs of frames the
-// operands (36 instructions per 64 frames and the 16 products) take as long as the 64 multiply-adds (4096 nodes x 8192 frames 132 us, multiply-adds 111).
+// each, in the time of two vector instructions where 16 fused multiply-adds per lane and four frames would take four.  Inputs 4 and 5 double the
+// columns and the rows: four products per frame, sixteen accumulator registers per lane and set instead of 64, and the sum over the quads at the
+// end takes 30 instructions instead of a transposition of 64 registers through LDS.  That end is what pays in a small layer; over long slabs of
+// frames the operands (44 instructions per 64 frames and the 16 products) take longer than the 64 multiply-adds.
 //
 // Lane 4 b + r of quad b supplies entry r of column and row.  The four frames of a quad take turns (t): entry r of frame 4 b + t needs that frame's
 // inputs in all four lanes, which a data-parallel move brings as an operand of the instruction that uses it.  A corner factor is one addition: x
 // where the lane's corner has the bit set, x - 1 = -(1 - x) where it has not; the sign is applied to the sum.
-template <int N>
+//
+// Rounding: every term is formed with its own factors before it is added (a sum of the terms with 1 - x taken as the difference of two sums without
+// that factor rounds to the size of those: 1.0e-7 of the largest entry for six inputs and 1000 frames where this gives 4.3e-8 and multiply-adds
+// per lane in slabs 4.9e-8, rms against 64 bits).  A register is one chain of four additions per 64 frames, or of two where the turns go to two SETS of
+// accumulators.  The callers give a wavefront at most 256 frames, or 512 with two sets, which keeps the error of every width at or below that of
+// the multiply-adds.
+template <int N, int SETS>
 struct TableGradient {
     static constexpr int CQ = (N > 4) ? 2 : 1, RQ = (N > 5) ? 2 : 1, R = 4 * CQ * RQ;
-    mfma_f4 acc[RQ][CQ];
+    mfma_f4 acc[SETS][RQ][CQ];
     float c0, c1;                   // 0 or -1: what the lane adds to inputs 0 / 2 and 1 / 3
 
     __device__ __forceinline__ void clear(int lane)
     {
 #pragma unroll
-        for (int i = 0; i < RQ * CQ; ++i) { acc[i / CQ][i % CQ] = mfma_f4{0.0f, 0.0f, 0.0f, 0.0f}; }
+        for (int i = 0; i < SETS * RQ * CQ; ++i) { acc[i / (RQ * CQ)][i / CQ % RQ][i % CQ] = mfma_f4{0.0f, 0.0f, 0.0f, 0.0f}; }
         c0 = (lane & 1) ? 0.0f : -1.0f;
         c1 = (lane & 2) ? 0.0f : -1.0f;
     }
@@ -43,12 +49,12 @@ struct TableGradient {
         if constexpr (N >= 4)      { row[0] = (quad_lane<T>(x[2]) + c0) * (quad_lane<T>(x[3]) + c1); }
         else if constexpr (N == 3) { row[0] = quad_lane<T>(x[2]) + c0; }
         else                       { row[0] = 1.0f; }
-        if constexpr (CQ == 2) { col[1] = quad_lane<T>(x[N > 4 ? 4 : 0]) * col[0]; }
-        if constexpr (RQ == 2) { row[1] = quad_lane<T>(x[N > 5 ? 5 : 0]) * row[0]; }
+        if constexpr (CQ == 2) { col[1] = quad_lane<T>(x[N > 4 ? 4 : 0]) * col[0]; col[0] = col[1] - col[0]; }
+        if constexpr (RQ == 2) { row[1] = quad_lane<T>(x[N > 5 ? 5 : 0]) * row[0]; row[0] = row[1] - row[0]; }
 #pragma unroll
         for (int q = 0; q < RQ; ++q) {
 #pragma unroll
-            for (int p = 0; p < CQ; ++p) { acc[q][p] = __builtin_amdgcn_mfma_f32_4x4x1f32(col[p], row[q], acc[q][p], 0, 0, 0); }
+            for (int p = 0; p < CQ; ++p) { acc[T % SETS][q][p] = __builtin_amdgcn_mfma_f32_4x4x1f32(col[p], row[q], acc[T % SETS][q][p], 0, 0, 0); }
         }
     }
     // 64 frames, one per lane: inputs in [0, 1] and the gradient of the LUT output (0 where the frame does not count)
@@ -102,17 +108,16 @@ struct TableGradient {
 #pragma unroll
             for (int p = 0; p < CQ; ++p) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) { v[(q * CQ + p) * 4 + r] = acc[q][p][r]; }
+                for (int r = 0; r < 4; ++r) { v[(q * CQ + p) * 4 + r] = SETS == 2 ? acc[0][q][p][r] + acc[SETS - 1][q][p][r] : acc[0][q][p][r]; }
             }
         }
         float s = fold<32, R>(v, lane);
-        // register index = ((row scaling) (column scaling) (bit of input 1) (bit of input 0)); the products with 1 - x are differences
-        constexpr int kCol = 16;                                        // lane bit of the column scaling
-        if constexpr (CQ == 2) { float const o = lane_xor(s, kCol); s = (lane & kCol) ? s : s - o; }
-        if constexpr (RQ == 2) { float const o = lane_xor(s, 32);   s = (lane & 32) ? s : s - o; }
+        // register index = ((bit of input 5) (bit of input 4) (bit of input 1) (bit of input 0)); a sign for each factor 1 - x
         int zeros = 2 - ((lane >> 2) & 1) - ((lane >> 3) & 1);
         if (N >= 3) { zeros += 1 - (lane & 1); }
         if (N >= 4) { zeros += 1 - ((lane >> 1) & 1); }
+        if (N >= 5) { zeros += 1 - ((lane >> 4) & 1); }
+        if (N >= 6) { zeros += 1 - ((lane >> 5) & 1); }
         return (zeros & 1) ? -s : s;
     }
     __device__ __forceinline__ static int table_entry(int lane)
@@ -350,7 +355,8 @@ __global__ __launch_bounds__(kNodeWaves * kWave) void lut_node_gradient_kernel(N
     float const shift = -(a.gamma * s0) * rstd * a.inv_frames;
     float const scale = -(a.gamma * s1) * (rstd * rstd) * rstd * a.inv_frames;
 
-    TableGradient<N> grad;
+    using Gradient = TableGradient<N, N <= 4 ? 2 : 1>;
+    Gradient grad;
     grad.clear(lane);
 #pragma unroll
     for (int s = 0; s < kNodeSteps; s += U) {
@@ -374,8 +380,8 @@ __global__ __launch_bounds__(kNodeWaves * kWave) void lut_node_gradient_kernel(N
         if (sub != 0) { return; }
         for (int k = 1; k < nw; ++k) { sum += part[wave + k][lane]; }
     }
-    if (live && TableGradient<N>::owns_entry(lane)) {
-        float *out = a.dW + (size_t)node * NN + TableGradient<N>::table_entry(lane);
+    if (live && Gradient::owns_entry(lane)) {
+        float *out = a.dW + (size_t)node * NN + Gradient::table_entry(lane);
         *out = a.overwrite ? sum : *out + sum;
     }
 }
