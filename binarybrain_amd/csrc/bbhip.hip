@@ -877,15 +877,18 @@ void launch_node_gradient(BackwardCall const &c, BwdArgs const &a, float const *
 
 // Plain layers on real-valued inputs whose backward pass is one launch (lut_small_backward_kernel).  Per frame that kernel does more than the two
 // launches of larger layers, the more so the wider the table: 1024 nodes x 1000 frames 25.0 us a training step instead of 29.2, 1000 x 2000 39.2 and 38.5,
-// 2000 x 2000 67 and 63; four inputs per node 1531 x 1999 31.0 instead of 33.1, 4000 x 4000 144 and 134; three inputs 2000 x 4000 53.7 instead of 55.1.
-// Long work lists (40 inputs, 2000 nodes of five, 1300 frames) 44 and 38.
+// 2000 x 2000 67 and 63; four inputs per node 1531 x 1999 31.0 instead of 33.1, three inputs 2000 x 4000 53.7 instead of 55.1.
+// Long work lists (40 inputs, 2000 nodes of five, 1300 frames) 44 and 38.  A node's frames stay in one workgroup here, so that few nodes over many
+// frames (a convolution) leave the device idle: the backward call alone of 36 nodes of six 7.7 us instead of 10.0 at 4096 frames, 12.2 and 12.8 at
+// 8192, 39.8 and 28.6 at 30000; of 4 nodes 6.7 instead of 8.4, 11.1 and 8.6, 32.3 and 13.1.  Four inputs, 1000 nodes: 16.9 and 16.7 at 2048
+// frames, 23.5 and 22.9 at 3072, 29.4 and 25.9 at 4096.
 bool small_plain_layer(BackwardCall const &c)
 {
     if (c.bn || c.xmode != kXClamp || bwd_slab_frames() > 0 || dx_chunk_frames_env() > 0 || dx_pass_steps_env() > 0) { return false; }
     if ((long long)c.input_node_size * c.x_stride >= (1LL << 30) || (long long)c.output_node_size * c.frame_stride >= (1LL << 30)) { return false; }
     long long const node_frames = (long long)c.output_node_size * c.frame_size;
-    if (c.rev_stride > 32 && node_frames > (5LL << 18)) { return false; }
-    return node_frames << c.n <= (c.n >= 5 ? 5LL << 24 : 1LL << 26);
+    if (c.frame_size > 4096 || (c.rev_stride > 32 && node_frames > (5LL << 18))) { return false; }
+    return node_frames << c.n <= (c.n >= 5 ? 5LL << 24 : c.n == 4 ? 3LL << 24 : 1LL << 26);
 }
 
 template <int N>

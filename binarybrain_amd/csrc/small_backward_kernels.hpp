@@ -118,6 +118,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
                 grad.add(x, (fb + u * kWave + lane < f_end) ? o.dy[u] : 0.0f);
             }
         };
+        float sum = 0.0f;
         Operands o0, o1;
         if (f_begin < f_end) { request(f_begin, o0); }
         for (int fb = f_begin; fb < f_end; fb += 2 * S * kWave) {
@@ -125,8 +126,10 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
             add(fb, o0);
             if (fb + 2 * S * kWave < f_end) { request(fb + 2 * S * kWave, o0); }
             if (fb + S * kWave < f_end) { add(fb + S * kWave, o1); }
+            // chains of at most 512 frames (TableGradient)
+            if (((fb - f_begin) & 511) == 512 - 2 * S * kWave && fb + 2 * S * kWave < f_end) { sum += grad.total(lane); grad.clear(lane); }
         }
-        float sum = grad.total(lane);
+        sum += grad.total(lane);
         if (nw > 1) {
             part[wave][0][lane] = sum;
             __syncthreads();

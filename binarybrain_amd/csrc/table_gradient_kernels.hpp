@@ -19,8 +19,8 @@ namespace bbhip {
 // Rounding: every term is formed with its own factors before it is added (a sum of the terms with 1 - x taken as the difference of two sums without
 // that factor rounds to the size of those: 1.0e-7 of the largest entry for six inputs and 1000 frames where this gives 4.3e-8 and multiply-adds
 // per lane in slabs 4.9e-8, rms against 64 bits).  A register is one chain of four additions per 64 frames, or of two where the turns go to two SETS of
-// accumulators.  The callers give a wavefront at most 256 frames, or 512 with two sets, which keeps the error of every width at or below that of
-// the multiply-adds.
+// accumulators.  The callers add at most 256 frames between two totals, or 512 with two sets, which keeps the error of every width at or below that
+// of the multiply-adds.
 template <int N, int SETS>
 struct TableGradient {
     static constexpr int CQ = (N > 4) ? 2 : 1, RQ = (N > 5) ? 2 : 1, R = 4 * CQ * RQ;

@@ -10,7 +10,7 @@ from util import assert_bwd, assert_fwd, dev, host
 pytestmark = pytest.mark.gpu
 
 SHAPES = [(9, 5, 1), (16, 9, 64), (7, 33, 65), (40, 6, 256), (12, 13, 257), (1100, 30, 300), (260, 11, 2047), (70, 1200, 130), (40, 3000, 20),
-          (300, 640, 2048), (300, 641, 2048)]
+          (300, 640, 2048), (300, 641, 2048), (27, 16, 2049), (216, 36, 3900), (27, 4, 4096), (27, 4, 4097), (27, 36, 30000), (7, 1, 70000)]
 
 
 @pytest.mark.parametrize("n", [2, 3, 4, 5, 6])
@@ -43,7 +43,7 @@ def test_small_plain_training(n, shape):
 
 
 @pytest.mark.parametrize("n, bound", [(4, 7.0e-8), (5, 6.5e-8), (6, 6.0e-8)])
-@pytest.mark.parametrize("frames", [1000, 2048])
+@pytest.mark.parametrize("frames", [1000, 2048, 4000])
 def test_table_gradient_rounding(n, bound, frames):
     """The sums over frames round no worse than multiply-adds per lane in slabs do.  rms error against 64 bits relative to a node's largest entry,
     of those multiply-adds by a model of their order in fp32: 6.9e-8, 5.9e-8, 5.1e-8 for four, five, six inputs; what rounds every term to
