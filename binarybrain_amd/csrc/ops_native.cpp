@@ -90,9 +90,16 @@ template <> struct FromPy<Clamp> {
         return Clamp{true, (float)l, (float)h};
     }
 };
-// a device buffer of a plain entry point: a tensor or None
+// a device buffer of a plain entry point: a tensor or None.  A buffer that the entry may write to is asked for as such: torch then gives a tensor
+// that shares its storage with a lazy clone storage of its own.
 template <class E> struct FromPy<E *> {
-    static E *get(PyObject *o) { return o == Py_None ? nullptr : reinterpret_cast<E *>(const_cast<void *>(tensor_arg(o).const_data_ptr())); }
+    static E *get(PyObject *o)
+    {
+        if (o == Py_None) { return nullptr; }
+        at::Tensor const &t = tensor_arg(o);
+        if constexpr (std::is_const_v<E>) { return static_cast<E *>(t.const_data_ptr()); }
+        else                              { return static_cast<E *>(t.mutable_data_ptr()); }
+    }
 };
 
 // ---- results -------------------------------------------------------------------------------------------------------------------

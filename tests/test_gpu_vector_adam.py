@@ -130,3 +130,18 @@ def test_rejects_bad_arguments(ops):
     assert lib.bbhip_fp32_Vector_add_ex(None, None, None, 1.0, 1.0, 0.0, 0, None) != 0
     assert lib.bbhip_fp32_OptimizerAdam(-1, None, None, None, None, None, 0.1, 0.9, 0.999, None) != 0
     assert lib.bbhip_fp32_OptimizerAdam(0, None, None, None, None, None, 0.1, 0.9, 0.999, None) == 0
+
+def test_lazily_cloned_tensors_stay_apart(ops):
+    """a tensor that shares its storage with a lazy clone is given storage of its own before an entry point writes into it"""
+    import torch
+    a = torch.rand(1000, device="cuda")
+    want = a.clone()
+    b = torch._lazy_clone(a)
+    ops.vector_set_(b, 3.0)
+    assert torch.equal(a, want) and bool((b == 3.0).all())
+    c = torch._lazy_clone(a)
+    ops.vector_add_ex(a, a, out=c)
+    assert torch.equal(a, want) and torch.equal(c, a + a)
+    d = torch._lazy_clone(a)
+    ops.vector_clamp_(a, 0.25, 0.5)
+    assert torch.equal(d, want) and torch.equal(a, want.clamp(0.25, 0.5))
