@@ -696,7 +696,7 @@ struct BackwardCall {
     int x_stride, frame_stride, tmp_frame_size, tmp_frame_stride;
     int xmode, lut_binarize; float bias;
     int bn;
-    float const *mean, *rstd; float *dmean_tmp, *dvar_tmp;
+    float const *mean, *rstd; float *dmean_tmp, *dvar_tmp;      // (the last two are not used: such sums are in the scratch arena)
     float gamma, beta;
 };
 
@@ -999,18 +999,23 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
     int const stat_chunk       = fwd_chunk_frames(c.xmode, c.frame_size, ceil_div(c.output_node_size, kWavesPerBlk * stat_npw));
     int const stat_chunk_count = ceil_div(c.frame_size, stat_chunk);
     size_t const stat_bytes = c.bn ? align256((size_t)stat_chunk_count * c.output_node_size * 2 * sizeof(float)) : 0;
+    // dmean and dvar of the nodes, where a launch of its own forms them from the statistics pass's sums
+    bool const stat_launch  = c.bn && stat_chunk_count > kInlineStatUnits;
+    size_t const sum_bytes  = stat_launch ? align256((size_t)c.output_node_size * 2 * sizeof(float)) : 0;
     size_t const term_count = (dxmode == kDxNone) ? (size_t)c.input_node_size * (size_t)(c.rev_stride - 1) * (kTermHead + NN / 2) : 0;
     size_t const dtab_bytes = align256(term_count * sizeof(int));
     size_t const dyh_bytes  = (dxmode == kDxNone && c.bn) ? align256((size_t)c.output_node_size * c.frame_stride * sizeof(float)) : 0;
     size_t const v_bytes = corner ? c_bytes : 0;
     char *base = nullptr;
-    if (arena_get(c_bytes + part_bytes + stat_bytes + dtab_bytes + dyh_bytes + v_bytes, &base, st)) { return 1; }
+    if (arena_get(c_bytes + part_bytes + stat_bytes + dtab_bytes + dyh_bytes + v_bytes + sum_bytes, &base, st)) { return 1; }
     float *V    = corner ? reinterpret_cast<float *>(base + c_bytes + part_bytes + stat_bytes + dtab_bytes + dyh_bytes) : nullptr;
     float *C    = reinterpret_cast<float *>(base);
     float *part = reinterpret_cast<float *>(base + c_bytes);
     float *stat = reinterpret_cast<float *>(base + c_bytes + part_bytes);
     int   *term = reinterpret_cast<int *>(base + c_bytes + part_bytes + stat_bytes);
     float *dyh  = reinterpret_cast<float *>(base + c_bytes + part_bytes + stat_bytes + dtab_bytes);
+    float *dmean = stat_launch ? reinterpret_cast<float *>(base + c_bytes + part_bytes + stat_bytes + dtab_bytes + dyh_bytes + v_bytes) : nullptr;
+    float *dvar  = stat_launch ? dmean + c.output_node_size : nullptr;
 
     // centred coefficients: needed where the LUT output is recomputed (batch-norm) or per-connection gradients are formed;
     // a caller that kept the tables of this step's forward call (same W, same kind of input) hands them back: nothing to prepare
@@ -1040,7 +1045,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
     BwdArgs a{};
     a.x = c.x; a.dy = c.dy; a.idx = c.idx; a.C = C;
     a.dw_partial = part;
-    a.mean = c.mean; a.rstd = c.rstd; a.dmean = c.dmean_tmp; a.dvar = c.dvar_tmp;
+    a.mean = c.mean; a.rstd = c.rstd; a.dmean = dmean; a.dvar = dvar;
     a.node_size = c.output_node_size; a.frame_size = c.frame_size;
     a.x_stride = c.x_stride; a.dy_stride = c.frame_stride;
     a.slab = slab; a.tiles = make_tile_divisor(tile_count);
@@ -1060,13 +1065,13 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         f.bias = c.bias; f.gamma = c.gamma; f.beta = c.beta;
         if (dispatch_forward<N>(c.xmode, kYClamp, 3, f, npw, st)) { return 1; }
         BBHIP_LAUNCH_CHECK();
-        if (stat_chunk_count <= kInlineStatUnits) {
+        if (!stat_launch) {
             a.stat_partial = stat; a.stat_count = stat_chunk_count;     // few units: the table-gradient wavefronts add them up themselves
         }
         else {
             int const npb = stat_nodes_per_block(stat_chunk_count);
             launch(bn_backward_finalize_kernel, dim3(ceil_div(c.output_node_size, npb)), dim3(kBlock), 0, st,
-                               stat, c.mean, c.rstd, c.dmean_tmp, c.dvar_tmp, c.gamma, c.output_node_size, stat_chunk_count, c.frame_size, npb);
+                               stat, c.mean, c.rstd, dmean, dvar, c.gamma, c.output_node_size, stat_chunk_count, c.frame_size, npb);
             BBHIP_LAUNCH_CHECK();
         }
     }

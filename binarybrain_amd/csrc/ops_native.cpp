@@ -376,24 +376,13 @@ at::Tensor differentiable_lut_forward_nobn(int n, T x, T idx, T W, int frames, f
     return y;
 }
 
-// dmean and dvar are scratch of the call, the two halves of one buffer; the library writes them only where a node has more than 256 units of at
-// least 64 frames.  Below, the call gets an address that it does not touch.
-struct SumsScratch { at::Tensor t; float *p; };
-SumsScratch sums_scratch(T like, int nodes, int frames, float *untouched)
-{
-    if (frames <= 256 * 64) { return SumsScratch{at::Tensor(), untouched}; }
-    SumsScratch s{line_f32(like, 2 * (int64_t)nodes), nullptr};
-    s.p = data<float>(s.t);
-    return s;
-}
-
 at::Tensor differentiable_lut_backward(int n, T x, T dy, T idx, T W, T dW, int frames, T mean, T rstd, OptTensor rev, float gamma, float beta, float bias,
                                        bool lut_binarize, bool binary_mode, double max_tmp_bytes, OptTensor packed, OptTensor tables, bool overwrite,
                                        bool hints)
 {
     int const I = rows_of(x), O = rows_of(idx), S = stride_of(dy);
     at::Tensor dx = rows_f32(x, I, S);
-    SumsScratch const sums = sums_scratch(x, O, frames, data<float>(dx));
+    float *const unused = data<float>(dx);          // dmean and dvar: any address that is not null (include/bbhip.h)
     DxTmp const tmp = dx_tmp_of(x, O, n, frames, (int64_t)max_tmp_bytes);
     if (hints) {
         hint_input(x, packed, true, false);
@@ -401,7 +390,7 @@ at::Tensor differentiable_lut_backward(int n, T x, T dy, T idx, T W, T dW, int f
     }
     if (overwrite) { bbhip_HintTableGradientOverwrite(1); }
     call(bbhip_fp32_DifferentiableLutN_Backward, n, data<float const>(x), data<float const>(dy), data<float>(dx), tmp.p, data<int const>(idx),
-         data<int const>(rev), data<float const>(W), data<float>(dW), data<float const>(mean), data<float const>(rstd), sums.p, sums.p + O,
+         data<int const>(rev), data<float const>(W), data<float>(dW), data<float const>(mean), data<float const>(rstd), unused, unused,
          gamma, beta, bias, rev ? stride_of(*rev) : 0, I, O, frames, S, tmp.frames, tmp.stride, (int)lut_binarize, (int)binary_mode,
          current_stream());
     return dx;
@@ -412,11 +401,11 @@ at::Tensor bit_differentiable_lut_backward(int n, T x, T dy, T idx, T W, T dW, i
 {
     int const I = rows_of(x), O = rows_of(idx), S = stride_of(dy);
     at::Tensor dx = rows_f32(dy, I, S);
-    SumsScratch const sums = sums_scratch(dy, O, frames, data<float>(dx));
+    float *const unused = data<float>(dx);          // dmean and dvar, as above
     DxTmp const tmp = dx_tmp_of(dy, O, n, frames, (int64_t)max_tmp_bytes);
     if (hints) { hint_tables(tables, true); }
     call(bbhip_bit_fp32_DifferentiableLutN_Backward, n, data<int const>(x), data<float const>(dy), data<float>(dx), tmp.p, data<int const>(idx),
-         data<int const>(rev), data<float const>(W), data<float>(dW), data<float const>(mean), data<float const>(rstd), sums.p, sums.p + O,
+         data<int const>(rev), data<float const>(W), data<float>(dW), data<float const>(mean), data<float const>(rstd), unused, unused,
          gamma, beta, bias, rev ? stride_of(*rev) : 0, I, O, frames, S, stride_of(x), tmp.frames, tmp.stride, (int)lut_binarize,
          current_stream());
     return dx;

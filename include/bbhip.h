@@ -542,14 +542,15 @@ int bbhip_bit_fp32_DifferentiableLutN_ForwardInference(int n, int const *dev_x_b
         int const *dev_input_index, float const *dev_W, float const *dev_running_mean_buf,
         float const *dev_running_var_buf, float gamma, float beta, float unbinarize_bias,
         int node_size, int frame_size, int frame_stride, int lut_binarize, void *stream);
-/* bbcu_fp32_DifferentiableLutN_Backward<N>, include/bbcu/bbcu.h:602-630 */
+/* bbcu_fp32_DifferentiableLutN_Backward<N>, include/bbcu/bbcu.h:602-630.  dev_dmean_tmp and dev_dvar_tmp are scratch of the reference's kernels: here
+ * they must not be null, as there, and are neither read nor written (the library's own scratch holds such sums). */
 int bbhip_fp32_DifferentiableLutN_Backward(int n, float const *dev_x_buf, float const *dev_dy_buf, float *dev_dx_buf,
         float *dev_dx_tmp, int const *dev_input_index, int const *dev_reverse_index, float const *dev_W,
         float *dev_dW, float const *dev_mean_buf, float const *dev_rstd_buf, float *dev_dmean_tmp,
         float *dev_dvar_tmp, float gamma, float beta, float unbinarize_bias, int reverse_index_stride,
         int input_node_size, int output_node_size, int frame_size, int frame_stride, int tmp_frame_size,
         int tmp_frame_stride, int lut_binarize, int binary_mode, void *stream);
-/* bbcu_bit_fp32_DifferentiableLutN_Backward<N>, include/bbcu/bbcu.h:632-660 */
+/* bbcu_bit_fp32_DifferentiableLutN_Backward<N>, include/bbcu/bbcu.h:632-660; dev_dmean_tmp and dev_dvar_tmp as above */
 int bbhip_bit_fp32_DifferentiableLutN_Backward(int n, int const *dev_x_buf, float const *dev_dy_buf, float *dev_dx_buf,
         float *dev_dx_tmp, int const *dev_input_index, int const *dev_reverse_index, float const *dev_W,
         float *dev_dW, float const *dev_mean_buf, float const *dev_rstd_buf, float *dev_dmean_tmp,

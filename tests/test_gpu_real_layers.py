@@ -42,3 +42,29 @@ def test_real_valued_training(n, shape):
             assert_bwd(host(dx)[:, :F], dx_ref[:, :F], "dx"); assert_bwd(host(dW) - 0.25, dW_ref, "dW")
         got.append((host(y)[:, :F], host(m), host(dx)[:, :F], host(dW)))
     assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
+def test_scratch_arguments_of_the_backward_call_are_not_used():
+    """66000 frames: more units than a wavefront adds up itself, so that dmean and dvar are formed by a launch of their own, in the library's scratch"""
+    import torch
+    from binarybrain_amd import ops
+    from binarybrain_amd.capi import check, lib, ptr, stream_ptr
+    ops.set_dx_mode(0)
+    n, I, O, F = 6, 12, 5, 66000
+    rng = np.random.default_rng(66)
+    stride = synth.frame_stride_fp32(F)
+    idx = synth.wiring(rng, I, O, n); W = synth.lut_tables(rng, O, n)
+    x = synth.uniform_frames(rng, I, F, stride); dy = synth.normal_frames(rng, O, F, stride)
+    _, mean, rstd, _, _ = oracle.differentiable_lut_forward_training(n, x, idx, W, F, np.zeros(O, np.float32), np.ones(O, np.float32), binary_mode=False)
+    dx_ref, dW_ref = oracle.differentiable_lut_backward(n, x, dy, idx, W, F, mean, rstd, binary_mode=False)
+    d_x, d_dy, d_idx, d_W, d_mean, d_rstd, dW = dev(x), dev(dy), dev(idx), dev(W), dev(mean), dev(rstd), dev(np.zeros_like(W))
+    rev = ops.reverse_table(d_idx, I)
+    dx = torch.empty((I, stride), device="cuda")
+    tmp = torch.full((2, O), 7.0, device="cuda")
+    check(lib().bbhip_fp32_DifferentiableLutN_Backward(n, ptr(d_x), ptr(d_dy), ptr(dx), None, ptr(d_idx), ptr(rev), ptr(d_W), ptr(dW), ptr(d_mean), ptr(d_rstd),
+                                                      ptr(tmp[0]), ptr(tmp[1]), 0.3, 0.5, 0.25, rev.shape[1], I, O, F, stride, 0, 0, 0, 0, stream_ptr()))
+    assert_bwd(host(dx)[:, :F], dx_ref[:, :F]); assert_bwd(host(dW), dW_ref)
+    assert bool((tmp == 7.0).all())
+    again = torch.zeros_like(dW)
+    got = ops.differentiable_lut_backward(n, d_x, d_dy, d_idx, d_W, again, F, d_mean, d_rstd, rev, binary_mode=False)
+    assert torch.equal(got[:, :F], dx[:, :F]) and torch.equal(again, dW)
