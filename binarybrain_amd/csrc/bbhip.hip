@@ -239,7 +239,7 @@ int arena_get(size_t bytes, char **out, hipStream_t st, Scratch const *fixed = n
 
 inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+inline int ceil_div(int a, int b) { return a / b + (a % b != 0); }      // (no sum that could leave the range)
 
 // A launch without the call-configuration stack and the copies that the <<<>>> form's host stub goes through: 2.7 us of host time for a kernel
 // with 400 bytes of arguments instead of 3.2, and the host is what a program of small layers waits for.  Errors are read by BBHIP_LAUNCH_CHECK.
@@ -2335,6 +2335,16 @@ static int launch_real_to_binary(float const *x, void *y, bool bit, bool zero_pa
     else if (wide) { launch((real_to_binary_kernel<false, 4>), grid, block, 0, st, a); }
     else           { launch((real_to_binary_kernel<false, 1>), grid, block, 0, st, a); }
     BBHIP_LAUNCH_CHECK();
+    // rows whose frames an int cannot count (256 MiB and more: few of them): the words that the launch was not made for
+    size_t const first = (size_t)((reach + 31) / 32);
+    if (zero_padding && first < y_frame_stride) {
+        size_t const count = y_frame_stride - first;
+        for (long long node = 0; node < y_nodes; ++node) {
+            launch(fill_kernel, dim3((unsigned)((count + kBlock * 4 - 1) / (kBlock * 4))), dim3(kBlock), 0, st,
+                   static_cast<float *>(y) + (size_t)node * y_frame_stride + first, 0.0f, count);
+        }
+        BBHIP_LAUNCH_CHECK();
+    }
     return 0;
 }
 

@@ -174,3 +174,14 @@ def test_bad_arguments(ops):
         ops.real_to_binary_forward(x, 1, 4, 64, frame_mod=0)
     with pytest.raises(BbhipError):
         ops.hard_tanh_forward(x, 65)
+
+
+@pytest.mark.parametrize("words", [(1 << 26) - 1, 1 << 26, (1 << 26) + 70])
+def test_padding_of_very_long_packed_rows(ops, words):
+    """a new packed output is zero behind its last frame, also where its row pitch reaches past 2^31 frames"""
+    import torch
+    rng = np.random.default_rng(3)
+    x = rng.random((2, 100)).astype(F32)
+    torch.full((2, words), -1, dtype=torch.int32, device="cuda")               # (what the allocator hands out again)
+    y = ops.real_to_binary_forward(dev(x), 1, 2, 100, bit=True, y_stride=words)
+    assert np.array_equal(host(y[:, :4]), oracle.real_to_binary_forward(x, 1, 2, 100, bit=True)) and not bool(y[:, 4:].any())
