@@ -176,6 +176,8 @@ int bwd_slab_frames(void)  { static int v = env_int("BBHIP_BWD_SLAB", 0);  retur
 // gathered rows are fp32 (what L2 holds); packed-bit rows leave room for 256 frames in passes of four, which halves the
 // per-term set-up per frame.  0: not set in the environment.
 int dx_chunk_frames_env(void) { static int v = env_int("BBHIP_DX_CHUNK", 0); return ((v + 63) / 64) * 64; }
+// the dx kernel over kept corner indices: groups of 256 frames per wavefront (1, 2, 4), 0: chosen per call
+int dx_quads_env(void)        { static int v = env_int("BBHIP_DX_QUADS", 0); return (v == 1 || v == 2 || v == 4) ? v : 0; }
 int dx_pass_steps_env(void)   { static int v = env_int("BBHIP_DX_STEPS", 0); return (v <= 0) ? 0 : (v <= 1) ? 1 : (v <= 2) ? 2 : 4; }
 // Wavefronts that share an input's work list in the dx kernels (DxArgs::split), 0 = none: four where one wavefront per (input node, unit) would
 // leave the launch with fewer than 4096 workgroups and the lists are long enough to share, sixteen where with four the launch
@@ -764,16 +766,15 @@ int dispatch_dx_table(int quads, DxTableArgs const &t, hipStream_t st)
     int const waves = t.dx.split ? t.dx.split : kWavesPerBlk;
     dim3 const grid(t.dx.chunk_count * t.dx.tiles.count), block(waves * kWave);
     ScopedTimer tm(kTimeDx, st);
-#define BBHIP_DX_CASE(Q, FAR)                                                                                                                  \
-    {                                                                                                                                          \
-        if (waves > kWavesPerBlk) { launch((lut_dx_table_kernel<N, BN, Q, kDxWaves, FAR>), grid, block, 0, st, t); }             \
-        else                      { launch((lut_dx_table_kernel<N, BN, Q, kWavesPerBlk, FAR>), grid, block, 0, st, t); }         \
+    bool const shared = waves > kWavesPerBlk;                   // (one group of 256 frames: run_backward_corner)
+    if (t.far) {
+        if (shared) { launch((lut_dx_table_kernel<N, BN, 1, kDxWaves, true>), grid, block, 0, st, t); }
+        else        { launch((lut_dx_table_kernel<N, BN, 1, kWavesPerBlk, true>), grid, block, 0, st, t); }
     }
-    if (t.far)           BBHIP_DX_CASE(1, true)
-    else if (quads == 1) BBHIP_DX_CASE(1, false)
-    else if (quads == 2) BBHIP_DX_CASE(2, false)
-    else                 BBHIP_DX_CASE(4, false)
-#undef BBHIP_DX_CASE
+    else if (shared)     { launch((lut_dx_table_kernel<N, BN, 1, kDxWaves>), grid, block, 0, st, t); }
+    else if (quads == 1) { launch((lut_dx_table_kernel<N, BN, 1, kWavesPerBlk>), grid, block, 0, st, t); }
+    else if (quads == 2) { launch((lut_dx_table_kernel<N, BN, 2, kWavesPerBlk>), grid, block, 0, st, t); }
+    else                 { launch((lut_dx_table_kernel<N, BN, 4, kWavesPerBlk>), grid, block, 0, st, t); }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -840,10 +841,9 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     DxTableArgs t{};
     // Frames per pass: a term's table and its loads are shared by the steps of a pass, so long passes where all the rows of dy and of indices
     // that a pass gathers from (5 bytes per node and frame) stay in an XCD's L2; halved while the launch would fall short of workgroups.
-    static int const quads_env = env_int("BBHIP_DX_QUADS", 0);
     int quads = (O <= 512) ? 4 : (O <= 1024) ? 2 : 1;
     while (quads > 1 && (long long)ceil_div(c.frame_size, quads * 256) * ceil_div(c.input_node_size, kWavesPerBlk) < 2048) { quads /= 2; }
-    if (quads_env == 1 || quads_env == 2 || quads_env == 4) { quads = quads_env; }
+    if (dx_quads_env() != 0) { quads = dx_quads_env(); }
     t.far = !s.dy_quads || (long long)O * c.frame_stride * 4 > 0xffffffffLL || (long long)O * own_words * 4 > 0xffffffffLL ||
             (long long)O * NN * 4 > 0xffffffffLL;
     if (t.far) { quads = 1; }
@@ -851,7 +851,9 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     d.dy = c.dy; d.dx = c.dx; d.rev = c.rev; d.rev_stride = c.rev_stride; d.input_node_size = c.input_node_size; d.frame_size = c.frame_size;
     d.dy_stride = c.frame_stride; d.dx_stride = c.frame_stride;
     d.chunk = quads * 256; d.chunk_count = ceil_div(c.frame_size, d.chunk);
-    int const split    = dx_split_lists(c.rev_stride - 1, c.input_node_size, O, c.frame_size, d.chunk_count);
+    int split          = dx_split_lists(c.rev_stride - 1, c.input_node_size, O, c.frame_size, d.chunk_count);
+    // Long passes leave at least 2048 workgroups, with which sixteen wavefronts never share a list: only BBHIP_DX_QUADS brings the two together
+    if (quads > 1 && split > kWavesPerBlk) { split = kWavesPerBlk; }
     int const in_tiles = split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
     if ((long long)d.chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
     d.tiles = make_tile_divisor(in_tiles); d.split = split;
@@ -924,7 +926,7 @@ int run_backward_small(BackwardCall const &c, hipStream_t st, int dw_overwrite)
         else                      { launch((lut_small_backward_kernel<N, U, kWavesPerBlk>), grid, block, 0, st, s); }
         if (steps == 1)      { BBHIP_SMALL_CASE(1) }
         else if (steps == 2) { BBHIP_SMALL_CASE(2) }
-        else                 { BBHIP_SMALL_CASE(4) }
+        else                 { launch((lut_small_backward_kernel<N, 4, kWavesPerBlk>), grid, block, 0, st, s); }       // (from 1024 workgroups: `enough`)
 #undef BBHIP_SMALL_CASE
     }
     BBHIP_LAUNCH_CHECK();
@@ -1401,6 +1403,7 @@ int bbhip_GetSwitch(char const *name)
     if (!strcmp(name, "corner")) { return use_corner_values(kXBit) ? 1 : 0; }
     if (!strcmp(name, "pack"))   { return pack_binarized_input() ? 1 : 0; }
     if (!strcmp(name, "inline_tables")) { return inline_tables() ? 1 : 0; }
+    if (!strcmp(name, "dx_quads")) { return dx_quads_env(); }
     return -1;
 }
 

@@ -73,7 +73,7 @@ size_t bbhip_GetScratchSize(void);
 /* ---- state of an environment switch as the library read it (instrumentation; no counterpart in the reference) ----
  * name "corner" (BBHIP_CORNER: lookup kernels for two-valued inputs) or "pack" (BBHIP_PACK: binarized fp32 frames are
  * packed to bits first): 1 on, 0 off, -1 unknown name.  A switch is off when its variable is 0 (or 2), on for any other
- * number, and takes its default (on) when unset. */
+ * number, and takes its default (on) when unset.  "inline_tables" (BBHIP_INLINE_TABLES) likewise; "dx_quads" (BBHIP_DX_QUADS): 1, 2 or 4, 0 = unset. */
 int bbhip_GetSwitch(char const *name);
 
 /* ---- how dx is accumulated over the fan-out of an input node (no counterpart in the reference) ----
