@@ -16,7 +16,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
                                  {"BBHIP_DX_STEPS": "1", "BBHIP_DX_CHUNK": "64", "BBHIP_BIN_NODES": "1", "BBHIP_BIN_CHUNK": "64"},
                                  {"BBHIP_DX_STEPS": "4", "BBHIP_DX_CHUNK": "512", "BBHIP_FWD_CHUNK": "512", "BBHIP_BIN_NODES": "2", "BBHIP_BIN_CHUNK": "256"},
                                  {"BBHIP_DX_SPLIT": "1"}, {"BBHIP_DX_SPLIT": "0", "BBHIP_BIN_NODES": "4"},
-                                 {"BBHIP_DX_WIDE": "0"}, {"BBHIP_INLINE_TABLES": "0"}, {"BBHIP_FWD_CHUNK": "2048"}, {"BBHIP_DX_INDEXED": "0"}, {"BBHIP_TERM_NODES": "0"}])
+                                 {"BBHIP_INLINE_TABLES": "0"}, {"BBHIP_FWD_CHUNK": "2048"}, {"BBHIP_DX_QUADS": "1"}, {"BBHIP_DX_QUADS": "2"},
+                                 {"BBHIP_DX_QUADS": "4"}, {"BBHIP_DX_QUADS": "4", "BBHIP_DX_SPLIT": "1"}])
 def test_two_valued_inputs_under_switches(env):
     child_env = dict(os.environ)
     child_env.update(env)
@@ -25,4 +26,5 @@ def test_two_valued_inputs_under_switches(env):
     assert p.returncode == 0 and "two-valued case ok" in p.stdout, (env, p.stdout[-2000:], p.stderr[-2000:])
     # the switches took effect: 0 and 2 turn a path off, unset leaves it on
     want = {name: 0 if env.get(var) in ("0", "2") else 1 for name, var in (("corner", "BBHIP_CORNER"), ("pack", "BBHIP_PACK"))}
-    assert "switches corner=%d pack=%d" % (want["corner"], want["pack"]) in p.stdout, (env, p.stdout[-500:])
+    assert "switches corner=%d pack=%d inline_tables=%d dx_quads=%d\n" % (want["corner"], want["pack"], 0 if env.get("BBHIP_INLINE_TABLES") == "0" else 1,
+                                                                         int(env.get("BBHIP_DX_QUADS", "0"))) in p.stdout, (env, p.stdout[-500:])

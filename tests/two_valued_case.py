@@ -63,7 +63,7 @@ def main():
     yb = ops.binary_lut6_forward(dev(xbb), dev(idx), dev(T), Fb)
     assert np.array_equal(host(yb), oracle.binary_lut6_forward(xbb, idx, T, Fb))
     from binarybrain_amd import capi
-    print("switches corner=%d pack=%d" % (capi.lib().bbhip_GetSwitch(b"corner"), capi.lib().bbhip_GetSwitch(b"pack")))
+    print("switches corner=%d pack=%d inline_tables=%d dx_quads=%d" % tuple(capi.lib().bbhip_GetSwitch(name) for name in (b"corner", b"pack", b"inline_tables", b"dx_quads")))
     print("two-valued case ok")
 
 
