@@ -1022,7 +1022,7 @@ def bench_forward_small(args, lib):
     out = {"metric": "G node-evals/s StochasticLut6 fp32 forward (784 -> 1024 nodes, 64 frames)", "value": O * F / dt / 1e9,
            "unit": "G node-evals/s", "n_gpus": 1, "steps": steps, "warmup": max(args.warmup, 20), "ms_per_step": dt * 1e3,
            "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f32", "data": "synthetic",
-           "config": {"workload": "StochasticLut6 forward fp32, 784 in x 1024 out x 64 frames (launch-bound: two launches per call)"},
+           "config": {"workload": "StochasticLut6 forward fp32, 784 in x 1024 out x 64 frames (launch-bound: one launch per call)"},
            "roofline": {"bound": "hbm", "kernel": "lut_forward_kernel<6>", "achieved": nbytes / (kernel_ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS,
                         "unit": "GB/s", "frac": nbytes / (kernel_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": None,
                         "kernel_ms": kernel_ms}}

@@ -40,7 +40,7 @@ __device__ __forceinline__ float wave_sum(float v)
 // ------------------------------------------------------------------------------------------------
 //  table preparation from W' (W' = lut_binarize ? W > 0.5 : W):
 //    C = coefficients in the centred monomial basis,  y = sum_S C[S] prod_{j in S} (x_j - 1/2)
-//  (the plain-basis coefficients P,  y = sum_S P[S] prod_{j in S} x_j,  are formed inside term_table_block)
+//  (the plain-basis coefficients P,  y = sum_S P[S] prod_{j in S} x_j,  are formed inside term_table_node_block)
 // ------------------------------------------------------------------------------------------------
 //  For two-valued inputs (x_j = 1/2 -+ bias) the layer is a table of 2^N values, V[p] = y at the corner whose bit j says
 //  which value input j takes: one more butterfly over C, (a, b) -> (a - bias b, a + bias b) per variable.
@@ -1245,7 +1245,7 @@ struct DxArgs {
     float const *dy;            // dL/d(LUT output) [O][dy_stride]
     float       *dx;            // [I][dx_stride]
     int const   *rev;           // reverse table [I][rev_stride]: count, then connection ids node*N + k
-    int const   *term;          // term table, see term_table_block
+    int const   *term;          // term table, see term_table_node_block
     int   rev_stride, input_node_size, frame_size;
     int   x_stride, dy_stride, dx_stride;
     int   chunk, chunk_count;
