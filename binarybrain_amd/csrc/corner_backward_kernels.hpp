@@ -220,14 +220,6 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
     for (int i = 0; i < (kCountSets ? NN : 1); ++i) { count[i] = 0; }
 
     for (int base = f_begin; base < f_end; base += kPasses * 4 * kWave) {
-        if (!SHORT && base - opened >= (skewed ? kSkewedChain : kFairChain)) {
-            opened = base;
-            skewed = false;
-            D += row_sum<NN, COLS>(reinterpret_cast<float4 const *>(mine), lane);
-            wave_fence();
-            clear_bins();
-            wave_fence();
-        }
         uint32_t quad[8];
         {
             uint32_t w[N];
@@ -304,9 +296,19 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
             }
         }
         wave_fence();
+        int const next = base + kPasses * 4 * kWave;
+        if (next >= f_end || next - opened >= (skewed ? kSkewedChain : kFairChain)) {           // (SHORT: one block)
+            D += row_sum<NN, COLS>(reinterpret_cast<float4 const *>(mine), lane);
+            if (next < f_end) {
+                opened = next;
+                skewed = false;
+                wave_fence();
+                clear_bins();
+                wave_fence();
+            }
+        }
     }
 
-    D += row_sum<NN, COLS>(reinterpret_cast<float4 const *>(mine), lane);
     uint32_t n = 0;
     if constexpr (BN && SHORT) { n = counts[wv][lane & (NN - 1)]; }
     if constexpr (kCountSets) {
