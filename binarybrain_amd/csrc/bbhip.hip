@@ -172,9 +172,8 @@ int fwd_chunk_frames(int xmode, int frame_size, int tile_count)
     return chunk;
 }
 int bwd_slab_frames(void)  { static int v = env_int("BBHIP_BWD_SLAB", 0);  return ((v + 63) / 64) * 64; }       // 0: chosen per call
-// dx units: frames per unit and wavefront-steps per pass over the work list.  128 frames in passes of two steps where the
-// gathered rows are fp32 (what L2 holds); packed-bit rows leave room for 256 frames in passes of four, which halves the
-// per-term set-up per frame.  0: not set in the environment.
+// dx units of lut_dx_kernel: frames per unit and wavefront-steps per pass over the work list, 128 frames (what L2 holds of fp32 rows) in passes of two
+// steps unless the environment says otherwise (0: not set)
 int dx_chunk_frames_env(void) { static int v = env_int("BBHIP_DX_CHUNK", 0); return ((v + 63) / 64) * 64; }
 // the dx kernel over kept corner indices: groups of 256 frames per wavefront (1, 2, 4), 0: chosen per call
 int dx_quads_env(void)        { static int v = env_int("BBHIP_DX_QUADS", 0); return (v == 1 || v == 2 || v == 4) ? v : 0; }
