@@ -739,7 +739,7 @@ int corner_slab_frames(int frame_size, int tile_count)
     return best;
 }
 
-template <int N, bool BN>
+template <int N, bool BN, bool QUADS>
 int launch_corner_backward(CornerSumsArgs const &s, int slab_count, hipStream_t st)
 {
     {
@@ -747,9 +747,9 @@ int launch_corner_backward(CornerSumsArgs const &s, int slab_count, hipStream_t 
         dim3 const grid(s.slab_count * s.tiles.count);
         bool launched = false;
         if constexpr (N >= 5) {             // (with few corners the atomics that count them collide, and the plain form has little to keep anyway)
-            if (slab_count == 1 && s.frame_size <= kShortSlab) { launch((lut_corner_sums_kernel<N, BN, true>), grid, dim3(kBlock), 0, st, s); launched = true; }
+            if (slab_count == 1 && s.frame_size <= kShortSlab) { launch((lut_corner_sums_kernel<N, BN, true, QUADS>), grid, dim3(kBlock), 0, st, s); launched = true; }
         }
-        if (!launched) { launch((lut_corner_sums_kernel<N, BN, false>), grid, dim3(kBlock), 0, st, s); }
+        if (!launched) { launch((lut_corner_sums_kernel<N, BN, false, QUADS>), grid, dim3(kBlock), 0, st, s); }
     }
     BBHIP_LAUNCH_CHECK();
     if (slab_count > 1) {
@@ -834,8 +834,9 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     s.fold.dW = c.dW; s.fold.overwrite = dw_overwrite; s.fold.node_consts = consts;
     static std::atomic<uint32_t> calls{0};
     s.fold.discard = reinterpret_cast<uint32_t *>(consts + O); s.fold.call = calls.fetch_add(1, std::memory_order_relaxed);
-    s.dy_quads = (c.frame_stride >= ((c.frame_size + 3) & ~3)) ? 1 : 0;
-    if (c.bn ? launch_corner_backward<N, true>(s, slab_count, st) : launch_corner_backward<N, false>(s, slab_count, st)) { return 1; }
+    bool const dy_quads = c.frame_stride >= ((c.frame_size + 3) & ~3);      // rows of dy hold whole groups of four frames: one 16-byte load per lane and pass
+    if (dy_quads ? (c.bn ? launch_corner_backward<N, true, true>(s, slab_count, st) : launch_corner_backward<N, false, true>(s, slab_count, st))
+                 : (c.bn ? launch_corner_backward<N, true, false>(s, slab_count, st) : launch_corner_backward<N, false, false>(s, slab_count, st))) { return 1; }
 
     DxTableArgs t{};
     // Frames per pass: a term's table and its loads are shared by the steps of a pass, so long passes where all the rows of dy and of indices
@@ -843,7 +844,7 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     int quads = (O <= 512) ? 4 : (O <= 1024) ? 2 : 1;
     while (quads > 1 && (long long)ceil_div(c.frame_size, quads * 256) * ceil_div(c.input_node_size, kWavesPerBlk) < 2048) { quads /= 2; }
     if (dx_quads_env() != 0) { quads = dx_quads_env(); }
-    t.far = !s.dy_quads || (long long)O * c.frame_stride * 4 > 0xffffffffLL || (long long)O * own_words * 4 > 0xffffffffLL ||
+    t.far = !dy_quads || (long long)O * c.frame_stride * 4 > 0xffffffffLL || (long long)O * own_words * 4 > 0xffffffffLL ||
             (long long)O * NN * 4 > 0xffffffffLL;
     if (t.far) { quads = 1; }
     DxArgs &d = t.dx;

@@ -91,17 +91,17 @@ struct CornerSumsArgs {
     int   node_size, frame_size, x_stride, dy_stride;
     int   slab, slab_count;     // frames per unit, a multiple of 256
     TileDivisor tiles;
-    int   dy_quads;             // rows of dy hold whole groups of four frames: one 16-byte load per lane and pass
     uint32_t *own;              // the corner index of every (node, frame), a byte each in frame order, for the dx kernel: rows of own_stride words
     int   own_stride;
     float *partial;             // several slabs: [slab][O][BN ? 2 : 1][2^N], D and then n
     CornerFoldArgs fold;        // one slab: the wavefront folds its sums itself
 };
 
-// four consecutive frames of a row from byte offset off; quads: the row holds whole groups of four
-__device__ __forceinline__ float4 load_quad(__amdgpu_buffer_rsrc_t r, uint32_t off, bool quads)
+// four consecutive frames of a row from byte offset off; QUADS: the row holds whole groups of four
+template <bool QUADS>
+__device__ __forceinline__ float4 load_quad(__amdgpu_buffer_rsrc_t r, uint32_t off)
 {
-    if (quads) {
+    if constexpr (QUADS) {
         auto const q = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
         return make_float4(__uint_as_float(q[0]), __uint_as_float(q[1]), __uint_as_float(q[2]), __uint_as_float(q[3]));
     }
@@ -148,18 +148,19 @@ __device__ __forceinline__ auto row_sum(V4 const *block, int lane)
 // cleared (256 clocks of LDS).  rms error of dW against 64 bits relative to a node's largest entry, by a model of the order of operations, 65536
 // frames, against multiply-adds in slabs of 4096 frames: inputs set in half of the frames 4e-8 (multiply-adds 8e-8), in 85 of 100 4e-8 (5e-8),
 // in 98 of 100 5e-8 (6e-8; 1.5e-7 as one chain).  4096 x 8192 and 216 x 230400 take 1 and 5 us longer where the bins are closed every 4096 frames.
-// The bins leave two workgroups per compute unit: dy is requested four passes ahead and the words a block ahead, as vector loads
-// (scalar loads would be waited for with the LDS accesses: 101 us for the first shape below).
-// Measured against the statistics and table-gradient launches that it replaces: 216 nodes x 230400 frames 65 us (3.8 TB/s of dy and indices)
-// instead of 53 + 141; 4096 x 8192 42 us instead of 31 + 106; 6144 x 1024 20 us instead of 11 + 30.
+// The bins leave two workgroups per compute unit, so what the wavefronts wait for shows: words and dy are requested a block ahead, on every path (a
+// load that a path may leave out makes the compiler wait for all that are under way), as vector loads (scalar loads would be waited for with the LDS
+// accesses: 101 us for the first shape below), and four frames' bins are read together.  4096 nodes x 8192 frames 40.0 -> 36.4 us, 3003 x 5005
+// 27.8 -> 23.0, 216 x 230400 65 -> 57 (4.4 TB/s of dy and indices).
+// QUADS: rows of dy hold whole groups of four frames.
+// The statistics and table-gradient launches that it replaces took 53 + 141 us for 216 nodes x 230400 frames, 31 + 106 for 4096 x 8192.
 // SHORT: up to kShortSlab frames in one slab.  Such a launch is a chain of latencies, so what counts is how many wavefronts share a compute unit: two
 // lanes share a column of bins (they add in turn), and the corners are counted by integer atomics (one instruction per step, and nothing to add up).
-// 6144 nodes x 1024 frames 20.5 -> 14.9 us, 6000 x 100 17.4 -> 9.6 us; four lanes per column measured the same or slower.
-template <int N, bool BN, bool SHORT>
-__global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs a)
+// 6144 nodes x 1024 frames 20.5 -> 13.6 us, 6000 x 100 17.4 -> 9.6 us; four lanes per column measured the same or slower.
+template <int N, bool BN, bool SHORT, bool QUADS>
+__global__ __launch_bounds__(kBlock, 2) void lut_corner_sums_kernel(CornerSumsArgs a)
 {
-    constexpr int NN = 1 << N, kAhead = 4, kPasses = SHORT ? kShortSlab / (4 * kWave) : 8, COLS = SHORT ? kShortColumns : kWave;
-    static_assert(!SHORT || kPasses <= kAhead, "all of dy requested ahead");
+    constexpr int NN = 1 << N, kPasses = SHORT ? kShortSlab / (4 * kWave) : 8, COLS = SHORT ? kShortColumns : kWave;
     __shared__ __align__(16) float bins[kWavesPerBlk][NN * COLS];
     __shared__ __align__(16) uint32_t quads[kWavesPerBlk][kPasses * kWave];
     __shared__ uint32_t counts[kWavesPerBlk][(BN && SHORT) ? NN : 1];
@@ -174,8 +175,7 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
 
     int const f_begin = sl * a.slab;
     int const f_end   = min(f_begin + a.slab, a.frame_size);
-    bool const quad_rows = a.dy_quads != 0;
-    __amdgpu_buffer_rsrc_t const dyr = row_descriptor(a.dy, node, a.dy_stride, quad_row_bytes(a.frame_size, quad_rows));
+    __amdgpu_buffer_rsrc_t const dyr = row_descriptor(a.dy, node, a.dy_stride, quad_row_bytes(f_end, QUADS));      // (past the slab: no access, zeros)
     uint32_t const x_row_bytes = (uint32_t)((a.frame_size + 31) >> 5) * 4u;
     __amdgpu_buffer_rsrc_t xr[N];
 #pragma unroll
@@ -186,10 +186,10 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
 #pragma unroll
         for (int k = 0; k < N; ++k) { w_next[k] = __builtin_amdgcn_raw_buffer_load_b32(xr[k], (uint32_t)((base >> 5) + lane) * 4u, 0, 0); }
     };
-    float4 dy[kAhead];
+    float4 dy[kPasses];
     request_words(f_begin);
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) { dy[i] = load_quad(dyr, (uint32_t)(f_begin + i * 4 * kWave + 4 * lane) * 4u, quad_rows); }
+    for (int i = 0; i < kPasses; ++i) { dy[i] = load_quad<QUADS>(dyr, (uint32_t)(f_begin + i * 4 * kWave + 4 * lane) * 4u); }
 
     CornerFoldInputs fold_in{};
     if (a.slab_count == 1) { fold_in = corner_fold_inputs<N, BN>(a.fold, node, lane); }
@@ -206,6 +206,19 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
     auto clear_bins = [&]() {
 #pragma unroll
         for (int i = 0; i < NN * COLS / (4 * kWave); ++i) { *reinterpret_cast<float4 *>(mine + (i * kWave + lane) * 4) = make_float4(0.0f, 0.0f, 0.0f, 0.0f); }
+    };
+    // Four frames into bins that may be the same: all four bins are read before any is written, a later frame takes an earlier one's sum.  (One
+    // after another, each waits for the bin that the one before it wrote.)
+    auto add_quad = [&](uint32_t corners, float4 const &d) {
+        uint32_t const p0 = corners & 0xffu, p1 = (corners >> 8) & 0xffu, p2 = (corners >> 16) & 0xffu, p3 = corners >> 24;
+        float *const col = mine + (lane & (COLS - 1));
+        float r0 = col[p0 * COLS], r1 = col[p1 * COLS], r2 = col[p2 * COLS], r3 = col[p3 * COLS];
+        asm("" : "+v"(r0), "+v"(r1), "+v"(r2), "+v"(r3));               // (no branch around a read whose value a lane does not need)
+        float const v0 = r0 + d.x;
+        float const v1 = (p1 == p0 ? v0 : r1) + d.y;
+        float const v2 = (p2 == p1 ? v1 : p2 == p0 ? v0 : r2) + d.z;
+        float const v3 = (p3 == p2 ? v2 : p3 == p1 ? v1 : p3 == p0 ? v0 : r3) + d.w;
+        col[p0 * COLS] = v0; col[p1 * COLS] = v1; col[p2 * COLS] = v2; col[p3 * COLS] = v3;
     };
     clear_bins();
     if (BN && SHORT && lane < NN) { counts[wv][lane] = 0; }
@@ -252,6 +265,7 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
                 for (int s = 1; s < NN; ++s) {
                     all[s] = all[s & (s - 1)] & w[__builtin_ctz(s)];
                     count[s] += __popc(all[s]);
+                    asm volatile("" : "+v"(count[s]));                  // (here, not moved behind the passes with all 2^N sets alive)
                 }
             }
         }
@@ -262,38 +276,34 @@ __global__ __launch_bounds__(kBlock) void lut_corner_sums_kernel(CornerSumsArgs 
 #pragma unroll
         for (int i = 0; i < kPasses; ++i) {
             int const fb = base + i * 4 * kWave;
-            if (fb >= f_end) { break; }                                 // wave-uniform
-            float4 d = dy[i % kAhead];
-            if (!SHORT) { dy[i % kAhead] = load_quad(dyr, (uint32_t)(fb + kAhead * 4 * kWave + 4 * lane) * 4u, quad_rows); }
-            if (fb + 4 * kWave > a.frame_size) {                        // the row's padding may hold anything
-                int const f = fb + 4 * lane;
-                if (f     >= a.frame_size) { d.x = 0.0f; }
-                if (f + 1 >= a.frame_size) { d.y = 0.0f; }
-                if (f + 2 >= a.frame_size) { d.z = 0.0f; }
-                if (f + 3 >= a.frame_size) { d.w = 0.0f; }
-            }
-            if constexpr (BN && SHORT) {
-                int const f = fb + 4 * lane;
-                if (f     < f_end) { atomicAdd(&counts[wv][at[i] & 0xffu], 1u); }
-                if (f + 1 < f_end) { atomicAdd(&counts[wv][(at[i] >> 8) & 0xffu], 1u); }
-                if (f + 2 < f_end) { atomicAdd(&counts[wv][(at[i] >> 16) & 0xffu], 1u); }
-                if (f + 3 < f_end) { atomicAdd(&counts[wv][at[i] >> 24], 1u); }
-            }
-            auto add_all = [&]() {
-                int const col = lane & (COLS - 1);
-                mine[(at[i] & 0xffu) * COLS + col] += d.x;
-                mine[((at[i] >> 8) & 0xffu) * COLS + col] += d.y;
-                mine[((at[i] >> 16) & 0xffu) * COLS + col] += d.z;
-                mine[(at[i] >> 24) * COLS + col] += d.w;
-            };
-            if constexpr (COLS == kWave) { add_all(); }
-            else {
+            if (fb < f_end) {                                           // wave-uniform
+                float4 d = dy[i];
+                if (fb + 4 * kWave > a.frame_size) {                    // the row's padding may hold anything
+                    int const f = fb + 4 * lane;
+                    if (f     >= a.frame_size) { d.x = 0.0f; }
+                    if (f + 1 >= a.frame_size) { d.y = 0.0f; }
+                    if (f + 2 >= a.frame_size) { d.z = 0.0f; }
+                    if (f + 3 >= a.frame_size) { d.w = 0.0f; }
+                }
+                if constexpr (BN && SHORT) {
+                    int const f = fb + 4 * lane;
+                    if (f     < f_end) { atomicAdd(&counts[wv][at[i] & 0xffu], 1u); }
+                    if (f + 1 < f_end) { atomicAdd(&counts[wv][(at[i] >> 8) & 0xffu], 1u); }
+                    if (f + 2 < f_end) { atomicAdd(&counts[wv][(at[i] >> 16) & 0xffu], 1u); }
+                    if (f + 3 < f_end) { atomicAdd(&counts[wv][at[i] >> 24], 1u); }
+                }
+                if constexpr (COLS == kWave) { add_quad(at[i], d); }
+                else {
 #pragma unroll
-                for (int turn = 0; turn < kWave / COLS; ++turn) {
-                    if (lane / COLS == turn) { add_all(); }
-                    wave_fence();
+                    for (int turn = 0; turn < kWave / COLS; ++turn) {
+                        if (lane / COLS == turn) { add_quad(at[i], d); }
+                        wave_fence();
+                    }
                 }
             }
+            // (outside of the condition: loads that a path may leave out make the compiler wait for all that are under way)
+            __builtin_amdgcn_sched_barrier(0);                          // (into the registers that are free now)
+            if (!SHORT) { dy[i] = load_quad<QUADS>(dyr, (uint32_t)(fb + kPasses * 4 * kWave + 4 * lane) * 4u); }
         }
         wave_fence();
         int const next = base + kPasses * 4 * kWave;
@@ -446,7 +456,7 @@ __global__ __launch_bounds__(WAVES * kWave) void lut_dx_table_kernel(DxTableArgs
         for (int q = 0; q < Q; ++q) { s.iw[q] = __builtin_amdgcn_raw_buffer_load_b32(i_row, (uint32_t)(f_lane + q * 4 * kWave), i_off, 0); }
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            if constexpr (FAR) { s.dy[q] = load_quad(d_row, (uint32_t)(f_lane + q * 4 * kWave) * 4u, false); continue; }
+            if constexpr (FAR) { s.dy[q] = load_quad<false>(d_row, (uint32_t)(f_lane + q * 4 * kWave) * 4u); continue; }
             auto const d = __builtin_amdgcn_raw_buffer_load_b128(d_row, (uint32_t)(f_lane + q * 4 * kWave) * 4u, d_off, 0);
             s.dy[q] = make_float4(__uint_as_float(d[0]), __uint_as_float(d[1]), __uint_as_float(d[2]), __uint_as_float(d[3]));
         }
