@@ -18,7 +18,7 @@
 #include "../../include/bbhip.h"
 #include "lut_kernels.hpp"
 #include "corner_forward_kernels.hpp"
-#include "corner_backward_kernels.hpp"
+#include "corner_small_backward_kernels.hpp"
 #include "table_gradient_kernels.hpp"
 #include "small_backward_kernels.hpp"
 #include "vector_kernels.hpp"
@@ -745,11 +745,8 @@ int launch_corner_backward(CornerSumsArgs const &s, int slab_count, hipStream_t 
     {
         ScopedTimer tm(kTimeBackward, st);
         dim3 const grid(s.slab_count * s.tiles.count);
-        bool launched = false;
-        if constexpr (N >= 5) {             // (with few corners the atomics that count them collide, and the plain form has little to keep anyway)
-            if (slab_count == 1 && s.frame_size <= kShortSlab) { launch((lut_corner_sums_kernel<N, BN, true, QUADS>), grid, dim3(kBlock), 0, st, s); launched = true; }
-        }
-        if (!launched) { launch((lut_corner_sums_kernel<N, BN, false, QUADS>), grid, dim3(kBlock), 0, st, s); }
+        if (N >= 5 && slab_count == 1 && s.frame_size <= kShortSlab) { launch((lut_corner_sums_kernel<N, BN, (N >= 5 ? kSumsShort : kSumsLong), QUADS>), grid, dim3(kBlock), 0, st, s); }
+        else { launch((lut_corner_sums_kernel<N, BN, kSumsLong, QUADS>), grid, dim3(kBlock), 0, st, s); }
     }
     BBHIP_LAUNCH_CHECK();
     if (slab_count > 1) {
@@ -778,7 +775,43 @@ int dispatch_dx_table(int quads, DxTableArgs const &t, hipStream_t st)
     return 0;
 }
 
-// Two-valued inputs with the deterministic dx (corner_backward_kernels.hpp): per-corner sums, fold, dx from kept corner indices.
+// Small layers on two-valued inputs whose backward pass is one launch (lut_corner_small_backward_kernel), 256 PASSES frames: what its wavefronts walk
+// one after another must be short, and what they do for every connection (the sums through the statistics) little in all.  Backward call alone,
+// microseconds, against two launches; links: connections, fan: the longest list.
+//   256 frames: 784 inputs x 1024 nodes (fan 18) 6.2 and 9.4, 1024 x 360 5.8 and 9.0, 784 x 6144 (fan 76) 16.1 and 18.5, 2001 x 3003 10.2 and 11.0;
+//               150 x 3000 (fan 155) 20.5 and 12.0
+//   512 frames: 300 x 300 (fan 14) 6.3 and 10.0, 784 x 1024 (4700 links) 8.8 and 9.4; 2000 x 2000 12.7 and 11.9, 400 x 2000 (fan 46) 14.5 and 12.5
+//   1024 frames: 360 x 70 5.9 and 8.8, 500 x 500 (3000 links) 9.0 and 10.8; 784 x 1024 12.1 and 11.3, 200 x 500 (fan 24) 10.8 and 9.6
+// Lists are shared by the wavefronts of a workgroup, except where there are many inputs with little to walk: 6144 x 1024 (256 frames, fan 8) 10.2
+// shared, 8.4 not, two launches 9.8; 4096 x 4096 (fan 17) 14.5, 13.5 and 13.3.
+bool small_corner_layer(BackwardCall const &c, int &passes, bool &share)
+{
+    if (c.frame_size > kShortSlab || bwd_slab_frames() > 0 || dx_quads_env() != 0) { return false; }
+    if ((long long)c.input_node_size * c.x_stride * 4 > 0xffffffffLL || (long long)c.output_node_size * c.frame_stride * 4 > 0xffffffffLL ||
+        (long long)c.output_node_size * (4 << c.n) > 0xffffffffLL) { return false; }                              // (32-bit offsets into whole buffers)
+    passes = c.frame_size <= 256 ? 1 : c.frame_size <= 512 ? 2 : 4;
+    int const fan = c.rev_stride - 1;
+    long long const links = (long long)c.output_node_size * c.n;
+    share = c.input_node_size <= (passes == 1 ? 2048 : 1536);
+    static_assert(8 <= kCornerSmallItems && 20 <= kCornerSmallItems, "the kernel holds a wavefront's items one per lane");
+    if (!share) { return passes == 1 && fan <= 8; }
+    return ceil_div(fan, kWavesPerBlk) <= (passes == 1 ? 20 : 16 / passes) && links * passes <= (passes == 1 ? 40000 : 12000);
+}
+
+template <int N, bool BN, bool QUADS>
+int launch_corner_small(CornerSmallArgs const &t, int passes, hipStream_t st)
+{
+    dim3 const grid(t.dx_blocks + ceil_div(t.sums.node_size, kWavesPerBlk));
+    ScopedTimer tm(kTimeBackward, st);
+    if (passes == 1)      { launch((lut_corner_small_backward_kernel<N, BN, 1, QUADS>), grid, dim3(kBlock), 0, st, t); }
+    else if (passes == 2) { launch((lut_corner_small_backward_kernel<N, BN, 2, QUADS>), grid, dim3(kBlock), 0, st, t); }
+    else                  { launch((lut_corner_small_backward_kernel<N, BN, 4, QUADS>), grid, dim3(kBlock), 0, st, t); }
+    BBHIP_LAUNCH_CHECK();
+    return 0;
+}
+
+// Two-valued inputs with the deterministic dx (corner_backward_kernels.hpp): per-corner sums, fold, dx from kept corner indices; small layers in
+// one launch.
 template <int N>
 int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHint packed, PreparedTablesHint tables, int dw_overwrite)
 {
@@ -793,18 +826,23 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     if (from_fp32) { c.x_stride = have_bits ? packed.row_words : packed_row_words(c.frame_size); }
 
     int const O = c.output_node_size, tile_count = ceil_div(O, kWavesPerBlk);
-    int slab = corner_slab_frames(c.frame_size, tile_count);
+    int slab = corner_slab_frames(c.frame_size, tile_count);            // (up to kShortSlab frames: one)
     size_t const slab_bytes = (size_t)O * NN * sizeof(float) * (c.bn ? 2 : 1);
     while ((size_t)ceil_div(c.frame_size, slab) * slab_bytes > ((size_t)256 << 20) && slab < c.frame_size) { slab *= 2; }
     int const slab_count = ceil_div(c.frame_size, slab);
     if ((long long)slab_count * tile_count > 0x7fffffffLL) { return fail("backward: grid too large"); }
     int const own_words = ceil_div(c.frame_size, 32) * 8;
 
-    // the nodes' corner values: from the buffer that the caller kept from this step's forward call, else derived by the sums kernel
+    int passes = 0;
+    bool share = false;
+    bool const small = small_corner_layer(c, passes, share);
+
+    // the nodes' corner values: from the buffer that the caller kept from this step's forward call, else derived by the sums kernel (small layers:
+    // by each wavefront that needs them)
     size_t const v_bytes     = align256((size_t)O * NN * sizeof(float));
     bool const   have_tables = tables.holds_tables && tables_fit(tables, 2 * v_bytes);
-    size_t const own_bytes   = align256((size_t)O * own_words * sizeof(uint32_t));
-    size_t const const_bytes = c.bn ? align256((size_t)O * sizeof(NodeConsts) + sizeof(uint32_t)) : 0;     // (and the word `discard` behind them)
+    size_t const own_bytes   = small ? 0 : align256((size_t)O * own_words * sizeof(uint32_t));
+    size_t const const_bytes = small ? 0 : c.bn ? align256((size_t)O * sizeof(NodeConsts) + sizeof(uint32_t)) : 0;     // (and the word `discard` behind them)
     size_t const part_bytes  = slab_count > 1 ? align256((size_t)slab_count * slab_bytes) : 0;
     size_t const bits_bytes  = (from_fp32 && !have_bits) ? align256((size_t)c.input_node_size * c.x_stride * sizeof(uint32_t)) : 0;
     char *base = nullptr;
@@ -824,17 +862,28 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     CornerSumsArgs s{};
     s.x = reinterpret_cast<uint32_t const *>(c.x); s.dy = c.dy; s.idx = c.idx;
     if (have_tables) { s.V = V; }
-    else             { s.W_inline = c.W; s.V_out = V; }
+    else             { s.W_inline = c.W; s.V_out = small ? nullptr : V; }
     s.lut_binarize = c.lut_binarize; s.bias = c.bias;
     s.node_size = O; s.frame_size = c.frame_size; s.x_stride = c.x_stride; s.dy_stride = c.frame_stride;
     s.slab = slab; s.slab_count = slab_count; s.tiles = make_tile_divisor(tile_count);
-    s.own = own; s.own_stride = own_words; s.partial = part;
+    s.own = small ? nullptr : own; s.own_stride = own_words; s.partial = part;
     s.fold.mean = c.mean; s.fold.rstd = c.rstd; s.fold.gamma = c.gamma; s.fold.beta = c.beta; s.fold.inv_frames = 1.0f / (float)c.frame_size;
     s.fold.frame_size = c.frame_size; s.fold.lo = 0.5f - c.bias; s.fold.hi = 0.5f + c.bias;
-    s.fold.dW = c.dW; s.fold.overwrite = dw_overwrite; s.fold.node_consts = consts;
+    s.fold.dW = c.dW; s.fold.overwrite = dw_overwrite; s.fold.node_consts = small ? nullptr : consts;
     static std::atomic<uint32_t> calls{0};
     s.fold.discard = reinterpret_cast<uint32_t *>(consts + O); s.fold.call = calls.fetch_add(1, std::memory_order_relaxed);
     bool const dy_quads = c.frame_stride >= ((c.frame_size + 3) & ~3);      // rows of dy hold whole groups of four frames: one 16-byte load per lane and pass
+    if (small) {
+        CornerSmallArgs t{};
+        t.sums = s;
+        t.inv_step = 1.0f / (s.fold.hi - s.fold.lo);
+        DxArgs &d = t.dx;
+        d.dx = c.dx; d.rev = c.rev; d.rev_stride = c.rev_stride; d.input_node_size = c.input_node_size; d.frame_size = c.frame_size; d.dx_stride = c.frame_stride;
+        d.split = share ? kWavesPerBlk : 0;
+        t.dx_blocks = share ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
+        return dy_quads ? (c.bn ? launch_corner_small<N, true, true>(t, passes, st) : launch_corner_small<N, false, true>(t, passes, st))
+                        : (c.bn ? launch_corner_small<N, true, false>(t, passes, st) : launch_corner_small<N, false, false>(t, passes, st));
+    }
     if (dy_quads ? (c.bn ? launch_corner_backward<N, true, true>(s, slab_count, st) : launch_corner_backward<N, false, true>(s, slab_count, st))
                  : (c.bn ? launch_corner_backward<N, true, false>(s, slab_count, st) : launch_corner_backward<N, false, false>(s, slab_count, st))) { return 1; }
 

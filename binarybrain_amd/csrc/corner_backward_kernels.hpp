@@ -27,7 +27,7 @@ struct CornerFoldArgs {
     float lo, hi;                       // the two input values, 1/2 -+ bias
     float *dW;
     int   overwrite;                    // dW = instead of dW +=
-    struct NodeConsts *node_consts;     // batch-norm: what the dx kernel needs of each node beside its corner values
+    struct NodeConsts *node_consts;     // batch-norm: what lut_dx_table_kernel needs of each node beside its corner values (null: nothing)
     // batch-norm: *discard = call where a discarded dy (one at a corner outside the hard-tanh window) may not be finite.  `call` is another number for
     // each call, so that nothing has to be cleared ahead; a stale equal value only sends the dx kernel to its slower walk
     uint32_t *discard;
@@ -67,8 +67,8 @@ __device__ __forceinline__ void corner_fold(CornerFoldArgs const &a, CornerFoldI
         float const inv_step = 1.0f / (a.hi - a.lo);
         // (one value that is not finite makes its corner's sum such)
         bool const discard = __ballot((t <= 0.0f || t >= 1.0f) && !(fabsf(D) < __builtin_inff())) != 0;
-        if (lane == 0 && discard) { *a.discard = a.call; }
-        if (lane == 0) { a.node_consts[node] = NodeConsts{mean, a.gamma * rstd * inv_step, shift * inv_step, scale * inv_step, open, 0}; }
+        if (lane == 0 && discard && a.node_consts != nullptr) { *a.discard = a.call; }
+        if (lane == 0 && a.node_consts != nullptr) { a.node_consts[node] = NodeConsts{mean, a.gamma * rstd * inv_step, shift * inv_step, scale * inv_step, open, 0}; }
     }
     // per input: (G0, G1) -> ((1 - lo) G0 + (1 - hi) G1, lo G0 + hi G1), and 1 - lo = hi: either lane keeps hi of its own and takes lo of the other's
 #pragma unroll
@@ -76,7 +76,26 @@ __device__ __forceinline__ void corner_fold(CornerFoldArgs const &a, CornerFoldI
     if (lane < NN) { a.dW[(size_t)node * NN + lane] = a.overwrite ? G : q.dW + G; }
 }
 
-constexpr int kShortSlab = 1024, kShortColumns = 32;            // see lut_corner_sums_kernel
+// How a wavefront adds up the frames of a node (see lut_corner_sums_kernel): kSumsLong any number of frames in blocks of 2048; the others up to
+// 256, 512 and 1024 frames, all of them requested at once
+enum SumsForm : int { kSumsLong = 0, kSums256 = 1, kSums512 = 2, kSumsShort = 4 };
+constexpr int kShortSlab = 1024;
+template <int N, bool BN, int FORM>
+struct SumsTraits {
+    static constexpr int  NN = 1 << N;
+    static constexpr bool kLoop = FORM == kSumsLong;
+    // (with few corners the atomics that count them collide, and the plain form has little to keep anyway)
+    static constexpr bool kAtomics = !kLoop && N >= 5, kCountSets = BN && !kAtomics, kCountFrames = BN && kAtomics;
+    static constexpr int  kPasses = kLoop ? 8 : FORM;
+    static constexpr int  kColumns = !kAtomics ? kWave : FORM == kSums256 ? 16 : 32;
+};
+template <int N, bool BN, int FORM>
+struct SumsShared {                     // a wavefront's LDS
+    using T = SumsTraits<N, BN, FORM>;
+    __align__(16) float    bins[T::NN * T::kColumns];
+    __align__(16) uint32_t quads[T::kPasses * kWave];
+    uint32_t counts[T::kCountFrames ? T::NN : 1];
+};
 constexpr int kSkewedChain = 4096, kFairChain = 16384;          // frames, see there
 
 struct CornerSumsArgs {
@@ -99,15 +118,15 @@ struct CornerSumsArgs {
 
 // four consecutive frames of a row from byte offset off; QUADS: the row holds whole groups of four
 template <bool QUADS>
-__device__ __forceinline__ float4 load_quad(__amdgpu_buffer_rsrc_t r, uint32_t off)
+__device__ __forceinline__ float4 load_quad(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t row_off = 0)
 {
     if constexpr (QUADS) {
-        auto const q = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+        auto const q = __builtin_amdgcn_raw_buffer_load_b128(r, off, row_off, 0);
         return make_float4(__uint_as_float(q[0]), __uint_as_float(q[1]), __uint_as_float(q[2]), __uint_as_float(q[3]));
     }
     float v[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) { v[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off + 4 * j, 0, 0)); }
+    for (int j = 0; j < 4; ++j) { v[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off + 4 * j, row_off, 0)); }
     return make_float4(v[0], v[1], v[2], v[3]);
 }
 
@@ -157,22 +176,12 @@ __device__ __forceinline__ auto row_sum(V4 const *block, int lane)
 // SHORT: up to kShortSlab frames in one slab.  Such a launch is a chain of latencies, so what counts is how many wavefronts share a compute unit: two
 // lanes share a column of bins (they add in turn), and the corners are counted by integer atomics (one instruction per step, and nothing to add up).
 // 6144 nodes x 1024 frames 20.5 -> 13.6 us, 6000 x 100 17.4 -> 9.6 us; four lanes per column measured the same or slower.
-template <int N, bool BN, bool SHORT, bool QUADS>
-__global__ __launch_bounds__(kBlock, 2) void lut_corner_sums_kernel(CornerSumsArgs a)
+template <int N, bool BN, int FORM, bool QUADS>
+__device__ __forceinline__ void corner_sums_unit(CornerSumsArgs const &a, SumsShared<N, BN, FORM> &sh, int node, int sl, int lane)
 {
-    constexpr int NN = 1 << N, kPasses = SHORT ? kShortSlab / (4 * kWave) : 8, COLS = SHORT ? kShortColumns : kWave;
-    __shared__ __align__(16) float bins[kWavesPerBlk][NN * COLS];
-    __shared__ __align__(16) uint32_t quads[kWavesPerBlk][kPasses * kWave];
-    __shared__ uint32_t counts[kWavesPerBlk][(BN && SHORT) ? NN : 1];
-    int const B   = a.slab_count * a.tiles.count;
-    int const lid = xcd_remap(blockIdx.x, B);
-    int sl, tile;
-    split_tile(lid, a.tiles, sl, tile);
-    int const wv   = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-    int const node = tile * kWavesPerBlk + wv;
-    if (node >= a.node_size) { return; }
-    int const lane = threadIdx.x & (kWave - 1);
-
+    using T = SumsTraits<N, BN, FORM>;
+    constexpr int NN = 1 << N, kPasses = T::kPasses, COLS = T::kColumns;
+    constexpr bool kLoop = T::kLoop, kCountSets = T::kCountSets, kCountFrames = T::kCountFrames;
     int const f_begin = sl * a.slab;
     int const f_end   = min(f_begin + a.slab, a.frame_size);
     __amdgpu_buffer_rsrc_t const dyr = row_descriptor(a.dy, node, a.dy_stride, quad_row_bytes(f_end, QUADS));      // (past the slab: no access, zeros)
@@ -202,7 +211,7 @@ __global__ __launch_bounds__(kBlock, 2) void lut_corner_sums_kernel(CornerSumsAr
         v = corner_butterfly<N>(centred_butterfly<N>(w, i), i, a.bias);
     }
 
-    float *const mine = bins[wv];
+    float *const mine = sh.bins;
     auto clear_bins = [&]() {
 #pragma unroll
         for (int i = 0; i < NN * COLS / (4 * kWave); ++i) { *reinterpret_cast<float4 *>(mine + (i * kWave + lane) * 4) = make_float4(0.0f, 0.0f, 0.0f, 0.0f); }
@@ -221,13 +230,12 @@ __global__ __launch_bounds__(kBlock, 2) void lut_corner_sums_kernel(CornerSumsAr
         col[p0 * COLS] = v0; col[p1 * COLS] = v1; col[p2 * COLS] = v2; col[p3 * COLS] = v3;
     };
     clear_bins();
-    if (BN && SHORT && lane < NN) { counts[wv][lane] = 0; }
+    if (kCountFrames && lane < NN) { sh.counts[lane] = 0; }
     wave_fence();
 
     float D = 0.0f;                                                     // lane p: sums of the bins that were closed
     int  opened = f_begin;
     bool skewed = false;
-    constexpr bool kCountSets = BN && !SHORT;
     uint32_t count[kCountSets ? NN : 1];                                // [S]: frames of the lane's words where every input of S is set
 #pragma unroll
     for (int i = 0; i < (kCountSets ? NN : 1); ++i) { count[i] = 0; }
@@ -238,22 +246,22 @@ __global__ __launch_bounds__(kBlock, 2) void lut_corner_sums_kernel(CornerSumsAr
             uint32_t w[N];
 #pragma unroll
             for (int k = 0; k < N; ++k) { w[k] = w_next[k]; }
-            if (!SHORT) { request_words(base + kPasses * 4 * kWave); }  // (past the row: zeros)
+            if (kLoop) { request_words(base + kPasses * 4 * kWave); }  // (past the row: zeros)
             corner_bytes<N>(w, quad);
-            if (!SHORT) {
+            if (kLoop) {
                 uint32_t elsewhere = 0;                                 // frames at another corner than the lane's first
 #pragma unroll
                 for (int k = 0; k < N; ++k) { elsewhere |= w[k] ^ (uint32_t)((int32_t)(w[k] << 31) >> 31); }
                 skewed |= __popcll(__ballot(__popc(elsewhere) < 16)) >= kWave / 4;
             }
             int const live = f_end - (base + 32 * lane);                // frames of the lane's words that belong to the slab
-            if (live > 0) {
+            if (live > 0 && a.own != nullptr) {
                 uint4 *out = reinterpret_cast<uint4 *>(a.own + (size_t)node * a.own_stride + ((base >> 2) + 8 * lane));
                 out[0] = make_uint4(quad[0], quad[1], quad[2], quad[3]);
                 out[1] = make_uint4(quad[4], quad[5], quad[6], quad[7]);
             }
-            if (!SHORT || lane < kPasses * 8) {                         // (the lanes whose words hold frames of the slab)
-                uint4 *ex = reinterpret_cast<uint4 *>(quads[wv] + 8 * lane);
+            if (kLoop || lane < kPasses * 8) {                         // (the lanes whose words hold frames of the slab)
+                uint4 *ex = reinterpret_cast<uint4 *>(sh.quads + 8 * lane);
                 ex[0] = make_uint4(quad[0], quad[1], quad[2], quad[3]);
                 ex[1] = make_uint4(quad[4], quad[5], quad[6], quad[7]);
             }
@@ -272,7 +280,7 @@ __global__ __launch_bounds__(kBlock, 2) void lut_corner_sums_kernel(CornerSumsAr
         wave_fence();
         uint32_t at[kPasses];
 #pragma unroll
-        for (int i = 0; i < kPasses; ++i) { at[i] = quads[wv][i * kWave + lane]; }
+        for (int i = 0; i < kPasses; ++i) { at[i] = sh.quads[i * kWave + lane]; }
 #pragma unroll
         for (int i = 0; i < kPasses; ++i) {
             int const fb = base + i * 4 * kWave;
@@ -285,12 +293,12 @@ __global__ __launch_bounds__(kBlock, 2) void lut_corner_sums_kernel(CornerSumsAr
                     if (f + 2 >= a.frame_size) { d.z = 0.0f; }
                     if (f + 3 >= a.frame_size) { d.w = 0.0f; }
                 }
-                if constexpr (BN && SHORT) {
+                if constexpr (kCountFrames) {
                     int const f = fb + 4 * lane;
-                    if (f     < f_end) { atomicAdd(&counts[wv][at[i] & 0xffu], 1u); }
-                    if (f + 1 < f_end) { atomicAdd(&counts[wv][(at[i] >> 8) & 0xffu], 1u); }
-                    if (f + 2 < f_end) { atomicAdd(&counts[wv][(at[i] >> 16) & 0xffu], 1u); }
-                    if (f + 3 < f_end) { atomicAdd(&counts[wv][at[i] >> 24], 1u); }
+                    if (f     < f_end) { atomicAdd(&sh.counts[at[i] & 0xffu], 1u); }
+                    if (f + 1 < f_end) { atomicAdd(&sh.counts[(at[i] >> 8) & 0xffu], 1u); }
+                    if (f + 2 < f_end) { atomicAdd(&sh.counts[(at[i] >> 16) & 0xffu], 1u); }
+                    if (f + 3 < f_end) { atomicAdd(&sh.counts[at[i] >> 24], 1u); }
                 }
                 if constexpr (COLS == kWave) { add_quad(at[i], d); }
                 else {
@@ -303,11 +311,11 @@ __global__ __launch_bounds__(kBlock, 2) void lut_corner_sums_kernel(CornerSumsAr
             }
             // (outside of the condition: loads that a path may leave out make the compiler wait for all that are under way)
             __builtin_amdgcn_sched_barrier(0);                          // (into the registers that are free now)
-            if (!SHORT) { dy[i] = load_quad<QUADS>(dyr, (uint32_t)(fb + kPasses * 4 * kWave + 4 * lane) * 4u); }
+            if (kLoop) { dy[i] = load_quad<QUADS>(dyr, (uint32_t)(fb + kPasses * 4 * kWave + 4 * lane) * 4u); }
         }
         wave_fence();
         int const next = base + kPasses * 4 * kWave;
-        if (next >= f_end || next - opened >= (skewed ? kSkewedChain : kFairChain)) {           // (SHORT: one block)
+        if (next >= f_end || next - opened >= (skewed ? kSkewedChain : kFairChain)) {           // (else: one block)
             D += row_sum<NN, COLS>(reinterpret_cast<float4 const *>(mine), lane);
             if (next < f_end) {
                 opened = next;
@@ -320,7 +328,7 @@ __global__ __launch_bounds__(kBlock, 2) void lut_corner_sums_kernel(CornerSumsAr
     }
 
     uint32_t n = 0;
-    if constexpr (BN && SHORT) { n = counts[wv][lane & (NN - 1)]; }
+    if constexpr (kCountFrames) { n = sh.counts[lane & (NN - 1)]; }
     if constexpr (kCountSets) {
         wave_fence();
         uint32_t *const cells = reinterpret_cast<uint32_t *>(mine);
@@ -342,6 +350,19 @@ __global__ __launch_bounds__(kBlock, 2) void lut_corner_sums_kernel(CornerSumsAr
         if (BN) { out[NN] = (float)n; }
     }
     if (a.V_out != nullptr && sl == 0 && lane < NN) { a.V_out[(size_t)node * NN + lane] = v; }
+}
+
+template <int N, bool BN, int FORM, bool QUADS>
+__global__ __launch_bounds__(kBlock, 2) void lut_corner_sums_kernel(CornerSumsArgs a)
+{
+    __shared__ SumsShared<N, BN, FORM> shared[kWavesPerBlk];
+    int const lid = xcd_remap(blockIdx.x, a.slab_count * a.tiles.count);
+    int sl, tile;
+    split_tile(lid, a.tiles, sl, tile);
+    int const wv   = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    int const node = tile * kWavesPerBlk + wv;
+    if (node >= a.node_size) { return; }
+    corner_sums_unit<N, BN, FORM, QUADS>(a, shared[wv], node, sl, threadIdx.x & (kWave - 1));
 }
 
 // Several slabs per node: a workgroup per node adds them up, each wavefront every fourth slab, and folds.
