@@ -1304,6 +1304,64 @@ int vector_op(float *dst, float const *src0, float const *src1, float a, float b
     return 0;
 }
 
+// ---- BinaryLutN ------------------------------------------------------------------------------------
+// row pitch (in words) up to which the rows of a wavefront's four nodes lie within one 32-bit extent
+constexpr int kBinMaxSharedPitch = 0x07ffffff;
+
+template <int N, int NPW, bool EXACT, bool PAD = false>
+void launch_binary_lut_as(BinArgs const &a, hipStream_t st)
+{
+    dim3 const grid(a.chunk_count * a.tiles.count), block(kBlock);
+    if constexpr (N == 6) { launch((binary_lut6_kernel<NPW, EXACT, PAD>), grid, block, 0, st, a); }
+    else                  { launch((binary_lutn_kernel<N, NPW, EXACT, PAD>), grid, block, 0, st, a); }
+}
+
+template <int N, int NPW>
+void launch_binary_lut(BinArgs const &a, bool exact, bool pad, hipStream_t st)
+{
+    if (pad)                    { launch_binary_lut_as<N, NPW, NPW == 1, true>(a, st); }
+    else if (NPW == 1 || exact) { launch_binary_lut_as<N, NPW, true>(a, st); }
+    else                        { launch_binary_lut_as<N, NPW, NPW == 1>(a, st); }
+}
+
+template <int N>
+int run_binary_lut(int const *x, int *y, int const *idx, int const *table, int node_size, int frame_size, int frame_stride, int zero_padding, hipStream_t st)
+{
+    BinArgs a{};
+    a.x = reinterpret_cast<uint32_t const *>(x);
+    a.frame_size = frame_size; a.stride = frame_stride;
+    a.word_count = ceil_div(frame_size, 32);
+    a.chunk = bin_chunk_words();
+    a.chunk_count = ceil_div(a.word_count, a.chunk);
+    // nodes per wavefront: four share a unit's set-up where that still leaves the launch 2048 workgroups
+    int npw = bin_nodes_per_wave();
+    if (npw == 0) {
+        npw = 4;
+        while (npw > 1 && (long long)a.chunk_count * ceil_div(node_size, kWavesPerBlk * npw) < 2048) { npw /= 2; }
+    }
+    if (frame_stride > kBinMaxSharedPitch) { npw = 1; }
+    bool const pad = zero_padding && frame_stride > a.word_count;
+    int const tiles_per_launch = (1 << 23) / a.chunk_count;         // (a launch holds fewer than 2^32 threads)
+    int const nodes_per_launch = (int)std::min<long long>(node_size, (long long)tiles_per_launch * kWavesPerBlk * npw);
+    ScopedTimer tm(kTimeBinary, st);
+    for (int n0 = 0; n0 < node_size; n0 += nodes_per_launch) {
+        a.node_size = std::min(nodes_per_launch, node_size - n0);
+        a.y = reinterpret_cast<uint32_t *>(y) + (size_t)n0 * frame_stride;
+        a.idx = idx + (size_t)n0 * N;
+        a.table = table + (size_t)n0 * (N == 6 ? 2 : 1);
+        a.tiles = make_tile_divisor(ceil_div(a.node_size, kWavesPerBlk * npw));
+        bool const exact = (a.node_size % npw) == 0;
+        switch (npw) {
+        case 1:  launch_binary_lut<N, 1>(a, exact, pad, st); break;
+        case 2:  launch_binary_lut<N, 2>(a, exact, pad, st); break;
+        default: launch_binary_lut<N, 4>(a, exact, pad, st); break;
+        }
+        BBHIP_LAUNCH_CHECK();
+        if (node_size - n0 <= nodes_per_launch) { break; }          // (n0 + nodes_per_launch may pass 2^31)
+    }
+    return 0;
+}
+
 }  // namespace
 
 
@@ -3022,7 +3080,7 @@ int bbhip_bit_fp32_DifferentiableLutN_Backward(int n, int const *dev_x_buf, floa
     return backward_entry(c, stream);
 }
 
-// ---- BinaryLut6 ------------------------------------------------------------------------------------
+// ---- BinaryLutN ------------------------------------------------------------------------------------
 
 int bbhip_bit_BinaryLut6_Forward(int const *dev_x_buf, int *dev_y_buf, int const *dev_input_index, int const *dev_table,
                                  int node_size, int frame_size, int frame_stride, void *stream)
@@ -3032,45 +3090,8 @@ int bbhip_bit_BinaryLut6_Forward(int const *dev_x_buf, int *dev_y_buf, int const
     BBHIP_REQUIRE(dev_x_buf != nullptr && dev_y_buf != nullptr && dev_input_index != nullptr && dev_table != nullptr);
     BBHIP_REQUIRE(node_size > 0 && node_size <= (0x7fffffff >> 6) && frame_size > 0);
     BBHIP_REQUIRE(frame_stride >= (frame_size + 31) / 32);
-    BBHIP_REQUIRE(frame_stride <= 0x07ffffff);          // row pitch in bytes, times the four nodes of a wavefront, stays a 32-bit extent
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    BinArgs a{};
-    a.x = reinterpret_cast<uint32_t const *>(dev_x_buf);
-    a.y = reinterpret_cast<uint32_t *>(dev_y_buf);
-    a.idx = dev_input_index; a.table = dev_table;
-    a.node_size = node_size; a.frame_size = frame_size; a.stride = frame_stride;
-    a.word_count = (frame_size + 31) / 32;
-    a.chunk = bin_chunk_words();
-    a.chunk_count = ceil_div(a.word_count, a.chunk);
-    // nodes per wavefront: four share a unit's set-up where that still leaves the launch 2048 workgroups
-    int npw = bin_nodes_per_wave();
-    if (npw == 0) {
-        npw = 4;
-        while (npw > 1 && (long long)a.chunk_count * ceil_div(node_size, kWavesPerBlk * npw) < 2048) { npw /= 2; }
-    }
-    a.tiles = make_tile_divisor(ceil_div(node_size, kWavesPerBlk * npw));
-    BBHIP_REQUIRE((long long)a.chunk_count * a.tiles.count <= 0x7fffffffLL);
-    {
-        ScopedTimer tm(kTimeBinary, st);
-        dim3 const grid(a.chunk_count * a.tiles.count), block(kBlock);
-        bool const exact = (node_size % npw) == 0;
-        bool const pad = zero_padding && frame_stride > a.word_count;
-        switch (npw) {
-        case 1: if (pad) { launch((binary_lut6_kernel<1, true, true>), grid, block, 0, st, a); }
-                else     { launch((binary_lut6_kernel<1, true>), grid, block, 0, st, a); }
-                break;
-        case 2: if (pad)        { launch((binary_lut6_kernel<2, false, true>), grid, block, 0, st, a); }
-                else if (exact) { launch((binary_lut6_kernel<2, true>), grid, block, 0, st, a); }
-                else       { launch((binary_lut6_kernel<2, false>), grid, block, 0, st, a); }
-                break;
-        default: if (pad)       { launch((binary_lut6_kernel<4, false, true>), grid, block, 0, st, a); }
-                 else if (exact) { launch((binary_lut6_kernel<4, true>), grid, block, 0, st, a); }
-                 else       { launch((binary_lut6_kernel<4, false>), grid, block, 0, st, a); }
-                 break;
-        }
-    }
-    BBHIP_LAUNCH_CHECK();
-    return 0;
+    BBHIP_REQUIRE(frame_stride <= kBinMaxSharedPitch);
+    return run_binary_lut<6>(dev_x_buf, dev_y_buf, dev_input_index, dev_table, node_size, frame_size, frame_stride, zero_padding, static_cast<hipStream_t>(stream));
 }
 
 int bbhip_bit_BinaryLutN_Forward(int n, int const *dev_x_buf, int *dev_y_buf, int const *dev_input_index, int const *dev_table,
@@ -3083,22 +3104,13 @@ int bbhip_bit_BinaryLutN_Forward(int n, int const *dev_x_buf, int *dev_y_buf, in
     BBHIP_REQUIRE(dev_x_buf != nullptr && dev_y_buf != nullptr && dev_input_index != nullptr && dev_table != nullptr);
     BBHIP_REQUIRE(node_size > 0 && node_size <= (0x7fffffff >> 6) && frame_size > 0);
     BBHIP_REQUIRE(frame_stride >= (frame_size + 31) / 32);
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    uint32_t const *x = reinterpret_cast<uint32_t const *>(dev_x_buf);
-    uint32_t *y = reinterpret_cast<uint32_t *>(dev_y_buf);
-    int const words = zero_padding ? frame_stride : (frame_size + 31) / 32;
-    ScopedTimer tm(kTimeBinary, st);
-    for (int n0 = 0; n0 < node_size; n0 += 65535) {            // grid.y is limited to 65535 nodes per launch
-        dim3 const grid(ceil_div(words, kBlock), (node_size - n0 < 65535) ? node_size - n0 : 65535), block(kBlock);
-        switch (n) {
-        case 2: launch(binary_lutn_kernel<2>, grid, block, 0, st, x, y, dev_input_index, dev_table, n0, frame_size, frame_stride); break;
-        case 3: launch(binary_lutn_kernel<3>, grid, block, 0, st, x, y, dev_input_index, dev_table, n0, frame_size, frame_stride); break;
-        case 4: launch(binary_lutn_kernel<4>, grid, block, 0, st, x, y, dev_input_index, dev_table, n0, frame_size, frame_stride); break;
-        default: launch(binary_lutn_kernel<5>, grid, block, 0, st, x, y, dev_input_index, dev_table, n0, frame_size, frame_stride); break;
-        }
-        BBHIP_LAUNCH_CHECK();
+    hipStream_t const st = static_cast<hipStream_t>(stream);
+    switch (n) {
+    case 2:  return run_binary_lut<2>(dev_x_buf, dev_y_buf, dev_input_index, dev_table, node_size, frame_size, frame_stride, zero_padding, st);
+    case 3:  return run_binary_lut<3>(dev_x_buf, dev_y_buf, dev_input_index, dev_table, node_size, frame_size, frame_stride, zero_padding, st);
+    case 4:  return run_binary_lut<4>(dev_x_buf, dev_y_buf, dev_input_index, dev_table, node_size, frame_size, frame_stride, zero_padding, st);
+    default: return run_binary_lut<5>(dev_x_buf, dev_y_buf, dev_input_index, dev_table, node_size, frame_size, frame_stride, zero_padding, st);
     }
-    return 0;
 }
 
 }  // extern "C"

@@ -1603,15 +1603,18 @@ __global__ __launch_bounds__(kBlock) void conv_bit_to_real_kernel(uint32_t const
 }
 
 // ------------------------------------------------------------------------------------------------
-//  BinaryLut6: y = table[x5 x4 x3 x2 x1 x0] on 32 frames per word
-//  (reference semantics: include/bb/BinaryLutN.h:436-463 — input k is index bit k, entries 0-31 in table word 0).
-//  Evaluated as a 6-level multiplexer tree whose first two levels are replaced by a register lookup: they turn each
-//  group of four table entries into one of the 16 Boolean functions of (x0, x1), and which one is the group's table
+//  BinaryLutN, N = 2 .. 6: y = table[x(N-1) .. x1 x0] on 32 frames per word
+//  (reference semantics: include/bb/BinaryLutN.h:436-463 — input k is index bit k, entries 0-31 in table word 0; the reference
+//  has a device kernel for N = 6 only).
+//  N = 4 .. 6: a multiplexer tree whose first two levels are replaced by a register lookup: they turn each
+//  group of four table entries into one of the 16 Boolean functions of (x0, x1); which one is the group's table
 //  nibble, the same for every frame.  Per word the kernel forms all 16 functions once (12 three-input bit operations),
 //  picks the group values out of that register array with the nibbles as wave-uniform register indices while
-//  multiplexing by x2 (16 instructions), and finishes with the last three levels (7 bit-selects): 35 vector
-//  instructions per word where the plain tree takes 63; the table is held as eight scalar registers per node, one 16-bit
-//  index field per nibble.
+//  multiplexing by x2 (two instructions per pair of groups), and finishes with the last N - 3 levels: 35 vector
+//  instructions per word for N = 6 (the plain tree takes 63), 23 for N = 5, 17 for N = 4; the table is held as scalar
+//  registers, one 16-bit index field per nibble.
+//  N = 2, 3: the polynomial over GF(2), y = XOR of c[S] AND of the inputs in S, with the coefficients as scalar masks (one
+//  scalar operand per instruction): 5 and 10 vector instructions.
 // ------------------------------------------------------------------------------------------------
 // bit-select d = (s & hi) | (~s & lo): one instruction per multiplexer of the tree
 __device__ __forceinline__ uint32_t bfi_vvv(uint32_t s, uint32_t hi, uint32_t lo)
@@ -1685,8 +1688,7 @@ __device__ __forceinline__ void bin_select_level2(bin_u32x16 const &fn, uint32_t
         "s_lshr_b32 m0, %[w7], 16\n\t"
         "v_bitop3_b32 %[t7], v48, %[x2], %[tmp] bitop3:0xe2\n\t"
         "s_set_gpr_idx_off"
-        : [t0] "=&v"(t[0]), [t1] "=&v"(t[1]), [t2] "=&v"(t[2]), [t3] "=&v"(t[3]),
-          [t4] "=&v"(t[4]), [t5] "=&v"(t[5]), [t6] "=&v"(t[6]), [t7] "=&v"(t[7]), [tmp] "=&v"(tmp)
+        : [t0] "=&v"(t[0]), [t1] "=&v"(t[1]), [t2] "=&v"(t[2]), [t3] "=&v"(t[3]), [t4] "=&v"(t[4]), [t5] "=&v"(t[5]), [t6] "=&v"(t[6]), [t7] "=&v"(t[7]), [tmp] "=&v"(tmp)
         : [w0] "s"(iw[0]), [w1] "s"(iw[1]), [w2] "s"(iw[2]), [w3] "s"(iw[3]), [w4] "s"(iw[4]), [w5] "s"(iw[5]), [w6] "s"(iw[6]), [w7] "s"(iw[7]),
           [x2] "v"(x2),
           "{v48}"(fn[0]), "{v49}"(fn[1]), "{v50}"(fn[2]), "{v51}"(fn[3]), "{v52}"(fn[4]), "{v53}"(fn[5]), "{v54}"(fn[6]), "{v55}"(fn[7]),
@@ -1694,23 +1696,138 @@ __device__ __forceinline__ void bin_select_level2(bin_u32x16 const &fn, uint32_t
         : "scc");                // (M0 is written too: it is reserved, the compiler keeps nothing there across statements)
 }
 
-// The index words of a node's table for bin_select_level2: word j holds 0x1000 | nibble 2j in its low half and
-// 0x1000 | nibble 2j+1 in its high half (nibble k = table entries 4k .. 4k+3).  Lane j < 8 forms word j with a few vector
-// instructions and the eight words are read back into scalar registers: the vector unit has the room, the scalar unit
-// does not.
-__device__ __forceinline__ void bin_index_words(uint32_t table_lo, uint32_t table_hi, int lane, uint32_t (&iw)[8])
+__device__ __forceinline__ void bin_select_level2(bin_u32x16 const &fn, uint32_t const (&iw)[4], uint32_t x2, uint32_t (&t)[4])
 {
-    uint32_t const w    = (lane & 4) ? table_hi : table_lo;
+    uint32_t tmp;
+    asm volatile(
+        "s_set_gpr_idx_on %[w0], gpr_idx(SRC0)\n\t"
+        "v_mov_b32 %[tmp], v48\n\t"
+        "s_lshr_b32 m0, %[w0], 16\n\t"
+        "v_bitop3_b32 %[t0], v48, %[x2], %[tmp] bitop3:0xe2\n\t"
+        "s_and_b32 m0, %[w1], 0xffff\n\t"
+        "v_mov_b32 %[tmp], v48\n\t"
+        "s_lshr_b32 m0, %[w1], 16\n\t"
+        "v_bitop3_b32 %[t1], v48, %[x2], %[tmp] bitop3:0xe2\n\t"
+        "s_and_b32 m0, %[w2], 0xffff\n\t"
+        "v_mov_b32 %[tmp], v48\n\t"
+        "s_lshr_b32 m0, %[w2], 16\n\t"
+        "v_bitop3_b32 %[t2], v48, %[x2], %[tmp] bitop3:0xe2\n\t"
+        "s_and_b32 m0, %[w3], 0xffff\n\t"
+        "v_mov_b32 %[tmp], v48\n\t"
+        "s_lshr_b32 m0, %[w3], 16\n\t"
+        "v_bitop3_b32 %[t3], v48, %[x2], %[tmp] bitop3:0xe2\n\t"
+        "s_set_gpr_idx_off"
+        : [t0] "=&v"(t[0]), [t1] "=&v"(t[1]), [t2] "=&v"(t[2]), [t3] "=&v"(t[3]), [tmp] "=&v"(tmp)
+        : [w0] "s"(iw[0]), [w1] "s"(iw[1]), [w2] "s"(iw[2]), [w3] "s"(iw[3]),
+          [x2] "v"(x2),
+          "{v48}"(fn[0]), "{v49}"(fn[1]), "{v50}"(fn[2]), "{v51}"(fn[3]), "{v52}"(fn[4]), "{v53}"(fn[5]), "{v54}"(fn[6]), "{v55}"(fn[7]),
+          "{v56}"(fn[8]), "{v57}"(fn[9]), "{v58}"(fn[10]), "{v59}"(fn[11]), "{v60}"(fn[12]), "{v61}"(fn[13]), "{v62}"(fn[14]), "{v63}"(fn[15])
+        : "scc");
+}
+
+__device__ __forceinline__ void bin_select_level2(bin_u32x16 const &fn, uint32_t const (&iw)[2], uint32_t x2, uint32_t (&t)[2])
+{
+    uint32_t tmp;
+    asm volatile(
+        "s_set_gpr_idx_on %[w0], gpr_idx(SRC0)\n\t"
+        "v_mov_b32 %[tmp], v48\n\t"
+        "s_lshr_b32 m0, %[w0], 16\n\t"
+        "v_bitop3_b32 %[t0], v48, %[x2], %[tmp] bitop3:0xe2\n\t"
+        "s_and_b32 m0, %[w1], 0xffff\n\t"
+        "v_mov_b32 %[tmp], v48\n\t"
+        "s_lshr_b32 m0, %[w1], 16\n\t"
+        "v_bitop3_b32 %[t1], v48, %[x2], %[tmp] bitop3:0xe2\n\t"
+        "s_set_gpr_idx_off"
+        : [t0] "=&v"(t[0]), [t1] "=&v"(t[1]), [tmp] "=&v"(tmp)
+        : [w0] "s"(iw[0]), [w1] "s"(iw[1]),
+          [x2] "v"(x2),
+          "{v48}"(fn[0]), "{v49}"(fn[1]), "{v50}"(fn[2]), "{v51}"(fn[3]), "{v52}"(fn[4]), "{v53}"(fn[5]), "{v54}"(fn[6]), "{v55}"(fn[7]),
+          "{v56}"(fn[8]), "{v57}"(fn[9]), "{v58}"(fn[10]), "{v59}"(fn[11]), "{v60}"(fn[12]), "{v61}"(fn[13]), "{v62}"(fn[14]), "{v63}"(fn[15])
+        : "scc");
+}
+
+// The index words of a node's table for bin_select_level2: word j holds 0x1000 | nibble 2j in its low half and
+// 0x1000 | nibble 2j+1 in its high half (nibble k = table entries 4k .. 4k+3).  Lane j forms word j with a few vector
+// instructions and the words are read back into scalar registers: the vector unit has the room, the scalar unit
+// does not.
+template <int WORDS>
+__device__ __forceinline__ void bin_index_words(uint32_t table_lo, uint32_t table_hi, int lane, uint32_t (&iw)[WORDS])
+{
+    uint32_t const w    = (WORDS > 4 && (lane & 4)) ? table_hi : table_lo;
     uint32_t const byte = (w >> ((lane & 3) * 8)) & 0xffu;
     uint32_t const v    = 0x10001000u | (byte & 15u) | ((byte >> 4) << 16);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) { iw[j] = (uint32_t)__builtin_amdgcn_readlane((int)v, j); }
+    for (int j = 0; j < WORDS; ++j) { iw[j] = (uint32_t)__builtin_amdgcn_readlane((int)v, j); }
 }
 
+// A node's table in scalar registers and its value for a word of 32 frames.
+template <int N, bool LOOKUP = (N >= 4)>
+struct BinTable {
+    static constexpr int kPairs = 1 << (N - 3);         // pairs of nibbles
+    uint32_t iw[kPairs];
+    __device__ __forceinline__ void load(uint32_t lo, uint32_t hi, int lane) { bin_index_words(lo, hi, lane, iw); }
+    __device__ __forceinline__ uint32_t value(uint32_t const (&x)[N]) const
+    {
+        uint32_t const x0 = x[0], x1 = x[1], nx1 = ~x1;
+        bin_u32x16 fn;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            // table position q = x0 + 2 * x1: bit q of c is the function's value there
+            uint32_t const g0 = bin_pick(c & 1, (c >> 2) & 1, x1, nx1);          // x0 = 0
+            uint32_t const g1 = bin_pick((c >> 1) & 1, (c >> 3) & 1, x1, nx1);   // x0 = 1
+            fn[c] = (x0 & g1) | (~x0 & g0);
+        }
+        uint32_t t[kPairs];
+        bin_select_level2(fn, iw, x[2], t);
+        // the next node's functions are formed after this point, straight into the fixed registers that are free
+        // again now (formed earlier, they would have to be moved there: fifteen moves per node)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int lv = 3; lv < N; ++lv) {
+#pragma unroll
+            for (int k = 0; k < ((1 << (N - 1)) >> lv); ++k) { t[k] = bfi_vvv(x[lv], t[2 * k + 1], t[2 * k]); }
+        }
+        return t[0];
+    }
+};
+
+template <int N>
+struct BinTable<N, false> {
+    static_assert(N == 2 || N == 3, "coefficients as masks pay for small tables only");
+    int c[1 << N];
+    __device__ __forceinline__ void load(uint32_t t, uint32_t, int)
+    {
+        t ^= (t & 0x55u) << 1;
+        t ^= (t & 0x33u) << 2;
+        if (N == 3) { t ^= (t & 0x0fu) << 4; }
+#pragma unroll
+        for (int i = 0; i < (1 << N); ++i) { c[i] = (int)(t << (31 - i)) >> 31; }
+    }
+    __device__ __forceinline__ uint32_t value(uint32_t const (&x)[N]) const
+    {
+        uint32_t const both = x[0] & x[1];
+        uint32_t v = 0u;
+#pragma unroll
+        for (int h = (1 << N) - 4; h >= 0; h -= 4) {
+            uint32_t low = (uint32_t)c[h + 3] & both;
+            low ^= (uint32_t)c[h + 2] & x[1];
+            low ^= (uint32_t)c[h + 1] & x[0];
+            low ^= (uint32_t)c[h];
+            v = (h == (1 << N) - 4) ? low : ((v & x[N - 1]) ^ low);
+        }
+        return v;
+    }
+};
+
+// Units of 128 words and four nodes per wavefront at every N: a wavefront sets up once and has 4 N rows' loads in flight, and the nodes of an XCD
+// read one window of the input rows at a time from its L2.  Measured against a thread per (node, word) in row order, whose rows came
+// from behind the L2 each time: 8192 x 16384 x 262144 at N = 2 / 3 / 4 / 5 212 / 244 / 248 / 267 us instead of 408 / 427 / 455 / 491
+// (64 words 228 / 273 / 261 / 291, two nodes 259 / 265 / 278 / 288), 1000 x 3000 x 100000 11.4 / 13.7 / 14.2 / 16.3 instead of 23 / 25 / 28 / 30.
+// What bounds it there is the output: its 537 MB alone, without a gather, take 165 us.
 // nodes per wavefront; EXACT: the node count is a multiple of NPW, no wavefront has nodes to skip; PAD: the wavefronts of a row's last unit write 0
 // behind the last frame's word, up to the row pitch (a branch at the kernel's end costs the large shape 1 %, hence a variant of its own)
-template <int NPW, bool EXACT, bool PAD = false>
-__global__ __launch_bounds__(kBlock) void binary_lut6_kernel(BinArgs a)
+template <int N, int NPW, bool EXACT, bool PAD>
+__device__ __forceinline__ void binary_lut_unit(BinArgs const &a)
 {
     int const B    = a.chunk_count * a.tiles.count;
     int const lid  = xcd_remap(blockIdx.x, B);
@@ -1725,27 +1842,30 @@ __global__ __launch_bounds__(kBlock) void binary_lut6_kernel(BinArgs a)
     // wiring and tables are read through the constant address space: wave-uniform scalar loads wherever the compiler
     // places them relative to the stores of this kernel (neither is written here)
     typedef __attribute__((address_space(4))) int const const_int;
-    const_int *idxc = (const_int *)a.idx + (size_t)node0 * 6;
-    const_int *tabc = (const_int *)a.table + (size_t)node0 * 2;
-    uint32_t iw[NPW][8];                    // the node's table as index words (bin_index_words)
-    char const *rows[NPW][6];               // wave-uniform row bases: loads take a scalar base and a 32-bit lane offset
+    constexpr int kTableWords = (N == 6) ? 2 : 1;
+    const_int *idxc = (const_int *)a.idx + (size_t)node0 * N;
+    const_int *tabc = (const_int *)a.table + (size_t)node0 * kTableWords;
+    BinTable<N> table[NPW];
+    char const *rows[NPW][N];               // wave-uniform row bases: loads take a scalar base and a 32-bit lane offset
     bool live[NPW];
 #pragma unroll
     for (int p = 0; p < NPW; ++p) {
         live[p] = EXACT || (node0 + p < a.node_size);
         int const rel = live[p] ? p : 0;                    // a wavefront past the last node repeats its first one and stores nothing
-        bin_index_words((uint32_t)tabc[rel * 2], (uint32_t)tabc[rel * 2 + 1], lane, iw[p]);
+        table[p].load((uint32_t)tabc[rel * kTableWords], (N == 6) ? (uint32_t)tabc[rel * kTableWords + 1] : 0u, lane);
 #pragma unroll
-        for (int k = 0; k < 6; ++k) {
+        for (int k = 0; k < N; ++k) {
             // unsigned 32 x 32 -> 64 bit: two scalar multiplies and an add with carry per row (the wiring is validated
-            // as non-negative by whoever builds it; a signed 64-bit product costs the scalar unit three times as much)
-            rows[p][k] = reinterpret_cast<char const *>(a.x) + (uint64_t)(uint32_t)idxc[rel * 6 + k] * (uint64_t)stride_bytes;
+            // as non-negative by whoever builds it; a signed 64-bit product costs the scalar unit three times as much).
+            // Only N = 6 bounds the pitch so that it fits 32 bits in bytes.
+            uint64_t const in = (uint32_t)idxc[rel * N + k];
+            rows[p][k] = reinterpret_cast<char const *>(a.x) + (N == 6 ? in * stride_bytes : (in * (uint32_t)a.stride) << 2);
         }
     }
     // Outputs of the wavefront's nodes go through one buffer descriptor over their NPW rows, the node's row added as the
     // scalar offset of the store (the range check covers that offset too, so the extent cannot end with a row: lanes
     // beyond the end of a row are masked in the one step of a row that has them).
-    __amdgpu_buffer_rsrc_t const yr = row_descriptor(a.y, node0, a.stride, (uint32_t)NPW * stride_bytes);
+    __amdgpu_buffer_rsrc_t const yr = row_descriptor(a.y, node0, a.stride, (uint32_t)(NPW - 1) * stride_bytes + row_bytes);
 
     int const w_begin = ck * a.chunk;
     int const w_end   = min(w_begin + a.chunk, a.word_count);
@@ -1755,36 +1875,17 @@ __global__ __launch_bounds__(kBlock) void binary_lut6_kernel(BinArgs a)
     uint32_t const last_off = (uint32_t)w_last * 4u;        // lanes beyond the row re-read its last word and store nothing
     uint32_t off = (uint32_t)(w_begin + lane) * 4u;
     for (int w0 = w_begin; w0 < w_end; w0 += kWave, off += kWave * 4u) {
-        uint32_t xv[NPW][6];
+        uint32_t xv[NPW][N];
         uint32_t const at = min(off, last_off);
 #pragma unroll
         for (int p = 0; p < NPW; ++p) {
 #pragma unroll
-            for (int k = 0; k < 6; ++k) { xv[p][k] = *reinterpret_cast<uint32_t const *>(rows[p][k] + at); }
+            for (int k = 0; k < N; ++k) { xv[p][k] = *reinterpret_cast<uint32_t const *>(rows[p][k] + at); }
         }
         bool const has_tail = (w0 + kWave > w_last);            // wave-uniform: only the last step of a row
 #pragma unroll
         for (int p = 0; p < NPW; ++p) {
-            uint32_t const x0 = xv[p][0], x1 = xv[p][1], nx1 = ~x1;
-            bin_u32x16 fn;
-#pragma unroll
-            for (int c = 0; c < 16; ++c) {
-                // table position q = x0 + 2 * x1: bit q of c is the function's value there
-                uint32_t const g0 = bin_pick(c & 1, (c >> 2) & 1, x1, nx1);          // x0 = 0
-                uint32_t const g1 = bin_pick((c >> 1) & 1, (c >> 3) & 1, x1, nx1);   // x0 = 1
-                fn[c] = (x0 & g1) | (~x0 & g0);
-            }
-            uint32_t t[8];
-            bin_select_level2(fn, iw[p], xv[p][2], t);
-            // the next node's functions are formed after this point, straight into the fixed registers that are free
-            // again now (formed earlier, they would have to be moved there: fifteen moves per node)
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int lv = 3; lv < 6; ++lv) {
-#pragma unroll
-                for (int k = 0; k < (32 >> lv); ++k) { t[k] = bfi_vvv(xv[p][lv], t[2 * k + 1], t[2 * k]); }
-            }
-            uint32_t r = t[0];
+            uint32_t r = table[p].value(xv[p]);
             // streamed once (non-temporal): keep it from displacing x rows in L2
             if (live[p]) {
                 if (!has_tail) { __builtin_amdgcn_raw_buffer_store_b32(r, yr, off, (uint32_t)p * stride_bytes, 2); }
@@ -1803,40 +1904,10 @@ __global__ __launch_bounds__(kBlock) void binary_lut6_kernel(BinArgs a)
     }
 }
 
-// ------------------------------------------------------------------------------------------------
-//  BinaryLutN for N = 2 .. 5 (reference: the generic loop of BinaryLutN<N>::Forward, include/bb/BinaryLutN.h:436-463; the
-//  reference has a device kernel for N = 6 only).  A table of 2^N <= 32 entries is one word per node.  One thread per (node, word of
-//  32 frames): the N input words are the select lines of a multiplexer tree over the table's entries, each entry spread to a word of
-//  all ones or all zeros — 2^N - 1 bit-selects per word, whose first level folds into constants.  The node (blockIdx.y), its wiring
-//  and its table are the same for the whole workgroup: scalar loads.  Bits of the last word beyond frame_size are written as 0.
-// ------------------------------------------------------------------------------------------------
-template <int N>
-__global__ __launch_bounds__(kBlock) void binary_lutn_kernel(uint32_t const *__restrict__ x, uint32_t *__restrict__ y, int const *__restrict__ idx,
-                                                            int const *__restrict__ table, int node0, int frame_size, int stride)
-{
-    static_assert(N >= 2 && N <= 5, "one table word per node");
-    int const node = node0 + (int)blockIdx.y;
-    int const w = blockIdx.x * kBlock + threadIdx.x;
-    int const words = (frame_size + 31) >> 5;
-    if (w >= words) {                               // (launched where the caller wants the row's padding zeroed)
-        if (w < stride) { y[(size_t)node * stride + w] = 0u; }
-        return;
-    }
-    uint32_t const t = (uint32_t)table[node];
-    uint32_t sel[N];
-#pragma unroll
-    for (int k = 0; k < N; ++k) { sel[k] = x[(size_t)idx[node * N + k] * stride + w]; }
-    uint32_t v[1 << N];
-#pragma unroll
-    for (int i = 0; i < (1 << N); ++i) { v[i] = ((t >> i) & 1u) ? 0xffffffffu : 0u; }
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-#pragma unroll
-        for (int i = 0; i < (1 << (N - 1 - k)); ++i) { v[i] = (sel[k] & v[2 * i + 1]) | (~sel[k] & v[2 * i]); }
-    }
-    uint32_t out = v[0];
-    if (w == words - 1 && (frame_size & 31)) { out &= (1u << (frame_size & 31)) - 1u; }
-    y[(size_t)node * stride + w] = out;
-}
+template <int NPW, bool EXACT, bool PAD = false>
+__global__ __launch_bounds__(kBlock) void binary_lut6_kernel(BinArgs a) { binary_lut_unit<6, NPW, EXACT, PAD>(a); }
+
+template <int N, int NPW, bool EXACT, bool PAD = false>
+__global__ __launch_bounds__(kBlock) void binary_lutn_kernel(BinArgs a) { binary_lut_unit<N, NPW, EXACT, PAD>(a); }
 
 }  // namespace bbhip

@@ -37,6 +37,33 @@ def test_bit_exact(ops, n, shape):
     assert np.array_equal(host(y), oracle.binary_lutn_forward(n, xb, idx, T, F))        # padding bits and words are zero on both sides
 
 
+@pytest.mark.parametrize("n", [2, 3, 4, 5])
+@pytest.mark.parametrize("nodes", [85, 175, 176])
+def test_several_nodes_per_wavefront(ops, n, nodes):
+    """201 units of 128 words: enough workgroups for two (85) and four (175, 176) nodes per wavefront, the last ones with nodes to skip or none"""
+    I, F = 37, 200 * 4096 + 33
+    rng = np.random.default_rng(nodes + n)
+    idx = synth.wiring(rng, I, nodes, n); T = tables(rng, nodes, n)
+    xb = synth.bernoulli_bits(rng, I, F, synth.frame_stride_bit(F))
+    y = ops.binary_lutn_forward(n, dev(xb), dev(idx), dev(T), F)
+    assert np.array_equal(host(y), oracle.binary_lutn_forward(n, xb, idx, T, F))
+
+
+@pytest.mark.parametrize("n", [2, 5])
+def test_rows_too_far_apart_for_one_extent(ops, n):
+    """a pitch of 2^27 words and more takes one node per wavefront, with 64-bit row offsets"""
+    import torch
+    I, O, F, pitch = 6, 5, 5000, (1 << 27) + 64
+    rng = np.random.default_rng(n)
+    idx = dev(synth.wiring(rng, I, O, n)); T = dev(tables(rng, O, n))
+    xb = dev(synth.bernoulli_bits(rng, I, F, synth.frame_stride_bit(F)))
+    far = torch.zeros((I, pitch), dtype=torch.int32, device="cuda")
+    far[:, :xb.shape[1]] = xb
+    words = (F + 31) // 32
+    y = ops.binary_lutn_forward(n, far, idx, T, F)
+    assert torch.equal(y[:, :words], ops.binary_lutn_forward(n, xb, idx, T, F)[:, :words])
+
+
 def test_reference_vectors_on_gpu(ops):
     for k in range(int(GOLD["count"][0])):
         p = "c%d_" % k
