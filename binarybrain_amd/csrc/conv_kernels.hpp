@@ -52,24 +52,28 @@ __device__ __forceinline__ bool im2col_source(Im2ColArgs const &a, int oy, int o
     return im2col_border(a.border_mode, ix, iy, a.w, a.h);
 }
 
-// block = (output node, 64 window positions of the flattened (oy, ox) plane, 64 input frames): rows of the input are read
-// along the frames, the tile is written along the window positions, which are contiguous in the output
+// block = (output node, QT window positions of the flattened (oy, ox) plane, 64 input frames): rows of the input are read
+// along the frames, the tile is written along the window positions, which are contiguous in the output.  The pieces of an output row do not
+// start on cache lines, so neighbouring pieces go to neighbouring workgroups of one XCD, whose L2 puts the lines together (27 nodes x 900 positions x
+// 256 frames 13.2 -> 12.4 us; the two directions of col2im_kernel 15.1 -> 14.6 and 13.1 -> 11.7).  A launch of one round is a chain of latencies (loads,
+// barrier, stores): shorter tiles where there are compute units to spare (9 nodes x 676 positions x 50 frames 6.0 -> 4.1 us with QT = 16).
+template <int QT>
 __global__ __launch_bounds__(kConvBlock) void im2col_forward_kernel(Im2ColArgs a)
 {
-    __shared__ float tile[kTile][kTile + 1];                 // [window position][frame]
-    int b = blockIdx.x;
-    int const ft = b % a.f_tiles;  b /= a.f_tiles;
+    __shared__ float tile[QT][kTile + 1];                    // [window position][frame]
+    int b = xcd_remap(blockIdx.x, gridDim.x);
     int const qt = b % a.q_tiles;  b /= a.q_tiles;
+    int const ft = b % a.f_tiles;  b /= a.f_tiles;
     int const node = b;                                      // (c*fh + fy)*fw + fx
     int const fx = node % a.fw, fy = (node / a.fw) % a.fh, c = node / (a.fw * a.fh);
     int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int const f0 = ft * kTile, q0 = qt * kTile;
+    int const f0 = ft * kTile, q0 = qt * QT;
     int const plane = a.oh * a.ow;
     float const *x = static_cast<float const *>(a.x);
     float *y = static_cast<float *>(a.y);
 
-    // all loads of a wavefront's 16 rows are issued before the first of them is used (one round trip instead of sixteen)
-    constexpr int kRows = kTile / (kConvBlock / 64);
+    // all loads of a wavefront's rows are issued before the first of them is used (one round trip instead of one per row)
+    constexpr int kRows = QT / (kConvBlock / 64);
     float v[kRows];
     int oy = (q0 + wave) / a.ow, ox = (q0 + wave) - oy * a.ow;      // of the wavefront's first row; the next rows step on from it
 #pragma unroll
@@ -91,11 +95,13 @@ __global__ __launch_bounds__(kConvBlock) void im2col_forward_kernel(Im2ColArgs a
 #pragma unroll
     for (int r = 0; r < kRows; ++r) { tile[wave + r * (kConvBlock / 64)][lane] = v[r]; }
     __syncthreads();
+    constexpr int kFrames = kConvBlock / QT;                 // frames per pass
+    int const q = threadIdx.x % QT;
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) {
-        int const f = wave + r * (kConvBlock / 64);
-        if (f0 + f < a.input_frame_size && q0 + lane < plane) {
-            y[(size_t)node * a.output_frame_stride + (size_t)(f0 + f) * plane + q0 + lane] = tile[lane][f];
+    for (int r = 0; r < kTile / kFrames; ++r) {
+        int const f = threadIdx.x / QT + r * kFrames;
+        if (f0 + f < a.input_frame_size && q0 + q < plane) {
+            y[(size_t)node * a.output_frame_stride + (size_t)(f0 + f) * plane + q0 + q] = tile[q][f];
         }
     }
 }
@@ -130,14 +136,14 @@ __global__ __launch_bounds__(kConvBlock) void im2col_forward_bit_kernel(Im2ColAr
 // (include/bb/ConvolutionIm2Col.h:411-452: border replicas carry no gradient).  block = (c, 64 pixels of the flattened
 // image, 64 frames): one lane per pixel forms the sums (pixels of one image row are contiguous along ox in dy), which are
 // then transposed through LDS so that the stores run along the frames.  Flattening keeps the lanes busy for images
-// narrower than a wavefront; TF (frames per block) is 64, or 16 when the batch is too small to fill the device otherwise.
+// narrower than a wavefront; TF (frames per block) is 64, or 16 or 4 when the batch is too small to fill the device otherwise.
 template <int TF>
 __global__ __launch_bounds__(kConvBlock) void im2col_backward_kernel(Im2ColArgs a, int p_tiles)
 {
     __shared__ float tile[kTile][TF + 1];                    // [pixel][frame]
-    int b = blockIdx.x;
-    int const ft = b % a.f_tiles; b /= a.f_tiles;
+    int b = xcd_remap(blockIdx.x, gridDim.x);                // (neighbouring pixels read the same cache lines of dy: one L2)
     int const pt = b % p_tiles;   b /= p_tiles;
+    int const ft = b % a.f_tiles; b /= a.f_tiles;
     int const c  = b;
     int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int const f0 = ft * TF, p0 = pt * kTile;
@@ -221,9 +227,9 @@ __global__ __launch_bounds__(kConvBlock) void col2im_kernel(float const *__restr
                                                            int narrow_stride, int frames, int wide_stride, int xy_tiles, int f_tiles)
 {
     __shared__ float tile[kTile][kTile + 1];
-    int b = blockIdx.x;
-    int const ft = b % f_tiles;  b /= f_tiles;
+    int b = xcd_remap(blockIdx.x, gridDim.x);               // (neighbouring pieces of a row of the narrow side, which are not whole cache lines, in one L2)
     int const xt = b % xy_tiles; b /= xy_tiles;
+    int const ft = b % f_tiles;  b /= f_tiles;
     int const c = b;
     int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int const f0 = ft * kTile, xy0 = xt * kTile;
@@ -289,17 +295,33 @@ struct PoolArgs {
     float const *dy;
     float       *out;       // y (forward) or dx (backward)
     int w, h, ow, oh, c, frame_size, frame_stride;
+    TileDivisor lanes;      // threads of a row: one per W frames, up to kConvBlock
+    int rows;               // output nodes per workgroup
+    int f_blocks;           // workgroups per row
 };
+
+// The thread's output node and first frame; false: none.  Rows shorter than a workgroup's threads share one: 4056 nodes x 50 frames are 214 workgroups
+// instead of 4056 of which 13 threads work (forward 5.0 -> 3.1 us, backward 7.2 -> 4.6; 8100 nodes x 256 frames, 64 threads a row, backward
+// 14.8 -> 12.3).
+template <int W>
+__device__ __forceinline__ bool pool_place(PoolArgs const &a, int &node, int &f)
+{
+    int row, lane;
+    split_tile((int)threadIdx.x, a.lanes, row, lane);
+    int const group = (int)blockIdx.x / a.f_blocks;
+    node = group * a.rows + row;
+    f = ((int)(blockIdx.x - group * a.f_blocks) * kConvBlock + lane) * W;
+    return row < a.rows && node < a.c * a.oh * a.ow && f < a.frame_size;
+}
 
 // y = 1 - prod over the window taps inside the image, (fy, fx) ascending, of (1 - x): the probability that at least one
 // of four independent binary inputs is 1 (include/bb/StochasticMaxPooling2x2.h:190-218).  One thread per (output node,
 // W frames), W = 4 with 128-bit accesses where rows are 16-byte aligned; the four taps are loaded before the first is used.
 template <int W>
-__global__ __launch_bounds__(kConvBlock) void stochastic_maxpool2x2_forward_kernel(PoolArgs a, int f_blocks)
+__global__ __launch_bounds__(kConvBlock) void stochastic_maxpool2x2_forward_kernel(PoolArgs a)
 {
-    int const f = ((int)(blockIdx.x % f_blocks) * kConvBlock + threadIdx.x) * W;
-    int const node = blockIdx.x / f_blocks;
-    if (f >= a.frame_size) { return; }
+    int node, f;
+    if (!pool_place<W>(a, node, f)) { return; }
     int const ox = node % a.ow, oy = (node / a.ow) % a.oh, c = node / (a.ow * a.oh);
     float v[2][2][W];
 #pragma unroll
@@ -333,11 +355,10 @@ __global__ __launch_bounds__(kConvBlock) void stochastic_maxpool2x2_forward_kern
 // dx of each tap = dy * prod over the other three taps of (1 - x), the product evaluated in double and rounded once, taps
 // outside the image reading as 0 (include/bb/StochasticMaxPooling2x2.h:262-306)
 template <int W>
-__global__ __launch_bounds__(kConvBlock) void stochastic_maxpool2x2_backward_kernel(PoolArgs a, int f_blocks)
+__global__ __launch_bounds__(kConvBlock) void stochastic_maxpool2x2_backward_kernel(PoolArgs a)
 {
-    int const f = ((int)(blockIdx.x % f_blocks) * kConvBlock + threadIdx.x) * W;
-    int const node = blockIdx.x / f_blocks;
-    if (f >= a.frame_size) { return; }
+    int node, f;
+    if (!pool_place<W>(a, node, f)) { return; }
     int const ox = node % a.ow, oy = (node / a.ow) % a.oh, c = node / (a.ow * a.oh);
     float v[2][2][W], gv[W];
 #pragma unroll

@@ -62,6 +62,34 @@ def test_im2col(ops, shape):
     assert np.array_equal(synth.unpack_bits(yb, of), synth.unpack_bits(yb_ref, of))
 
 
+# blocks of 16 and 64 window positions (forward), of 4 and 16 frames (backward), each with ragged last tiles
+@pytest.mark.parametrize("geometry", [(3, 19, 23, 130), (3, 20, 24, 130), (3, 33, 31, 100), (1, 28, 28, 50)])
+def test_im2col_tiles(ops, geometry):
+    c, h, w, F = geometry
+    rng = np.random.default_rng(sum(geometry))
+    x = rng.random((c * h * w, F)).astype(F32)
+    y_ref = oracle.im2col_forward(x, c, h, w, F, 3, 3, 1, 1, "valid", "reflect_101", 0.0)
+    of = y_ref.shape[1]
+    y = host(ops.im2col_forward(dev(_pad(x, synth.frame_stride_fp32(F))), c, h, w, F, 3, 3))
+    assert np.array_equal(y[:, :of], y_ref)
+    dy = rng.standard_normal((c * 9, of)).astype(F32)
+    dx = host(ops.im2col_backward(dev(_pad(dy, synth.frame_stride_fp32(of))), c, h, w, F, 3, 3))
+    assert np.array_equal(dx[:, :F], oracle.im2col_backward(dy, c, h, w, F, 3, 3, 1, 1, "valid"))
+
+
+# rows that share a workgroup, at its edges: one to 256 threads a row, with four frames and (odd pitch) one frame per thread
+@pytest.mark.parametrize("frames, pitch", [(1, 64), (50, 64), (130, 132), (1020, 1024), (1021, 1024), (1025, 1028), (50, 51), (127, 127), (257, 259)])
+def test_stochastic_maxpool_rows_in_a_workgroup(ops, frames, pitch):
+    c, h, w = 5, 7, 6
+    rng = np.random.default_rng(frames + pitch)
+    x = _pad(rng.random((c * h * w, frames)).astype(F32), pitch)
+    dy = _pad(rng.standard_normal((c * 4 * 3, frames)).astype(F32), pitch)
+    y = host(ops.stochastic_maxpool2x2_forward(dev(x), c, h, w, frames))
+    assert np.array_equal(y[:, :frames], oracle.stochastic_maxpool2x2_forward(x, c, h, w, frames)[:, :frames])
+    dx = host(ops.stochastic_maxpool2x2_backward(dev(x), dev(dy), c, h, w, frames))
+    assert np.array_equal(dx[:, :frames], oracle.stochastic_maxpool2x2_backward(x, dy, c, h, w, frames)[:, :frames])
+
+
 def test_im2col_reference_vectors(ops):
     for k in range(int(GOLD["im2col_count"][0])):
         c, h, w, F, fh, fw, ys, xs, same, border = [int(v) for v in GOLD["i%d_geom" % k]]
