@@ -870,7 +870,7 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     s.fold.mean = c.mean; s.fold.rstd = c.rstd; s.fold.gamma = c.gamma; s.fold.beta = c.beta; s.fold.inv_frames = 1.0f / (float)c.frame_size;
     s.fold.frame_size = c.frame_size; s.fold.lo = 0.5f - c.bias; s.fold.hi = 0.5f + c.bias;
     s.fold.dW = c.dW; s.fold.overwrite = dw_overwrite; s.fold.node_consts = small ? nullptr : consts;
-    static std::atomic<uint32_t> calls{0};
+    static std::atomic<uint32_t> calls{1};          // (0 is what new scratch memory mostly holds: see CornerFoldArgs::call)
     s.fold.discard = reinterpret_cast<uint32_t *>(consts + O); s.fold.call = calls.fetch_add(1, std::memory_order_relaxed);
     bool const dy_quads = c.frame_stride >= ((c.frame_size + 3) & ~3);      // rows of dy hold whole groups of four frames: one 16-byte load per lane and pass
     if (small) {

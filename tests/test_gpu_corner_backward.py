@@ -153,3 +153,10 @@ def test_corner_sums_of_long_skewed_rows():
     rms = float((e * e).mean().sqrt())
     print("rms %.2e" % rms)
     assert rms <= 9e-8
+
+
+@pytest.mark.parametrize("n", [5, 6])
+@pytest.mark.parametrize("frames", [20485, 40965])
+def test_a_discarded_gradient_in_long_passes(n, frames):
+    """the same where a wavefront of the dx kernel takes two (20485) and four (40965) groups of 256 frames: the launch has workgroups enough"""
+    test_a_discarded_gradient_may_hold_anything(n, (216, 36, frames, 0))
