@@ -97,14 +97,15 @@ class AdamState:
         return np.float32(np.float32(self.lr * np.sqrt(one - self.b2, dtype=np.float32)) / (one - self.b1))
 
     def step(self):
-        native.fp32_OptimizerAdam(len(self.params), self.t_size, self.t_params, self.t_grads, self.t_m, self.t_v, self.lr_t(), self.beta1, self.beta2)
+        native.fp32_OptimizerAdam(len(self.params), self.t_size, self.t_params, self.t_grads, self.t_m, self.t_v,
+                                  native.adam_rate(self.lr, self.b1, self.b2), self.beta1, self.beta2)
         self.b1 = self.b1 * self.beta1
         self.b2 = self.b2 * self.beta2
 
     def update(self):
         """Optimizer::Update of the reference = step, then the gradients set to zero (include/bb/Optimizer.h:31-35), in one launch."""
-        native.fp32_OptimizerAdam_Update(len(self.params), self.t_size, self.t_params, self.t_grads, self.t_m, self.t_v, self.lr_t(), self.beta1,
-                                         self.beta2)
+        native.fp32_OptimizerAdam_Update(len(self.params), self.t_size, self.t_params, self.t_grads, self.t_m, self.t_v,
+                                         native.adam_rate(self.lr, self.b1, self.b2), self.beta1, self.beta2)
         self.b1 = self.b1 * self.beta1
         self.b2 = self.b2 * self.beta2
 

@@ -244,3 +244,28 @@ def test_classifier_tail_limits(ops):
         ops.classifier_tail(x, torch.zeros((4, 3), dtype=torch.int32, device="cuda"), t, 64, t_sum=1.0)          # too many input nodes for one launch
     with pytest.raises(RuntimeError):
         ops.classifier_tail(x[:20], torch.zeros((17, 3), dtype=torch.int32, device="cuda"), torch.zeros((17, 64), device="cuda"), 64, t_sum=1.0)
+
+
+@pytest.mark.parametrize("frames", [1, 7, 63, 64, 65, 1000])
+def test_small_outputs_share_no_memory(frames):
+    """outputs of one call that come from one allocation are apart, aligned and of their own size: each keeps its values while the others are overwritten"""
+    import torch
+    from binarybrain_amd import ops, synth
+    rng = np.random.default_rng(frames)
+    stride = synth.frame_stride_fp32(frames)
+    x = torch.rand((21, stride), device="cuda")
+    idx = torch.arange(21, dtype=torch.int32, device="cuda").reshape(3, 7).contiguous()
+    t = torch.zeros((3, stride), device="cuda")
+    t[0] = 1.0
+    tail = ops.classifier_tail(x, idx, t, frames, t_sum=float(frames), want_dy=True)
+    W = torch.rand((5, 64), device="cuda")
+    layer = ops.differentiable_lut_forward_training(6, x, torch.from_numpy(synth.wiring(rng, 21, 5)).cuda(), W, frames, torch.zeros(5, device="cuda"),
+                                                    torch.ones(5, device="cuda"))
+    for outputs in ([o for o in tail if o is not None], list(layer)):
+        kept = [o.clone() for o in outputs]
+        for k, o in enumerate(outputs):
+            assert o.is_contiguous() and o.data_ptr() % 256 == 0
+            o.fill_(7)
+            assert all(torch.equal(a, b) for j, (a, b) in enumerate(zip(outputs, kept)) if j > k)
+            assert bool((o == 7).all())
+        assert all(bool((o == 7).all()) for o in outputs)

@@ -117,3 +117,13 @@ def test_against_compiled_reference():
         assert _close_at(oracle.vector_op(name, *args), oracle.ref_vector_op(name, *args), scale), name
     for name, args in [("sqrt", (np.abs(x),)), ("exp", (x,)), ("min", (x, y)), ("max", (x, y)), ("min_v", (x, None, -0.2)), ("max_v", (x, None, -0.2))]:
         assert _ulp_close(oracle.vector_op(name, *args), oracle.ref_vector_op(name, *args), 2), name
+
+
+def test_rate_formed_natively_is_the_numpy_one():
+    """the step size that AdamState passes on, formed in C++: the same bits as lr_t(), from the first step to the limits of the products"""
+    from binarybrain_amd.capi import native
+    rng = np.random.default_rng(5)
+    for _ in range(5000):
+        lr, b1, b2 = (F32(v) for v in (10.0 ** rng.uniform(-6, 0), rng.random() ** 4, rng.random() ** 4))
+        want = F32(F32(lr * np.sqrt(F32(1) - b2, dtype=F32)) / (F32(1) - b1))
+        assert native.adam_rate(lr, b1, b2) == float(want)
