@@ -180,15 +180,16 @@ int dx_quads_env(void)        { static int v = env_int("BBHIP_DX_QUADS", 0); ret
 int dx_pass_steps_env(void)   { static int v = env_int("BBHIP_DX_STEPS", 0); return (v <= 0) ? 0 : (v <= 1) ? 1 : (v <= 2) ? 2 : 4; }
 // Wavefronts that share an input's work list in the dx kernels (DxArgs::split), 0 = none: four where one wavefront per (input node, unit) would
 // leave the launch with fewer than 4096 workgroups and the lists are long enough to share, sixteen where with four the launch
-// would still have less than two wavefronts per SIMD (not where the rows of dy outgrow the L2s: the wavefronts of a launch then walk the nodes together,
-// and sixteen places in the lists at a time cost 6 % at 40 inputs, 8000 nodes, 4000 frames).  BBHIP_DX_SPLIT = 0 / 1 forces none / four.
+// would still have less than two wavefronts per SIMD (the wavefronts walk the nodes together, each taking every fourth or sixteenth item of its list:
+// packed training steps of 40 inputs x 8000 nodes x 4000 frames 140 us with sixteen and 170 with four, 32 x 2000 x 3000 37 and 53; with more workgroups
+// four are better: 100 x 8000 x 4000 128 and 148).  BBHIP_DX_SPLIT = 0 / 1 forces none / four.
 // Measured: training step of 59 inputs x 1594 nodes x 27 frames 30.0 -> 18.9 us, 50 x 3000 x 200 (StochasticLut4) 39.3 -> 22.3 us.
-int dx_split_lists(int max_fan, int input_node_size, int node_size, int frame_size, int chunk_count)
+int dx_split_lists(int max_fan, int input_node_size, int chunk_count)
 {
     static int const env = env_int("BBHIP_DX_SPLIT", 2);
     if (env == 0 || env == 1) { return env * kWavesPerBlk; }
     if (max_fan < 16 || (long long)chunk_count * ((input_node_size + kWavesPerBlk - 1) / kWavesPerBlk) >= 4096) { return 0; }
-    return (max_fan >= 32 && (long long)chunk_count * input_node_size < 1024 && (long long)node_size * frame_size <= (1 << 22)) ? kDxWaves : kWavesPerBlk;
+    return (max_fan >= 32 && (long long)chunk_count * input_node_size < 1024) ? kDxWaves : kWavesPerBlk;
 }
 // BinaryLut6 units of 128 words: 8192 input rows x 512 bytes is what an XCD's 4 MiB L2 holds (1.2 GB fetched per launch at
 // the benchmark shape; 192-word units fetch 1.9 GB, 256-word units 2.3 GB).  With the per-wavefront set-up at its
@@ -889,9 +890,15 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
 
     DxTableArgs t{};
     // Frames per pass: a term's table and its loads are shared by the steps of a pass, so long passes where all the rows of dy and of indices
-    // that a pass gathers from (5 bytes per node and frame) stay in an XCD's L2; halved while the launch would fall short of workgroups.
+    // that a pass gathers from (5 bytes per node and frame) stay in an XCD's L2; halved while the launch would fall short of workgroups: a workgroup
+    // is four inputs, or one whose list its wavefronts share (27 inputs x 87 nodes x 94500 frames in passes of 256 / 512 / 1024 frames, convolutional
+    // block with 10000 / 5000 / 2500 workgroups: 125 / 117 / 122 us; 27 x 216 x 230400 371 / 348 / 346).
     int quads = (O <= 512) ? 4 : (O <= 1024) ? 2 : 1;
-    while (quads > 1 && (long long)ceil_div(c.frame_size, quads * 256) * ceil_div(c.input_node_size, kWavesPerBlk) < 2048) { quads /= 2; }
+    auto const enough = [&](int q) {
+        long long const chunks = ceil_div(c.frame_size, q * 256);
+        return chunks * ceil_div(c.input_node_size, kWavesPerBlk) >= 2048 || (c.rev_stride > 16 && chunks * c.input_node_size >= 3072);
+    };
+    while (quads > 1 && !enough(quads)) { quads /= 2; }
     if (dx_quads_env() != 0) { quads = dx_quads_env(); }
     t.far = !dy_quads || (long long)O * c.frame_stride * 4 > 0xffffffffLL || (long long)O * own_words * 4 > 0xffffffffLL ||
             (long long)O * NN * 4 > 0xffffffffLL;
@@ -900,7 +907,7 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     d.dy = c.dy; d.dx = c.dx; d.rev = c.rev; d.rev_stride = c.rev_stride; d.input_node_size = c.input_node_size; d.frame_size = c.frame_size;
     d.dy_stride = c.frame_stride; d.dx_stride = c.frame_stride;
     d.chunk = quads * 256; d.chunk_count = ceil_div(c.frame_size, d.chunk);
-    int split          = dx_split_lists(c.rev_stride - 1, c.input_node_size, O, c.frame_size, d.chunk_count);
+    int split          = dx_split_lists(c.rev_stride - 1, c.input_node_size, d.chunk_count);
     // Long passes leave at least 2048 workgroups, with which sixteen wavefronts never share a list: only BBHIP_DX_QUADS brings the two together
     if (quads > 1 && split > kWavesPerBlk) { split = kWavesPerBlk; }
     int const in_tiles = split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
@@ -955,7 +962,7 @@ int run_backward_small(BackwardCall const &c, hipStream_t st, int dw_overwrite)
     int steps = 4, in_tiles = 0;
     for (;; steps /= 2) {
         d.chunk = steps * kWave; d.chunk_count = ceil_div(c.frame_size, d.chunk);
-        d.split = dx_split_lists(c.rev_stride - 1, c.input_node_size, c.output_node_size, c.frame_size, d.chunk_count);
+        d.split = dx_split_lists(c.rev_stride - 1, c.input_node_size, d.chunk_count);
         in_tiles = d.split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
         bool const enough = (long long)d.chunk_count * in_tiles >= ((d.split && steps == 4) ? 1024 : 256) && c.frame_size > d.chunk / 2;
         if (steps == 1 || enough) { break; }
@@ -1164,7 +1171,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         int const chunk  = ((frames + kWave * steps - 1) / (kWave * steps)) * (kWave * steps);
         int const chunk_count = ceil_div(c.frame_size, chunk);
         // few input nodes with long work lists: the wavefronts of a workgroup share one input node (DxArgs::split)
-        int const split    = dx_split_lists(c.rev_stride - 1, c.input_node_size, c.output_node_size, c.frame_size, chunk_count);
+        int const split    = dx_split_lists(c.rev_stride - 1, c.input_node_size, chunk_count);
         int const in_tiles = split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
         if ((long long)chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
         DxArgs d{};

@@ -447,9 +447,9 @@ __global__ __launch_bounds__(WAVES * kWave) void lut_dx_table_kernel(DxTableArgs
     typedef __attribute__((address_space(4))) uint32_t const const_word;
     int const fan = list[0];
     uint32_t const discard_word = BN ? *(const_word *)t.discard : 0u;   // (on the way with the list's length)
-    int t_begin, t_end;
-    dx_list_range<WAVES>(fan, share, t_begin, t_end);
-    list += 1;
+    int first, step, items;
+    dx_list_steps<WAVES>(fan, share, first, step, items);
+    list += 1 + first;
     int const f_lane = ck * kPass + 4 * lane;
     uint32_t const dy_bytes = (uint32_t)(t.node_size - 1) * (uint32_t)a.dy_stride * 4u + quad_row_bytes(a.frame_size, true);
     __amdgpu_buffer_rsrc_t const dyr = row_descriptor(a.dy, 0, 0, FAR ? 0u : dy_bytes);
@@ -514,20 +514,20 @@ __global__ __launch_bounds__(WAVES * kWave) void lut_dx_table_kernel(DxTableArgs
     auto walk = [&](auto gated) {
         Stage s0, s1;
         int e_ahead = 0;
-        if (t_begin < t_end) {
-            request(list[t_begin], s0);
-            e_ahead = list[min(t_begin + 1, t_end - 1)];
+        if (items > 0) {
+            request(list[0], s0);
+            e_ahead = list[min(1, items - 1) * step];
         }
-        for (int i = t_begin; i < t_end; i += 2) {
-            if (i + 1 < t_end) {
+        for (int i = 0; i < items; i += 2) {
+            if (i + 1 < items) {
                 request(e_ahead, s1);
-                e_ahead = list[min(i + 2, t_end - 1)];
+                e_ahead = list[min(i + 2, items - 1) * step];
             }
             add(s0, table[wave][0], gated);
-            if (i + 1 < t_end) {
-                if (i + 2 < t_end) {
+            if (i + 1 < items) {
+                if (i + 2 < items) {
                     request(e_ahead, s0);
-                    e_ahead = list[min(i + 3, t_end - 1)];
+                    e_ahead = list[min(i + 3, items - 1) * step];
                 }
                 add(s1, table[wave][1], gated);
             }

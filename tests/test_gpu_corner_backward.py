@@ -160,3 +160,25 @@ def test_corner_sums_of_long_skewed_rows():
 def test_a_discarded_gradient_in_long_passes(n, frames):
     """the same where a wavefront of the dx kernel takes two (20485) and four (40965) groups of 256 frames: the launch has workgroups enough"""
     test_a_discarded_gradient_may_hold_anything(n, (216, 36, frames, 0))
+
+
+# a list of exactly as many items as wavefronts share it, one more, one less; sixteen and four wavefronts; a short list among long ones; two groups of
+# 256 frames per wavefront
+@pytest.mark.parametrize("shape", [(7, 17, 2000), (7, 19, 1100), (12, 31, 1500), (12, 67, 1300), (40, 700, 6200), (9, 40, 90000)])
+def test_shared_lists(shape):
+    test_corner_backward(6, shape + (0,))
+
+
+@pytest.mark.parametrize("n, shape", [(6, (7, 17, 5000)), (6, (12, 67, 4500)), (4, (9, 150, 4200)), (6, (40, 700, 4100))])
+def test_shared_lists_of_real_valued_inputs(n, shape):
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    I, O, F = shape
+    stride = synth.frame_stride_fp32(F)
+    rng = np.random.default_rng(O)
+    idx = synth.wiring(rng, I, O, n); W = synth.lut_tables(rng, O, n)
+    x = synth.uniform_frames(rng, I, F, stride); dy = synth.normal_frames(rng, O, F, stride)
+    dx_ref, dW_ref = oracle.stochastic_lut_backward(n, x, dy, idx, W, F)
+    d_idx, dW = dev(idx), dev(np.zeros_like(W))
+    dx = ops.stochastic_lut_backward(n, dev(x), dev(dy), d_idx, dev(W), dW, F, ops.reverse_table(d_idx, I))
+    assert_bwd(host(dx)[:, :F], dx_ref[:, :F], "dx"); assert_bwd(host(dW), dW_ref, "dW")
