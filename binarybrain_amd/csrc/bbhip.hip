@@ -358,7 +358,7 @@ int dispatch_backward(int xmode, int kind, int dxmode, BwdArgs const &a, hipStre
 }
 
 template <int N, int U>
-int dispatch_dx_u(int xmode, DxArgs const &a, hipStream_t st)
+int dispatch_dx_u(int xmode, bool wide, DxArgs const &a, hipStream_t st)
 {
     dim3 const grid(a.fin_blocks + a.chunk_count * a.tiles.count), block((a.split ? a.split : kWavesPerBlk) * kWave);
 #define BBHIP_DX_CASE(X)                                                                                                       \
@@ -367,18 +367,21 @@ int dispatch_dx_u(int xmode, DxArgs const &a, hipStream_t st)
         else                        { launch((lut_dx_kernel<N, X, U, kWavesPerBlk>), grid, block, 0, st, a); }   \
         return 0;                                                                                                              \
     }
+    if constexpr (U == 4) {
+        if (wide && a.split <= kWavesPerBlk) { launch((lut_dx_kernel<N, kXClamp, U, kWavesPerBlk, true>), grid, block, 0, st, a); return 0; }
+    }
     BBHIP_DX_CASE(kXClamp) BBHIP_DX_CASE(kXBinary) BBHIP_DX_CASE(kXBit)
 #undef BBHIP_DX_CASE
     return fail("dx variant (x=%d) not built", xmode);
 }
 
 template <int N>
-int dispatch_dx(int xmode, int steps, DxArgs const &a, hipStream_t st)
+int dispatch_dx(int xmode, int steps, bool wide, DxArgs const &a, hipStream_t st)
 {
     switch (steps) {
-    case 1: return dispatch_dx_u<N, 1>(xmode, a, st);
-    case 2: return dispatch_dx_u<N, 2>(xmode, a, st);
-    case 4: return dispatch_dx_u<N, 4>(xmode, a, st);
+    case 1: return dispatch_dx_u<N, 1>(xmode, wide, a, st);
+    case 2: return dispatch_dx_u<N, 2>(xmode, wide, a, st);
+    case 4: return dispatch_dx_u<N, 4>(xmode, wide, a, st);
     }
     return fail("dx kernel with %d wavefront-steps per pass not built", steps);
 }
@@ -997,6 +1000,19 @@ int run_backward_small(BackwardCall const &c, hipStream_t st, int dw_overwrite)
     return 0;
 }
 
+// Real-valued inputs: passes of 256 frames, four consecutive ones per lane (lut_dx_kernel, WIDE), where a term's coefficients and addresses serve twice the
+// frames of the usual 128 and its rows come by a quarter of the loads.  All rows of x and dy that a window touches, 1 KB each, should be what an
+// L2 holds (training steps with and without: 1024 inputs + 2000 nodes x 4000 frames 106 and 112 us, 300 + 4000 x 4000 179 and 186, 500 + 1000 x 4000
+// with batch-norm 67 and 72.5, 1024 + 1024 x 1000 31.8 and 35.0; 3000 + 3000 x 6000 239 either way, 4096 + 4096 x 8192 498 and 457), and the launch should
+// have workgroups enough: one per input and pass where lists are shared (batch-norm, 300 + 1000 x 1200, 1500 of them, 39.8 and 40.3; 128 + 1500 x 2100,
+// 1152, 91.6 and 89.4; 40 + 3000 x 2000, 320, 103 and 92), else one per four inputs and pass, and items enough (1500 + 800 x 700, lists of three, 29.8 and 29.2).
+bool dx_wide_passes(int input_node_size, int output_node_size, int frame_size, int max_fan, long long links)
+{
+    long long const chunks = ceil_div(frame_size, 256);
+    if ((long long)input_node_size + output_node_size > 5000) { return false; }
+    return max_fan >= 16 ? chunks * input_node_size >= 1400 : (chunks * ceil_div(input_node_size, kWavesPerBlk) >= 1024 && chunks * links >= 20480);
+}
+
 template <int N>
 int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packed = PackedInputHint{nullptr, 0, 0, 0},
                  PreparedTablesHint tables = PreparedTablesHint{nullptr, 0, 0}, int dw_overwrite = 0)
@@ -1174,8 +1190,12 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
     }
 
     if (dxmode == kDxNone) {
-        int const steps  = dx_pass_steps_env() ? dx_pass_steps_env() : 2;                             // wavefront-steps per pass: {1, 2, 4}
-        int const frames = dx_chunk_frames_env() ? dx_chunk_frames_env() : 128;
+        int const whole = (c.frame_size + 3) & ~3;
+        bool const quads = c.xmode == kXClamp && c.x_stride >= whole && c.frame_stride >= whole;      // rows hold whole groups of four frames
+        bool const wide  = quads && (dx_pass_steps_env() == 4 || (dx_pass_steps_env() == 0 && dx_chunk_frames_env() == 0 &&
+                                     dx_wide_passes(c.input_node_size, c.output_node_size, c.frame_size, c.rev_stride - 1, (long long)c.output_node_size * N)));
+        int const steps  = wide ? 4 : dx_pass_steps_env() ? dx_pass_steps_env() : 2;                  // wavefront-steps per pass: {1, 2, 4}
+        int const frames = dx_chunk_frames_env() ? dx_chunk_frames_env() : wide ? 256 : 128;
         int const chunk  = ((frames + kWave * steps - 1) / (kWave * steps)) * (kWave * steps);
         int const chunk_count = ceil_div(c.frame_size, chunk);
         // few input nodes with long work lists: the wavefronts of a workgroup share one input node (DxArgs::split)
@@ -1188,6 +1208,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         d.x_stride = c.x_stride; d.dy_stride = c.frame_stride; d.dx_stride = c.frame_stride;
         d.chunk = chunk; d.chunk_count = chunk_count; d.tiles = make_tile_divisor(in_tiles);
         d.bias = c.bias; d.split = split;
+        d.dx_quads = (c.frame_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(c.dx) & 15u) == 0) ? 1 : 0;
         // folding the slab sums into dW rides at the end of this launch
         d.fin_partial = part; d.fin_dW = c.dW; d.fin_node_size = c.output_node_size; d.fin_slab_count = slab_total;
         d.fin_overwrite = dw_overwrite;
@@ -1195,7 +1216,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         if ((long long)d.fin_blocks + (long long)chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
         {
             ScopedTimer tm(kTimeDx, st);
-            if (dispatch_dx<N>(c.xmode, steps, d, st)) { return 1; }
+            if (dispatch_dx<N>(c.xmode, steps, wide, d, st)) { return 1; }
         }
         BBHIP_LAUNCH_CHECK();
         return 0;

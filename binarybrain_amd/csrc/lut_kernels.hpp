@@ -1261,6 +1261,7 @@ struct DxArgs {
     float       *fin_dW;
     int   fin_node_size, fin_slab_count, fin_blocks;
     int   fin_overwrite;        // dW = instead of dW += (the caller's dW holds nothing: bbhip_HintTableGradientOverwrite)
+    int   dx_quads;             // rows of dx start on 16 bytes
 };
 
 // ------------------------------------------------------------------------------------------------
@@ -1300,7 +1301,7 @@ __device__ __forceinline__ float input_value(uint32_t raw, int bit, float lo, fl
 
 // One term of the work list.  The gathered rows live in a Stage (vector registers); the coefficients are fetched
 // into scalar registers right before the term is evaluated.
-template <int N, int XMODE, int U>          // U wavefront-steps per pass
+template <int N, int XMODE, int U, bool WIDE>          // U wavefront-steps per pass; WIDE: see lut_dx_kernel
 struct DxTerm {
     static constexpr int M  = N - 1;        // variables of the derivative LUT
     static constexpr int ML = M / 2, MH = M - ML;
@@ -1318,6 +1319,19 @@ struct DxTerm {
                                                  uint32_t x_row_bytes, uint32_t y_row_bytes, Stage &st)
     {
         constexpr uint32_t xstep = (XMODE == kXBit) ? (kWave / 32) * 4u : kWave * 4u;
+        if constexpr (WIDE) {
+#pragma unroll
+            for (int j = 0; j <= M; ++j) {
+                __amdgpu_buffer_rsrc_t const r = address_descriptor((uint32_t)rec[2 * j], (uint32_t)rec[2 * j + 1], j < M ? x_row_bytes : y_row_bytes);
+                auto const q = __builtin_amdgcn_raw_buffer_load_b128(r, j < M ? xoff : yoff, 0, 0);
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (j < M) { st.raw[u][j < M ? j : 0] = q[u]; }
+                    else       { st.dyv[u] = __uint_as_float(q[u]); }
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < M; ++j) {
             __amdgpu_buffer_rsrc_t const r = address_descriptor((uint32_t)rec[2 * j], (uint32_t)rec[2 * j + 1], x_row_bytes);
@@ -1405,7 +1419,7 @@ __device__ __forceinline__ void dx_list_steps(int cnt, int share, int &t_first, 
 // ... and the end of a pass: the lane's U sums go to dx — directly, or in split mode added over the workgroup's wavefronts
 // in wavefront order (a fixed order: results do not depend on timing) by the first of them.  Every wavefront of the
 // workgroup must come here (the barrier).
-template <int U, int WAVES>
+template <int U, int WAVES, bool WIDE>
 __device__ __forceinline__ void dx_store_pass(DxArgs const &a, float (&part)[WAVES][U][kWave], int in, int wave, int lane,
                                               int f_begin, float (&acc)[U])
 {
@@ -1425,6 +1439,19 @@ __device__ __forceinline__ void dx_store_pass(DxArgs const &a, float (&part)[WAV
         __syncthreads();                    // the next pass writes part again
         if (wave != 0) { return; }
     }
+    if constexpr (WIDE) {
+        int const f = f_begin + U * lane;
+        float *const row = a.dx + (size_t)in * a.dx_stride + f;
+        if (a.dx_quads && f + U <= a.frame_size) {
+            typedef float f32x4 __attribute__((ext_vector_type(4)));
+            f32x4 const o = {acc[0], acc[1], acc[2], acc[3]};
+            __builtin_nontemporal_store(o, reinterpret_cast<f32x4 *>(row));
+            return;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) { if (f + u < a.frame_size) { row[u] = acc[u]; } }
+        return;
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         int const f = f_begin + u * kWave + lane;
@@ -1432,11 +1459,13 @@ __device__ __forceinline__ void dx_store_pass(DxArgs const &a, float (&part)[WAV
     }
 }
 
-// WAVES: wavefronts of a workgroup; kDxWaves: split mode
-template <int N, int XMODE, int U, int WAVES>
+// WAVES: wavefronts of a workgroup; kDxWaves: split mode.  WIDE: a lane's U = 4 steps are four consecutive frames of fp32 rows that hold whole groups of
+// four, one 16-byte load each (what lies behind the last frame enters frames that are not stored)
+template <int N, int XMODE, int U, int WAVES, bool WIDE = false>
 __global__ __launch_bounds__(WAVES * kWave) void lut_dx_kernel(DxArgs a)
 {
-    using T = DxTerm<N, XMODE, U>;
+    static_assert(!WIDE || (U == 4 && XMODE != kXBit), "four frames per lane");
+    using T = DxTerm<N, XMODE, U, WIDE>;
     // the table-gradient partial sums are complete before this launch and independent of it: folding them into dW rides at
     // the end of this launch instead of taking a launch of its own
     int const bid = blockIdx.x;
@@ -1463,7 +1492,7 @@ __global__ __launch_bounds__(WAVES * kWave) void lut_dx_kernel(DxArgs a)
     typedef __attribute__((address_space(4))) int const const_int;
     const_int *rec = (const_int *)(a.term + ((size_t)in * (a.rev_stride - 1) + t_first) * T::REC);
     size_t const rec_step = (size_t)t_step * T::REC;
-    uint32_t const y_row_bytes = (uint32_t)a.frame_size * 4u;
+    uint32_t const y_row_bytes = (uint32_t)(WIDE ? (a.frame_size + 3) & ~3 : a.frame_size) * 4u;
     uint32_t const x_row_bytes = (XMODE == kXBit) ? (uint32_t)((a.frame_size + 31) >> 5) * 4u : y_row_bytes;
     float const lo = 0.5f - a.bias, hi = 0.5f + a.bias;
     int const bit = lane & 31;
@@ -1473,7 +1502,7 @@ __global__ __launch_bounds__(WAVES * kWave) void lut_dx_kernel(DxArgs a)
     // with 8 wavefronts per SIMD the other wavefronts already cover the latency, and more loads in flight only
     // lengthen the queues.)
     for (int f_begin = ck * a.chunk; f_begin < min((ck + 1) * a.chunk, a.frame_size); f_begin += kWave * U) {
-        uint32_t const f0   = (uint32_t)(f_begin + lane);
+        uint32_t const f0   = (uint32_t)(f_begin + (WIDE ? U : 1) * lane);
         uint32_t const yoff = f0 * 4u;
         uint32_t const xoff = (XMODE == kXBit) ? (f0 >> 5) * 4u : yoff;
         float acc[U];
@@ -1502,7 +1531,7 @@ __global__ __launch_bounds__(WAVES * kWave) void lut_dx_kernel(DxArgs a)
             T::load_coefficients(rec + (size_t)t * rec_step, Dk);
             T::accumulate(st, Dk, bit, lo, hi, acc);
         }
-        dx_store_pass<U, WAVES>(a, part, in, wave, lane, f_begin, acc);
+        dx_store_pass<U, WAVES, WIDE>(a, part, in, wave, lane, f_begin, acc);
     }
 }
 

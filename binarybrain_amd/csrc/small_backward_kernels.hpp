@@ -209,7 +209,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
             acc[u] = __builtin_fmaf(dy[u], slope(x), acc[u]);
         }
     }
-    dx_store_pass<U, WAVES>(a, part, in, wave, lane, f_begin, acc);
+    dx_store_pass<U, WAVES, false>(a, part, in, wave, lane, f_begin, acc);
 }
 
 }  // namespace bbhip

@@ -68,3 +68,22 @@ def test_scratch_arguments_of_the_backward_call_are_not_used():
     again = torch.zeros_like(dW)
     got = ops.differentiable_lut_backward(n, d_x, d_dy, d_idx, d_W, again, F, d_mean, d_rstd, rev, binary_mode=False)
     assert torch.equal(got[:, :F], dx[:, :F]) and torch.equal(again, dW)
+
+
+# passes of four consecutive frames per lane: last groups of one to four frames, one lane and 64 lanes in the last pass, shared and own lists, rows of dx on 16
+# bytes and not (pitch 8197, 4101), rows too short for whole groups (pitch = frames)
+@pytest.mark.parametrize("n", [2, 4, 6])
+@pytest.mark.parametrize("shape", [(600, 500, 8191, 0), (520, 400, 8193, 8197), (90, 700, 4100, 4101), (80, 300, 4354, 0), (520, 400, 8193, 8193), (530, 400, 7936, 7936)])
+def test_four_frames_per_lane(n, shape):
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    I, O, F, stride = shape
+    stride = stride or synth.frame_stride_fp32(F)
+    rng = np.random.default_rng(F + n)
+    idx = synth.wiring(rng, I, O, n); W = synth.lut_tables(rng, O, n)
+    x = synth.uniform_frames(rng, I, F, stride, -0.1, 1.1); dy = synth.normal_frames(rng, O, F, stride)
+    dx_ref, dW_ref = oracle.stochastic_lut_backward(n, x, dy, idx, W, F)
+    x[:, F:] = np.nan; dy[:, F:] = np.nan           # what lies behind the frames enters nothing
+    d_idx, dW = dev(idx), dev(np.zeros_like(W))
+    dx = ops.stochastic_lut_backward(n, dev(x), dev(dy), d_idx, dev(W), dW, F, ops.reverse_table(d_idx, I))
+    assert_bwd(host(dx)[:, :F], dx_ref[:, :F], "dx"); assert_bwd(host(dW), dW_ref, "dW")
