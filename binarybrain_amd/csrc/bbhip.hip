@@ -986,6 +986,8 @@ int run_backward_small(BackwardCall const &c, hipStream_t st, int dw_overwrite)
     s.node_tiles = ceil_div(c.output_node_size, waves / s.node_waves);
     if ((long long)s.node_tiles + (long long)d.chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
     dim3 const grid(s.node_tiles + d.chunk_count * in_tiles), block(waves * kWave);
+    bool const quads = c.x_stride >= ((c.frame_size + 3) & ~3) && c.frame_stride >= ((c.frame_size + 3) & ~3);      // rows hold whole groups of four frames
+    d.dx_quads = (c.frame_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(c.dx) & 15u) == 0) ? 1 : 0;
     {
         ScopedTimer tm(kTimeBackward, st);
 #define BBHIP_SMALL_CASE(U)                                                                                                  \
@@ -993,7 +995,8 @@ int run_backward_small(BackwardCall const &c, hipStream_t st, int dw_overwrite)
         else                      { launch((lut_small_backward_kernel<N, U, kWavesPerBlk>), grid, block, 0, st, s); }
         if (steps == 1)      { BBHIP_SMALL_CASE(1) }
         else if (steps == 2) { BBHIP_SMALL_CASE(2) }
-        else                 { launch((lut_small_backward_kernel<N, 4, kWavesPerBlk>), grid, block, 0, st, s); }       // (from 1024 workgroups: `enough`)
+        else if (quads)      { launch((lut_small_backward_kernel<N, 4, kWavesPerBlk, true>), grid, block, 0, st, s); }      // (from 1024 workgroups: `enough`)
+        else                 { launch((lut_small_backward_kernel<N, 4, kWavesPerBlk>), grid, block, 0, st, s); }
 #undef BBHIP_SMALL_CASE
     }
     BBHIP_LAUNCH_CHECK();

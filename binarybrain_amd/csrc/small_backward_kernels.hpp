@@ -77,10 +77,13 @@ struct SmallBackwardArgs {
 // others, spares the 2^(N-1) moves to scalar registers.  That is 40 vector instructions per term more than lut_dx_kernel has.
 // Training step (with the forward pass that derives its tables, two launches instead of four): 100 inputs x 100 nodes x 300 frames 18.2 -> 11.5 us,
 // 300 x 1000 x 500 20.7 -> 16.6, 4000 x 400 x 2000 32.8 -> 24.9.
+// WIDE: the four steps of a lane are four consecutive frames of rows that hold whole groups of four, one load each (lut_dx_kernel): 1001 inputs x 1531
+// nodes x 1999 frames, four inputs per node, 26.6 us a training step instead of 30.6.
 // (waves_per_eu: results of the matrix unit in ordinary registers, without a move for each)
-template <int N, int U, int WAVES>
+template <int N, int U, int WAVES, bool WIDE = false>
 __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2))) void lut_small_backward_kernel(SmallBackwardArgs s)
 {
+    static_assert(!WIDE || U == 4, "four frames per lane");
     constexpr int NN = 1 << N, M = N - 1;
     DxArgs const &a = s.dx;
     int const lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
@@ -157,12 +160,13 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
     dx_list_range<WAVES>(list[0], share, t_begin, t_end);
     list += 1;
     // whole buffers of less than 4 GiB: rows are 32-bit offsets into them, and a lane past the last frame reads what lies there (its sum is not stored)
-    uint32_t const x_pitch = (uint32_t)a.x_stride * 4u, y_pitch = (uint32_t)a.dy_stride * 4u, row_bytes = (uint32_t)a.frame_size * 4u;
+    uint32_t const x_pitch = (uint32_t)a.x_stride * 4u, y_pitch = (uint32_t)a.dy_stride * 4u;
+    uint32_t const row_bytes = (uint32_t)(WIDE ? (a.frame_size + 3) & ~3 : a.frame_size) * 4u;
     __amdgpu_buffer_rsrc_t const xr = row_descriptor(a.x, 0, 0, (uint32_t)(a.input_node_size - 1) * x_pitch + row_bytes);
     __amdgpu_buffer_rsrc_t const yr = row_descriptor(a.dy, 0, 0, (uint32_t)(s.node_size - 1) * y_pitch + row_bytes);
     __amdgpu_buffer_rsrc_t const wr = row_descriptor(s.W, 0, 0, (uint32_t)s.node_size * (NN * 4u));
     int const f_begin = ck * U * kWave;
-    uint32_t const off = (uint32_t)(f_begin + lane) * 4u;
+    uint32_t const off = (uint32_t)(f_begin + (WIDE ? U : 1) * lane) * 4u;
 
     // a term's wiring and table are requested while the term before it is evaluated (and not looked at before), its list entry another term ahead
     struct Head { int ins[N]; float w; int node, k; };
@@ -190,11 +194,24 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
         for (int j = 0; j < M; ++j) {
             uint32_t const row = (uint32_t)(j < h.k ? h.ins[j] : h.ins[j + 1]) * x_pitch;
+            if constexpr (WIDE) {
+                auto const q = __builtin_amdgcn_raw_buffer_load_b128(xr, off, row, 0);
+#pragma unroll
+                for (int u = 0; u < U; ++u) { raw[u][j] = q[u]; }
+                continue;
+            }
 #pragma unroll
             for (int u = 0; u < U; ++u) { raw[u][j] = __builtin_amdgcn_raw_buffer_load_b32(xr, off + u * (kWave * 4u), row, 0); }
         }
+        if constexpr (WIDE) {
+            auto const q = __builtin_amdgcn_raw_buffer_load_b128(yr, off, (uint32_t)h.node * y_pitch, 0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) { dy[u] = __uint_as_float(q[u]); }
+        }
+        else {
 #pragma unroll
         for (int u = 0; u < U; ++u) { dy[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yr, off + u * (kWave * 4u), (uint32_t)h.node * y_pitch, 0)); }
+        }
         LutSlope<N> slope;
         slope.take(s.lut_binarize ? (h.w > 0.5f ? 1.0f : 0.0f) : h.w, h.k, lane);
         __builtin_amdgcn_sched_barrier(0);              // (the permutation is waited for with the scalar loads issued ahead of it: none of the next term's)
@@ -209,7 +226,7 @@ __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(2
             acc[u] = __builtin_fmaf(dy[u], slope(x), acc[u]);
         }
     }
-    dx_store_pass<U, WAVES, false>(a, part, in, wave, lane, f_begin, acc);
+    dx_store_pass<U, WAVES, WIDE>(a, part, in, wave, lane, f_begin, acc);
 }
 
 }  // namespace bbhip

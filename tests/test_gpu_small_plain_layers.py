@@ -68,3 +68,22 @@ def test_table_gradient_rounding(n, bound, frames):
     rms = float(np.sqrt((e * e).mean()))
     print("n=%d frames=%d rms %.2e" % (n, frames, rms))
     assert rms <= bound
+
+
+# four wavefront-steps per unit as four consecutive frames per lane: last groups of one to four frames, pitches that put dx rows off 16 bytes, and rows too
+# short for whole groups (pitch = frames); own lists and shared ones
+@pytest.mark.parametrize("n", [2, 4, 6])
+@pytest.mark.parametrize("shape", [(1030, 300, 257, 0), (1030, 300, 510, 513), (700, 200, 511, 511), (520, 160, 768, 768), (300, 700, 1021, 0), (300, 700, 1023, 1025)])
+def test_four_frames_per_lane(n, shape):
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    I, O, F, stride = shape
+    stride = stride or synth.frame_stride_fp32(F)
+    rng = np.random.default_rng(F + n)
+    idx = synth.wiring(rng, I, O, n); W = synth.lut_tables(rng, O, n)
+    x = synth.uniform_frames(rng, I, F, stride, -0.1, 1.1); dy = synth.normal_frames(rng, O, F, stride)
+    dx_ref, dW_ref = oracle.stochastic_lut_backward(n, x, dy, idx, W, F)
+    x[:, F:] = np.nan; dy[:, F:] = np.nan           # what lies behind the frames enters nothing
+    d_idx, dW = dev(idx), dev(np.zeros_like(W))
+    dx = ops.stochastic_lut_backward(n, dev(x), dev(dy), d_idx, dev(W), dW, F, ops.reverse_table(d_idx, I))
+    assert_bwd(host(dx)[:, :F], dx_ref[:, :F], "dx"); assert_bwd(host(dW), dW_ref, "dW")
