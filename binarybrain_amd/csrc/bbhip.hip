@@ -182,13 +182,15 @@ int dx_pass_steps_env(void)   { static int v = env_int("BBHIP_DX_STEPS", 0); ret
 // leave the launch with fewer than 4096 workgroups and the lists are long enough to share, sixteen where with four the launch
 // would still have less than two wavefronts per SIMD (the wavefronts walk the nodes together, each taking every fourth or sixteenth item of its list:
 // packed training steps of 40 inputs x 8000 nodes x 4000 frames 140 us with sixteen and 170 with four, 32 x 2000 x 3000 37 and 53; with more workgroups
-// four are better: 100 x 8000 x 4000 128 and 148).  BBHIP_DX_SPLIT = 0 / 1 forces none / four.
+// four are better: 100 x 8000 x 4000 128 and 148).  real_valued: lut_dx_kernel, whose terms take long enough for lists from eight items in launches of fewer than
+// 2048 workgroups (batch-norm, 1500 + 800 x 700 27.8 us and 29.0, 1024 + 1024 x 1000 30.5 and 33.5; packed 500 + 500 x 4000 26 and 23.5).  BBHIP_DX_SPLIT = 0 / 1 forces none / four.
 // Measured: training step of 59 inputs x 1594 nodes x 27 frames 30.0 -> 18.9 us, 50 x 3000 x 200 (StochasticLut4) 39.3 -> 22.3 us.
-int dx_split_lists(int max_fan, int input_node_size, int chunk_count)
+int dx_split_lists(int max_fan, int input_node_size, int chunk_count, bool real_valued = false)
 {
     static int const env = env_int("BBHIP_DX_SPLIT", 2);
     if (env == 0 || env == 1) { return env * kWavesPerBlk; }
-    if (max_fan < 16 || (long long)chunk_count * ((input_node_size + kWavesPerBlk - 1) / kWavesPerBlk) >= 4096) { return 0; }
+    long long const groups = (long long)chunk_count * ((input_node_size + kWavesPerBlk - 1) / kWavesPerBlk);
+    if (groups >= 4096 || max_fan < (real_valued && groups < 2048 ? 8 : 16)) { return 0; }
     return (max_fan >= 32 && (long long)chunk_count * input_node_size < 1024) ? kDxWaves : kWavesPerBlk;
 }
 // BinaryLut6 units of 128 words: 8192 input rows x 512 bytes is what an XCD's 4 MiB L2 holds (1.2 GB fetched per launch at
@@ -1013,7 +1015,8 @@ bool dx_wide_passes(int input_node_size, int output_node_size, int frame_size, i
 {
     long long const chunks = ceil_div(frame_size, 256);
     if ((long long)input_node_size + output_node_size > 5000) { return false; }
-    return max_fan >= 16 ? chunks * input_node_size >= 1400 : (chunks * ceil_div(input_node_size, kWavesPerBlk) >= 1024 && chunks * links >= 20480);
+    long long const groups = chunks * ceil_div(input_node_size, kWavesPerBlk);
+    return max_fan >= (groups < 2048 ? 8 : 16) ? chunks * input_node_size >= 1400 : (chunks * ceil_div(input_node_size, kWavesPerBlk) >= 1024 && chunks * links >= 20480);
 }
 
 template <int N>
@@ -1202,7 +1205,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         int const chunk  = ((frames + kWave * steps - 1) / (kWave * steps)) * (kWave * steps);
         int const chunk_count = ceil_div(c.frame_size, chunk);
         // few input nodes with long work lists: the wavefronts of a workgroup share one input node (DxArgs::split)
-        int const split    = dx_split_lists(c.rev_stride - 1, c.input_node_size, chunk_count);
+        int const split    = dx_split_lists(c.rev_stride - 1, c.input_node_size, chunk_count, true);
         int const in_tiles = split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
         if ((long long)chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
         DxArgs d{};
