@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/bbhip.h"
+#include "launch_rules.hpp"
 #include "lut_kernels.hpp"
 #include "corner_forward_kernels.hpp"
 #include "corner_small_backward_kernels.hpp"
@@ -243,7 +244,6 @@ int arena_get(size_t bytes, char **out, hipStream_t st, Scratch const *fixed = n
 
 inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-inline int ceil_div(int a, int b) { return a / b + (a % b != 0); }      // (no sum that could leave the range)
 
 // A launch without the call-configuration stack and the copies that the <<<>>> form's host stub goes through: 2.7 us of host time for a kernel
 // with 400 bytes of arguments instead of 3.2, and the host is what a program of small layers waits for.  Errors are read by BBHIP_LAUNCH_CHECK.
@@ -730,29 +730,6 @@ int check_backward(BackwardCall const &c, int dxmode)
     return 0;
 }
 
-// Frames per unit of the per-corner sums.  A launch runs in ceil(workgroups / 512) rounds of resident workgroups (two per compute unit: 64 KB of
-// bins each), a unit costs its frames plus about 1024 frames' worth of set-up and closing sums, and more than one slab per node needs the fold
-// launch (about 3072 frames' worth on top): the number of equal slabs that fills one to four rounds with the least of it (slab lengths of a power of two
-// left a round short or a slab nearly empty: 216 nodes x 230400 frames in 9 slabs instead of 8, convolutional block 345.8 -> 340.6 us; 87 x 94500 in 22
-// instead of 93, 120.4 -> 114.3).
-int corner_slab_frames(int frame_size, int tile_count)
-{
-    if (bwd_slab_frames() > 0) { return ceil_div(bwd_slab_frames(), 256) * 256; }
-    int const whole = ceil_div(frame_size, 256) * 256;
-    auto cost = [&](int frames) {
-        long long const slabs = ceil_div(frame_size, frames), rounds = (slabs * tile_count + 511) / 512;
-        return rounds * ((frames < frame_size ? frames : frame_size) + 1024) + (slabs > 1 ? 3072 : 0);
-    };
-    int best = whole;
-    for (int rounds = 1; rounds <= 4; ++rounds) {
-        int const slabs = rounds * 512 / tile_count;
-        if (slabs < 2) { continue; }
-        int const frames = std::max(ceil_div(ceil_div(frame_size, slabs), 256) * 256, 1024);
-        if (frames < whole && cost(frames) < cost(best)) { best = frames; }
-    }
-    return best;
-}
-
 template <int N, bool BN, bool QUADS>
 int launch_corner_backward(CornerSumsArgs const &s, int slab_count, hipStream_t st)
 {
@@ -840,9 +817,10 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     if (from_fp32) { c.x_stride = have_bits ? packed.row_words : packed_row_words(c.frame_size); }
 
     int const O = c.output_node_size, tile_count = ceil_div(O, kWavesPerBlk);
-    int slab = corner_slab_frames(c.frame_size, tile_count);            // (up to kShortSlab frames: one)
-    size_t const slab_bytes = (size_t)O * NN * sizeof(float) * (c.bn ? 2 : 1);
-    while ((size_t)ceil_div(c.frame_size, slab) * slab_bytes > ((size_t)256 << 20) && slab < c.frame_size) { slab *= 2; }
+    // up to 256 MiB of partial sums; up to kShortSlab frames: one slab
+    size_t const slab_bytes = (size_t)O * NN * sizeof(float) * (c.bn ? 2 : 1), max_slabs = ((size_t)256 << 20) / slab_bytes;
+    int slab = bwd_slab_frames() > 0 ? ceil_div(bwd_slab_frames(), 256) * 256 : corner_slab_frames(c.frame_size, tile_count, (long long)max_slabs);
+    while ((size_t)ceil_div(c.frame_size, slab) > max_slabs && slab < c.frame_size) { slab *= 2; }
     int const slab_count = ceil_div(c.frame_size, slab);
     if ((long long)slab_count * tile_count > 0x7fffffffLL) { return fail("backward: grid too large"); }
     int const own_words = ceil_div(c.frame_size, 32) * 8;

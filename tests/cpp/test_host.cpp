@@ -15,6 +15,7 @@
 #include "bb/MaxPooling.h"
 #include "bb/UpSampling.h"
 #include "bb/Shuffle.h"
+#include "../../binarybrain_amd/csrc/launch_rules.hpp"
 #include "../../binarybrain_amd/csrc/tile_divisor.hpp"
 
 extern "C" int oracle_ReverseTable(int n, std::int32_t const *idx, int input_node_size, int output_node_size, std::int32_t *rev, int rev_cap);
@@ -279,6 +280,28 @@ int main(void)
             }
             check(0x7fffffffu);
         }
+    }
+    // slabs of the per-corner sums: never dearer than the best power of two, or than equal slabs that fill whole rounds of 512 workgroups, whatever the
+    // node count; within the number of slabs that the scratch memory holds
+    {
+        std::uint64_t state = 0x2545f4914f6cdd1dull;
+        auto draw = [&](int lo, int hi) { state ^= state << 13; state ^= state >> 7; state ^= state << 17; return lo + (int)((state >> 20) % (std::uint64_t)(hi - lo + 1)); };
+        auto check = [&](int nodes, int frames, long long max_slabs) {
+            int const tiles = bbhip::ceil_div(nodes, 4), slab = bbhip::corner_slab_frames(frames, tiles, max_slabs);
+            long long const cost = bbhip::corner_slab_cost(frames, tiles, slab);
+            bool ok = slab > 0 && slab % 256 == 0 && bbhip::ceil_div(frames, slab) <= max_slabs && (frames > 1024 || slab >= frames);
+            auto not_dearer = [&](long long than) { if ((frames + than - 1) / than <= max_slabs) { ok = ok && cost <= bbhip::corner_slab_cost(frames, tiles, than); } };
+            not_dearer(bbhip::ceil_div(frames, 256) * 256);
+            for (int power = 1024; power < frames && power <= 65536; power *= 2) { not_dearer(power); }
+            for (int rounds = 1; rounds <= 4; ++rounds) {
+                int const slabs = rounds * 512 / tiles, equal = slabs < 1 ? 0 : bbhip::ceil_div(bbhip::ceil_div(frames, slabs), 256) * 256;
+                if (equal >= 1024) { not_dearer(equal); }
+            }
+            if (!ok) { std::printf("%d nodes x %d frames, at most %lld slabs: %d\n", nodes, frames, max_slabs, slab); CHECK(!"corner_slab_frames"); }
+        };
+        int const sizes[][2] = {{4200, 65536}, {4200, 230400}, {4500, 65536}, {4200, 32768}, {2100, 230400}, {4200, 1 << 20}, {216, 230400}, {87, 94500}, {4096, 8192}, {1, 1}};
+        for (auto const &s : sizes) { check(s[0], s[1], 1 << 20); }
+        for (int i = 0; i < 20000; ++i) { check(draw(1, 1 << draw(0, 14)), draw(1, 1 << draw(0, 20)), 1 + draw(0, 1 << draw(0, 12))); }
     }
 
     std::printf("%s (%d failed checks)\n", g_fail ? "FAILED" : "OK", g_fail);
