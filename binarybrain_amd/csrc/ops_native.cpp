@@ -176,29 +176,13 @@ PyObject *wrapped(PyObject *, PyObject *const *args, Py_ssize_t n)
 }
 
 // ---- buffers -------------------------------------------------------------------------------------------------------------------
-// (what at::empty comes to for device tensors, without the dispatcher's passes)
+// (what at::empty comes to for device tensors, without the dispatcher's passes.  Every output has storage of its own, 0.6 us of host time each: one that a
+// program keeps must not keep the others of its call, be saved with them, or grow into them.)
 at::Tensor new_tensor(T like, at::IntArrayRef sizes, at::ScalarType type) { return at::Tensor(at::detail::empty_cuda(sizes, type, like.device(), std::nullopt)); }
 at::Tensor rows_f32(T like, int64_t rows, int64_t stride) { return new_tensor(like, {rows, stride}, at::kFloat); }
 at::Tensor rows_i32(T like, int64_t rows, int64_t words)  { return new_tensor(like, {rows, words}, at::kInt); }
 at::Tensor zeros_i32(T like, int64_t rows, int64_t words) { return at::zeros({rows, words}, like.options().dtype(at::kInt)); }
 at::Tensor line_f32(T like, int64_t n) { return new_tensor(like, {n}, at::kFloat); }
-
-// Several small outputs of one call in one allocation: 0.6 us of host time for each tensor more, 0.15 as a piece (offsets in bytes)
-struct Pieces {
-    at::Tensor whole;
-    int64_t used = 0;
-    static int64_t padded(int64_t bytes) { return (bytes + 255) & ~(int64_t)255; }
-    Pieces(T like, int64_t bytes) : whole(new_tensor(like, {bytes}, at::kByte)) {}
-    at::Tensor take(at::IntArrayRef sizes, at::ScalarType type)
-    {
-        auto impl = c10::make_intrusive<c10::TensorImpl>(c10::Storage(whole.storage()), c10::DispatchKeySet(c10::DispatchKey::CUDA),
-                                                         caffe2::TypeMeta::fromScalarType(type));
-        impl->set_sizes_contiguous(sizes);
-        impl->set_storage_offset(used / (int64_t)c10::elementSize(type));
-        used += padded(impl->numel() * (int64_t)c10::elementSize(type));
-        return at::Tensor(std::move(impl));
-    }
-};
 
 template <class E> E *data(T t) { return static_cast<E *>(t.data_ptr()); }
 template <class E> E *data(OptTensor t) { return t ? static_cast<E *>((*t).data_ptr()) : nullptr; }
@@ -318,8 +302,7 @@ differentiable_lut_forward_training(int n, T x, T idx, T W, int frames, T runnin
 {
     int const O = rows_of(idx), S = stride_of(x);
     at::Tensor y = rows_f32(x, O, S);
-    Pieces statistics(x, 2 * Pieces::padded(4 * (int64_t)O));
-    at::Tensor mean = statistics.take({O}, at::kFloat), rstd = statistics.take({O}, at::kFloat);
+    at::Tensor mean = line_f32(x, O), rstd = line_f32(x, O);
     if (hints) {
         hint_input(x, packed, holds, true);
         hint_tables(tables, false);
@@ -344,8 +327,7 @@ bit_differentiable_lut_forward_training(int n, T x, T idx, T W, int frames, T ru
 {
     int const O = rows_of(idx), S = stride_of(x);
     at::Tensor y = packed_output(out, x, O, S);
-    Pieces statistics(x, 2 * Pieces::padded(4 * (int64_t)O));
-    at::Tensor mean = statistics.take({O}, at::kFloat), rstd = statistics.take({O}, at::kFloat);
+    at::Tensor mean = line_f32(x, O), rstd = line_f32(x, O);
     if (hints) { hint_tables(tables, false); }
     if (clamp.on) {
         call(bbhip_bit_fp32_DifferentiableLutN_ForwardTrainingClampW, n, data<int const>(x), data<int>(y), data<int const>(idx), data<float>(W),
@@ -449,12 +431,10 @@ classifier_tail(T x, T idx, T t, int frames, float t_sum, bool input_binary, boo
     int const ch = rows_of(idx), n = stride_of(idx), S = stride_of(x), I = rows_of(x);
     require(t.size(1) == S, "classifier_tail: t must have the row pitch of x");
     require(frames >= 0, "classifier_tail: frames");
-    int64_t const rows = Pieces::padded(4 * (int64_t)ch * S), ints = Pieces::padded(4 * (int64_t)frames);
-    Pieces small(x, Pieces::padded(8 * (int64_t)frames) + (want_y + want_dy) * rows + 2 * want_accuracy * ints);
-    at::Tensor y, dy, accuracy, category, dx = rows_f32(x, I, S), loss = small.take({frames}, at::kDouble);
-    if (want_y)  { y = small.take({ch, S}, at::kFloat); }
-    if (want_dy) { dy = small.take({ch, S}, at::kFloat); }
-    if (want_accuracy) { accuracy = small.take({frames}, at::kInt); category = small.take({frames}, at::kInt); }
+    at::Tensor y, dy, accuracy, category, dx = rows_f32(x, I, S), loss = new_tensor(x, {frames}, at::kDouble);
+    if (want_y)  { y = rows_f32(x, ch, S); }
+    if (want_dy) { dy = rows_f32(x, ch, S); }
+    if (want_accuracy) { accuracy = new_tensor(x, {frames}, at::kInt); category = new_tensor(x, {frames}, at::kInt); }
     auto const f = [](at::Tensor const &a) { return a.defined() ? data<float>(a) : nullptr; };
     auto const i = [](at::Tensor const &a) { return a.defined() ? data<int>(a) : nullptr; };
     call(bbhip_fp32_ClassifierTail_ForwardBackward, data<float const>(x), f(y), data<float>(dx), data<int const>(idx), data<float const>(t), f(dy),

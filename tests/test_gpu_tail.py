@@ -248,7 +248,7 @@ def test_classifier_tail_limits(ops):
 
 @pytest.mark.parametrize("frames", [1, 7, 63, 64, 65, 1000])
 def test_small_outputs_share_no_memory(frames):
-    """outputs of one call that come from one allocation are apart, aligned and of their own size: each keeps its values while the others are overwritten"""
+    """outputs of one call are apart, aligned and of their own size: each keeps its values while the others are overwritten"""
     import torch
     from binarybrain_amd import ops, synth
     rng = np.random.default_rng(frames)
@@ -261,11 +261,45 @@ def test_small_outputs_share_no_memory(frames):
     W = torch.rand((5, 64), device="cuda")
     layer = ops.differentiable_lut_forward_training(6, x, torch.from_numpy(synth.wiring(rng, 21, 5)).cuda(), W, frames, torch.zeros(5, device="cuda"),
                                                     torch.ones(5, device="cuda"))
+    raw = lambda a: a.view(torch.uint8)          # (rows end in memory that no call writes: any bits, also those of no number)
     for outputs in ([o for o in tail if o is not None], list(layer)):
         kept = [o.clone() for o in outputs]
         for k, o in enumerate(outputs):
             assert o.is_contiguous() and o.data_ptr() % 256 == 0
             o.fill_(7)
-            assert all(torch.equal(a, b) for j, (a, b) in enumerate(zip(outputs, kept)) if j > k)
+            assert all(torch.equal(raw(a), raw(b)) for j, (a, b) in enumerate(zip(outputs, kept)) if j > k)
             assert bool((o == 7).all())
         assert all(bool((o == 7).all()) for o in outputs)
+
+
+@pytest.mark.parametrize("frames", [1, 65, 1000])
+def test_outputs_have_storage_of_their_own(frames):
+    """a program that keeps one output (the losses of a loop) keeps no other one of the call: its storage holds its own values and nothing else, it is saved
+    without the others, and it grows without running into them"""
+    import io
+    import torch
+    from binarybrain_amd import ops, synth
+    rng = np.random.default_rng(frames)
+    stride = synth.frame_stride_fp32(frames)
+    x = torch.rand((21, stride), device="cuda")
+    bits = torch.zeros((21, synth.frame_stride_bit(frames)), dtype=torch.int32, device="cuda")
+    idx = torch.arange(21, dtype=torch.int32, device="cuda").reshape(3, 7).contiguous()
+    t = torch.zeros((3, stride), device="cuda")
+    t[0] = 1.0
+    wiring = torch.from_numpy(synth.wiring(rng, 21, 5)).cuda()
+    W, rm, rv = torch.rand((5, 64), device="cuda"), torch.zeros(5, device="cuda"), torch.ones(5, device="cuda")
+    raw = lambda a: a.view(torch.uint8)
+    for outputs in (ops.classifier_tail(x, idx, t, frames, t_sum=float(frames), want_dy=True),
+                    ops.differentiable_lut_forward_training(6, x, wiring, W, frames, rm, rv),
+                    ops.bit_differentiable_lut_forward_training(6, bits, wiring, W, frames, rm, rv)):
+        outputs = [o for o in outputs if o is not None]
+        assert len({o.untyped_storage().data_ptr() for o in outputs}) == len(outputs)
+        for o in outputs:
+            assert o.storage_offset() == 0 and o.untyped_storage().nbytes() == o.numel() * o.element_size()
+        kept = [o.clone() for o in outputs]
+        for k, o in enumerate(outputs):
+            saved = io.BytesIO()
+            torch.save(o, saved)
+            assert saved.tell() < o.numel() * o.element_size() + 4096
+            o.resize_(o.numel() + 4096).fill_(7)
+            assert all(torch.equal(raw(a), raw(b)) for j, (a, b) in enumerate(zip(outputs, kept)) if j > k)
