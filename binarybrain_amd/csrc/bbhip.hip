@@ -766,37 +766,27 @@ int dispatch_dx_table(int quads, DxTableArgs const &t, hipStream_t st)
     return 0;
 }
 
-// Small layers on two-valued inputs whose backward pass is one launch (lut_corner_small_backward_kernel), 256 PASSES frames: what its wavefronts walk
-// one after another must be short, and what they do for every connection (the sums through the statistics) little in all.  Backward call alone,
-// microseconds, against two launches; links: connections, fan: the longest list.
-//   256 frames: 784 inputs x 1024 nodes (fan 18) 6.2 and 9.4, 1024 x 360 5.8 and 9.0, 784 x 6144 (fan 76) 16.1 and 18.5, 2001 x 3003 10.2 and 11.0;
-//               150 x 3000 (fan 155) 20.5 and 12.0
-//   512 frames: 300 x 300 (fan 14) 6.3 and 10.0, 784 x 1024 (4700 links) 8.8 and 9.4; 2000 x 2000 12.7 and 11.9, 400 x 2000 (fan 46) 14.5 and 12.5
-//   1024 frames: 360 x 70 5.9 and 8.8, 500 x 500 (3000 links) 9.0 and 10.8; 784 x 1024 12.1 and 11.3, 200 x 500 (fan 24) 10.8 and 9.6
-// Lists are shared by the wavefronts of a workgroup, except where there are many inputs with little to walk: 6144 x 1024 (256 frames, fan 8) 10.2
-// shared, 8.4 not, two launches 9.8; 4096 x 4096 (fan 17) 14.5, 13.5 and 13.3.
-bool small_corner_layer(BackwardCall const &c, int &passes, bool &share)
+// Small layers on two-valued inputs whose backward pass is one launch (lut_corner_small_backward_kernel): the wavefronts that walk an input's list (0: two
+// launches), by corner_small_waves
+int small_corner_layer(BackwardCall const &c)
 {
-    if (c.frame_size > kShortSlab || bwd_slab_frames() > 0 || dx_quads_env() != 0) { return false; }
+    if (c.frame_size > kShortSlab || bwd_slab_frames() > 0 || dx_quads_env() != 0) { return 0; }
     if ((long long)c.input_node_size * c.x_stride * 4 > 0xffffffffLL || (long long)c.output_node_size * c.frame_stride * 4 > 0xffffffffLL ||
-        (long long)c.output_node_size * (4 << c.n) > 0xffffffffLL) { return false; }                              // (32-bit offsets into whole buffers)
-    passes = c.frame_size <= 256 ? 1 : c.frame_size <= 512 ? 2 : 4;
-    int const fan = c.rev_stride - 1;
-    long long const links = (long long)c.output_node_size * c.n;
-    share = c.input_node_size <= (passes == 1 ? 2048 : 1536);
-    static_assert(8 <= kCornerSmallItems && 20 <= kCornerSmallItems, "the kernel holds a wavefront's items one per lane");
-    if (!share) { return passes == 1 && fan <= 8; }
-    return ceil_div(fan, kWavesPerBlk) <= (passes == 1 ? 20 : 16 / passes) && links * passes <= (passes == 1 ? 40000 : 12000);
+        (long long)c.output_node_size * (4 << c.n) > 0xffffffffLL) { return 0; }                                  // (32-bit offsets into whole buffers)
+    static_assert(kCornerSmallShare <= kCornerSmallItems, "the kernel holds a wavefront's items one per lane");
+    return corner_small_waves(c.n, c.bn, c.frame_size, c.input_node_size, c.output_node_size, c.rev_stride - 1);
 }
 
 template <int N, bool BN, bool QUADS>
-int launch_corner_small(CornerSmallArgs const &t, int passes, hipStream_t st)
+int launch_corner_small(CornerSmallArgs const &t, int waves, hipStream_t st)
 {
-    dim3 const grid(t.dx_blocks + ceil_div(t.sums.node_size, kWavesPerBlk));
+    dim3 const grid(t.dx_blocks + ceil_div(t.sums.node_size, waves)), block(waves * kWave);
     ScopedTimer tm(kTimeBackward, st);
-    if (passes == 1)      { launch((lut_corner_small_backward_kernel<N, BN, 1, QUADS>), grid, dim3(kBlock), 0, st, t); }
-    else if (passes == 2) { launch((lut_corner_small_backward_kernel<N, BN, 2, QUADS>), grid, dim3(kBlock), 0, st, t); }
-    else                  { launch((lut_corner_small_backward_kernel<N, BN, 4, QUADS>), grid, dim3(kBlock), 0, st, t); }
+    int const frames = t.sums.frame_size;
+    if (waves == kDxWaves)  { launch((lut_corner_small_backward_kernel<N, BN, 1, QUADS, kDxWaves>), grid, block, 0, st, t); }        // (up to 256 frames)
+    else if (frames <= 256) { launch((lut_corner_small_backward_kernel<N, BN, 1, QUADS, kWavesPerBlk>), grid, block, 0, st, t); }
+    else if (frames <= 512) { launch((lut_corner_small_backward_kernel<N, BN, 2, QUADS, kWavesPerBlk>), grid, block, 0, st, t); }
+    else                    { launch((lut_corner_small_backward_kernel<N, BN, 4, QUADS, kWavesPerBlk>), grid, block, 0, st, t); }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }
@@ -825,9 +815,7 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     if ((long long)slab_count * tile_count > 0x7fffffffLL) { return fail("backward: grid too large"); }
     int const own_words = ceil_div(c.frame_size, 32) * 8;
 
-    int passes = 0;
-    bool share = false;
-    bool const small = small_corner_layer(c, passes, share);
+    int const small = small_corner_layer(c);
 
     // the nodes' corner values: from the buffer that the caller kept from this step's forward call, else derived by the sums kernel (small layers:
     // by each wavefront that needs them)
@@ -871,10 +859,11 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
         t.inv_step = 1.0f / (s.fold.hi - s.fold.lo);
         DxArgs &d = t.dx;
         d.dx = c.dx; d.rev = c.rev; d.rev_stride = c.rev_stride; d.input_node_size = c.input_node_size; d.frame_size = c.frame_size; d.dx_stride = c.frame_stride;
-        d.split = share ? kWavesPerBlk : 0;
-        t.dx_blocks = share ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
-        return dy_quads ? (c.bn ? launch_corner_small<N, true, true>(t, passes, st) : launch_corner_small<N, false, true>(t, passes, st))
-                        : (c.bn ? launch_corner_small<N, true, false>(t, passes, st) : launch_corner_small<N, false, false>(t, passes, st));
+        d.split = small > 1 ? small : 0;
+        t.dx_blocks = d.split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
+        int const waves = d.split ? d.split : kWavesPerBlk;
+        return dy_quads ? (c.bn ? launch_corner_small<N, true, true>(t, waves, st) : launch_corner_small<N, false, true>(t, waves, st))
+                        : (c.bn ? launch_corner_small<N, true, false>(t, waves, st) : launch_corner_small<N, false, false>(t, waves, st));
     }
     if (dy_quads ? (c.bn ? launch_corner_backward<N, true, true>(s, slab_count, st) : launch_corner_backward<N, false, true>(s, slab_count, st))
                  : (c.bn ? launch_corner_backward<N, true, false>(s, slab_count, st) : launch_corner_backward<N, false, false>(s, slab_count, st))) { return 1; }

@@ -67,7 +67,7 @@ struct CornerSmallDxShared {            // a wavefront's LDS
     float4 part[PASSES][kWave];
 };
 
-// dx[input][all frames] by one wavefront (or, in split mode, the wavefronts of a workgroup), consumer by consumer in the reverse table's order.  A
+// dx[input][all frames] by one wavefront (or, in split mode, the WAVES wavefronts of a workgroup), consumer by consumer in the reverse table's order.  A
 // wavefront sees all frames of a consumer, so it forms the two sums that the gradient through the statistics needs (s0, s1 of
 // corner_backward_kernels.hpp) itself instead of waiting for a launch that does: as many times as the node has inputs, but side by side.
 // The lists are in registers (lane l: an item, its node's wiring and statistics), and the next item's rows are requested while one is evaluated, on
@@ -75,7 +75,7 @@ struct CornerSmallDxShared {            // a wavefront's LDS
 // Bound by latency: an item takes 0.45 us of a wavefront's time (256 frames; 0.75 and 1.1 with 512 and 1024), about 160 instructions that wait for one
 // another, a launch 4.5 to 5 us.  Backward call of 1024 inputs x 360 nodes x 256 frames 9.0 -> 5.8 us, 784 x 1024 9.4 -> 6.2, 360 x 70 x 1024
 // 8.8 -> 5.9 (the rule with both sides of the line: small_corner_layer).
-template <int N, bool BN, int PASSES, bool QUADS>
+template <int N, bool BN, int PASSES, bool QUADS, int WAVES>
 __device__ __forceinline__ void corner_small_dx_unit(CornerSmallArgs const &t, CornerSmallDxShared<N, BN, PASSES> *shared, int tile, int wave, int lane)
 {
     constexpr int NN = 1 << N;
@@ -87,7 +87,7 @@ __device__ __forceinline__ void corner_small_dx_unit(CornerSmallArgs const &t, C
     if (in >= a.input_node_size) { return; }                            // (workgroup-uniform in split mode)
     int const *const list = a.rev + (size_t)in * a.rev_stride;
     int t_begin, t_end;
-    dx_list_range<kWavesPerBlk>(list[0], share, t_begin, t_end);
+    dx_list_range<WAVES>(list[0], share, t_begin, t_end);
 
     // (byte offsets into the whole buffers, which the host keeps below 4 GiB here)
     struct Slots { int e; uint32_t row[N], dy; float mean, rstd; };
@@ -202,7 +202,7 @@ __device__ __forceinline__ void corner_small_dx_unit(CornerSmallArgs const &t, C
 #pragma unroll
         for (int p = 0; p < PASSES; ++p) {
 #pragma unroll
-            for (int w = 1; w < kWavesPerBlk; ++w) {
+            for (int w = 1; w < WAVES; ++w) {
                 float4 const o = shared[w].part[p][lane];
                 acc[p].x += o.x; acc[p].y += o.y; acc[p].z += o.z; acc[p].w += o.w;
             }
@@ -219,17 +219,18 @@ __device__ __forceinline__ void corner_small_dx_unit(CornerSmallArgs const &t, C
     }
 }
 
-template <int N, bool BN, int PASSES, bool QUADS>
-__global__ __launch_bounds__(kBlock) void lut_corner_small_backward_kernel(CornerSmallArgs t)
+// WAVES: wavefronts of a workgroup, that is nodes of one, or wavefronts that share an input's list
+template <int N, bool BN, int PASSES, bool QUADS, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void lut_corner_small_backward_kernel(CornerSmallArgs t)
 {
     constexpr int FORM = PASSES;                // (kSums256, kSums512, kSumsShort)
     using Sums = SumsShared<N, BN, FORM>;
     using Dx = CornerSmallDxShared<N, BN, PASSES>;
-    __shared__ __align__(16) unsigned char shared[kWavesPerBlk * (sizeof(Sums) > sizeof(Dx) ? sizeof(Sums) : sizeof(Dx))];
+    __shared__ __align__(16) unsigned char shared[WAVES * (sizeof(Sums) > sizeof(Dx) ? sizeof(Sums) : sizeof(Dx))];
     int const wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave)), lane = threadIdx.x & (kWave - 1);
     int const bid = blockIdx.x;
-    if (bid < t.dx_blocks) { corner_small_dx_unit<N, BN, PASSES, QUADS>(t, reinterpret_cast<Dx *>(shared), bid, wave, lane); return; }
-    int const node = (bid - t.dx_blocks) * kWavesPerBlk + wave;
+    if (bid < t.dx_blocks) { corner_small_dx_unit<N, BN, PASSES, QUADS, WAVES>(t, reinterpret_cast<Dx *>(shared), bid, wave, lane); return; }
+    int const node = (bid - t.dx_blocks) * WAVES + wave;
     if (node >= t.sums.node_size) { return; }
     corner_sums_unit<N, BN, FORM, QUADS>(t.sums, reinterpret_cast<Sums *>(shared)[wave], node, 0, lane);
 }

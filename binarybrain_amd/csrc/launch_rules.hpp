@@ -38,4 +38,38 @@ inline int corner_slab_frames(int frame_size, int tile_count, long long max_slab
     return (int)best;
 }
 
+// Wavefronts that walk an input's list in the one-launch backward pass of a small layer on two-valued inputs: 1, or 4 or 16 that share it, or 0: two
+// launches.  What its wavefronts walk one after another must be short: an item costs 0.45 us, 0.65 where the wavefront also derives the node's corner
+// values (no prepared tables); and what they do for every connection (the sums through the statistics) little in all.  The rule does not ask for prepared
+// tables: a hint changes no bit of a result, and these forms add in different orders.  Device time of the backward call of a batch-norm layer of six
+// inputs per node, with prepared tables / without, in microseconds; fan: the longest list.
+//   up to 256 frames                         4 wavefronts    16              two launches
+//   784 inputs x 1024 nodes (fan 19)         5.8 /  6.9       -              7.8 /  8.4
+//   26 x 104 (fan 35)                        6.7 /  8.2      5.3 /  6.2      7.4 /  7.8
+//   347 x 1643 (fan 44)                      8.3 / 10.5      9.2 / 11.3      9.1 /  9.7
+//   207 x 1495 (fan 63)                     10.3 / 13.1      8.9 / 10.3      8.7 /  9.5
+//   645 x 4947 (fan 69)                     14.0 / 18.4     18.0 / 22.3     13.9 / 15.9
+//   650 x 4818, four inputs (fan 49)        10.1 / 11.8     13.9 / 15.8     13.4 / 14.3
+//   784 x 6144, plain (fan 71)              12.1 / 17.2     14.0 / 16.9     15.9 / 18.3
+//   47 x 469 (fan 76)                       11.7 / 14.9      7.7 /  9.7      8.6 /  9.0 (one launch less for the host)
+//   34 x 598 (fan 129)                      18.4 / 23.9     10.3 / 13.7      9.7 / 10.3
+//   512 frames: 300 x 300 (fan 15) 6.2 / 6.9 with four, 10.3 / 10.8 in two; 784 x 1024 (fan 19) 8.5 / 9.6 and 9.1 / 9.7
+//   1024 frames: 360 x 70 (fan 6) 4.5 / 4.8 and 7.3 / 7.6, 500 x 500 (fan 16) 8.7 / 9.3 and 9.6 / 10.0
+// Many inputs with little to walk: a wavefront each.  6144 x 1024 (256 frames, fan 6) 7.1 / 8.8, shared 9.2 / 10.0, two launches 8.4 / 8.9.
+constexpr int kCornerSmallShare = 20;           // items of a list that a wavefront takes at most
+inline int corner_small_waves(int n, bool batch_norm, int frame_size, int input_node_size, int node_size, int max_fan)
+{
+    int const items = ceil_div(max_fan, 4);
+    long long const links = (long long)node_size * n;
+    if (frame_size > 256) {
+        int const passes = frame_size <= 512 ? 2 : 4;
+        return (input_node_size <= 1536 && items <= 16 / passes && links * passes <= 12000) ? 4 : 0;
+    }
+    if (input_node_size > 2048) { return max_fan <= 8 ? 1 : 0; }
+    if (items > kCornerSmallShare || links > 40000) { return 0; }
+    // (two launches take longer as there is more to do in all)
+    if (input_node_size <= 256) { return items <= 8 + links / 6000 ? 4 : 16; }
+    return items <= (!batch_norm ? 13 : n >= 5 ? 9 : 12) + links / 6000 ? 4 : 0;
+}
+
 }  // namespace bbhip

@@ -54,3 +54,36 @@ def test_small_backward(n, shape):
     dW = torch.zeros_like(d_W)
     dx = ops.bit_stochastic_lut_backward(n, d_xb, d_dy, d_idx, d_W, dW, F, rev)
     assert_bwd(host(dx)[:, :F], want_plain[0][:, :F], "plain dx"); assert_bwd(host(dW), want_plain[1], "plain dW")
+
+
+@pytest.mark.parametrize("frames,pitch", [(1, 1), (63, 63), (64, 0), (255, 255), (256, 0)])
+def test_lists_shared_by_sixteen_wavefronts(frames, pitch):
+    """few inputs with long lists: 0, 1, 15, 16, 17, 77, 78 and 80 consumers, so that wavefronts of one list have none, one or five items"""
+    import torch
+    from binarybrain_amd import ops
+    n, counts = 6, [0, 1, 15, 16, 17, 80, 77, 80, 78, 80, 0, 80, 80, 80]
+    I, O, F = len(counts), sum(counts) // n, frames
+    assert sum(counts) == O * n
+    S, rng = pitch or synth.frame_stride_fp32(F), np.random.default_rng(frames)
+    slots = np.repeat(np.arange(I, dtype=np.int32), counts)
+    idx = np.ascontiguousarray(rng.permutation(slots).reshape(O, n)); W = synth.lut_tables(rng, O, n)
+    x = np.zeros((I, S), np.float32); x[:, :F] = rng.random((I, F)) > 0.5
+    xb = np.zeros((I, synth.frame_stride_bit(F)), np.int32)
+    xb[:, :(F + 31) // 32] = synth.pack_bits(x[:, :F].astype(np.uint8), (F + 31) // 32)
+    dy = synth.normal_frames(rng, O, F, S)
+    _, mean, rstd, _, _ = oracle.differentiable_lut_forward_training(n, x, idx, W, F, np.zeros(O, np.float32), np.ones(O, np.float32))
+    want_bn = oracle.differentiable_lut_backward(n, x, dy, idx, W, F, mean, rstd)
+    want_plain = oracle.stochastic_lut_backward(n, x, dy, idx, W, F, input_binary=True, simd=False)
+    d_xb, d_dy, d_idx, d_W = dev(xb), dev(dy), dev(idx), dev(W)
+    rev = ops.reverse_table(d_idx, I)
+    dW = torch.zeros_like(d_W)
+    dx = ops.bit_stochastic_lut_backward(n, d_xb, d_dy, d_idx, d_W, dW, F, rev)
+    assert_bwd(host(dx)[:, :F], want_plain[0][:, :F], "plain dx"); assert_bwd(host(dW), want_plain[1], "plain dW")
+    tables = ops.prepared_tables_buffer(n, O)
+    ops.bit_differentiable_lut_forward_training(n, d_xb, d_idx, d_W, F, dev(np.zeros(O, np.float32)), dev(np.ones(O, np.float32)), tables=tables)
+    for t in (tables, None):
+        dW = torch.zeros_like(d_W)
+        dx = ops.bit_differentiable_lut_backward(n, d_xb, d_dy, d_idx, d_W, dW, F, dev(mean), dev(rstd), rev, tables=t)
+        assert not host(dx)[[0, 10], :F].any()
+        if F > 1:                       # (a single frame is its own mean: rstd is that of rounding, and the gradient through it has no digits)
+            assert_bwd(host(dx)[:, :F], want_bn[0][:, :F], "dx"); assert_bwd(host(dW), want_bn[1], "dW")
