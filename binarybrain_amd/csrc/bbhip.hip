@@ -893,6 +893,7 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     int const in_tiles = split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
     if ((long long)d.chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
     d.tiles = make_tile_divisor(in_tiles); d.split = split;
+    d.in_turn = dx_items_in_turn(c.bn, (long long)d.chunk_count * in_tiles, c.rev_stride - 1);
     t.dx_quads = (c.frame_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(c.dx) & 15u) == 0) ? 1 : 0;
     t.own = own; t.own_stride = own_words; t.node_size = O; t.V = V; t.node_consts = consts; t.inv_step = 1.0f / (s.fold.hi - s.fold.lo);
     t.discard = s.fold.discard; t.call = s.fold.call;

@@ -448,7 +448,7 @@ __global__ __launch_bounds__(WAVES * kWave) void lut_dx_table_kernel(DxTableArgs
     int const fan = list[0];
     uint32_t const discard_word = BN ? *(const_word *)t.discard : 0u;   // (on the way with the list's length)
     int first, step, items;
-    dx_list_steps<WAVES>(fan, share, first, step, items);
+    dx_list_steps<WAVES>(a.in_turn != 0, fan, share, first, step, items);
     list += 1 + first;
     int const f_lane = ck * kPass + 4 * lane;
     uint32_t const dy_bytes = (uint32_t)(t.node_size - 1) * (uint32_t)a.dy_stride * 4u + quad_row_bytes(a.frame_size, true);

@@ -72,4 +72,17 @@ inline int corner_small_waves(int n, bool batch_norm, int frame_size, int input_
     return items <= (!batch_norm ? 13 : n >= 5 ? 9 : 12) + links / 6000 ? 4 : 0;
 }
 
+// Whether the sixteen wavefronts that share an input's list in lut_dx_table_kernel take its items in turn (they then walk the nodes together, and rows that
+// outgrow an L2 come from behind it once) or consecutive ones.  A launch of fewer workgroups than compute units leaves the L2s room; what counts there is that
+// an item's list entry, row and index are requested one item ahead only, and consecutive entries of a long list share a cache line.  Backward call, plain,
+// in turn and consecutive: 12 inputs x 3623 nodes x 297 frames (24 workgroups, lists of 1840) 57.2 and 48.1 us, 17 x 2078 x 1839 (136, 653) 28.1 and 24.2,
+// 22 x 5774 x 1449 (132, 1645) 63.7 and 55.1; 12 x 707 x 108
+// (12, 388) 13.9 and 14.4, 60 x 5776 x 3633 (900, 621) 77.9 and 103.0.  The longer items of
+// batch-norm layers hide more: 14 x 2990 x 1129 (70, 1361) 57.8 and 53.2, 11 x 2343 x 127 (11, 897) 31.5 and 33.8, 35 x 5912 x 5652 (805) 103.7 and 151.3.
+inline bool dx_items_in_turn(bool batch_norm, long long workgroups, int max_fan)
+{
+    if (workgroups >= 256) { return true; }
+    return batch_norm ? workgroups < 64 || max_fan < 700 : max_fan < 400;
+}
+
 }  // namespace bbhip

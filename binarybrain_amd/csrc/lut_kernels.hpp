@@ -1251,11 +1251,13 @@ struct DxArgs {
     int   chunk, chunk_count;
     TileDivisor tiles;
     float bias;
-    // split != 0: the wavefronts of a workgroup share ONE input node, every fourth (sixteenth) item of its work list each; their sums are
+    // split != 0: the wavefronts of a workgroup share ONE input node, every fourth (sixteenth) item of its work list each (in_turn; else consecutive
+    // items); their sums are
     // added in wavefront order through LDS.  For layers with few input nodes and long lists (784 inputs feeding 6144 nodes:
     // 47 consumers each), where one wavefront per (input, unit) leaves most of the device idle behind a long serial walk.
     // tiles then counts input nodes, not groups of four.
     int   split;
+    int   in_turn;
     // the last fin_blocks workgroups of the launch fold the table-gradient partial sums into dW (dw_finalize_block)
     float const *fin_partial;
     float       *fin_dW;
@@ -1401,16 +1403,23 @@ __device__ __forceinline__ void dx_list_share(DxArgs const &a, int tile, int wav
 template <int WAVES>
 __device__ __forceinline__ void dx_list_range(int cnt, int share, int &t_begin, int &t_end)
 {
-    t_begin = (share < 0) ? 0   : (cnt * share) / WAVES;
-    t_end   = (share < 0) ? cnt : (cnt * (share + 1)) / WAVES;
+    t_begin = (share < 0) ? 0   : (int)((long long)cnt * share / WAVES);
+    t_end   = (share < 0) ? cnt : (int)((long long)cnt * (share + 1) / WAVES);
 }
 
 // The same with every WAVES-th item for each, so that the wavefronts of a launch walk the nodes together, at one place instead of WAVES: rows that
 // outgrow an L2 come from behind it once.  Training steps of 100 inputs x 8000 nodes x 4000 frames of packed bits 154 -> 128 us, 300 x 8000 x 2000 97 -> 83,
 // classifier 784-6144-1024 at 1024 frames 95.6 -> 92.5.
 template <int WAVES>
-__device__ __forceinline__ void dx_list_steps(int cnt, int share, int &t_first, int &t_step, int &items)
+__device__ __forceinline__ void dx_list_steps(bool in_turn, int cnt, int share, int &t_first, int &t_step, int &items)
 {
+    if (!in_turn) {
+        int t_end;
+        dx_list_range<WAVES>(cnt, share, t_first, t_end);
+        t_step = 1;
+        items  = t_end - t_first;
+        return;
+    }
     t_first = (share < 0) ? 0 : share;
     t_step  = (share < 0) ? 1 : WAVES;
     items   = (share < 0) ? cnt : (cnt - share + WAVES - 1) / WAVES;
@@ -1486,7 +1495,7 @@ __global__ __launch_bounds__(WAVES * kWave) void lut_dx_kernel(DxArgs a)
 
     int const cnt = a.rev[(size_t)in * a.rev_stride];
     int t_first, t_step, items;
-    dx_list_steps<WAVES>(cnt, share, t_first, t_step, items);
+    dx_list_steps<WAVES>(true, cnt, share, t_first, t_step, items);
     // The term table is read through the constant address space: its wave-uniform loads stay scalar loads wherever
     // they are placed relative to the stores of this kernel (the table is written by an earlier kernel).
     typedef __attribute__((address_space(4))) int const const_int;

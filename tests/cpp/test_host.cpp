@@ -338,6 +338,18 @@ int main(void)
         }
     }
 
+    // items of shared lists in turn or one after another, where both were measured (backward calls, microseconds): at most a twentieth slower than the faster
+    {
+        struct { bool batch_norm; int workgroups, fan; double in_turn, consecutive; } const rows[] = {
+            {false, 24, 1840, 57.2, 48.1}, {false, 34, 1128, 39.1, 34.6}, {false, 54, 973, 33.4, 29.6},  {false, 58, 1031, 36.9, 32.7},  {false, 70, 948, 36.1, 31.7},
+            {false, 132, 1645, 63.7, 55.1}, {false, 136, 653, 28.1, 24.2}, {false, 12, 388, 13.9, 14.4}, {false, 900, 621, 77.9, 103.0}, {false, 286, 447, 27.2, 29.9},
+            {true, 70, 1361, 57.8, 53.2},  {true, 11, 897, 31.5, 33.8},   {true, 805, 889, 103.7, 151.3}, {true, 640, 1280, 126.6, 173.2}, {true, 42, 524, 21.6, 23.0}};
+        for (auto const &r : rows) {
+            double const taken = bbhip::dx_items_in_turn(r.batch_norm, r.workgroups, r.fan) ? r.in_turn : r.consecutive;
+            if (taken > 1.05 * std::min(r.in_turn, r.consecutive)) { std::printf("%d workgroups, lists of %d\n", r.workgroups, r.fan); CHECK(!"dx_items_in_turn"); }
+        }
+    }
+
     std::printf("%s (%d failed checks)\n", g_fail ? "FAILED" : "OK", g_fail);
     return g_fail ? 1 : 0;
 }

@@ -182,3 +182,9 @@ def test_shared_lists_of_real_valued_inputs(n, shape):
     d_idx, dW = dev(idx), dev(np.zeros_like(W))
     dx = ops.stochastic_lut_backward(n, dev(x), dev(dy), d_idx, dev(W), dW, F, ops.reverse_table(d_idx, I))
     assert_bwd(host(dx)[:, :F], dx_ref[:, :F], "dx"); assert_bwd(host(dW), dW_ref, "dW")
+
+
+# lists of 400 items and more in fewer workgroups than compute units, whose wavefronts take consecutive items: plain layers, and (the last two) batch-norm
+@pytest.mark.parametrize("n, shape", [(6, (8, 560, 300)), (3, (7, 1000, 70)), (6, (40, 4750, 300)), (5, (64, 9100, 33))])
+def test_long_lists_in_few_workgroups(n, shape):
+    test_corner_backward(n, shape + (0,))
