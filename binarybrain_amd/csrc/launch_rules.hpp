@@ -51,6 +51,7 @@ inline int corner_slab_frames(int frame_size, int tile_count, long long max_slab
 //   645 x 4947 (fan 69)                     14.0 / 18.4     18.0 / 22.3     13.9 / 15.9
 //   650 x 4818, four inputs (fan 49)        10.1 / 11.8     13.9 / 15.8     13.4 / 14.3
 //   784 x 6144, plain (fan 71)              12.1 / 17.2     14.0 / 16.9     15.9 / 18.3
+//   149 x 2247, three inputs (fan 66)        9.8 / 11.2      6.5 /  7.4      9.4 /  9.7
 //   47 x 469 (fan 76)                       11.7 / 14.9      7.7 /  9.7      8.6 /  9.0 (one launch less for the host)
 //   34 x 598 (fan 129)                      18.4 / 23.9     10.3 / 13.7      9.7 / 10.3
 //   512 frames: 300 x 300 (fan 15) 6.2 / 6.9 with four, 10.3 / 10.8 in two; 784 x 1024 (fan 19) 8.5 / 9.6 and 9.1 / 9.7
@@ -68,7 +69,7 @@ inline int corner_small_waves(int n, bool batch_norm, int frame_size, int input_
     if (input_node_size > 2048) { return max_fan <= 8 ? 1 : 0; }
     if (items > kCornerSmallShare || links > 40000) { return 0; }
     // (two launches take longer as there is more to do in all)
-    if (input_node_size <= 256) { return items <= 8 + links / 6000 ? 4 : 16; }
+    if (input_node_size <= (batch_norm && n >= 5 ? 128 : 256)) { return items <= 8 + links / 6000 ? 4 : 16; }
     return items <= (!batch_norm ? 13 : n >= 5 ? 9 : 12) + links / 6000 ? 4 : 0;
 }
 
