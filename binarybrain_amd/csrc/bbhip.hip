@@ -736,8 +736,10 @@ int launch_corner_backward(CornerSumsArgs const &s, int slab_count, hipStream_t 
     {
         ScopedTimer tm(kTimeBackward, st);
         dim3 const grid(s.slab_count * s.tiles.count);
-        if (N >= 5 && slab_count == 1 && s.frame_size <= kShortSlab) { launch((lut_corner_sums_kernel<N, BN, (N >= 5 ? kSumsShort : kSumsLong), QUADS>), grid, dim3(kBlock), 0, st, s); }
-        else { launch((lut_corner_sums_kernel<N, BN, kSumsLong, QUADS>), grid, dim3(kBlock), 0, st, s); }
+        SumsForm const form = corner_sums_form(s.frame_size, slab_count);
+        if (form == kSumsShort)      { launch((lut_corner_sums_kernel<N, BN, kSumsShort, QUADS>), grid, dim3(kBlock), 0, st, s); }
+        else if (form == kSumsBlock) { launch((lut_corner_sums_kernel<N, BN, kSumsBlock, QUADS>), grid, dim3(kBlock), 0, st, s); }
+        else                         { launch((lut_corner_sums_kernel<N, BN, kSumsLong, QUADS>), grid, dim3(kBlock), 0, st, s); }
     }
     BBHIP_LAUNCH_CHECK();
     if (slab_count > 1) {

@@ -76,16 +76,14 @@ __device__ __forceinline__ void corner_fold(CornerFoldArgs const &a, CornerFoldI
     if (lane < NN) { a.dW[(size_t)node * NN + lane] = a.overwrite ? G : q.dW + G; }
 }
 
-// How a wavefront adds up the frames of a node (see lut_corner_sums_kernel): kSumsLong any number of frames in blocks of 2048; the others up to
-// 256, 512 and 1024 frames, all of them requested at once
-enum SumsForm : int { kSumsLong = 0, kSums256 = 1, kSums512 = 2, kSumsShort = 4 };
-constexpr int kShortSlab = 1024;
+// How a wavefront adds up the frames of a node (SumsForm, see lut_corner_sums_kernel)
 template <int N, bool BN, int FORM>
 struct SumsTraits {
     static constexpr int  NN = 1 << N;
     static constexpr bool kLoop = FORM == kSumsLong;
-    // (with few corners the atomics that count them collide, and the plain form has little to keep anyway)
-    static constexpr bool kAtomics = !kLoop && N >= 5, kCountSets = BN && !kAtomics, kCountFrames = BN && kAtomics;
+    // (with few corners the atomics that count them collide, and the plain form has little to keep anyway; over 2048 frames the chains of columns that
+    // two lanes share would be longer: rms error of dW, inputs set in 98 of 100 frames, 9.4e-8 instead of 7.0e-8)
+    static constexpr bool kAtomics = !kLoop && N >= 5 && FORM != kSumsBlock, kCountSets = BN && !kAtomics, kCountFrames = BN && kAtomics;
     static constexpr int  kPasses = kLoop ? 8 : FORM;
     static constexpr int  kColumns = !kAtomics ? kWave : FORM == kSums256 ? 16 : 32;
 };
@@ -173,9 +171,10 @@ __device__ __forceinline__ auto row_sum(V4 const *block, int lane)
 // 27.8 -> 23.0, 216 x 230400 65 -> 57 (4.4 TB/s of dy and indices).
 // QUADS: rows of dy hold whole groups of four frames.
 // The statistics and table-gradient launches that it replaces took 53 + 141 us for 216 nodes x 230400 frames, 31 + 106 for 4096 x 8192.
-// SHORT: up to kShortSlab frames in one slab.  Such a launch is a chain of latencies, so what counts is how many wavefronts share a compute unit: two
-// lanes share a column of bins (they add in turn), and the corners are counted by integer atomics (one instruction per step, and nothing to add up).
-// 6144 nodes x 1024 frames 20.5 -> 13.6 us, 6000 x 100 17.4 -> 9.6 us; four lanes per column measured the same or slower.
+// kSumsShort: up to kShortSlab frames in one slab.  Such a launch is a chain of latencies, so what counts is how many wavefronts share a compute unit: for five
+// and six inputs two lanes share a column of bins (they add in turn), and the corners are counted by integer atomics (one instruction per step, and nothing
+// to add up).  6144 nodes x 1024 frames 20.5 -> 13.6 us, 6000 x 100 17.4 -> 9.6 us; four lanes per column measured the same or slower.
+// kSumsBlock: up to 2048 frames, a column for each lane (corner_sums_form has both sides of the lines).
 template <int N, bool BN, int FORM, bool QUADS>
 __device__ __forceinline__ void corner_sums_unit(CornerSumsArgs const &a, SumsShared<N, BN, FORM> &sh, int node, int sl, int lane)
 {

@@ -86,4 +86,17 @@ inline bool dx_items_in_turn(bool batch_norm, long long workgroups, int max_fan)
     return batch_norm ? workgroups < 64 || max_fan < 700 : max_fan < 400;
 }
 
+// How a wavefront of lut_corner_sums_kernel adds up a node's frames (see there): in blocks of 2048 whose next one is requested ahead, or all frames of one slab
+// requested at once: 256, 512, 1024 (kSumsShort) or 2048 (kSumsBlock) of them.  Where a slab ends with its first block, the requests ahead and the
+// registers that they take are for nothing.  Sums launch, in blocks and at once: 2932 inputs x 3358 nodes x 489 frames, three inputs, rows of 489:
+// 11.2 and 8.2 us; 296 x 6754 x 747, two inputs, rows of 747: 15.6 and 11.1; 141 x 5121 x 82, two: 8.7 and 8.0; 126 x 4657 x 1981, four: 16.1 and
+// 15.2; 307 x 3081 x 1140, five: 13.7 and 13.3; 67 x 5667 x 1696, five: 20.3 and 18.4; six inputs, 1638 x 5110 x 1045: 21.7 and 21.0, 111 x 5234 x 1928: 25.3
+// and 24.8.
+enum SumsForm : int { kSumsLong = 0, kSums256 = 1, kSums512 = 2, kSumsShort = 4, kSumsBlock = 8 };
+constexpr int kShortSlab = 1024, kBlockSlab = 2048;
+constexpr SumsForm corner_sums_form(int frame_size, int slab_count)
+{
+    return (slab_count > 1 || frame_size > kBlockSlab) ? kSumsLong : frame_size <= kShortSlab ? kSumsShort : kSumsBlock;
+}
+
 }  // namespace bbhip

@@ -350,6 +350,22 @@ int main(void)
         }
     }
 
+    // per-corner sums of one slab: in blocks requested ahead, or all frames at once, where both were measured (sums launch, microseconds)
+    {
+        struct { int frames; double blocks, at_once; } const rows[] = {
+            {489, 11.2, 8.2}, {747, 15.6, 11.1}, {82, 8.7, 8.0}, {150, 10.7, 8.7}, {1981, 16.1, 15.2}, {1140, 13.7, 13.3}, {1696, 20.3, 18.4}, {102, 23.9, 13.3},
+            {1008, 25.3, 16.9}, {911, 13.8, 11.8}, {1045, 21.7, 21.0}};
+        for (auto const &r : rows) {
+            bool const blocks = bbhip::corner_sums_form(r.frames, 1) == bbhip::kSumsLong;
+            if ((blocks ? r.blocks : r.at_once) > std::min(r.blocks, r.at_once)) { std::printf("%d frames\n", r.frames); CHECK(!"corner_sums_form"); }
+        }
+        for (int frames = 1; frames <= 5000; ++frames) {        // (what does not fit the form that is taken would be left out of the sums)
+            int const form = bbhip::corner_sums_form(frames, 1);
+            CHECK(form == bbhip::kSumsLong || frames <= form * 256);
+            CHECK(bbhip::corner_sums_form(frames, 2) == bbhip::kSumsLong);
+        }
+    }
+
     std::printf("%s (%d failed checks)\n", g_fail ? "FAILED" : "OK", g_fail);
     return g_fail ? 1 : 0;
 }

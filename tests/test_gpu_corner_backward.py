@@ -188,3 +188,10 @@ def test_shared_lists_of_real_valued_inputs(n, shape):
 @pytest.mark.parametrize("n, shape", [(6, (8, 560, 300)), (3, (7, 1000, 70)), (6, (40, 4750, 300)), (5, (64, 9100, 33))])
 def test_long_lists_in_few_workgroups(n, shape):
     test_corner_backward(n, shape + (0,))
+
+
+# the largest frame counts of the forms that request all frames at once, one more, rows that hold no whole groups of four; enough nodes for every wavefront
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 6])
+@pytest.mark.parametrize("shape", [(30, 33, 1024, 0), (30, 33, 1023, 1023), (30, 33, 1025, 1025), (30, 33, 2048, 0), (9, 700, 60, 0), (1600, 41, 700, 703)])
+def test_sums_of_one_slab(n, shape):
+    test_corner_backward(n, shape)
