@@ -20,6 +20,9 @@ inline long long corner_slab_cost(int frame_size, int tile_count, long long fram
 // such slabs (2100 nodes two or three, 4200 nodes none), and over many frames more rounds of shorter slabs leave less of the device idle in the last one:
 // backward call of 512 inputs x 4200 nodes x 65536 frames 1061 us in one slab and 1012 in eight, 4200 x 4200 x 32768 711 and 693, 512 x 4200 x 230400
 // 3789 and 3668; 512 x 2100 x 230400 1651 in three slabs, 1628 in 29.
+// Several slabs have to promise more than 4 % over one, since the figures above are no better than that: 64 inputs x 2666 nodes x 8646 frames, promised 0.7 %,
+// 58.3 us in one slab and 62.5 in two (with batch-norm and six inputs 75.3 and 81.6), 2795 x 10066, promised 3 %, 79.3 and 83.9; 89 x 4352, promised 5 %,
+// 11.5 and 11.0 in five.
 inline int corner_slab_frames(int frame_size, int tile_count, long long max_slabs)
 {
     long long const whole = (long long)ceil_div(frame_size, 256) * 256;
@@ -35,6 +38,7 @@ inline int corner_slab_frames(int frame_size, int tile_count, long long max_slab
         consider(frames < 1024 ? 1024 : frames);
     }
     for (long long frames = 1024; frames < frame_size; frames *= 2) { consider(frames); }
+    if (corner_slab_cost(frame_size, tile_count, best) * 25 > corner_slab_cost(frame_size, tile_count, whole) * 24) { best = whole; }
     return (int)best;
 }
 
