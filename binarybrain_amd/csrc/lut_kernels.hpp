@@ -1413,16 +1413,20 @@ __device__ __forceinline__ void dx_list_range(int cnt, int share, int &t_begin, 
 template <int WAVES>
 __device__ __forceinline__ void dx_list_steps(bool in_turn, int cnt, int share, int &t_first, int &t_step, int &items)
 {
-    if (!in_turn) {
+    t_first = 0;
+    t_step  = 1;
+    items   = cnt;
+    if (share < 0) { return; }                  // (a branch: a wavefront with a short list of its own is mostly what comes before its first term)
+    if (in_turn) {
+        t_first = share;
+        t_step  = WAVES;
+        items   = (cnt - share + WAVES - 1) / WAVES;
+    }
+    else {
         int t_end;
         dx_list_range<WAVES>(cnt, share, t_first, t_end);
-        t_step = 1;
-        items  = t_end - t_first;
-        return;
+        items = t_end - t_first;
     }
-    t_first = (share < 0) ? 0 : share;
-    t_step  = (share < 0) ? 1 : WAVES;
-    items   = (share < 0) ? cnt : (cnt - share + WAVES - 1) / WAVES;
 }
 
 // ... and the end of a pass: the lane's U sums go to dx — directly, or in split mode added over the workgroup's wavefronts
