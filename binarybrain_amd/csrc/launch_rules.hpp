@@ -7,11 +7,13 @@ inline int ceil_div(int a, int b) { return a / b + (a % b != 0); }      // (no s
 
 // What a launch of the per-corner sums costs in slabs of `frames` frames, in frames' worth of a workgroup: ceil(workgroups / 512) rounds of resident workgroups
 // (two per compute unit: 64 KB of bins each), a unit costs its frames plus about 1024 frames' worth of set-up and closing sums, and more than one slab per
-// node needs the fold launch (about 3072 frames' worth on top).
+// node needs the fold launch (about 2700 frames' worth on top, and 2.5 for each node: a workgroup each).  1000 frames' worth is about 1.25 us.  Several slabs
+// against one, promised with 3072 on top for any node count and measured: 64 inputs x 2666 nodes x 8646 frames, five per node, 0.2 us less and 4.2 more (58.3 us in
+// one slab), 2795 x 10066 0.8 less and 4.5 more (79.3), 1420 x 31338 3.0 less and 3.6 more (117.7); 24 x 4223 0.2 and 0.6 less (14.7).
 inline long long corner_slab_cost(int frame_size, int tile_count, long long frames)
 {
     long long const slabs = (frame_size + frames - 1) / frames, rounds = (slabs * tile_count + 511) / 512;
-    return rounds * ((frames < frame_size ? frames : frame_size) + 1024) + (slabs > 1 ? 3072 : 0);
+    return rounds * ((frames < frame_size ? frames : frame_size) + 1024) + (slabs > 1 ? 2700 + 10LL * tile_count : 0);
 }
 
 // Frames per unit of the per-corner sums, in at most max_slabs slabs: the cheapest of one slab, the equal slabs that fill one to four rounds, and
@@ -20,9 +22,6 @@ inline long long corner_slab_cost(int frame_size, int tile_count, long long fram
 // such slabs (2100 nodes two or three, 4200 nodes none), and over many frames more rounds of shorter slabs leave less of the device idle in the last one:
 // backward call of 512 inputs x 4200 nodes x 65536 frames 1061 us in one slab and 1012 in eight, 4200 x 4200 x 32768 711 and 693, 512 x 4200 x 230400
 // 3789 and 3668; 512 x 2100 x 230400 1651 in three slabs, 1628 in 29.
-// Several slabs have to promise more than 4 % over one, since the figures above are no better than that: 64 inputs x 2666 nodes x 8646 frames, promised 0.7 %,
-// 58.3 us in one slab and 62.5 in two (with batch-norm and six inputs 75.3 and 81.6), 2795 x 10066, promised 3 %, 79.3 and 83.9; 89 x 4352, promised 5 %,
-// 11.5 and 11.0 in five.
 inline int corner_slab_frames(int frame_size, int tile_count, long long max_slabs)
 {
     long long const whole = (long long)ceil_div(frame_size, 256) * 256;
@@ -38,7 +37,6 @@ inline int corner_slab_frames(int frame_size, int tile_count, long long max_slab
         consider(frames < 1024 ? 1024 : frames);
     }
     for (long long frames = 1024; frames < frame_size; frames *= 2) { consider(frames); }
-    if (corner_slab_cost(frame_size, tile_count, best) * 25 > corner_slab_cost(frame_size, tile_count, whole) * 24) { best = whole; }
     return (int)best;
 }
 
