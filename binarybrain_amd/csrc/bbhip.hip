@@ -183,15 +183,14 @@ int dx_pass_steps_env(void)   { static int v = env_int("BBHIP_DX_STEPS", 0); ret
 // leave the launch with fewer than 4096 workgroups and the lists are long enough to share, sixteen where with four the launch
 // would still have less than two wavefronts per SIMD (the wavefronts walk the nodes together, each taking every fourth or sixteenth item of its list:
 // packed training steps of 40 inputs x 8000 nodes x 4000 frames 140 us with sixteen and 170 with four, 32 x 2000 x 3000 37 and 53; with more workgroups
-// four are better: 100 x 8000 x 4000 128 and 148).  real_valued: lut_dx_kernel, whose terms take long enough for lists from eight items in launches of fewer than
-// 2048 workgroups (batch-norm, 1500 + 800 x 700 27.8 us and 29.0, 1024 + 1024 x 1000 30.5 and 33.5; packed 500 + 500 x 4000 26 and 23.5).  BBHIP_DX_SPLIT = 0 / 1 forces none / four.
+// four are better: 100 x 8000 x 4000 128 and 148).  shortest: the shortest list that is long enough (packed 500 + 500 x 4000, lists from eight items, 26 us and
+// 23.5; real-valued inputs: dx_shortest_shared_list).  BBHIP_DX_SPLIT = 0 / 1 forces none / four.
 // Measured: training step of 59 inputs x 1594 nodes x 27 frames 30.0 -> 18.9 us, 50 x 3000 x 200 (StochasticLut4) 39.3 -> 22.3 us.
-int dx_split_lists(int max_fan, int input_node_size, int chunk_count, bool real_valued = false)
+int dx_split_lists(int max_fan, int input_node_size, int chunk_count, int shortest = 16)
 {
     static int const env = env_int("BBHIP_DX_SPLIT", 2);
     if (env == 0 || env == 1) { return env * kWavesPerBlk; }
-    long long const groups = (long long)chunk_count * ((input_node_size + kWavesPerBlk - 1) / kWavesPerBlk);
-    if (groups >= 4096 || max_fan < (real_valued && groups < 2048 ? 8 : 16)) { return 0; }
+    if ((long long)chunk_count * ((input_node_size + kWavesPerBlk - 1) / kWavesPerBlk) >= 4096 || max_fan < shortest) { return 0; }
     return (max_fan >= 32 && (long long)chunk_count * input_node_size < 1024) ? kDxWaves : kWavesPerBlk;
 }
 // BinaryLut6 units of 128 words: 8192 input rows x 512 bytes is what an XCD's 4 MiB L2 holds (1.2 GB fetched per launch at
@@ -975,20 +974,6 @@ int run_backward_small(BackwardCall const &c, hipStream_t st, int dw_overwrite)
     return 0;
 }
 
-// Real-valued inputs: passes of 256 frames, four consecutive ones per lane (lut_dx_kernel, WIDE), where a term's coefficients and addresses serve twice the
-// frames of the usual 128 and its rows come by a quarter of the loads.  All rows of x and dy that a window touches, 1 KB each, should be what an
-// L2 holds (training steps with and without: 1024 inputs + 2000 nodes x 4000 frames 106 and 112 us, 300 + 4000 x 4000 179 and 186, 500 + 1000 x 4000
-// with batch-norm 67 and 72.5, 1024 + 1024 x 1000 31.8 and 35.0; 3000 + 3000 x 6000 239 either way, 4096 + 4096 x 8192 498 and 457), and the launch should
-// have workgroups enough: one per input and pass where lists are shared (batch-norm, 300 + 1000 x 1200, 1500 of them, 39.8 and 40.3; 128 + 1500 x 2100,
-// 1152, 91.6 and 89.4; 40 + 3000 x 2000, 320, 103 and 92), else one per four inputs and pass, and items enough (1500 + 800 x 700, lists of three, 29.8 and 29.2).
-bool dx_wide_passes(int input_node_size, int output_node_size, int frame_size, int max_fan, long long links)
-{
-    long long const chunks = ceil_div(frame_size, 256);
-    if ((long long)input_node_size + output_node_size > 5000) { return false; }
-    long long const groups = chunks * ceil_div(input_node_size, kWavesPerBlk);
-    return max_fan >= (groups < 2048 ? 8 : 16) ? chunks * input_node_size >= 1400 : (chunks * ceil_div(input_node_size, kWavesPerBlk) >= 1024 && chunks * links >= 20480);
-}
-
 template <int N>
 int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packed = PackedInputHint{nullptr, 0, 0, 0},
                  PreparedTablesHint tables = PreparedTablesHint{nullptr, 0, 0}, int dw_overwrite = 0)
@@ -1175,7 +1160,8 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         int const chunk  = ((frames + kWave * steps - 1) / (kWave * steps)) * (kWave * steps);
         int const chunk_count = ceil_div(c.frame_size, chunk);
         // few input nodes with long work lists: the wavefronts of a workgroup share one input node (DxArgs::split)
-        int const split    = dx_split_lists(c.rev_stride - 1, c.input_node_size, chunk_count, true);
+        int const split    = dx_split_lists(c.rev_stride - 1, c.input_node_size, chunk_count, dx_shortest_shared_list(c.input_node_size, c.output_node_size,
+                                            c.frame_size, (long long)chunk_count * ceil_div(c.input_node_size, kWavesPerBlk)));
         int const in_tiles = split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
         if ((long long)chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }
         DxArgs d{};

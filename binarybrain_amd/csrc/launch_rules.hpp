@@ -101,4 +101,33 @@ constexpr SumsForm corner_sums_form(int frame_size, int slab_count)
     return (slab_count > 1 || frame_size > kBlockSlab) ? kSumsLong : frame_size <= kShortSlab ? kSumsShort : kSumsBlock;
 }
 
+// The shortest list that the wavefronts of a workgroup share in lut_dx_kernel (real-valued inputs), in a launch that would otherwise have `groups` workgroups of
+// four inputs each.  Its terms take long enough for lists from eight items where the launch falls short of wavefronts: training call of batch-norm
+// layers, six inputs per node, shared and not, 69 inputs x 66 nodes x 906 frames (list of 13) 10.4 and 15.0 us, 1500 x 800 x 700 (14) 20.6 and 23.0, 1024 x 1024 x
+// 1000 (14) 23.8 and 26.1.  Many frames of few inputs have wavefronts enough, whose rows all lie close: 16 x 26 x 29705 (14) 20.1 and 16.8, 40 x 63 x
+// 15921 (9) 11.2 and 9.8, 116 x 321 x 8625 (12) 25.8 and 23.3, but 16 x 26 x 14420 (13) 12.7 and 14.4.  Nor do layers of more than 5000 rows gain, which
+// have passes of 128 frames: 3383 x 3689 x 235 (14) 19.6 and 18.4, 3817 x 6000 x 253 (15) 21.3 and 19.9.
+constexpr int kDxWideRows = 5000;       // (dx_wide_passes)
+inline int dx_shortest_shared_list(int input_node_size, int output_node_size, int frame_size, long long groups)
+{
+    if (groups >= 2048 || (long long)input_node_size + output_node_size > kDxWideRows) { return 16; }
+    long long const passes = ceil_div(frame_size, 256);
+    return (passes <= 32 || passes * input_node_size < 1000) ? 8 : 16;
+}
+
+// Real-valued inputs: passes of 256 frames, four consecutive ones per lane (lut_dx_kernel, WIDE), where a term's coefficients and addresses serve twice the
+// frames of the usual 128 and its rows come by a quarter of the loads.  All rows of x and dy that a window touches, 1 KB each, should be what an
+// L2 holds (training steps with and without: 1024 inputs + 2000 nodes x 4000 frames 106 and 112 us, 300 + 4000 x 4000 179 and 186, 500 + 1000 x 4000
+// with batch-norm 67 and 72.5, 1024 + 1024 x 1000 31.8 and 35.0; 3000 + 3000 x 6000 239 either way, 4096 + 4096 x 8192 498 and 457), and the launch should
+// have workgroups enough.  Over 400 shapes of two to six inputs, drawn: where lists are shared (a workgroup per input and pass) passes of 256 frames take 1.04
+// times as long below 700 workgroups, 0.95 to 1.00 from 700 to 1400, 0.95 to 2000, 0.93 to 4000 and 0.84 to 0.90 above; else (a workgroup per four inputs)
+// 1.03 below 512 workgroups, 1.02 to 1024, 0.97 to 2048 and 0.92 to 0.98 above; few items make it worse (1500 + 800 x 700, lists of three, 29.8 and 29.2).
+inline bool dx_wide_passes(int input_node_size, int output_node_size, int frame_size, int max_fan, long long links)
+{
+    if ((long long)input_node_size + output_node_size > kDxWideRows) { return false; }
+    long long const passes = ceil_div(frame_size, 256), groups = passes * ceil_div(input_node_size, 4);
+    if (max_fan >= dx_shortest_shared_list(input_node_size, output_node_size, frame_size, groups)) { return passes * input_node_size >= 1400; }
+    return groups >= 1024 && passes * links >= 20480;
+}
+
 }  // namespace bbhip
