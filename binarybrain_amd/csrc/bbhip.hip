@@ -1664,10 +1664,11 @@ int bbhip_fp32_Im2Col_Forward(float const *dev_x_buf, float *dev_y_buf, int x_st
     clear_hints();                                 // a hint is for the next LUT forward call only
     Im2ColArgs a{dev_x_buf, dev_y_buf, x_stride, y_stride, x_offset, y_offset, input_frame_size, input_frame_stride, input_w_size,
                  input_h_size, input_c_size, output_w_size, output_h_size, output_frame_stride, filter_w_size, filter_h_size,
-                 border_mode, border_value, 0, 0};
+                 border_mode, border_value, 0, 0, 0};
     if (check_im2col(a, false, __func__)) { return 1; }
     if ((long long)a.oh * a.ow > 0x7fffffffLL) { return fail("%s: output plane too large", __func__); }
     a.f_tiles  = ceil_div(a.input_frame_size, kTile);
+    a.frames_first = im2col_frames_first(a.f_tiles, kTile);
     // 64 window positions per block, or 16 when that leaves fewer than two blocks per compute unit
     long long const columns = (long long)a.c * a.fh * a.fw * a.f_tiles;
     int const qt = (columns * ceil_div(a.oh * a.ow, kTile) >= 512) ? kTile : 16;
@@ -1689,7 +1690,7 @@ int bbhip_bit_Im2Col_Forward(int const *dev_x_buf, int *dev_y_buf, int x_stride,
     clear_hints();                                 // a hint is for the next LUT forward call only
     Im2ColArgs a{dev_x_buf, dev_y_buf, x_stride, y_stride, x_offset, y_offset, input_frame_size, input_frame_stride, input_w_size,
                  input_h_size, input_c_size, output_w_size, output_h_size, output_frame_stride, filter_w_size, filter_h_size,
-                 border_mode, 0.0f, 0, 0};
+                 border_mode, 0.0f, 0, 0, 0};
     if (check_im2col(a, true, __func__)) { return 1; }
     long long const out_frames = (long long)a.input_frame_size * a.oh * a.ow;
     int const words = (int)((out_frames + 31) / 32);
@@ -1710,7 +1711,7 @@ int bbhip_fp32_Im2Col_Backward(float const *dev_dy_buf, float *dev_dx_buf, int x
     clear_hints();                                 // a hint is for the next LUT forward call only
     Im2ColArgs a{dev_dy_buf, dev_dx_buf, x_stride, y_stride, x_offset, y_offset, input_frame_size, input_frame_stride, input_w_size,
                  input_h_size, input_c_size, output_w_size, output_h_size, output_frame_stride, filter_w_size, filter_h_size,
-                 0, 0.0f, 0, 0};
+                 0, 0.0f, 0, 0, 0};
     if (check_im2col(a, false, __func__)) { return 1; }
     if ((long long)a.h * a.w > 0x7fffffffLL) { return fail("%s: image too large", __func__); }
     int const p_tiles = ceil_div(a.h * a.w, kTile);
@@ -1719,6 +1720,7 @@ int bbhip_fp32_Im2Col_Backward(float const *dev_dy_buf, float *dev_dx_buf, int x
     auto const blocks_of = [&](int frames) { return (long long)a.c * p_tiles * ceil_div(a.input_frame_size, frames); };
     int const tf = blocks_of(64) >= 2048 ? 64 : blocks_of(16) >= 256 ? 16 : 4;
     a.f_tiles = ceil_div(a.input_frame_size, tf);
+    a.frames_first = im2col_frames_first(a.f_tiles, tf);
     long long const blocks = (long long)a.c * p_tiles * a.f_tiles;
     if (blocks > 0x7fffffffLL) { return fail("%s: grid too large", __func__); }
     ScopedTimer tm(kTimeOther, static_cast<hipStream_t>(stream));

@@ -29,6 +29,7 @@ struct Im2ColArgs {
     int border_mode;
     float border_value;
     int q_tiles, f_tiles;      // q_tiles: 64-position tiles of the flattened output plane (forward)
+    int frames_first;          // order of the workgroups: im2col_frames_first
 };
 
 // include/bb/ConvolutionIm2Col.h:251-286
@@ -52,6 +53,23 @@ __device__ __forceinline__ bool im2col_source(Im2ColArgs const &a, int oy, int o
     return im2col_border(a.border_mode, ix, iy, a.w, a.h);
 }
 
+// the workgroup's tile of positions, of frames, and its row
+__device__ __forceinline__ void im2col_place(Im2ColArgs const &a, int p_tiles, int &pt, int &ft, int &row)
+{
+    if (a.frames_first) {
+        int b = blockIdx.x;
+        ft = b % a.f_tiles;  b /= a.f_tiles;
+        pt = b % p_tiles;
+        row = b / p_tiles;
+    }
+    else {
+        int b = xcd_remap(blockIdx.x, gridDim.x);
+        pt = b % p_tiles;    b /= p_tiles;
+        ft = b % a.f_tiles;
+        row = b / a.f_tiles;
+    }
+}
+
 // block = (output node, QT window positions of the flattened (oy, ox) plane, 64 input frames): rows of the input are read
 // along the frames, the tile is written along the window positions, which are contiguous in the output.  The pieces of an output row do not
 // start on cache lines, so neighbouring pieces go to neighbouring workgroups of one XCD, whose L2 puts the lines together (27 nodes x 900 positions x
@@ -61,10 +79,8 @@ template <int QT>
 __global__ __launch_bounds__(kConvBlock) void im2col_forward_kernel(Im2ColArgs a)
 {
     __shared__ float tile[QT][kTile + 1];                    // [window position][frame]
-    int b = xcd_remap(blockIdx.x, gridDim.x);
-    int const qt = b % a.q_tiles;  b /= a.q_tiles;
-    int const ft = b % a.f_tiles;  b /= a.f_tiles;
-    int const node = b;                                      // (c*fh + fy)*fw + fx
+    int qt, ft, node;                                        // node: (c*fh + fy)*fw + fx
+    im2col_place(a, a.q_tiles, qt, ft, node);
     int const fx = node % a.fw, fy = (node / a.fw) % a.fh, c = node / (a.fw * a.fh);
     int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int const f0 = ft * kTile, q0 = qt * QT;
@@ -141,10 +157,8 @@ template <int TF>
 __global__ __launch_bounds__(kConvBlock) void im2col_backward_kernel(Im2ColArgs a, int p_tiles)
 {
     __shared__ float tile[kTile][TF + 1];                    // [pixel][frame]
-    int b = xcd_remap(blockIdx.x, gridDim.x);                // (neighbouring pixels read the same cache lines of dy: one L2)
-    int const pt = b % p_tiles;   b /= p_tiles;
-    int const ft = b % a.f_tiles; b /= a.f_tiles;
-    int const c  = b;
+    int pt, ft, c;
+    im2col_place(a, p_tiles, pt, ft, c);                     // (neighbouring pixels read the same cache lines of dy: one L2)
     int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int const f0 = ft * TF, p0 = pt * kTile;
     int const hw = a.h * a.w;

@@ -130,4 +130,11 @@ inline bool dx_wide_passes(int input_node_size, int output_node_size, int frame_
     return groups >= 1024 && passes * links >= 20480;
 }
 
+// Order of the workgroups of the Im2Col kernels.  Neighbouring pieces of a row share cache lines and belong in one L2: either the workgroups of an XCD are
+// consecutive ones, pieces first, or, where the tiles of 64 frames are a multiple of the eight XCDs, frames come first and every XCD has frames of its own, with
+// all pieces and all rows, so that its L2 also keeps the input for the next tap of the window.  Forward, pieces and frames first: 3 x 32 x 32 x 1024 frames, 3 x 3,
+// 31.5 and 27.5 us, 6 x 23 x 36 x 1024 48.7 and 42.0, 43 x 39 x 23 x 1521, 1 x 1, 108.8 and 92.5; 32 x 32 x 32 x 64 20.4 and 23.0 (one tile), 216 x 30 x 30 x 256, 1 x 1,
+// 78 and 97 (four).
+inline bool im2col_frames_first(int f_tiles, int tile_frames) { return tile_frames == 64 && f_tiles % 8 == 0; }
+
 }  // namespace bbhip

@@ -78,6 +78,12 @@ def test_im2col_tiles(ops, geometry):
 
 
 # rows that share a workgroup, at its edges: one to 256 threads a row, with four frames and (odd pitch) one frame per thread
+# 8 and 16 tiles of frames, the last one short or whole: workgroups in the order of the frames; backward in tiles of 64 frames (c = 70)
+@pytest.mark.parametrize("geometry", [(3, 12, 11, 449), (2, 9, 14, 512), (2, 9, 14, 513), (1, 7, 9, 1000), (70, 9, 8, 961)])
+def test_im2col_frames_first(ops, geometry):
+    test_im2col_tiles(ops, geometry)
+
+
 @pytest.mark.parametrize("frames, pitch", [(1, 64), (50, 64), (130, 132), (1020, 1024), (1021, 1024), (1025, 1028), (50, 51), (127, 127), (257, 259)])
 def test_stochastic_maxpool_rows_in_a_workgroup(ops, frames, pitch):
     c, h, w = 5, 7, 6
