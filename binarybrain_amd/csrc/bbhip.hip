@@ -257,6 +257,16 @@ void launch(void (*kernel)(P...), dim3 grid, dim3 block, unsigned lds_bytes, hip
     }, held);
 }
 
+// words [first, stride) of packed rows = 0 (first: packed_padding_end)
+int zero_row_ends(void *y, int rows, int stride, int first, hipStream_t st)
+{
+    if (first >= stride) { return 0; }
+    long long const pieces = ((long long)stride - first + kZeroPiece - 1) / kZeroPiece * rows;
+    launch(zero_row_ends_kernel, dim3((unsigned)std::min<long long>(pieces, 16384)), dim3(kBlock), 0, st, static_cast<uint32_t *>(y), rows, stride, first);
+    BBHIP_LAUNCH_CHECK();
+    return 0;
+}
+
 // ------------------------------------------------------------------------------------------------
 //  dispatch helpers
 // ------------------------------------------------------------------------------------------------
@@ -611,7 +621,8 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
     a.x_stride = c.x_stride; a.y_stride = c.y_stride;
     a.chunk = chunk; a.chunk_count = chunk_count; a.tiles = make_tile_divisor(tile_count);
     a.bias = c.bias; a.gamma = c.gamma; a.beta = c.beta;
-    a.zero_padding = c.zero_padding;
+    int const y_words = ceil_div(c.frame_size, 32);
+    a.pad_end = c.zero_padding ? packed_padding_end(y_words, c.y_stride) : 0;
     if (direct && to_caller) {
         int const row_blocks = ceil_div(packed.row_words * 8, kBlock);
         if ((long long)input_rows * row_blocks + (long long)chunk_count * tile_count > 0x7fffffffLL) { return fail("forward: grid too large"); }
@@ -672,7 +683,7 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
         if (dispatch_forward<N>(c.xmode, c.ymode, kind, a, npw, st)) { return 1; }
     }
     BBHIP_LAUNCH_CHECK();
-    return 0;
+    return (c.zero_padding && c.ymode == kYBit) ? zero_row_ends(c.y, c.node_size, c.y_stride, a.pad_end, st) : 0;
 }
 
 int forward_entry(ForwardCall const &call, void *stream, Scratch const *fixed = nullptr)
@@ -1339,6 +1350,7 @@ int run_binary_lut(int const *x, int *y, int const *idx, int const *table, int n
     }
     if (frame_stride > kBinMaxSharedPitch) { npw = 1; }
     bool const pad = zero_padding && frame_stride > a.word_count;
+    a.pad_end = packed_padding_end(a.word_count, frame_stride);
     int const tiles_per_launch = (1 << 23) / a.chunk_count;         // (a launch holds fewer than 2^32 threads)
     int const nodes_per_launch = (int)std::min<long long>(node_size, (long long)tiles_per_launch * kWavesPerBlk * npw);
     ScopedTimer tm(kTimeBinary, st);
@@ -1357,7 +1369,7 @@ int run_binary_lut(int const *x, int *y, int const *idx, int const *table, int n
         BBHIP_LAUNCH_CHECK();
         if (node_size - n0 <= nodes_per_launch) { break; }          // (n0 + nodes_per_launch may pass 2^31)
     }
-    return 0;
+    return pad ? zero_row_ends(y, node_size, frame_stride, a.pad_end, st) : 0;
 }
 
 }  // namespace

@@ -137,4 +137,10 @@ inline bool dx_wide_passes(int input_node_size, int output_node_size, int frame_
 // 78 and 97 (four).
 inline bool im2col_frames_first(int f_tiles, int tile_frames) { return tile_frames == 64 && f_tiles % 8 == 0; }
 
+// Packed rows whose padding the caller wants as 0: the wavefront of a row's last unit writes that much of it, an iteration per 64 words, and what a longer pitch
+// leaves is a launch of its own (zero_row_ends_kernel).  BinaryLut5, rows of 1000 frames, by the wavefronts and by the launch: 1000 rows of 2080 words 3.8 and
+// 5.7 us, 10000 words 8.7 and 9.7; 4 rows of 100000 words 42.1 and 4.5, 64 of 1000000 395 and 35.
+constexpr int kPaddingWords = 4096;
+inline int packed_padding_end(int words, int stride) { return (long long)words + kPaddingWords < stride ? words + kPaddingWords : stride; }
+
 }  // namespace bbhip

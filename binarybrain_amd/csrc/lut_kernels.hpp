@@ -275,7 +275,7 @@ struct FwdArgs {
     // lut_forward_corner_kernel over the fp32 frames of a small batch-norm training pass: the last pack.blocks workgroups make the packed copy of the
     // input that the backward call takes
     PackRider pack;
-    int   zero_padding;         // packed output: the wavefront of a node's last unit writes 0 behind the last frame's word, up to the row pitch
+    int   pad_end;              // packed output: the wavefront of a node's last unit writes 0 from behind the last frame's word up to this one (0: nothing)
 };
 
 // kStatInline: the call has one unit per node, so the wavefront that writes a node's output first sums the node's statistics
@@ -343,13 +343,13 @@ __device__ __forceinline__ void forward_stage(FwdArgs const &a, float v, bool ok
 __device__ __forceinline__ void zero_packed_tail(FwdArgs const &a, int ck, int node, bool live, int lane)
 {
     if (a.y_bits == nullptr || ck != a.chunk_count - 1 || !live) { return; }
-    for (int w = ((a.frame_size + 31) >> 5) + lane; w < a.y_bits_stride; w += kWave) { a.y_bits[(size_t)node * a.y_bits_stride + w] = 0u; }
+    for (uint32_t w = (uint32_t)((a.frame_size + 31) >> 5) + lane; w < (uint32_t)a.y_bits_stride; w += kWave) { a.y_bits[(size_t)node * a.y_bits_stride + w] = 0u; }
 }
 
 __device__ __forceinline__ void zero_output_padding(FwdArgs const &a, int ck, int node, bool live, int lane)
 {
-    if (a.zero_padding == 0 || ck != a.chunk_count - 1 || !live) { return; }
-    for (int w = ((a.frame_size + 31) >> 5) + lane; w < a.y_stride; w += kWave) { reinterpret_cast<uint32_t *>(a.y)[(size_t)node * a.y_stride + w] = 0u; }
+    if (a.pad_end == 0 || ck != a.chunk_count - 1 || !live) { return; }
+    for (int w = ((a.frame_size + 31) >> 5) + lane; w < a.pad_end; w += kWave) { reinterpret_cast<uint32_t *>(a.y)[(size_t)node * a.y_stride + w] = 0u; }
 }
 
 // per (unit, node) partial sums of the statistics kinds
@@ -1687,6 +1687,7 @@ struct BinArgs {
     int chunk;                  // words per unit, multiple of 64
     int chunk_count;
     TileDivisor tiles;
+    int pad_end;                // PAD: words behind the last frame's that the wavefronts of a row's last unit write as 0 end here
 };
 
 typedef uint32_t bin_u32x16 __attribute__((ext_vector_type(16)));
@@ -1879,7 +1880,7 @@ struct BinTable<N, false> {
 // (64 words 228 / 273 / 261 / 291, two nodes 259 / 265 / 278 / 288), 1000 x 3000 x 100000 11.4 / 13.7 / 14.2 / 16.3 instead of 23 / 25 / 28 / 30.
 // What bounds it there is the output: its 537 MB alone, without a gather, take 165 us.
 // nodes per wavefront; EXACT: the node count is a multiple of NPW, no wavefront has nodes to skip; PAD: the wavefronts of a row's last unit write 0
-// behind the last frame's word, up to the row pitch (a branch at the kernel's end costs the large shape 1 %, hence a variant of its own)
+// behind the last frame's word, up to pad_end (a branch at the kernel's end costs the large shape 1 %, hence a variant of its own)
 template <int N, int NPW, bool EXACT, bool PAD>
 __device__ __forceinline__ void binary_lut_unit(BinArgs const &a)
 {
@@ -1953,7 +1954,7 @@ __device__ __forceinline__ void binary_lut_unit(BinArgs const &a)
     if (PAD && w_end == a.word_count) {                          // wave-uniform
 #pragma unroll
         for (int p = 0; p < NPW; ++p) {
-            for (int w = a.word_count + lane; live[p] && w < a.stride; w += kWave) { a.y[(size_t)(node0 + p) * a.stride + w] = 0u; }
+            for (int w = a.word_count + lane; live[p] && w < a.pad_end; w += kWave) { a.y[(size_t)(node0 + p) * a.stride + w] = 0u; }
         }
     }
 }
@@ -1963,5 +1964,18 @@ __global__ __launch_bounds__(kBlock) void binary_lut6_kernel(BinArgs a) { binary
 
 template <int N, int NPW, bool EXACT, bool PAD = false>
 __global__ __launch_bounds__(kBlock) void binary_lutn_kernel(BinArgs a) { binary_lut_unit<N, NPW, EXACT, PAD>(a); }
+
+// Words [first, stride) of the rows of y = 0, in pieces of 16 words per lane: padding of packed rows that is too long for the wavefront that writes a row's end
+constexpr int kZeroPiece = 16 * kBlock;
+__global__ __launch_bounds__(kBlock) void zero_row_ends_kernel(uint32_t *__restrict__ y, int rows, int stride, int first)
+{
+    long long const pieces = ((long long)stride - first + kZeroPiece - 1) / kZeroPiece, count = pieces * rows;
+    for (long long p = blockIdx.x; p < count; p += gridDim.x) {
+        long long const row = p / pieces, word = first + (p - row * pieces) * kZeroPiece + threadIdx.x;
+        uint32_t *const out = y + row * stride + word;
+#pragma unroll
+        for (int i = 0; i < kZeroPiece / kBlock; ++i) { if (word + i * kBlock < stride) { out[i * kBlock] = 0u; } }
+    }
+}
 
 }  // namespace bbhip

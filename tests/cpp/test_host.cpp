@@ -397,6 +397,14 @@ int main(void)
         }
     }
 
+    // padding that the kernel of a packed output writes: no word number near the end of the range, and a bounded number of iterations
+    for (int words : {1, 3, 1 << 24}) {
+        for (int stride : {words, words + 1, words + 4095, words + 4096, words + 4097, 0x7fffffff}) {
+            int const end = bbhip::packed_padding_end(words, stride);
+            CHECK(end <= stride && end - words <= 4096 && (end == stride || end - words == 4096));
+        }
+    }
+
     std::printf("%s (%d failed checks)\n", g_fail ? "FAILED" : "OK", g_fail);
     return g_fail ? 1 : 0;
 }

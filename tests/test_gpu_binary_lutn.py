@@ -64,6 +64,52 @@ def test_rows_too_far_apart_for_one_extent(ops, n):
     assert torch.equal(y[:, :words], ops.binary_lutn_forward(n, xb, idx, T, F)[:, :words])
 
 
+def _wide_rows(bits, pitch):
+    """the rows of `bits` at another pitch, and memory of that shape that holds anything for the call's output"""
+    import torch
+    wide = torch.zeros((bits.shape[0], pitch), dtype=torch.int32, device="cuda")
+    wide[:, :bits.shape[1]] = bits
+    return wide
+
+
+# padding that the wavefront of a row's end writes (up to 4096 words), one word more, and far more; nodes to skip in the last wavefront, and none
+@pytest.mark.parametrize("n", [2, 5, 6])
+@pytest.mark.parametrize("nodes", [5, 64])
+@pytest.mark.parametrize("frames, padding", [(70, 1), (70, 4096), (70, 4097), (4096 * 3, 5000), (4096 * 3 + 1, 100003)])
+def test_padding_of_far_rows_is_zero(ops, n, nodes, frames, padding):
+    import torch
+    I, words = 9, (frames + 31) // 32
+    rng = np.random.default_rng(frames + n)
+    idx = dev(synth.wiring(rng, I, nodes, n)); T = dev(tables(rng, nodes, n))
+    xb = dev(synth.bernoulli_bits(rng, I, frames, words))
+    far = _wide_rows(xb, words + padding)
+    dirty = torch.full((nodes, words + padding), -1, dtype=torch.int32, device="cuda")
+    del dirty                                       # (its memory is what the call's output is made of)
+    y = ops.binary_lutn_forward(n, far, idx, T, frames)
+    assert torch.equal(y[:, :words], ops.binary_lutn_forward(n, xb, idx, T, frames)) and not y[:, words:].any()
+    W = torch.rand((nodes, 1 << n), device="cuda")
+    dirty = torch.full((nodes, words + padding), -1, dtype=torch.int32, device="cuda")
+    del dirty
+    y = ops.bit_bit_stochastic_lut_forward(n, far, idx, W, frames)
+    assert torch.equal(y[:, :words], ops.bit_bit_stochastic_lut_forward(n, xb, idx, W, frames)) and not y[:, words:].any()
+
+
+def test_padding_of_the_farthest_rows(ops):
+    """a pitch of 2^31 - 1 words: no word number that leaves the range of an int"""
+    import torch
+    frames, pitch = 70, (1 << 31) - 1
+    x = torch.zeros((1, pitch), dtype=torch.int32, device="cuda")
+    x[0, :3] = torch.tensor([0x12345678, -3, 63], dtype=torch.int32)
+    idx = torch.zeros((1, 2), dtype=torch.int32, device="cuda")
+    dirty = torch.full((1, pitch), -1, dtype=torch.int32, device="cuda")
+    del dirty
+    y = ops.binary_lutn_forward(2, x, idx, torch.full((1, 1), 8, dtype=torch.int32, device="cuda"), frames)      # x AND x
+    assert torch.equal(y[0, :3], x[0, :3])
+    assert all(not part.any() for part in y[0, 3:].split(1 << 28))
+    del x, y
+    torch.cuda.empty_cache()
+
+
 def test_reference_vectors_on_gpu(ops):
     for k in range(int(GOLD["count"][0])):
         p = "c%d_" % k
