@@ -196,7 +196,7 @@ int dx_split_lists(int max_fan, int input_node_size, int chunk_count, int shorte
 // BinaryLut6 units of 128 words: 8192 input rows x 512 bytes is what an XCD's 4 MiB L2 holds (1.2 GB fetched per launch at
 // the benchmark shape; 192-word units fetch 1.9 GB, 256-word units 2.3 GB).  With the per-wavefront set-up at its
 // present cost the shorter units are also the fastest (241 us; 192 words 278 us, 256 words 332 us, 64 words 282 us).
-int bin_chunk_words(void)  { static int v = env_int("BBHIP_BIN_CHUNK", 128); return (((v > 0 ? v : 128) + 63) / 64) * 64; }
+int bin_chunk_words(void)  { static int v = env_int("BBHIP_BIN_CHUNK", 0); return v > 0 ? ceil_div(v, 64) * 64 : 0; }      // 0: chosen per call (binary_unit_words)
 int bin_nodes_per_wave(void) { static int v = env_int("BBHIP_BIN_NODES", 0); return v >= 4 ? 4 : v >= 2 ? 2 : v == 1 ? 1 : 0; }     // 0: chosen per call
 
 // ------------------------------------------------------------------------------------------------
@@ -1340,7 +1340,7 @@ int run_binary_lut(int const *x, int *y, int const *idx, int const *table, int n
     a.x = reinterpret_cast<uint32_t const *>(x);
     a.frame_size = frame_size; a.stride = frame_stride;
     a.word_count = ceil_div(frame_size, 32);
-    a.chunk = bin_chunk_words();
+    a.chunk = bin_chunk_words() ? bin_chunk_words() : binary_unit_words(a.word_count, node_size);
     a.chunk_count = ceil_div(a.word_count, a.chunk);
     // nodes per wavefront: four share a unit's set-up where that still leaves the launch 2048 workgroups
     int npw = bin_nodes_per_wave();

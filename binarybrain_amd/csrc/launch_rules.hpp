@@ -139,8 +139,16 @@ inline bool im2col_frames_first(int f_tiles, int tile_frames) { return tile_fram
 
 // Packed rows whose padding the caller wants as 0: the wavefront of a row's last unit writes that much of it, an iteration per 64 words, and what a longer pitch
 // leaves is a launch of its own (zero_row_ends_kernel).  BinaryLut5, rows of 1000 frames, by the wavefronts and by the launch: 1000 rows of 2080 words 3.8 and
-// 5.7 us, 10000 words 8.7 and 9.7; 4 rows of 100000 words 42.1 and 4.5, 64 of 1000000 395 and 35.
+// 5.7 us, 10000 words 8.7 and 11.3; 4 rows of 100000 words 42.1 and 5.8, 64 of 1000000 397 and 36.
 constexpr int kPaddingWords = 4096;
 inline int packed_padding_end(int words, int stride) { return (long long)words + kPaddingWords < stride ? words + kPaddingWords : stride; }
+
+// Words per unit of the BinaryLut kernels: 128 (see there), or 64 where the launch still has fewer than 512 workgroups then, that is compute units to spare, and a
+// unit's second step only takes time.  3 inputs per node, 30 nodes x 93 words 2.24 -> 2.00 us, 239 nodes x 261 words, five, 2.26 -> 2.13, 183 x 688, three, 2.21 -> 2.09
+// (506 workgroups); 29 x 6663, two, 2.19 and 2.29 (840), 4708 x 69, three, 3.19 and 3.84 (2354).
+inline int binary_unit_words(int words, int node_size)
+{
+    return (long long)ceil_div(words, 64) * ceil_div(node_size, 4) < 512 ? 64 : 128;
+}
 
 }  // namespace bbhip

@@ -405,6 +405,13 @@ int main(void)
         }
     }
 
+    // units of the BinaryLut kernels, where both were measured (microseconds, units of 64 and of 128 words)
+    {
+        struct { int nodes, words; double short_units, long_units; } const rows[] = {{30, 93, 2.00, 2.24}, {40, 256, 2.01, 2.24}, {239, 261, 2.13, 2.26}, {183, 688, 2.09, 2.21},
+            {154, 69, 2.01, 2.18}, {354, 394, 2.43, 2.38}, {29, 6663, 2.29, 2.19}, {4708, 69, 3.84, 3.19}, {5405, 5653, 59.97, 41.02}};
+        for (auto const &r : rows) { CHECK((bbhip::binary_unit_words(r.words, r.nodes) == 64) == (r.short_units < r.long_units)); }
+    }
+
     std::printf("%s (%d failed checks)\n", g_fail ? "FAILED" : "OK", g_fail);
     return g_fail ? 1 : 0;
 }
