@@ -343,7 +343,7 @@ __global__ __launch_bounds__(kConvBlock) void stochastic_maxpool2x2_forward_kern
 #pragma unroll
         for (int fx = 0; fx < 2; ++fx) {
             int const iy = oy * 2 + fy, ix = ox * 2 + fx;
-            if (iy < a.h && ix < a.w) { bn_load<W>(a.x + ((size_t)(c * a.h + iy) * a.w + ix) * a.frame_stride, f, a.frame_size, v[fy][fx]); }
+            if (iy < a.h && ix < a.w) { bn_load<W>(a.x + (((size_t)c * a.h + iy) * a.w + ix) * a.frame_stride, f, a.frame_size, v[fy][fx]); }
         }
     }
     float out[W];
@@ -380,7 +380,7 @@ __global__ __launch_bounds__(kConvBlock) void stochastic_maxpool2x2_backward_ker
 #pragma unroll
         for (int fx = 0; fx < 2; ++fx) {
             int const iy = oy * 2 + fy, ix = ox * 2 + fx;
-            if (iy < a.h && ix < a.w) { bn_load<W>(a.x + ((size_t)(c * a.h + iy) * a.w + ix) * a.frame_stride, f, a.frame_size, v[fy][fx]); }
+            if (iy < a.h && ix < a.w) { bn_load<W>(a.x + (((size_t)c * a.h + iy) * a.w + ix) * a.frame_stride, f, a.frame_size, v[fy][fx]); }
             else {
 #pragma unroll
                 for (int j = 0; j < W; ++j) { v[fy][fx][j] = 0.0f; }
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(kConvBlock) void stochastic_maxpool2x2_backward_ker
 #pragma unroll
         for (int fx = 0; fx < 2; ++fx) {
             int const iy = oy * 2 + fy, ix = ox * 2 + fx;
-            if (iy < a.h && ix < a.w) { bn_store<W>(a.out + ((size_t)(c * a.h + iy) * a.w + ix) * a.frame_stride, f, a.frame_size, gr[fy][fx]); }
+            if (iy < a.h && ix < a.w) { bn_store<W>(a.out + (((size_t)c * a.h + iy) * a.w + ix) * a.frame_stride, f, a.frame_size, gr[fy][fx]); }
         }
     }
 }

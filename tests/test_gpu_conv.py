@@ -96,6 +96,21 @@ def test_stochastic_maxpool_rows_in_a_workgroup(ops, frames, pitch):
     assert np.array_equal(dx[:, :frames], oracle.stochastic_maxpool2x2_backward(x, dy, c, h, w, frames)[:, :frames])
 
 
+def test_stochastic_maxpool_of_very_many_rows(ops):
+    """2^31 rows of one frame and more (a launch holds them since short rows share a workgroup): row numbers beyond the range of an int"""
+    import torch
+    c, h, w = (1 << 30) + 9, 2, 1
+    x = torch.full((c * h * w, 1), 0.5, device="cuda")
+    x[0], x[1], x[-2], x[-1] = 0.25, 0.75, 1.0, 0.125
+    y = ops.stochastic_maxpool2x2_forward(x, c, h, w, 1)
+    assert y[0].item() == 1 - 0.75 * 0.25 and y[-1].item() == 1.0 and bool((y[1:-1] == 0.75).all())
+    y.fill_(2.0)
+    dx = ops.stochastic_maxpool2x2_backward(x, y, c, h, w, 1)
+    assert dx[:2, 0].tolist() == [0.5, 1.5] and dx[-2:, 0].tolist() == [1.75, 0.0] and bool((dx[2:-2] == 1.0).all())
+    del x, y, dx
+    torch.cuda.empty_cache()
+
+
 def test_im2col_reference_vectors(ops):
     for k in range(int(GOLD["im2col_count"][0])):
         c, h, w, F, fh, fw, ys, xs, same, border = [int(v) for v in GOLD["i%d_geom" % k]]
