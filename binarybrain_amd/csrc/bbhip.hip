@@ -1814,10 +1814,11 @@ static int launch_pool(PoolArgs const &call, bool backward, void *stream, char c
     uintptr_t const bits = reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(backward ? a.dy : a.x);
     bool const wide = (bits & 15u) == 0 && (a.frame_stride & 3) == 0;
     int const lanes = std::min(ceil_div(a.frame_size, wide ? 4 : 1), kConvBlock);
-    a.lanes = make_tile_divisor(lanes);
-    a.rows = kConvBlock / lanes;
-    a.f_blocks = ceil_div(a.frame_size, kConvBlock * (wide ? 4 : 1));
     long long const nodes = (long long)a.c * a.oh * a.ow;
+    static_assert(kConvBlock == 256, "pool_shared_rows");
+    a.rows = pool_shared_rows(lanes, nodes);
+    a.lanes = make_tile_divisor(a.rows == 1 ? kConvBlock : lanes);
+    a.f_blocks = ceil_div(a.frame_size, kConvBlock * (wide ? 4 : 1));
     if (nodes > 0x7fffffffLL) { return fail("%s: grid too large", name); }
     long long const blocks = (nodes + a.rows - 1) / a.rows * a.f_blocks;
     if (blocks > 0x7fffffffLL) { return fail("%s: grid too large", name); }

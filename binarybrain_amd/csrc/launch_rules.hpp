@@ -151,4 +151,14 @@ inline int binary_unit_words(int words, int node_size)
     return (long long)ceil_div(words, 64) * ceil_div(node_size, 4) < 512 ? 64 : 128;
 }
 
+// Rows that share a workgroup of 256 threads in the pooling kernels, `lanes` threads each.  A row has a workgroup of its own where sharing saves no more than
+// one or two idle wavefronts of it and there are workgroups for every compute unit either way: up to 256 rows (120 rows x 203 frames, backward, 3.31 us shared and
+// 3.08 not), and where whole wavefronts stream through memory (48600 x 256 forward 35.4 and 33.3, backward 82.1 and 79.7; 46740 x 512 backward 151.8 and
+// 146.4).  7056 x 256 4.8 and 5.8, backward 10.3 and 11.5; 90000 x 128 32.4 and 40.8, 29070 x 280 backward 49.8 and 61.3.
+inline int pool_shared_rows(int lanes, long long nodes)
+{
+    bool const full = lanes % 64 == 0 || lanes % 64 >= 48;              // the last wavefront of a row
+    return (lanes > 32 && (nodes <= 256 || (nodes > 16384 && full))) ? 1 : 256 / lanes;
+}
+
 }  // namespace bbhip

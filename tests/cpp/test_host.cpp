@@ -412,6 +412,18 @@ int main(void)
         for (auto const &r : rows) { CHECK((bbhip::binary_unit_words(r.words, r.nodes) == 64) == (r.short_units < r.long_units)); }
     }
 
+    // rows that share a workgroup in the pooling kernels, where both were measured (microseconds): at most 3 % slower than the faster
+    {
+        struct { int nodes, lanes; double shared, own; } const rows[] = {{120, 51, 3.31, 3.08}, {180, 64, 3.12, 2.93}, {48600, 64, 82.1, 79.7}, {50445, 64, 35.0, 32.9},
+            {46740, 128, 151.8, 146.4}, {73872, 61, 133.5, 129.9}, {7056, 64, 10.3, 11.5}, {90000, 32, 32.4, 40.8}, {29070, 70, 49.8, 61.3}, {4056, 13, 2.6, 4.1}, {16, 1, 2.16, 2.30},
+            {12936, 45, 14.1, 16.3}, {4482, 83, 8.9, 10.2}, {60, 15, 2.30, 2.47}};
+        for (auto const &r : rows) {
+            int const count = bbhip::pool_shared_rows(r.lanes, r.nodes);
+            CHECK(count >= 1 && count * r.lanes <= 256);
+            if ((count > 1 ? r.shared : r.own) > 1.03 * std::min(r.shared, r.own)) { std::printf("%d rows, %d threads\n", r.nodes, r.lanes); CHECK(!"pool_shared_rows"); }
+        }
+    }
+
     std::printf("%s (%d failed checks)\n", g_fail ? "FAILED" : "OK", g_fail);
     return g_fail ? 1 : 0;
 }
