@@ -1810,9 +1810,9 @@ static int launch_pool(PoolArgs const &call, bool backward, void *stream, char c
     if (!(a.w > 0 && a.h > 0 && a.c > 0 && a.frame_size > 0)) { return fail("%s: sizes must be positive", name); }
     if (a.ow != (a.w + 1) / 2 || a.oh != (a.h + 1) / 2) { return fail("%s: output size must be ceil(input / 2)", name); }
     if (a.frame_stride < a.frame_size) { return fail("%s: frame stride shorter than the frames", name); }
-    // four frames per thread with 128-bit accesses where every row starts on 16 bytes
+    // four frames per thread with 128-bit accesses where every row starts on 16 bytes, but for very short rows
     uintptr_t const bits = reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(backward ? a.dy : a.x);
-    bool const wide = (bits & 15u) == 0 && (a.frame_stride & 3) == 0;
+    bool const wide = (bits & 15u) == 0 && (a.frame_stride & 3) == 0 && pool_four_frames(a.frame_size);
     int const lanes = std::min(ceil_div(a.frame_size, wide ? 4 : 1), kConvBlock);
     long long const nodes = (long long)a.c * a.oh * a.ow;
     static_assert(kConvBlock == 256, "pool_shared_rows");

@@ -151,6 +151,12 @@ inline int binary_unit_words(int words, int node_size)
     return (long long)ceil_div(words, 64) * ceil_div(node_size, 4) < 512 ? 64 : 128;
 }
 
+// Whether a thread of the pooling kernels takes four frames (rows start on 16 bytes): not for rows of less than 16 frames that are no whole groups of four, where
+// every wavefront would do the last group's frames one by one beside the whole groups.  One frame and four per thread, forward / backward: 2280 rows of 3 frames
+// 2.3 / 2.9 and 3.5 / 4.8 us, 840 of 11 2.2 / 2.7 and 2.7 / 3.5, 31995 of 11 3.6 / 6.0 and 3.9 / 7.1; many rows of more frames gain from four, 27183 of 18
+// 4.0 / 6.9 and 3.6 / 6.9, the more so the longer they are.
+inline bool pool_four_frames(int frame_size) { return frame_size >= 16 || frame_size % 4 == 0; }
+
 // Rows that share a workgroup of 256 threads in the pooling kernels, `lanes` threads each.  A row has a workgroup of its own where sharing saves no more than
 // one or two idle wavefronts of it and there are workgroups for every compute unit either way: up to 256 rows (120 rows x 203 frames, backward, 3.31 us shared and
 // 3.08 not), and where whole wavefronts stream through memory (48600 x 256 forward 35.4 and 33.3, backward 82.1 and 79.7; 46740 x 512 backward 151.8 and

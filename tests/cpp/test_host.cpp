@@ -424,6 +424,12 @@ int main(void)
         }
     }
 
+    // frames per thread of the pooling kernels, as measured (share of the time of four frames that one frame per thread takes, few rows, backward)
+    {
+        struct { int frames; double one; } const rows[] = {{2, 0.79}, {3, 0.65}, {5, 0.81}, {6, 0.74}, {7, 0.71}, {9, 0.83}, {11, 0.78}, {13, 0.83}, {15, 0.79}, {4, 1.1}, {8, 1.1}, {50, 1.22}, {99, 1.39}};
+        for (auto const &r : rows) { CHECK(bbhip::pool_four_frames(r.frames) == (r.one > 1.0)); }
+    }
+
     std::printf("%s (%d failed checks)\n", g_fail ? "FAILED" : "OK", g_fail);
     return g_fail ? 1 : 0;
 }

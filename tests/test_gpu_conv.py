@@ -96,6 +96,12 @@ def test_stochastic_maxpool_rows_in_a_workgroup(ops, frames, pitch):
     assert np.array_equal(dx[:, :frames], oracle.stochastic_maxpool2x2_backward(x, dy, c, h, w, frames)[:, :frames])
 
 
+@pytest.mark.parametrize("frames", [2, 3, 4, 13, 15, 16, 17])
+def test_stochastic_maxpool_short_rows(ops, frames):
+    """one frame per thread below 16 frames that are no whole groups of four, four from there on, at a pitch that allows both"""
+    test_stochastic_maxpool_rows_in_a_workgroup(ops, frames, 20)
+
+
 def test_stochastic_maxpool_of_very_many_rows(ops):
     """2^31 rows of one frame and more (a launch holds them since short rows share a workgroup): row numbers beyond the range of an int"""
     import torch
