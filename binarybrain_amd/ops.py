@@ -7,6 +7,7 @@ packed bits.  Nothing here has a CPU fallback: without the built library, or off
 The calls go through the extension module built from csrc/ops_native.cpp (`native` below), which checks every tensor argument (device,
 contiguous), allocates outputs and takes the current stream: what a call costs on the host bounds every pass over small layers.
 """
+import numpy as np
 import torch
 
 from . import capi, synth
@@ -76,7 +77,6 @@ class AdamState:
     on the host as the reference does (include/bb/OptimizerAdam.h:104-110, 166-180)."""
 
     def __init__(self, params, grads, learning_rate=0.001, beta1=0.9, beta2=0.999):
-        import numpy as np
         for tensor in (*params, *grads):
             if not tensor.is_cuda or not tensor.is_contiguous():
                 raise capi.BbhipError("bbhip ops need contiguous device tensors")
@@ -92,20 +92,19 @@ class AdamState:
         self.b1, self.b2 = f32(beta1), f32(beta2)
 
     def lr_t(self):
-        import numpy as np
-        one = np.float32(1.0)
-        return np.float32(np.float32(self.lr * np.sqrt(one - self.b2, dtype=np.float32)) / (one - self.b1))
+        """the bias-corrected rate of the next step: lr * sqrt(1 - b2) / (1 - b1), every operation rounded to float"""
+        return np.float32(native.adam_rate(self.lr, self.b1, self.b2))
 
     def step(self):
         native.fp32_OptimizerAdam(len(self.params), self.t_size, self.t_params, self.t_grads, self.t_m, self.t_v,
-                                  native.adam_rate(self.lr, self.b1, self.b2), self.beta1, self.beta2)
+                                  self.lr_t(), self.beta1, self.beta2)
         self.b1 = self.b1 * self.beta1
         self.b2 = self.b2 * self.beta2
 
     def update(self):
         """Optimizer::Update of the reference = step, then the gradients set to zero (include/bb/Optimizer.h:31-35), in one launch."""
         native.fp32_OptimizerAdam_Update(len(self.params), self.t_size, self.t_params, self.t_grads, self.t_m, self.t_v,
-                                         native.adam_rate(self.lr, self.b1, self.b2), self.beta1, self.beta2)
+                                         self.lr_t(), self.beta1, self.beta2)
         self.b1 = self.b1 * self.beta1
         self.b2 = self.b2 * self.beta2
 
@@ -410,7 +409,6 @@ def loss_mean_squared_error(y, t, frame_size, loss_buf, batch_size=None, reducti
     loss_buf.sum() / frames seen (the sum itself with reduction "sum")."""
     nodes = y.shape[0]
     batch_size = frame_size if batch_size is None else batch_size
-    import numpy as np
     grad_reduction = np.float32(1.0) if reduction_sum else np.float32(1.0) / np.float32(nodes * batch_size)
     loss_reduction = 1.0 if reduction_sum else 1.0 / nodes
     dy = torch.empty_like(y)
@@ -581,7 +579,6 @@ def reverse_table(idx, input_nodes):
     """Reverse connection table as the reference builds it (include/bb/FixedSizeConnectionTable.h:180-215):
     ``[input_nodes, 1 + max fan-out]`` int32, row r = [count, node*n + input ... ascending, zero tail].
     Built on the host with numpy (index bookkeeping, not on the timed path); returned on idx's device."""
-    import numpy as np
     h = idx.detach().cpu().numpy().astype(np.int64)
     O, n = h.shape
     flat = h.reshape(-1)

@@ -120,10 +120,37 @@ def test_against_compiled_reference():
 
 
 def test_rate_formed_natively_is_the_numpy_one():
-    """the step size that AdamState passes on, formed in C++: the same bits as lr_t(), from the first step to the limits of the products"""
+    """the step size that AdamState passes on, formed in C++: the same bits as numpy's, from the first step to the limits of the products"""
     from binarybrain_amd.capi import native
     rng = np.random.default_rng(5)
     for _ in range(5000):
         lr, b1, b2 = (F32(v) for v in (10.0 ** rng.uniform(-6, 0), rng.random() ** 4, rng.random() ** 4))
         want = F32(F32(lr * np.sqrt(F32(1) - b2, dtype=F32)) / (F32(1) - b1))
         assert native.adam_rate(lr, b1, b2) == float(want)
+
+
+@pytest.mark.parametrize("name", ["step", "update"])
+def test_steps_take_the_rate_of_lr_t(name, monkeypatch):
+    """the rate that a step passes on is that of lr_t(), the oracle's from the first step on; a class that has a rate of its own (a schedule) overrides it"""
+    from binarybrain_amd import ops
+    native = ops.native
+    native.adam_rate                                # (loads the extension module)
+    passed = []
+    monkeypatch.setitem(native.__dict__, "fp32_OptimizerAdam" + ("_Update" if name == "update" else ""), lambda *args: passed.append(args[6]))
+
+    class Halved(ops.AdamState):
+        def lr_t(self):
+            return super().lr_t() / F32(2)
+
+    for cls, factor in ((ops.AdamState, F32(1)), (Halved, F32(2))):
+        state = object.__new__(cls)
+        state.params = []
+        state.t_size = state.t_params = state.t_grads = state.t_m = state.t_v = None
+        state.lr, state.beta1, state.beta2 = F32(0.002), F32(0.9), F32(0.999)
+        state.b1, state.b2 = state.beta1, state.beta2
+        b1, b2 = state.b1, state.b2
+        for _ in range(5):
+            assert isinstance(state.lr_t(), F32)
+            getattr(state, name)()
+            assert passed[-1] * factor == oracle.adam_lr_t(0.002, b1, b2)
+            b1, b2 = b1 * F32(0.9), b2 * F32(0.999)
