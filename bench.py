@@ -1060,9 +1060,10 @@ def gather_probe_library():
 
 
 def bench_gather_ceiling(args, lib):
-    """What the GPU sustains on the dx kernel's access pattern alone (instrumentation, a kernel of the bench's own): per (input row,
+    """A rate of gathered rows at the dx kernel's access pattern (instrumentation, a kernel of the bench's own): per (input row,
     128-frame window) 36 pseudo-randomly chosen rows' 512-byte segments are read and discarded — 6 consumers x (5 rows + dy) as in the
-    headline shape.  Reported as a rate through L1; the dx kernel moves the same bytes and does its arithmetic on top."""
+    headline shape.  Reported as a rate through L1.  It includes a remainder that the probe takes per row to choose the next one, which is what
+    bounds it at 512 bytes: compute units take 25 to 31 TB/s from rows that an L2 holds, so this is no ceiling of the dx kernel."""
     import ctypes as C
     import torch
     from binarybrain_amd import synth
@@ -1098,8 +1099,8 @@ def bench_gather_ceiling(args, lib):
 
 def other_configs(args, lib):
     """The other BASELINE configurations, measured after the headline workload in the same process: configuration 1 (forward
-    784 -> 1024 x 64), 3 (classifier training step), 4 (BinaryLut6 inference), 5 (convolutional block), and the gather
-    ceiling that the dx kernel is judged against.  Each entry keeps its own roofline and CPU baseline."""
+    784 -> 1024 x 64), 3 (classifier training step), 4 (BinaryLut6 inference), 5 (convolutional block), and the rate of the
+    gather probe (`bench_gather_ceiling`; not a bound of the dx kernel).  Each entry keeps its own roofline and CPU baseline."""
     import copy
     sub = copy.copy(args)
     sub.ramp_seconds = min(args.ramp_seconds, 0.15)

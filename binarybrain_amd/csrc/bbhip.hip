@@ -193,7 +193,7 @@ int dx_split_lists(int max_fan, int input_node_size, int chunk_count, int shorte
     if ((long long)chunk_count * ((input_node_size + kWavesPerBlk - 1) / kWavesPerBlk) >= 4096 || max_fan < shortest) { return 0; }
     return (max_fan >= 32 && (long long)chunk_count * input_node_size < 1024) ? kDxWaves : kWavesPerBlk;
 }
-// BinaryLut6 units of 128 words: 8192 input rows x 512 bytes is what an XCD's 4 MiB L2 holds (1.2 GB fetched per launch at
+// BinaryLut6 units of 128 words (64 in small launches: binary_unit_words): 8192 input rows x 512 bytes is what an XCD's 4 MiB L2 holds (1.2 GB fetched per launch at
 // the benchmark shape; 192-word units fetch 1.9 GB, 256-word units 2.3 GB).  With the per-wavefront set-up at its
 // present cost the shorter units are also the fastest (241 us; 192 words 278 us, 256 words 332 us, 64 words 282 us).
 int bin_chunk_words(void)  { static int v = env_int("BBHIP_BIN_CHUNK", 0); return v > 0 ? ceil_div(v, 64) * 64 : 0; }      // 0: chosen per call (binary_unit_words)
@@ -242,7 +242,6 @@ int arena_get(size_t bytes, char **out, hipStream_t st, Scratch const *fixed = n
 }
 
 inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
-
 
 // A launch without the call-configuration stack and the copies that the <<<>>> form's host stub goes through: 2.7 us of host time for a kernel
 // with 400 bytes of arguments instead of 3.2, and the host is what a program of small layers waits for.  Errors are read by BBHIP_LAUNCH_CHECK.

@@ -72,7 +72,7 @@ __device__ __forceinline__ void im2col_place(Im2ColArgs const &a, int p_tiles, i
 
 // block = (output node, QT window positions of the flattened (oy, ox) plane, 64 input frames): rows of the input are read
 // along the frames, the tile is written along the window positions, which are contiguous in the output.  The pieces of an output row do not
-// start on cache lines, so neighbouring pieces go to neighbouring workgroups of one XCD, whose L2 puts the lines together (27 nodes x 900 positions x
+// start on cache lines, so neighbouring pieces go to one XCD (im2col_place), whose L2 puts the lines together (27 nodes x 900 positions x
 // 256 frames 13.2 -> 12.4 us; the two directions of col2im_kernel 15.1 -> 14.6 and 13.1 -> 11.7).  A launch of one round is a chain of latencies (loads,
 // barrier, stores): shorter tiles where there are compute units to spare (9 nodes x 676 positions x 50 frames 6.0 -> 4.1 us with QT = 16).
 template <int QT>
@@ -316,7 +316,7 @@ struct PoolArgs {
 
 // The thread's output node and first frame; false: none.  Rows shorter than a workgroup's threads share one: 4056 nodes x 50 frames are 214 workgroups
 // instead of 4056 of which 13 threads work (forward 5.0 -> 3.1 us, backward 7.2 -> 4.6; 8100 nodes x 256 frames, 64 threads a row, backward
-// 14.8 -> 12.3).
+// 14.8 -> 12.3, forward 7.3 -> 7.8).  Not all do: pool_shared_rows.
 template <int W>
 __device__ __forceinline__ bool pool_place(PoolArgs const &a, int &node, int &f)
 {

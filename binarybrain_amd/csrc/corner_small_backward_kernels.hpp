@@ -74,7 +74,7 @@ struct CornerSmallDxShared {            // a wavefront's LDS
 // every path alike: an item past the end reads from buffers of no length.
 // Bound by latency: an item takes 0.45 us of a wavefront's time (256 frames; 0.75 and 1.1 with 512 and 1024), about 160 instructions that wait for one
 // another, a launch 4.5 to 5 us.  Backward call of 1024 inputs x 360 nodes x 256 frames 9.0 -> 5.8 us, 784 x 1024 9.4 -> 6.2, 360 x 70 x 1024
-// 8.8 -> 5.9 (the rule with both sides of the line: small_corner_layer).
+// 8.8 -> 5.9 (the rule with both sides of the line: corner_small_waves).
 template <int N, bool BN, int PASSES, bool QUADS, int WAVES>
 __device__ __forceinline__ void corner_small_dx_unit(CornerSmallArgs const &t, CornerSmallDxShared<N, BN, PASSES> *shared, int tile, int wave, int lane)
 {

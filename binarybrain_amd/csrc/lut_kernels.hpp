@@ -1874,7 +1874,7 @@ struct BinTable<N, false> {
     }
 };
 
-// Units of 128 words and four nodes per wavefront at every N: a wavefront sets up once and has 4 N rows' loads in flight, and the nodes of an XCD
+// Units of 128 words (64 in small launches: binary_unit_words) and four nodes per wavefront at every N: a wavefront sets up once and has 4 N rows' loads in flight, and the nodes of an XCD
 // read one window of the input rows at a time from its L2.  Measured against a thread per (node, word) in row order, whose rows came
 // from behind the L2 each time: 8192 x 16384 x 262144 at N = 2 / 3 / 4 / 5 212 / 244 / 248 / 267 us instead of 408 / 427 / 455 / 491
 // (64 words 228 / 273 / 261 / 291, two nodes 259 / 265 / 278 / 288), 1000 x 3000 x 100000 11.4 / 13.7 / 14.2 / 16.3 instead of 23 / 25 / 28 / 30.
