@@ -19,6 +19,7 @@
 #include "launch_rules.hpp"
 #include "lut_kernels.hpp"
 #include "corner_forward_kernels.hpp"
+#include "corner_few_inputs_kernels.hpp"
 #include "corner_small_backward_kernels.hpp"
 #include "table_gradient_kernels.hpp"
 #include "small_backward_kernels.hpp"
@@ -777,6 +778,16 @@ int dispatch_dx_table(int quads, DxTableArgs const &t, hipStream_t st)
     return 0;
 }
 
+template <int N, bool BN>
+int launch_dx_few_inputs(FewInputsArgs const &a, hipStream_t st)
+{
+    dim3 const grid(ceil_div(a.frame_size, kFewUnits * kFewFrames * kWave));
+    ScopedTimer tm(kTimeDx, st);
+    launch((lut_dx_few_inputs_kernel<N, BN>), grid, dim3(kFewWaves * kWave), (unsigned)few_inputs_lds(N, a.node_size), st, a);
+    BBHIP_LAUNCH_CHECK();
+    return 0;
+}
+
 // Small layers on two-valued inputs whose backward pass is one launch (lut_corner_small_backward_kernel): the wavefronts that walk an input's list (0: two
 // launches), by corner_small_waves
 int small_corner_layer(BackwardCall const &c)
@@ -786,6 +797,17 @@ int small_corner_layer(BackwardCall const &c)
         (long long)c.output_node_size * (4 << c.n) > 0xffffffffLL) { return 0; }                                  // (32-bit offsets into whole buffers)
     static_assert(kCornerSmallShare <= kCornerSmallItems, "the kernel holds a wavefront's items one per lane");
     return corner_small_waves(c.n, c.bn, c.frame_size, c.input_node_size, c.output_node_size, c.rev_stride - 1);
+}
+
+// Layers of few inputs whose dx is formed node by node (lut_dx_few_inputs_kernel): by few_inputs_dx, where rows are whole 16-byte groups and offsets into
+// whole buffers fit 32 bits
+bool few_inputs_layer(BackwardCall const &c)
+{
+    if (dx_quads_env() != 0 || !few_inputs_dx(c.n, c.input_node_size, c.output_node_size, c.frame_size)) { return false; }
+    static_assert(kFewInputs <= kFewMost, "a register for every input");
+    return c.frame_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(c.dy) & 15u) == 0 && (reinterpret_cast<uintptr_t>(c.dx) & 7u) == 0 &&
+           (long long)c.input_node_size * c.x_stride * 4 <= 0xffffffffLL && (long long)c.output_node_size * c.frame_stride * 4 <= 0xffffffffLL &&
+           (long long)few_entry_bytes(c.n, c.output_node_size) <= 0x7fffffffLL;
 }
 
 template <int N, bool BN, bool QUADS>
@@ -827,22 +849,25 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     int const own_words = ceil_div(c.frame_size, 32) * 8;
 
     int const small = small_corner_layer(c);
+    bool const few = !small && few_inputs_layer(c);
 
     // the nodes' corner values: from the buffer that the caller kept from this step's forward call, else derived by the sums kernel (small layers:
     // by each wavefront that needs them)
     size_t const v_bytes     = align256((size_t)O * NN * sizeof(float));
     bool const   have_tables = tables.holds_tables && tables_fit(tables, 2 * v_bytes);
-    size_t const own_bytes   = small ? 0 : align256((size_t)O * own_words * sizeof(uint32_t));
+    size_t const own_bytes   = (small || few) ? 0 : align256((size_t)O * own_words * sizeof(uint32_t));
     size_t const const_bytes = small ? 0 : c.bn ? align256((size_t)O * sizeof(NodeConsts) + sizeof(uint32_t)) : 0;     // (and the word `discard` behind them)
     size_t const part_bytes  = slab_count > 1 ? align256((size_t)slab_count * slab_bytes) : 0;
     size_t const bits_bytes  = (from_fp32 && !have_bits) ? align256((size_t)c.input_node_size * c.x_stride * sizeof(uint32_t)) : 0;
     char *base = nullptr;
-    if (arena_get(v_bytes + own_bytes + const_bytes + part_bytes + bits_bytes, &base, st)) { return 1; }
+    size_t const entry_bytes = few ? align256(few_entry_bytes(N, O)) : 0;
+    if (arena_get(v_bytes + own_bytes + const_bytes + part_bytes + entry_bytes + bits_bytes, &base, st)) { return 1; }
     float    *V      = reinterpret_cast<float *>(base);
     uint32_t *own    = reinterpret_cast<uint32_t *>(base + v_bytes);
     NodeConsts *consts = reinterpret_cast<NodeConsts *>(base + v_bytes + own_bytes);
     float    *part   = reinterpret_cast<float *>(base + v_bytes + own_bytes + const_bytes);
-    uint32_t *bits   = reinterpret_cast<uint32_t *>(base + v_bytes + own_bytes + const_bytes + part_bytes);
+    float4   *entries = reinterpret_cast<float4 *>(base + v_bytes + own_bytes + const_bytes + part_bytes);
+    uint32_t *bits   = reinterpret_cast<uint32_t *>(base + v_bytes + own_bytes + const_bytes + part_bytes + entry_bytes);
     if (have_tables) { V = reinterpret_cast<float *>(reinterpret_cast<char *>(tables.buf) + v_bytes); }
     if (have_bits) { c.x = packed.bits; }
     else if (from_fp32) {
@@ -857,10 +882,11 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     s.lut_binarize = c.lut_binarize; s.bias = c.bias;
     s.node_size = O; s.frame_size = c.frame_size; s.x_stride = c.x_stride; s.dy_stride = c.frame_stride;
     s.slab = slab; s.slab_count = slab_count; s.tiles = make_tile_divisor(tile_count);
-    s.own = small ? nullptr : own; s.own_stride = own_words; s.partial = part;
+    s.own = (small || few) ? nullptr : own; s.own_stride = own_words; s.partial = part;
     s.fold.mean = c.mean; s.fold.rstd = c.rstd; s.fold.gamma = c.gamma; s.fold.beta = c.beta; s.fold.inv_frames = 1.0f / (float)c.frame_size;
     s.fold.frame_size = c.frame_size; s.fold.lo = 0.5f - c.bias; s.fold.hi = 0.5f + c.bias;
     s.fold.dW = c.dW; s.fold.overwrite = dw_overwrite; s.fold.node_consts = small ? nullptr : consts;
+    s.fold.entries = few ? entries : nullptr;
     static std::atomic<uint32_t> calls{1};          // (0 is what new scratch memory mostly holds: see CornerFoldArgs::call)
     s.fold.discard = reinterpret_cast<uint32_t *>(consts + O); s.fold.call = calls.fetch_add(1, std::memory_order_relaxed);
     bool const dy_quads = c.frame_stride >= ((c.frame_size + 3) & ~3);      // rows of dy hold whole groups of four frames: one 16-byte load per lane and pass
@@ -878,6 +904,15 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     }
     if (dy_quads ? (c.bn ? launch_corner_backward<N, true, true>(s, slab_count, st) : launch_corner_backward<N, false, true>(s, slab_count, st))
                  : (c.bn ? launch_corner_backward<N, true, false>(s, slab_count, st) : launch_corner_backward<N, false, false>(s, slab_count, st))) { return 1; }
+
+    if (few) {
+        FewInputsArgs f{};
+        f.x = reinterpret_cast<uint32_t const *>(c.x); f.idx = c.idx; f.dy = c.dy; f.dx = c.dx; f.entries = reinterpret_cast<few_f32x4 const *>(s.fold.entries); f.node_consts = consts;
+        f.discard = s.fold.discard; f.call = s.fold.call;
+        f.input_node_size = c.input_node_size; f.node_size = O; f.frame_size = c.frame_size;
+        f.x_stride = c.x_stride; f.dy_stride = c.frame_stride; f.dx_stride = c.frame_stride;
+        return c.bn ? launch_dx_few_inputs<N, true>(f, st) : launch_dx_few_inputs<N, false>(f, st);
+    }
 
     DxTableArgs t{};
     // Frames per pass: a term's table and its loads are shared by the steps of a pass, so long passes where all the rows of dy and of indices

@@ -20,6 +20,9 @@
 
 namespace bbhip {
 
+// quads of a node's table for lut_dx_few_inputs_kernel: (gain, E, d0, d1) of every corner, then (d2 .. d5)
+constexpr int few_entry_quads(int n) { return (n > 2 ? 2 : 1) << n; }
+
 struct CornerFoldArgs {
     float const *mean, *rstd;           // batch-norm
     float gamma, beta, inv_frames;
@@ -32,6 +35,7 @@ struct CornerFoldArgs {
     // each call, so that nothing has to be cleared ahead; a stale equal value only sends the dx kernel to its slower walk
     uint32_t *discard;
     uint32_t call;
+    float4 *entries;                    // the node's table for lut_dx_few_inputs_kernel (null: none)
 };
 
 // A[p] and B[p] of the dx kernel are, for a connection with difference d[p] = V[input at hi] - V[input at lo],
@@ -54,6 +58,8 @@ __device__ __forceinline__ void corner_fold(CornerFoldArgs const &a, CornerFoldI
 {
     constexpr int NN = 1 << N;
     float G = D;
+    float const inv_step = 1.0f / (a.hi - a.lo);
+    float gain = inv_step, e = 0.0f;                                    // of the lane's corner, for a.entries
     if (BN) {
         float const mean = q.mean, rstd = q.rstd;
         float const t = batch_norm_output(v, mean, rstd, a.gamma, a.beta);
@@ -64,11 +70,25 @@ __device__ __forceinline__ void corner_fold(CornerFoldArgs const &a, CornerFoldI
         float const scale = -(a.gamma * s1) * (rstd * rstd) * rstd * a.inv_frames;
         G = __builtin_fmaf(g, a.gamma * rstd, n * __builtin_fmaf(v - mean, scale, shift));
         uint64_t const open = __ballot(!(t <= 0.0f || t >= 1.0f));
-        float const inv_step = 1.0f / (a.hi - a.lo);
+        gain = __builtin_amdgcn_inverse_ballot_w64(open) ? a.gamma * rstd * inv_step : 0.0f;
+        e = __builtin_fmaf(v - mean, scale * inv_step, shift * inv_step);
         // (one value that is not finite makes its corner's sum such)
         bool const discard = __ballot((t <= 0.0f || t >= 1.0f) && !(fabsf(D) < __builtin_inff())) != 0;
         if (lane == 0 && discard && a.node_consts != nullptr) { *a.discard = a.call; }
         if (lane == 0 && a.node_consts != nullptr) { a.node_consts[node] = NodeConsts{mean, a.gamma * rstd * inv_step, shift * inv_step, scale * inv_step, open, 0}; }
+    }
+    if (a.entries != nullptr) {
+        float d[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < N; ++k) {                                   // V[k at hi] - V[k at lo]
+            float const o = lane_xor(v, 1 << k);
+            d[k] = ((lane >> k) & 1) ? v - o : o - v;
+        }
+        if (lane < NN) {
+            float4 *const to = a.entries + (size_t)node * few_entry_quads(N) + lane;
+            to[0] = make_float4(gain, e, d[0], d[1]);
+            if (N > 2) { to[NN] = make_float4(d[2], d[3], d[4], d[5]); }
+        }
     }
     // per input: (G0, G1) -> ((1 - lo) G0 + (1 - hi) G1, lo G0 + hi G1), and 1 - lo = hi: either lane keeps hi of its own and takes lo of the other's
 #pragma unroll

@@ -101,6 +101,19 @@ constexpr SumsForm corner_sums_form(int frame_size, int slab_count)
     return (slab_count > 1 || frame_size > kBlockSlab) ? kSumsLong : frame_size <= kShortSlab ? kSumsShort : kSumsBlock;
 }
 
+// Whether dx over two-valued inputs is formed node by node, with the sums of all inputs in registers (lut_dx_few_inputs_kernel), instead of input by input from
+// kept corner indices.  It reads dy once where the other reads it once per connection, and asks for frames for every compute unit (a workgroup
+// takes 512) and for nodes enough to pay for its set-up and closing sums.  Backward call, input by input and node by node, batch-norm unless said otherwise:
+// 27 inputs x 216 nodes x 230400 frames 117 and 90 us, x 115200 64.7 and 53.6, x 80000 50.2 and 49.1, x 50000 40.2 and 44.5; 9 x 72 x 230400 48.6 and 38.5;
+// 6 x 216 x 262144 142 and 88; four inputs per node, 9 x 100 x 230400 48.8 and 40.2; two, 9 x 216 x 100000 41.7 and 35.6.  Few connections in all, or for each
+// input: 27 x 24 x 230400 25.2 and 25.7, 18 x 24 x 400000 34.6 and 35.2, 12 x 16 x 180000, two per node, plain, 13.9 and 16.4; but 27 x 36 x 700000 68.6 and 63.9.
+constexpr int kFewInputs = 28, kFewInputNodes = 4096;
+inline bool few_inputs_dx(int n, int input_node_size, int node_size, int frame_size)
+{
+    long long const links = (long long)node_size * n;
+    return input_node_size <= kFewInputs && node_size <= kFewInputNodes && frame_size > 191 * 512 && links >= 200 && links >= 8LL * input_node_size;
+}
+
 // The shortest list that the wavefronts of a workgroup share in lut_dx_kernel (real-valued inputs), in a launch that would otherwise have `groups` workgroups of
 // four inputs each.  Its terms take long enough for lists from eight items where the launch falls short of wavefronts: training call of batch-norm
 // layers, six inputs per node, shared and not, 69 inputs x 66 nodes x 906 frames (list of 13) 10.4 and 15.0 us, 1500 x 800 x 700 (14) 20.6 and 23.0, 1024 x 1024 x

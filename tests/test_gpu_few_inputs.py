@@ -1,0 +1,89 @@
+"""GPU parity of dx formed node by node (layers of few inputs over many frames, two-valued inputs): widths, one to 28 inputs, last words, last pairs of
+frames, last rounds of nodes, gradients that are not finite behind a closed window."""
+import numpy as np
+import pytest
+import torch
+
+from binarybrain_amd import synth
+from util import host
+
+pytestmark = pytest.mark.gpu
+LEAST = 191 * 512 + 1           # frames
+
+
+def layer(n, I, O, F, seed):
+    rng = np.random.default_rng(seed)
+    gen = torch.Generator(device="cuda"); gen.manual_seed(seed)
+    idx = torch.from_numpy(synth.wiring(rng, I, O, n) if I >= n else rng.integers(0, I, (O, n)).astype(np.int32)).cuda()
+    W = torch.rand((O, 1 << n), device="cuda", generator=gen)
+    x = torch.randint(-(1 << 31), 1 << 31, (I, synth.frame_stride_bit(F)), device="cuda", generator=gen).to(torch.int32)
+    dy = torch.full((O, synth.frame_stride_fp32(F)), float("nan"), device="cuda")            # what lies behind the frames enters nothing
+    dy[:, :F] = torch.randn((O, F), device="cuda", generator=gen)
+    return idx, W, x, dy
+
+
+def reference(n, idx, W, x, dy, F, bias, norm=None):
+    """dx in 64 bits, by the corner values and their differences; norm: (mean, rstd, gamma, beta) of a batch-norm layer"""
+    O, I, dev = idx.shape[0], x.shape[0], "cuda"
+    hi, lo = 0.5 + bias, 0.5 - bias
+    p = torch.arange(1 << n, device=dev)
+    V = torch.zeros((O, 1 << n), dtype=torch.float64, device=dev)
+    for i in range(1 << n):
+        f = torch.ones(1 << n, dtype=torch.float64, device=dev)
+        for k in range(n):
+            v = torch.where((p >> k) & 1 == 1, hi, lo).double()
+            f *= v if (i >> k) & 1 else 1 - v
+        V += W[:, i:i + 1].double() * f
+    words, shift = x[:, :(F + 31) // 32], torch.arange(32, device=dev, dtype=torch.int32)
+    bits = ((words[:, :, None] >> shift) & 1).reshape(I, -1)[:, :F]
+    dx = torch.zeros((I, F), dtype=torch.float64, device=dev)
+    for o in range(O):
+        corner = sum(bits[idx[o, k].long()].long() << k for k in range(n))
+        g = dy[o, :F].double()
+        if norm is not None:
+            mean, rstd, gamma, beta = norm[0][o].double(), norm[1][o].double(), norm[2], norm[3]
+            t = (V[o] - mean) * rstd * gamma + beta
+            g = torch.where(((t > 0) & (t < 1))[corner], g, torch.zeros_like(g))
+            v = V[o][corner] - mean
+            g = gamma * rstd * (g - g.sum() / F - v * rstd * rstd * (g * v).sum() / F)
+        for k in range(n):
+            slope = (V[o][p | (1 << k)] - V[o][p & ~(1 << k)]) / (hi - lo)
+            dx[idx[o, k].long()] += slope[corner] * g
+    return dx
+
+
+@pytest.mark.parametrize("n, I, O, F", [(6, 28, 38, LEAST), (6, 27, 216, LEAST + 30), (5, 9, 41, LEAST + 1), (4, 1, 50, LEAST + 127), (3, 13, 67, LEAST + 129), (2, 25, 121, LEAST + 510)])
+def test_dx_node_by_node(n, I, O, F):
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    idx, W, x, dy = layer(n, I, O, F, 10 * n + O)
+    rev = ops.reverse_table(idx, I)
+    mean, rstd = W.mean(dim=1).contiguous(), (0.5 / W.std(dim=1)).contiguous()
+    for norm in (None, (mean, rstd, 0.7, 0.5)):
+        dW = torch.zeros_like(W)
+        if norm is None:
+            dx = ops.bit_stochastic_lut_backward(n, x, dy, idx, W, dW, F, rev, bias=0.25)
+        else:
+            dx = ops.bit_differentiable_lut_backward(n, x, dy, idx, W, dW, F, mean, rstd, rev, gamma=0.7, beta=0.5, bias=0.25)
+        want = reference(n, idx, W, x, dy, F, 0.25, norm)
+        # a sum over an input's connections, in fp32: their number times half a unit of rounding, relative to the largest sum, and as much for each factor
+        links = int(rev[:, 0].max())
+        assert float((dx[:, :F] - want).abs().max()) <= 2 * links * 2.0 ** -24 * float(want.abs().max()) + 1e-6, norm is None
+
+
+def test_a_discarded_gradient_may_hold_anything():
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    n, I, O, F = 6, 27, 40, LEAST + 3
+    idx, W, x, dy = layer(n, I, O, F, 4)
+    rev = ops.reverse_table(idx, I)
+    mean, rstd = W.mean(dim=1).contiguous(), (2.0 / W.std(dim=1)).contiguous()
+    y = ops.bit_stochastic_lut_forward(n, x, idx, W, F, dy.shape[1], bias=0.25)[:, :F].double()
+    t = (y - mean[:, None].double()) * rstd[:, None].double() + 0.5
+    closed = (t < -1e-3) | (t > 1.001)
+    assert 0.2 < float(closed.double().mean()) < 0.95
+    zeros, poisoned = dy.clone(), dy.clone()
+    zeros[:, :F][closed] = 0.0
+    poisoned[:, :F][closed] = torch.tensor([np.inf, -np.inf, np.nan, 3.0e38], device="cuda")[torch.arange(int(closed.sum()), device="cuda") % 4]
+    got = [host(ops.bit_differentiable_lut_backward(n, x, g, idx, W, torch.zeros_like(W), F, mean, rstd, rev, gamma=1.0, beta=0.5, bias=0.25))[:, :F] for g in (zeros, poisoned)]
+    assert np.isfinite(got[1]).all() and np.array_equal(*got)
