@@ -88,6 +88,17 @@ def test_binary_to_real(ops, shape, aligned):
     assert np.array_equal(dx[:, :F], oracle.binary_to_real_backward(dy, I, Fy, fm, x_stride=xs)[:, :F])
 
 
+@pytest.mark.parametrize("mux", [1, 2, 3, 5, 7, 8, 9, 15, 17])
+@pytest.mark.parametrize("fm", [1, 31, 32, 33, 63, 65])
+def test_binary_to_real_row_groups(ops, mux, fm):
+    """packed rows are read up to eight at a time and 32 frames at a time: every remainder of both"""
+    O, Fy = 3, 67
+    rng = np.random.default_rng(100 * mux + fm)
+    xb = synth.bernoulli_bits(rng, O * mux, Fy * fm, (Fy * fm + 31) // 32)
+    y = host(ops.binary_to_real_forward(dev(xb), O, Fy, fm, y_stride=Fy))
+    assert np.array_equal(y, oracle.binary_to_real_forward(xb, O, Fy, fm, y_stride=Fy, bit=True))
+
+
 @pytest.mark.parametrize("shape", [(6144, 1024), (70, 37), (3, 1), (1, 5000), (70000, 3), (216, 230400 // 64)])
 @pytest.mark.parametrize("aligned", [True, False])
 def test_binarize_and_hard_tanh(ops, shape, aligned):
