@@ -2244,9 +2244,17 @@ int bbhip_fp32_ClassifierTail_ForwardBackward(float const *dev_x_buf, float *dev
     size_t const lds = 5 * CH * 64 * sizeof(float) + (size_t)ch_size * n * sizeof(int);
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
-    launch(classifier_tail_kernel<CH>, dim3((unsigned)ceil_div(frame_stride, 64)), dim3(64 * CH), lds, st, dev_x_buf, dev_y_buf, dev_dx_buf,
-                       dev_input_index, dev_t_buf, dev_dy_buf, dev_loss_buf, dev_accuracy_buf, dev_category_buf, t_sum,
-                       output_sum ? 1.0f : 1.0f / (float)n, n, input_node_size, ch_size, frame_size, frame_stride, binarize_input);
+    float const scale = output_sum ? 1.0f : 1.0f / (float)n;
+    if (tail_small(n, input_node_size, ch_size, frame_stride)) {
+        launch(classifier_tail_small_kernel, dim3((unsigned)ceil_div(frame_stride, kTailFrames)), dim3(kWave), 0, st, dev_x_buf, dev_y_buf, dev_dx_buf,
+                           dev_input_index, dev_t_buf, dev_dy_buf, dev_loss_buf, dev_accuracy_buf, dev_category_buf, t_sum,
+                           scale, n, input_node_size, ch_size, frame_size, frame_stride, binarize_input);
+    }
+    else {
+        launch(classifier_tail_kernel<CH>, dim3((unsigned)ceil_div(frame_stride, 64)), dim3(64 * CH), lds, st, dev_x_buf, dev_y_buf, dev_dx_buf,
+                           dev_input_index, dev_t_buf, dev_dy_buf, dev_loss_buf, dev_accuracy_buf, dev_category_buf, t_sum,
+                           scale, n, input_node_size, ch_size, frame_size, frame_stride, binarize_input);
+    }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }

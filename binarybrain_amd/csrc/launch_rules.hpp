@@ -170,6 +170,17 @@ inline int binary_unit_words(int words, int node_size)
 // 4.0 / 6.9 and 3.6 / 6.9, the more so the longer they are.
 inline bool pool_four_frames(int frame_size) { return frame_size >= 16 || frame_size % 4 == 0; }
 
+// Whether the classifier tail runs with a row of 16 lanes per frame (classifier_tail_small_kernel): where there are as many inputs as connections (the wiring policies then
+// give every input to one node, which that form writes at once; a table of the caller's own that shares inputs takes 10 us instead of 7), channels fill half a row or more, and frames are few, of which it has four to a wavefront and 16 bytes of a row to a cache line.  70 -> 10 nodes, by a
+// wavefront per channel and by a row of lanes: 64 frames 6.35 and 4.40 us, 1024 6.69 and 4.91, 2048 6.72 and 5.45, 4000 6.82 and 6.24, 6000 6.93 and 6.91, 16384 8.6 and
+// 12.9, 65536 20.6 and 31.8; 60 inputs, 1024 frames, 6.4 and 9.1; 80 -> 5 nodes, 2000 frames 6.5 and 7.0; 30 inputs per
+// node 7.1 and 8.0.
+constexpr int kTailInputs = 16;                 // most inputs of a node there
+inline bool tail_small(int n, int input_node_size, int ch_size, int frame_stride)
+{
+    return n <= kTailInputs && ch_size >= 8 && input_node_size == ch_size * n && frame_stride <= 4096;
+}
+
 // Rows that share a workgroup of 256 threads in the pooling kernels, `lanes` threads each.  A row has a workgroup of its own where sharing saves no more than
 // one or two idle wavefronts of it and there are workgroups for every compute unit either way: up to 256 rows (120 rows x 203 frames, backward, 3.31 us shared and
 // 3.08 not), and where whole wavefronts stream through memory (48600 x 256 forward 35.4 and 33.3, backward 82.1 and 79.7; 46740 x 512 backward 151.8 and

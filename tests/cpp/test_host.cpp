@@ -425,6 +425,14 @@ int main(void)
         for (auto const &r : rows) { CHECK((bbhip::binary_unit_words(r.words, r.nodes) == 64) == (r.short_units < r.long_units)); }
     }
 
+    // the classifier tail by a wavefront per channel or by a row of lanes, where both were measured (microseconds)
+    {
+        struct { int n, inputs, channels, stride; double wavefront, row; } const rows[] = {{7, 70, 10, 64, 6.35, 4.40}, {7, 70, 10, 1152, 6.69, 4.91}, {7, 70, 10, 2176, 6.72, 5.45},
+            {12, 192, 16, 1152, 12.4, 7.35}, {7, 70, 10, 16512, 8.64, 12.9}, {7, 70, 10, 65664, 20.6, 31.8}, {30, 90, 3, 640, 7.07, 8.04}, {7, 60, 10, 1152, 6.43, 9.11},
+            {16, 80, 5, 2176, 6.45, 6.95}, {15, 45, 3, 640, 4.86, 5.48}};
+        for (auto const &r : rows) { CHECK(bbhip::tail_small(r.n, r.inputs, r.channels, r.stride) == (r.row < r.wavefront)); }
+    }
+
     // rows that share a workgroup in the pooling kernels, where both were measured (microseconds): at most 3 % slower than the faster
     {
         struct { int nodes, lanes; double shared, own; } const rows[] = {{120, 51, 3.31, 3.08}, {180, 64, 3.12, 2.93}, {48600, 64, 82.1, 79.7}, {50445, 64, 35.0, 32.9},

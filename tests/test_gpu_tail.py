@@ -237,6 +237,32 @@ def test_classifier_tail_in_one_launch(ops, case, mean):
     assert torch.equal(dx0, dx2) and torch.equal(loss0, loss2) and acc2 is None
 
 
+@pytest.mark.parametrize("wired", ["apart", "anyhow", "few"])
+@pytest.mark.parametrize("CH, n, F", [(8, 1, 1), (9, 3, 5), (10, 7, 63), (16, 13, 66), (13, 16, 130), (8, 9, 2000), (10, 7, 4030), (10, 7, 4100)])
+def test_classifier_tail_of_as_many_inputs_as_connections(ops, CH, n, F, wired):
+    """as many inputs as the nodes take: each its own, some left out and others shared, or nearly all left out; up to 4096 columns, 16 channels and 16 inputs per node, and beyond.
+    Logits beyond all bounds too."""
+    import torch
+    I, S = CH * n, synth.frame_stride_fp32(F)
+    rng = np.random.default_rng(I + F)
+    idx = (rng.permutation(I) if wired == "apart" else rng.integers(0, I if wired == "anyhow" else 1 + I // 20, I)).reshape(CH, n).astype(np.int32)
+    x = np.zeros((I, S), np.float32); x[:, :F] = rng.integers(0, 2, (I, F)) if F % 2 else rng.standard_normal((I, F))
+    if F > 60:
+        x[0, 3], x[I - 1, 11], x[I // 2, 20], x[:, 30] = np.nan, np.inf, -np.inf, -np.inf
+    t = np.zeros((CH, S), np.float32)
+    t[rng.integers(0, CH, F), np.arange(F)] = 1.0
+    t[:, F // 2] = 0.0
+    t[:, F // 3] = 0.5                                                   # targets on every channel
+    xd, td, idxd = dev(x), dev(t), dev(idx)
+    y0 = ops.average_lut_forward(xd, idxd, F, False, False, mean=True)
+    dy0, loss0, t_sum = ops.loss_softmax_cross_entropy(y0, td, CH, 1, F)
+    acc0, cat0 = ops.metrics_categorical_accuracy(y0, td, CH, 1, F)
+    dx0 = ops.average_lut_backward(dy0, idxd, I, F)
+    y1, dx1, loss1, acc1, cat1, dy1 = ops.classifier_tail(xd, idxd, td, F, t_sum=t_sum, mean=True, want_dy=True)
+    for got, want in ((y1[:, :F], y0[:, :F]), (dy1[:, :F], dy0[:, :F]), (dx1, dx0), (loss1, loss0), (acc1, acc0), (cat1, cat0)):
+        assert np.array_equal(host(got), host(want), equal_nan=got.dtype.is_floating_point)
+
+
 def test_classifier_tail_limits(ops):
     import torch
     x = torch.zeros((300, 64), device="cuda"); t = torch.zeros((4, 64), device="cuda")
