@@ -295,6 +295,12 @@ void launch_forward(FwdArgs const &a, int npw, hipStream_t st)
     if constexpr (XMODE == kXBit || XMODE == kXBinary) {
         // two-valued inputs: the corner-value kernel wherever the caller prepared the values (one node per wavefront)
         if (a.V != nullptr) {
+            if constexpr (KIND == 0 || KIND == 1) {
+                if (a.quad_passes == 0) { launch((lut_forward_quads_kernel<N, XMODE, YMODE, KIND, 0>), grid, block, 0, st, a); return; }
+                if (a.quad_passes == 1) { launch((lut_forward_quads_kernel<N, XMODE, YMODE, KIND, 1>), grid, block, 0, st, a); return; }
+                if (a.quad_passes == 2) { launch((lut_forward_quads_kernel<N, XMODE, YMODE, KIND, 2>), grid, block, 0, st, a); return; }
+                if (a.quad_passes == 4) { launch((lut_forward_quads_kernel<N, XMODE, YMODE, KIND, 4>), grid, block, 0, st, a); return; }
+            }
             if constexpr (KIND != 3 && (XMODE == kXBit || (YMODE == kYBinarize && KIND == 1))) {
                 if (a.node_waves > 0) {
                     bool const fused = (KIND == 1) && a.stat_mode == kStatInline;
@@ -310,15 +316,17 @@ void launch_forward(FwdArgs const &a, int npw, hipStream_t st)
                     return;
                 }
             }
-            if constexpr (XMODE == kXBit) {
+            if constexpr (XMODE == kXBit && KIND == 3) {
                 // 32-byte scalar loads where they stay inside the row pitch and never straddle a unit
                 if (a.x_stride % 8 == 0 && a.chunk % 256 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 3u) == 0) {
                     launch((lut_forward_corner_kernel<N, XMODE, YMODE, KIND, true>), grid, block, 0, st, a);
                     return;
                 }
             }
-            launch((lut_forward_corner_kernel<N, XMODE, YMODE, KIND>), grid, block, 0, st, a);
-            return;
+            if constexpr (XMODE == kXBinary || KIND == 3) {
+                launch((lut_forward_corner_kernel<N, XMODE, YMODE, KIND>), grid, block, 0, st, a);
+                return;
+            }
         }
     }
     if (npw == 2) { launch((lut_forward_kernel<N, XMODE, YMODE, KIND, 2>), grid, block, 0, st, a); }
@@ -557,13 +565,14 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
     bool const byte_bits  = corner && c.xmode == kXBit && c.frame_size > 1024;
     bool const byte_fused = (c.bn == 1) && corner && c.frame_size > 1024 && c.frame_size <= kByteFusedFrames && fwd_chunk_frames_env() == 0 &&
                             (byte_bits || (fixed == nullptr && (long long)c.node_size * c.frame_size <= (1 << 21)));
+    // up to kQuadMost frames: all frames of a node in one place, a wavefront per 256
+    bool const quads = corner && c.frame_size <= kQuadMost;
+    int const quad_passes = quads ? forward_quad_passes(c.node_size, c.frame_size) : -1;
     // wavefronts per node: a block of 2048 frames for each, up to a workgroup
-    int node_waves = (byte_bits || byte_fused) ? 1 : 0;
+    int node_waves = quads ? (quad_passes != 1 || c.frame_size <= kQuadFrames ? 1 : c.frame_size <= 2 * kQuadFrames ? 2 : kWavesPerBlk) : (byte_bits || byte_fused) ? 1 : 0;
     while (byte_fused && node_waves < kByteWaves && node_waves * kByteBlock < c.frame_size) { node_waves *= 2; }
-    int const tile_count  = ceil_div(c.node_size, node_waves > 1 ? (node_waves < kWavesPerBlk ? kWavesPerBlk / node_waves : 1) : kWavesPerBlk * npw);
-    // Batch-norm training pass of a small batch on the corner-value kernels: one unit per node, so that the wavefronts that write a
-    // node's output can sum the node's statistics themselves (kStatInline) and the statistics launch falls away.  BBHIP_FWD_CHUNK set in the environment keeps its say.
-    bool const one_unit   = byte_fused || ((c.bn == 1) && corner && c.frame_size <= 1024 && fwd_chunk_frames_env() == 0);
+    int const tile_count  = ceil_div(c.node_size, (quads || node_waves > 1) ? (node_waves < kWavesPerBlk ? kWavesPerBlk / node_waves : 1) : kWavesPerBlk * npw);
+    bool const one_unit   = byte_fused || quads;
     int const chunk       = byte_fused ? ceil_div(c.frame_size, kByteBlock) * kByteBlock : one_unit ? 1024 :
                             (byte_bits && fwd_chunk_frames_env() == 0) ? kByteBlock : fwd_chunk_frames(c.xmode, c.frame_size, tile_count);
     int const chunk_count = ceil_div(c.frame_size, chunk);
@@ -628,7 +637,7 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
         if ((long long)input_rows * row_blocks + (long long)chunk_count * tile_count > 0x7fffffffLL) { return fail("forward: grid too large"); }
         a.pack = PackRider{reinterpret_cast<float const *>(call.x), packed.bits, call.x_stride, packed.row_words, make_tile_divisor(row_blocks), input_rows * row_blocks};
     }
-    a.node_waves = node_waves;
+    a.node_waves = node_waves; a.quad_passes = quad_passes;
     a.y_quads = (c.y_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(c.y) & 15u) == 0) ? 1 : 0;
 
     int kind = 0;
@@ -1150,7 +1159,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         f.dy = c.dy; f.dy_stride = c.frame_stride;
         f.node_size = c.output_node_size; f.frame_size = c.frame_size; f.x_stride = c.x_stride;
         f.chunk = stat_chunk; f.chunk_count = stat_chunk_count; f.tiles = make_tile_divisor(stat_tiles);
-        f.bias = c.bias; f.gamma = c.gamma; f.beta = c.beta;
+        f.bias = c.bias; f.gamma = c.gamma; f.beta = c.beta; f.quad_passes = -1;
         if (dispatch_forward<N>(c.xmode, kYClamp, 3, f, npw, st)) { return 1; }
         BBHIP_LAUNCH_CHECK();
         if (!stat_launch) {

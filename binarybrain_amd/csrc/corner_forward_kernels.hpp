@@ -282,4 +282,207 @@ __global__ __launch_bounds__(kByteWaves * kWave) void lut_forward_bytes_kernel(F
     }
 }
 
+static_assert(kQuadFrames == 4 * kWave && kQuadMost == kWavesPerBlk * kQuadFrames, "four frames per lane, a workgroup per node");
+// Up to kQuadMost frames: a.node_waves wavefronts (1, 2 or 4) = one node, PASSES x 256 frames each, four consecutive ones per lane and pass (PASSES 0: up to 64 frames, one per lane).  All kinds that need the node's frames
+// in one place: plain (0), batch-norm (1) with running statistics or those of the call (kStatInline), which the node's wavefronts add up and exchange in LDS.
+// A frame's corner index is formed from the input words' four bits (spread to bytes by a multiplication) or from the fp32 frames, its corner value fetched once from the
+// lane that holds it, and what follows is arithmetic on the value.  The fp32 frames of a small training pass may also be packed, by extra workgroups.
+// Such a launch is a chain (wiring, inputs, index, value, sums, output), and the less a wavefront does in turn the shorter.  Against a wavefront per node in
+// steps of 64 frames, whose input masks were scalar loads, training calls on packed bits: 70 nodes x 1024 frames 5.8 -> 3.6 us, 1024 x 1024 6.0 -> 4.9, 6144 x 1024
+// 9.7 -> 9.5, 700 x 1000 5.9 -> 4.2, 210 x 236 4.4 -> 3.5, 360 x 64 3.95 -> 3.5; inference 4000 x 1024 9.5 -> 5.6, 8000 x 1000 10.8 -> 8.2, 120 x 8 3.5 -> 3.0.
+template <int N, int XMODE, int YMODE, int KIND, int PASSES>
+__global__ __launch_bounds__(kBlock) void lut_forward_quads_kernel(FwdArgs a)
+{
+    static_assert((XMODE == kXBit || XMODE == kXBinary) && (KIND == 0 || KIND == 1), "two-valued inputs, all frames of a node");
+    // LANE: consecutive frames of a lane; PASSES 0: one pass of one frame per lane, up to 64 frames
+    constexpr int NN = 1 << N, LANE = PASSES == 0 ? 1 : 4, P = PASSES == 0 ? 1 : PASSES;
+    __shared__ float sums[kWavesPerBlk][2];
+    int const B = a.tiles.count;
+    if constexpr (XMODE == kXBinary && YMODE == kYBinarize && KIND == 1) {
+        if ((int)blockIdx.x >= B) {
+            int row, block;
+            split_tile(blockIdx.x - B, a.pack.row_blocks, row, block);
+            binarize_pack4_block(a.pack.x, a.pack.bits, a.frame_size, a.pack.x_stride, a.pack.y_stride, row, block);
+            return;
+        }
+    }
+    int const wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave)), lane = threadIdx.x & (kWave - 1);
+    int const nw = a.node_waves, sub = wave & (nw - 1), slot = wave / nw;
+    int node = xcd_remap(blockIdx.x, B) * (kWavesPerBlk / nw) + slot;
+    bool const live = node < a.node_size;
+    if (!live) {
+        if (nw == 1) { return; }
+        node = a.node_size - 1;                      // (with a barrier ahead: repeats the last node and stores nothing)
+    }
+    int const f0 = sub * kQuadFrames + LANE * lane;              // (PASSES != 1: one wavefront per node)
+
+    int in[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) { in[k] = a.idx[node * N + k]; }
+    int const i = lane & (NN - 1);
+    float t = 0.0f, corner = 0.0f, c0 = 0.0f, table_c = 0.0f;
+    bool const own_tables = a.W_inline != nullptr;
+    if (own_tables) { t = a.W_inline[(size_t)node * NN + i]; }
+    else {
+        corner = a.V[(size_t)node * NN + i];
+        if (KIND == 1) { c0 = a.C[(size_t)node * NN]; }
+    }
+    uint32_t const x_bytes = XMODE == kXBit ? (uint32_t)((a.frame_size + 31) >> 5) * 4u : quad_row_bytes(a.frame_size, a.x_stride >= ((a.frame_size + 3) & ~3));
+    __amdgpu_buffer_rsrc_t rows[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) { rows[k] = row_descriptor(a.x, in[k], a.x_stride, x_bytes); }
+    uint32_t w[XMODE == kXBit ? P : 1][N];
+    std::conditional_t<LANE == 4, float4, float> x[XMODE == kXBit ? 1 : N];
+    auto fetch = [&](int p) {                        // (past the row: zeros)
+        int const f = f0 + p * kQuadFrames;
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            if constexpr (XMODE == kXBit) { w[p][k] = __builtin_amdgcn_raw_buffer_load_b32(rows[k], (uint32_t)(f >> 5) * 4u, 0, 0); }
+            else if constexpr (LANE == 1) { x[k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows[k], (uint32_t)f * 4u, 0, 0)); }
+            else if (a.x_stride >= ((a.frame_size + 3) & ~3)) { x[k] = load_quad<true>(rows[k], (uint32_t)f * 4u); }
+            else { x[k] = load_quad<false>(rows[k], (uint32_t)f * 4u); }
+        }
+    };
+    if constexpr (XMODE == kXBit) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) { fetch(p); }
+    }
+    else { fetch(0); }
+
+    // the node's tables (as in lut_forward_corner_kernel)
+    bool clamp_store = false;
+    float table_w = 0.0f;
+    if (own_tables) {
+        if (a.clamp_W != nullptr) {
+            float const tc = fminf(a.clamp_hi, fmaxf(a.clamp_lo, t));
+            clamp_store = (tc != t);
+            t = tc;
+        }
+        table_w = t;
+        if (a.lut_binarize) { t = (t > 0.5f) ? 1.0f : 0.0f; }
+        table_c = centred_butterfly<N>(t, i);
+        corner = corner_butterfly<N>(table_c, i, a.bias);
+        c0 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(table_c)));
+    }
+
+    float v[P][LANE];                                // the frames' corner values
+    float s1 = 0.0f, s2 = 0.0f;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        if (PASSES > 1 && p * kQuadFrames >= a.frame_size) { break; }              // wave-uniform
+        uint32_t at[LANE];                           // corner indices, times 4
+        if constexpr (LANE == 1) {
+            uint32_t c = 0;
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                uint32_t bit;
+                if constexpr (XMODE == kXBit) { bit = (w[0][k] >> (f0 & 31)) & 1u; }
+                else                          { bit = x[k] > 0.5f ? 1u : 0u; }
+                c |= bit << k;
+            }
+            at[0] = c << 2;
+        }
+        else if constexpr (XMODE == kXBit) {
+            uint32_t quad = 0;
+#pragma unroll
+            for (int k = 0; k < N; ++k) { quad |= ((((w[p][k] >> (f0 & 31)) & 15u) * 0x00204081u) & 0x01010101u) << (k + 2); }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { at[j] = (quad >> (8 * j)) & 0xffu; }
+        }
+        else {
+            if (p > 0) { fetch(p); }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { at[j] = 0; }
+#pragma unroll
+            for (int k = N - 1; k >= 0; --k) {
+                at[0] = 2 * at[0] + (x[k].x > 0.5f ? 1 : 0); at[1] = 2 * at[1] + (x[k].y > 0.5f ? 1 : 0);
+                at[2] = 2 * at[2] + (x[k].z > 0.5f ? 1 : 0); at[3] = 2 * at[3] + (x[k].w > 0.5f ? 1 : 0);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { at[j] <<= 2; }
+        }
+#pragma unroll
+        for (int j = 0; j < LANE; ++j) { v[p][j] = __int_as_float(__builtin_amdgcn_ds_bpermute((int)at[j], __float_as_int(corner))); }
+        if (KIND == 1 && a.stat_mode == kStatInline) {
+#pragma unroll
+            for (int j = 0; j < LANE; ++j) {
+                float const d = (f0 + p * kQuadFrames + j < a.frame_size) ? v[p][j] - c0 : 0.0f;
+                s1 += d;
+                s2 = __builtin_fmaf(d, d, s2);
+            }
+        }
+    }
+
+    float mean = 0.0f, var = 0.0f, rstd = 1.0f;
+    if (KIND == 1) {
+        if (a.stat_mode == kStatInline) {
+            s1 = wave_sum(s1);
+            s2 = wave_sum(s2);
+            if (nw > 1) {
+                if (lane == 0) { sums[wave][0] = s1; sums[wave][1] = s2; }
+                __syncthreads();
+                s1 = 0.0f; s2 = 0.0f;
+                for (int k = 0; k < nw; ++k) { s1 += sums[slot * nw + k][0]; s2 += sums[slot * nw + k][1]; }
+            }
+            batch_statistics(s1, s2, c0, a.frame_size, mean, var, rstd);
+        }
+        else { forward_statistics(a, node, lane, c0, mean, var, rstd); }
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        int const f = f0 + p * kQuadFrames, frames = a.frame_size - f;              // frames: how many of the lane's four there are, and more
+        if (PASSES > 1 && p * kQuadFrames >= a.frame_size) { break; }
+        uint32_t m = 0;                              // the lane's bits of the packed output
+#pragma unroll
+        for (int j = 0; j < LANE; ++j) {
+            float y = (KIND == 1) ? batch_norm_output(v[p][j], mean, rstd, a.gamma, a.beta) : v[p][j];
+            if (YMODE == kYClamp) { v[p][j] = __builtin_amdgcn_fmed3f(y, 0.0f, 1.0f); }
+            else {
+                m |= (y > 0.5f && j < frames) ? 1u << j : 0u;
+                v[p][j] = (y > 0.5f) ? 1.0f : 0.0f;
+            }
+        }
+        if (live && frames > 0 && YMODE != kYBit) {
+            float *const row = reinterpret_cast<float *>(a.y) + (size_t)node * a.y_stride + f;
+            if constexpr (LANE == 1) { __builtin_nontemporal_store(v[p][0], row); }
+            else if (a.y_quads && frames >= 4) {
+                typedef float f32x4 __attribute__((ext_vector_type(4)));
+                f32x4 const q = {v[p][0], v[p][1], v[p][2], v[p][3]};
+                __builtin_nontemporal_store(q, reinterpret_cast<f32x4 *>(row));
+            }
+            else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) { if (j < frames) { row[j] = v[p][j]; } }
+            }
+        }
+        if (YMODE == kYBit || (YMODE == kYBinarize && a.y_bits != nullptr)) {       // a word of 32 / LANE lanes
+            constexpr int kWordLanes = 32 / LANE;
+            if constexpr (LANE == 1) {
+                uint64_t const all = __ballot(m != 0);
+                m = (lane & 32) ? (uint32_t)(all >> 32) : (uint32_t)all;
+            }
+            else {
+                m <<= 4 * (lane & 7);
+                m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xf, 0xf, true);      // quad_perm [1, 0, 3, 2]
+                m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xf, 0xf, true);      // quad_perm [2, 3, 0, 1]
+                m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xf, 0xf, true);     // row_half_mirror
+            }
+            if (live && frames > 0 && (lane & (kWordLanes - 1)) == 0) {
+                if (YMODE == kYBit) { reinterpret_cast<uint32_t *>(a.y)[(size_t)node * a.y_stride + (f >> 5)] = m; }
+                else                { a.y_bits[(size_t)node * a.y_bits_stride + (f >> 5)] = m; }
+            }
+        }
+    }
+
+    if (sub != 0) { return; }
+    if (KIND == 1) { forward_store_statistics(a, node, live, 0, lane, mean, var, rstd); }
+    if (YMODE == kYBinarize) { zero_packed_tail(a, 0, node, live, lane); }
+    if (YMODE == kYBit)      { zero_output_padding(a, 0, node, live, lane); }
+    if (own_tables && live && lane < NN) {
+        if (clamp_store)         { a.clamp_W[(size_t)node * NN + lane] = table_w; }
+        if (a.C_out != nullptr)  { a.C_out[(size_t)node * NN + lane] = table_c; }
+        if (a.V_out != nullptr)  { a.V_out[(size_t)node * NN + lane] = corner; }
+    }
+}
+
 }  // namespace bbhip

@@ -1,4 +1,4 @@
-// Corner indices of two-valued inputs, 32 frames per lane at a time: shared by the forward and the backward kernels over packed bits.
+// Corner indices of two-valued inputs, 32 frames per lane at a time, and rows read four frames per lane: shared by the forward and the backward kernels.
 #pragma once
 
 #include "lut_math.hpp"
@@ -44,6 +44,26 @@ __device__ __forceinline__ void wave_fence(void)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// four consecutive frames of a row from byte offset off; QUADS: the row holds whole groups of four
+template <bool QUADS>
+__device__ __forceinline__ float4 load_quad(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t row_off = 0)
+{
+    if constexpr (QUADS) {
+        auto const q = __builtin_amdgcn_raw_buffer_load_b128(r, off, row_off, 0);
+        return make_float4(__uint_as_float(q[0]), __uint_as_float(q[1]), __uint_as_float(q[2]), __uint_as_float(q[3]));
+    }
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { v[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off + 4 * j, row_off, 0)); }
+    return make_float4(v[0], v[1], v[2], v[3]);
+}
+
+// valid bytes of a row for load_quad: whole groups of four where the row holds them (frames past the last read 0 or the row's padding)
+__device__ __forceinline__ uint32_t quad_row_bytes(int frame_size, bool quads)
+{
+    return (uint32_t)(quads ? (frame_size + 3) & ~3 : frame_size) * 4u;
 }
 
 }  // namespace bbhip

@@ -150,6 +150,12 @@ inline bool dx_wide_passes(int input_node_size, int output_node_size, int frame_
 // 78 and 97 (four).
 inline bool im2col_frames_first(int f_tiles, int tile_frames) { return tile_frames == 64 && f_tiles % 8 == 0; }
 
+// Passes of 256 frames that a wavefront of lut_forward_quads_kernel makes (0: up to 64 frames, one per lane, 7372 nodes x 31 5.8 -> 4.9 us): one, the node's passes side by side (they wait for each other where they exchange sums), or
+// all, one after another, where nodes alone fill the device.  Batch-norm training call, side by side and one after another: 700 nodes x 1000 frames 4.25 and 4.55 us,
+// 1024 x 1024 4.90 and 5.14; 1500 x 600 5.71 and 4.72, 4000 x 300 6.7 and 5.3, 6144 x 1024 15.4 and 9.5.
+constexpr int kQuadFrames = 256, kQuadMost = 1024;               // frames of a pass, most frames of a node there
+inline int forward_quad_passes(int node_size, int frame_size) { return frame_size <= 64 ? 0 : (node_size <= 1024 || frame_size <= kQuadFrames) ? 1 : frame_size <= 2 * kQuadFrames ? 2 : 4; }
+
 // Packed rows whose padding the caller wants as 0: the wavefront of a row's last unit writes that much of it, an iteration per 64 words, and what a longer pitch
 // leaves is a launch of its own (zero_row_ends_kernel).  BinaryLut5, rows of 1000 frames, by the wavefronts and by the launch: 1000 rows of 2080 words 3.8 and
 // 5.7 us, 10000 words 8.7 and 11.3; 4 rows of 100000 words 42.1 and 5.8, 64 of 1000000 397 and 36.

@@ -227,7 +227,7 @@ struct FwdArgs {
     void        *y;
     int const   *idx;
     float const *C;             // [O][2^N] centred coefficients
-    float const *V;             // [O][2^N] corner values (two-valued inputs: lut_forward_corner_kernel)
+    float const *V;             // [O][2^N] corner values (two-valued inputs)
     float const *mean;          // BN: per node (nullptr otherwise)
     float const *rstd;
     float       *stat_partial;  // STATS: [O][chunk][2] partial sums of (v - C0), (v - C0)^2;  kind 3: of g, g (v - mean)
@@ -272,7 +272,8 @@ struct FwdArgs {
     // lut_forward_bytes_kernel (node_waves > 0 where a call takes it): wavefronts that share a node in a one-launch training pass, and whether
     // rows of fp32 output start on 16 bytes
     int   node_waves, y_quads;
-    // lut_forward_corner_kernel over the fp32 frames of a small batch-norm training pass: the last pack.blocks workgroups make the packed copy of the
+    int   quad_passes;          // up to kQuadMost frames: the form of lut_forward_quads_kernel, by node_waves wavefronts per node; -1: another kernel
+    // lut_forward_quads_kernel over the fp32 frames of a small batch-norm training pass: the last pack.blocks workgroups make the packed copy of the
     // input that the backward call takes
     PackRider pack;
     int   pad_end;              // packed output: the wavefront of a node's last unit writes 0 from behind the last frame's word up to this one (0: nothing)
@@ -281,7 +282,6 @@ struct FwdArgs {
 // kStatInline: the call has one unit per node, so the wavefront that writes a node's output first sums the node's statistics
 // itself (a pass of its own over the unit) instead of reading them from a statistics launch
 enum StatMode : int { kStatGiven = 0, kStatRunning = 1, kStatPartial = 2, kStatInline = 3 };
-constexpr int kInlineUnitPasses = 4;         // kStatInline: passes (of 256 frames) whose corner indices a wavefront keeps in registers
 constexpr int kInlineStatUnits = 4 * kWave; // most units whose partial sums a wavefront adds up itself: up to four loads per lane
 
 // What a forward kernel does with the LUT output v of (node, frame f = f0 + lane): accumulate statistics (kinds 2, 3) or
@@ -647,9 +647,8 @@ __device__ __forceinline__ CornerTables corner_tables(FwdArgs const &a, float v,
 
 // A corner-value wavefront's pass over U wavefront-steps from frame fb of its unit (see lut_forward_corner_kernel).
 // OWN: where the corner indices come from.  kOwnNone: from the gathered inputs; kOwnMemory: from the bytes that the statistics launch
-// of the call kept (FwdArgs::own_index); kOwnRegister: from `own`, which an earlier pass of the same wavefront over the same frames
-// left there.  `own` always returns the indices of the pass, byte u = 4 x the index of frame fb + 64 u + lane.
-enum OwnIndex : int { kOwnNone = 0, kOwnMemory = 1, kOwnRegister = 2 };
+// of the call kept (FwdArgs::own_index).  `own` returns the indices of the pass, byte u = 4 x the index of frame fb + 64 u + lane.
+enum OwnIndex : int { kOwnNone = 0, kOwnMemory = 1 };
 // RAGGED: the pass may reach beyond the unit's last frame (else all of its U steps are whole, and nothing is masked)
 template <int N, int XMODE, int YMODE, int KIND, bool WIDE, int OWN, bool RAGGED = true>
 __device__ __forceinline__ void corner_pass(FwdArgs const &a, void const *(&rows)[N], CornerTables tabs, int node, int lane, int fb,
@@ -752,7 +751,8 @@ __device__ __forceinline__ void corner_unit_pass(FwdArgs const &a, void const *(
 }
 
 // ------------------------------------------------------------------------------------------------
-//  Forward for two-valued inputs (packed bits, or fp32 frames binarized at 0.5): the LUT output is one of the 2^N corner
+//  Forward for two-valued inputs that the kernels of corner_forward_kernels.hpp do not take (more than kQuadMost fp32 frames whose row count nobody told, and
+//  the statistics of a polynomial backward pass): the LUT output is one of the 2^N corner
 //  values V of the node.  A lane builds the corner index of its frame from the N input bits (one add-with-carry per input:
 //  index = 2 index + bit, the bit arriving as a lane mask in a scalar register pair) and fetches V[index] from the lane
 //  that holds it (ds_bpermute): N + 2 instructions per (node, 64 frames) instead of the polynomial's 45.
@@ -770,14 +770,6 @@ __global__ __launch_bounds__(kBlock) void lut_forward_corner_kernel(FwdArgs a)
     static_assert(OWN == kOwnNone || (OWN == kOwnMemory && XMODE == kXBit && !WIDE && FWD_KIND == 1), "kept corner indices: output launch only");
     constexpr int NN = 1 << N;
     int const B    = a.chunk_count * a.tiles.count;
-    if constexpr (XMODE == kXBinary && YMODE == kYBinarize && FWD_KIND == 1) {
-        if ((int)blockIdx.x >= B) {
-            int row, block;
-            split_tile(blockIdx.x - B, a.pack.row_blocks, row, block);
-            binarize_pack4_block(a.pack.x, a.pack.bits, a.frame_size, a.pack.x_stride, a.pack.y_stride, row, block);
-            return;
-        }
-    }
     int const lid  = xcd_remap(blockIdx.x, B);
     int ck, tile;
     split_tile(lid, a.tiles, ck, tile);
@@ -815,7 +807,7 @@ __global__ __launch_bounds__(kBlock) void lut_forward_corner_kernel(FwdArgs a)
                                    : (void const *)(reinterpret_cast<float const *>(a.x) + (size_t)in * a.x_stride);
     }
     float mean = 0.0f, rstd = 1.0f;
-    if (a.W_inline == nullptr && (FWD_KIND == 2 || (FWD_KIND == 1 && (a.stat_mode == kStatPartial || a.stat_mode == kStatInline)))) {
+    if (a.W_inline == nullptr && (FWD_KIND == 2 || (FWD_KIND == 1 && a.stat_mode == kStatPartial))) {
         c0 = a.C[(size_t)node * NN];
     }
     float var = 0.0f;
@@ -824,54 +816,12 @@ __global__ __launch_bounds__(kBlock) void lut_forward_corner_kernel(FwdArgs a)
     int const f_end   = min(f_begin + a.chunk, a.frame_size);
     int const f_last  = a.frame_size - 1;
     float s1 = 0.0f, s2 = 0.0f;
-    bool f_done = false;
 
-    if (FWD_KIND == 1) {
-        if (a.stat_mode == kStatInline) {
-            // one unit per node: the sums of the statistics kind, by the same steps in the same order, then what the
-            // statistics launch and the partial-sum read would have delivered (same bits)
-            // up to kInlineUnitPasses passes of four steps: the corner indices of the passes stay in registers for the output pass,
-            // which then gathers nothing
-            constexpr bool kKeep = (XMODE == kXBinary || WIDE) && (OWN == kOwnNone);
-            bool const keep = kKeep && (f_end - f_begin <= kInlineUnitPasses * 4 * kWave);      // wave-uniform
-            uint32_t kept[kInlineUnitPasses];
-            CornerTables const stat_tabs = corner_tables<YMODE, 2>(a, __int_as_float(corner), 0.0f, 1.0f, c0);
-            if (keep) {
-                if constexpr (kKeep) {
-#pragma unroll
-                    for (int q = 0; q < kInlineUnitPasses; ++q) {
-                        int const fb = f_begin + q * 4 * kWave;
-                        kept[q] = 0;
-                        if (fb < f_end) { corner_pass_any<N, XMODE, YMODE, 2, WIDE, kOwnNone>(a, rows, stat_tabs, node, lane, fb, f_end, f_last, s1, s2, kept[q]); }
-                    }
-                }
-            }
-            else { corner_unit_pass<N, XMODE, YMODE, 2, WIDE, OWN>(a, rows, stat_tabs, node, lane, f_begin, f_end, f_last, s1, s2); }
-            batch_statistics(wave_sum(s1), wave_sum(s2), c0, a.frame_size, mean, var, rstd);
-            mean = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(mean)));
-            var  = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(var)));
-            rstd = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(rstd)));
-            s1 = 0.0f; s2 = 0.0f;
-            if (keep) {
-                if constexpr (kKeep) {
-                    CornerTables const out_tabs = corner_tables<YMODE, FWD_KIND>(a, __int_as_float(corner), mean, rstd, c0);
-#pragma unroll
-                    for (int q = 0; q < kInlineUnitPasses; ++q) {
-                        int const fb = f_begin + q * 4 * kWave;
-                        if (fb < f_end) { corner_pass_any<N, XMODE, YMODE, FWD_KIND, WIDE, kOwnRegister>(a, rows, out_tabs, node, lane, fb, f_end, f_last, s1, s2, kept[q]); }
-                    }
-                }
-                f_done = true;
-            }
-        }
-        else { forward_statistics(a, node, lane, c0, mean, var, rstd); }
-    }
+    if (FWD_KIND == 1) { forward_statistics(a, node, lane, c0, mean, var, rstd); }
     if (FWD_KIND == 3) { mean = a.mean[node]; rstd = a.rstd[node]; }
 
-    if (!f_done) {
-        CornerTables const tabs = corner_tables<YMODE, FWD_KIND>(a, __int_as_float(corner), mean, rstd, c0);
-        corner_unit_pass<N, XMODE, YMODE, FWD_KIND, WIDE, OWN>(a, rows, tabs, node, lane, f_begin, f_end, f_last, s1, s2);
-    }
+    CornerTables const tabs = corner_tables<YMODE, FWD_KIND>(a, __int_as_float(corner), mean, rstd, c0);
+    corner_unit_pass<N, XMODE, YMODE, FWD_KIND, WIDE, OWN>(a, rows, tabs, node, lane, f_begin, f_end, f_last, s1, s2);
     if (FWD_KIND == 2 || FWD_KIND == 3) { forward_store_stats(a, ck, node, true, lane, s1, s2); }
     if (FWD_KIND == 1) { forward_store_statistics(a, node, true, ck, lane, mean, var, rstd); }
     if (YMODE == kYBinarize && (FWD_KIND == 0 || FWD_KIND == 1)) { zero_packed_tail(a, ck, node, true, lane); }
