@@ -305,7 +305,7 @@ void launch_forward(FwdArgs const &a, int npw, hipStream_t st)
                 if (a.node_waves > 0) {
                     bool const fused = (KIND == 1) && a.stat_mode == kStatInline;
                     int const waves = a.node_waves > kWavesPerBlk ? a.node_waves : kWavesPerBlk;
-                    int const index_blocks = fused ? waves / a.node_waves * ceil_div(a.frame_size, kByteBlock) : waves;
+                    int const index_blocks = fused ? waves / a.node_waves * a.out_blocks : waves;
                     launch((lut_forward_bytes_kernel<N, XMODE, YMODE, KIND>), grid, dim3(waves * kWave), forward_bytes_lds(waves, index_blocks), st, a);
                     return;
                 }
@@ -575,12 +575,14 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
     bool const one_unit   = byte_fused || quads;
     int const chunk       = byte_fused ? ceil_div(c.frame_size, kByteBlock) * kByteBlock : one_unit ? 1024 :
                             (byte_bits && fwd_chunk_frames_env() == 0) ? kByteBlock : fwd_chunk_frames(c.xmode, c.frame_size, tile_count);
-    int const chunk_count = ceil_div(c.frame_size, chunk);
+    // (in one launch: workgroups that share a node's output, each with statistics of its own)
+    int const blocks      = ceil_div(c.frame_size, kByteBlock), out_blocks = c.ymode == kYBit ? blocks : forward_out_blocks(tile_count, node_waves, blocks);
+    int const chunk_count = byte_fused ? ceil_div(blocks, out_blocks) : ceil_div(c.frame_size, chunk);
     if ((long long)chunk_count * tile_count > 0x7fffffffLL) { return fail("forward: grid too large"); }
 
     size_t const c_bytes    = align256((size_t)c.node_size * NN * sizeof(float));
     size_t const v_bytes    = corner ? c_bytes : 0;
-    size_t const stat_bytes = (c.bn == 1) ? align256((size_t)chunk_count * c.node_size * 2 * sizeof(float)) : 0;
+    size_t const stat_bytes = (c.bn == 1) ? align256((size_t)(one_unit ? 1 : chunk_count) * c.node_size * 2 * sizeof(float)) : 0;
     size_t const bits_bytes = (pack && !to_caller) ? align256((size_t)input_rows * c.x_stride * sizeof(uint32_t)) : 0;
     // fp32 frames of binary mode whose row count nobody told (nothing to pack ahead), batch-norm training pass in two launches: the
     // statistics launch keeps the corner index that it forms of every (node, frame), a byte each, and the output launch reads those
@@ -637,11 +639,11 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
         if ((long long)input_rows * row_blocks + (long long)chunk_count * tile_count > 0x7fffffffLL) { return fail("forward: grid too large"); }
         a.pack = PackRider{reinterpret_cast<float const *>(call.x), packed.bits, call.x_stride, packed.row_words, make_tile_divisor(row_blocks), input_rows * row_blocks};
     }
-    a.node_waves = node_waves; a.quad_passes = quad_passes;
+    a.node_waves = node_waves; a.quad_passes = quad_passes; a.out_blocks = out_blocks;
     a.y_quads = (c.y_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(c.y) & 15u) == 0) ? 1 : 0;
 
     int kind = 0;
-    if (c.bn == 1 && corner && chunk_count == 1) {
+    if (c.bn == 1 && one_unit) {
         // one unit per node on a corner-value kernel: its wavefronts sum the statistics of their node themselves before they write its output
         a.stat_mode = kStatInline; a.momentum = c.momentum;
         a.mean_out = c.mean; a.rstd_out = c.rstd; a.running_mean = c.running_mean; a.running_var = c.running_var;

@@ -55,6 +55,16 @@ struct WordLoad {
     }
 };
 
+// the word of eight lanes of four frames each, from the lanes' four bits
+__device__ __forceinline__ uint32_t quad_word(uint32_t m, int lane)
+{
+    m <<= 4 * (lane & 7);
+    m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xf, 0xf, true);                  // quad_perm [1, 0, 3, 2]
+    m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xf, 0xf, true);                  // quad_perm [2, 3, 0, 1]
+    m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xf, 0xf, true);                 // row_half_mirror
+    return m;
+}
+
 // One wavefront = one node x one unit of frames in blocks of 2048 (kinds 0, 1, 2 as in lut_forward_kernel), or, for a batch-norm training pass
 // in one launch (kStatInline), a.node_waves wavefronts = one node and all its frames.  A lane loads the words of 32 frames of each input and turns
 // them into corner indices (corner_bytes: two instructions per frame and lane where the scalar lane masks of lut_forward_corner_kernel take
@@ -63,7 +73,8 @@ struct WordLoad {
 //   output      the index bytes go through LDS to the lanes that hold four consecutive frames each (16-byte stores of y; the packed copy collects
 //               its words over a block and leaves by one store), packed output is assembled by the lane that formed the indices.
 // In one launch the indices of all frames stay in LDS between the two, so nothing is gathered or formed twice, and the wavefronts of a node
-// exchange their two sums there.  The kernel is bound by the fp32 output where there is one, else by its chain of latencies (wiring, words, tables).
+// exchange their two sums there; where nodes are few, several workgroups hold the indices of a part of a node's frames each and write its output
+// (forward_out_blocks), and all of them sum the statistics of all frames.  The kernel is bound by the fp32 output where there is one, else by its chain of latencies (wiring, words, tables).
 // Measured against lut_forward_corner_kernel's statistics and output launches: 4096 x 4096 x 8192 fp32 output 36 us (3.8 TB/s written) instead of
 // 25 + 31; 2001 x 3003 x 5005 packed 14 us instead of 15 + 13; 216 nodes x 230400 frames (two launches) 14 + 46 us instead of 22 + 46; packed
 // inference of 2048 nodes x 3500 frames 6.2 us instead of 11.5.
@@ -89,9 +100,12 @@ __global__ __launch_bounds__(kByteWaves * kWave) void lut_forward_bytes_kernel(F
         if (nw == 1) { return; }
         node = a.node_size - 1;                      // (with barriers ahead: repeats the last node and stores nothing)
     }
-    int const f_begin = ck * a.chunk, f_end = min(f_begin + a.chunk, a.frame_size);
+    int const f_begin = (YMODE != kYBit && fused) ? 0 : ck * a.chunk, f_end = min(f_begin + a.chunk, a.frame_size);
     int const blocks = (f_end - f_begin + kByteBlock - 1) / kByteBlock;
-    uint32_t *const bytes = lds + waves * (2 * kWave + 2) + (fused ? slot * blocks : wave) * kBlockWords;
+    // in one launch with fp32 output: the blocks whose output is this workgroup's
+    bool const parted = YMODE != kYBit && fused && a.out_blocks < blocks;
+    int const out_first = parted ? ck * a.out_blocks : 0, out_end = parted ? min(out_first + a.out_blocks, blocks) : blocks;
+    uint32_t *const bytes = lds + waves * (2 * kWave + 2) + (fused ? slot * (parted ? a.out_blocks : blocks) : wave) * kBlockWords;
 
     int in[N];
 #pragma unroll
@@ -168,6 +182,29 @@ __global__ __launch_bounds__(kByteWaves * kWave) void lut_forward_bytes_kernel(F
         if (frames < 32) { word &= (frames > 0) ? (1u << frames) - 1u : 0u; }
         if (live && frames > 0) { reinterpret_cast<uint32_t *>(a.y)[(size_t)node * a.y_stride + (f >> 5)] = word; }
     };
+    // fp32 output of one pass of 256 frames whose index bytes are in LDS
+    auto output_pass = [&](uint32_t const *pass, int fb) {
+        float *const row = reinterpret_cast<float *>(a.y) + (size_t)node * a.y_stride;
+        int const f = fb + 4 * lane;
+        uint32_t const at = pass[lane];
+        typedef float f32x4 __attribute__((ext_vector_type(4)));
+        f32x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) { v[j] = lookup(out_tab, at, j); }
+        if (YMODE == kYBinarize && a.y_bits != nullptr) {
+            uint32_t m = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { m |= (v[j] != 0.0f && f + j < f_end) ? 1u << j : 0u; }
+            m = quad_word(m, lane);
+            if (live && f < f_end && (lane & 7) == 0) { a.y_bits[(size_t)node * a.y_bits_stride + (f >> 5)] = m; }
+        }
+        if (!live) { return; }
+        if (a.y_quads && f + 3 < f_end) { __builtin_nontemporal_store(v, reinterpret_cast<f32x4 *>(row + f)); }
+        else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { if (f + j < f_end) { row[f + j] = v[j]; } }
+        }
+    };
     // fp32 output of a block whose index bytes are in LDS
     auto output_rows = [&](uint32_t const *block, int base) {
         float *const row = reinterpret_cast<float *>(a.y) + (size_t)node * a.y_stride;
@@ -185,10 +222,7 @@ __global__ __launch_bounds__(kByteWaves * kWave) void lut_forward_bytes_kernel(F
                 uint32_t m = 0;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) { m |= (v[j] != 0.0f && f + j < f_end) ? 1u << j : 0u; }
-                m <<= 4 * (lane & 7);
-                m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xf, 0xf, true);          // quad_perm [1, 0, 3, 2]
-                m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xf, 0xf, true);          // quad_perm [2, 3, 0, 1]
-                m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xf, 0xf, true);         // row_half_mirror
+                m = quad_word(m, lane);
                 mine = ((lane & 7) == p) ? m : mine;
             }
             if (!live) { continue; }
@@ -223,7 +257,7 @@ __global__ __launch_bounds__(kByteWaves * kWave) void lut_forward_bytes_kernel(F
             if (XMODE != kXBit) { words.load(base, lane, f_end, w); }
             corner_bytes<N, 2>(w, quad);
             if (XMODE == kXBit && b + nw < blocks) { words.load(base + nw * kByteBlock, lane, f_end, w); }
-            if (fused) { keep(quad, bytes + b * kBlockWords); }
+            if (fused && (YMODE == kYBit || (b >= out_first && b < out_end))) { keep(quad, bytes + (b - out_first) * kBlockWords); }
             statistics(quad, f_end - (base + 32 * lane));
         }
         if (KIND == 2) { forward_store_stats(a, ck, node, live, lane, s1, s2); }
@@ -238,16 +272,27 @@ __global__ __launch_bounds__(kByteWaves * kWave) void lut_forward_bytes_kernel(F
             }
             batch_statistics(s1, s2, c0, a.frame_size, mean, var, rstd);
             write_out_table(mean, rstd);
-            for (int b = sub; b < blocks; b += nw) {
-                int const base = f_begin + b * kByteBlock;
-                uint32_t const *block = bytes + b * kBlockWords;
-                if (YMODE == kYBit) {
-                    uint4 const *own = reinterpret_cast<uint4 const *>(block + 8 * lane);
-                    uint4 const lo = own[0], hi = own[1];
-                    uint32_t const q[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-                    output_word(q, base);
+            if (parted) {
+                // a few blocks for all wavefronts of the node: pass by pass, whoever formed the bytes (a barrier lies between)
+                int const passes = (out_end - out_first) * kPasses;
+                for (int q = sub; q < passes; q += nw) {
+                    int const fb = out_first * kByteBlock + q * 4 * kWave;
+                    if (fb < f_end) { output_pass(bytes + q * kWave, fb); }
                 }
-                else { output_rows(block, base); }
+            }
+            else {
+                // the blocks that this wavefront formed
+                for (int b = sub; b < blocks; b += nw) {
+                    int const base = f_begin + b * kByteBlock;
+                    uint32_t const *block = bytes + b * kBlockWords;
+                    if (YMODE == kYBit) {
+                        uint4 const *own = reinterpret_cast<uint4 const *>(block + 8 * lane);
+                        uint4 const lo = own[0], hi = own[1];
+                        uint32_t const q[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                        output_word(q, base);
+                    }
+                    else { output_rows(block, base); }
+                }
             }
         }
     }
@@ -462,10 +507,7 @@ __global__ __launch_bounds__(kBlock) void lut_forward_quads_kernel(FwdArgs a)
                 m = (lane & 32) ? (uint32_t)(all >> 32) : (uint32_t)all;
             }
             else {
-                m <<= 4 * (lane & 7);
-                m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xB1, 0xf, 0xf, true);      // quad_perm [1, 0, 3, 2]
-                m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4E, 0xf, 0xf, true);      // quad_perm [2, 3, 0, 1]
-                m |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xf, 0xf, true);     // row_half_mirror
+                m = quad_word(m, lane);
             }
             if (live && frames > 0 && (lane & (kWordLanes - 1)) == 0) {
                 if (YMODE == kYBit) { reinterpret_cast<uint32_t *>(a.y)[(size_t)node * a.y_stride + (f >> 5)] = m; }

@@ -156,6 +156,17 @@ inline bool im2col_frames_first(int f_tiles, int tile_frames) { return tile_fram
 constexpr int kQuadFrames = 256, kQuadMost = 1024;               // frames of a pass, most frames of a node there
 inline int forward_quad_passes(int node_size, int frame_size) { return frame_size <= 64 ? 0 : (node_size <= 1024 || frame_size <= kQuadFrames) ? 1 : frame_size <= 2 * kQuadFrames ? 2 : 4; }
 
+// Blocks of 2048 frames whose fp32 output a workgroup of lut_forward_bytes_kernel writes in a one-launch training pass: all of its nodes', or, where nodes are few, a part,
+// with the statistics of all frames in each of the workgroups that share a node (they cost a third of the output, and an exchange would be a launch).  Up to 256
+// workgroups, a node each, 1024 threads where rows are long: 512 of those are two rounds.  Training call, whole nodes and parts: 72 nodes x 33800 frames 10.1 and 8.2 us
+// (13.2 in parts for 512 workgroups), 24 x 33800 9.4 and 6.9, 12 x 49000 10.4 and 7.1, 24 x 12000 7.1 and 5.5, 36 x 4000 6.9 and 6.0, 5 x 20000 7.7 and 5.9.  Packed
+// output is too little to share: 24 x 33800 6.75 and 6.6, 70 x 3500 5.0 and 5.2.
+inline int forward_out_blocks(int tile_count, int node_waves, int blocks)
+{
+    int const parts = 256 / tile_count;
+    return (node_waves < 2 || parts < 2) ? blocks : parts < blocks ? ceil_div(blocks, parts) : 1;
+}
+
 // Packed rows whose padding the caller wants as 0: the wavefront of a row's last unit writes that much of it, an iteration per 64 words, and what a longer pitch
 // leaves is a launch of its own (zero_row_ends_kernel).  BinaryLut5, rows of 1000 frames, by the wavefronts and by the launch: 1000 rows of 2080 words 3.8 and
 // 5.7 us, 10000 words 8.7 and 11.3; 4 rows of 100000 words 42.1 and 5.8, 64 of 1000000 397 and 36.

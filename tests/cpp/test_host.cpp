@@ -361,6 +361,17 @@ int main(void)
               bbhip::forward_quad_passes(8000, 512) == 2 && bbhip::forward_quad_passes(8000, 513) == 4);
     }
 
+    {
+        // workgroups that share a node's fp32 output: at most 256 of them altogether, every block in one share, no share empty, none for a single wavefront or block
+        for (int tiles : {1, 2, 3, 24, 72, 85, 100, 127, 128, 129, 255, 256, 257, 4096}) {
+            for (int blocks = 1; blocks <= 24; ++blocks) {
+                int const share = bbhip::forward_out_blocks(tiles, 4, blocks), parts = (blocks + share - 1) / share;
+                CHECK(share >= 1 && share <= blocks && (parts == 1 || tiles * parts <= 256) && (parts - 1) * share < blocks);
+                CHECK(bbhip::forward_out_blocks(tiles, 1, blocks) == blocks && (tiles <= 128 || parts == 1));
+            }
+        }
+    }
+
     // dx of few inputs input by input or node by node, where both were measured (backward call, microseconds): at most 5 % slower than the faster
     {
         struct { int n, inputs, nodes, frames; double by_input, by_node; } const rows[] = {

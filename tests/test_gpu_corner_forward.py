@@ -14,6 +14,10 @@ SHAPES = [(9, 5, 1025, 0, 0), (16, 9, 2047, 2047, 67), (12, 70, 2048, 0, 0), (7,
           (11, 2, 32769, 0, 0), (6, 3, 49152, 0, 0), (6, 5, 49153, 49153, 1537), (30, 40, 55000, 0, 0)]
 
 
+# few nodes, whose output several workgroups share: two blocks and more, remainders of the shares, one to sixteen wavefronts per node
+SHAPES += [(9, 130, 2049, 0, 0), (7, 60, 6145, 6145, 0), (12, 100, 10241, 0, 0), (6, 24, 33800, 0, 0), (8, 90, 40961, 40963, 0)]
+
+
 @pytest.mark.parametrize("n", [2, 3, 4, 5, 6])
 @pytest.mark.parametrize("shape", SHAPES)
 def test_corner_forward(n, shape):
@@ -51,3 +55,19 @@ def test_corner_forward(n, shape):
         y, mean, rstd = ops.differentiable_lut_forward_training(n, dev(x), d_idx, d_W, F, *stats(), gamma=gamma, beta=beta, packed_out=copy, **kw)
         check(host(y)[:, :F], mean, rstd)
         assert np.array_equal(synth.unpack_bits(host(copy), copy.shape[1] * 32)[:, :F], host(y)[:, :F].astype(np.uint8)) and not host(copy)[:, nw:].any()
+
+
+@pytest.mark.parametrize("nodes,frames", [(24, 33800), (100, 2049), (130, 33800)])
+def test_running_statistics_of_shared_nodes_move_once(nodes, frames):
+    """However many workgroups share a node's fp32 output, its running statistics take one step per call."""
+    import torch
+    from binarybrain_amd import ops
+    rng = np.random.default_rng(frames)
+    idx = synth.wiring(rng, 12, nodes, 6); W = rng.random((nodes, 64), dtype=np.float32)
+    d_x, d_idx, d_W = dev(synth.uniform_frames(rng, 12, frames)), dev(idx), dev(W)
+    rm, rv = torch.full((nodes,), 0.25, device="cuda"), torch.ones(nodes, device="cuda")
+    want_m, want_v = host(rm), host(rv)
+    for _ in range(3):
+        _, mean, rstd = ops.differentiable_lut_forward_training(6, d_x, d_idx, d_W, frames, rm, rv, gamma=0.3, beta=0.5, momentum=0.75)
+        want_m, want_v = 0.75 * want_m + 0.25 * host(mean), 0.75 * want_v + 0.25 / host(rstd) ** 2
+    assert np.allclose(host(rm), want_m, rtol=1e-5) and np.allclose(host(rv), want_v, rtol=1e-4)
