@@ -752,13 +752,14 @@ int check_backward(BackwardCall const &c, int dxmode)
 }
 
 template <int N, bool BN, bool QUADS>
-int launch_corner_backward(CornerSumsArgs const &s, int slab_count, hipStream_t st)
+int launch_corner_backward(CornerSumsArgs const &s, int slab_count, bool node_sums, hipStream_t st)
 {
     {
         ScopedTimer tm(kTimeBackward, st);
         dim3 const grid(s.slab_count * s.tiles.count);
         SumsForm const form = corner_sums_form(s.frame_size, slab_count);
-        if (form == kSumsShort)      { launch((lut_corner_sums_kernel<N, BN, kSumsShort, QUADS>), grid, dim3(kBlock), 0, st, s); }
+        if (node_sums)               { launch((lut_corner_sums_node_kernel<N, BN, QUADS>), dim3(s.node_size), dim3(kNodeSumsWaves * kWave), 0, st, s); }
+        else if (form == kSumsShort) { launch((lut_corner_sums_kernel<N, BN, kSumsShort, QUADS>), grid, dim3(kBlock), 0, st, s); }
         else if (form == kSumsBlock) { launch((lut_corner_sums_kernel<N, BN, kSumsBlock, QUADS>), grid, dim3(kBlock), 0, st, s); }
         else                         { launch((lut_corner_sums_kernel<N, BN, kSumsLong, QUADS>), grid, dim3(kBlock), 0, st, s); }
     }
@@ -855,7 +856,9 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     size_t const slab_bytes = (size_t)O * NN * sizeof(float) * (c.bn ? 2 : 1), max_slabs = ((size_t)256 << 20) / slab_bytes;
     int slab = bwd_slab_frames() > 0 ? ceil_div(bwd_slab_frames(), 256) * 256 : corner_slab_frames(c.frame_size, tile_count, (long long)max_slabs);
     while ((size_t)ceil_div(c.frame_size, slab) > max_slabs && slab < c.frame_size) { slab *= 2; }
-    int const slab_count = ceil_div(c.frame_size, slab);
+    bool const in_one = bwd_slab_frames() == 0 && node_sums(N, O, c.frame_size);      // a workgroup per node, and a slab per wavefront of it
+    if (in_one) { slab = ceil_div(ceil_div(c.frame_size, kNodeSumsWaves), 256) * 256; }
+    int const slab_count = in_one ? 1 : ceil_div(c.frame_size, slab);
     if ((long long)slab_count * tile_count > 0x7fffffffLL) { return fail("backward: grid too large"); }
     int const own_words = ceil_div(c.frame_size, 32) * 8;
 
@@ -913,8 +916,8 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
         return dy_quads ? (c.bn ? launch_corner_small<N, true, true>(t, waves, st) : launch_corner_small<N, false, true>(t, waves, st))
                         : (c.bn ? launch_corner_small<N, true, false>(t, waves, st) : launch_corner_small<N, false, false>(t, waves, st));
     }
-    if (dy_quads ? (c.bn ? launch_corner_backward<N, true, true>(s, slab_count, st) : launch_corner_backward<N, false, true>(s, slab_count, st))
-                 : (c.bn ? launch_corner_backward<N, true, false>(s, slab_count, st) : launch_corner_backward<N, false, false>(s, slab_count, st))) { return 1; }
+    if (dy_quads ? (c.bn ? launch_corner_backward<N, true, true>(s, slab_count, in_one, st) : launch_corner_backward<N, false, true>(s, slab_count, in_one, st))
+                 : (c.bn ? launch_corner_backward<N, true, false>(s, slab_count, in_one, st) : launch_corner_backward<N, false, false>(s, slab_count, in_one, st))) { return 1; }
 
     if (few) {
         FewInputsArgs f{};

@@ -175,8 +175,9 @@ __device__ __forceinline__ auto row_sum(V4 const *block, int lane)
 // and six inputs two lanes share a column of bins (they add in turn), and the corners are counted by integer atomics (one instruction per step, and nothing
 // to add up).  6144 nodes x 1024 frames 20.5 -> 13.6 us, 6000 x 100 17.4 -> 9.6 us; four lanes per column measured the same or slower.
 // kSumsBlock: up to 2048 frames, a column for each lane (corner_sums_form has both sides of the lines).
+struct CornerSums { float v, D, n; CornerFoldInputs in; };          // lane p (of every group of 2^N lanes): of corner p
 template <int N, bool BN, int FORM, bool QUADS>
-__device__ __forceinline__ void corner_sums_unit(CornerSumsArgs const &a, SumsShared<N, BN, FORM> &sh, int node, int sl, int lane)
+__device__ __forceinline__ CornerSums corner_sums(CornerSumsArgs const &a, SumsShared<N, BN, FORM> &sh, int node, int sl, int lane, bool fold)
 {
     using T = SumsTraits<N, BN, FORM>;
     constexpr int NN = 1 << N, kPasses = T::kPasses, COLS = T::kColumns;
@@ -200,7 +201,7 @@ __device__ __forceinline__ void corner_sums_unit(CornerSumsArgs const &a, SumsSh
     for (int i = 0; i < kPasses; ++i) { dy[i] = load_quad<QUADS>(dyr, (uint32_t)(f_begin + i * 4 * kWave + 4 * lane) * 4u); }
 
     CornerFoldInputs fold_in{};
-    if (a.slab_count == 1) { fold_in = corner_fold_inputs<N, BN>(a.fold, node, lane); }
+    if (fold) { fold_in = corner_fold_inputs<N, BN>(a.fold, node, lane); }
     float v;                                                            // lane p: V[p]
     if (a.V != nullptr) { v = a.V[(size_t)node * NN + (lane & (NN - 1))]; }
     else {
@@ -342,13 +343,20 @@ __device__ __forceinline__ void corner_sums_unit(CornerSumsArgs const &a, SumsSh
         }
     }
 
-    if (a.slab_count == 1) { corner_fold<N, BN>(a.fold, fold_in, node, lane, v, D, (float)n); }
+    if (a.V_out != nullptr && sl == 0 && lane < NN) { a.V_out[(size_t)node * NN + lane] = v; }
+    return CornerSums{v, D, (float)n, fold_in};
+}
+template <int N, bool BN, int FORM, bool QUADS>
+__device__ __forceinline__ void corner_sums_unit(CornerSumsArgs const &a, SumsShared<N, BN, FORM> &sh, int node, int sl, int lane)
+{
+    constexpr int NN = 1 << N;
+    CornerSums const q = corner_sums<N, BN, FORM, QUADS>(a, sh, node, sl, lane, a.slab_count == 1);
+    if (a.slab_count == 1) { corner_fold<N, BN>(a.fold, q.in, node, lane, q.v, q.D, q.n); }
     else if (lane < NN) {
         float *out = a.partial + ((size_t)sl * a.node_size + node) * (BN ? 2 * NN : NN) + lane;
-        out[0] = D;
-        if (BN) { out[NN] = (float)n; }
+        out[0] = q.D;
+        if (BN) { out[NN] = q.n; }
     }
-    if (a.V_out != nullptr && sl == 0 && lane < NN) { a.V_out[(size_t)node * NN + lane] = v; }
 }
 
 template <int N, bool BN, int FORM, bool QUADS>
@@ -362,6 +370,26 @@ __global__ __launch_bounds__(kBlock, 2) void lut_corner_sums_kernel(CornerSumsAr
     int const node = tile * kWavesPerBlk + wv;
     if (node >= a.node_size) { return; }
     corner_sums_unit<N, BN, FORM, QUADS>(a, shared[wv], node, sl, threadIdx.x & (kWave - 1));
+}
+
+// Few nodes (node_sums): a workgroup per node, whose wavefronts take a part of up to kBlockSlab frames each (a.slab) and leave their sums in LDS to the first,
+// which folds them.  A chain of latencies like the forms of one slab, but without partial sums in memory and the launch that folds them.  Backward call of 40 inputs, six per node: 100 nodes x 4000 frames 12.6 -> 10.9 us, 130 x 10000 16.6 -> 13.9, 256 x 4500 16.5 -> 13.6.
+template <int N, bool BN, bool QUADS>
+__global__ __launch_bounds__(kNodeSumsWaves * kWave) void lut_corner_sums_node_kernel(CornerSumsArgs a)
+{
+    __shared__ SumsShared<N, BN, kSumsBlock> shared[kNodeSumsWaves];
+    static_assert((1 << N) * kWave >= 2 * kWave, "room for both sums");
+    int const wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave)), lane = threadIdx.x & (kWave - 1), node = blockIdx.x;
+    CornerSums q = corner_sums<N, BN, kSumsBlock, QUADS>(a, shared[wave], node, wave, lane, wave == 0);   // (past the last frame: zeros)
+    wave_fence();
+    float *const mine = shared[wave].bins;                              // (the bins are added up)
+    mine[lane] = q.D;
+    mine[kWave + lane] = q.n;
+    __syncthreads();
+    if (wave != 0) { return; }
+#pragma unroll
+    for (int w = 1; w < kNodeSumsWaves; ++w) { q.D += shared[w].bins[lane]; q.n += shared[w].bins[kWave + lane]; }
+    corner_fold<N, BN>(a.fold, q.in, node, lane, q.v, q.D, q.n);
 }
 
 // Several slabs per node: a workgroup per node adds them up, each wavefront every fourth slab, and folds.

@@ -101,6 +101,17 @@ constexpr SumsForm corner_sums_form(int frame_size, int slab_count)
     return (slab_count > 1 || frame_size > kBlockSlab) ? kSumsLong : frame_size <= kShortSlab ? kSumsShort : kSumsBlock;
 }
 
+// Whether a workgroup of eight wavefronts sums a node's frames (lut_corner_sums_node_kernel) instead of slabs and a launch that folds them.  Up to 2048 frames
+// for each wavefront, in one block, and up to a node per compute unit with five and six inputs, whose bins leave room for one workgroup, two with fewer.
+// Backward call of 40 inputs in slabs and by workgroups: six per node, 12 nodes x 2300 frames 10.8 and 9.5 us, 80 x 14000 15.9 and 13.4, 256 x 4500 16.6 and 13.6,
+// 256 x 16384 22.4 and 21.6; four, 30 x 10000 11.6 and 9.2, 512 x 6000 17.2 and 15.9.  Beyond: six, 80 x 24000 18.6 and 17.7, but 40 x 24000 14.9 and 15.1, 30 x
+// 100000 20.5 and 29.4; 300 x 4500 17.0 and 18.7; five, 300 x 4000 14.4 and 16.0; up to 2048 frames, one slab, 100 x 1500 9.9 and 10.2.
+constexpr int kNodeSumsWaves = 8;
+inline bool node_sums(int n, int node_size, int frame_size)
+{
+    return frame_size > kBlockSlab && frame_size <= kNodeSumsWaves * kBlockSlab && node_size <= (n > 4 ? 256 : 512);
+}
+
 // Whether dx over two-valued inputs is formed node by node, with the sums of all inputs in registers (lut_dx_few_inputs_kernel), instead of input by input from
 // kept corner indices.  It reads dy once where the other reads it once per connection, and asks for frames for every compute unit (a workgroup
 // takes 512) and for nodes enough to pay for its set-up and closing sums.  Backward call, input by input and node by node, batch-norm unless said otherwise:

@@ -372,6 +372,18 @@ int main(void)
         }
     }
 
+    // per-corner sums in slabs or a node by a workgroup, where both were measured (backward call, microseconds): at most 5 % slower than the faster
+    {
+        struct { int n, nodes, frames; double slabs, workgroups; } const rows[] = {
+            {6, 12, 2300, 10.8, 9.5}, {6, 80, 14000, 15.9, 13.4}, {6, 256, 4500, 16.6, 13.6}, {6, 256, 16384, 22.4, 21.6}, {6, 40, 24000, 14.9, 15.1}, {6, 30, 100000, 20.5, 29.4},
+            {6, 300, 4500, 17.0, 18.7}, {5, 300, 4000, 14.4, 16.0}, {5, 256, 6000, 16.1, 13.6}, {4, 30, 10000, 11.6, 9.2}, {4, 512, 6000, 17.2, 15.9}, {2, 400, 10000, 13.8, 12.3}, {6, 100, 1500, 9.9, 10.2}};
+        for (auto const &r : rows) {
+            double const taken = bbhip::node_sums(r.n, r.nodes, r.frames) ? r.workgroups : r.slabs;
+            if (taken > 1.05 * std::min(r.slabs, r.workgroups)) { std::printf("%d x %d\n", r.nodes, r.frames); CHECK(!"node_sums"); }
+        }
+        CHECK(!bbhip::node_sums(6, 256, 2048) && bbhip::node_sums(6, 256, 2049) && bbhip::node_sums(6, 256, 16384) && !bbhip::node_sums(6, 256, 16385) && !bbhip::node_sums(2, 513, 4000));
+    }
+
     // dx of few inputs input by input or node by node, where both were measured (backward call, microseconds): at most 5 % slower than the faster
     {
         struct { int n, inputs, nodes, frames; double by_input, by_node; } const rows[] = {
