@@ -929,16 +929,7 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     }
 
     DxTableArgs t{};
-    // Frames per pass: a term's table and its loads are shared by the steps of a pass, so long passes where all the rows of dy and of indices
-    // that a pass gathers from (5 bytes per node and frame) stay in an XCD's L2; halved while the launch would fall short of workgroups: a workgroup
-    // is four inputs, or one whose list its wavefronts share (27 inputs x 87 nodes x 94500 frames in passes of 256 / 512 / 1024 frames, convolutional
-    // block with 10000 / 5000 / 2500 workgroups: 125 / 117 / 122 us; 27 x 216 x 230400 371 / 348 / 346).
-    int quads = (O <= 512) ? 4 : (O <= 1024) ? 2 : 1;
-    auto const enough = [&](int q) {
-        long long const chunks = ceil_div(c.frame_size, q * 256);
-        return chunks * ceil_div(c.input_node_size, kWavesPerBlk) >= 2048 || (c.rev_stride > 16 && chunks * c.input_node_size >= 3072);
-    };
-    while (quads > 1 && !enough(quads)) { quads /= 2; }
+    int quads = dx_table_quads(N, c.input_node_size, O, c.frame_size, c.rev_stride > 16);
     if (dx_quads_env() != 0) { quads = dx_quads_env(); }
     t.far = !dy_quads || (long long)O * c.frame_stride * 4 > 0xffffffffLL || (long long)O * own_words * 4 > 0xffffffffLL ||
             (long long)O * NN * 4 > 0xffffffffLL;

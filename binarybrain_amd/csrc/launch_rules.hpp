@@ -75,6 +75,24 @@ inline int corner_small_waves(int n, bool batch_norm, int frame_size, int input_
     return items <= (!batch_norm ? 13 : n >= 5 ? 9 : 12) + links / 6000 ? 4 : 0;
 }
 
+// Passes of 256 frames, 1, 2 or 4, of a wavefront of lut_dx_table_kernel.  A term's table and its loads are shared by the passes, so more of them where the rows of
+// dy and of indices that they gather from (5 bytes per node and frame) stay in an XCD's L2, and where the launch does not fall short of workgroups: a
+// workgroup is four inputs, or one whose list its wavefronts share (27 inputs x 87 nodes x 94500 frames in passes of 256 / 512 / 1024 frames, convolutional
+// block with 10000 / 5000 / 2500 workgroups: 125 / 117 / 122 us; 27 x 216 x 230400 371 / 348 / 346).
+// Two passes, training call with one and with two: from 1000 groups of four inputs and up to 1350 nodes six inputs 560 x 1055 x 3778 32.9 and 29.4 us, 1500 x
+// 1200 x 4000 33.6 and 31.5, 3664 x 1195 x 7782 60.9 and 55.0, 333 x 469 x 5793 25.1 and 24.5; five, 632 x 1175 x 5013 37.4 and 32.8; four, 2909 x 1145 x 1358 21.2 and
+// 20.0; 35 drawn shapes with two passes here where the lines were 2048 groups and 1024 nodes 0.88 to 1.05, 0.96 on average.  Tables of five and six inputs also up to 1600 nodes where two passes end in one round of the 2048
+// workgroups that fit: 1000 x 1500 x 3000 34.4 and 30.5, 877 x 1425 x 3698 36.4 and 33.0; but 1727 x 1444 x 9479 67.0 and 68.6, 3987 x 1569 x
+// 514 19.1 and 19.9, four inputs 1888 x 1524 x 1628 22.0 and 22.5, 1000 x 2000 x 8000, six, 67.7 and 69.1.  Fewer workgroups: six, 2754 x 1341 x 498 (689) 16.2 and 17.8, 98 x 1550 x 1284 (75) 24.4 and 28.6.
+inline int dx_table_quads(int n, int input_node_size, int output_node_size, int frame_size, bool long_lists)
+{
+    auto const groups = [&](int q) { return (long long)ceil_div(frame_size, q * 256) * ceil_div(input_node_size, 4); };
+    auto const shared = [&](int q) { return long_lists && (long long)ceil_div(frame_size, q * 256) * input_node_size >= 3072; };
+    if (output_node_size <= 512 && (groups(4) >= 2048 || shared(4))) { return 4; }
+    if (output_node_size <= 1350 && (groups(2) >= 1000 || shared(2))) { return 2; }
+    return (n >= 5 && output_node_size <= 1600 && frame_size > 1024 && groups(2) >= 1000 && groups(2) <= 2048) ? 2 : 1;
+}
+
 // Whether the sixteen wavefronts that share an input's list in lut_dx_table_kernel take its items in turn (they then walk the nodes together, and rows that
 // outgrow an L2 come from behind it once) or consecutive ones.  A launch of fewer workgroups than compute units leaves the L2s room; what counts there is that
 // an item's list entry, row and index are requested one item ahead only, and consecutive entries of a long list share a cache line.  Backward call, plain,

@@ -397,6 +397,20 @@ int main(void)
         CHECK(!bbhip::few_inputs_dx(6, 29, 216, 230400) && !bbhip::few_inputs_dx(6, 27, 4097, 230400));
     }
 
+    // dx from kept indices in passes of 256 or 512 frames, where both were measured (training call, microseconds): at most 5 % slower than the faster
+    {
+        struct { int n, inputs, nodes, frames, max_fan; double one, two; } const rows[] = {
+            {6, 560, 1055, 3778, 22, 32.9, 29.4}, {5, 632, 1175, 5013, 21, 37.2, 32.8}, {6, 3664, 1195, 7782, 8, 60.8, 55.0}, {6, 807, 1033, 12218, 18, 62.8, 59.4},
+            {6, 877, 1425, 3698, 21, 36.5, 33.0}, {6, 1727, 1444, 9479, 14, 67.0, 68.6}, {6, 3987, 1569, 514, 9, 19.0, 19.9}, {5, 1833, 1530, 6448, 12, 46.9, 48.9},
+            {4, 2909, 1145, 1358, 8, 20.6, 20.0}, {2, 825, 468, 4363, 5, 18.7, 17.4}, {5, 333, 469, 5793, 14, 25.4, 24.5}, {6, 2754, 1341, 498, 11, 16.2, 17.8},
+            {6, 2046, 2018, 1150, 15, 25.6, 27.1}, {6, 98, 1550, 1284, 117, 24.2, 28.6}, {6, 585, 772, 5509, 16, 35.0, 30.2}};
+        for (auto const &r : rows) {
+            double const taken = bbhip::dx_table_quads(r.n, r.inputs, r.nodes, r.frames, r.max_fan > 15) == 1 ? r.one : r.two;
+            if (taken > 1.05 * std::min(r.one, r.two)) { std::printf("%d x %d x %d\n", r.inputs, r.nodes, r.frames); CHECK(!"dx_table_quads"); }
+        }
+        CHECK(bbhip::dx_table_quads(6, 27, 216, 230400, true) == 4 && bbhip::dx_table_quads(6, 6144, 1024, 1024, true) == 2 && bbhip::dx_table_quads(6, 4096, 4096, 8192, false) == 1);
+    }
+
     // per-corner sums of one slab: in blocks requested ahead, or all frames at once, where both were measured (sums launch, microseconds)
     {
         struct { int frames; double blocks, at_once; } const rows[] = {
