@@ -153,8 +153,9 @@ __global__ __launch_bounds__(kFewWaves * kWave) __attribute__((amdgpu_waves_per_
     constexpr int kPieces = kTable / kWave, kEach = (kPieces + kFewWaves - 1) / kFewWaves;
     uint32_t const lds_tables = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)tables;
     uint32_t const lds_rows = lds_tables + 2 * kTable * 16 + (uint32_t)wave * (kFewBatch * kFrames * 4);
+    // (M0 must be written a wait state before such a load reads it; the compiler, which does not look into the asm, would put the s_nop there too)
     auto load_to_lds = [](uint32_t lds, uint32_t off, __amdgpu_buffer_rsrc_t from, uint32_t base) {
-        asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" :: "s"(lds), "v"(off), "s"(from), "s"(base) : "memory");
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" :: "s"(lds), "v"(off), "s"(from), "s"(base) : "memory");
     };
     __amdgpu_buffer_rsrc_t const er = row_descriptor(a.entries, 0, 0, (uint32_t)a.node_size * (kQuads * 16u) + kTable * 16u);
     int const last_round = last / kRound;
