@@ -558,15 +558,16 @@ int run_forward(ForwardCall const &call, int input_rows, hipStream_t st, Scratch
         return run_forward_real_node<N>(c, st, tables);
     }
     int const npw         = corner ? 1 : fwd_nodes_per_wave();
-    // Two-valued inputs from 1025 frames: the kernel that forms the corner indices of 32 frames per lane at a time (below that most of its lanes
+    // Two-valued inputs of up to kQuadMost frames: all frames of a node in one place, a wavefront per 256.  BBHIP_FWD_CHUNK set in the environment keeps its say: units
+    // of that many frames, and a batch-norm training pass in two launches.
+    bool const quads = corner && c.frame_size <= kQuadMost && fwd_chunk_frames_env() == 0;
+    // More frames: the kernel that forms the corner indices of 32 frames per lane at a time (below that most of its lanes
     // have no frames: 11.2 us instead of 9.6 for 6144 nodes x 1024 frames, 5.3 instead of 4.0 for 1024 x 64).  A batch-norm training pass is one
     // launch of it while the indices of a node's frames fit in LDS.  fp32 frames whose row count nobody told come along, gathered, while
     // there is little to gather: a launch over all frames at a time loses the order in which the L2s hold pieces of large inputs.
-    bool const byte_bits  = corner && c.xmode == kXBit && c.frame_size > 1024;
-    bool const byte_fused = (c.bn == 1) && corner && c.frame_size > 1024 && c.frame_size <= kByteFusedFrames && fwd_chunk_frames_env() == 0 &&
+    bool const byte_bits  = corner && c.xmode == kXBit && !quads;
+    bool const byte_fused = (c.bn == 1) && corner && !quads && c.frame_size <= kByteFusedFrames && fwd_chunk_frames_env() == 0 &&
                             (byte_bits || (fixed == nullptr && (long long)c.node_size * c.frame_size <= (1 << 21)));
-    // up to kQuadMost frames: all frames of a node in one place, a wavefront per 256
-    bool const quads = corner && c.frame_size <= kQuadMost;
     int const quad_passes = quads ? forward_quad_passes(c.node_size, c.frame_size) : -1;
     // wavefronts per node: a block of 2048 frames for each, up to a workgroup
     int node_waves = quads ? (quad_passes != 1 || c.frame_size <= kQuadFrames ? 1 : c.frame_size <= 2 * kQuadFrames ? 2 : kWavesPerBlk) : (byte_bits || byte_fused) ? 1 : 0;

@@ -67,5 +67,38 @@ def main():
     print("two-valued case ok")
 
 
+def small():
+    """Forward passes of up to 1024 frames; prints the units per node that a batch-norm training pass took, told from the scratch memory that it asked for."""
+    import torch
+    from binarybrain_amd import capi
+    rng = np.random.default_rng(13)
+    I, O, F = 48, 40, 1000
+    idx = synth.wiring(rng, I, O, 6); W = synth.lut_tables(rng, O, 6)
+    x = synth.uniform_frames(rng, I, F, synth.frame_stride_fp32(F))
+    xb = oracle.binarize_forward(x, F, 0.5, bit=True)
+    d_idx, d_W, stats = dev(idx), dev(W), lambda: (torch.zeros(O, device="cuda"), torch.ones(O, device="cuda"))          # noqa: E731
+    v = oracle.bit_stochastic_lut_forward(6, xb, idx, W, F, x.shape[1], 0)[:, :F]
+    assert_fwd(host(ops.bit_stochastic_lut_forward(6, dev(xb), d_idx, d_W, F, x.shape[1], 0))[:, :F], v, "packed, plain")
+    assert_fwd(host(ops.stochastic_lut_forward(6, dev(x), d_idx, d_W, F, input_binary=True))[:, :F], v, "fp32, plain")
+    y_ref, m_ref, r_ref, _, _ = oracle.differentiable_lut_forward_training(6, x, idx, W, F, np.zeros(O, np.float32), np.ones(O, np.float32))
+    assert capi.lib().bbhip_ReleaseScratch() == 0
+    y, mean, rstd = ops.bit_differentiable_lut_forward_training(6, dev(xb), d_idx, d_W, F, *stats())
+    held = (capi.lib().bbhip_GetScratchSize() - (1 << 20)) * 2 // 3          # (a new arena is half as large again and 1 MB)
+    partial = held - 2 * O * 64 * 4                                         # behind the tables: [units][O][2] fp32, in whole pieces of 256 bytes
+    units = [u for u in range(1, 17) if 0 <= partial - (u * O * 8 + 255) // 256 * 256 < 2]
+    def check(y, mean, rstd):
+        assert np.mean(y[:, :F] != y_ref[:, :F]) < 1e-3
+        assert np.allclose(host(mean), m_ref, rtol=1e-4, atol=1e-6) and np.allclose(host(rstd), r_ref, rtol=1e-4)
+    check(synth.unpack_bits(host(y), y.shape[1] * 32), mean, rstd)
+    for kw in ({}, {"packed": ops.packed_input_buffer(I, F)}):
+        copy = ops.packed_input_buffer(O, F)
+        y, mean, rstd = ops.differentiable_lut_forward_training(6, dev(x), d_idx, d_W, F, *stats(), packed_out=copy, **kw)
+        check(host(y), mean, rstd)
+        assert np.array_equal(synth.unpack_bits(host(copy), copy.shape[1] * 32)[:, :F], host(y)[:, :F].astype(np.uint8))
+    y = ops.bit_differentiable_lut_forward_inference(6, dev(xb), d_idx, d_W, F, mean, 1 / rstd ** 2)
+    assert np.mean(synth.unpack_bits(host(y), y.shape[1] * 32)[:, :F] != y_ref[:, :F]) < 1e-3
+    print("small passes ok, units of a training pass: %s" % units)
+
+
 if __name__ == "__main__":
-    sys.exit(main())
+    sys.exit(small() if sys.argv[1:] == ["small"] else main())
