@@ -753,7 +753,7 @@ int check_backward(BackwardCall const &c, int dxmode)
 }
 
 template <int N, bool BN, bool QUADS>
-int launch_corner_backward(CornerSumsArgs const &s, int slab_count, bool node_sums, hipStream_t st)
+int launch_corner_backward(CornerSumsArgs const &s, int slab_count, bool node_sums, ReverseRows const &rows, hipStream_t st)
 {
     {
         ScopedTimer tm(kTimeBackward, st);
@@ -766,7 +766,11 @@ int launch_corner_backward(CornerSumsArgs const &s, int slab_count, bool node_su
     }
     BBHIP_LAUNCH_CHECK();
     if (slab_count > 1) {
-        launch((lut_corner_fold_kernel<N, BN>), dim3(s.node_size), dim3(kBlock), 0, st, s.fold, s.partial, s.V ? s.V : s.V_out, s.node_size, slab_count);
+        launch((lut_corner_fold_kernel<N, BN>), dim3(s.node_size + rows.inputs), dim3(kBlock), 0, st, s.fold, rows, s.partial, s.V ? s.V : s.V_out, s.node_size, slab_count);
+        BBHIP_LAUNCH_CHECK();
+    }
+    else if (rows.inputs > 0) {
+        launch(reverse_rows_kernel, dim3(rows.inputs), dim3(kBlock), 0, st, rows);
         BBHIP_LAUNCH_CHECK();
     }
     return 0;
@@ -875,14 +879,16 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     size_t const part_bytes  = slab_count > 1 ? align256((size_t)slab_count * slab_bytes) : 0;
     size_t const bits_bytes  = (from_fp32 && !have_bits) ? align256((size_t)c.input_node_size * c.x_stride * sizeof(uint32_t)) : 0;
     char *base = nullptr;
-    size_t const entry_bytes = few ? align256(few_entry_bytes(N, O)) : 0;
-    if (arena_get(v_bytes + own_bytes + const_bytes + part_bytes + entry_bytes + bits_bytes, &base, st)) { return 1; }
+    size_t const entry_bytes = few ? align256(few_entry_bytes(N, O)) : 0, rows_bytes = few ? align256(kFewMost * sizeof(int)) : 0;
+    if (arena_get(v_bytes + own_bytes + const_bytes + part_bytes + entry_bytes + rows_bytes + bits_bytes, &base, st)) { return 1; }
     float    *V      = reinterpret_cast<float *>(base);
     uint32_t *own    = reinterpret_cast<uint32_t *>(base + v_bytes);
     NodeConsts *consts = reinterpret_cast<NodeConsts *>(base + v_bytes + own_bytes);
     float    *part   = reinterpret_cast<float *>(base + v_bytes + own_bytes + const_bytes);
     float4   *entries = reinterpret_cast<float4 *>(base + v_bytes + own_bytes + const_bytes + part_bytes);
-    uint32_t *bits   = reinterpret_cast<uint32_t *>(base + v_bytes + own_bytes + const_bytes + part_bytes + entry_bytes);
+    ReverseRows rows{};
+    if (few) { rows = ReverseRows{c.rev, c.idx, c.rev_stride, O * N, c.input_node_size, reinterpret_cast<int *>(base + v_bytes + own_bytes + const_bytes + part_bytes + entry_bytes)}; }
+    uint32_t *bits   = reinterpret_cast<uint32_t *>(base + v_bytes + own_bytes + const_bytes + part_bytes + entry_bytes + rows_bytes);
     if (have_tables) { V = reinterpret_cast<float *>(reinterpret_cast<char *>(tables.buf) + v_bytes); }
     if (have_bits) { c.x = packed.bits; }
     else if (from_fp32) {
@@ -917,12 +923,12 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
         return dy_quads ? (c.bn ? launch_corner_small<N, true, true>(t, waves, st) : launch_corner_small<N, false, true>(t, waves, st))
                         : (c.bn ? launch_corner_small<N, true, false>(t, waves, st) : launch_corner_small<N, false, false>(t, waves, st));
     }
-    if (dy_quads ? (c.bn ? launch_corner_backward<N, true, true>(s, slab_count, in_one, st) : launch_corner_backward<N, false, true>(s, slab_count, in_one, st))
-                 : (c.bn ? launch_corner_backward<N, true, false>(s, slab_count, in_one, st) : launch_corner_backward<N, false, false>(s, slab_count, in_one, st))) { return 1; }
+    if (dy_quads ? (c.bn ? launch_corner_backward<N, true, true>(s, slab_count, in_one, rows, st) : launch_corner_backward<N, false, true>(s, slab_count, in_one, rows, st))
+                 : (c.bn ? launch_corner_backward<N, true, false>(s, slab_count, in_one, rows, st) : launch_corner_backward<N, false, false>(s, slab_count, in_one, rows, st))) { return 1; }
 
     if (few) {
         FewInputsArgs f{};
-        f.x = reinterpret_cast<uint32_t const *>(c.x); f.idx = c.idx; f.dy = c.dy; f.dx = c.dx; f.entries = reinterpret_cast<few_f32x4 const *>(s.fold.entries); f.node_consts = consts;
+        f.x = reinterpret_cast<uint32_t const *>(c.x); f.idx = c.idx; f.rev = c.rev; f.rev_stride = c.rev_stride; f.dy = c.dy; f.dx = c.dx; f.entries = reinterpret_cast<few_f32x4 const *>(s.fold.entries); f.node_consts = consts; f.listed = rows.listed;
         f.discard = s.fold.discard; f.call = s.fold.call;
         f.input_node_size = c.input_node_size; f.node_size = O; f.frame_size = c.frame_size;
         f.x_stride = c.x_stride; f.dy_stride = c.frame_stride; f.dx_stride = c.frame_stride;

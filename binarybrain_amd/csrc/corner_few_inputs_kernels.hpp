@@ -22,14 +22,16 @@ constexpr int kFewMost = 28;            // most inputs: 56 registers of sums
 struct FewInputsArgs {
     uint32_t const *x;                  // packed input rows
     int const   *idx;                   // [O][N]
+    int const   *rev;                   // reverse table [I][rev_stride]
     float const *dy;
     float       *dx;
     few_f32x4 const *entries;           // [O][few_entry_quads]
     NodeConsts const *node_consts;      // batch-norm
+    int const   *listed;                // [I]: see ReverseRows
     uint32_t const *discard;            // batch-norm: see CornerFoldArgs
     uint32_t call;
     int   input_node_size, node_size, frame_size;
-    int   x_stride, dy_stride, dx_stride;
+    int   x_stride, dy_stride, dx_stride, rev_stride;
 };
 
 // quads of a round's tables, whole instructions of 64 (the entries' buffer has room for that much behind the last node)
@@ -123,11 +125,55 @@ __device__ __forceinline__ void few_inputs_add(FewSums &s, int at0, float const 
                  : [at0] "s"(at0), [g0] "v"(g[0]), [g1] "v"(g[1]), [a0] "v"(a[0]), [a1] "v"(a[1]));
 }
 
+// dx of a lane's frames from the lists of the reverse table, for inputs `first`, first + kShares, ...: whatever the lists say, the tables of lut_dx_few_inputs_kernel
+// and its arithmetic.  (An entry that is no connection adds nothing.)
+template <int N, bool BN>
+__device__ __forceinline__ void few_inputs_by_lists(FewInputsArgs const &a, int first, int f_lane, bool gated)
+{
+    constexpr int NN = 1 << N, kQuads = few_entry_quads(N);
+    typedef __attribute__((address_space(4))) int const const_int;
+    typedef __attribute__((address_space(4))) NodeConsts const const_consts;
+    const_consts *consts = (const_consts *)a.node_consts;
+#pragma nounroll
+    for (int i = first; i < a.input_node_size; i += kFewWaves / kFewUnits) {
+        const_int *list = (const_int *)(a.rev + (size_t)i * a.rev_stride);
+        int const fan = list[0];
+        few_f32x2 sum = 0.0f;
+#pragma nounroll
+        for (int t = 1; t <= fan; ++t) {
+            uint32_t const e = (uint32_t)list[t], node = e / (uint32_t)N;
+            int const k = (int)(e - node * N);
+            if (node >= (uint32_t)a.node_size) { continue; }             // wave-uniform
+            const_int *in = (const_int *)(a.idx + (size_t)node * N);
+#pragma unroll
+            for (int q = 0; q < kFewFrames; ++q) {
+                int const f = min(f_lane + q, a.frame_size - 1);
+                uint32_t corner = 0;
+#pragma unroll
+                for (int j = 0; j < N; ++j) { corner |= ((a.x[(size_t)min((uint32_t)in[j], (uint32_t)a.input_node_size - 1) * a.x_stride + (f >> 5)] >> (f & 31)) & 1u) << j; }
+                float d = a.dy[(size_t)node * a.dy_stride + f];
+                if (BN && gated) {
+                    uint64_t const open = consts[node].open;
+                    uint32_t const half = (corner & 32u) ? (uint32_t)(open >> 32) : (uint32_t)open;
+                    d = ((half >> (corner & 31u)) & 1u) ? d : 0.0f;
+                }
+                float const *entry = reinterpret_cast<float const *>(a.entries + (size_t)node * kQuads + corner);
+                float const g = BN ? __builtin_fmaf(d, entry[0], entry[1]) : d * entry[0];
+                sum[q] = __builtin_fmaf(k < 2 ? entry[2 + k] : entry[NN * 4 + k - 2], g, sum[q]);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kFewFrames; ++q) { if (f_lane + q < a.frame_size) { a.dx[(size_t)i * a.dx_stride + f_lane + q] = sum[q]; } }
+    }
+}
+
 // A wavefront owns 128 frames, two consecutive ones per lane, and the sums dx[input][frame] of all (up to 28) inputs for them.  It walks the nodes; a frame's
 // corner index p comes from the input bits in registers, the frame's entry of the node's table from LDS, and each of the node's inputs k gets
 //     dx[in_k] += d_k[p] g,      g = gain[p] dy + E[p]        (A[p] = d_k[p] gain[p] and B[p] = d_k[p] E[p] of lut_dx_table_kernel; E = 0 in plain layers),
 // so that dy is read once, where a walk over every input's consumers reads it once per connection, and no corner indices are kept by the launch before.
-// The node's tables are formed by corner_fold, once per call.  The wiring is that of the index table alone (the reverse table says the same).
+// The node's tables are formed by corner_fold, once per call.
+// The wiring is that of the index table where the launch before has found the same in the reverse table (ReverseRows); else (a caller's own table that
+// leaves connections out, say) the workgroup goes by the lists, an input after another, without hurry.
 // Bound by LDS (two random 16-byte reads per frame and node: 20 clocks per 64 frames; four 8-byte reads take 18 if the compiler leaves them apart, 40 if it
 // pairs them) and by what the four wavefronts of a SIMD leave idle around it.  27 inputs x 216 nodes x 230400 frames, six per node: 80 -> 52 us (dy at 3.9 TB/s), and
 // the sums launch, which has no indices to keep, 50 -> 38; with tables formed by the workgroups themselves 59 us, with dy through registers 53.
@@ -145,6 +191,12 @@ __global__ __launch_bounds__(kFewWaves * kWave) __attribute__((amdgpu_waves_per_
     int const f_unit = (xcd_remap(blockIdx.x, gridDim.x) * kFewUnits + unit) * kFrames, f_lane = f_unit + Q * lane;
     int const last = a.node_size - 1;
     uint32_t const last_input = (uint32_t)a.input_node_size - 1;
+
+    typedef __attribute__((address_space(4))) uint32_t const const_word;
+    typedef __attribute__((address_space(4))) NodeConsts const const_consts;
+    const_consts *consts = (const_consts *)a.node_consts;
+    uint32_t const discard_word = BN ? *(const_word *)a.discard : 0u;
+    int listed = lane < a.input_node_size ? a.listed[lane] : 0;
 
     // Tables and rows of dy go from memory to LDS without a stop in registers, 1 KB per instruction: 16 bytes per lane, to the address in M0 and up.  A round's
     // tables are consecutive, a part of them for every wavefront; dy comes in pairs of nodes, half a wavefront for each.  Loads return in order, so that what
@@ -195,11 +247,6 @@ __global__ __launch_bounds__(kFewWaves * kWave) __attribute__((amdgpu_waves_per_
     FewSums sums;
     sums.s0 = 0.0f; sums.s1 = 0.0f; sums.s2 = 0.0f;
 
-    typedef __attribute__((address_space(4))) uint32_t const const_word;
-    typedef __attribute__((address_space(4))) NodeConsts const const_consts;
-    const_consts *consts = (const_consts *)a.node_consts;
-    uint32_t const discard_word = BN ? *(const_word *)a.discard : 0u;
-
 #pragma unroll
     for (int p = 0; p < kPairs; ++p) { request_rows(begin + 2 * p, p); }
 
@@ -213,6 +260,14 @@ __global__ __launch_bounds__(kFewWaves * kWave) __attribute__((amdgpu_waves_per_
     };
     auto wiring_of = [&](int base) { return wiring[min(base + (lane < kFewBatch ? lane : 0), last)]; };        // lane j: of node j of the share's round
     __syncthreads();
+#pragma unroll
+    for (int o = 1; o < 32; o <<= 1) { listed += lane_xor(listed, o); }
+    static_assert(kFewMost <= 32, "half a wavefront's lanes");
+    if (__builtin_amdgcn_readfirstlane(listed) != a.node_size * N) {     // the same for all wavefronts
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // (nothing is on its way to LDS when the workgroup ends)
+        few_inputs_by_lists<N, BN>(a, share, f_lane, discard_word == a.call);
+        return;
+    }
     uint32_t words = wiring_of(begin), quad = take_index(words, 0);
     few_f32x2 const *const my_rows = rows + wave * (kFewBatch * kWave) + lane;
 

@@ -22,9 +22,15 @@ def layer(n, I, O, F, seed):
     return idx, W, x, dy
 
 
-def reference(n, idx, W, x, dy, F, bias, norm=None):
-    """dx in 64 bits, by the corner values and their differences; norm: (mean, rstd, gamma, beta) of a batch-norm layer"""
+def reference(n, idx, W, x, dy, F, bias, norm=None, rev=None):
+    """dx in 64 bits, by the corner values and their differences; norm: (mean, rstd, gamma, beta) of a batch-norm layer; rev: the reverse table where it is not the
+    one of the wiring (a connection's gradient goes to the inputs whose rows list it, as often as they do)"""
     O, I, dev = idx.shape[0], x.shape[0], "cuda"
+    rows = [[[int(idx[o, k])] for k in range(n)] for o in range(O)] if rev is None else [[[] for _ in range(n)] for _ in range(O)]
+    if rev is not None:
+        for i, row in enumerate(host(rev)):
+            for e in row[1:1 + row[0]]:
+                rows[e // n][e % n].append(i)
     hi, lo = 0.5 + bias, 0.5 - bias
     p = torch.arange(1 << n, device=dev)
     V = torch.zeros((O, 1 << n), dtype=torch.float64, device=dev)
@@ -48,7 +54,8 @@ def reference(n, idx, W, x, dy, F, bias, norm=None):
             g = gamma * rstd * (g - g.sum() / F - v * rstd * rstd * (g * v).sum() / F)
         for k in range(n):
             slope = (V[o][p | (1 << k)] - V[o][p & ~(1 << k)]) / (hi - lo)
-            dx[idx[o, k].long()] += slope[corner] * g
+            for i in rows[o][k]:
+                dx[i] += slope[corner] * g
     return dx
 
 
@@ -87,3 +94,30 @@ def test_a_discarded_gradient_may_hold_anything():
     poisoned[:, :F][closed] = torch.tensor([np.inf, -np.inf, np.nan, 3.0e38], device="cuda")[torch.arange(int(closed.sum()), device="cuda") % 4]
     got = [host(ops.bit_differentiable_lut_backward(n, x, g, idx, W, torch.zeros_like(W), F, mean, rstd, rev, gamma=1.0, beta=0.5, bias=0.25))[:, :F] for g in (zeros, poisoned)]
     assert np.isfinite(got[1]).all() and np.array_equal(*got)
+
+
+@pytest.mark.parametrize("n, I, O, F", [(6, 27, 40, LEAST + 1), (4, 9, 600, LEAST), (2, 5, 130, LEAST + 257)])
+@pytest.mark.parametrize("how", ["left out", "twice", "descending", "elsewhere"])
+def test_dx_goes_by_the_reverse_table(n, I, O, F, how):
+    """A caller's reverse table need not be the wiring's own: the deterministic dx walks its lists, in layers of this size as in others."""
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    idx, W, x, dy = layer(n, I, O, F, 7 * n + O)
+    rows = [list(r[1:1 + r[0]]) for r in host(ops.reverse_table(idx, I))]
+    if how == "left out":     del rows[1][2]; rows[3] = []                           # a connection, and all of an input
+    if how == "twice":        rows[0].append(rows[0][-1]); rows[2].pop(0)           # (as many entries as connections)
+    if how == "descending":   rows = [r[::-1] for r in rows]
+    if how == "elsewhere":    rows[4].append(rows[0].pop(0))
+    rev = np.zeros((I, 1 + max(len(r) for r in rows)), np.int32)
+    for i, r in enumerate(rows):
+        rev[i, 0], rev[i, 1:1 + len(r)] = len(r), r
+    rev = torch.from_numpy(rev).cuda()
+    mean, rstd = W.mean(dim=1).contiguous(), (0.5 / W.std(dim=1)).contiguous()
+    for norm in (None, (mean, rstd, 0.7, 0.5)):
+        dW = torch.zeros_like(W)
+        if norm is None:
+            dx = ops.bit_stochastic_lut_backward(n, x, dy, idx, W, dW, F, rev, bias=0.25)
+        else:
+            dx = ops.bit_differentiable_lut_backward(n, x, dy, idx, W, dW, F, mean, rstd, rev, gamma=0.7, beta=0.5, bias=0.25)
+        want = reference(n, idx, W, x, dy, F, 0.25, norm, rev)
+        assert float((dx[:, :F] - want).abs().max()) <= 2 * int(rev[:, 0].max()) * 2.0 ** -24 * float(want.abs().max()) + 1e-6, (how, norm is None)
