@@ -136,6 +136,10 @@ inline bool node_sums(int n, int node_size, int frame_size)
 // 27 inputs x 216 nodes x 230400 frames 117 and 90 us, x 115200 64.7 and 53.6, x 80000 50.2 and 49.1, x 50000 40.2 and 44.5; 9 x 72 x 230400 48.6 and 38.5;
 // 6 x 216 x 262144 142 and 88; four inputs per node, 9 x 100 x 230400 48.8 and 40.2; two, 9 x 216 x 100000 41.7 and 35.6.  Few connections in all, or for each
 // input: 27 x 24 x 230400 25.2 and 25.7, 18 x 24 x 400000 34.6 and 35.2, 12 x 16 x 180000, two per node, plain, 13.9 and 16.4; but 27 x 36 x 700000 68.6 and 63.9.
+// 512 workgroups are resident, so that 262145 frames begin a second round that is nearly empty: 27 x 216 x 262144 141 and 90, x 262656 141 and 109; with few connections
+// the two are even there, 27 x 44 x 263000 39.6 and 39.7, 27 x 52 x 263000 43.3 and 44.1, 27 x 36 x 180000 28.7 and 29.2, the widest of 85 shapes on that side.  More nodes: 27 x 1000 x 97793 307 and
+// 192, 27 x 1600 x 150000 777 and 467; from about 2000 nodes on, whose wiring leaves a compute unit's LDS room for one workgroup, 27 x 2100 x 150000 1098 and 735, 27 x 4000 x 97793
+// 1484 and 711; four inputs, 9 x 4000 x 120000, 1409 and 699.
 constexpr int kFewInputs = 28, kFewInputNodes = 4096;
 inline bool few_inputs_dx(int n, int input_node_size, int node_size, int frame_size)
 {

@@ -389,7 +389,9 @@ int main(void)
         struct { int n, inputs, nodes, frames; double by_input, by_node; } const rows[] = {
             {6, 27, 216, 230400, 117.5, 90.8}, {6, 27, 216, 115200, 64.7, 53.6}, {6, 27, 216, 50000, 40.2, 44.5}, {6, 27, 87, 94500, 31.4, 31.7}, {6, 28, 300, 60000, 53.5, 58.4},
             {6, 9, 150, 100000, 49.0, 39.1}, {2, 9, 216, 100000, 41.7, 35.6}, {4, 9, 100, 230400, 48.8, 40.2}, {6, 27, 36, 700000, 68.6, 63.9}, {6, 27, 24, 230400, 25.2, 25.7},
-            {4, 9, 16, 400000, 21.6, 25.9}, {2, 18, 16, 180000, 14.4, 17.5}, {3, 28, 16, 262144, 19.3, 21.4}, {6, 20, 500, 30000, 54.2, 77.1}, {4, 27, 216, 80000, 40.7, 43.2}};
+            {4, 9, 16, 400000, 21.6, 25.9}, {2, 18, 16, 180000, 14.4, 17.5}, {3, 28, 16, 262144, 19.3, 21.4}, {6, 20, 500, 30000, 54.2, 77.1}, {4, 27, 216, 80000, 40.7, 43.2},
+            {6, 27, 216, 262144, 140.9, 90.4}, {6, 27, 216, 262656, 140.8, 109.3}, {6, 27, 52, 263000, 43.3, 44.1}, {6, 27, 36, 180000, 28.7, 29.2}, {6, 27, 72, 530000, 92.9, 80.8},
+            {6, 27, 1000, 97793, 307, 192}, {6, 27, 2100, 150000, 1098, 735}, {6, 27, 4000, 97793, 1484, 711}, {4, 9, 4000, 120000, 1409, 699}, {2, 9, 130, 263000, 63.1, 56.9}};
         for (auto const &r : rows) {
             double const taken = bbhip::few_inputs_dx(r.n, r.inputs, r.nodes, r.frames) ? r.by_node : r.by_input;
             if (taken > 1.05 * std::min(r.by_input, r.by_node)) { std::printf("%d x %d x %d\n", r.inputs, r.nodes, r.frames); CHECK(!"few_inputs_dx"); }

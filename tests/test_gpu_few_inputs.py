@@ -1,5 +1,5 @@
-"""GPU parity of dx formed node by node (layers of few inputs over many frames, two-valued inputs): widths, one to 28 inputs, last words, last pairs of
-frames, last rounds of nodes, gradients that are not finite behind a closed window."""
+"""GPU parity of dx formed node by node (layers of few inputs over many frames, two-valued inputs): widths, one to 28 inputs, up to 4096 nodes, last words, last pairs
+of frames, last rounds of nodes, more workgroups than are resident, gradients that are not finite behind a closed window, reverse tables of the caller's own, fp32 frames."""
 import numpy as np
 import pytest
 import torch
@@ -59,7 +59,9 @@ def reference(n, idx, W, x, dy, F, bias, norm=None, rev=None):
     return dx
 
 
-@pytest.mark.parametrize("n, I, O, F", [(6, 28, 38, LEAST), (6, 27, 216, LEAST + 30), (5, 9, 41, LEAST + 1), (4, 1, 50, LEAST + 127), (3, 13, 67, LEAST + 129), (2, 25, 121, LEAST + 510)])
+# (from 513 nodes on the threads of a workgroup fill the wiring in several rounds; 4096 nodes are the most, with the most LDS; 262144 frames fill the device once)
+@pytest.mark.parametrize("n, I, O, F", [(6, 28, 38, LEAST), (6, 27, 216, LEAST + 30), (5, 9, 41, LEAST + 1), (4, 1, 50, LEAST + 127), (3, 13, 67, LEAST + 129), (2, 25, 121, LEAST + 510),
+                                        (6, 27, 513, LEAST + 3), (6, 28, 4096, LEAST), (2, 3, 4096, LEAST + 2), (4, 9, 50, 262144), (6, 6, 37, 262146)])
 def test_dx_node_by_node(n, I, O, F):
     from binarybrain_amd import ops
     ops.set_dx_mode(0)
@@ -121,3 +123,24 @@ def test_dx_goes_by_the_reverse_table(n, I, O, F, how):
             dx = ops.bit_differentiable_lut_backward(n, x, dy, idx, W, dW, F, mean, rstd, rev, gamma=0.7, beta=0.5, bias=0.25)
         want = reference(n, idx, W, x, dy, F, 0.25, norm, rev)
         assert float((dx[:, :F] - want).abs().max()) <= 2 * int(rev[:, 0].max()) * 2.0 ** -24 * float(want.abs().max()) + 1e-6, (how, norm is None)
+
+
+@pytest.mark.parametrize("n, I, O, F", [(6, 27, 40, LEAST + 1), (4, 9, 60, LEAST)])
+def test_fp32_frames_of_binary_mode(n, I, O, F):
+    """fp32 frames are packed to bits by the call itself, behind the tables that dx is formed from in the same scratch memory: the bits of the packed call"""
+    from binarybrain_amd import ops
+    ops.set_dx_mode(0)
+    idx, W, xb, dy = layer(n, I, O, F, n + O)
+    shift = torch.arange(32, device="cuda", dtype=torch.int32)
+    x = torch.full((I, dy.shape[1]), float("nan"), device="cuda")
+    x[:, :F] = ((xb[:, :(F + 31) // 32, None] >> shift) & 1).reshape(I, -1)[:, :F].float()
+    rev = ops.reverse_table(idx, I)
+    mean, rstd = W.mean(dim=1).contiguous(), (0.5 / W.std(dim=1)).contiguous()
+    for bn in (False, True):
+        got = []
+        for call, inputs in (("bit_", xb), ("", x)):
+            dW = torch.zeros_like(W)
+            if bn: dx = getattr(ops, call + "differentiable_lut_backward")(n, inputs, dy, idx, W, dW, F, mean, rstd, rev, gamma=0.7, beta=0.5, bias=0.25)
+            else:  dx = getattr(ops, call + "stochastic_lut_backward")(n, inputs, dy, idx, W, dW, F, rev, bias=0.25, **({} if call else {"input_binary": True}))
+            got.append((dx[:, :F], dW))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]), bn
