@@ -221,10 +221,12 @@ inline int binary_unit_words(int words, int node_size)
 inline bool pool_four_frames(int frame_size) { return frame_size >= 16 || frame_size % 4 == 0; }
 
 // Whether the classifier tail runs with a row of 16 lanes per frame (classifier_tail_small_kernel): where there are as many inputs as connections (the wiring policies then
-// give every input to one node, which that form writes at once; a table of the caller's own that shares inputs takes 10 us instead of 7), channels fill half a row or more, and frames are few, of which it has four to a wavefront and 16 bytes of a row to a cache line.  70 -> 10 nodes, by a
-// wavefront per channel and by a row of lanes: 64 frames 6.35 and 4.40 us, 1024 6.69 and 4.91, 2048 6.72 and 5.45, 4000 6.82 and 6.24, 6000 6.93 and 6.91, 16384 8.6 and
-// 12.9, 65536 20.6 and 31.8; 60 inputs, 1024 frames, 6.4 and 9.1; 80 -> 5 nodes, 2000 frames 6.5 and 7.0; 30 inputs per
-// node 7.1 and 8.0.
+// give every input to one node, which that form writes at once), channels fill half a row or more, and frames are few, of which it has four to a wavefront and
+// 16 bytes of a row to a cache line.  70 -> 10 nodes, by a wavefront per channel and by a row of lanes: 64 frames 6.35 and 3.66 us, 1024 6.64 and 3.99, 2048 6.66 and 4.41, 4000
+// 6.75 and 5.44, 6000 6.89 and 6.90, 16384 8.37 and 13.7, 65536 20.6 and 44.8; 192 -> 16 nodes, 1024 frames, 12.4 and 6.15.  A table of the caller's own whose nodes
+// share inputs: 70 -> 10 nodes, 64 frames 6.16 and 5.19, 1024 6.40 and 5.51, 2000 6.47 and 5.95, 4000 6.56 and 6.74, and where a node takes an input twice 6.10 and 5.41, 6.32
+// and 5.89, 6.38 and 6.27, 6.48 and 7.21; 208 -> 16, 4000 frames, 14.7 and 12.8.  Other counts of inputs and fewer channels stay with the wider
+// form, though this one would serve them too (60 inputs, 1024 frames, 6.35 and 4.98, 80 -> 5 nodes x 2000 frames 6.39 and 5.79, 40 -> 4 x 1000 4.88 and 4.65).
 constexpr int kTailInputs = 16;                 // most inputs of a node there
 inline bool tail_small(int n, int input_node_size, int ch_size, int frame_stride)
 {

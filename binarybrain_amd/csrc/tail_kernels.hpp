@@ -566,13 +566,14 @@ __global__ __launch_bounds__(64 * CH) void classifier_tail_kernel(float const *_
 // The same for a small batch of as many inputs as connections (each its own, as a rule): a wavefront owns four frames and all nodes, lane 16 i + ch is
 // channel ch of frame i (a row of 16 lanes: what the channels exchange goes by data-parallel moves, without LDS and barriers), and every
 // wavefront is a workgroup, with a compute unit of its own.
-//   1. a lane loads its n inputs and sums them; while they are on the way, the wavefront counts in LDS how many nodes take each input;
+//   1. a lane loads its n inputs and sums them; while they are on the way, the wavefront counts in LDS how many connections take each input;
 //   2. the row takes its maximum, every lane its exponential, the sum of the row's in channel order, its softmax, gradient and loss term; the loss terms are added
 //      up in channel order, masks of the wavefront give the accuracy;
-//   3. a lane writes its gradient dy / n to those of its inputs that no other node has; for an input that no node or several have, the row
-//      adds up the matches, ascending.
-// The same bits.  Latency: above, a SIMD issues for four wavefronts that each go through all channels, and meet four times.  70 -> 10 nodes, 64 frames 6.4 -> 4.5 us,
-// 1024 frames 6.7 -> 5.0 (tail_small has both sides of its lines).
+//   3. where every input is one connection's, a lane writes its gradient dy / n to those of its node; else a lane takes every 16th input and adds up what its
+//      connections give it, ascending, by counts per input and node.
+// The same bits.  Latency: above, a SIMD issues for four wavefronts that each go through all channels, and meet four times.  70 -> 10 nodes, 64 frames 6.35 -> 3.66 us,
+// 1024 frames 6.64 -> 3.99; nodes that share inputs, 1024 frames, 6.40 -> 5.51 (11.4 where such inputs were gone through one by one), 208 -> 16 nodes 14.3 -> 9.7
+// (25.2).  tail_small has both sides of its lines.
 constexpr int kTailChannels = 16, kTailFrames = kWave / kTailChannels;
 // the value of lane CH of the lane's row of 16
 template <int CH> __device__ __forceinline__ float of_channel(float v)
@@ -596,6 +597,31 @@ template <class V, int CH = 0> __device__ __forceinline__ V sum_of_channels(V v,
     else { return sum; }
 }
 
+// s[g] += the gradients `v` of channels 0 .. ch_size - 1 of the lane's row, in that order, each as often as its byte of count[g] says, ONCE: not more than once (adding 0 for those that have none
+// leaves a sum that began as +0 as it is)
+template <bool ONCE, int G, int CH = 0> __device__ __forceinline__ void add_of_takers(float (&s)[G], unsigned const (&count)[G][kTailChannels / 4], float v, int ch_size)
+{
+    if constexpr (CH < kTailChannels) {
+        if (CH < ch_size) {                                                     // wave-uniform
+            float const b = of_channel<CH>(v);
+            unsigned c[G], most = 0;
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                c[g] = (count[g][CH / 4] >> (8 * (CH % 4))) & 0xffu;
+                s[g] += c[g] != 0 ? b : 0.0f;
+                most = max(most, c[g]);
+            }
+            if constexpr (!ONCE) {
+                for (unsigned r = 1; __ballot(most > r) != 0; ++r) {
+#pragma unroll
+                    for (int g = 0; g < G; ++g) { s[g] += c[g] > r ? b : 0.0f; }
+                }
+            }
+        }
+        add_of_takers<ONCE, G, CH + 1>(s, count, v, ch_size);
+    }
+}
+
 __global__ __launch_bounds__(kWave) void classifier_tail_small_kernel(float const *__restrict__ x, float *__restrict__ y, float *__restrict__ dx,
                                                              int const *__restrict__ idx, float const *__restrict__ t,
                                                              float *__restrict__ dy_out, double *__restrict__ loss_buf,
@@ -603,14 +629,19 @@ __global__ __launch_bounds__(kWave) void classifier_tail_small_kernel(float cons
                                                              float t_sum, float scale, int n, int input_node_size, int ch_size,
                                                              int frame_size, int frame_stride, int binarize_input)
 {
-    __shared__ int takers[kTailChannels * kTailInputs];                         // [input]: nodes that take it
+    __shared__ unsigned taken[kTailChannels * kTailInputs];                     // [input]: connections that take it
+    __shared__ __align__(16) unsigned takers[kTailChannels * kTailInputs][kTailChannels / 4];      // [input]: a byte per node, its connections that do
     int const lane = threadIdx.x, ch = lane % kTailChannels, f = blockIdx.x * kTailFrames + lane / kTailChannels;
     int const total = ch_size * n;
     bool const in_row = f < frame_stride, live = f < frame_size, mine = ch < ch_size;
     int const fc = live ? f : 0;                                                // (a lane without a frame or channel loads another's and stores nothing)
     int const *const row = idx + (mine ? ch : 0) * n;
 
-    for (int in = lane; in < input_node_size; in += kWave) { takers[in] = 0; }
+    for (int in = lane; in < input_node_size; in += kWave) { taken[in] = 0; }
+    constexpr int kPieces = kTailChannels * kTailInputs / kWave;                // the table, 64 entries to a register
+    int piece[kPieces];
+#pragma unroll
+    for (int q = 0; q < kPieces; ++q) { piece[q] = (q * kWave + lane < total) ? idx[q * kWave + lane] : -1; }
     float const tv = t[(size_t)(mine ? ch : 0) * frame_stride + fc];
     constexpr int kAhead = 8;
     int in[kAhead];
@@ -622,14 +653,26 @@ __global__ __launch_bounds__(kWave) void classifier_tail_small_kernel(float cons
         for (int j = 0; j < kAhead; ++j) { v[j] = x[(size_t)in[j] * frame_stride + fc]; }
     };
     request(0);
-    constexpr int kPieces = kTailChannels * kTailInputs / kWave;                // the table, 64 entries to a register
-    int piece[kPieces];
-#pragma unroll
-    for (int q = 0; q < kPieces; ++q) { piece[q] = (q * kWave + lane < total) ? idx[q * kWave + lane] : -1; }
     wave_fence();
+    // (as many connections as inputs, each within them and the first to take its input: each takes one of its own)
+    bool second = false;
 #pragma unroll
-    for (int q = 0; q < kPieces; ++q) { if ((unsigned)piece[q] < (unsigned)input_node_size) { atomicAdd(&takers[piece[q]], 1); } }
-    wave_fence();
+    for (int q = 0; q < kPieces; ++q) {
+        if (q * kWave + lane < total) { second |= (unsigned)piece[q] >= (unsigned)input_node_size || atomicAdd(&taken[piece[q]], 1u) != 0; }
+    }
+    bool const apart = total == input_node_size && __ballot(second) == 0;       // wave-uniform
+    if (!apart) {
+        for (int in_at = lane; in_at < input_node_size; in_at += kWave) { *reinterpret_cast<uint4 *>(takers[in_at]) = make_uint4(0, 0, 0, 0); }
+        wave_fence();
+#pragma unroll
+        for (int q = 0; q < kPieces; ++q) {
+            if ((unsigned)piece[q] < (unsigned)input_node_size) {
+                int const node = (q * kWave + lane) / n;
+                atomicAdd(&takers[piece[q]][node / 4], 1u << (8 * (node % 4)));
+            }
+        }
+        wave_fence();
+    }
     float sum = 0.0f;
     for (int i0 = 0; i0 < n; i0 += kAhead) {
         if (i0 > 0) { request(i0); }
@@ -655,35 +698,38 @@ __global__ __launch_bounds__(kWave) void classifier_tail_small_kernel(float cons
     float const g = (rounded_mul(t_max, softmax) - tv) / t_sum;
     float const slope = g / (float)n;
 
-    // the row's inputs, and then those that are not one node's
-    for (int i0 = 0; i0 < n; i0 += kAhead) {
-        if (n > kAhead) {
+    if (apart) {
+        for (int i0 = 0; i0 < n; i0 += kAhead) {
+            if (n > kAhead) {
 #pragma unroll
-            for (int j = 0; j < kAhead; ++j) { in[j] = row[(i0 + j < n) ? i0 + j : 0]; }
-        }
+                for (int j = 0; j < kAhead; ++j) { in[j] = row[(i0 + j < n) ? i0 + j : 0]; }
+            }
 #pragma unroll
-        for (int j = 0; j < kAhead; ++j) {
-            bool const inside = (unsigned)in[j] < (unsigned)input_node_size;
-            if (i0 + j < n && mine && in_row && inside && takers[inside ? in[j] : 0] == 1) { dx[(size_t)in[j] * frame_stride + f] = live ? 0.0f + slope : 0.0f; }
+            for (int j = 0; j < kAhead; ++j) {
+                if (i0 + j < n && mine && in_row) { dx[(size_t)in[j] * frame_stride + f] = live ? 0.0f + slope : 0.0f; }
+            }
         }
     }
-    for (int i0 = 0; i0 < input_node_size; i0 += kWave) {
-        int const taken = (i0 + lane < input_node_size) ? takers[i0 + lane] : 1;
-        uint64_t none = __ballot(taken == 0), several = __ballot(taken > 1);
-        for (; none != 0; none &= none - 1) {                                   // wave-uniform
-            if (ch == 0 && in_row) { dx[(size_t)(i0 + (int)__builtin_ctzll(none)) * frame_stride + f] = 0.0f; }
-        }
-        for (; several != 0; several &= several - 1) {
-            int const input = i0 + (int)__builtin_ctzll(several);
-            float s = 0.0f;
+    else {
+        constexpr int kTogether = 4;                                            // inputs of a lane
+        for (int i0 = 0; i0 < input_node_size; i0 += kTogether * kTailChannels) {
+            unsigned count[kTogether][kTailChannels / 4], most = 0;
+            float s[kTogether];
 #pragma unroll
-            for (int q = 0; q < kPieces; ++q) {
-                for (uint64_t hits = __ballot(piece[q] == input); hits != 0; hits &= hits - 1) {
-                    int const node = (q * kWave + (int)__builtin_ctzll(hits)) / n;
-                    s += __int_as_float(__builtin_amdgcn_ds_bpermute(((lane & ~(kTailChannels - 1)) + node) * 4, __float_as_int(slope)));
-                }
+            for (int g = 0; g < kTogether; ++g) {
+                int const input = i0 + g * kTailChannels + ch;
+                uint4 const c = *reinterpret_cast<uint4 const *>(takers[min(input, input_node_size - 1)]);
+                count[g][0] = c.x; count[g][1] = c.y; count[g][2] = c.z; count[g][3] = c.w;
+                most |= c.x | c.y | c.z | c.w;
+                s[g] = 0.0f;
             }
-            if (ch == 0 && in_row) { dx[(size_t)input * frame_stride + f] = live ? s : 0.0f; }
+            if (__ballot((most & 0xfefefefeu) != 0) == 0) { add_of_takers<true>(s, count, slope, ch_size); }      // wave-uniform
+            else                                          { add_of_takers<false>(s, count, slope, ch_size); }
+#pragma unroll
+            for (int g = 0; g < kTogether; ++g) {
+                int const input = i0 + g * kTailChannels + ch;
+                if (input < input_node_size && in_row) { dx[(size_t)input * frame_stride + f] = live ? s[g] : 0.0f; }
+            }
         }
     }
 

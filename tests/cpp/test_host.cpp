@@ -474,10 +474,11 @@ int main(void)
 
     // the classifier tail by a wavefront per channel or by a row of lanes, where both were measured (microseconds)
     {
-        struct { int n, inputs, channels, stride; double wavefront, row; } const rows[] = {{7, 70, 10, 64, 6.35, 4.40}, {7, 70, 10, 1152, 6.69, 4.91}, {7, 70, 10, 2176, 6.72, 5.45},
-            {12, 192, 16, 1152, 12.4, 7.35}, {7, 70, 10, 16512, 8.64, 12.9}, {7, 70, 10, 65664, 20.6, 31.8}, {30, 90, 3, 640, 7.07, 8.04}, {7, 60, 10, 1152, 6.43, 9.11},
-            {16, 80, 5, 2176, 6.45, 6.95}, {15, 45, 3, 640, 4.86, 5.48}};
+        struct { int n, inputs, channels, stride; double wavefront, row; } const rows[] = {{7, 70, 10, 64, 6.35, 3.66}, {7, 70, 10, 1152, 6.64, 3.99}, {7, 70, 10, 2176, 6.66, 4.41},
+            {7, 70, 10, 4096, 6.75, 5.44}, {12, 192, 16, 1152, 12.4, 6.15}, {13, 208, 16, 4096, 14.7, 11.8}, {7, 70, 10, 6144, 6.89, 6.90}, {7, 70, 10, 16512, 8.37, 13.7}, {7, 70, 10, 65664, 20.6, 44.8}};
         for (auto const &r : rows) { CHECK(bbhip::tail_small(r.n, r.inputs, r.channels, r.stride) == (r.row < r.wavefront)); }
+        // other counts of inputs, fewer channels, and more inputs per node than that form has room for
+        CHECK(!bbhip::tail_small(7, 60, 10, 1152) && !bbhip::tail_small(16, 80, 5, 2176) && !bbhip::tail_small(15, 45, 3, 640) && !bbhip::tail_small(30, 240, 8, 640) && !bbhip::tail_small(30, 90, 3, 640));
     }
 
     // rows that share a workgroup in the pooling kernels, where both were measured (microseconds): at most 3 % slower than the faster

@@ -237,15 +237,16 @@ def test_classifier_tail_in_one_launch(ops, case, mean):
     assert torch.equal(dx0, dx2) and torch.equal(loss0, loss2) and acc2 is None
 
 
-@pytest.mark.parametrize("wired", ["apart", "anyhow", "few"])
+@pytest.mark.parametrize("wired", ["apart", "anyhow", "few", "distinct", "one"])
 @pytest.mark.parametrize("CH, n, F", [(8, 1, 1), (9, 3, 5), (10, 7, 63), (16, 13, 66), (13, 16, 130), (8, 9, 2000), (10, 7, 4030), (10, 7, 4100)])
 def test_classifier_tail_of_as_many_inputs_as_connections(ops, CH, n, F, wired):
-    """as many inputs as the nodes take: each its own, some left out and others shared, or nearly all left out; up to 4096 columns, 16 channels and 16 inputs per node, and beyond.
-    Logits beyond all bounds too."""
+    """as many inputs as the nodes take: each its own, some left out and others shared, or nearly all left out, a node's own distinct, or one input for all connections; up to 4096
+    columns, 16 channels and 16 inputs per node, and beyond.  Logits beyond all bounds too."""
     import torch
     I, S = CH * n, synth.frame_stride_fp32(F)
     rng = np.random.default_rng(I + F)
-    idx = (rng.permutation(I) if wired == "apart" else rng.integers(0, I if wired == "anyhow" else 1 + I // 20, I)).reshape(CH, n).astype(np.int32)
+    idx = (rng.permutation(I) if wired == "apart" else np.stack([rng.permutation(I)[:n] for _ in range(CH)]) if wired == "distinct" else np.full(I, I - 1) if wired == "one" else
+           rng.integers(0, I if wired == "anyhow" else 1 + I // 20, I)).reshape(CH, n).astype(np.int32)
     x = np.zeros((I, S), np.float32); x[:, :F] = rng.integers(0, 2, (I, F)) if F % 2 else rng.standard_normal((I, F))
     if F > 60:
         x[0, 3], x[I - 1, 11], x[I // 2, 20], x[:, 30] = np.nan, np.inf, -np.inf, -np.inf
