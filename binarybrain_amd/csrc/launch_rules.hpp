@@ -183,9 +183,12 @@ inline bool dx_wide_passes(int input_node_size, int output_node_size, int frame_
 // 78 and 97 (four).
 inline bool im2col_frames_first(int f_tiles, int tile_frames) { return tile_frames == 64 && f_tiles % 8 == 0; }
 
-// Passes of 256 frames that a wavefront of lut_forward_quads_kernel makes (0: up to 64 frames, one per lane, 7372 nodes x 31 5.8 -> 4.9 us): one, the node's passes side by side (they wait for each other where they exchange sums), or
+// Passes of 256 frames that a wavefront of lut_forward_quads_kernel makes: one, the node's passes side by side (they wait for each other where they exchange sums), or
 // all, one after another, where nodes alone fill the device.  Batch-norm training call, side by side and one after another: 700 nodes x 1000 frames 4.25 and 4.55 us,
-// 1024 x 1024 4.90 and 5.14; 1500 x 600 5.71 and 4.72, 4000 x 300 6.7 and 5.3, 6144 x 1024 15.4 and 9.5.
+// 1024 x 1024 4.90 and 5.14; 1500 x 600 5.71 and 4.72, 3000 x 400 5.44 and 4.61, 4000 x 300 6.7 and 5.3, 6144 x 1024 15.4 and 9.5.  0: up to 64 frames, one per lane.
+// Each count has a form of its own, whose inputs are all requested at once: two passes in the form for two and in that for four, 1100 x 512 4.03 and 4.18 us, 3000 x 300 4.65 and 4.73, packed
+// inference 1500 x 512 3.50 and 3.74, four inputs per node, 6144 x 400, 5.52 and 5.68; up to 64 frames in the form for one frame per lane and in that for one pass, 360 x 64 3.18
+// and 3.35, fp32 frames 3.34 and 3.63, 7372 x 31 6.32 and 6.54, fp32 6.52 and 7.46.
 constexpr int kQuadFrames = 256, kQuadMost = 1024;               // frames of a pass, most frames of a node there
 inline int forward_quad_passes(int node_size, int frame_size) { return frame_size <= 64 ? 0 : (node_size <= 1024 || frame_size <= kQuadFrames) ? 1 : frame_size <= 2 * kQuadFrames ? 2 : 4; }
 
