@@ -289,17 +289,17 @@ void launch_table_prep(float const *W, float *C, int node_size, int lut_binarize
 }
 
 template <int N, int XMODE, int YMODE, int KIND>
-void launch_forward(FwdArgs const &a, int npw, hipStream_t st)
+int launch_forward(FwdArgs const &a, int npw, hipStream_t st)
 {
     dim3 const grid(a.chunk_count * a.tiles.count + a.pack.blocks), block(kBlock);
     if constexpr (XMODE == kXBit || XMODE == kXBinary) {
         // two-valued inputs: the corner-value kernel wherever the caller prepared the values (one node per wavefront)
         if (a.V != nullptr) {
             if constexpr (KIND == 0 || KIND == 1) {
-                if (a.quad_passes == 0) { launch((lut_forward_quads_kernel<N, XMODE, YMODE, KIND, 0>), grid, block, 0, st, a); return; }
-                if (a.quad_passes == 1) { launch((lut_forward_quads_kernel<N, XMODE, YMODE, KIND, 1>), grid, block, 0, st, a); return; }
-                if (a.quad_passes == 2) { launch((lut_forward_quads_kernel<N, XMODE, YMODE, KIND, 2>), grid, block, 0, st, a); return; }
-                if (a.quad_passes == 4) { launch((lut_forward_quads_kernel<N, XMODE, YMODE, KIND, 4>), grid, block, 0, st, a); return; }
+                if (a.quad_passes == 0) { launch((lut_forward_quads_kernel<N, XMODE, YMODE, KIND, 0>), grid, block, 0, st, a); return 0; }
+                if (a.quad_passes == 1) { launch((lut_forward_quads_kernel<N, XMODE, YMODE, KIND, 1>), grid, block, 0, st, a); return 0; }
+                if (a.quad_passes == 2) { launch((lut_forward_quads_kernel<N, XMODE, YMODE, KIND, 2>), grid, block, 0, st, a); return 0; }
+                if (a.quad_passes == 4) { launch((lut_forward_quads_kernel<N, XMODE, YMODE, KIND, 4>), grid, block, 0, st, a); return 0; }
             }
             if constexpr (KIND != 3 && (XMODE == kXBit || (YMODE == kYBinarize && KIND == 1))) {
                 if (a.node_waves > 0) {
@@ -307,37 +307,39 @@ void launch_forward(FwdArgs const &a, int npw, hipStream_t st)
                     int const waves = a.node_waves > kWavesPerBlk ? a.node_waves : kWavesPerBlk;
                     int const index_blocks = fused ? waves / a.node_waves * a.out_blocks : waves;
                     launch((lut_forward_bytes_kernel<N, XMODE, YMODE, KIND>), grid, dim3(waves * kWave), forward_bytes_lds(waves, index_blocks), st, a);
-                    return;
+                    return 0;
                 }
             }
             if constexpr (XMODE == kXBit && YMODE == kYBinarize && KIND == 1) {
                 if (a.own_index != nullptr) {      // corner indices kept by the statistics launch of the same call
                     launch((lut_forward_corner_kernel<N, XMODE, YMODE, KIND, false, kOwnMemory>), grid, block, 0, st, a);
-                    return;
+                    return 0;
                 }
             }
             if constexpr (XMODE == kXBit && KIND == 3) {
                 // 32-byte scalar loads where they stay inside the row pitch and never straddle a unit
                 if (a.x_stride % 8 == 0 && a.chunk % 256 == 0 && (reinterpret_cast<uintptr_t>(a.x) & 3u) == 0) {
                     launch((lut_forward_corner_kernel<N, XMODE, YMODE, KIND, true>), grid, block, 0, st, a);
-                    return;
+                    return 0;
                 }
             }
             if constexpr (XMODE == kXBinary || KIND == 3) {
                 launch((lut_forward_corner_kernel<N, XMODE, YMODE, KIND>), grid, block, 0, st, a);
-                return;
+                return 0;
             }
+            else { return fail("forward: no kernel takes this call on packed bits (y=%d, kind=%d, %d frames)", YMODE, KIND, a.frame_size); }
         }
     }
     if (npw == 2) { launch((lut_forward_kernel<N, XMODE, YMODE, KIND, 2>), grid, block, 0, st, a); }
     else          { launch((lut_forward_kernel<N, XMODE, YMODE, KIND, 1>), grid, block, 0, st, a); }
+    return 0;
 }
 
 // xmode / ymode / kind are runtime values here; the combinations that exist are enumerated explicitly
 template <int N>
 int dispatch_forward(int xmode, int ymode, int kind, FwdArgs const &a, int npw, hipStream_t st)
 {
-#define BBHIP_FWD_CASE(X, Y, K) if (xmode == X && ymode == Y && kind == K) { launch_forward<N, X, Y, K>(a, npw, st); return 0; }
+#define BBHIP_FWD_CASE(X, Y, K) if (xmode == X && ymode == Y && kind == K) { return launch_forward<N, X, Y, K>(a, npw, st); }
     BBHIP_FWD_CASE(kXClamp,  kYClamp,    0)
     BBHIP_FWD_CASE(kXBinary, kYClamp,    0)
     BBHIP_FWD_CASE(kXBit,    kYClamp,    0)
@@ -1162,7 +1164,7 @@ int run_backward(BackwardCall const &call, hipStream_t st, PackedInputHint packe
         f.dy = c.dy; f.dy_stride = c.frame_stride;
         f.node_size = c.output_node_size; f.frame_size = c.frame_size; f.x_stride = c.x_stride;
         f.chunk = stat_chunk; f.chunk_count = stat_chunk_count; f.tiles = make_tile_divisor(stat_tiles);
-        f.bias = c.bias; f.gamma = c.gamma; f.beta = c.beta; f.quad_passes = -1;
+        f.bias = c.bias; f.gamma = c.gamma; f.beta = c.beta;
         if (dispatch_forward<N>(c.xmode, kYClamp, 3, f, npw, st)) { return 1; }
         BBHIP_LAUNCH_CHECK();
         if (!stat_launch) {

@@ -327,6 +327,7 @@ __global__ __launch_bounds__(kByteWaves * kWave) void lut_forward_bytes_kernel(F
     }
 }
 
+static_assert(FwdArgs{}.quad_passes < 0, "a call that says nothing takes another kernel than lut_forward_quads_kernel");
 static_assert(kQuadFrames == 4 * kWave && kQuadMost == kWavesPerBlk * kQuadFrames, "four frames per lane, a workgroup per node");
 // Up to kQuadMost frames: a.node_waves wavefronts (1, 2 or 4) = one node, PASSES x 256 frames each, four consecutive ones per lane and pass (PASSES 0: up to 64 frames, one per lane).  All kinds that need the node's frames
 // in one place: plain (0), batch-norm (1) with running statistics or those of the call (kStatInline), which the node's wavefronts add up and exchange in LDS.

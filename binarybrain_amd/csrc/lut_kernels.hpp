@@ -273,7 +273,7 @@ struct FwdArgs {
     // rows of fp32 output start on 16 bytes
     int   node_waves, y_quads;
     int   out_blocks;           // ... blocks of 2048 frames whose output is a workgroup's: all, or the chunk_count workgroups of a node share them
-    int   quad_passes;          // up to kQuadMost frames: the form of lut_forward_quads_kernel, by node_waves wavefronts per node; -1: another kernel
+    int   quad_passes = -1;     // up to kQuadMost frames: the form of lut_forward_quads_kernel, by node_waves wavefronts per node; -1: another kernel
     // lut_forward_quads_kernel over the fp32 frames of a small batch-norm training pass: the last pack.blocks workgroups make the packed copy of the
     // input that the backward call takes
     PackRider pack;
