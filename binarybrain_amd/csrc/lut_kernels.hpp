@@ -247,10 +247,10 @@ struct FwdArgs {
     // Not null (plain output of calls of few units): no table-preparation launch has run; the wavefront brings its node's table W' into
     // the centred basis itself — 2^N loads, one per lane, and the butterfly of table_prep_block over the lanes.  A call of a few hundred
     // frames is two launches' worth of latency, not work.  With clamp_W (below) the table is first clamped, and written back by the wavefront
-    // of the node's first unit (the others read either value and clamp it too), as in the corner-value kernel.
+    // of the node's first unit (the others read either value and clamp it too), as in the kernels for two-valued inputs.
     float const *W_inline;
     int   lut_binarize;
-    // lut_forward_corner_kernel with W_inline: the node's tables go to C_out / V_out as well (the wavefront of the node's first unit
+    // the kernels for two-valued inputs with W_inline: the node's tables go to C_out / V_out as well (the wavefront of the node's first unit
     // stores them: for a later launch of the same call, and for the caller that keeps them for the backward pass), and the table is
     // first clamped to [clamp_lo, clamp_hi] and written back where clamp_W (W itself) is given — all as table_prep_block does
     float *C_out, *V_out;
@@ -695,11 +695,6 @@ __device__ __forceinline__ void corner_pass(FwdArgs const &a, void const *(&rows
             s1 += d;
             s2 = __builtin_fmaf(d, t1, s2);
         }
-        else if (YMODE == kYBit) {
-            uint64_t const m = __ballot(ok && (t0 > 0.5f));
-            asm("s_nop 3\n\tv_writelane_b32 %0, %1, %2" : "+v"(words) : "s"((uint32_t)m), "n"(2 * u));         // (as below)
-            asm("s_nop 3\n\tv_writelane_b32 %0, %1, %2" : "+v"(words) : "s"((uint32_t)(m >> 32)), "n"(2 * u + 1));
-        }
         else {
             if (kPackedCopy && a.y_bits != nullptr) {         // wave-uniform
                 uint64_t const m = __ballot(ok && (t0 > 0.5f));
@@ -715,10 +710,6 @@ __device__ __forceinline__ void corner_pass(FwdArgs const &a, void const *(&rows
     // the packed copy of the pass: its 2 U words by one store (a store per step would double the kernel's store instructions)
     if (kPackedCopy && a.y_bits != nullptr && lane < 2 * U && (!RAGGED || fb + 32 * lane < f_end)) {
         a.y_bits[(size_t)node * a.y_bits_stride + (fb >> 5) + lane] = words;
-    }
-    // packed output: the same, to the words of the output row that hold frames of the unit
-    if (YMODE == kYBit && (KIND == 0 || KIND == 1) && lane < 2 * U && (!RAGGED || fb + 32 * lane < f_end)) {
-        reinterpret_cast<uint32_t *>(a.y)[(size_t)node * a.y_stride + (fb >> 5) + lane] = words;
     }
 }
 
@@ -767,6 +758,7 @@ template <int N, int XMODE, int YMODE, int FWD_KIND, bool WIDE = false, int OWN 
 __global__ __launch_bounds__(kBlock) void lut_forward_corner_kernel(FwdArgs a)
 {
     static_assert(XMODE == kXBit || XMODE == kXBinary, "corner values need two-valued inputs");
+    static_assert(YMODE != kYBit, "packed output comes from the kernels over packed bits");
     static_assert(!WIDE || XMODE == kXBit, "wide loads are for packed bits");
     static_assert(OWN == kOwnNone || (OWN == kOwnMemory && XMODE == kXBit && !WIDE && FWD_KIND == 1), "kept corner indices: output launch only");
     constexpr int NN = 1 << N;
@@ -826,7 +818,6 @@ __global__ __launch_bounds__(kBlock) void lut_forward_corner_kernel(FwdArgs a)
     if (FWD_KIND == 2 || FWD_KIND == 3) { forward_store_stats(a, ck, node, true, lane, s1, s2); }
     if (FWD_KIND == 1) { forward_store_statistics(a, node, true, ck, lane, mean, var, rstd); }
     if (YMODE == kYBinarize && (FWD_KIND == 0 || FWD_KIND == 1)) { zero_packed_tail(a, ck, node, true, lane); }
-    if (YMODE == kYBit) { zero_output_padding(a, ck, node, true, lane); }
     if (a.W_inline != nullptr && ck == 0 && lane < NN) {
         if (clamp_store)         { a.clamp_W[(size_t)node * NN + lane] = table_w; }
         if (a.C_out != nullptr)  { a.C_out[(size_t)node * NN + lane] = table_c; }
