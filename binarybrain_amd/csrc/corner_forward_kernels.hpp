@@ -333,9 +333,10 @@ static_assert(kQuadFrames == 4 * kWave && kQuadMost == kWavesPerBlk * kQuadFrame
 // in one place: plain (0), batch-norm (1) with running statistics or those of the call (kStatInline), which the node's wavefronts add up and exchange in LDS.
 // A frame's corner index is formed from the input words' four bits (spread to bytes by a multiplication) or from the fp32 frames, its corner value fetched once from the
 // lane that holds it, and what follows is arithmetic on the value.  The fp32 frames of a small training pass may also be packed, by extra workgroups.
-// Such a launch is a chain (wiring, inputs, index, value, sums, output), and the less a wavefront does in turn the shorter.  Against a wavefront per node in
-// steps of 64 frames, whose input masks were scalar loads, training calls on packed bits: 70 nodes x 1024 frames 5.8 -> 3.6 us, 1024 x 1024 6.0 -> 4.9, 6144 x 1024
-// 9.7 -> 9.5, 700 x 1000 5.9 -> 4.2, 210 x 236 4.4 -> 3.5, 360 x 64 3.95 -> 3.5; inference 4000 x 1024 9.5 -> 5.6, 8000 x 1000 10.8 -> 8.2, 120 x 8 3.5 -> 3.0.
+// Such a launch is a chain (wiring, inputs, index, value, sums, output), and the less a wavefront does in turn the shorter; with thousands of nodes its scalar
+// instructions count (169 per wavefront with a division by the wavefronts of a node and products of signed numbers, 7372 plain nodes x 31 frames 4.80 us; 3.89 without).  Against a
+// wavefront per node in steps of 64 frames, whose input masks were scalar loads, training calls on packed bits: 70 nodes x 1024 frames 5.0 -> 3.4 us, 1024 x 1024 5.0 -> 4.3, 6144 x 1024
+// 7.8 -> 7.6, 700 x 1000 5.3 -> 3.9, 210 x 236 3.9 -> 3.1, 360 x 64 3.6 -> 3.0; inference 4000 x 1024 9.3 -> 5.3, 8000 x 1000 10.7 -> 7.6, 120 x 8 3.0 -> 2.5; plain 7372 x 31 4.5 -> 3.9.
 template <int N, int XMODE, int YMODE, int KIND, int PASSES>
 __global__ __launch_bounds__(kBlock) void lut_forward_quads_kernel(FwdArgs a)
 {
@@ -353,8 +354,9 @@ __global__ __launch_bounds__(kBlock) void lut_forward_quads_kernel(FwdArgs a)
         }
     }
     int const wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave)), lane = threadIdx.x & (kWave - 1);
-    int const nw = a.node_waves, sub = wave & (nw - 1), slot = wave / nw;
-    int node = xcd_remap(blockIdx.x, B) * (kWavesPerBlk / nw) + slot;
+    // (a power of two: no division, which would head the chain; one wavefront in the forms that make several passes)
+    int const nw = PASSES == 1 ? a.node_waves : 1, shift = PASSES == 1 ? __builtin_ctz((unsigned)nw) : 0, sub = wave & (nw - 1), slot = wave >> shift;
+    int node = xcd_remap(blockIdx.x, B) * (kWavesPerBlk >> shift) + slot;
     bool const live = node < a.node_size;
     if (!live) {
         if (nw == 1) { return; }
@@ -376,7 +378,10 @@ __global__ __launch_bounds__(kBlock) void lut_forward_quads_kernel(FwdArgs a)
     uint32_t const x_bytes = XMODE == kXBit ? (uint32_t)((a.frame_size + 31) >> 5) * 4u : quad_row_bytes(a.frame_size, a.x_stride >= ((a.frame_size + 3) & ~3));
     __amdgpu_buffer_rsrc_t rows[N];
 #pragma unroll
-    for (int k = 0; k < N; ++k) { rows[k] = row_descriptor(a.x, in[k], a.x_stride, x_bytes); }
+    for (int k = 0; k < N; ++k) {                    // (row_descriptor takes the product of signed 64-bit numbers: twice the scalar instructions)
+        rows[k] = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(reinterpret_cast<char const *>(a.x)) + (uint64_t)(uint32_t)in[k] * (uint32_t)a.x_stride * 4u,
+                                                    0, (int)x_bytes, 0x00020000);
+    }
     uint32_t w[XMODE == kXBit ? P : 1][N];
     std::conditional_t<LANE == 4, float4, float> x[XMODE == kXBit ? 1 : N];
     auto fetch = [&](int p) {                        // (past the row: zeros)

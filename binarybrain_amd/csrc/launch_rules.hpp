@@ -184,11 +184,12 @@ inline bool dx_wide_passes(int input_node_size, int output_node_size, int frame_
 inline bool im2col_frames_first(int f_tiles, int tile_frames) { return tile_frames == 64 && f_tiles % 8 == 0; }
 
 // Passes of 256 frames that a wavefront of lut_forward_quads_kernel makes: one, the node's passes side by side (they wait for each other where they exchange sums), or
-// all, one after another, where nodes alone fill the device.  Batch-norm training call, side by side and one after another: 700 nodes x 1000 frames 4.25 and 4.55 us,
-// 1024 x 1024 4.90 and 5.14; 1500 x 600 5.71 and 4.72, 3000 x 400 5.44 and 4.61, 4000 x 300 6.7 and 5.3, 6144 x 1024 15.4 and 9.5.  0: up to 64 frames, one per lane.
-// Each count has a form of its own, whose inputs are all requested at once: two passes in the form for two and in that for four, 1100 x 512 4.03 and 4.18 us, 3000 x 300 4.65 and 4.73, packed
-// inference 1500 x 512 3.50 and 3.74, four inputs per node, 6144 x 400, 5.52 and 5.68; up to 64 frames in the form for one frame per lane and in that for one pass, 360 x 64 3.18
-// and 3.35, fp32 frames 3.34 and 3.63, 7372 x 31 6.32 and 6.54, fp32 6.52 and 7.46.
+// all, one after another, where nodes alone fill the device.  Side by side and one after another, 784 inputs: batch-norm training call on fp32 frames 700 nodes x 1000 frames
+// 4.89 and 5.93 us, 1024 x 1024 5.18 and 5.73, 1200 x 1024 6.99 and 7.11; 1500 x 600 6.46 and 5.60, 3000 x 400 7.57 and 7.13, 4000 x 300 8.81 and 7.98, 6144 x 1024 15.0 and 10.9 (packed
+// frames 700 x 1000 4.03 and 4.12, 1024 x 1024 4.21 and 3.96, 1500 x 600 5.19 and 4.34, packed inference 1024 x 1024 3.41 and 3.56).  0: up to 64 frames, one per lane.
+// Each count has a form of its own, whose inputs are all requested at once: two passes in the form for two and in that for four, packed training call 1100 x 512 3.81 and 3.93 us,
+// 3000 x 300 4.35 and 4.68, inference 1500 x 512 3.27 and 3.42, four inputs per node, 6144 x 400, training call 5.19 and 5.23; up to 64 frames in the form for one frame per lane and
+// in that for one pass, 360 x 64 2.89 and 3.06, fp32 frames 2.93 and 3.39, 7372 x 31 5.68 and 6.22, fp32 5.75 and 6.99.
 constexpr int kQuadFrames = 256, kQuadMost = 1024;               // frames of a pass, most frames of a node there
 inline int forward_quad_passes(int node_size, int frame_size) { return frame_size <= 64 ? 0 : (node_size <= 1024 || frame_size <= kQuadFrames) ? 1 : frame_size <= 2 * kQuadFrames ? 2 : 4; }
 

@@ -355,7 +355,7 @@ int main(void)
 
     // passes of a wavefront in the forward pass of up to 1024 frames, where both were measured (microseconds)
     {
-        struct { int nodes, frames; double side_by_side, in_turn; } const rows[] = {{700, 1000, 4.25, 4.55}, {1024, 1024, 4.90, 5.14}, {1500, 600, 5.71, 4.72}, {4000, 300, 6.73, 5.25}, {6144, 1024, 15.4, 9.5}};
+        struct { int nodes, frames; double side_by_side, in_turn; } const rows[] = {{700, 1000, 4.89, 5.93}, {1024, 1024, 5.18, 5.73}, {1500, 600, 6.46, 5.60}, {3000, 400, 7.57, 7.13}, {4000, 300, 8.81, 7.98}, {6144, 1024, 15.0, 10.9}};
         for (auto const &r : rows) { CHECK((bbhip::forward_quad_passes(r.nodes, r.frames) == 1) == (r.side_by_side < r.in_turn)); }
         CHECK(bbhip::forward_quad_passes(8000, 64) == 0 && bbhip::forward_quad_passes(8000, 65) == 1 && bbhip::forward_quad_passes(8000, 256) == 1 &&
               bbhip::forward_quad_passes(8000, 512) == 2 && bbhip::forward_quad_passes(8000, 513) == 4);
