@@ -2587,8 +2587,11 @@ static int launch_binary_to_real_forward(void const *x, bool bit, float *y, int 
     if (modulation_grid(y_node_size, y_frame_size, false, a.f_blocks, blocks, name)) { return 1; }
     hipStream_t const st = static_cast<hipStream_t>(stream);
     ScopedTimer tm(kTimeOther, st);
-    if (bit) { launch((binary_to_real_forward_kernel<true>), dim3(blocks), dim3(kModBlock), 0, st, a); }
-    else     { launch((binary_to_real_forward_kernel<false>), dim3(blocks), dim3(kModBlock), 0, st, a); }
+    FoldedWords const words = folded_words(frame_mux_size);
+    if (!bit)                     { launch((binary_to_real_forward_kernel<false, kManyWords>), dim3(blocks), dim3(kModBlock), 0, st, a); }
+    else if (words == kWholeWord) { launch((binary_to_real_forward_kernel<true, kWholeWord>), dim3(blocks), dim3(kModBlock), 0, st, a); }
+    else if (words == kTwoWords)  { launch((binary_to_real_forward_kernel<true, kTwoWords>), dim3(blocks), dim3(kModBlock), 0, st, a); }
+    else                          { launch((binary_to_real_forward_kernel<true, kManyWords>), dim3(blocks), dim3(kModBlock), 0, st, a); }
     BBHIP_LAUNCH_CHECK();
     return 0;
 }

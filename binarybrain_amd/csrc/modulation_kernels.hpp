@@ -189,9 +189,13 @@ struct BinaryToRealArgs {
 };
 
 // y[o][g] = (number of inputs > 0 among nodes o, O + o, ... and frames g * fmux ... g * fmux + fmux - 1) / their number
-// A launch of this is latency: packed rows are requested up to eight at a time (one after another, each waited for the one before: 70 nodes -> 10, 500 frames of
-// seven 3.2 us and 2.2 as it is, 1600 -> 100, 10000 of seven 20.9 and 6.6).
-template <bool BIT>
+// A launch of this is latency: packed rows are requested up to eight at a time, each of them a word or, where frames reach into the next, two (one after another,
+// each waited for the one before: 70 nodes -> 10, 500 frames of seven 3.5 us and 2.6 as it is, 1600 -> 100, 10000 of seven 21.4 and 6.8).  More than 32 frames go word by word,
+// a group's words before the next group's rows; in pieces of 32 frames, two words for each, 5 rows x 64 frames, 138 -> 1367, took 4.5 us, 4 rows x 127, 28 -> 6481, 7.4 and
+// 1 row x 64, 850 -> 2635, 8.8, now 3.4, 5.4 and 7.2.  A kernel for each of the three: as branches of one they cost the second shape above 1.6 us.
+enum FoldedWords : int { kWholeWord = 1, kTwoWords = 2, kManyWords = 3 };                    // what the frames of a packed row that fold into one lie in, at most
+inline FoldedWords folded_words(int frame_mux_size) { return frame_mux_size > 32 ? kManyWords : 32 % frame_mux_size == 0 ? kWholeWord : kTwoWords; }
+template <bool BIT, int WORDS>
 __global__ __launch_bounds__(kModBlock) void binary_to_real_forward_kernel(BinaryToRealArgs a)
 {
     int o, block;
@@ -201,29 +205,46 @@ __global__ __launch_bounds__(kModBlock) void binary_to_real_forward_kernel(Binar
     int const first = g * a.frame_mux_size;
     unsigned count = 0;                                 // below 2^24: a whole number in fp32 too
     if constexpr (BIT) {
-        unsigned f = (unsigned)first;
-        for (int left = a.frame_mux_size; left > 0; f += 32, left -= 32) {           // up to 32 frames of every row: two words, shifted together
-            unsigned const take = (unsigned)min(left, 32), lo = f >> 5, hi = (f + take - 1) >> 5;
-            uint32_t const mask = 0xffffffffu >> (32 - take);
-            int m = 0;
-            auto rows = [&](auto together) {                                                   // of so many rows at a time
-                constexpr int R = decltype(together)::value;
-                for (; m + R <= a.node_mux_size; m += R) {
+        unsigned const f = (unsigned)first, lo = f >> 5, hi = (f + (unsigned)a.frame_mux_size - 1u) >> 5;
+        uint32_t const mask = 0xffffffffu >> (32 - min(a.frame_mux_size, 32));
+        int m = 0;
+        auto rows = [&](auto together) {                                                   // of so many rows at a time
+            constexpr int R = decltype(together)::value;
+            for (; m + R <= a.node_mux_size; m += R) {
+                uint32_t const *__restrict__ xr[R];
+#pragma unroll
+                for (int j = 0; j < R; ++j) { xr[j] = static_cast<uint32_t const *>(a.x) + (size_t)((m + j) * a.y_node_size + o) * a.x_stride; }
+                if constexpr (WORDS != kManyWords) {
                     uint32_t w0[R], w1[R];
 #pragma unroll
                     for (int j = 0; j < R; ++j) {
-                        uint32_t const *__restrict__ xr = static_cast<uint32_t const *>(a.x) + (size_t)((m + j) * a.y_node_size + o) * a.x_stride;
-                        w0[j] = xr[lo]; w1[j] = xr[hi];
+                        w0[j] = xr[j][lo];
+                        if constexpr (WORDS == kTwoWords) { w1[j] = xr[j][hi]; }            // (the same one, shifted in behind itself, where there is no other)
+                        else                              { w1[j] = 0; }
                     }
 #pragma unroll
                     for (int j = 0; j < R; ++j) { count += __popc(__builtin_amdgcn_alignbit(w1[j], w0[j], f & 31u) & mask); }
                 }
-            };
-            rows(std::integral_constant<int, 8>{});
-            rows(std::integral_constant<int, 4>{});
-            rows(std::integral_constant<int, 2>{});
-            rows(std::integral_constant<int, 1>{});
-        }
+                else {
+                    unsigned from = f;
+                    for (int left = a.frame_mux_size; left > 0;) {
+                        unsigned const at = from & 31u;
+                        int const take = min(32 - (int)at, left);
+                        uint32_t const in_frames = (0xffffffffu >> (32 - take)) << at;
+                        uint32_t w[R];
+#pragma unroll
+                        for (int j = 0; j < R; ++j) { w[j] = xr[j][from >> 5]; }
+#pragma unroll
+                        for (int j = 0; j < R; ++j) { count += __popc(w[j] & in_frames); }
+                        from += (unsigned)take; left -= take;
+                    }
+                }
+            }
+        };
+        rows(std::integral_constant<int, 8>{});
+        rows(std::integral_constant<int, 4>{});
+        rows(std::integral_constant<int, 2>{});
+        rows(std::integral_constant<int, 1>{});
     }
     else {
         for (int m = 0; m < a.node_mux_size; ++m) {

@@ -89,9 +89,9 @@ def test_binary_to_real(ops, shape, aligned):
 
 
 @pytest.mark.parametrize("mux", [1, 2, 3, 5, 7, 8, 9, 15, 17])
-@pytest.mark.parametrize("fm", [1, 31, 32, 33, 63, 65])
+@pytest.mark.parametrize("fm", [1, 31, 32, 33, 63, 64, 65, 128])
 def test_binary_to_real_row_groups(ops, mux, fm):
-    """packed rows are read up to eight at a time and 32 frames at a time: every remainder of both"""
+    """packed rows are read up to eight at a time, a word or parts of two up to 32 frames, else word by word: every remainder, aligned and not"""
     O, Fy = 3, 67
     rng = np.random.default_rng(100 * mux + fm)
     xb = synth.bernoulli_bits(rng, O * mux, Fy * fm, (Fy * fm + 31) // 32)
