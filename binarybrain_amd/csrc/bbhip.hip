@@ -948,7 +948,8 @@ int run_backward_corner(BackwardCall const &call, hipStream_t st, PackedInputHin
     d.dy_stride = c.frame_stride; d.dx_stride = c.frame_stride;
     d.chunk = quads * 256; d.chunk_count = ceil_div(c.frame_size, d.chunk);
     int split          = dx_split_lists(c.rev_stride - 1, c.input_node_size, d.chunk_count);
-    // Long passes leave at least 2048 workgroups, with which sixteen wavefronts never share a list: only BBHIP_DX_QUADS brings the two together
+    // Long passes leave a thousand groups of four inputs (dx_table_quads), with which sixteen wavefronts do not share a list: only a layer of one input and BBHIP_DX_QUADS
+    // bring the two together
     if (quads > 1 && split > kWavesPerBlk) { split = kWavesPerBlk; }
     int const in_tiles = split ? c.input_node_size : ceil_div(c.input_node_size, kWavesPerBlk);
     if ((long long)d.chunk_count * in_tiles > 0x7fffffffLL) { return fail("backward: grid too large"); }

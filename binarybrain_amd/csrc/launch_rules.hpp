@@ -79,18 +79,22 @@ inline int corner_small_waves(int n, bool batch_norm, int frame_size, int input_
 // dy and of indices that they gather from (5 bytes per node and frame) stay in an XCD's L2, and where the launch does not fall short of workgroups: a
 // workgroup is four inputs, or one whose list its wavefronts share (27 inputs x 87 nodes x 94500 frames in passes of 256 / 512 / 1024 frames, convolutional
 // block with 10000 / 5000 / 2500 workgroups: 125 / 117 / 122 us; 27 x 216 x 230400 371 / 348 / 346).
-// Two passes, training call with one and with two: from 1000 groups of four inputs and up to 1350 nodes six inputs 560 x 1055 x 3778 32.9 and 29.4 us, 1500 x
-// 1200 x 4000 33.6 and 31.5, 3664 x 1195 x 7782 60.9 and 55.0, 333 x 469 x 5793 25.1 and 24.5; five, 632 x 1175 x 5013 37.4 and 32.8; four, 2909 x 1145 x 1358 21.2 and
-// 20.0; 35 drawn shapes with two passes here where the lines were 2048 groups and 1024 nodes 0.88 to 1.05, 0.96 on average.  Tables of five and six inputs also up to 1600 nodes where two passes end in one round of the 2048
-// workgroups that fit: 1000 x 1500 x 3000 34.4 and 30.5, 877 x 1425 x 3698 36.4 and 33.0; but 1727 x 1444 x 9479 67.0 and 68.6, 3987 x 1569 x
-// 514 19.1 and 19.9, four inputs 1888 x 1524 x 1628 22.0 and 22.5, 1000 x 2000 x 8000, six, 67.7 and 69.1.  Fewer workgroups: six, 2754 x 1341 x 498 (689) 16.2 and 17.8, 98 x 1550 x 1284 (75) 24.4 and 28.6.
+// Two passes of 256 frames: up to 1350 nodes, 1024 of two and three inputs, from 1000 groups of four inputs with frames for both passes.  Backward call, batch-norm, with one and with two: six inputs 605 x 1347
+// x 3349 28.0 and 25.6 us, 3418 x 753 x 988 12.6 and 11.7, 168 x 959 x 17363 60.1 and 53.5; five, 242 x 1186 x 18195 65.5 and 58.3, 1724 x 675 x 1937 14.4 and 13.1; four, 701 x 1067 x 3501 21.7 and
+// 19.0; three, 1775 x 945 x 1869 13.5 and 12.3; but 1708 x 1259 x 14639 54.4 and 57.4, two, 527 x 1189 x 15747 42.6 and 45.0, 785 x 1317 x 2914 16.3
+// and 17.3.  The count leaves out passes that the last frames do not fill: six, 1418 x 705 x 1150 (888; 1065 with them) 13.0 and 14.0, 1348 x 896 x 1164 (842) 14.2
+// and 15.0; fewer, 367 x 820 x 4634 (874) 25.0 and 23.1, but 2756 x 1341 x 498 (689) 16.2 and 17.8, 1074 x 1160 x 1222, four, (672) 13.3 and 14.5.
+// Tables of five and six inputs also up to 1600 nodes where wavefronts share the lists and two passes end in one round of the 2048 workgroups that fit: six, 457 x 1398 x 5546 36.7 and 32.8, 1206 x
+// 1382 x 1813 22.0 and 19.6, 1511 x 1428 x 2118 28.4 and 24.7; five, 773 x 1482 x 3855 29.1 and 24.6; but lists of up to 15, six, 2354 x 1398 x 1030 17.4 and 18.1, 1462 x 1444 x 2122 23.9 and 24.9, five, 1529 x
+// 1382 x 1275 15.0 and 16.0, and 2048 workgroups and more, 1762 x 1542 x 2740, 24.5 and 26.5.  What lies beyond is mixed: six, 510 x 1482 x 10237 (2560 groups) 55.6 and 49.7, 548 x 1723 x 5985 42.5 and 38.5,
+// 2613 x 1769 x 1058 19.1 and 21.2; three, 537 x 1525 x 6560 31.7 and 28.4, 1266 x 1522 x 1667 15.3 and 16.0.
 inline int dx_table_quads(int n, int input_node_size, int output_node_size, int frame_size, bool long_lists)
 {
     auto const groups = [&](int q) { return (long long)ceil_div(frame_size, q * 256) * ceil_div(input_node_size, 4); };
     auto const shared = [&](int q) { return long_lists && (long long)ceil_div(frame_size, q * 256) * input_node_size >= 3072; };
     if (output_node_size <= 512 && (groups(4) >= 2048 || shared(4))) { return 4; }
-    if (output_node_size <= 1350 && (groups(2) >= 1000 || shared(2))) { return 2; }
-    return (n >= 5 && output_node_size <= 1600 && frame_size > 1024 && groups(2) >= 1000 && groups(2) <= 2048) ? 2 : 1;
+    if (output_node_size <= (n >= 4 ? 1350 : 1024) && (groups(1) >= 2000 || shared(2))) { return 2; }
+    return (n >= 5 && output_node_size <= 1600 && frame_size > 1024 && long_lists && groups(2) >= 1000 && groups(2) <= 2048) ? 2 : 1;
 }
 
 // Whether the sixteen wavefronts that share an input's list in lut_dx_table_kernel take its items in turn (they then walk the nodes together, and rows that

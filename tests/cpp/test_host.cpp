@@ -405,7 +405,10 @@ int main(void)
             {6, 560, 1055, 3778, 22, 32.9, 29.4}, {5, 632, 1175, 5013, 21, 37.2, 32.8}, {6, 3664, 1195, 7782, 8, 60.8, 55.0}, {6, 807, 1033, 12218, 18, 62.8, 59.4},
             {6, 877, 1425, 3698, 21, 36.5, 33.0}, {6, 1727, 1444, 9479, 14, 67.0, 68.6}, {6, 3987, 1569, 514, 9, 19.0, 19.9}, {5, 1833, 1530, 6448, 12, 46.9, 48.9},
             {4, 2909, 1145, 1358, 8, 20.6, 20.0}, {2, 825, 468, 4363, 5, 18.7, 17.4}, {5, 333, 469, 5793, 14, 25.4, 24.5}, {6, 2754, 1341, 498, 11, 16.2, 17.8},
-            {6, 2046, 2018, 1150, 15, 25.6, 27.1}, {6, 98, 1550, 1284, 117, 24.2, 28.6}, {6, 585, 772, 5509, 16, 35.0, 30.2}};
+            {6, 2046, 2018, 1150, 15, 25.6, 27.1}, {6, 98, 1550, 1284, 117, 24.2, 28.6}, {6, 585, 772, 5509, 16, 35.0, 30.2},
+            // (backward call alone)
+            {6, 1418, 705, 1150, 12, 13.0, 14.0}, {6, 1348, 896, 1164, 13, 14.2, 15.0}, {6, 3418, 753, 988, 8, 12.6, 11.7}, {3, 1775, 945, 1869, 7, 13.5, 12.3}, {5, 1529, 1382, 1275, 14, 15.0, 16.0},
+            {6, 1206, 1382, 1813, 19, 22.0, 19.6}, {6, 1511, 1428, 2118, 16, 28.4, 24.7}, {5, 773, 1482, 3855, 20, 29.1, 24.6}, {6, 168, 959, 17363, 50, 60.1, 53.5}, {6, 2919, 482, 519, 6, 10.3, 10.6}, {3, 1708, 1259, 14639, 9, 54.4, 57.4}, {2, 527, 1189, 15747, 11, 42.6, 45.0}, {2, 2386, 762, 12598, 5, 40.3, 39.5}};
         for (auto const &r : rows) {
             double const taken = bbhip::dx_table_quads(r.n, r.inputs, r.nodes, r.frames, r.max_fan > 15) == 1 ? r.one : r.two;
             if (taken > 1.05 * std::min(r.one, r.two)) { std::printf("%d x %d x %d\n", r.inputs, r.nodes, r.frames); CHECK(!"dx_table_quads"); }
