@@ -174,10 +174,10 @@ __device__ __forceinline__ void few_inputs_by_lists(FewInputsArgs const &a, int 
 // The node's tables are formed by corner_fold, once per call.
 // The wiring is that of the index table where the launch before has found the same in the reverse table (ReverseRows); else (a caller's own table that
 // leaves connections out, say) the workgroup goes by the lists, an input after another, without hurry.
-// Bound by LDS (two random 16-byte reads per frame and node: 20 clocks per 64 frames; four 8-byte reads take 18 if the compiler leaves them apart, 40 if it
-// pairs them) and by what the four wavefronts of a SIMD leave idle around it.  27 inputs x 216 nodes x 230400 frames, six per node: 80 -> 52 us (dy at 3.9 TB/s), and
+// Bound by LDS (two random 16-byte reads per frame and node: 20 clocks per 64 frames, 22 with the row of dy by the counters, 12 of them for bank conflicts, LDS
+// busy for 68 % of the time; four 8-byte reads take 18 if the compiler leaves them apart, 40 if it pairs them) and by what the four wavefronts of a SIMD leave idle around it.  27 inputs x 216 nodes x 230400 frames, six per node: 80 -> 52 us (dy at 3.9 TB/s), and
 // the sums launch, which has no indices to keep, 50 -> 38; with tables formed by the workgroups themselves 59 us, with dy through registers 53.
-// One frame of 1800 x 128 per wavefront leaves 450 workgroups for 512 places.
+// (230400 frames are 450 workgroups of 512 frames, of which the device holds 512 at once.)
 template <int N, bool BN>
 __global__ __launch_bounds__(kFewWaves * kWave) __attribute__((amdgpu_waves_per_eu(4, 4))) void lut_dx_few_inputs_kernel(FewInputsArgs a)
 {

@@ -80,6 +80,8 @@ int bbhip_GetSwitch(char const *name);
  * 0 (default): deterministic, no scratch — one wavefront per (input node, frame chunk) walks reverse_index in the
  *              reference's order (cuda/Common.cuh:174-202, include/bb/FixedSizeConnectionTable.h:198-214) and
  *              re-evaluates each consumer's dy/dx from that consumer's other inputs; needs reverse_index, ignores dx_tmp.
+ *              (Up to 28 two-valued inputs over more than 97792 frames: node by node, after a look through reverse_index;
+ *              one that is not the reverse of input_index is walked as anywhere else.)
  * 1          : fp32 atomic adds into a zero-filled dx; dx_tmp and reverse_index may be NULL; summation order is
  *              not reproducible between runs.
  * 2          : the reference's scheme — per-connection gradients go to dx_tmp ([output_node_size*n][tmp_frame_stride],
