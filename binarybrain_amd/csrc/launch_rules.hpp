@@ -79,21 +79,25 @@ inline int corner_small_waves(int n, bool batch_norm, int frame_size, int input_
 // dy and of indices that they gather from (5 bytes per node and frame) stay in an XCD's L2, and where the launch does not fall short of workgroups: a
 // workgroup is four inputs, or one whose list its wavefronts share (27 inputs x 87 nodes x 94500 frames in passes of 256 / 512 / 1024 frames, convolutional
 // block with 10000 / 5000 / 2500 workgroups: 125 / 117 / 122 us; 27 x 216 x 230400 371 / 348 / 346).
-// Two passes of 256 frames: up to 1350 nodes, 1024 of two and three inputs, from 1000 groups of four inputs with frames for both passes.  Backward call, batch-norm, with one and with two: six inputs 605 x 1347
-// x 3349 28.0 and 25.6 us, 3418 x 753 x 988 12.6 and 11.7, 168 x 959 x 17363 60.1 and 53.5; five, 242 x 1186 x 18195 65.5 and 58.3, 1724 x 675 x 1937 14.4 and 13.1; four, 701 x 1067 x 3501 21.7 and
-// 19.0; three, 1775 x 945 x 1869 13.5 and 12.3; but 1708 x 1259 x 14639 54.4 and 57.4, two, 527 x 1189 x 15747 42.6 and 45.0, 785 x 1317 x 2914 16.3
-// and 17.3.  The count leaves out passes that the last frames do not fill: six, 1418 x 705 x 1150 (888; 1065 with them) 13.0 and 14.0, 1348 x 896 x 1164 (842) 14.2
-// and 15.0; fewer, 367 x 820 x 4634 (874) 25.0 and 23.1, but 2756 x 1341 x 498 (689) 16.2 and 17.8, 1074 x 1160 x 1222, four, (672) 13.3 and 14.5.
-// Tables of five and six inputs also up to 1600 nodes where wavefronts share the lists and two passes end in one round of the 2048 workgroups that fit: six, 457 x 1398 x 5546 36.7 and 32.8, 1206 x
-// 1382 x 1813 22.0 and 19.6, 1511 x 1428 x 2118 28.4 and 24.7; five, 773 x 1482 x 3855 29.1 and 24.6; but lists of up to 15, six, 2354 x 1398 x 1030 17.4 and 18.1, 1462 x 1444 x 2122 23.9 and 24.9, five, 1529 x
-// 1382 x 1275 15.0 and 16.0, and 2048 workgroups and more, 1762 x 1542 x 2740, 24.5 and 26.5.  What lies beyond is mixed: six, 510 x 1482 x 10237 (2560 groups) 55.6 and 49.7, 548 x 1723 x 5985 42.5 and 38.5,
-// 2613 x 1769 x 1058 19.1 and 21.2; three, 537 x 1525 x 6560 31.7 and 28.4, 1266 x 1522 x 1667 15.3 and 16.0.
+// Two passes, training call whose inputs and buffers are other ones than those of the call before (four sets in turn; from one set, which the L2s hold in part, two passes look up to 12 % better), with
+// one and with two: from 2000 groups of four inputs in passes of 256 frames, which leaves out what the last frames do not fill, lists of 4.5 items on average up to 1350 nodes, 1024 of two and three
+// inputs: six inputs 605 x 1347 x 3349 32.5 and 30.7 us, 585 x 772 x 5509 34.3 and 30.1, 168 x 959 x 17363 78.7 and 73.2; five, 632 x 1175 x 5013 36.5 and 31.7, 750 x 1231 x 2879 29.1 and 26.2; four,
+// 701 x 1067 x 3501 27.2 and 25.6, 910 x 1232 x 2723 26.7 and 25.3; three, 408 x 943 x 7051 31.0 and 28.6.  Shorter lists gain only where workgroups abound: six, 1336 x 804 x 1505 20.1 and 20.6, 2740 x
+// 921 x 734 16.6 and 17.6, 1023 x 695 x 1921 20.1 and 20.8; four, 1341 x 902 x 1385 18.1 and 19.1, 1764 x 1151 x 1263 19.1 and 20.5, 3845 x 1301 x 687 17.0 and 17.9, 2328 x 1331 x 3232 (7566
+// groups) 28.8 and 29.6; but six, 6144 x 1024 x 1024 (3072 groups in passes of 512) 19.3 and 18.6, 3664 x 1195 x 7782 (28396 in passes of 256) 57.9 and 52.8, five, 6653 x 1291 x 1828 (13312) 28.5 and 27.0.  Up
+// to 512 nodes any list: 1391 x 128 x 1469, six, 16.8 and 16.5, 337 x 445 x 6515 30.0 and 27.3, 511 x 128 x 9917, two, 17.7 and 17.1, but 111 x 237 x 38759 31.3 and 32.2.  Fewer groups: six, 1418 x 705 x 1150 18.5 and 19.9, 1348 x 896 x
+// 1164 19.7 and 21.0, 2754 x 1341 x 498 16.7 and 17.6; three inputs, 1708 x 1259 x 14639 74.2 and 73.1, two, 527 x 1189 x 15747 58.8 and 61.0.
+// Tables of five and six inputs also up to 1600 nodes where wavefronts share the lists and two passes end in one round of the 2048 workgroups that fit: six, 457 x 1398 x 5546 41.6 and 39.0, 1206 x
+// 1382 x 1813 27.9 and 25.4, 1000 x 1500 x 3000 34.1 and 30.8; five, 773 x 1482 x 3855 34.2 and 30.1; but lists of up to 15, six, 2354 x 1398 x 1030 23.6 and 24.6, five, 1529 x 1382 x 1275 21.2
+// and 22.6, and 2048 workgroups and more, 1762 x 1542 x 2740, 32.7 and 35.1, five, 1833 x 1530 x 6448 47.2 and 48.9.
 inline int dx_table_quads(int n, int input_node_size, int output_node_size, int frame_size, bool long_lists)
 {
     auto const groups = [&](int q) { return (long long)ceil_div(frame_size, q * 256) * ceil_div(input_node_size, 4); };
     auto const shared = [&](int q) { return long_lists && (long long)ceil_div(frame_size, q * 256) * input_node_size >= 3072; };
     if (output_node_size <= 512 && (groups(4) >= 2048 || shared(4))) { return 4; }
-    if (output_node_size <= (n >= 4 ? 1350 : 1024) && (groups(1) >= 2000 || shared(2))) { return 2; }
+    bool const many = output_node_size <= 512 ? groups(1) >= 2000 : output_node_size <= 1024 ? groups(2) >= 2048 : groups(1) >= 10000;
+    bool const listed = groups(1) >= 2000 && 2LL * output_node_size * n >= 9LL * input_node_size;
+    if (output_node_size <= (n >= 4 ? 1350 : 1024) && (many || listed || shared(2))) { return 2; }
     return (n >= 5 && output_node_size <= 1600 && frame_size > 1024 && long_lists && groups(2) >= 1000 && groups(2) <= 2048) ? 2 : 1;
 }
 

@@ -406,9 +406,13 @@ int main(void)
             {6, 877, 1425, 3698, 21, 36.5, 33.0}, {6, 1727, 1444, 9479, 14, 67.0, 68.6}, {6, 3987, 1569, 514, 9, 19.0, 19.9}, {5, 1833, 1530, 6448, 12, 46.9, 48.9},
             {4, 2909, 1145, 1358, 8, 20.6, 20.0}, {2, 825, 468, 4363, 5, 18.7, 17.4}, {5, 333, 469, 5793, 14, 25.4, 24.5}, {6, 2754, 1341, 498, 11, 16.2, 17.8},
             {6, 2046, 2018, 1150, 15, 25.6, 27.1}, {6, 98, 1550, 1284, 117, 24.2, 28.6}, {6, 585, 772, 5509, 16, 35.0, 30.2},
-            // (backward call alone)
-            {6, 1418, 705, 1150, 12, 13.0, 14.0}, {6, 1348, 896, 1164, 13, 14.2, 15.0}, {6, 3418, 753, 988, 8, 12.6, 11.7}, {3, 1775, 945, 1869, 7, 13.5, 12.3}, {5, 1529, 1382, 1275, 14, 15.0, 16.0},
-            {6, 1206, 1382, 1813, 19, 22.0, 19.6}, {6, 1511, 1428, 2118, 16, 28.4, 24.7}, {5, 773, 1482, 3855, 20, 29.1, 24.6}, {6, 168, 959, 17363, 50, 60.1, 53.5}, {6, 2919, 482, 519, 6, 10.3, 10.6}, {3, 1708, 1259, 14639, 9, 54.4, 57.4}, {2, 527, 1189, 15747, 11, 42.6, 45.0}, {2, 2386, 762, 12598, 5, 40.3, 39.5}};
+            // (with other inputs and buffers than the call before)
+            {6, 1418, 705, 1150, 12, 18.5, 19.9}, {6, 1348, 896, 1164, 13, 19.7, 21.0}, {6, 3418, 753, 988, 8, 17.2, 17.0}, {3, 1775, 945, 1869, 7, 18.9, 19.3}, {5, 1529, 1382, 1275, 14, 21.2, 22.6},
+            {6, 1206, 1382, 1813, 19, 27.9, 25.4}, {6, 1511, 1428, 2118, 16, 31.3, 30.4}, {5, 773, 1482, 3855, 20, 34.2, 30.1}, {6, 168, 959, 17363, 50, 78.7, 73.2}, {6, 2919, 482, 519, 6, 15.9, 15.9},
+            {3, 1708, 1259, 14639, 9, 74.2, 73.1}, {2, 527, 1189, 15747, 11, 58.8, 61.0}, {2, 2386, 762, 12598, 5, 47.1, 46.6}, {6, 1336, 804, 1505, 12, 20.1, 20.6}, {6, 2740, 921, 734, 9, 16.6, 17.6},
+            {4, 1341, 902, 1385, 10, 18.1, 19.1}, {4, 1764, 1151, 1263, 10, 19.1, 20.5}, {4, 1016, 898, 1816, 12, 18.5, 19.4}, {4, 3845, 1301, 687, 7, 17.0, 17.9}, {5, 3141, 1142, 568, 8, 16.9, 17.8},
+            {5, 6653, 1291, 1828, 6, 28.5, 27.0}, {5, 440, 623, 8009, 15, 34.9, 30.8}, {5, 968, 1345, 3056, 17, 30.8, 27.6}, {4, 910, 1232, 2723, 14, 26.7, 25.3}, {4, 5773, 1346, 3968, 6, 38.0, 34.8},
+            {6, 2316, 1272, 1222, 11, 23.0, 24.2}, {6, 605, 1347, 3349, 26, 32.5, 30.7}, {6, 851, 1206, 2832, 19, 32.1, 28.9}};
         for (auto const &r : rows) {
             double const taken = bbhip::dx_table_quads(r.n, r.inputs, r.nodes, r.frames, r.max_fan > 15) == 1 ? r.one : r.two;
             if (taken > 1.05 * std::min(r.one, r.two)) { std::printf("%d x %d x %d\n", r.inputs, r.nodes, r.frames); CHECK(!"dx_table_quads"); }

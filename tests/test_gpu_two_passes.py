@@ -1,4 +1,4 @@
-"""GPU parity of dx over two-valued inputs at the lines between passes of 256 and of 512 frames: 1350 and 1600 nodes, 1000 groups, long and short lists, a second pass of one frame."""
+"""GPU parity of dx over two-valued inputs at the lines between passes of 256 and of 512 frames: 512, 1024, 1350 and 1600 nodes, 2000 and 10000 groups, long and short lists, a second pass of one frame."""
 import pytest
 import torch
 
@@ -8,7 +8,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n, I, O, F", [(6, 800, 1350, 2049), (6, 800, 1350, 2048), (4, 800, 1351, 2049), (5, 1400, 1600, 1025), (2, 1333, 1025, 1281), (3, 40, 24, 51201),
-                                        (6, 892, 1350, 2049), (6, 1000, 1350, 2048), (6, 996, 1350, 2048), (5, 480, 1600, 4097), (5, 480, 1601, 4097), (4, 1600, 700, 1025)])
+                                        (6, 892, 1350, 2049), (6, 1000, 1350, 2048), (6, 996, 1350, 2048), (5, 480, 1600, 4097), (5, 480, 1601, 4097), (4, 1600, 700, 1025), (4, 3000, 1030, 3585), (4, 3000, 1030, 3300),
+                                        (6, 1333, 1000, 1281), (6, 1333, 999, 1281), (2, 900, 512, 2049), (2, 900, 513, 2049)])
 def test_dx_in_two_passes(n, I, O, F):
     from binarybrain_amd import ops
     ops.set_dx_mode(0)
